@@ -182,15 +182,16 @@ namespace en {
 // ---------------------------------------------------------------------------------------------------------------
 // Single-pass decode attention: ctx = softmax(scale * q K^T) V for one query per sequence, K and V each read
 // once, scores and probabilities never written.  One workgroup per (batch, head); LPK lanes cover one cached row
-// (16 bytes each), so the workgroup's NT / LPK lane groups take NT / LPK keys per step.  Two stages of registers:
-// the K and V pieces of the next step are in flight while this step's are worked on, and the kernel stays within
-// 64 registers so that two 1024-lane workgroups share a CU (measured on 72 heads x 64 caches of up to 2048
-// positions, 2.6 GB: 6.7 TB/s; four pieces per lane and stage at one workgroup per CU 5.9, one stage of four
-// pieces as in the two-kernel forms 5.3; a third stage spills).  Each lane group carries its own running maximum, sum and
-// output slice (online softmax, maximum and exponent in the log2 domain with the scale folded in); the groups are
-// combined once, through LDS, at the end.  The sequences are taken longest first (rank computed inside each
-// workgroup from the lengths, batches of up to kRankBatch): the launch then ends on its short units instead of on
-// whatever the last batch index happens to hold.
+// (16 bytes each), so the workgroup's NT / LPK lane groups take U * NT / LPK keys per stage.  Two stages of registers:
+// the K and V pieces of the next one are in flight while this one's are worked on.  Bound by the reads of the caches
+// (large batches: 6.8 TB/s, what a kernel that only reads reaches) and, for small batches, by what a launch costs before
+// its first byte arrives and after its last (an empty launch 2.8 us, 16 keys 4.4 us).  NT and U: see AttnForm.
+// Each lane group carries its own running maximum, sum and output slice (online softmax, maximum and exponent in the
+// log2 domain with the scale folded in).  At the end the groups of a wave are combined in registers and the waves
+// through LDS: every group through LDS (33 KB, one lane per channel adding up 64 rows) took 2 us of a workgroup's life
+// and left no room for a third workgroup (72 units of 1655 keys, unsplit: 38 -> 21.8 us at 1024 x 1).
+// The sequences are taken longest first (rank computed inside each workgroup from the lengths, batches of up to
+// kRankBatch): the launch then ends on its short units instead of on whatever the last batch index happens to hold.
 // ---------------------------------------------------------------------------------------------------------------
 struct DecodeAttnArgs {
   const void *q;      // [B,H,D]
@@ -216,34 +217,55 @@ __device__ __forceinline__ int split_share(int kl, int nsplit) {
 
 constexpr int kRankBatch = 256;
 
-template <int DT, int LPK, bool STREAM, bool BIG, bool PAGED = false>
-__global__ __launch_bounds__(BIG ? kStreamBlock : kBlock, 8) void decode_attn_kernel(DecodeAttnArgs a) {
-  constexpr int NT = BIG ? kStreamBlock : en::kBlock;
+// From this size on (K and V together) the single pass reads the caches with non-temporal loads: a step walks the caches
+// of every layer before it comes back to these, and four layers of 64 MB are the whole memory-side cache (61 MB read
+// cold: 14.1 -> 13.2 us; 18 MB still in that cache: 6.3 -> 6.7 us).
+constexpr int64_t kAttnStreamBytes = 64ll << 20;
+
+// Sum or maximum over the lane groups of a wave (lanes that hold the same channels): every lane ends with the result.
+// Rows of 16 lanes are swapped with permlane swaps, groups of 8 and 4 lanes inside a row rotated with DPP: no LDS.
+template <typename Op, int LPK>
+__device__ __forceinline__ float across_groups(float v) {
+  if (LPK <= 4) v = Op::apply(v, dpp_move<0x124>(v));   // row_ror:4
+  if (LPK <= 8) v = Op::apply(v, dpp_move<0x128>(v));   // row_ror:8
+  if (LPK <= 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = Op::apply(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  if (LPK <= 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = Op::apply(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  return v;
+}
+
+template <int DT, int LPK, int NT, int U, bool STREAM, bool PAGED = false>
+__global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeAttnArgs a) {
   typedef Elem<DT> E;
   typedef typename E::T T;
   constexpr int EPV = 16 / E::kSize;
   constexpr int G = NT / LPK;        // lane groups = keys per step
-  constexpr int U = 1;               // keys per lane group and stage
+  constexpr int NW = NT / kWave;
   constexpr int W = LPK * EPV;       // channels the lanes of a group cover (>= D)
-  __shared__ float s_m[G], s_l[G], s_w[G];
-  __shared__ float s_acc[G][W + 1];
+  __shared__ float s_m[NW], s_l[NW];
+  __shared__ float s_acc[NW][W];
   __shared__ int s_len[kRankBatch];
   __shared__ int s_b;
   const int tid = threadIdx.x;
   const int h = blockIdx.x;
   int b = blockIdx.y;
-  if (a.B <= kRankBatch && a.B > 1) {
+  if (a.nsplit == 1 && a.B <= kRankBatch && a.B > 1) {
     // batch index whose length ranks blockIdx.y-th (longest first, ties by index)
-    if (tid < a.B) s_len[tid] = min(a.kv_lens[tid], a.Sk);
+    for (int i = tid; i < a.B; i += NT) s_len[i] = min(a.kv_lens[i], a.Sk);
     __syncthreads();
-    if (tid < a.B) {
-      const int mine = s_len[tid];
+    for (int i = tid; i < a.B; i += NT) {
+      const int mine = s_len[i];
       int rank = 0;
       for (int j = 0; j < a.B; ++j) {
         const int lj = s_len[j];
-        rank += (lj > mine || (lj == mine && j < tid)) ? 1 : 0;
+        rank += (lj > mine || (lj == mine && j < i)) ? 1 : 0;
       }
-      if (rank == (int)blockIdx.y) s_b = tid;
+      if (rank == (int)blockIdx.y) s_b = i;
     }
     __syncthreads();
     b = s_b;
@@ -364,21 +386,30 @@ __global__ __launch_bounds__(BIG ? kStreamBlock : kBlock, 8) void decode_attn_ke
       compute_stage(kr[st], vr[st], k0 + st * STEP);
     }
   }
-  if (c == 0) { s_m[g] = m_run; s_l[g] = l_run; }
+  // the lane groups of a wave share one maximum, add up in registers, and the waves combine through LDS
+  const float m_w = across_groups<OpMax, LPK>(m_run);
+  const float scale_g = m_run > -INFINITY ? __builtin_amdgcn_exp2f(m_run - m_w) : 0.f;
+  l_run = across_groups<OpSum, LPK>(l_run * scale_g);
 #pragma unroll
-  for (int e = 0; e < EPV; ++e) s_acc[g][c * EPV + e] = acc[e];
-  __syncthreads();
-  float m_all = -INFINITY;
-  for (int j = 0; j < G; ++j) m_all = fmaxf(m_all, s_m[j]);
-  if (tid < G) s_w[tid] = s_m[tid] > -INFINITY ? __builtin_amdgcn_exp2f(s_m[tid] - m_all) : 0.f;
+  for (int e = 0; e < EPV; ++e) acc[e] = across_groups<OpSum, LPK>(acc[e] * scale_g);
+  const int lane = tid % kWave, wave = tid / kWave;
+  if (lane < LPK) {
+#pragma unroll
+    for (int e = 0; e < EPV; ++e) s_acc[wave][c * EPV + e] = acc[e];
+    if (lane == 0) { s_m[wave] = m_w; s_l[wave] = l_run; }
+  }
   __syncthreads();
   float *part = a.nsplit > 1 ? a.partial + (((int64_t)b * a.H + h) * a.nsplit + blockIdx.z) * (a.D + 2) : nullptr;
   for (int d = tid; d < a.D; d += NT) {
+    float m_all = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) m_all = fmaxf(m_all, s_m[w]);
     float l = 0.f, o = 0.f;
-#pragma unroll 4
-    for (int j = 0; j < G; ++j) {
-      l += s_l[j] * s_w[j];
-      o += s_acc[j][d] * s_w[j];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = s_m[w] > -INFINITY ? __builtin_amdgcn_exp2f(s_m[w] - m_all) : 0.f;
+      l += s_l[w] * f;
+      o += s_acc[w][d] * f;
     }
     if (part) {
       part[d] = o;
@@ -389,44 +420,89 @@ __global__ __launch_bounds__(BIG ? kStreamBlock : kBlock, 8) void decode_attn_ke
   }
 }
 
-// Combines the partial results of the workgroups that shared a unit's keys: one workgroup per (batch, head).
+// Combines the partial results of the workgroups that shared a unit's keys: one workgroup per (batch, head).  The
+// partials of kAhead shares are sent for together with the length that says how many of them were written (the
+// workspace holds nsplit of them whatever the length), so that one trip to memory is waited for instead of three.
 template <int DT>
 __global__ __launch_bounds__(kBlock) void decode_attn_combine_kernel(DecodeAttnArgs a) {
   typedef Elem<DT> E;
   typedef typename E::T T;
+  constexpr int kAhead = 8;
   const int unit = blockIdx.x, b = unit / a.H;
-  const int kl = max(min(a.kv_lens[b], a.Sk), 0);
-  const int share = split_share(kl, a.nsplit);
-  const int nvalid = share > 0 ? (kl + share - 1) / share : 0;       // shares that had keys
   const float *part = a.partial + (int64_t)unit * a.nsplit * (a.D + 2);
   T *ctx = reinterpret_cast<T *>(a.ctx) + (int64_t)unit * a.D;
-  float m_all = -INFINITY;
-  for (int z = 0; z < nvalid; ++z) m_all = fmaxf(m_all, part[z * (a.D + 2) + a.D]);
-  float l = 0.f;
-  for (int z = 0; z < nvalid; ++z) {
-    const float m = part[z * (a.D + 2) + a.D];
-    l += m > -INFINITY ? part[z * (a.D + 2) + a.D + 1] * __builtin_amdgcn_exp2f(m - m_all) : 0.f;
-  }
-  const float inv = l > 0.f ? 1.0f / l : 0.f;
   for (int d = threadIdx.x; d < a.D; d += kBlock) {
-    float o = 0.f;
-    for (int z = 0; z < nvalid; ++z) {
-      const float m = part[z * (a.D + 2) + a.D];
-      o += m > -INFINITY ? part[z * (a.D + 2) + d] * __builtin_amdgcn_exp2f(m - m_all) : 0.f;
+    float m_run = -INFINITY, l_run = 0.f, o_run = 0.f;
+    int nvalid = a.nsplit;
+    for (int z0 = 0; z0 < nvalid; z0 += kAhead) {
+      float m[kAhead], l[kAhead], o[kAhead];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const float *p = part + min(z0 + i, a.nsplit - 1) * (a.D + 2);
+        o[i] = p[d];
+        m[i] = p[a.D];
+        l[i] = p[a.D + 1];
+      }
+      if (z0 == 0) {
+        const int kl = max(min(a.kv_lens[b], a.Sk), 0);
+        const int share = split_share(kl, a.nsplit);
+        nvalid = share > 0 ? (kl + share - 1) / share : 0;       // shares that had keys
+      }
+      float m_new = m_run;
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        if (z0 + i >= nvalid) m[i] = -INFINITY;
+        m_new = fmaxf(m_new, m[i]);
+      }
+      if (m_new == -INFINITY) continue;
+      const float keep = __builtin_amdgcn_exp2f(m_run - m_new);        // exp2(-inf) = 0 before the first share
+      l_run *= keep;
+      o_run *= keep;
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        if (m[i] == -INFINITY) continue;                               // never written, or no key: whatever it holds stays out
+        const float f = __builtin_amdgcn_exp2f(m[i] - m_new);
+        l_run += l[i] * f;
+        o_run += o[i] * f;
+      }
+      m_run = m_new;
     }
-    ctx[d] = E::from_float(o * inv);
+    ctx[d] = E::from_float(l_run > 0.f ? o_run / l_run : 0.f);
   }
 }
 
-template <int DT, int LPK, bool PAGED = false> struct AttnLauncher {
-  // stream_cache: caches too large to stay in the memory-side cache between steps are read with non-temporal loads;
-  // big: 1024-lane workgroups (large caches, and whenever a unit's keys are split: few units, long rows)
-  static void go(const DecodeAttnArgs &a, dim3 grid, bool stream_cache, bool big, hipStream_t s) {
-    if (stream_cache) decode_attn_kernel<DT, LPK, true, true, PAGED><<<grid, kStreamBlock, 0, s>>>(a);
-    else if (big) decode_attn_kernel<DT, LPK, false, true, PAGED><<<grid, kStreamBlock, 0, s>>>(a);
-    else decode_attn_kernel<DT, LPK, false, false, PAGED><<<grid, kBlock, 0, s>>>(a);
+// Which form of the kernel a call runs (lanes per workgroup x keys per lane group and stage; all hold two stages):
+//   kSmall  256 x 2   the keys of a unit are shared between workgroups, or the caches are short: start-up and the
+//                     final combination count.  72 units of 1655 keys (61 MB), four shares each, without the combine
+//                     kernel: 13.2 us against 17.2 for 1024 x 1, 15.0 for 512 x 2; 96 units of ~70 keys 4.4 us.
+//   kDeep   512 x 4   enough units for the chip but not many rounds of them: more bytes in flight per workgroup.
+//                     640 units of 200..1000 keys 36.9 us (1024 x 1: 39.3, 256 x 4: 38.9), 768 units of 1..4000
+//                     keys 113.9 us (512 x 2: 116.1, 256 x 4: 116.0).
+//   kMany   256 x 4   many units, and few units on caches too short to share: 4608 units of 1..2048 keys (2.6 GB)
+//                     388 us, 6.8 TB/s (512 x 4: 396, 1024 x 1: 402); 72 units of 512 keys 7.9 us (256 x 2: 10.4).
+enum class AttnForm { kSmall, kDeep, kMany };
+
+static AttnForm attn_form(const DecodeAttnArgs &a) {
+  const int64_t units = (int64_t)a.B * a.H;
+  if (a.nsplit > 1) return AttnForm::kSmall;
+  if (units >= 512 && units < 2048) return AttnForm::kDeep;
+  return units < 512 && a.Sk <= 256 ? AttnForm::kSmall : AttnForm::kMany;
+}
+
+template <int DT, int LPK, bool PAGED, int NT, int U>
+static void launch_attn(const DecodeAttnArgs &a, dim3 grid, bool stream_cache, hipStream_t s) {
+  if (stream_cache) decode_attn_kernel<DT, LPK, NT, U, true, PAGED><<<grid, NT, 0, s>>>(a);
+  else decode_attn_kernel<DT, LPK, NT, U, false, PAGED><<<grid, NT, 0, s>>>(a);
+}
+
+template <int DT, int LPK, bool PAGED>
+static void launch_attn_form(const DecodeAttnArgs &a, dim3 grid, bool stream_cache, hipStream_t s) {
+  switch (attn_form(a)) {
+    case AttnForm::kSmall: launch_attn<DT, LPK, PAGED, 256, 2>(a, grid, stream_cache, s); break;
+    case AttnForm::kDeep: launch_attn<DT, LPK, PAGED, 512, 4>(a, grid, stream_cache, s); break;
+    default: launch_attn<DT, LPK, PAGED, 256, 4>(a, grid, stream_cache, s); break;
   }
-};
+}
 
 template <int DT, bool PAGED = false>
 static int dispatch_attn(const DecodeAttnArgs &a, bool stream_cache, hipStream_t s) {
@@ -434,13 +510,12 @@ static int dispatch_attn(const DecodeAttnArgs &a, bool stream_cache, hipStream_t
   int lpk = 4;
   while (lpk * EPV < a.D) lpk *= 2;
   dim3 grid((unsigned)a.H, (unsigned)a.B, (unsigned)a.nsplit);
-  const bool big = stream_cache || a.nsplit > 1;
   switch (lpk) {
-    case 4: AttnLauncher<DT, 4, PAGED>::go(a, grid, stream_cache, big, s); break;
-    case 8: AttnLauncher<DT, 8, PAGED>::go(a, grid, stream_cache, big, s); break;
-    case 16: AttnLauncher<DT, 16, PAGED>::go(a, grid, stream_cache, big, s); break;
-    case 32: AttnLauncher<DT, 32, PAGED>::go(a, grid, stream_cache, big, s); break;
-    case 64: AttnLauncher<DT, 64, PAGED>::go(a, grid, stream_cache, big, s); break;
+    case 4: launch_attn_form<DT, 4, PAGED>(a, grid, stream_cache, s); break;
+    case 8: launch_attn_form<DT, 8, PAGED>(a, grid, stream_cache, s); break;
+    case 16: launch_attn_form<DT, 16, PAGED>(a, grid, stream_cache, s); break;
+    case 32: launch_attn_form<DT, 32, PAGED>(a, grid, stream_cache, s); break;
+    case 64: launch_attn_form<DT, 64, PAGED>(a, grid, stream_cache, s); break;
     default: return EN_ERR_UNSUPPORTED;
   }
   EN_RETURN_IF_LAUNCH_FAILED();
@@ -451,9 +526,9 @@ static int dispatch_attn(const DecodeAttnArgs &a, bool stream_cache, hipStream_t
   return EN_OK;
 }
 
-// How many workgroups share one unit's keys: none while the units alone fill the chip's 512 slots of 1024 lanes;
-// else enough for about two slots' worth per CU, each share at least 512 keys long (shorter shares cost more in
-// workgroup start-up and in the combine pass than they win: 22 us instead of 25 for one sequence of 2048 keys).
+// How many workgroups share one unit's keys: none while the units alone fill the chip (512 units and more); else
+// enough for about four workgroups per CU, each share at least 512 keys long (shorter shares cost more in start-up
+// and in the combine pass than they win: 22 us instead of 25 for one sequence of 2048 keys).
 static int decode_split(int batch, int head_num, int k_seq_len) {
   constexpr int kTargetWorkgroups = 1024, kMinShare = 512;
   const int64_t units = (int64_t)batch * head_num;
@@ -639,7 +714,7 @@ int en_decode_attn(const void *q, const void *k_cache, const void *v_cache, void
   DecodeAttnArgs a{q, k_cache, v_cache, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
                    k_strides[2], v_strides[0], v_strides[1], v_strides[2], scale * 1.4426950408889634f,
                    split ? decode_split(batch, head_num, k_seq_len) : 1, static_cast<float *>(workspace)};
-  const bool stream_cache = 2 * cache_bytes(batch, head_num, k_seq_len, size_per_head, dtype) >= kStreamCacheBytes;
+  const bool stream_cache = 2 * cache_bytes(batch, head_num, k_seq_len, size_per_head, dtype) >= kAttnStreamBytes;
   hipStream_t s = (hipStream_t)stream;
   switch (dtype) {
     case EN_F32: return dispatch_attn<EN_F32>(a, stream_cache, s);
@@ -733,7 +808,7 @@ int en_decode_attn_paged(const void *q, const void *k_pool, const void *v_pool, 
                    k_strides[2], v_strides[0], v_strides[1], v_strides[2], scale * 1.4426950408889634f,
                    split ? decode_split(batch, head_num, k_seq_len) : 1, static_cast<float *>(workspace),
                    page_table, max_pages_per_seq, lg, num_pages};
-  const bool stream_cache = 2 * cache_bytes(batch, head_num, k_seq_len, size_per_head, dtype) >= kStreamCacheBytes;
+  const bool stream_cache = 2 * cache_bytes(batch, head_num, k_seq_len, size_per_head, dtype) >= kAttnStreamBytes;
   hipStream_t s = (hipStream_t)stream;
   switch (dtype) {
     case EN_F32: return dispatch_attn<EN_F32, true>(a, stream_cache, s);

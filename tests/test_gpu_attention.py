@@ -244,6 +244,36 @@ def test_decode_attn_single_pass(dtype, B, H, S, D, kv):
         assert bool((ws[need:] == 0xFF).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("B,H,S,D", [
+    (12, 3, 256, 64),       # 256 lanes x 2 keys: short caches
+    (12, 3, 257, 128),      # 256 lanes x 4 keys: few units, caches too short to share
+    (12, 43, 260, 96),      # 512 lanes x 4 keys: 516 units
+    (24, 86, 130, 32),      # 256 lanes x 4 keys: 2064 units
+    (12, 2, 1100, 80),      # shared keys: two shares per unit
+])
+def test_decode_attn_forms_at_the_edges_of_their_stages(dtype, B, H, S, D):
+    """Each form of the single-pass kernel with lengths around its lane groups, stages and shares."""
+    k = _kernel()
+    announce("decode attn forms", dtype, B, H, S, D)
+    g = torch.Generator().manual_seed(B * S + D)
+    edges = [0, 1, 15, 17, 63, 64, 65, 127, 129, S - 1, S, min(S, 255)]
+    kv = [min(n, S) for n in (edges * 2)[:B]]
+    q = torch.randn(B, H, 1, D, generator=g).to(dtype)
+    kc = torch.randn(B, H, S, D, generator=g).to(dtype)
+    vc = torch.randn(B, H, S, D, generator=g).to(dtype)
+    for b, n in enumerate(kv):
+        kc[b, :, n:] = float("nan")
+        vc[b, :, n:] = float("nan")
+    _, _, want = eager.decode_attention(q, torch.nan_to_num(kc, nan=0.0), torch.nan_to_num(vc, nan=0.0), kv, D ** -0.5,
+                                        acc_dtype=torch.float64)
+    for b, n in enumerate(kv):
+        if n == 0:
+            want[b] = 0
+    got = k.decode_attn(q.cuda(), kc.cuda(), vc.cuda(), torch.tensor(kv, dtype=torch.int32).cuda(), scale=D ** -0.5)
+    assert_ctx_close(got.cpu(), want, dtype, "decode_attn")
+
+
 def test_decode_attn_agrees_with_the_three_launch_route():
     """decode_qk -> scale_mask_softmax -> decode_pv store scores and probabilities in fp16 on the way; the single
     pass keeps them in fp32.  Both meet the bound against the oracle, so they agree within twice that bound."""
