@@ -26,10 +26,16 @@
 // K/V tiles travel from memory straight into LDS (bounds-checked loads that
 // write LDS): no registers hold a tile in flight and no instruction copies
 // one.  Rows keep their 16-byte chunks in XOR-swizzled slots so that both kinds
-// of fragment read are free of bank conflicts.  K has two buffers and is a tile
-// ahead; V has one buffer, is sent for at the top of its own tile and arrives
-// behind the score and softmax work: 48 KB of LDS per workgroup, so that three
+// of fragment read are free of bank conflicts.  Rows of up to 96 channels: K and V have two buffers each and are
+// a tile ahead, one barrier per tile (24 sequences of up to 384 keys, 16 heads x 64, non-causal, eight layers:
+// 274 -> 267 us against one V buffer; 48 KB of LDS at 96 channels is the same three workgroups per CU either way, and
+// a fourth one would need 128 registers: 28 bytes of scratch, 69 -> 88 us).  Rows of 128 channels: K has two buffers, V
+// one, sent for at the top of its own tile to arrive behind the score and softmax work: 48 KB of LDS, so that three
 // workgroups fit a CU.  The barriers order LDS only, as in the unfused kernels.
+//
+// Heads of 65..96 channels have rows of 12 slots of their own instead of the 128-channel form's 16: three quarters of
+// the tile loads and LDS, 22 (up to 80 channels) or 24 MFMAs per wave and tile instead of 32, and registers for the
+// second V buffer.  7 sequences of up to 1531 keys, 20 heads x 80, bf16: 80.2 -> 69.1 us.
 //
 // Everything that crosses the memory interface does so as whole rows: the K and
 // V tiles, the workgroup's Q rows (loaded straight into the buffers that are
@@ -42,8 +48,9 @@
 
 namespace en {
 
-template <int DT, int DP>
-__global__ __launch_bounds__(kBlock, 3) void attn_fused_kernel(FusedArgs fa) {
+// DP: channels of a row in LDS (the head size rounded up to 64, 96 or 128); NVS: MFMA steps of 16 channels that hold any.
+template <int DT, int DP, int NVS>
+__global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_kernel(FusedArgs fa) {
   static_assert(DT != EN_F32, "the fused kernel is built for 16-bit storage");
   typedef Elem<DT> E;
   typedef typename E::T T;
@@ -52,16 +59,20 @@ __global__ __launch_bounds__(kBlock, 3) void attn_fused_kernel(FusedArgs fa) {
   constexpr int EPV = 8;
   constexpr int BK = 64;                         // keys per tile
   constexpr int KB = BK / 32;                    // 32-key MFMA blocks per tile
-  constexpr int NVS = DP / 16;                   // MFMA steps over the head dim
   constexpr int DMT = DP / 32;                   // 32-channel MFMA tiles of the output
   constexpr int ROW = DP;                        // LDS pitch of a K or V row: tiles are written by direct loads, unpadded
   constexpr int KVEC_ROW = DP / EPV;             // 16-byte slots per row
   constexpr int KLOADS = BK * KVEC_ROW / kBlock; // direct-load instructions per wave and tile, for each of K and V
   constexpr float kLog2e = 1.4426950408889634f;
-  static_assert(DP == 64 || DP == 128, "swizzles are written for 8 or 16 slots per row");
-  static_assert(BK * KVEC_ROW % kBlock == 0, "tiles must divide over the block");
+  constexpr int NVB = DP <= 96 ? 2 : 1;          // V buffers
+  static_assert(DP == 64 || DP == 96 || DP == 128, "swizzles are written for 8, 12 or 16 slots per row");
+  static_assert(NVS * 16 <= DP, "a step reads channels the tile has");
+  static_assert(BK * KVEC_ROW % kBlock == 0 && 32 * KVEC_ROW % kWave == 0, "tiles must divide over the block");
   __shared__ __attribute__((aligned(16))) T lds_k[2][BK * ROW];
-  __shared__ __attribute__((aligned(16))) T lds_v[BK * ROW];
+  __shared__ __attribute__((aligned(16))) T lds_v[NVB][BK * ROW];
+  // chunk held by slot c of row r: c ^ kswz(r) in a K tile (and in the staged Q rows), c ^ vswz(r) in a V tile
+  auto kswz = [](int row) { return DP == 128 ? (row & 15) : DP == 96 ? ((row >> 2) & 3) : ((row >> 1) & 7); };
+  auto vswz = [](int row) { return DP == 128 ? 4 * (row & 3) : DP == 96 ? 0 : 4 * ((row >> 1) & 1); };
 
   int unit, qi;
   if (!map_block(a, unit, qi)) return;
@@ -104,15 +115,13 @@ __global__ __launch_bounds__(kBlock, 3) void attn_fused_kernel(FusedArgs fa) {
   // each lane then reads its own row's chunks: sixteen-byte pieces fetched by every lane from a row of its own
   // kept the address unit busy with 32 rows per instruction.
   uint4 qf[NVS];
-  T *q_stage = (wave < 2 ? lds_k[1] : lds_v) + (wave & 1) * 32 * ROW;
+  T *q_stage = (wave < 2 ? lds_k[1] : lds_v[NVB - 1]) + (wave & 1) * 32 * ROW;
   {
     const desc_t q_desc = make_desc(qbase, (uint32_t)(((int64_t)(ql - 1) * a.q_ss + a.D) * E::kSize));
-    constexpr int RPLQ = kWave / KVEC_ROW;         // rows one direct load of a wave covers
-    const int row = lane / KVEC_ROW, slot = lane % KVEC_ROW;
 #pragma unroll
-    for (int n = 0; n < 32 / RPLQ; ++n) {
-      const int rr = n * RPLQ + row;               // row of the wave's 32
-      const int c = slot ^ (DP == 128 ? (rr & 15) : ((rr >> 1) & 7));
+    for (int n = 0; n < 32 * KVEC_ROW / kWave; ++n) {
+      const int rr = (n * kWave + lane) / KVEC_ROW, slot = (n * kWave + lane) % KVEC_ROW;   // row of the wave's 32
+      const int c = slot ^ kswz(rr);
       const int qq = q0 + wave * 32 + rr;
       const uint32_t off = (uint32_t)(((int64_t)qq * a.q_ss + c * EPV) * E::kSize);
       buffer_load16_to_lds(q_desc, lds_address(q_stage) + n * kWave * 16, ((unsigned)qq < (unsigned)ql && c * EPV < a.D) ? off : kOutOfRange);
@@ -121,45 +130,47 @@ __global__ __launch_bounds__(kBlock, 3) void attn_fused_kernel(FusedArgs fa) {
 
   // K / V tiles: the descriptors end with the last valid key, so rows past it (and whole tiles past the last
   // one) arrive as zeros with no traffic and no branches.  One direct load of a wave fills 1 KB of LDS, lane i
-  // the 16 bytes at 16 i: that is slot i % KVEC_ROW of tile row (64 / KVEC_ROW) * (4 n + wave) + i / KVEC_ROW
-  // for the wave's n-th load.  Which 16-byte chunk of the row a slot holds is the lane's choice of offset:
-  //   K: slot c of row r holds chunk c ^ kswz(r), kswz = r & 15 (16 slots) or (r >> 1) & 7 (8 slots): the
-  //      128-bit fragment reads of 16 consecutive rows at one chunk then cover all 64 banks once;
-  //   V: slot c of key k holds chunk c ^ vswz(k), vswz = 4 (k & 3) (16 slots) or 4 ((k >> 1) & 1) (8 slots):
-  //      a transposing read takes 64 bytes from each of four consecutive keys, which the swizzle spreads over
-  //      the four quarters of the banks.
-  // Both swizzles depend on the row only through bits the lane's position fixes, so each lane keeps one byte
-  // offset per operand and advances it by a tile per load; lanes whose chunk lies past the head size sit at an
-  // offset that stays out of range.
+  // the 16 bytes at 16 i: the tile's slots in order, 64 of them from slot 256 n + 64 wave on for the wave's n-th load.
+  // Which 16-byte chunk of the row a slot holds is the lane's choice of offset:
+  //   K: slot c of row r holds chunk c ^ kswz(r), kswz = r & 15 (16 slots), (r >> 2) & 3 (12 slots: rows lie 48 banks
+  //      apart, so every fourth row starts at the same bank) or (r >> 1) & 7 (8 slots): the 128-bit fragment reads of
+  //      16 consecutive rows at one chunk then cover all 64 banks once;
+  //   V: slot c of key k holds chunk c ^ vswz(k), vswz = 4 (k & 3) (16 slots), 0 (12 slots) or 4 ((k >> 1) & 1)
+  //      (8 slots): a transposing read takes 64 bytes from each of four consecutive keys, which the swizzle (with 12
+  //      slots the pitch itself) spreads over the four quarters of the banks.
+  // With 8 and 16 slots both swizzles depend on the row only through bits the lane's position fixes, so each lane keeps
+  // one byte offset per operand and advances it by a tile per load; 12 slots do not divide the 256 lanes, and each load
+  // of a tile has an offset of its own.  Lanes whose chunk lies past the head size sit at an offset that stays out of range.
   const uint32_t k_bytes = kl > 0 ? (uint32_t)(((int64_t)(kl - 1) * a.k_ss + a.D) * E::kSize) : 0u;
   const uint32_t v_bytes = kl > 0 ? (uint32_t)(((int64_t)(kl - 1) * fa.v_ss + a.D) * E::kSize) : 0u;
   const desc_t k_desc = make_desc(kbase, k_bytes);
   const desc_t v_desc = make_desc(vbase, v_bytes);
   const uint32_t k_row_bytes = (uint32_t)(a.k_ss * E::kSize), v_row_bytes = (uint32_t)(fa.v_ss * E::kSize);
-  constexpr int RPL = kWave / KVEC_ROW;          // rows one direct load of a wave covers
-  const int ld_row = wave * RPL + lane / KVEC_ROW, ld_slot = lane % KVEC_ROW;
-  const int k_c = ld_slot ^ (DP == 128 ? (ld_row & 15) : ((ld_row >> 1) & 7));
-  const int v_c = ld_slot ^ (DP == 128 ? 4 * (ld_row & 3) : 4 * ((ld_row >> 1) & 1));
-  uint32_t k_off = (k_c * EPV < a.D) ? ld_row * k_row_bytes + k_c * EPV * E::kSize : kOutOfRange;
-  uint32_t v_off = (v_c * EPV < a.D) ? ld_row * v_row_bytes + v_c * EPV * E::kSize : kOutOfRange;
-  auto fetch_k = [&](T *kdst) {
-    const uint32_t k_lds = lds_address(kdst) + wave * kWave * 16;
+  constexpr int NOFF = DP == 96 ? KLOADS : 1;
+  uint32_t k_off[NOFF], v_off[NOFF];
 #pragma unroll
-    for (int i = 0; i < KLOADS; ++i) buffer_load16_to_lds(k_desc, k_lds + i * kBlock * 16, k_off + i * (kBlock / KVEC_ROW) * k_row_bytes);
-    k_off += BK * k_row_bytes;
-  };
-  auto fetch_v = [&]() {
-    const uint32_t v_lds = lds_address(lds_v) + wave * kWave * 16;
+  for (int i = 0; i < NOFF; ++i) {
+    const int row = (i * kBlock + tid) / KVEC_ROW, slot = (i * kBlock + tid) % KVEC_ROW;
+    const int k_c = slot ^ kswz(row), v_c = slot ^ vswz(row);
+    k_off[i] = (k_c * EPV < a.D) ? row * k_row_bytes + k_c * EPV * E::kSize : kOutOfRange;
+    v_off[i] = (v_c * EPV < a.D) ? row * v_row_bytes + v_c * EPV * E::kSize : kOutOfRange;
+  }
+  auto fetch_tile = [&](const desc_t &desc, T *dst, uint32_t (&off)[NOFF], uint32_t row_bytes) {
+    const uint32_t lds = lds_address(dst) + wave * kWave * 16;
 #pragma unroll
-    for (int i = 0; i < KLOADS; ++i) buffer_load16_to_lds(v_desc, v_lds + i * kBlock * 16, v_off + i * (kBlock / KVEC_ROW) * v_row_bytes);
-    v_off += BK * v_row_bytes;
+    for (int i = 0; i < KLOADS; ++i)
+      buffer_load16_to_lds(desc, lds + i * kBlock * 16, NOFF > 1 ? off[i % NOFF] : off[0] + i * (kBlock / KVEC_ROW) * row_bytes);
+#pragma unroll
+    for (int i = 0; i < NOFF; ++i) off[i] += BK * row_bytes;
   };
+  auto fetch_k = [&](T *dst) { fetch_tile(k_desc, dst, k_off, k_row_bytes); };
+  auto fetch_v = [&](T *dst) { fetch_tile(v_desc, dst, v_off, v_row_bytes); };
   // fragment addresses.  K: row 32 kb + r, chunk 2 vs + g.  V (transposing read): lane j of a 16-lane group
   // points at key j / 4 of the group's four keys and at channels 4 (j % 4) .. + 3 of the group's sixteen; the
   // read hands lane i of the group channel i of those sixteen at the four keys.
-  const int ksw = DP == 128 ? (r & 15) : ((r >> 1) & 7);
+  const int ksw = kswz(r);
   const int tj = lane & 15, tg = (lane >> 4) & 1;     // position in the 16-lane group; which half of a 32-channel tile
-  const int vsw = DP == 128 ? (tj >> 2) : ((tj >> 3) & 1);
+  const int vsw = vswz(tj >> 2) / 4;
   uint32_t v_frag[DMT];                                // byte offset of this lane's read for channel tile mt, keys 4g + 0..3
 #pragma unroll
   for (int mt = 0; mt < DMT; ++mt)
@@ -178,24 +189,31 @@ __global__ __launch_bounds__(kBlock, 3) void attn_fused_kernel(FusedArgs fa) {
   // range, and the final division by the row sum cancels the common factor.
   const float lazy_gap = 8.0f / c_exp;
 
-  // K tile kt is read out of buffer kt & 1 while K tile kt + 1 travels into the other one; V tile kt is sent for
-  // at the top of iteration kt (its buffer was in use until the barrier that ended iteration kt - 1) and waited
-  // for between the softmax and the second contraction.  Two barriers per tile.
+  // K tile kt is read out of buffer kt & 1 while K tile kt + 1 travels into the other one.  Two V buffers: V goes the
+  // same way, one barrier per tile.  One V buffer: V tile kt is sent for at the top of iteration kt (its buffer was in use
+  // until the barrier that ended iteration kt - 1) and waited for between the softmax and the second contraction, two
+  // barriers per tile.
   fetch_k(lds_k[0]);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  {  // the wave's own rows have landed; the barrier below also keeps the tiles of the key loop off them until all have read
-    const int qsw = DP == 128 ? (r & 15) : ((r >> 1) & 7);
+  if constexpr (NVB == 2) fetch_v(lds_v[0]);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NVB == 2 ? 2 : 1) * KLOADS) : "memory");
+  // the wave's own Q rows have landed; the barrier below keeps the tiles of the key loop off them until all have read
 #pragma unroll
-    for (int vs = 0; vs < NVS; ++vs)
-      qf[vs] = *reinterpret_cast<const uint4 *>(&q_stage[r * ROW + (((2 * vs + g) ^ qsw) * EPV)]);
-  }
+  for (int vs = 0; vs < NVS; ++vs)
+    qf[vs] = *reinterpret_cast<const uint4 *>(&q_stage[r * ROW + (((2 * vs + g) ^ ksw) * EPV)]);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVB == 2 ? KLOADS : 0) : "memory");
   lds_barrier();
 
   for (int kt = 0; kt < nkt; ++kt) {
     const int k0 = kt * BK;
     const T *ksrc = lds_k[kt & 1];
-    fetch_v();                                   // V tile kt
-    fetch_k(lds_k[(kt + 1) & 1]);                // K tile kt + 1 (past the end: out of range, zeros, no traffic)
+    const T *vsrc = lds_v[NVB == 2 ? kt & 1 : 0];
+    if constexpr (NVB == 2) {
+      fetch_k(lds_k[(kt + 1) & 1]);              // tiles kt + 1 (past the end: out of range, zeros, no traffic)
+      fetch_v(lds_v[(kt + 1) & 1]);
+    } else {
+      fetch_v(lds_v[0]);                         // V tile kt
+      fetch_k(lds_k[(kt + 1) & 1]);              // K tile kt + 1
+    }
     uint4 pf[KB * 2];                            // B operands of the second MFMA: the probabilities of this tile
     const bool live = k0 < vis_max;              // wave-uniform: later tiles are masked for all of this wave's queries
 
@@ -284,10 +302,15 @@ __global__ __launch_bounds__(kBlock, 3) void attn_fused_kernel(FusedArgs fa) {
 
     }
 
-    // V tile kt was sent for before K tile kt + 1 and the loads complete in order: it has landed once only the
-    // K loads are outstanding; the barrier publishes every wave's share
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(KLOADS) : "memory");
-    lds_barrier();
+    // One V buffer: V tile kt was sent for before K tile kt + 1 and the loads complete in order: it has landed once only
+    // the K loads are outstanding; the barrier publishes every wave's share
+    if constexpr (NVB == 1) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(KLOADS) : "memory");
+      lds_barrier();
+    } else if (kt == 0) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * KLOADS) : "memory");
+      lds_barrier();
+    }
 
     if (live) {
       // ---- O^T += V^T P^T; the A operand reads V at the keys the B registers hold:
@@ -295,7 +318,7 @@ __global__ __launch_bounds__(kBlock, 3) void attn_fused_kernel(FusedArgs fa) {
       constexpr int NG = KB * 2;                      // groups of 16 keys
       uint4 va[2][DMT];
       auto load_group = [&](int gi, uint4 (&dst)[DMT]) {
-        const char *vt = reinterpret_cast<const char *>(lds_v) + gi * 16 * ROW * E::kSize;
+        const char *vt = reinterpret_cast<const char *>(vsrc) + gi * 16 * ROW * E::kSize;
 #pragma unroll
         for (int mt = 0; mt < DMT; ++mt) {
           const uint2 lo = lds_read_tr16(vt + v_frag[mt]);                          // keys 16 gi + 4 g + 0..3
@@ -314,8 +337,8 @@ __global__ __launch_bounds__(kBlock, 3) void attn_fused_kernel(FusedArgs fa) {
       }
     }
 
-    // K tile kt + 1 has landed once none of this wave's loads is outstanding; the barrier publishes it and
-    // frees the V buffer and the other K buffer
+    // The next tiles have landed once none of this wave's loads is outstanding; the barrier publishes them and
+    // frees the buffers of this one
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();
   }
@@ -326,8 +349,9 @@ __global__ __launch_bounds__(kBlock, 3) void attn_fused_kernel(FusedArgs fa) {
   if (fa.c_vec16) {
     // A lane holds 8-byte pieces of its own row, 32 rows per store instruction; through LDS (the K buffers are free
     // behind the loop's last barrier, each wave takes the 32 rows' worth that is its own, so no barrier is needed)
-    // the wave's tile leaves as whole rows: 16 bytes per lane, 64 / KVEC_ROW rows per instruction.  Chunk c of row r
-    // sits in slot c ^ (r % KVEC_ROW): writes and reads both spread over all banks.
+    // the wave's tile leaves as whole rows: 16 bytes per lane, four to eight rows per instruction.  Chunk c of row r
+    // sits in slot c ^ oswz(r): writes and reads both spread over all banks.
+    auto oswz = [](int row) { return DP == 96 ? (row >> 2) & 3 : row & (KVEC_ROW - 1); };
     char *stage = reinterpret_cast<char *>(&lds_k[0][0]) + wave * 32 * ROW * E::kSize;
 #pragma unroll
     for (int mt = 0; mt < DMT; ++mt)
@@ -337,14 +361,13 @@ __global__ __launch_bounds__(kBlock, 3) void attn_fused_kernel(FusedArgs fa) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) pk.v[i] = E::from_float(o[mt][4 * j + i] * inv);
         const int c = 4 * mt + j;
-        *reinterpret_cast<Pack<T, 4> *>(stage + r_e * ROW * E::kSize + ((c ^ (r_e & (KVEC_ROW - 1))) * 16) + g_e * 8) = pk;
+        *reinterpret_cast<Pack<T, 4> *>(stage + r_e * ROW * E::kSize + ((c ^ oswz(r_e)) * 16) + g_e * 8) = pk;
       }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own writes, before its lanes read each other's
-    constexpr int RPI = kWave / KVEC_ROW;              // rows per store instruction
 #pragma unroll
-    for (int i = 0; i < 32 / RPI; ++i) {
-      const int row = i * RPI + lane_e / KVEC_ROW, c = lane_e % KVEC_ROW;
-      const uint4 v = *reinterpret_cast<const uint4 *>(stage + row * ROW * E::kSize + ((c ^ (row & (KVEC_ROW - 1))) * 16));
+    for (int i = 0; i < 32 * KVEC_ROW / kWave; ++i) {
+      const int row = (i * kWave + lane_e) / KVEC_ROW, c = (i * kWave + lane_e) % KVEC_ROW;
+      const uint4 v = *reinterpret_cast<const uint4 *>(stage + row * ROW * E::kSize + ((c ^ oswz(row)) * 16));
       const int qrow = q0 + wave * 32 + row;
       if ((unsigned)qrow < (unsigned)ql && c * EPV < a.D) *reinterpret_cast<uint4 *>(cbase + (int64_t)qrow * fa.c_ss + c * EPV) = v;
     }
@@ -371,8 +394,10 @@ template <int DT>
 static int launch_fused(FusedArgs &fa, hipStream_t s) {
   const AttnArgs &a = fa.base;
   const unsigned grid = (unsigned)(ceil_div(a.units, kXcds) * kXcds * a.ntq);
-  if (a.D <= 64) attn_fused_kernel<DT, 64><<<grid, kBlock, 0, s>>>(fa);
-  else attn_fused_kernel<DT, 128><<<grid, kBlock, 0, s>>>(fa);
+  if (a.D <= 64) attn_fused_kernel<DT, 64, 4><<<grid, kBlock, 0, s>>>(fa);
+  else if (a.D <= 80) attn_fused_kernel<DT, 96, 5><<<grid, kBlock, 0, s>>>(fa);
+  else if (a.D <= 96) attn_fused_kernel<DT, 96, 6><<<grid, kBlock, 0, s>>>(fa);
+  else attn_fused_kernel<DT, 128, 8><<<grid, kBlock, 0, s>>>(fa);
   EN_RETURN_IF_LAUNCH_FAILED();
   return EN_OK;
 }

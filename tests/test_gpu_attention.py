@@ -397,6 +397,18 @@ def test_attn_fused_packed(dtype, causal, B, H, S, D, lens):
     assert bool((g[0] == sentinel).all()) and bool((g[T + 1] == sentinel).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [64, 72, 80, 88, 96, 104])
+def test_attn_fused_head_sizes_between_the_tile_widths(dtype, D):
+    """Heads on either side of the 64-, 96- and 128-channel forms (72 and 80: five MFMA steps of a 96-channel row), with
+    lengths around the query and key tiles; the output 16-byte aligned and not."""
+    B, H, S = 9, 3, 260
+    lens = [260, 1, 63, 64, 65, 127, 128, 129, 193]
+    test_attn_fused_packed(dtype, True, B, H, S, D, lens)
+    test_attn_fused_packed(dtype, False, B, H, S, D, lens)
+    test_attn_fused_and_pv_write_an_output_that_is_not_16_byte_aligned(D)
+
+
 @pytest.mark.parametrize("slope", [0.002, 0.02, 0.3])
 def test_attn_fused_growing_maximum(slope):
     """Scores that rise with the key index: the running maximum keeps moving, slowly (the kernel
