@@ -28,13 +28,17 @@ struct LnArgs {
   float eps;
 };
 
-template <int DTI, int DTO, int VPL, int TPR, bool STREAM, bool STREAM_LD = false>
-__global__ __launch_bounds__(TPR < kBlock ? kBlock : TPR) void layernorm_rows_kernel(LnArgs a) {
+// One wave per row: four rows share a workgroup and no barrier; else a workgroup is a row.
+constexpr int rows_block(int tpr) { return tpr == kWave ? kBlock : tpr; }
+
+// STREAM: the tensors are too large for the memory-side cache and pass by it with non-temporal accesses.
+template <int DTI, int DTO, int VPL, int TPR, bool STREAM>
+__global__ __launch_bounds__(rows_block(TPR)) void layernorm_rows_kernel(LnArgs a) {
   typedef Elem<DTI> EI;
   typedef Elem<DTO> EO;
   typedef typename EI::T TI;
   typedef typename EO::T TO;
-  constexpr int BLOCK = TPR < kBlock ? kBlock : TPR;
+  constexpr int BLOCK = rows_block(TPR);
   constexpr int EPV = 16 / EI::kSize;  // elements per 128-bit input vector
   constexpr int NW = TPR / kWave;      // waves sharing a row
   constexpr int ROWS_PER_BLOCK = BLOCK / TPR;
@@ -50,15 +54,40 @@ __global__ __launch_bounds__(TPR < kBlock ? kBlock : TPR) void layernorm_rows_ke
   const TI *in = reinterpret_cast<const TI *>(a.in) + row * a.n2;
   TI *sum_out = a.sum_out ? reinterpret_cast<TI *>(a.sum_out) + row * a.n2 : nullptr;
 
-  // The row's own loads go out first: where the residual row is found through res_off, its address hangs on a
-  // load of its own, and loads issue in order -- placed first it would hold the others back for its whole latency.
-  uint4 raw[VPL];
+  // Rows that come out of a cache are bound by the length of their chain, so everything they need is sent for before the
+  // first reduction waits for anything: gamma and beta behind the reductions would be a second trip (in a layer, 8300
+  // rows of 768 fp16 9.3 -> 8.6 us, 5000 rows of 1024 bf16 7.9 -> 7.4 us; alone, 64 rows of 9216 4.5 -> 3.9 us).  Rows
+  // streamed from memory are bound by what is in flight, and the registers that hold gamma and beta cost waves: there
+  // they are loaded where they are used (14213 rows of 12288 fp16 166 us against 180; 9304 of 7168 67 against 70).
+  // The row's own loads go out first: where the residual row is found through res_off, its address hangs on a load of
+  // its own.
+  constexpr bool EARLY = VPL <= 4 && !STREAM;
+  uint4 raw[VPL], rraw[VPL];
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
     const int v = t + TPR * j;
-    raw[j] = (v < nvec) ? load16<STREAM_LD>(in + v * EPV) : make_uint4(0u, 0u, 0u, 0u);
+    raw[j] = (v < nvec) ? load16<STREAM>(in + v * EPV) : make_uint4(0u, 0u, 0u, 0u);
   }
+  const TO *gamma = reinterpret_cast<const TO *>(a.gamma);
+  const TO *beta = reinterpret_cast<const TO *>(a.beta);
+  Pack<TO, EPV> g[VPL], bt[VPL];
+  auto load_affine = [&]() {
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      const int v = min(t + TPR * j, nvec - 1);
+      g[j] = load_pack<TO, EPV>(gamma + v * EPV);
+      bt[j] = load_pack<TO, EPV>(beta + v * EPV);
+    }
+  };
   const TI *res = a.residual ? reinterpret_cast<const TI *>(a.residual) + (row + (a.res_off ? a.res_off[row] : 0)) * a.n2 : nullptr;
+  if constexpr (EARLY) load_affine();
+  if (res) {
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      const int v = t + TPR * j;
+      rraw[j] = (v < nvec) ? load16<STREAM>(res + v * EPV) : make_uint4(0u, 0u, 0u, 0u);
+    }
+  }
 
   float x[VPL][EPV];
   float s = 0.f;
@@ -70,7 +99,7 @@ __global__ __launch_bounds__(TPR < kBlock ? kBlock : TPR) void layernorm_rows_ke
 #pragma unroll
       for (int e = 0; e < EPV; ++e) x[j][e] = EI::to_float(pk.v[e]);
       if (res) {
-        const Pack<TI, EPV> rk = __builtin_bit_cast(Pack<TI, EPV>, load16<STREAM_LD>(res + v * EPV));
+        const Pack<TI, EPV> rk = __builtin_bit_cast(Pack<TI, EPV>, rraw[j]);
 #pragma unroll
         for (int e = 0; e < EPV; ++e) x[j][e] += EI::to_float(rk.v[e]);
       }
@@ -105,19 +134,16 @@ __global__ __launch_bounds__(TPR < kBlock ? kBlock : TPR) void layernorm_rows_ke
   const float var = d2 / (float)a.n2;
   const float inv = 1.0f / sqrtf(var + a.eps);
 
-  const TO *gamma = reinterpret_cast<const TO *>(a.gamma);
-  const TO *beta = reinterpret_cast<const TO *>(a.beta);
+  if constexpr (!EARLY) load_affine();
   TO *out = reinterpret_cast<TO *>(a.out) + row * a.n2;
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
     const int v = t + TPR * j;
     if (v < nvec) {
-      const Pack<TO, EPV> g = load_pack<TO, EPV>(gamma + v * EPV);
-      const Pack<TO, EPV> bt = load_pack<TO, EPV>(beta + v * EPV);
       Pack<TO, EPV> o;
 #pragma unroll
       for (int e = 0; e < EPV; ++e)
-        o.v[e] = EO::from_float((x[j][e] - mu) * inv * EO::to_float(g.v[e]) + EO::to_float(bt.v[e]));
+        o.v[e] = EO::from_float((x[j][e] - mu) * inv * EO::to_float(g[j].v[e]) + EO::to_float(bt[j].v[e]));
       if constexpr (sizeof(TO) * EPV == 16) store16<STREAM>(out + v * EPV, __builtin_bit_cast(uint4, o));
       else store_pack<TO, EPV>(out + v * EPV, o);
     }
@@ -174,27 +200,26 @@ __global__ __launch_bounds__(kBlock) void layernorm_generic_kernel(LnArgs a) {
 
 template <int DTI, int DTO, int VPL, int TPR>
 static void launch_rows(const LnArgs &a, hipStream_t s) {
-  constexpr int BLOCK = TPR < kBlock ? kBlock : TPR;
+  constexpr int BLOCK = rows_block(TPR);
   constexpr int ROWS_PER_BLOCK = BLOCK / TPR;
   const unsigned grid = (unsigned)ceil_div(a.n1, ROWS_PER_BLOCK);
-  // outputs too large to stay in the memory-side cache are written with non-temporal stores
-  // and inputs too large to have stayed there are read with non-temporal loads
+  // From this size on neither the inputs are still in the memory-side cache in full nor does the output stay there, and all
+  // of them go by it (in a layer: 14213 rows of 12288 fp16 with cached loads 180 us, non-temporal 166; 9304 rows of 7168,
+  // whose input the attention has just written, 68.2 against 67.2).
   const int64_t bytes = a.n1 * a.n2 * Elem<DTO>::kSize;
-  if (bytes >= kStreamLoadBytes) layernorm_rows_kernel<DTI, DTO, VPL, TPR, true, true><<<grid, BLOCK, 0, s>>>(a);
-  else if (bytes >= kStreamStoreBytes) layernorm_rows_kernel<DTI, DTO, VPL, TPR, true><<<grid, BLOCK, 0, s>>>(a);
+  if (bytes >= kStreamStoreBytes) layernorm_rows_kernel<DTI, DTO, VPL, TPR, true><<<grid, BLOCK, 0, s>>>(a);
   else layernorm_rows_kernel<DTI, DTO, VPL, TPR, false><<<grid, BLOCK, 0, s>>>(a);
 }
 
-template <int DTI, int DTO, int TPR>
-static bool launch_vpl(const LnArgs &a, int vpl, hipStream_t s) {
-  if (vpl <= 1) launch_rows<DTI, DTO, 1, TPR>(a, s);
-  else if (vpl <= 2) launch_rows<DTI, DTO, 2, TPR>(a, s);
-  else if (vpl <= 3) launch_rows<DTI, DTO, 3, TPR>(a, s);
-  else if (vpl <= 4) launch_rows<DTI, DTO, 4, TPR>(a, s);
-  else if (vpl <= 6) launch_rows<DTI, DTO, 6, TPR>(a, s);
-  else if (vpl <= 8) launch_rows<DTI, DTO, 8, TPR>(a, s);
-  else return false;
-  return true;
+// Launches the instance with the fewest of VPLS vectors per lane that cover the row.
+template <int DTI, int DTO, int TPR, int VPL, int... MORE>
+static bool launch_vpl(const LnArgs &a, int nvec, hipStream_t s) {
+  if (nvec <= VPL * TPR) {
+    launch_rows<DTI, DTO, VPL, TPR>(a, s);
+    return true;
+  }
+  if constexpr (sizeof...(MORE) > 0) return launch_vpl<DTI, DTO, TPR, MORE...>(a, nvec, s);
+  return false;
 }
 
 template <int DTI, int DTO>
@@ -208,16 +233,15 @@ static int dispatch(const LnArgs &a, hipStream_t s) {
   const int nvec = vec_ok ? a.n2 / EPV : 0;
   bool done = false;
   if (vec_ok) {
-    if (nvec <= 2 * 64) done = launch_vpl<DTI, DTO, 64>(a, (nvec + 63) / 64, s);
-    // at most four vectors per lane while the row fits 512 lanes: rows of 1025..2048 vectors measured 288 us
-    // with 256 lanes x 6 vectors against 267 us with 512 lanes x 3 (20142 rows of 12288 fp16, residual added)
-    // rows that would put four vectors on each of 256 lanes go to 512 lanes x 2 when there are many of them:
-    // 7168-wide fp16 rows (896 vectors) x 9244: 60.6 -> 58.8 us, 8192-wide x 32768: 264 -> 256 us; with fewer
-    // vectors (5120-wide: 48 -> 52 us) or few rows (2048 rows: 15.4 -> 16.3 us) 256 lanes stay ahead
-    else if (nvec > 3 * 256 && nvec <= 4 * 256 && a.n1 >= 4096) done = launch_vpl<DTI, DTO, 512>(a, 2, s);
-    else if (nvec <= 4 * 256) done = launch_vpl<DTI, DTO, 256>(a, (nvec + 255) / 256, s);
-    else if (nvec <= 4 * 512) done = launch_vpl<DTI, DTO, 512>(a, (nvec + 511) / 512, s);
-    else if (nvec <= 8 * 1024) done = launch_vpl<DTI, DTO, 1024>(a, (nvec + 1023) / 1024, s);
+    // Lanes per row, measured for widths of 768..12288 fp16 (96..1536 vectors) at a few hundred and at thousands of rows:
+    // one wave per row (no barrier) up to three vectors per lane (1536-wide x 6000: 9.7 us, 128 x 2 10.4, 256 x 1 11.0;
+    // 1600-wide x 5400: 64 x 4 13.9, 128 x 2 12.8); then two vectors per lane on 128 lanes, three where they fit
+    // (3072-wide x 4000: 128 x 3 12.4, 256 x 2 13.0; 4096-wide: 128 x 4 18.1, 256 x 2 18.1, and 3.8 against 3.7 at 300 rows),
+    // 256 lanes up to three (5120-wide x 3000: 17.4, 512 x 2 18.0), 512 up to four (7168-wide x 3000: 512 x 2 26.3, 256 x 4
+    // 26.8; 12288-wide x 12410: 512 x 3 152.7, 256 x 6 157.6, 1024 x 2 153.3)
+    done = launch_vpl<DTI, DTO, 64, 1, 2, 3>(a, nvec, s) || launch_vpl<DTI, DTO, 128, 2, 3>(a, nvec, s) ||
+           launch_vpl<DTI, DTO, 256, 2, 3>(a, nvec, s) || launch_vpl<DTI, DTO, 512, 2, 3, 4>(a, nvec, s) ||
+           launch_vpl<DTI, DTO, 1024, 3, 4, 6, 8>(a, nvec, s);
   }
   if (!done) layernorm_generic_kernel<DTI, DTO><<<(unsigned)a.n1, kBlock, 0, s>>>(a);
   EN_RETURN_IF_LAUNCH_FAILED();

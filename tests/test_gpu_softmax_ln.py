@@ -231,3 +231,27 @@ def test_softmax_tiled_tail(dtype, causal, tile, scale):
             assert bool((tiled[b, :, q0:q0 + rows, lim:lim_v] == 0).all())
             assert torch.equal(tiled[b, :, q0:q0 + rows, lim_v:], src[b, :, q0:q0 + rows, lim_v:])
         assert torch.equal(tiled[b, :, n:], src[b, :, n:])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("vectors", [1, 64, 65, 128, 129, 192, 193, 256, 257, 384, 385, 512, 513, 768, 769, 1024, 1025, 1536,
+                                     1537, 2048, 2049, 3073, 4097, 6145, 8192, 8193])
+def test_layernorm_at_the_edges_of_its_lane_configurations(dtype, vectors):
+    """Row widths on either side of every lanes x vectors instance, with residual, row offsets, sum and statistics; the
+    reference is LayerNorm in float64 and the bound the module's: BASE plus half an ulp of the stored value."""
+    from energonai_amd import kernel as K
+    epv = 16 // torch.empty(0, dtype=dtype).element_size()
+    width, rows = vectors * epv, 7
+    announce("layernorm lane edges", dtype, width)
+    g = torch.Generator().manual_seed(vectors)
+    x, res = torch.randn(rows, width, generator=g).to(dtype), torch.randn(rows + 5, width, generator=g).to(dtype)
+    gamma, beta = (1 + 0.02 * torch.randn(width, generator=g)).to(dtype), (0.02 * torch.randn(width, generator=g)).to(dtype)
+    off = torch.tensor([0, 0, 1, 1, 3, 5, 5], dtype=torch.int32)
+    s = x.double() + res[torch.arange(rows) + off].double()
+    want = torch.nn.functional.layer_norm(s, (width,), gamma.double(), beta.double(), 1e-5)
+    y, mean, inv, total = K.layer_norm_forward(x.cuda(), gamma.cuda(), beta.cuda(), (width,), 1e-5, residual=res.cuda(),
+                                               return_stats=True, return_sum=True, residual_row_offsets=off.cuda())
+    assert_stored_close(y.cpu(), want, dtype)
+    assert torch.equal(total.cpu(), (x.float() + res[torch.arange(rows) + off].float()).to(dtype))
+    assert max_abs(mean.cpu(), s.mean(-1)) <= 1e-5
+    assert max_abs(inv.cpu() * s.var(-1, unbiased=False).add(1e-5).sqrt(), torch.ones(rows)) <= 1e-5
