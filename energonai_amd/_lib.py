@@ -48,12 +48,15 @@ SIGNATURES = {
                            c_int, c_void_p, c_void_p]),
     "en_attn_tile_table_elems": (c_int64, [c_int] * 4),
     "en_attn_tile_table": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
+    "en_layer_tables": (c_int, [c_void_p] * 2 + [c_int] * 5 + [c_void_p] * 3),
     "en_attn_fused_query_tile": (c_int, [c_int] * 5),
     "en_packed_scores_elems": (c_int64, [c_int] * 4),
     "en_scale_mask_softmax_packed": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_void_p]),
     "en_decode_qk": (c_int, [c_void_p] * 4 + [c_int] * 4 + [c_int64] * 3 + [c_float, c_int, c_void_p]),
     "en_decode_pv": (c_int, [c_void_p] * 4 + [c_int] * 4 + [c_int64] * 3 + [c_int, c_void_p]),
     "en_decode_attn": (c_int, [c_void_p] * 5 + [c_int] * 4 + [c_void_p, c_void_p, c_float, c_int, c_void_p, c_int64, c_void_p]),
+    "en_decode_layer": (c_int, [c_void_p] * 5 + [c_int] * 4 + [c_void_p, c_void_p, c_float] + [c_void_p] * 5 +
+                        [c_int64, c_float, c_int, c_int, c_void_p, c_int64, c_void_p]),
     "en_decode_attn_workspace_bytes": (c_int64, [c_int] * 4),
     "en_decode_attn_paged": (c_int, [c_void_p] * 6 + [c_int] * 6 + [c_void_p, c_void_p, c_float, c_int, c_void_p, c_int64, c_void_p]),
     "en_kv_append_paged": (c_int, [c_void_p] * 6 + [c_int] * 6 + [c_int64, c_int64, c_void_p, c_int, c_void_p, c_void_p]),
@@ -78,6 +81,7 @@ LINEAR_SIGNATURES = {
 
 _lib = None
 _linear_lib = None
+_front = None
 
 
 def _refuse_stale(lib, symbol: str, expected: str, path: str) -> None:
@@ -133,6 +137,27 @@ def load() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _lib = lib
     return _lib
+
+
+def load_front():
+    """Loads the native host module once; raises RuntimeError if it is not built."""
+    global _front
+    if _front is None:
+        load()
+        from . import build
+        if not os.path.exists(build.FRONT_PATH):
+            raise RuntimeError("energonai_amd requires cuda extensions: _front.so is not built "
+                               "(run `python -m energonai_amd.build`)")
+        try:
+            from . import _front as module
+        except ImportError as exc:
+            raise RuntimeError(f"energonai_amd requires cuda extensions: cannot load {build.FRONT_PATH}: {exc}") from exc
+        if module.source_hash() != build.front_source_hash():
+            raise RuntimeError(f"energonai_amd requires cuda extensions: {build.FRONT_PATH} was built from other sources "
+                               f"(library {module.source_hash()}, tree {build.front_source_hash()}); "
+                               f"run `python -m energonai_amd.build`")
+        _front = module
+    return _front
 
 
 def check(status: int, op: str) -> None:
@@ -200,3 +225,15 @@ class _Fns:
 
 
 fn = _Fns()
+
+
+class _Front:
+    """Attribute access to the native host module: ``front.layer(...)``; loads it on first use."""
+
+    def __getattr__(self, name):
+        f = getattr(load_front(), name)
+        setattr(self, name, f)
+        return f
+
+
+front = _Front()

@@ -1,10 +1,11 @@
 """Builds libenergon_hip.so (gfx950) from energonai_amd/csrc/*.hip with hipcc, and
-libenergon_linear.so (host code over hipBLASLt) from csrc/linear_blaslt.cpp.
+libenergon_linear.so (host code over hipBLASLt) from csrc/linear_blaslt.cpp and the
+Python module _front (host code of the layer and decode steps over torch) from csrc/front.cpp.
 
     python -m energonai_amd.build            # compile every source, link the library
     python -m energonai_amd.build --force    # recompile even if objects look fresh
 
-The library is a plain C-ABI shared object (see include/energon_hip.h); it
+The kernel library is a plain C-ABI shared object (see include/energon_hip.h); it
 links against the HIP runtime only, never against torch.  hipcc cross-compiles
 for gfx950 without a GPU present.
 """
@@ -27,6 +28,9 @@ LIB_PATH = os.path.join(PKG_DIR, "libenergon_hip.so")
 # host-only hipBLASLt front end for the projection GEMMs; the only piece that links more than the HIP runtime
 LINEAR_SRC = os.path.join(CSRC, "linear_blaslt.cpp")
 LINEAR_LIB_PATH = os.path.join(PKG_DIR, "libenergon_linear.so")
+# host-only CPython module over torch's C++ API and the two libraries above
+FRONT_SRC = os.path.join(CSRC, "front.cpp")
+FRONT_PATH = os.path.join(PKG_DIR, "_front.so")
 
 ARCH = "gfx950"
 # packed fp32 VALU ops are switched off for device code on purpose (they have
@@ -73,6 +77,10 @@ def linear_source_hash() -> str:
     return _digest([LINEAR_SRC, os.path.join(INCLUDE, "energon_linear.h")])
 
 
+def front_source_hash() -> str:
+    return _digest([FRONT_SRC, os.path.join(INCLUDE, "energon_hip.h")])
+
+
 def _stale(src: str, obj: str) -> bool:
     if not os.path.exists(obj):
         return True
@@ -109,6 +117,7 @@ def build(force: bool = True, verbose: bool = False, jobs: int = 4) -> str:
         raise RuntimeError("link failed:\n" + proc.stdout)
     os.replace(tmp, LIB_PATH)
     build_linear()
+    build_front()
     return LIB_PATH
 
 
@@ -125,10 +134,29 @@ def build_linear() -> str:
     return LINEAR_LIB_PATH
 
 
+def build_front() -> str:
+    import sysconfig
+
+    from torch.utils.cpp_extension import include_paths, library_paths
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
+    libs = [p for p in library_paths("cuda") if os.path.isdir(p)]
+    tmp = FRONT_PATH + ".tmp"
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-I{INCLUDE}", f"-I{sysconfig.get_paths()['include']}", *[f"-I{p}" for p in include_paths("cuda")],
+           f"-I{rocm}/include", f'-DEN_SOURCE_HASH="{front_source_hash()}"', FRONT_SRC, "-o", tmp,
+           f"-L{PKG_DIR}", "-lenergon_hip", *[f"-L{p}" for p in libs], "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+           "-lc10_hip", f"-L{rocm}/lib", "-lamdhip64", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError("building _front.so failed:\n" + proc.stdout)
+    os.replace(tmp, FRONT_PATH)
+    return FRONT_PATH
+
+
 def ensure_built() -> None:
-    """Builds the two libraries if, and only if, one of them is missing (tests, the smoke run and the
+    """Builds the libraries if, and only if, one of them is missing (tests, the smoke run and the
     benchmark load what is there; they compile only when nothing is)."""
-    if not (os.path.exists(LIB_PATH) and os.path.exists(LINEAR_LIB_PATH)):
+    if not all(os.path.exists(p) for p in (LIB_PATH, LINEAR_LIB_PATH, FRONT_PATH)):
         build(force=False)
 
 

@@ -202,7 +202,9 @@ struct DecodeAttnArgs {
   int64_t k_sb, k_sh, k_ss, v_sb, v_sh, v_ss;
   float c_exp;        // scale * log2(e)
   int nsplit;         // workgroups that share one (batch, head) unit's keys (grid z); 1: none
-  float *partial;     // nsplit > 1: [B*H][nsplit][D + 2] unnormalised output, maximum (log2 domain), sum
+  // nsplit > 1, share z of unit u at u * nsplit + z: its unnormalised output [B*H*nsplit][D], and behind all of those its
+  // maximum (log2 domain) and sum [B*H*nsplit][2]
+  float *partial;
   // paged caches: k and v are pools of pages, page p of head h at p * k_sb + h * k_sh (k_sb is the page stride),
   // position s of sequence b in page page_table[b * max_pages + s / page] at row s % page
   const int32_t *page_table;
@@ -216,6 +218,10 @@ __device__ __forceinline__ int split_share(int kl, int nsplit) {
 }
 
 constexpr int kRankBatch = 256;
+
+__device__ __forceinline__ float2 *partial_ml(const DecodeAttnArgs &a, int64_t share_index) {
+  return reinterpret_cast<float2 *>(a.partial + (int64_t)a.B * a.H * a.nsplit * a.D) + share_index;
+}
 
 // From this size on (K and V together) the single pass reads the caches with non-temporal loads: a step walks the caches
 // of every layer before it comes back to these, and four layers of 64 MB are the whole memory-side cache (61 MB read
@@ -399,7 +405,7 @@ __global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeA
     if (lane == 0) { s_m[wave] = m_w; s_l[wave] = l_run; }
   }
   __syncthreads();
-  float *part = a.nsplit > 1 ? a.partial + (((int64_t)b * a.H + h) * a.nsplit + blockIdx.z) * (a.D + 2) : nullptr;
+  const int64_t share_index = ((int64_t)b * a.H + h) * a.nsplit + blockIdx.z;
   for (int d = tid; d < a.D; d += NT) {
     float m_all = -INFINITY;
 #pragma unroll
@@ -411,64 +417,165 @@ __global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeA
       l += s_l[w] * f;
       o += s_acc[w][d] * f;
     }
-    if (part) {
-      part[d] = o;
-      if (d == 0) { part[a.D] = m_all; part[a.D + 1] = l; }
+    if (a.nsplit > 1) {
+      a.partial[share_index * a.D + d] = o;
+      if (d == 0) *partial_ml(a, share_index) = make_float2(m_all, l);
     } else {
       ctx[d] = E::from_float(l > 0.f ? o / l : 0.f);
     }
   }
 }
 
-// Combines the partial results of the workgroups that shared a unit's keys: one workgroup per (batch, head).  The
-// partials of kAhead shares are sent for together with the length that says how many of them were written (the
-// workspace holds nsplit of them whatever the length), so that one trip to memory is waited for instead of three.
+// Combines N channels, from channel d on, of the partial results of a unit's shares.  The partials of kAhead shares are
+// sent for together with the length that says how many of them were written (the workspace holds nsplit of them whatever
+// the length), so that one trip to memory is waited for instead of three.
+template <int N>
+__device__ __forceinline__ void combine_shares(const DecodeAttnArgs &a, int b, int64_t unit, int d, float (&out)[N]) {
+  constexpr int kAhead = 4;
+  typedef Pack<float, N> P;
+  float m_run = -INFINITY, l_run = 0.f;
+#pragma unroll
+  for (int e = 0; e < N; ++e) out[e] = 0.f;
+  int nvalid = a.nsplit;
+  for (int z0 = 0; z0 < nvalid; z0 += kAhead) {
+    float2 ml[kAhead];
+    P o[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int64_t share_index = unit * a.nsplit + min(z0 + i, a.nsplit - 1);
+      o[i] = *reinterpret_cast<const P *>(a.partial + share_index * a.D + d);
+      ml[i] = *partial_ml(a, share_index);
+    }
+    if (z0 == 0) {
+      const int kl = max(min(a.kv_lens[b], a.Sk), 0);
+      const int share = split_share(kl, a.nsplit);
+      nvalid = share > 0 ? (kl + share - 1) / share : 0;       // shares that had keys
+    }
+    float m_new = m_run;
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      if (z0 + i >= nvalid) ml[i].x = -INFINITY;
+      m_new = fmaxf(m_new, ml[i].x);
+    }
+    if (m_new == -INFINITY) continue;
+    const float keep = __builtin_amdgcn_exp2f(m_run - m_new);        // exp2(-inf) = 0 before the first share
+    l_run *= keep;
+#pragma unroll
+    for (int e = 0; e < N; ++e) out[e] *= keep;
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      if (ml[i].x == -INFINITY) continue;                            // never written, or no key: whatever it holds stays out
+      const float f = __builtin_amdgcn_exp2f(ml[i].x - m_new);
+      l_run += ml[i].y * f;
+#pragma unroll
+      for (int e = 0; e < N; ++e) out[e] += o[i].v[e] * f;
+    }
+    m_run = m_new;
+  }
+  const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+#pragma unroll
+  for (int e = 0; e < N; ++e) out[e] *= inv;
+}
+
 template <int DT>
 __global__ __launch_bounds__(kBlock) void decode_attn_combine_kernel(DecodeAttnArgs a) {
   typedef Elem<DT> E;
   typedef typename E::T T;
-  constexpr int kAhead = 8;
   const int unit = blockIdx.x, b = unit / a.H;
-  const float *part = a.partial + (int64_t)unit * a.nsplit * (a.D + 2);
   T *ctx = reinterpret_cast<T *>(a.ctx) + (int64_t)unit * a.D;
   for (int d = threadIdx.x; d < a.D; d += kBlock) {
-    float m_run = -INFINITY, l_run = 0.f, o_run = 0.f;
-    int nvalid = a.nsplit;
-    for (int z0 = 0; z0 < nvalid; z0 += kAhead) {
-      float m[kAhead], l[kAhead], o[kAhead];
-#pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        const float *p = part + min(z0 + i, a.nsplit - 1) * (a.D + 2);
-        o[i] = p[d];
-        m[i] = p[a.D];
-        l[i] = p[a.D + 1];
-      }
-      if (z0 == 0) {
-        const int kl = max(min(a.kv_lens[b], a.Sk), 0);
-        const int share = split_share(kl, a.nsplit);
-        nvalid = share > 0 ? (kl + share - 1) / share : 0;       // shares that had keys
-      }
-      float m_new = m_run;
-#pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        if (z0 + i >= nvalid) m[i] = -INFINITY;
-        m_new = fmaxf(m_new, m[i]);
-      }
-      if (m_new == -INFINITY) continue;
-      const float keep = __builtin_amdgcn_exp2f(m_run - m_new);        // exp2(-inf) = 0 before the first share
-      l_run *= keep;
-      o_run *= keep;
-#pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        if (m[i] == -INFINITY) continue;                               // never written, or no key: whatever it holds stays out
-        const float f = __builtin_amdgcn_exp2f(m[i] - m_new);
-        l_run += l[i] * f;
-        o_run += o[i] * f;
-      }
-      m_run = m_new;
-    }
-    ctx[d] = E::from_float(l_run > 0.f ? o_run / l_run : 0.f);
+    float o[1];
+    combine_shares<1>(a, b, unit, d, o);
+    ctx[d] = E::from_float(o[0]);
   }
+}
+
+// The decode step whose shared units are followed by nothing but residual + LayerNorm (no projection in between, LayerNorm
+// width = heads * size_per_head): the combine pass is the LayerNorm's input and has no launch or round trip of its own.
+// One workgroup of 1024 lanes per sequence, four channels per lane and vector: a row of 9216 channels is 2.25 vectors.
+// One sequence of 72 heads x 128, 1655 keys: combine + LayerNorm 4.8 + 3.5 us as two launches, one of 4.4.
+struct DecodeNormArgs {
+  DecodeAttnArgs attn;
+  const void *residual, *gamma, *beta;
+  void *y;
+  int hidden;
+  float eps;
+};
+
+constexpr int kNormLanes = 1024;
+
+template <int DT, int VPL>
+__global__ __launch_bounds__(kNormLanes) void decode_combine_norm_kernel(DecodeNormArgs n) {
+  typedef Elem<DT> E;
+  typedef typename E::T T;
+  constexpr int N = 4;                 // channels per vector
+  typedef Pack<T, N> P;
+  __shared__ float s_a[kNormLanes / kWave], s_b[kNormLanes / kWave];
+  const DecodeAttnArgs &a = n.attn;
+  const int b = blockIdx.x, t = threadIdx.x;
+  const int nvec = n.hidden / N;
+  const T *res = reinterpret_cast<const T *>(n.residual) + (int64_t)b * n.hidden;
+  const T *gamma = reinterpret_cast<const T *>(n.gamma), *beta = reinterpret_cast<const T *>(n.beta);
+  P r[VPL], g[VPL], bt[VPL];
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int v = min(t + kNormLanes * j, nvec - 1);
+    r[j] = load_pack<T, N>(res + v * N);
+    g[j] = load_pack<T, N>(gamma + v * N);
+    bt[j] = load_pack<T, N>(beta + v * N);
+  }
+  float x[VPL][N];
+  float s = 0.f;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int v = t + kNormLanes * j;
+    if (v < nvec) {
+      const int h = v * N / a.D, d = v * N - h * a.D;
+      combine_shares<N>(a, b, (int64_t)b * a.H + h, d, x[j]);
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        x[j][e] += E::to_float(r[j].v[e]);
+        s += x[j][e];
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < N; ++e) x[j][e] = 0.f;
+    }
+  }
+  s = block_allreduce<OpSum, kNormLanes / kWave>(s, s_a);
+  const float mu = s / (float)n.hidden;
+  float d2 = 0.f;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j)
+    if (t + kNormLanes * j < nvec)
+#pragma unroll
+      for (int e = 0; e < N; ++e) d2 += (x[j][e] - mu) * (x[j][e] - mu);
+  d2 = block_allreduce<OpSum, kNormLanes / kWave>(d2, s_b);
+  const float inv = 1.0f / sqrtf(d2 / (float)n.hidden + n.eps);
+  T *y = reinterpret_cast<T *>(n.y) + (int64_t)b * n.hidden;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int v = t + kNormLanes * j;
+    if (v < nvec) {
+      P o;
+#pragma unroll
+      for (int e = 0; e < N; ++e)
+        o.v[e] = E::from_float((x[j][e] - mu) * inv * E::to_float(g[j].v[e]) + E::to_float(bt[j].v[e]));
+      store_pack<T, N>(y + v * N, o);
+    }
+  }
+}
+
+template <int DT>
+static int launch_combine_norm(const DecodeNormArgs &n, hipStream_t s) {
+  const int vpl = (int)ceil_div(n.hidden / 4, kNormLanes);
+  const unsigned grid = (unsigned)n.attn.B;
+  if (vpl <= 1) decode_combine_norm_kernel<DT, 1><<<grid, kNormLanes, 0, s>>>(n);
+  else if (vpl == 2) decode_combine_norm_kernel<DT, 2><<<grid, kNormLanes, 0, s>>>(n);
+  else if (vpl == 3) decode_combine_norm_kernel<DT, 3><<<grid, kNormLanes, 0, s>>>(n);
+  else decode_combine_norm_kernel<DT, 4><<<grid, kNormLanes, 0, s>>>(n);
+  EN_RETURN_IF_LAUNCH_FAILED();
+  return EN_OK;
 }
 
 // Which form of the kernel a call runs (lanes per workgroup x keys per lane group and stage; all hold two stages):
@@ -505,7 +612,7 @@ static void launch_attn_form(const DecodeAttnArgs &a, dim3 grid, bool stream_cac
 }
 
 template <int DT, bool PAGED = false>
-static int dispatch_attn(const DecodeAttnArgs &a, bool stream_cache, hipStream_t s) {
+static int dispatch_attn(const DecodeAttnArgs &a, bool stream_cache, hipStream_t s, bool combine = true) {
   constexpr int EPV = 16 / Elem<DT>::kSize;
   int lpk = 4;
   while (lpk * EPV < a.D) lpk *= 2;
@@ -519,7 +626,7 @@ static int dispatch_attn(const DecodeAttnArgs &a, bool stream_cache, hipStream_t
     default: return EN_ERR_UNSUPPORTED;
   }
   EN_RETURN_IF_LAUNCH_FAILED();
-  if (a.nsplit > 1) {
+  if (a.nsplit > 1 && combine) {
     decode_attn_combine_kernel<DT><<<(unsigned)(a.B * a.H), kBlock, 0, s>>>(a);
     EN_RETURN_IF_LAUNCH_FAILED();
   }
@@ -637,6 +744,43 @@ __global__ __launch_bounds__(kBlock) void kv_fill_paged_kernel(PagedFillArgs a) 
   }
 }
 
+// Checks the arguments of the contiguous-cache entry points and fills the kernel's.
+static int attn_args(DecodeAttnArgs &a, const void *q, const void *k_cache, const void *v_cache, void *ctx,
+                     const int32_t *kv_lens, int batch, int head_num, int k_seq_len, int size_per_head,
+                     const int64_t *k_strides, const int64_t *v_strides, float scale, int dtype, void *workspace,
+                     int64_t workspace_bytes) {
+  if (!k_strides || !v_strides || !v_cache) return EN_ERR_NULL;
+  int rc = check_decode(q, k_cache, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
+                        k_strides[2], dtype);
+  if (rc) return rc;
+  const int es = dtype_size(dtype), epv = 16 / es;
+  if (!aligned_to(v_cache, 16) || (v_strides[0] % epv) || (v_strides[1] % epv) || (v_strides[2] % epv)) return EN_ERR_ALIGN;
+  if (!aligned_to(q, 16) || !aligned_to(ctx, es)) return EN_ERR_ALIGN;
+  if (size_per_head > 64 * epv) return EN_ERR_UNSUPPORTED;
+  // 32-bit byte offsets inside a (batch, head) unit, two stages of keys past the end included
+  if (((int64_t)k_seq_len + 4096) * k_strides[2] * es >= (1ll << 31) || ((int64_t)k_seq_len + 4096) * v_strides[2] * es >= (1ll << 31))
+    return EN_ERR_UNSUPPORTED;
+  if (!(scale > 0.f)) return EN_ERR_UNSUPPORTED;     // the running maximum is kept in units of scale * log2(e)
+  for (int i = 0; i < 3; ++i)
+    if (k_strides[i] < 0 || v_strides[i] < 0) return EN_ERR_UNSUPPORTED;
+  // a unit's keys are shared between workgroups only when the caller brought the room for their partial results
+  const int64_t need = en_decode_attn_workspace_bytes(batch, head_num, k_seq_len, size_per_head);
+  const bool split = need > 0 && workspace && workspace_bytes >= need && aligned_to(workspace, 16);
+  a = DecodeAttnArgs{q, k_cache, v_cache, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
+                     k_strides[2], v_strides[0], v_strides[1], v_strides[2], scale * 1.4426950408889634f,
+                     split ? decode_split(batch, head_num, k_seq_len) : 1, static_cast<float *>(workspace)};
+  return EN_OK;
+}
+
+static int dispatch_attn_dtype(const DecodeAttnArgs &a, int dtype, hipStream_t s, bool combine) {
+  const bool stream_cache = 2 * cache_bytes(a.B, a.H, a.Sk, a.D, dtype) >= kAttnStreamBytes;
+  switch (dtype) {
+    case EN_F32: return dispatch_attn<EN_F32>(a, stream_cache, s, combine);
+    case EN_F16: return dispatch_attn<EN_F16>(a, stream_cache, s, combine);
+    default: return dispatch_attn<EN_BF16>(a, stream_cache, s, combine);
+  }
+}
+
 static int log2_exact(int v) {
   int lg = 0;
   while ((1 << lg) < v) ++lg;
@@ -694,32 +838,38 @@ int en_decode_attn(const void *q, const void *k_cache, const void *v_cache, void
                    int head_num, int k_seq_len, int size_per_head, const int64_t *k_strides, const int64_t *v_strides,
                    float scale, int dtype, void *workspace, int64_t workspace_bytes, en_stream_t stream) {
   using namespace en;
-  if (!k_strides || !v_strides || !v_cache) return EN_ERR_NULL;
-  int rc = check_decode(q, k_cache, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
-                        k_strides[2], dtype);
+  DecodeAttnArgs a;
+  const int rc = attn_args(a, q, k_cache, v_cache, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides,
+                           v_strides, scale, dtype, workspace, workspace_bytes);
+  return rc ? rc : dispatch_attn_dtype(a, dtype, (hipStream_t)stream, true);
+}
+
+int en_decode_layer(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens, int batch,
+                    int head_num, int k_seq_len, int size_per_head, const int64_t *k_strides, const int64_t *v_strides,
+                    float scale, const void *dense_out, const void *residual, const void *gamma, const void *beta, void *y,
+                    int64_t hidden, float eps, int dtype, int out_dtype, void *workspace, int64_t workspace_bytes,
+                    en_stream_t stream) {
+  using namespace en;
+  if (!residual || !gamma || !beta || !y) return EN_ERR_NULL;
+  if (hidden < 1 || (!dense_out && hidden != (int64_t)head_num * size_per_head)) return EN_ERR_SHAPE;
+  DecodeAttnArgs a;
+  int rc = attn_args(a, q, k_cache, v_cache, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides, v_strides,
+                     scale, dtype, workspace, workspace_bytes);
   if (rc) return rc;
-  const int es = dtype_size(dtype), epv = 16 / es;
-  if (!aligned_to(v_cache, 16) || (v_strides[0] % epv) || (v_strides[1] % epv) || (v_strides[2] % epv)) return EN_ERR_ALIGN;
-  if (!aligned_to(q, 16) || !aligned_to(ctx, es)) return EN_ERR_ALIGN;
-  if (size_per_head > 64 * epv) return EN_ERR_UNSUPPORTED;
-  // 32-bit byte offsets inside a (batch, head) unit, two stages of keys past the end included
-  if (((int64_t)k_seq_len + 4096) * k_strides[2] * es >= (1ll << 31) || ((int64_t)k_seq_len + 4096) * v_strides[2] * es >= (1ll << 31))
-    return EN_ERR_UNSUPPORTED;
-  if (!(scale > 0.f)) return EN_ERR_UNSUPPORTED;     // the running maximum is kept in units of scale * log2(e)
-  for (int i = 0; i < 3; ++i)
-    if (k_strides[i] < 0 || v_strides[i] < 0) return EN_ERR_UNSUPPORTED;
-  // a unit's keys are shared between workgroups only when the caller brought the room for their partial results
-  const int64_t need = en_decode_attn_workspace_bytes(batch, head_num, k_seq_len, size_per_head);
-  const bool split = need > 0 && workspace && workspace_bytes >= need && aligned_to(workspace, 4);
-  DecodeAttnArgs a{q, k_cache, v_cache, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
-                   k_strides[2], v_strides[0], v_strides[1], v_strides[2], scale * 1.4426950408889634f,
-                   split ? decode_split(batch, head_num, k_seq_len) : 1, static_cast<float *>(workspace)};
-  const bool stream_cache = 2 * cache_bytes(batch, head_num, k_seq_len, size_per_head, dtype) >= kAttnStreamBytes;
+  const int vec = 4 * dtype_size(dtype);
+  const bool one_pass = a.nsplit > 1 && !dense_out && out_dtype == dtype && hidden <= 4 * 4 * kNormLanes &&
+                        aligned_to(residual, vec) && aligned_to(gamma, vec) && aligned_to(beta, vec) && aligned_to(y, vec);
   hipStream_t s = (hipStream_t)stream;
+  rc = dispatch_attn_dtype(a, dtype, s, !one_pass);
+  if (rc) return rc;
+  if (!one_pass)
+    return en_layernorm_fwd(y, nullptr, nullptr, nullptr, dense_out ? dense_out : ctx, residual, nullptr, gamma, beta, batch,
+                            hidden, eps, dtype, out_dtype, stream);
+  const DecodeNormArgs n{a, residual, gamma, beta, y, (int)hidden, eps};
   switch (dtype) {
-    case EN_F32: return dispatch_attn<EN_F32>(a, stream_cache, s);
-    case EN_F16: return dispatch_attn<EN_F16>(a, stream_cache, s);
-    default: return dispatch_attn<EN_BF16>(a, stream_cache, s);
+    case EN_F32: return launch_combine_norm<EN_F32>(n, s);
+    case EN_F16: return launch_combine_norm<EN_F16>(n, s);
+    default: return launch_combine_norm<EN_BF16>(n, s);
   }
 }
 
@@ -803,7 +953,7 @@ int en_decode_attn_paged(const void *q, const void *k_pool, const void *v_pool, 
   for (int i = 0; i < 3; ++i)
     if (k_strides[i] < 0 || v_strides[i] < 0) return EN_ERR_UNSUPPORTED;
   const int64_t need = en_decode_attn_workspace_bytes(batch, head_num, k_seq_len, size_per_head);
-  const bool split = need > 0 && workspace && workspace_bytes >= need && aligned_to(workspace, 4);
+  const bool split = need > 0 && workspace && workspace_bytes >= need && aligned_to(workspace, 16);
   DecodeAttnArgs a{q, k_pool, v_pool, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
                    k_strides[2], v_strides[0], v_strides[1], v_strides[2], scale * 1.4426950408889634f,
                    split ? decode_split(batch, head_num, k_seq_len) : 1, static_cast<float *>(workspace),

@@ -1,0 +1,300 @@
+// The host side of a layer step, a decode step and a batch's bookkeeping as one native call each: argument checks, output
+// allocation (torch's caching allocator), stream lookup and the C ABI call.  The same work in Python and ctypes costs 16 us
+// per layer step and 23 us per decode step against 6 us of kernel launches, which is more than the GPU needs for a short
+// prompt (9 us) or a decode step of one sequence.  Nothing is computed here; every launch is an entry point of
+// libenergon_hip.so.
+//
+// A plain CPython module (METH_FASTCALL, no pybind11): a call has up to twenty arguments, and converting them costs more
+// than what the call does if each goes through a type caster.
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include <stdexcept>
+#include <string>
+
+#include "energon_hip.h"
+
+#ifndef EN_SOURCE_HASH
+#define EN_SOURCE_HASH "unknown"
+#endif
+
+namespace {
+
+using at::Tensor;
+
+[[noreturn]] void fail(const std::string &msg) { throw std::runtime_error(msg); }
+
+void check(int status, const char *op) {
+  if (status == EN_OK) return;
+  std::string msg = std::string(op) + ": " + en_status_string(status);
+  if (status == EN_ERR_HIP)
+    msg += std::string(": ") + en_last_hip_error_string() + " (hipError " + std::to_string(en_last_hip_error()) + ")";
+  fail(msg);
+}
+
+// ---- arguments -----------------------------------------------------------------------------------------------------
+
+const Tensor &tensor(PyObject *o, const char *name) {
+  if (!THPVariable_Check(o)) fail(std::string(name) + " must be a CUDA tensor");
+  return THPVariable_Unpack(o);
+}
+
+const Tensor &gpu(PyObject *o, const char *name, bool contiguous = true) {
+  const Tensor &t = tensor(o, name);
+  if (!t.is_cuda()) fail(std::string(name) + " must be a CUDA tensor");
+  if (contiguous && !t.is_contiguous()) fail(std::string(name) + " must be contiguous");
+  return t;
+}
+
+int64_t integer(PyObject *o) {
+  const int64_t v = PyLong_AsLongLong(o);
+  if (v == -1 && PyErr_Occurred()) fail("an integer is required");
+  return v;
+}
+
+float real(PyObject *o) {
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) fail("a number is required");
+  return (float)v;
+}
+
+int dtype_tag(const Tensor &t, const char *op) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return EN_F32;
+    case at::kHalf: return EN_F16;
+    case at::kBFloat16: return EN_BF16;
+    default:
+      fail(std::string(op) + ": Datatype not implemented (" + c10::toString(t.scalar_type()) +
+           "); expected float32, float16 or bfloat16");
+  }
+}
+
+hipStream_t stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+const int32_t *i32(const Tensor &t) { return t.data_ptr<int32_t>(); }
+
+// Launches run without the interpreter lock: a launch may wait for room in the stream's queue.
+template <typename F> int without_gil(F &&f) {
+  PyThreadState *saved = PyEval_SaveThread();
+  const int rc = f();
+  PyEval_RestoreThread(saved);
+  return rc;
+}
+
+// ---- events (SeqInfo orders other streams behind the kernels that produced its arrays) -------------------------------
+
+void destroy_event(PyObject *capsule) {
+  void *p = PyCapsule_GetPointer(capsule, "energonai_amd.event");
+  if (p) (void)hipEventDestroy(static_cast<hipEvent_t>(p));
+}
+
+PyObject *record_event(PyObject *const *a) {
+  const Tensor &t = gpu(a[0], "lens");
+  const c10::DeviceGuard guard(t.device());
+  hipEvent_t e;
+  if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) fail("record_event: hipEventCreate failed");
+  PyObject *capsule = PyCapsule_New(e, "energonai_amd.event", destroy_event);
+  if (!capsule) {
+    (void)hipEventDestroy(e);
+    return nullptr;
+  }
+  if (hipEventRecord(e, stream_of(t)) != hipSuccess) {
+    Py_DECREF(capsule);
+    fail("record_event: hipEventRecord failed");
+  }
+  return capsule;
+}
+
+PyObject *wait_event(PyObject *const *a) {
+  void *p = PyCapsule_GetPointer(a[0], "energonai_amd.event");
+  if (!p) return nullptr;
+  const Tensor &t = gpu(a[1], "lens");
+  const c10::DeviceGuard guard(t.device());
+  if (hipStreamWaitEvent(stream_of(t), static_cast<hipEvent_t>(p), 0) != hipSuccess) fail("wait_event: hipStreamWaitEvent failed");
+  Py_RETURN_NONE;
+}
+
+PyObject *pair(const Tensor &x, const Tensor &y) {
+  PyObject *px = THPVariable_Wrap(x), *py = THPVariable_Wrap(y);
+  PyObject *r = (px && py) ? PyTuple_Pack(2, px, py) : nullptr;
+  Py_XDECREF(px);
+  Py_XDECREF(py);
+  return r;
+}
+
+// prefix_sum(lens, batch) -> (cu_seqlens [batch + 1], lens [batch]), both int32
+PyObject *prefix_sum(PyObject *const *a) {
+  const Tensor &lens = gpu(a[0], "seq_lens");
+  const int64_t batch = integer(a[1]);
+  const bool i64 = lens.scalar_type() == at::kLong;
+  if ((!i64 && lens.scalar_type() != at::kInt) || lens.numel() < batch) fail("prefix_sum: lens must hold batch int32 or int64 values");
+  const c10::DeviceGuard guard(lens.device());
+  const auto opt = lens.options().dtype(at::kInt);
+  const Tensor cu = at::empty({batch + 1}, opt), lens32 = at::empty({batch}, opt);
+  check(without_gil([&] {
+          return en_prefix_sum(lens.data_ptr(), i64, (int)batch, cu.data_ptr<int32_t>(), lens32.data_ptr<int32_t>(), stream_of(lens));
+        }), "prefix_sum");
+  return pair(cu, lens32);
+}
+
+// layer_tables(lens, cu_seqlens, batch, max_seq_len, left_padded, total, heads, tiles_first) -> (row offsets, tile table)
+PyObject *layer_tables(PyObject *const *a) {
+  const Tensor &lens = gpu(a[0], "lens"), &cu = gpu(a[1], "cu_seqlens");
+  const int64_t batch = integer(a[2]), S = integer(a[3]), left = integer(a[4]), total = integer(a[5]), heads = integer(a[6]),
+                tiles_first = integer(a[7]);
+  const c10::DeviceGuard guard(lens.device());
+  const int64_t n = en_attn_tile_table_elems((int)batch, (int)heads, (int)S, 0);
+  const Tensor offs = at::empty({total > 0 ? total : 1}, lens.options()), table = at::empty({n > 0 ? n : 1}, lens.options());
+  check(without_gil([&] {
+          return en_layer_tables(i32(lens), i32(cu), (int)batch, (int)S, (int)left, (int)heads, (int)tiles_first,
+                                 table.data_ptr<int32_t>(), offs.data_ptr<int32_t>(), stream_of(lens));
+        }), "layer_tables");
+  return pair(offs, table);
+}
+
+// layer(hidden_padded, qkv_packed, dense_out, gamma, beta, ctx_out, cu_seqlens, lens, row offsets or None, tile table or None,
+//       heads, size_per_head, total, scale, eps, causal, left_padded, form) -> y
+PyObject *layer(PyObject *const *a) {
+  static const std::string who = "padding_removal_layer: ";
+  const Tensor &hidden = gpu(a[0], "hidden_padded"), &qkv = gpu(a[1], "qkv_packed");
+  const bool has_dense = a[2] != Py_None, has_ctx = a[5] != Py_None;
+  const Tensor &gamma = tensor(a[3], "gamma"), &beta = tensor(a[4], "beta");
+  const Tensor &cu = tensor(a[6], "cu_seqlens"), &lens = tensor(a[7], "lens");
+  const int32_t *offs = a[8] == Py_None ? nullptr : i32(tensor(a[8], "offsets"));
+  const int32_t *table = a[9] == Py_None ? nullptr : i32(tensor(a[9], "tile_table"));
+  const int64_t H = integer(a[10]), D = integer(a[11]), T = integer(a[12]);
+  const float scale = real(a[13]), eps = real(a[14]);
+  const int causal = (int)integer(a[15]), left = (int)integer(a[16]), form = (int)integer(a[17]);
+  const int64_t B = hidden.size(0), S = hidden.size(1), hid = hidden.size(2);
+  const auto dt = hidden.scalar_type();
+  if (qkv.numel() != T * H * 3 * D || qkv.scalar_type() != dt) fail(who + "qkv_packed must be [1,T,H,3D] of the activation dtype");
+  if (gamma.scalar_type() != dt || beta.scalar_type() != dt || gamma.numel() != hid || beta.numel() != hid)
+    fail(who + "gamma and beta must be [hidden] of the activation dtype");
+  const void *dense = nullptr;
+  if (has_dense) {
+    const Tensor &d = gpu(a[2], "dense_out");
+    if (d.numel() != T * hid || d.scalar_type() != dt) fail(who + "dense_out must be [1,T,hidden] of the activation dtype");
+    dense = d.data_ptr();
+  } else if (hid != H * D) {
+    fail(who + "without dense_out the LayerNorm width must equal heads * size_per_head");
+  }
+  const int tag = dtype_tag(hidden, "padding_removal_layer");
+  if (form == 4 && dt == at::kFloat) fail(who + "the packed scores are for float16 and bfloat16");
+  if ((form == 1 || form == 2) && dt == at::kFloat && D > 64) fail(who + "the fused kernel takes float32 heads of up to 64 channels");
+  if (form == 4 && !causal) fail(who + "the packed score layout is that of a causal mask");
+  const c10::DeviceGuard guard(hidden.device());
+  const auto opt = hidden.options();
+  const Tensor y = at::empty({1, T, hid}, opt);
+  Tensor x, padded, ctx, scores, ctx_packed;
+  if (!offs) x = at::empty({1, T, hid}, opt);
+  if (has_ctx) {
+    const Tensor &c = gpu(a[5], "ctx_out", false);
+    if (c.numel() != T * H * D || c.scalar_type() != dt || !c.is_contiguous())
+      fail(who + "ctx_out must be a contiguous [1,T,H,D] tensor of the activation dtype");
+    ctx_packed = c;
+  } else {
+    ctx_packed = at::empty({1, T, H, D}, opt);
+  }
+  if (form < 2) {
+    padded = at::empty({B, H, S, 3 * D}, opt);
+    ctx = at::empty({B, H, S, D}, opt);
+  }
+  if (form == 0 || form == 3) scores = at::empty({B, H, S, S}, opt);
+  if (form == 4) {
+    const int64_t n = en_packed_scores_elems((int)B, (int)H, (int)S, tag);
+    if (n <= 0) fail("packed_scores_elems: bad arguments");
+    scores = at::empty({n}, opt);
+  }
+  auto ptr = [](const Tensor &t) -> void * { return t.defined() ? t.data_ptr() : nullptr; };
+  check(without_gil([&] {
+          return en_padding_removal_layer(hidden.data_ptr(), qkv.data_ptr(), dense, gamma.data_ptr(), beta.data_ptr(), ptr(x),
+                                          ptr(padded), ptr(scores), ptr(ctx), ctx_packed.data_ptr(), y.data_ptr(), i32(cu), i32(lens),
+                                          (int)B, (int)S, (int)H, (int)D, hid, T, scale, eps, causal, left, form, offs, tag, table,
+                                          stream_of(hidden));
+        }), "padding_removal_layer");
+  return THPVariable_Wrap(y);
+}
+
+// decode_layer(q, k_cache, v_cache, lens, residual, gamma, beta, dense_out, eps, scale) -> y
+PyObject *decode_layer(PyObject *const *a) {
+  const Tensor &q_in = gpu(a[0], "q", false), &k = gpu(a[1], "k_cache", false), &v = gpu(a[2], "v_cache", false);
+  const Tensor &lens = tensor(a[3], "lens"), &residual = gpu(a[4], "residual", false), &gamma_in = gpu(a[5], "gamma", false),
+               &beta_in = gpu(a[6], "beta", false);
+  const float eps = real(a[8]), scale = real(a[9]);
+  for (const Tensor *c : {&k, &v}) {
+    const char *name = c == &k ? "k_cache" : "v_cache";
+    if (c->dim() != 4) fail(std::string(name) + " must be [batch, head, seq, size_per_head]");
+    if (c->stride(3) != 1) fail(std::string(name) + ": the last dimension must be contiguous");
+  }
+  const int64_t B = k.size(0), H = k.size(1), S = k.size(2), D = k.size(3), hid = gamma_in.numel();
+  const auto dt = q_in.scalar_type();
+  if (v.sizes() != k.sizes() || v.scalar_type() != k.scalar_type()) fail("decode_attn: k_cache and v_cache must share shape and dtype");
+  if (q_in.numel() != B * H * D || dt != k.scalar_type()) fail("decode_attn: q must be [B,H,1,D] of the caches' dtype");
+  const int tag = dtype_tag(q_in, "decode_attn"), out_tag = dtype_tag(gamma_in, "layer_norm");
+  if (gamma_in.scalar_type() != beta_in.scalar_type()) fail("gamma and beta must share one dtype");
+  if (beta_in.numel() != hid) fail("gamma and beta must have normalized_shape");
+  Tensor dense;
+  if (a[7] != Py_None) dense = gpu(a[7], "dense_out", false).contiguous();
+  const auto in_dt = dense.defined() ? dense.scalar_type() : dt;
+  if (in_dt != dt || (tag != out_tag && tag != EN_F32))
+    fail("layer_norm: unsupported (input, output) dtypes (" + std::string(c10::toString(in_dt)) + ", " + c10::toString(gamma_in.scalar_type()) + ")");
+  if (dense.defined() ? (dense.size(-1) != hid || dense.numel() != B * hid) : H * D != hid)
+    fail("Given normalized_shape=[" + std::to_string(hid) + "], the LayerNorm input must have that last dimension and batch rows");
+  if (residual.scalar_type() != dt || residual.numel() != B * hid || residual.size(-1) != hid) fail("residual must match input in shape and dtype");
+  const c10::DeviceGuard guard(k.device());
+  const Tensor q = q_in.contiguous(), res = residual.contiguous(), gamma = gamma_in.contiguous(), beta = beta_in.contiguous();
+  const Tensor ctx = at::empty({B, H, 1, D}, q.options());
+  const Tensor y = at::empty(dense.defined() ? dense.sizes() : c10::IntArrayRef({1, B, hid}), gamma.options());
+  const int64_t need = en_decode_attn_workspace_bytes((int)B, (int)H, (int)S, (int)D);
+  Tensor ws;
+  if (need > 0) ws = at::empty({need}, q.options().dtype(at::kByte));
+  const int64_t ks[3] = {k.stride(0), k.stride(1), k.stride(2)}, vs[3] = {v.stride(0), v.stride(1), v.stride(2)};
+  check(without_gil([&] {
+          return en_decode_layer(q.data_ptr(), k.data_ptr(), v.data_ptr(), ctx.data_ptr(), i32(lens), (int)B, (int)H, (int)S, (int)D,
+                                 ks, vs, scale, dense.defined() ? dense.data_ptr() : nullptr, res.data_ptr(), gamma.data_ptr(),
+                                 beta.data_ptr(), y.data_ptr(), hid, eps, tag, out_tag, need > 0 ? ws.data_ptr() : nullptr, need,
+                                 stream_of(k));
+        }), "decode_layer");
+  return THPVariable_Wrap(y);
+}
+
+// ---- module --------------------------------------------------------------------------------------------------------
+
+template <PyObject *(*F)(PyObject *const *), int N>
+PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  if (n != N) {
+    PyErr_Format(PyExc_TypeError, "%d arguments expected, %zd given", N, n);
+    return nullptr;
+  }
+  try {
+    PyObject *r = F(args);
+    return r;
+  } catch (const std::exception &e) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+PyObject *source_hash(PyObject *, PyObject *) { return PyUnicode_FromString(EN_SOURCE_HASH); }
+
+#define EN_FAST(name, nargs, doc) \
+  {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&entry<name, nargs>)), METH_FASTCALL, doc}
+
+PyMethodDef kMethods[] = {
+    {"source_hash", source_hash, METH_NOARGS, "digest of the sources this module was built from"},
+    EN_FAST(record_event, 1, "event recorded on the current stream of the tensor's device"),
+    EN_FAST(wait_event, 2, "makes the current stream of the tensor's device wait for the event"),
+    EN_FAST(prefix_sum, 2, "(cu_seqlens, lens) of a batch"),
+    EN_FAST(layer_tables, 8, "(row offsets, tile table) of a batch"),
+    EN_FAST(layer, 18, "en_padding_removal_layer on new outputs"),
+    EN_FAST(decode_layer, 10, "en_decode_layer on new outputs"),
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_front", "host side of the layer and decode steps", -1, kMethods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__front(void) { return PyModule_Create(&kModule); }

@@ -92,8 +92,8 @@ def padding_removal_layer(hidden_padded: torch.Tensor, qkv_packed: torch.Tensor,
     if fold_depad is None:
         fold_depad = not keep
     if not keep:
-        return _layer_one_call(hidden_padded, qkv_packed, info, B, S, H, D, hid, T, gamma, beta, eps, scale, causal,
-                               left_padded, dense_out, fused_attention, fold_depad, ctx_out)
+        return _layer_one_call(hidden_padded, qkv_packed, info, S, H, D, T, gamma, beta, eps, scale, causal, left_padded,
+                               dense_out, fused_attention, fold_depad, ctx_out)
     if fold_depad:
         raise RuntimeError("padding_removal_layer: fold_depad has no intermediates to keep")
 
@@ -133,56 +133,22 @@ def padding_removal_layer(hidden_padded: torch.Tensor, qkv_packed: torch.Tensor,
 _FORMS = {False: 0, True: 1, "packed": 2, "varlen": 3, "varlen_packed": 4}
 
 
-def _layer_one_call(hidden_padded, qkv_packed, info, B, S, H, D, hid, T, gamma, beta, eps, scale, causal, left_padded,
+def _layer_one_call(hidden_padded, qkv_packed, info, S, H, D, T, gamma, beta, eps, scale, causal, left_padded,
                     dense_out, fused_attention, fold_depad=False, ctx_out=None):
-    """The same seven ops through ``en_padding_removal_layer``: one foreign call per step."""
-    dev, dt = hidden_padded.device, hidden_padded.dtype
+    """The same seven ops through ``en_padding_removal_layer``: one native call per step."""
     form = _FORMS[fused_attention]
-    _lib.require_gpu(hidden_padded, "hidden_padded")
-    _lib.require_gpu(qkv_packed, "qkv_packed")
-    if qkv_packed.numel() != T * H * 3 * D or qkv_packed.dtype != dt:
-        raise RuntimeError("padding_removal_layer: qkv_packed must be [1,T,H,3D] of the activation dtype")
-    if gamma.dtype != dt or beta.dtype != dt or gamma.numel() != hid or beta.numel() != hid:
-        raise RuntimeError("padding_removal_layer: gamma and beta must be [hidden] of the activation dtype")
-    if dense_out is not None:
-        _lib.require_gpu(dense_out, "dense_out")
-        if dense_out.numel() != T * hid or dense_out.dtype != dt:
-            raise RuntimeError("padding_removal_layer: dense_out must be [1,T,hidden] of the activation dtype")
-    elif hid != H * D:
-        raise RuntimeError("padding_removal_layer: without dense_out the LayerNorm width must equal heads * size_per_head")
-    if form == 4 and dt == torch.float32:
-        raise RuntimeError("padding_removal_layer: the packed scores are for float16 and bfloat16")
-    if form in (1, 2) and dt == torch.float32 and D > 64:
-        raise RuntimeError("padding_removal_layer: the fused kernel takes float32 heads of up to 64 channels")
-    if form == 4 and not causal:
-        raise RuntimeError("padding_removal_layer: the packed score layout is that of a causal mask")
-    x = None if fold_depad else torch.empty((1, T, hid), dtype=dt, device=dev)
-    offs = info.row_offsets(S, left_padded) if fold_depad else None
-    y = torch.empty((1, T, hid), dtype=dt, device=dev)
-    if ctx_out is None:
-        ctx_packed = torch.empty((1, T, H, D), dtype=dt, device=dev)
+    left = bool(left_padded)
+    fused_f32 = hidden_padded.dtype == torch.float32 and form in (1, 2)      # the fp32 kernel's tiles are not the table's
+    kv_bytes = 2 * S * D * hidden_padded.element_size()
+    table = None
+    if fold_depad and not fused_f32 and not info.ephemeral:
+        offs, table = info.layer_tables(S, left, H, kv_bytes)
     else:
-        _lib.require_gpu(ctx_out, "ctx_out")
-        if ctx_out.numel() != T * H * D or ctx_out.dtype != dt or not ctx_out.is_contiguous():
-            raise RuntimeError("padding_removal_layer: ctx_out must be a contiguous [1,T,H,D] tensor of the activation dtype")
-        ctx_packed = ctx_out
-    qkv = torch.empty((B, H, S, 3 * D), dtype=dt, device=dev) if form < 2 else None
-    ctx = torch.empty((B, H, S, D), dtype=dt, device=dev) if form < 2 else None
-    scores = None
-    if form in (0, 3):
-        scores = torch.empty((B, H, S, S), dtype=dt, device=dev)
-    elif form == 4:
-        scores = torch.empty(packed_scores_elems(B, H, S, dt), dtype=dt, device=dev)
-    with _lib.device_guard(hidden_padded):
-        _lib.check(_lib.fn.en_padding_removal_layer(
-            hidden_padded.data_ptr(), qkv_packed.data_ptr(), _lib.ptr(dense_out), gamma.data_ptr(), beta.data_ptr(),
-            _lib.ptr(x), _lib.ptr(qkv), _lib.ptr(scores), _lib.ptr(ctx), ctx_packed.data_ptr(), y.data_ptr(),
-            info.cu_seqlens.data_ptr(), info.lens.data_ptr(), B, S, H, D, hid, T, float(scale), float(eps),
-            int(bool(causal)), int(bool(left_padded)), form, _lib.ptr(offs),
-            _lib.dtype_tag(hidden_padded, "padding_removal_layer"),
-            info.tile_table_ptr(H, S, 2 * S * D * hidden_padded.element_size()),
-            _lib.stream_of(hidden_padded)), "padding_removal_layer")
-    return y
+        offs = info.row_offsets(S, left) if fold_depad else None
+        if not fused_f32 and not info.ephemeral:
+            table = info.tile_table(H, S, kv_bytes)
+    return _lib.front.layer(hidden_padded, qkv_packed, dense_out, gamma, beta, ctx_out, info.cu_seqlens, info.lens, offs, table,
+                            H, D, T, scale, eps, bool(causal), left, form)
 
 
 def padding_removal_layer_noalloc(hidden_padded: torch.Tensor, qkv_packed: torch.Tensor, seq_lens: torch.Tensor,
@@ -253,6 +219,8 @@ def decode_layer(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
     scale = float(D) ** -0.5 if scale is None else scale
     if single_pass is None:
         single_pass = not keep and scale > 0
+    if single_pass and not keep:
+        return _lib.front.decode_layer(q, k_cache, v_cache, info.lens, residual, gamma, beta, dense_out, eps, scale)
     probs = None
     if single_pass:
         ctx = decode_attn(q, k_cache, v_cache, info, scale=scale)

@@ -44,9 +44,7 @@ class SeqInfo:
         in the launching stream where they are complete."""
         if not self.lens.is_cuda:
             return
-        ev = torch.cuda.Event()
-        ev.record(torch.cuda.current_stream(self.lens.device))
-        self._ready.append(ev)
+        self._ready.append(_lib.front.record_event(self.lens))
         del self._ready[:-8]            # lengths that change every step rebuild their tables every step
         self._ordered = {_lib.stream_of(self.lens)}
 
@@ -58,9 +56,8 @@ class SeqInfo:
         raw = _lib.stream_of(self.lens)
         if raw in self._ordered:
             return
-        cur = torch.cuda.current_stream(self.lens.device)
         for ev in self._ready:
-            cur.wait_event(ev)
+            _lib.front.wait_event(ev, self.lens)
         self._ordered.add(raw)
 
     @property
@@ -114,6 +111,28 @@ class SeqInfo:
                 self._row_offsets = {k: o for k, o in self._row_offsets.items() if k[2] == version}
                 self._row_offsets[key] = off
         return off
+
+    def layer_tables(self, max_seq_len: int, left_padded: bool, head_num: int, unit_kv_bytes: int):
+        """``(row_offsets, tile_table)`` of a layer step (128-row tiles), built by one launch when the batch has neither."""
+        version = self._lens_version()
+        first = unit_kv_bytes <= TILES_FIRST_MAX_KV_BYTES
+        if self.cu_seqlens is None or (version is None and self._mutable()):
+            return self.row_offsets(max_seq_len, left_padded), self.tile_table(head_num, max_seq_len, unit_kv_bytes)
+        off_key, tab_key = (max_seq_len, left_padded, version), (head_num, max_seq_len, first, version, 128)
+        off, tab = self._row_offsets.get(off_key), self._tile_tables.get(tab_key)
+        if off is not None and tab is not None:
+            return off, tab
+        if off is not None or tab is not None:
+            return self.row_offsets(max_seq_len, left_padded), self.tile_table(head_num, max_seq_len, unit_kv_bytes)
+        self.order_current_stream()
+        off, tab = _lib.front.layer_tables(self.lens, self.cu_seqlens, self.batch_size, max_seq_len, left_padded, self.total,
+                                           head_num, first)
+        self.produced_on_current_stream()
+        self._row_offsets = {k: o for k, o in self._row_offsets.items() if k[2] == version}
+        self._row_offsets[off_key] = off
+        self._tile_tables = {k: t for k, t in self._tile_tables.items() if k[3] == version}
+        self._tile_tables[tab_key] = tab
+        return off, tab
 
     def _mutable(self) -> bool:
         """True when the lengths belong to a caller that may edit them in place (no prefix was computed from
@@ -175,15 +194,9 @@ def build_seq_info(seq_lens, batch_size: int, device=None, total: Optional[int] 
         if device is None:
             device = torch.device("cuda", torch.cuda.current_device())
         seq_lens = seq_lens.to(device, non_blocking=False)
-    seq_lens = seq_lens.contiguous()
-    lib = _lib.load()
-    with _lib.device_guard(seq_lens):
-        cu = torch.empty(batch_size + 1, dtype=torch.int32, device=seq_lens.device)
-        lens32 = torch.empty(batch_size, dtype=torch.int32, device=seq_lens.device)
-        _lib.check(lib.en_prefix_sum(seq_lens.data_ptr(), int(seq_lens.dtype == torch.int64), batch_size,
-                                     cu.data_ptr(), lens32.data_ptr(), _lib.stream_of(seq_lens)), "prefix_sum")
-        info = SeqInfo(lens32, cu, batch_size, total, source)
-        info.produced_on_current_stream()
+    cu, lens32 = _lib.front.prefix_sum(seq_lens.contiguous(), batch_size)
+    info = SeqInfo(lens32, cu, batch_size, total, source)
+    info.produced_on_current_stream()
     return info
 
 

@@ -262,6 +262,17 @@ int en_decode_attn(const void *q, const void *k_cache, const void *v_cache, void
                    int head_num, int k_seq_len, int size_per_head, const int64_t *k_strides, const int64_t *v_strides,
                    float scale, int dtype, void *workspace, int64_t workspace_bytes, en_stream_t stream);
 
+/* The decode step behind one call: en_decode_attn, then y = LayerNorm(input + residual) on the `batch` new tokens
+ * ([batch, hidden] rows), its input being dense_out or, with dense_out NULL (hidden == head_num * size_per_head), the
+ * context.  Where the keys of a unit are shared between workgroups and no projection follows, the combination of the
+ * shares is the LayerNorm's own first step: one launch less, and ctx (which is then not written) stays unrounded.
+ * out_dtype: type of gamma, beta and y, as in en_layernorm_fwd. */
+int en_decode_layer(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens, int batch,
+                    int head_num, int k_seq_len, int size_per_head, const int64_t *k_strides, const int64_t *v_strides,
+                    float scale, const void *dense_out, const void *residual, const void *gamma, const void *beta, void *y,
+                    int64_t hidden, float eps, int dtype, int out_dtype, void *workspace, int64_t workspace_bytes,
+                    en_stream_t stream);
+
 /* Appends the new token's K and V rows to [B,H,Smax,D] caches at position
  * kv_lens[b] (the caller then adds one to kv_lens); replaces the reference's
  * torch.cat of the whole projection history on every step
@@ -340,6 +351,10 @@ int en_attn_fused(const void *q, const void *k, const void *v, void *ctx, const 
 int64_t en_attn_tile_table_elems(int batch, int head_num, int q_seq_len, int query_tile);
 int en_attn_tile_table(const int32_t *seq_lens, int batch, int head_num, int q_seq_len, int tiles_first,
                        int query_tile, int32_t *table, en_stream_t stream);
+/* The tile table (128-row tiles) and the row offsets of en_padding_offsets in one launch, for a batch whose prefix
+ * sums exist: row_offsets gets cu_seqlens[batch] entries. */
+int en_layer_tables(const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int max_seq_len, int left_padded,
+                    int head_num, int tiles_first, int32_t *tile_table, int32_t *row_offsets, en_stream_t stream);
 
 /* ---- measurement helper ------------------------------------------------- */
 

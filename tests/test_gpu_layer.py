@@ -432,3 +432,54 @@ def test_padding_offsets_against_closed_form(left):
             row = b * S + (S - n if left else 0) + i
             want.append(row - len(want))
     assert got[:len(want)] == want
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,S,D", [
+    (1, 2, 1100, 64),       # 32 vectors of four channels on 1024 lanes
+    (3, 32, 1024, 128),     # exactly one vector per lane
+    (2, 33, 1030, 128),     # a second vector for some lanes
+    (5, 72, 2048, 128),     # 2.25 vectors
+    (1, 128, 1500, 128),    # four, the most the one-pass form takes
+    (1, 130, 1024, 128),    # wider: combine and LayerNorm as two launches
+    (2, 4, 300, 80),        # nothing is shared
+])
+def test_decode_layer_one_native_call(dtype, B, H, S, D):
+    """Decode step through ``en_decode_layer`` where the shares of a unit are combined inside the LayerNorm and where they
+    are not, against the float64 oracle; the LayerNorm bound is BASE plus half an ulp of the stored value."""
+    from energonai_amd import layer
+    announce("decode layer native", dtype, B, H, S, D)
+    g = torch.Generator().manual_seed(S + H)
+    kv = [S, 1, 513, 700, 64][:B] if B > 1 else [S - 3]
+    kv = [min(n, S) for n in kv]
+    q = torch.randn(B, H, 1, D, generator=g).to(dtype)
+    kc, vc = (torch.randn(B, H, S, D, generator=g).to(dtype) for _ in range(2))
+    res = torch.randn(1, B, H * D, generator=g).to(dtype)
+    gamma, beta = (1 + 0.02 * torch.randn(H * D, generator=g)).to(dtype), (0.02 * torch.randn(H * D, generator=g)).to(dtype)
+    _, _, ctx = eager.decode_attention(q, kc, vc, kv, D ** -0.5, acc_dtype=torch.float64)
+    want = torch.nn.functional.layer_norm(ctx.view(1, B, H * D) + res.double(), (H * D,), gamma.double(), beta.double(), 1e-5)
+    got = layer.decode_layer(q.cuda(), kc.cuda(), vc.cuda(), torch.tensor(kv, dtype=torch.int32).cuda(), res.cuda(), gamma.cuda(),
+                             beta.cuda(), 1e-5)
+    assert got.shape == want.shape
+    assert_stored_close(got.cpu(), want, dtype)
+    # a projection in between: its output takes the context's place
+    dense = torch.randn(1, B, H * D, generator=g).to(dtype)
+    got = layer.decode_layer(q.cuda(), kc.cuda(), vc.cuda(), torch.tensor(kv, dtype=torch.int32).cuda(), res.cuda(), gamma.cuda(),
+                             beta.cuda(), 1e-5, dense_out=dense.cuda())
+    want = torch.nn.functional.layer_norm(dense.double() + res.double(), (H * D,), gamma.double(), beta.double(), 1e-5)
+    assert_stored_close(got.cpu(), want, dtype)
+
+
+@pytest.mark.parametrize("lens,S,H,left", [([1], 17, 1, False), ([64, 0, 300, 7, 128, 129], 300, 5, True),
+                                           ([5] * 1030, 40, 2, False)])
+def test_layer_tables_in_one_launch(lens, S, H, left):
+    """Row offsets and tile table built together are the ones that their own kernels build."""
+    from energonai_amd.seqinfo import build_seq_info
+    announce("layer tables", len(lens), S, H, left)
+    t = torch.tensor(lens, dtype=torch.int32).cuda()
+    for kv_bytes in (1 << 10, 1 << 30):
+        both, one = build_seq_info(t, len(lens), total=sum(lens)), build_seq_info(t, len(lens), total=sum(lens))
+        off, tab = both.layer_tables(S, left, H, kv_bytes)
+        assert torch.equal(off[:sum(lens)], one.row_offsets(S, left)[:sum(lens)])
+        assert torch.equal(tab, one.tile_table(H, S, kv_bytes))
+        assert both.row_offsets(S, left) is off and both.tile_table(H, S, kv_bytes) is tab
