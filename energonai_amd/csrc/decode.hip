@@ -209,7 +209,10 @@ struct DecodeAttnArgs {
   // position s of sequence b in page page_table[b * max_pages + s / page] at row s % page
   const int32_t *page_table;
   int max_pages, lg_page, num_pages;
+  int len_add;        // 1: the newest token sits at position kv_lens[b] already, the length does not count it yet
 };
+
+__device__ __forceinline__ int cached_len(const DecodeAttnArgs &a, int b) { return max(min(a.kv_lens[b] + a.len_add, a.Sk), 0); }
 
 // Keys of one workgroup when nsplit share a unit: a multiple of 64, so that the keys of one wave (at most 16) never
 // straddle a share or a page.  The combine kernel derives the same shares from the length.
@@ -262,7 +265,7 @@ __global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeA
   int b = blockIdx.y;
   if (a.nsplit == 1 && a.B <= kRankBatch && a.B > 1) {
     // batch index whose length ranks blockIdx.y-th (longest first, ties by index)
-    for (int i = tid; i < a.B; i += NT) s_len[i] = min(a.kv_lens[i], a.Sk);
+    for (int i = tid; i < a.B; i += NT) s_len[i] = cached_len(a, i);
     __syncthreads();
     for (int i = tid; i < a.B; i += NT) {
       const int mine = s_len[i];
@@ -277,7 +280,7 @@ __global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeA
     b = s_b;
   }
   const int c = tid % LPK, g = tid / LPK;
-  const int kl = max(min(a.kv_lens[b], a.Sk), 0);
+  const int kl = cached_len(a, b);
   // with the keys of a unit split over nsplit workgroups this one takes [kbeg, kend); a share past the end has no
   // workgroup's worth of work and leaves no partial (the combine kernel derives the same shares from the length)
   const int share = split_share(kl, a.nsplit);
@@ -447,7 +450,7 @@ __device__ __forceinline__ void combine_shares(const DecodeAttnArgs &a, int b, i
       ml[i] = *partial_ml(a, share_index);
     }
     if (z0 == 0) {
-      const int kl = max(min(a.kv_lens[b], a.Sk), 0);
+      const int kl = cached_len(a, b);
       const int share = split_share(kl, a.nsplit);
       nvalid = share > 0 ? (kl + share - 1) / share : 0;       // shares that had keys
     }
@@ -744,6 +747,12 @@ __global__ __launch_bounds__(kBlock) void kv_fill_paged_kernel(PagedFillArgs a) 
   }
 }
 
+static int log2_exact(int v) {
+  int lg = 0;
+  while ((1 << lg) < v) ++lg;
+  return (1 << lg) == v ? lg : -1;
+}
+
 // Checks the arguments of the contiguous-cache entry points and fills the kernel's.
 static int attn_args(DecodeAttnArgs &a, const void *q, const void *k_cache, const void *v_cache, void *ctx,
                      const int32_t *kv_lens, int batch, int head_num, int k_seq_len, int size_per_head,
@@ -781,10 +790,60 @@ static int dispatch_attn_dtype(const DecodeAttnArgs &a, int dtype, hipStream_t s
   }
 }
 
-static int log2_exact(int v) {
-  int lg = 0;
-  while ((1 << lg) < v) ++lg;
-  return (1 << lg) == v ? lg : -1;
+static int paged_attn_args(DecodeAttnArgs &a, const void *q, const void *k_pool, const void *v_pool, void *ctx,
+                           const int32_t *kv_lens, const int32_t *page_table, int batch, int head_num, int max_pages_per_seq,
+                           int page_size, int num_pages, int size_per_head, const int64_t *k_strides, const int64_t *v_strides,
+                           float scale, int dtype, void *workspace, int64_t workspace_bytes) {
+  if (!k_strides || !v_strides || !v_pool || !page_table) return EN_ERR_NULL;
+  if (max_pages_per_seq < 1 || num_pages < 1) return EN_ERR_SHAPE;
+  const int lg = log2_exact(page_size);
+  if (lg < 4) return EN_ERR_UNSUPPORTED;                                  // a power of two, at least 16: a wave's keys share a page
+  if ((int64_t)max_pages_per_seq * page_size >= (1ll << 30)) return EN_ERR_SHAPE;
+  const int k_seq_len = max_pages_per_seq * page_size;
+  int rc = check_decode(q, k_pool, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
+                        k_strides[2], dtype);
+  if (rc) return rc;
+  const int es = dtype_size(dtype), epv = 16 / es;
+  if (!aligned_to(v_pool, 16) || (v_strides[0] % epv) || (v_strides[1] % epv) || (v_strides[2] % epv)) return EN_ERR_ALIGN;
+  if (!aligned_to(q, 16) || !aligned_to(ctx, es)) return EN_ERR_ALIGN;
+  if (size_per_head > 64 * epv) return EN_ERR_UNSUPPORTED;
+  // 32-bit byte offsets inside a page
+  if ((int64_t)page_size * k_strides[2] * es >= (1ll << 31) || (int64_t)page_size * v_strides[2] * es >= (1ll << 31))
+    return EN_ERR_UNSUPPORTED;
+  if (!(scale > 0.f)) return EN_ERR_UNSUPPORTED;
+  for (int i = 0; i < 3; ++i)
+    if (k_strides[i] < 0 || v_strides[i] < 0) return EN_ERR_UNSUPPORTED;
+  const int64_t need = en_decode_attn_workspace_bytes(batch, head_num, k_seq_len, size_per_head);
+  const bool split = need > 0 && workspace && workspace_bytes >= need && aligned_to(workspace, 16);
+  a = DecodeAttnArgs{q, k_pool, v_pool, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
+                     k_strides[2], v_strides[0], v_strides[1], v_strides[2], scale * 1.4426950408889634f,
+                     split ? decode_split(batch, head_num, k_seq_len) : 1, static_cast<float *>(workspace),
+                     page_table, max_pages_per_seq, lg, num_pages};
+  return EN_OK;
+}
+
+static int dispatch_paged_dtype(const DecodeAttnArgs &a, int dtype, hipStream_t s) {
+  const bool stream_cache = 2 * cache_bytes(a.B, a.H, a.Sk, a.D, dtype) >= kAttnStreamBytes;
+  switch (dtype) {
+    case EN_F32: return dispatch_attn<EN_F32, true>(a, stream_cache, s);
+    case EN_F16: return dispatch_attn<EN_F16, true>(a, stream_cache, s);
+    default: return dispatch_attn<EN_BF16, true>(a, stream_cache, s);
+  }
+}
+
+int decode_attn_ahead(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens,
+                      const int32_t *page_table, int batch, int head_num, int cache_len, int max_pages_per_seq, int page_size,
+                      int num_pages, int size_per_head, const int64_t *strides, float scale, int dtype, void *workspace,
+                      int64_t workspace_bytes, hipStream_t stream) {
+  DecodeAttnArgs a;
+  const int rc = page_table ? paged_attn_args(a, q, k_cache, v_cache, ctx, kv_lens, page_table, batch, head_num, max_pages_per_seq,
+                                              page_size, num_pages, size_per_head, strides, strides, scale, dtype, workspace,
+                                              workspace_bytes)
+                            : attn_args(a, q, k_cache, v_cache, ctx, kv_lens, batch, head_num, cache_len, size_per_head, strides,
+                                        strides, scale, dtype, workspace, workspace_bytes);
+  if (rc) return rc;
+  a.len_add = 1;
+  return page_table ? dispatch_paged_dtype(a, dtype, stream) : dispatch_attn_dtype(a, dtype, stream, true);
 }
 
 }  // namespace en
@@ -933,38 +992,10 @@ int en_decode_attn_paged(const void *q, const void *k_pool, const void *v_pool, 
                          int num_pages, int size_per_head, const int64_t *k_strides, const int64_t *v_strides, float scale,
                          int dtype, void *workspace, int64_t workspace_bytes, en_stream_t stream) {
   using namespace en;
-  if (!k_strides || !v_strides || !v_pool || !page_table) return EN_ERR_NULL;
-  if (max_pages_per_seq < 1 || num_pages < 1) return EN_ERR_SHAPE;
-  const int lg = log2_exact(page_size);
-  if (lg < 4) return EN_ERR_UNSUPPORTED;                                  // a power of two, at least 16: a wave's keys share a page
-  if ((int64_t)max_pages_per_seq * page_size >= (1ll << 30)) return EN_ERR_SHAPE;
-  const int k_seq_len = max_pages_per_seq * page_size;
-  int rc = check_decode(q, k_pool, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
-                        k_strides[2], dtype);
-  if (rc) return rc;
-  const int es = dtype_size(dtype), epv = 16 / es;
-  if (!aligned_to(v_pool, 16) || (v_strides[0] % epv) || (v_strides[1] % epv) || (v_strides[2] % epv)) return EN_ERR_ALIGN;
-  if (!aligned_to(q, 16) || !aligned_to(ctx, es)) return EN_ERR_ALIGN;
-  if (size_per_head > 64 * epv) return EN_ERR_UNSUPPORTED;
-  // 32-bit byte offsets inside a page
-  if ((int64_t)page_size * k_strides[2] * es >= (1ll << 31) || (int64_t)page_size * v_strides[2] * es >= (1ll << 31))
-    return EN_ERR_UNSUPPORTED;
-  if (!(scale > 0.f)) return EN_ERR_UNSUPPORTED;
-  for (int i = 0; i < 3; ++i)
-    if (k_strides[i] < 0 || v_strides[i] < 0) return EN_ERR_UNSUPPORTED;
-  const int64_t need = en_decode_attn_workspace_bytes(batch, head_num, k_seq_len, size_per_head);
-  const bool split = need > 0 && workspace && workspace_bytes >= need && aligned_to(workspace, 16);
-  DecodeAttnArgs a{q, k_pool, v_pool, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
-                   k_strides[2], v_strides[0], v_strides[1], v_strides[2], scale * 1.4426950408889634f,
-                   split ? decode_split(batch, head_num, k_seq_len) : 1, static_cast<float *>(workspace),
-                   page_table, max_pages_per_seq, lg, num_pages};
-  const bool stream_cache = 2 * cache_bytes(batch, head_num, k_seq_len, size_per_head, dtype) >= kAttnStreamBytes;
-  hipStream_t s = (hipStream_t)stream;
-  switch (dtype) {
-    case EN_F32: return dispatch_attn<EN_F32, true>(a, stream_cache, s);
-    case EN_F16: return dispatch_attn<EN_F16, true>(a, stream_cache, s);
-    default: return dispatch_attn<EN_BF16, true>(a, stream_cache, s);
-  }
+  DecodeAttnArgs a;
+  const int rc = paged_attn_args(a, q, k_pool, v_pool, ctx, kv_lens, page_table, batch, head_num, max_pages_per_seq, page_size,
+                                 num_pages, size_per_head, k_strides, v_strides, scale, dtype, workspace, workspace_bytes);
+  return rc ? rc : dispatch_paged_dtype(a, dtype, (hipStream_t)stream);
 }
 
 int en_decode_qk(const void *q, const void *k_cache, void *scores, const int32_t *kv_lens, int batch, int head_num,

@@ -261,6 +261,72 @@ PyObject *decode_layer(PyObject *const *a) {
   return THPVariable_Wrap(y);
 }
 
+// block_decode(hidden, norm1 w, b, eps, qkv w, b, dense w, b, norm2 w, b, eps, mlp1 w, b, mlp2 w, b, activation, heads, scale,
+//              k_cache, v_cache, lens, page_table or None, cache_len, out [B, positions, hidden], position)
+// -> out[:, :position + 1] with the block's output for the newest position of `hidden` at `position`, or None, with nothing
+// done, where en_block_decode has no kernel for these tensors.
+PyObject *block_decode(PyObject *const *a) {
+  const Tensor &x = gpu(a[0], "hidden_states", false);
+  const Tensor &out = gpu(a[23], "out", false);
+  const Tensor &k = gpu(a[18], "k_cache", false), &v = gpu(a[19], "v_cache", false), &lens = gpu(a[20], "lens");
+  const auto dt = x.scalar_type();
+  const int64_t heads = integer(a[16]);
+  if ((dt != at::kHalf && dt != at::kBFloat16) || x.dim() != 3 || x.stride(2) != 1 || out.scalar_type() != dt || out.stride(2) != 1 ||
+      k.scalar_type() != dt || k.dim() != 4 || k.stride(3) != 1 || v.sizes() != k.sizes() || v.strides() != k.strides())
+    Py_RETURN_NONE;
+  const int64_t B = x.size(0), hid = x.size(2), D = k.size(3), position = integer(a[24]);
+  if (heads * D != hid || k.size(1) != heads || out.size(0) != B || out.size(2) != hid || position < 0 || position >= out.size(1) ||
+      lens.numel() != B || lens.scalar_type() != at::kInt)
+    Py_RETURN_NONE;
+  bool usable = true;
+  auto weight = [&](int i, int64_t rows, int64_t cols) -> const void * {
+    if (a[i] == Py_None) return nullptr;
+    const Tensor &t = tensor(a[i], "weight");
+    if (!t.is_cuda() || t.device() != x.device() || t.scalar_type() != dt || !t.is_contiguous() || t.numel() != rows * cols) usable = false;
+    return t.data_ptr();
+  };
+  const Tensor &w1 = tensor(a[11], "weight");
+  if (w1.dim() != 2) Py_RETURN_NONE;
+  const int64_t mlp = w1.size(0);
+  en_block_decode_args p{};
+  p.x = static_cast<const char *>(x.data_ptr()) + (x.size(1) - 1) * x.stride(1) * 2;
+  p.x_stride = B > 1 ? x.stride(0) : hid;
+  p.norm1_weight = weight(1, 1, hid); p.norm1_bias = weight(2, 1, hid); p.norm1_eps = real(a[3]);
+  p.qkv_weight = weight(4, 3 * hid, hid); p.qkv_bias = weight(5, 1, 3 * hid);
+  p.dense_weight = weight(6, hid, hid); p.dense_bias = weight(7, 1, hid);
+  p.norm2_weight = weight(8, 1, hid); p.norm2_bias = weight(9, 1, hid); p.norm2_eps = real(a[10]);
+  p.mlp1_weight = weight(11, mlp, hid); p.mlp1_bias = weight(12, 1, mlp);
+  p.mlp2_weight = weight(13, hid, mlp); p.mlp2_bias = weight(14, 1, hid);
+  if (!usable) Py_RETURN_NONE;
+  p.activation = (int)integer(a[15]);
+  p.scale = real(a[17]);
+  p.dtype = dtype_tag(x, "block_decode");
+  p.batch = (int)B; p.head_num = (int)heads; p.size_per_head = (int)D; p.mlp_width = mlp;
+  p.k_cache = k.data_ptr(); p.v_cache = v.data_ptr();
+  for (int i = 0; i < 3; ++i) p.cache_strides[i] = k.stride(i);
+  p.cache_len = (int)integer(a[22]);
+  p.kv_lens = lens.data_ptr<int32_t>();
+  if (a[21] != Py_None) {
+    const Tensor &table = gpu(a[21], "page_table");
+    if (table.scalar_type() != at::kInt || table.dim() != 2 || table.size(0) != B) Py_RETURN_NONE;
+    p.page_table = i32(table);
+    p.max_pages_per_seq = (int)table.size(1); p.page_size = (int)k.size(2); p.num_pages = (int)k.size(0);
+  } else if (k.size(0) != B || k.size(2) != p.cache_len) {
+    Py_RETURN_NONE;
+  }
+  p.y = static_cast<char *>(out.data_ptr()) + position * out.stride(1) * 2;
+  p.y_stride = out.stride(0);
+  const c10::DeviceGuard guard(x.device());
+  p.workspace_bytes = en_block_decode_workspace_bytes(p.batch, p.head_num, p.size_per_head, p.mlp_width, p.cache_len);
+  const Tensor ws = at::empty({p.workspace_bytes}, x.options().dtype(at::kByte));
+  p.workspace = ws.data_ptr();
+  const int rc = without_gil([&] { return en_block_decode(&p, stream_of(x)); });
+  if (rc == EN_ERR_UNSUPPORTED || rc == EN_ERR_ALIGN) Py_RETURN_NONE;      // found before anything was launched
+  check(rc, "block_decode");
+  if (!lens.is_inference()) lens.unsafeGetTensorImpl()->bump_version();      // the lengths have moved on
+  return THPVariable_Wrap(out.narrow(1, 0, position + 1));
+}
+
 // ---- module --------------------------------------------------------------------------------------------------------
 
 template <PyObject *(*F)(PyObject *const *), int N>
@@ -291,6 +357,7 @@ PyMethodDef kMethods[] = {
     EN_FAST(layer_tables, 8, "(row offsets, tile table) of a batch"),
     EN_FAST(layer, 18, "en_padding_removal_layer on new outputs"),
     EN_FAST(decode_layer, 10, "en_decode_layer on new outputs"),
+    EN_FAST(block_decode, 25, "en_block_decode into a position of an output history"),
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_front", "host side of the layer and decode steps", -1, kMethods};

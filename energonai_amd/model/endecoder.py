@@ -10,11 +10,13 @@ from typing import Callable, Optional
 import torch
 from torch import nn
 
+from .. import _lib
 from ..kernel import LayerNorm, depad, layer_norm_forward, repad
 from ..seqinfo import SeqInfo, seq_info
 from .attention import MultiHeadAttention1D, lens_from_mask
+from .gemm import gemm_tuning
 from .kv_cache import OutputHistory
-from .mlp import MLP1D
+from .mlp import MLP1D, activation_code
 
 
 class Block1D(nn.Module):
@@ -51,6 +53,41 @@ class Block1D(nn.Module):
                                     self.norm2.normalized_shape, self.norm2.eps, residual=x, return_sum=True)
         return s1 + self.mlp.forward_rows(h2)
 
+    def _native_decode(self, hidden_states) -> Optional[torch.Tensor]:
+        """One decode step of a pre-LN block of plain modules as ``en_block_decode``: five launches, the output written
+        straight into the history.  ``None``, with nothing done, where it does not apply (post-LN, separate q, k, v
+        projections, gradients, autocast or tuned GEMMs asked for, modules replaced or hooked, shapes without a kernel)."""
+        m = self._modules
+        attn, mlp, norm1, norm2 = m["attn"], m["mlp"], m["norm1"], m["norm2"]
+        if self.apply_post_layernorm or type(self)._rows is not Block1D._rows or type(attn) is not MultiHeadAttention1D \
+                or type(mlp) is not MLP1D or type(norm1) is not LayerNorm or type(norm2) is not LayerNorm or not attn.fused_qkv \
+                or attn.kv_cache is None or hidden_states.dim() != 3 or torch.is_grad_enabled() or torch.is_autocast_enabled() \
+                or gemm_tuning():
+            return None
+        am, mm = attn._modules, mlp._modules
+        qkv, dense, fc1, fc2 = am["query_key_value"], am["dense"], mm["dense_1"], mm["dense_2"]
+        for sub in (qkv, dense, fc1, fc2):
+            if type(sub) is not nn.Linear:
+                return None
+        for sub in (attn, mlp, norm1, norm2, qkv, dense, fc1, fc2):
+            if sub._forward_hooks or sub._forward_pre_hooks:
+                return None
+        act = activation_code(mlp.activation)
+        if act is None:
+            return None
+        cache, history = attn.kv_cache, self._history
+        cache.prepare_append()
+        buf = history.reserve()
+        p1, p2, pq, pd, pf, pg = (sub._parameters for sub in (norm1, norm2, qkv, dense, fc1, fc2))
+        out = _lib.front.block_decode(hidden_states, p1["weight"], p1["bias"], norm1.eps, pq["weight"], pq["bias"], pd["weight"],
+                                      pd["bias"], p2["weight"], p2["bias"], norm2.eps, pf["weight"], pf["bias"], pg["weight"],
+                                      pg["bias"], act, attn.num_heads, attn.scaling, cache.k, cache.v, cache.lens,
+                                      cache.page_table, cache.max_seq_len, buf, history.cur)
+        if out is not None:
+            cache.appended()
+            history.cur += 1
+        return out
+
     def forward_packed(self, x: torch.Tensor, info: SeqInfo, batch_size: int, max_seq_len: int,
                        fill_cache: bool = False) -> torch.Tensor:
         """``[1,T,hid]`` valid tokens in, ``[1,T,hid]`` out: lets a model drop the padding once
@@ -60,6 +97,9 @@ class Block1D(nn.Module):
     def forward(self, hidden_states, attention_mask=None, first_cache=False, seq_lens=None):
         B, S, hid = hidden_states.shape
         if not self.disable_past_cache and not first_cache:
+            out = self._native_decode(hidden_states)
+            if out is not None:
+                return out
             return self._history.push(self._rows(hidden_states[:, -1:, :].contiguous(), self.attn.forward_last))
         if seq_lens is None:
             seq_lens = lens_from_mask(attention_mask) if attention_mask is not None else \

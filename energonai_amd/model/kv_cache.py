@@ -42,14 +42,23 @@ class KVCache:
         # caller has the true maximum on the host
         self._longest = self.max_seq_len if longest is None else min(int(longest), self.max_seq_len)
 
-    def append(self, k_new: torch.Tensor, v_new: torch.Tensor) -> None:
-        """One new ``[B,H,D]`` row per sequence; lengths advance by one.  Raises when a sequence may already
-        fill the cache: the kernel would drop its new row and decoding would go on without the newest token
+    page_table = None       # one buffer per sequence
+
+    def prepare_append(self) -> None:
+        """The host's side of one more position per sequence, before its rows are written.  Raises when a sequence may
+        already fill the cache: the kernel would drop its new row and decoding would go on without the newest token
         (the reference's torch.cat cache grows instead, energonai/model/attention.py:66-71)."""
         if self._longest >= self.max_seq_len:
             raise RuntimeError(f"KVCache.append: the cache holds max_seq_len = {self.max_seq_len} positions and a "
                                f"sequence may already be that long; allocate the cache for prompt + generated tokens")
+
+    def appended(self) -> None:
         self._longest += 1
+
+    def append(self, k_new: torch.Tensor, v_new: torch.Tensor) -> None:
+        """One new ``[B,H,D]`` row per sequence; lengths advance by one (see ``prepare_append``)."""
+        self.prepare_append()
+        self.appended()
         kv_cache_append(k_new, v_new, self.k, self.v, self.info)
         self.lens.add_(1)
 
@@ -141,14 +150,27 @@ class PagedKVCache:
         self.lens.copy_(info.lens)
         self._host_lens = lens_host
 
-    def append(self, k_new: torch.Tensor, v_new: torch.Tensor) -> None:
-        """One new ``[B,H,D]`` row per sequence; lengths advance by one.  A sequence whose length sits on a page
-        boundary is given a page first (raises when the pool or the sequence's table row is full)."""
+    @property
+    def page_table(self):
+        return self.table
+
+    def prepare_append(self) -> None:
+        """Gives a sequence whose length sits on a page boundary its next page (raises when the pool or the
+        sequence's table row is full)."""
         P = self.page_size
-        self._assign([(b, n // P + 1) for b, n in enumerate(self._host_lens) if n % P == 0])
+        wants = [(b, n // P + 1) for b, n in enumerate(self._host_lens) if n % P == 0]
+        if wants:
+            self._assign(wants)
+
+    def appended(self) -> None:
+        self._host_lens = [n + 1 for n in self._host_lens]
+
+    def append(self, k_new: torch.Tensor, v_new: torch.Tensor) -> None:
+        """One new ``[B,H,D]`` row per sequence; lengths advance by one (see ``prepare_append``)."""
+        self.prepare_append()
         kv_pages_append(k_new, v_new, self.k, self.v, self.info, self.table)
         self.lens.add_(1)
-        self._host_lens = [n + 1 for n in self._host_lens]
+        self.appended()
 
     def attend(self, q: torch.Tensor, scale: float) -> torch.Tensor:
         return decode_attn_paged(q, self.k, self.v, self.info, self.table, scale=scale)
@@ -171,7 +193,8 @@ class OutputHistory:
         self.cur = S
         return self.buf[:, :S]
 
-    def push(self, new: torch.Tensor) -> torch.Tensor:
+    def reserve(self) -> torch.Tensor:
+        """The buffer, with room at position ``cur``."""
         if self.buf is None:
             raise RuntimeError("decode step before a first_cache=True call")
         if self.cur == self.buf.shape[1]:      # past the planned length: grow geometrically
@@ -179,6 +202,10 @@ class OutputHistory:
                                 device=self.buf.device)
             grown[:, :self.cur].copy_(self.buf)
             self.buf = grown
+        return self.buf
+
+    def push(self, new: torch.Tensor) -> torch.Tensor:
+        self.reserve()
         self.buf[:, self.cur:self.cur + 1].copy_(new)
         self.cur += 1
         return self.buf[:, :self.cur]

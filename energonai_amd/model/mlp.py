@@ -22,6 +22,13 @@ def _epilogue_of(activation) -> Optional[str]:
     return None
 
 
+def activation_code(activation) -> Optional[int]:
+    """The ``en_activation`` that computes ``activation`` exactly, if there is one."""
+    if activation is nn.functional.gelu or (isinstance(activation, nn.GELU) and activation.approximate == "none"):
+        return 3
+    return {"relu": 1, "gelu_tanh": 2}.get(_epilogue_of(activation))
+
+
 class MLP1D(nn.Module):
 
     def __init__(self, hidden_size: int, mlp_ratio: float, activation: Callable, dtype: torch.dtype = torch.float16,

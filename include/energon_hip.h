@@ -356,6 +356,39 @@ int en_attn_tile_table(const int32_t *seq_lens, int batch, int head_num, int q_s
 int en_layer_tables(const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int max_seq_len, int left_padded,
                     int head_num, int tiles_first, int32_t *tile_table, int32_t *row_offsets, en_stream_t stream);
 
+/* ---- one decode step of a pre-LN transformer block -------------------------------------------------------------------
+ *
+ *   s = x + Wd attention(LN1(x)) + bd,   y = s + W2 act(W1 LN2(s) + b1) + b2          (energonai/model/endecoder.py:48-70)
+ *
+ * for the newest token of up to 32 sequences, fp16 or bf16, hidden = head_num * size_per_head of up to 2048 channels: five
+ * launches (seven where attention shares a unit's keys between workgroups).  The new K and V rows go to position kv_lens[b]
+ * of the caches, attention sees them, and kv_lens is advanced by one; a sequence without room keeps its rows and loses the
+ * new one (en_kv_append).  Weights are [out, in] as torch.nn.Linear holds them, the fused projection's outputs ordered
+ * k, v, q (attention.py:74); biases may be NULL.  s stays fp32 between its two uses. */
+enum en_activation { EN_ACT_NONE = 0, EN_ACT_RELU = 1, EN_ACT_GELU_TANH = 2, EN_ACT_GELU = 3 };
+typedef struct en_block_decode_args {
+  const void *x;              /* [batch] rows of hidden, x_stride elements apart */
+  int64_t x_stride;
+  const void *norm1_weight, *norm1_bias, *qkv_weight, *qkv_bias, *dense_weight, *dense_bias;
+  const void *norm2_weight, *norm2_bias, *mlp1_weight, *mlp1_bias, *mlp2_weight, *mlp2_bias;
+  float norm1_eps, norm2_eps, scale;
+  int activation;             /* en_activation */
+  int dtype, batch, head_num, size_per_head;
+  int64_t mlp_width;
+  void *k_cache, *v_cache;    /* [batch, head_num, cache_len, size_per_head] or pools of pages */
+  int64_t cache_strides[3];   /* batch (pages: page), head, position, in elements */
+  int cache_len;              /* positions a sequence can hold (pages: max_pages_per_seq * page_size) */
+  int32_t *kv_lens;
+  const int32_t *page_table;  /* NULL: contiguous caches */
+  int max_pages_per_seq, page_size, num_pages;
+  void *y;                    /* [batch] rows of hidden, y_stride elements apart */
+  int64_t y_stride;
+  void *workspace;            /* 16-byte aligned, en_block_decode_workspace_bytes */
+  int64_t workspace_bytes;
+} en_block_decode_args;
+int64_t en_block_decode_workspace_bytes(int batch, int head_num, int size_per_head, int64_t mlp_width, int cache_len);
+int en_block_decode(const en_block_decode_args *args, en_stream_t stream);
+
 /* ---- measurement helper ------------------------------------------------- */
 
 /* The whole step in one call: depad, transpose_pad, QK^T, scale_mask_softmax, PV,

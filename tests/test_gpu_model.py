@@ -325,3 +325,48 @@ def test_block_random_shapes(seed):
         got = blk(x.cuda(), attention_mask=mask.to(dtype).cuda(), first_cache=False).float().cpu()
         want = models.block_forward(x, p, heads, 1e-5, post, True, mask, activation=act, fused_qkv=fused_qkv)
         assert max_abs(got[:, -1], want[:, -1]) <= tol * ref_scale, step
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,heads,D,ratio,act,bias,page", [
+    (1, 1, 64, 4.0, "relu", True, None),          # one row, one step of 64 channels
+    (3, 12, 64, 4.0, "gelu", True, 16),           # 768 channels: three steps on four waves; pages
+    (16, 3, 80, 4.0, "gelu_tanh", True, None),    # a full row tile; 240 channels end inside a step
+    (17, 5, 40, 2.6, "relu", False, None),        # a second row tile of one row; 200 channels, no bias, an odd MLP width
+    (32, 8, 128, 1.0, "relu", True, 32),          # the most rows; 1024 channels
+    (2, 16, 128, 4.0, "gelu", True, None),        # 2048 channels, 8192 in the MLP
+    (2, 17, 128, 1.0, "relu", True, None),        # too wide: the general path
+    (33, 2, 64, 1.0, "relu", True, None),         # too many rows: the general path
+])
+def test_block_decode_in_one_native_call(dtype, B, heads, D, ratio, act, bias, page):
+    """Decode steps of a pre-LN block through ``en_block_decode`` (where it applies) against the block recomputed over the
+    whole extended batch in fp32, at the tolerance of the block's general path; lengths, caches and history move on alike."""
+    _, M = _mods()
+    hid, S = heads * D, 20
+    fn = {"relu": F.relu, "gelu": F.gelu, "gelu_tanh": torch.nn.GELU(approximate="tanh")}[act]
+    announce("block decode native", dtype, B, heads, D, ratio, act, bias, page)
+    blk = M.Block1D(hid, heads, ratio, activation=fn, dtype=dtype, bias=bias, max_seq_len=32, kv_page_size=page).cuda()
+    _init(blk, 41)
+    p = _fp32_params(blk)
+    lens = [S - (3 * b) % S for b in range(B)]
+    x, valid = _padded_batch(B, S, hid, lens, True, dtype, 42)
+    g = torch.Generator().manual_seed(43)
+    tol = {torch.float16: 1.5e-2, torch.bfloat16: 1.2e-1}[dtype]
+    with torch.no_grad():
+        blk(x.cuda(), attention_mask=models.additive_mask(valid).to(dtype).cuda(), first_cache=True)
+        native = B <= 32 and hid <= 2048
+        if native:      # the call itself must be what runs: with it in place the general path is never entered
+            blk.attn.forward_last = None
+        for step in range(3):
+            new = torch.randn(B, 1, hid, generator=g).to(dtype)
+            x, valid = torch.cat((x, new), 1), torch.cat((valid, torch.ones(B, 1)), 1)
+            before = blk.attn.kv_cache.lens._version
+            # the newest position of a longer, strided view, as the block before hands it on
+            wide = torch.zeros(B, 3, hid + 8, dtype=dtype)
+            wide[:, 2:, :hid] = new
+            got = blk(wide.cuda()[:, :, :hid], first_cache=False)
+            want = models.block_forward(x, p, heads, 1e-5, False, True, models.additive_mask(valid), activation=fn)
+            assert got.shape == want.shape
+            assert max_abs(got[:, -1].float().cpu(), want[:, -1]) <= tol, step
+            assert blk.attn.kv_cache.lens.tolist() == [n + step + 1 for n in lens]
+            assert blk.attn.kv_cache.lens._version > before
