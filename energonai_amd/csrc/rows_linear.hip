@@ -4,18 +4,16 @@
 //
 //   y = act(LayerNorm(x) W^T + b) (+ residual)         x [R,K], W [N,K] (torch.nn.Linear's layout), R <= 32
 //
-// What bounds it: for narrow models the chain launch -> first weight bytes -> last MFMA -> store (3.5..5 us a kernel, of
-// which 2.8 are an empty launch), for wide ones the weights' bytes.  So a workgroup takes 16 output columns only (N / 16
-// workgroups) and its waves split K between them, 64 channels a step: every lane's weight loads of the first steps are
-// sent for before anything is waited for, each wave needs few steps (three for K = 768 on four waves), and the partial
-// sums meet once, in LDS.  W rows are the A operand of the 16x16x32 MFMA (lane j of 16 holds row n0 + j, 32 bytes = 16
-// channels of it per step: the four lane groups together 128 contiguous bytes a row), the x rows the B operand with the
-// same channel order, so the result leaves each lane with four consecutive columns of one row.
+// What bounds it: for narrow models the chain launch -> first weight bytes -> last MFMA -> store, for wide ones the bytes of
+// the weights.  So a workgroup takes few output columns (eight or sixteen a tile) and its waves split K between them, 64 or
+// 128 channels a step: every lane's weight loads of the first steps are sent for before anything is waited for, each wave
+// needs few steps, and the partial sums meet once, in LDS.  W rows are the A operand of the 16x16x32 MFMA (lane j of 16 holds
+// row n0 + j, 32 bytes = 16 channels of it per step: the four lane groups together 128 contiguous bytes a row), the x rows
+// the B operand with the same channel order, so the result leaves each lane with four consecutive columns of one row.
 //
-// The LayerNorm in front of a projection is computed where its result is consumed: 16 lanes per row take mean and centred
-// squares (two passes, fp32), and the B fragments are normalised and rounded to the storage type as they are loaded,
-// exactly what a LayerNorm kernel would have stored.  Every workgroup repeats the statistics, so this is for rows of up to
-// kMaxWidth channels.
+// The LayerNorm in front of a projection is computed where its result is consumed: the B fragments of all waves together
+// are the rows, so mean and centred squares (fp32) come from registers, and each fragment is normalised and rounded to the
+// storage type, exactly what a LayerNorm kernel would have stored.  That takes rows that fit: up to kMaxWidth channels.
 #include "common.hip.h"
 
 #include <math.h>
@@ -71,138 +69,178 @@ __device__ __forceinline__ float activate(float v, int act) {
   }
 }
 
-template <int DT, int IN, int OUT, int NW, int RT>
+// RT: row tiles.  1, 2: sixteen rows each, sixteen columns per column tile, a step is 64 channels.  0: up to eight rows.  The
+// MFMA's sixteen A rows are then eight columns at the lower and the same eight at the upper half of a step of 128 channels,
+// its sixteen B columns the eight rows at those halves; the two quadrants where the halves meet are the result and the other
+// two are dropped.  No lane loads a row that is not there, and a column tile of eight makes twice the workgroups.
+// CT: column tiles per workgroup.
+template <int DT, int IN, int OUT, int NW, int U, int RT, int CT>
 __global__ __launch_bounds__(NW * kWave) void rows_linear_kernel(RowsArgs a) {
   typedef Elem<DT> E;
   typedef typename E::T T;
   typedef Pack<T, 8> P8;
-  constexpr int BK = 64;                        // channels per wave and step: two MFMAs
-  constexpr int U = RT == 1 ? 3 : 2;            // steps in flight
+  constexpr bool HALF = RT == 0;
+  constexpr int RTILES = HALF ? 1 : RT;
+  constexpr int ROWS = HALF ? 8 : 16;           // rows per row tile, columns per column tile
+  constexpr int BK = HALF ? 128 : 64;           // channels per wave and step: two MFMAs per tile
   constexpr int XV = IN == kNormF32 ? 4 : 2;    // 16-byte loads of 16 channels of a row
   constexpr bool NORM = IN != kPlain;
-  __shared__ __attribute__((aligned(16))) float s_acc[NW][RT][kWave][4];
-  __shared__ float s_mu[RT * 16], s_inv[RT * 16];
+  constexpr bool AFFINE_EARLY = NORM && RTILES == 1 && CT == 1;   // gamma and beta travel with the weights where registers allow
+  __shared__ __attribute__((aligned(16))) float s_acc[NW][RTILES * CT][kWave][4];
+  __shared__ float s_sum[NORM ? 2 : 1][NW][RTILES * 16];
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int j = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16;
+  const int jr = HALF ? (j & 7) : j;            // row of the tile and column of the tile that this lane loads
+  const int kl = (HALF ? (j >> 3) * 64 : 0) + g * 16;   // its 16 channels of a step
+  const int n0 = blockIdx.x * ROWS * CT;
   const int nsteps = (a.K + BK - 1) / BK;
 
-  const T *wrow = reinterpret_cast<const T *>(a.w) + (int64_t)min(n0 + j, a.N - 1) * a.K;
-  const unsigned char *xrow[RT];
+  // Bounds-checked buffer loads: columns past N, rows past R, channels past K and steps past the end arrive as zeros without
+  // a branch (branches around the loads, each with its own wait, cost a factor of 2.5).
+  constexpr int XS = IN == kNormF32 ? 4 : 2;
+  const rsrc_t w_rsrc = make_rsrc(reinterpret_cast<const T *>(a.w) + (int64_t)n0 * a.K, (uint32_t)min(ROWS * CT, a.N - n0) * (uint32_t)a.K * 2u);
+  const rsrc_t x_rsrc = make_rsrc(a.x, (uint32_t)(((int64_t)(a.R - 1) * a.x_stride + a.K) * XS));
+  const rsrc_t g_rsrc = make_rsrc(a.gamma, NORM ? (uint32_t)a.K * 2u : 0u), b_rsrc = make_rsrc(a.beta, NORM ? (uint32_t)a.K * 2u : 0u);
+  uint32_t xrow[RTILES];
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
-    xrow[t] = reinterpret_cast<const unsigned char *>(a.x) + (int64_t)min(t * 16 + j, a.R - 1) * a.x_stride * (IN == kNormF32 ? 4 : 2);
-  const T *gamma = reinterpret_cast<const T *>(a.gamma), *beta = reinterpret_cast<const T *>(a.beta);
+  for (int t = 0; t < RTILES; ++t) xrow[t] = t * 16 + jr < a.R ? (uint32_t)((int64_t)(t * 16 + jr) * a.x_stride * XS) : kOutOfRange;
 
-  uint4 w[U][2], x[U][RT][XV], ga[NORM ? U : 1][2], be[NORM ? U : 1][2];
-  auto fetch = [&](int u, int step) {           // a step past the end, and channels past K, arrive as zeros
-    const int k = step * BK + g * 16;
+  uint4 w[U][CT][2], x[U][RTILES][XV], ga[AFFINE_EARLY ? U : 1][2], be[AFFINE_EARLY ? U : 1][2];
+  auto load_affine = [&](int slot, int half, int k) {
+    ga[slot][half] = buffer_load16(g_rsrc, (uint32_t)(k + 8 * half) * 2u);
+    be[slot][half] = buffer_load16(b_rsrc, (uint32_t)(k + 8 * half) * 2u);
+  };
+  auto fetch = [&](int u, int step) {
+    const int k = step * BK + kl;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
-      const bool in = k + 8 * half < a.K;
-      w[u][half] = in ? load16<false>(wrow + k + 8 * half) : make_uint4(0, 0, 0, 0);
-      if constexpr (NORM) {
-        ga[u][half] = in ? load16<false>(gamma + k + 8 * half) : make_uint4(0, 0, 0, 0);
-        be[u][half] = in ? load16<false>(beta + k + 8 * half) : make_uint4(0, 0, 0, 0);
-      }
+      const uint32_t in = k + 8 * half < a.K ? 0u : kOutOfRange;
 #pragma unroll
-      for (int t = 0; t < RT; ++t)
+      for (int c = 0; c < CT; ++c)
+        w[u][c][half] = buffer_load16(w_rsrc, ((uint32_t)(c * ROWS + jr) * (uint32_t)a.K + (uint32_t)(k + 8 * half)) * 2u | in);
+#pragma unroll
+      for (int t = 0; t < RTILES; ++t)
 #pragma unroll
         for (int v = 0; v < XV / 2; ++v)
-          x[u][t][half * (XV / 2) + v] = in ? load16<false>(xrow[t] + (int64_t)(k + 8 * half) * (XV / 2) * 2 + v * 16) : make_uint4(0, 0, 0, 0);
+          x[u][t][half * (XV / 2) + v] = buffer_load16(x_rsrc, xrow[t] + (uint32_t)(k + 8 * half) * XS + v * 16 | xrow[t] & kOutOfRange | in);
+      if constexpr (AFFINE_EARLY) load_affine(u, half, k);
     }
   };
 #pragma unroll
   for (int u = 0; u < U; ++u) fetch(u, wave + u * NW);
 
-  float mu[RT], inv[RT];
+  // element e of the 16 channels that this lane holds of row tile t in step u
+  auto x_at = [&](int u, int t, int e) {
+    if constexpr (IN == kNormF32) return __builtin_bit_cast(Pack<float, 4>, x[u][t][e / 4]).v[e % 4];
+    else return E::to_float(__builtin_bit_cast(P8, x[u][t][e / 8]).v[e % 8]);
+  };
+  float mu[RTILES], inv[RTILES];
   if constexpr (NORM) {
-    constexpr int EX = IN == kNormF32 ? 4 : 8;  // elements per 16-byte vector of a row
-    constexpr int UV = 8;                       // vectors in flight per lane
-    for (int r = tid / 16; r < a.R; r += NW * 4) {
-      const unsigned char *row = reinterpret_cast<const unsigned char *>(a.x) + (int64_t)r * a.x_stride * (16 / EX);
-      const int nvec = a.K / EX;
-      auto pass = [&](auto &&f) {
-        for (int v0 = j; v0 < nvec; v0 += 16 * UV) {
-          uint4 q[UV];
+    // The U steps of the NW waves are the whole row (the host sees to it): mean and centred squares come from the fragments
+    // in registers, over the lane groups by permlane swaps and over the waves through LDS.
+    auto row_sum = [&](float (&v)[RTILES], float (&slots)[NW][RTILES * 16]) {
 #pragma unroll
-          for (int i = 0; i < UV; ++i)
-            if (v0 + 16 * i < nvec) q[i] = load16<false>(row + (int64_t)(v0 + 16 * i) * 16);
+      for (int t = 0; t < RTILES; ++t) {
+        float f = v[t];
+        if constexpr (HALF) f += dpp_move<0x128>(f);        // row_ror:8, the other half of the step
+        auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(f), __float_as_uint(f), false, false);
+        f = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        r = __builtin_amdgcn_permlane32_swap(__float_as_uint(f), __float_as_uint(f), false, false);
+        f = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        if (g == 0) slots[wave][t * 16 + j] = f;
+      }
+      __syncthreads();
 #pragma unroll
-          for (int i = 0; i < UV; ++i)
-            if (v0 + 16 * i < nvec) {
-              if constexpr (IN == kNormF32) {
-                const Pack<float, 4> p = __builtin_bit_cast(Pack<float, 4>, q[i]);
+      for (int t = 0; t < RTILES; ++t) {
+        v[t] = 0.f;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) f(p.v[e]);
-              } else {
-                const P8 p = __builtin_bit_cast(P8, q[i]);
+        for (int k = 0; k < NW; ++k) v[t] += slots[k][t * 16 + j];
+      }
+    };
+    float s[RTILES], d2[RTILES];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) f(E::to_float(p.v[e]));
-              }
+    for (int t = 0; t < RTILES; ++t) {
+      s[t] = 0.f;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[t] += x_at(u, t, e);      // channels past K are zeros
+    }
+    row_sum(s, s_sum[0]);
+#pragma unroll
+    for (int t = 0; t < RTILES; ++t) {
+      mu[t] = s[t] / (float)a.K;
+      d2[t] = 0.f;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+          if ((wave + u * NW) * BK + kl + 8 * half < a.K) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float d = x_at(u, t, 8 * half + e) - mu[t];
+              d2[t] += d * d;
             }
-        }
-      };
-      float s = 0.f, d2 = 0.f;
-      pass([&](float v) { s += v; });
-      const float m = group_allreduce<OpSum, 16>(s) / (float)a.K;
-      pass([&](float v) { d2 += (v - m) * (v - m); });
-      d2 = group_allreduce<OpSum, 16>(d2);
-      if (j == 0) { s_mu[r] = m; s_inv[r] = 1.0f / sqrtf(d2 / (float)a.K + a.eps); }
+          }
     }
-    __syncthreads();
+    row_sum(d2, s_sum[NORM ? 1 : 0]);
 #pragma unroll
-    for (int t = 0; t < RT; ++t) {
-      const int r = min(t * 16 + j, a.R - 1);
-      mu[t] = s_mu[r];
-      inv[t] = s_inv[r];
-    }
+    for (int t = 0; t < RTILES; ++t) inv[t] = 1.0f / sqrtf(d2[t] / (float)a.K + a.eps);
   }
 
-  floatx4 acc[RT];
+  floatx4 acc[RTILES][CT];
 #pragma unroll
-  for (int t = 0; t < RT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < RTILES; ++t)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[t][c] = floatx4{0.f, 0.f, 0.f, 0.f};
   for (int s0 = wave; s0 < nsteps; s0 += NW * U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
-      for (int half = 0; half < 2; ++half)
+      for (int half = 0; half < 2; ++half) {
+        if constexpr (NORM && !AFFINE_EARLY) load_affine(0, half, (s0 + u * NW) * BK + kl);
 #pragma unroll
-        for (int t = 0; t < RT; ++t) {
+        for (int t = 0; t < RTILES; ++t) {
           uint4 b;
           if constexpr (NORM) {
-            const P8 gp = __builtin_bit_cast(P8, ga[u][half]), bp = __builtin_bit_cast(P8, be[u][half]);
+            constexpr int slot = AFFINE_EARLY ? 1 : 0;
+            const P8 gp = __builtin_bit_cast(P8, ga[slot * u][half]), bp = __builtin_bit_cast(P8, be[slot * u][half]);
             P8 o;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              float v;
-              if constexpr (IN == kNormF32) v = __builtin_bit_cast(Pack<float, 4>, x[u][t][half * 2 + e / 4]).v[e % 4];
-              else v = E::to_float(__builtin_bit_cast(P8, x[u][t][half]).v[e]);
-              o.v[e] = E::from_float((v - mu[t]) * inv[t] * E::to_float(gp.v[e]) + E::to_float(bp.v[e]));
-            }
+            for (int e = 0; e < 8; ++e)
+              o.v[e] = E::from_float((x_at(u, t, half * 8 + e) - mu[t]) * inv[t] * E::to_float(gp.v[e]) + E::to_float(bp.v[e]));
             b = __builtin_bit_cast(uint4, o);
           } else {
             b = x[u][t][half];
           }
-          acc[t] = mfma16<DT>(w[u][half], b, acc[t]);
+#pragma unroll
+          for (int c = 0; c < CT; ++c) acc[t][c] = mfma16<DT>(w[u][c][half], b, acc[t][c]);
         }
-      fetch(u, s0 + (u + U) * NW);
+      }
+      if constexpr (!NORM) fetch(u, s0 + (u + U) * NW);
     }
   }
 
 #pragma unroll
-  for (int t = 0; t < RT; ++t) *reinterpret_cast<floatx4 *>(s_acc[wave][t][lane]) = acc[t];
+  for (int t = 0; t < RTILES; ++t)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) *reinterpret_cast<floatx4 *>(s_acc[wave][t * CT + c][lane]) = acc[t][c];
   if (a.advance && blockIdx.x == 0 && tid < a.R) a.advance[tid] += 1;
   __syncthreads();
-  if (wave >= RT) return;
-  // wave t finishes row tile t: lane (j, g) has columns n0 + 4g .. + 3 of row 16 t + j
-  const int r = wave * 16 + j, n = n0 + 4 * g;
-  if (r >= a.R || n >= a.N) return;
+  if (wave >= RTILES * CT) return;
+  // wave t CT + c finishes row tile t of column tile c: lane (j, g) has columns 4g .. 4g + 3 of row j; with eight rows lanes
+  // (j, g) and (j + 8, g + 2) hold the halves of columns 4g .. of row j, j < 8, g < 2
+  const int t = wave / CT, c = wave % CT;
+  const int r = t * 16 + j, n = n0 + c * ROWS + 4 * g;
+  if (r >= a.R || n >= a.N || (HALF && (j >= 8 || g >= 2))) return;
   float v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int k = 0; k < NW; ++k)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] += s_acc[k][wave][lane][i];
+    for (int i = 0; i < 4; ++i) {
+      v[i] += s_acc[k][wave][lane][i];
+      if constexpr (HALF) v[i] += s_acc[k][wave][(lane + 40) % kWave][i];
+    }
   typedef Pack<T, 4> P4;
   typedef Pack<float, 4> F4;
   if (a.bias) {
@@ -247,23 +285,54 @@ __global__ __launch_bounds__(NW * kWave) void rows_linear_kernel(RowsArgs a) {
   }
 }
 
-template <int DT, int IN, int OUT, int NW>
-static void launch_rows_linear(const RowsArgs &a, hipStream_t s) {
-  const unsigned grid = (unsigned)ceil_div(a.N, 16);
-  if (a.R <= 16) rows_linear_kernel<DT, IN, OUT, NW, 1><<<grid, NW * kWave, 0, s>>>(a);
-  else rows_linear_kernel<DT, IN, OUT, NW, 2><<<grid, NW * kWave, 0, s>>>(a);
-}
-
-// Waves per workgroup: about three steps of 64 channels each for narrow rows, so that all of a wave's weights are in flight
-// at once; sixteen waves where K is long enough to keep them busy.
-template <int DT, int IN, int OUT>
-static int rows_linear(const RowsArgs &a, hipStream_t s) {
-  const int64_t steps = ceil_div(a.K, 64);
-  if (steps <= 16) launch_rows_linear<DT, IN, OUT, 4>(a, s);
-  else if (IN != kPlain || steps <= 32) launch_rows_linear<DT, IN, OUT, 8>(a, s);
-  else if constexpr (IN == kPlain) launch_rows_linear<DT, IN, OUT, 16>(a, s);
+template <int DT, int IN, int OUT, int NW, int U, int RT, int CT = 1>
+static int launch_rows_linear(const RowsArgs &a, hipStream_t s) {
+  constexpr int COLS = (RT == 0 ? 8 : 16) * CT;
+  rows_linear_kernel<DT, IN, OUT, NW, U, RT, CT><<<(unsigned)ceil_div(a.N, COLS), NW * kWave, 0, s>>>(a);
   EN_RETURN_IF_LAUNCH_FAILED();
   return EN_OK;
+}
+
+// Waves per workgroup, steps in flight per wave, row tiles and column tiles, by the rows R and the width K.  With a LayerNorm
+// in front the waves and steps have to hold the whole row, and its arithmetic is shared by more columns.  Measured alone with
+// cold weights (launch to launch, 2.8 us of it an empty launch; the library's GEMM, without LayerNorm, in brackets), 8 rows:
+//   768 -> 768   3 x 2 steps 2.9 us, 6 x 1 3.1, sixteen rows' tile 4 x 3 3.3 (4.0)
+//   3072 -> 768  8 x 3 5.6 us, 12 x 2 5.8, sixteen rows' tile 16 x 3 7.8 (5.4);      8192 -> 2048 10.7 us, 15.7 (9.6)
+//   768 -> 2304 with LayerNorm 6 x 1, two column tiles 4.1 us, one 4.6, sixteen rows' tile 4.5 (4.0 + a LayerNorm)
+//   2048 -> 6144 with LayerNorm 8 x 2, four column tiles 7.8 us, two 9.5, one 10.2 (8.9 + a LayerNorm)
+// 16 rows 2048 -> 6144 with LayerNorm: two column tiles 9.7 us, one 14.9; 24 rows: 14.0, 20.6.
+template <int DT, int IN, int OUT>
+static int rows_linear(const RowsArgs &a, hipStream_t s) {
+  const int64_t steps = ceil_div(a.K, 64), wide = ceil_div(a.K, 128);
+  if constexpr (IN == kPlain) {
+    if (a.R <= 8) {
+      if (wide <= 6) return launch_rows_linear<DT, IN, OUT, 3, 2, 0, 1>(a, s);
+      if (wide <= 16) return launch_rows_linear<DT, IN, OUT, 8, 2, 0, 1>(a, s);
+      return launch_rows_linear<DT, IN, OUT, 8, 3, 0, 1>(a, s);
+    }
+    if (a.R <= 16) {
+      if (steps <= 16) return launch_rows_linear<DT, IN, OUT, 4, 3, 1, 1>(a, s);
+      if (steps <= 32) return launch_rows_linear<DT, IN, OUT, 8, 3, 1, 1>(a, s);
+      return launch_rows_linear<DT, IN, OUT, 16, 3, 1, 1>(a, s);
+    }
+    if (steps <= 16) return launch_rows_linear<DT, IN, OUT, 4, 2, 2, 1>(a, s);
+    if (steps <= 32) return launch_rows_linear<DT, IN, OUT, 8, 2, 2, 1>(a, s);
+    return launch_rows_linear<DT, IN, OUT, 16, 2, 2, 1>(a, s);
+  } else {
+    if (steps > 32) return EN_ERR_UNSUPPORTED;
+    if (a.R <= 8) {
+      if (wide <= 6) return launch_rows_linear<DT, IN, OUT, 6, 1, 0, 2>(a, s);
+      if (a.N < 4096) return launch_rows_linear<DT, IN, OUT, 8, 2, 0, 2>(a, s);
+      return launch_rows_linear<DT, IN, OUT, 8, 2, 0, 4>(a, s);
+    }
+    if (a.R <= 16) {
+      if (steps <= 12) return launch_rows_linear<DT, IN, OUT, 4, 3, 1, 2>(a, s);
+      if (steps <= 24) return launch_rows_linear<DT, IN, OUT, 8, 3, 1, 2>(a, s);
+      return launch_rows_linear<DT, IN, OUT, 16, 2, 1, 2>(a, s);
+    }
+    if (steps <= 16) return launch_rows_linear<DT, IN, OUT, 8, 2, 2, 2>(a, s);
+    return launch_rows_linear<DT, IN, OUT, 16, 2, 2, 2>(a, s);
+  }
 }
 
 static int log2_page(int v) {
@@ -342,7 +411,7 @@ int en_block_decode(const en_block_decode_args *p, en_stream_t stream) {
   const int64_t hid = (int64_t)p->head_num * p->size_per_head;
   if (p->batch > kMaxRows || hid > kMaxWidth || p->size_per_head % 8 || p->size_per_head > 512 || p->mlp_width % 8 || p->mlp_width > INT32_MAX)
     return EN_ERR_UNSUPPORTED;
-  if (p->activation < EN_ACT_NONE || p->activation > EN_ACT_GELU) return EN_ERR_UNSUPPORTED;
+  if ((int64_t)p->batch * p->x_stride * 2 >= (1ll << 31) || p->activation < EN_ACT_NONE || p->activation > EN_ACT_GELU) return EN_ERR_UNSUPPORTED;
   if (p->page_table && (log2_page(p->page_size) < 4 || p->max_pages_per_seq < 1 || p->num_pages < 1)) return EN_ERR_UNSUPPORTED;
   if (p->workspace_bytes < en_block_decode_workspace_bytes(p->batch, p->head_num, p->size_per_head, p->mlp_width, p->cache_len))
     return EN_ERR_SCRATCH;
