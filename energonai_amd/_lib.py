@@ -48,7 +48,10 @@ SIGNATURES = {
                            c_int, c_void_p, c_void_p]),
     "en_attn_tile_table_elems": (c_int64, [c_int] * 4),
     "en_attn_tile_table": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
-    "en_layer_tables": (c_int, [c_void_p] * 2 + [c_int] * 5 + [c_void_p] * 3),
+    "en_layer_tables": (c_int, [c_void_p] * 2 + [c_int] * 5 + [c_void_p] * 4),
+    "en_attn_fused_norm_arrivals": (c_int64, [c_int] * 2),
+    "en_attn_fused_norm": (c_int, [c_void_p] * 4 + [c_int] * 4 + [c_int64, c_float, c_int, c_int] + [c_void_p] * 6 +
+                           [c_float, c_void_p, c_int, c_void_p]),
     "en_attn_fused_query_tile": (c_int, [c_int] * 5),
     "en_packed_scores_elems": (c_int64, [c_int] * 4),
     "en_scale_mask_softmax_packed": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_void_p]),

@@ -889,17 +889,20 @@ __global__ __launch_bounds__(1024) void attn_tile_table_kernel(const int32_t *__
 }
 
 // Both arrays a layer step looks rows up in, once per batch: workgroup 0 fills the tile table, workgroup 1 + b the row
-// offsets of sequence b (row of token t in the padded [B*S] numbering minus t).  Two launches took 2.8 + 4.7 us and the gap
+// offsets of sequence b (row of token t in the padded [B*S] numbering minus t) and clears its `words` meeting words.  Two launches took 2.8 + 4.7 us and the gap
 // between them for 32 sequences; together they take the longer one.
 __global__ __launch_bounds__(1024) void layer_tables_kernel(const int32_t *__restrict__ lens, const int32_t *__restrict__ cu,
                                                             int batch, int heads, int seq_len, int ntq,
                                                             int32_t *__restrict__ table, int capacity, int tiles_first,
-                                                            int32_t *__restrict__ row_offsets, int left_padded) {
+                                                            int32_t *__restrict__ row_offsets, int left_padded,
+                                                            unsigned long long *__restrict__ arrivals, int words) {
   if (blockIdx.x == 0) {
     fill_tile_table(lens, batch, heads, seq_len, ntq, table, capacity, tiles_first, kQTile);
     return;
   }
   const int b = blockIdx.x - 1;
+  if (arrivals)
+    for (int i = threadIdx.x; i < words; i += 1024) arrivals[(int64_t)b * words + i] = 0;
   const int t0 = cu[b], n = lens[b];
   const int off = b * seq_len - t0 + (left_padded ? seq_len - n : 0);
   for (int j = threadIdx.x; j < n; j += 1024) row_offsets[t0 + j] = off;
@@ -1031,7 +1034,8 @@ int en_attn_tile_table(const int32_t *seq_lens, int batch, int head_num, int q_s
 }
 
 int en_layer_tables(const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int max_seq_len, int left_padded,
-                    int head_num, int tiles_first, int32_t *tile_table, int32_t *row_offsets, en_stream_t stream) {
+                    int head_num, int tiles_first, int32_t *tile_table, int32_t *row_offsets, uint64_t *arrivals,
+                    en_stream_t stream) {
   using namespace en;
   if (!seq_lens || !cu_seqlens || !tile_table || !row_offsets) return EN_ERR_NULL;
   if (batch < 1 || batch > 65536 || head_num < 1 || max_seq_len < 1) return EN_ERR_SHAPE;
@@ -1039,7 +1043,9 @@ int en_layer_tables(const int32_t *seq_lens, const int32_t *cu_seqlens, int batc
   if (cap > INT32_MAX || (int64_t)batch * head_num > INT32_MAX / 64) return EN_ERR_SHAPE;
   layer_tables_kernel<<<1 + batch, 1024, 0, (hipStream_t)stream>>>(seq_lens, cu_seqlens, batch, head_num, max_seq_len,
                                                                    (int)ceil_div(max_seq_len, kQTile), tile_table, (int)cap,
-                                                                   tiles_first ? 1 : 0, row_offsets, left_padded ? 1 : 0);
+                                                                   tiles_first ? 1 : 0, row_offsets, left_padded ? 1 : 0,
+                                                                   reinterpret_cast<unsigned long long *>(arrivals),
+                                                                   (int)(en_attn_fused_norm_arrivals(batch, max_seq_len) / batch));
   EN_RETURN_IF_LAUNCH_FAILED();
   return EN_OK;
 }

@@ -117,11 +117,17 @@ PyObject *wait_event(PyObject *const *a) {
   Py_RETURN_NONE;
 }
 
-PyObject *pair(const Tensor &x, const Tensor &y) {
-  PyObject *px = THPVariable_Wrap(x), *py = THPVariable_Wrap(y);
-  PyObject *r = (px && py) ? PyTuple_Pack(2, px, py) : nullptr;
-  Py_XDECREF(px);
-  Py_XDECREF(py);
+PyObject *tuple(std::initializer_list<Tensor> ts) {
+  PyObject *r = PyTuple_New((Py_ssize_t)ts.size());
+  Py_ssize_t i = 0;
+  for (const Tensor &t : ts) {
+    PyObject *p = r ? THPVariable_Wrap(t) : nullptr;
+    if (!p) {
+      Py_XDECREF(r);
+      return nullptr;
+    }
+    PyTuple_SET_ITEM(r, i++, p);
+  }
   return r;
 }
 
@@ -137,26 +143,29 @@ PyObject *prefix_sum(PyObject *const *a) {
   check(without_gil([&] {
           return en_prefix_sum(lens.data_ptr(), i64, (int)batch, cu.data_ptr<int32_t>(), lens32.data_ptr<int32_t>(), stream_of(lens));
         }), "prefix_sum");
-  return pair(cu, lens32);
+  return tuple({cu, lens32});
 }
 
-// layer_tables(lens, cu_seqlens, batch, max_seq_len, left_padded, total, heads, tiles_first) -> (row offsets, tile table)
+// layer_tables(lens, cu_seqlens, batch, max_seq_len, left_padded, total, heads, tiles_first)
+// -> (row offsets, tile table, meeting words of en_attn_fused_norm)
 PyObject *layer_tables(PyObject *const *a) {
   const Tensor &lens = gpu(a[0], "lens"), &cu = gpu(a[1], "cu_seqlens");
   const int64_t batch = integer(a[2]), S = integer(a[3]), left = integer(a[4]), total = integer(a[5]), heads = integer(a[6]),
                 tiles_first = integer(a[7]);
   const c10::DeviceGuard guard(lens.device());
   const int64_t n = en_attn_tile_table_elems((int)batch, (int)heads, (int)S, 0);
-  const Tensor offs = at::empty({total > 0 ? total : 1}, lens.options()), table = at::empty({n > 0 ? n : 1}, lens.options());
+  const Tensor offs = at::empty({total > 0 ? total : 1}, lens.options()), table = at::empty({n > 0 ? n : 1}, lens.options()),
+               arrivals = at::empty({en_attn_fused_norm_arrivals((int)batch, (int)S)}, lens.options().dtype(at::kLong));
   check(without_gil([&] {
           return en_layer_tables(i32(lens), i32(cu), (int)batch, (int)S, (int)left, (int)heads, (int)tiles_first,
-                                 table.data_ptr<int32_t>(), offs.data_ptr<int32_t>(), stream_of(lens));
+                                 table.data_ptr<int32_t>(), offs.data_ptr<int32_t>(),
+                                 reinterpret_cast<uint64_t *>(arrivals.data_ptr<int64_t>()), stream_of(lens));
         }), "layer_tables");
-  return pair(offs, table);
+  return tuple({offs, table, arrivals});
 }
 
 // layer(hidden_padded, qkv_packed, dense_out, gamma, beta, ctx_out, cu_seqlens, lens, row offsets or None, tile table or None,
-//       heads, size_per_head, total, scale, eps, causal, left_padded, form) -> y
+//       heads, size_per_head, total, scale, eps, causal, left_padded, form, meeting words or None) -> y
 PyObject *layer(PyObject *const *a) {
   static const std::string who = "padding_removal_layer: ";
   const Tensor &hidden = gpu(a[0], "hidden_padded"), &qkv = gpu(a[1], "qkv_packed");
@@ -209,6 +218,18 @@ PyObject *layer(PyObject *const *a) {
     scores = at::empty({n}, opt);
   }
   auto ptr = [](const Tensor &t) -> void * { return t.defined() ? t.data_ptr() : nullptr; };
+  if (form == 2 && !has_dense && offs && a[18] != Py_None && T > 0) {      // small enough: one launch
+    const Tensor &arrivals = tensor(a[18], "arrivals");
+    const int rc = without_gil([&] {
+      return en_attn_fused_norm(qkv.data_ptr(), ctx_packed.data_ptr(), i32(lens), i32(cu), (int)B, (int)H, (int)S, (int)D, T, scale, causal,
+                                tag, table, hidden.data_ptr(), offs, gamma.data_ptr(), beta.data_ptr(), y.data_ptr(), eps,
+                                reinterpret_cast<uint64_t *>(arrivals.data_ptr<int64_t>()), -1, stream_of(hidden));
+    });
+    if (rc != EN_ERR_UNSUPPORTED) {
+      check(rc, "padding_removal_layer");
+      return THPVariable_Wrap(y);
+    }
+  }
   check(without_gil([&] {
           return en_padding_removal_layer(hidden.data_ptr(), qkv.data_ptr(), dense, gamma.data_ptr(), beta.data_ptr(), ptr(x),
                                           ptr(padded), ptr(scores), ptr(ctx), ctx_packed.data_ptr(), y.data_ptr(), i32(cu), i32(lens),
@@ -354,8 +375,8 @@ PyMethodDef kMethods[] = {
     EN_FAST(record_event, 1, "event recorded on the current stream of the tensor's device"),
     EN_FAST(wait_event, 2, "makes the current stream of the tensor's device wait for the event"),
     EN_FAST(prefix_sum, 2, "(cu_seqlens, lens) of a batch"),
-    EN_FAST(layer_tables, 8, "(row offsets, tile table) of a batch"),
-    EN_FAST(layer, 18, "en_padding_removal_layer on new outputs"),
+    EN_FAST(layer_tables, 8, "(row offsets, tile table, meeting words) of a batch"),
+    EN_FAST(layer, 19, "en_padding_removal_layer on new outputs"),
     EN_FAST(decode_layer, 10, "en_decode_layer on new outputs"),
     EN_FAST(block_decode, 25, "en_block_decode into a position of an output history"),
     {nullptr, nullptr, 0, nullptr}};

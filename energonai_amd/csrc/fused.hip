@@ -46,11 +46,14 @@
 // stands full and holds back the tile loads of every wave on the CU.
 #include "fused_common.hip.h"
 
+#include <algorithm>
+
 namespace en {
 
 // DP: channels of a row in LDS (the head size rounded up to 64, 96 or 128); NVS: MFMA steps of 16 channels that hold any.
-template <int DT, int DP, int NVS>
-__global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_kernel(FusedArgs fa) {
+// NORM: the residual + LayerNorm of fused_common.hip.h follows (16-byte context rows, no separate query lengths).
+template <int DT, int DP, int NVS, bool NORM>
+__device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *norm) {
   static_assert(DT != EN_F32, "the fused kernel is built for 16-bit storage");
   typedef Elem<DT> E;
   typedef typename E::T T;
@@ -346,12 +349,13 @@ __global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_kernel(Fu
   // ---- normalise and store: register 4j+i of tile mt holds channel 32mt + 8j + 4g + i of this lane's query
   const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
   const int lane_e = lane_now(), r_e = lane_e & 31, g_e = lane_e >> 5;
-  if (fa.c_vec16) {
+  if (NORM || fa.c_vec16) {
     // A lane holds 8-byte pieces of its own row, 32 rows per store instruction; through LDS (the K buffers are free
     // behind the loop's last barrier, each wave takes the 32 rows' worth that is its own, so no barrier is needed)
     // the wave's tile leaves as whole rows: 16 bytes per lane, four to eight rows per instruction.  Chunk c of row r
     // sits in slot c ^ oswz(r): writes and reads both spread over all banks.
     auto oswz = [](int row) { return DP == 96 ? (row >> 2) & 3 : row & (KVEC_ROW - 1); };
+    const rsrc_t c_rsrc = make_rsrc(cbase, (uint32_t)(((int64_t)(ql - 1) * fa.c_ss + a.D) * E::kSize));
     char *stage = reinterpret_cast<char *>(&lds_k[0][0]) + wave * 32 * ROW * E::kSize;
 #pragma unroll
     for (int mt = 0; mt < DMT; ++mt)
@@ -369,7 +373,16 @@ __global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_kernel(Fu
       const int row = (i * kWave + lane_e) / KVEC_ROW, c = (i * kWave + lane_e) % KVEC_ROW;
       const uint4 v = *reinterpret_cast<const uint4 *>(stage + row * ROW * E::kSize + ((c ^ oswz(row)) * 16));
       const int qrow = q0 + wave * 32 + row;
+      if constexpr (NORM) {
+        const uint32_t at = (uint32_t)((int64_t)qrow * fa.c_ss + c * EPV) * E::kSize;
+        buffer_store16<kAgentScope>(c_rsrc, (unsigned)qrow < (unsigned)ql && c * EPV < a.D ? at : kOutOfRange, v);
+        continue;
+      }
       if ((unsigned)qrow < (unsigned)ql && c * EPV < a.D) *reinterpret_cast<uint4 *>(cbase + (int64_t)qrow * fa.c_ss + c * EPV) = v;
+    }
+    if constexpr (NORM) {
+      const int first = max(q0, 0);
+      norm_tile<DT>(*norm, norm->arrivals + ((int64_t)b * a.ntq + qi) * kNormWordStride, qr + first, min(q0 + kQTile, ql) - first, h, a.H);
     }
     return;
   }
@@ -390,14 +403,29 @@ __global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_kernel(Fu
     }
 }
 
+template <int DT, int DP, int NVS>
+__global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_kernel(FusedArgs fa) {
+  fused_tile<DT, DP, NVS, false>(fa, nullptr);
+}
+template <int DT, int DP, int NVS>
+__global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_norm_kernel(FusedArgs fa, NormArgs norm) {
+  fused_tile<DT, DP, NVS, true>(fa, &norm);
+}
+
+template <int DT, int DP, int NVS>
+static void launch_form(const FusedArgs &fa, const NormArgs *norm, unsigned grid, hipStream_t s) {
+  if (norm) attn_fused_norm_kernel<DT, DP, NVS><<<grid, kBlock, 0, s>>>(fa, *norm);
+  else attn_fused_kernel<DT, DP, NVS><<<grid, kBlock, 0, s>>>(fa);
+}
+
 template <int DT>
-static int launch_fused(FusedArgs &fa, hipStream_t s) {
+static int launch_fused(FusedArgs &fa, const NormArgs *norm, hipStream_t s) {
   const AttnArgs &a = fa.base;
   const unsigned grid = (unsigned)(ceil_div(a.units, kXcds) * kXcds * a.ntq);
-  if (a.D <= 64) attn_fused_kernel<DT, 64, 4><<<grid, kBlock, 0, s>>>(fa);
-  else if (a.D <= 80) attn_fused_kernel<DT, 96, 5><<<grid, kBlock, 0, s>>>(fa);
-  else if (a.D <= 96) attn_fused_kernel<DT, 96, 6><<<grid, kBlock, 0, s>>>(fa);
-  else attn_fused_kernel<DT, 128, 8><<<grid, kBlock, 0, s>>>(fa);
+  if (a.D <= 64) launch_form<DT, 64, 4>(fa, norm, grid, s);
+  else if (a.D <= 80) launch_form<DT, 96, 5>(fa, norm, grid, s);
+  else if (a.D <= 96) launch_form<DT, 96, 6>(fa, norm, grid, s);
+  else launch_form<DT, 128, 8>(fa, norm, grid, s);
   EN_RETURN_IF_LAUNCH_FAILED();
   return EN_OK;
 }
@@ -413,13 +441,13 @@ extern "C" int en_attn_fused_query_tile(int q_seq_len, int k_seq_len, int size_p
   return dtype == EN_F32 ? 64 : en::kQTile;     // fp32: the kernel of fused_f32.hip, 64-row tiles
 }
 
-extern "C" int en_attn_fused(const void *q, const void *k, const void *v, void *ctx, const int32_t *k_lens,
-                             const int32_t *q_lens, int batch, int head_num, int q_seq_len, int k_seq_len,
-                             int size_per_head, const int64_t *q_strides, const int64_t *k_strides,
-                             const int64_t *v_strides, const int64_t *c_strides, const int32_t *q_row_offsets,
-                             const int32_t *k_row_offsets, float scale, int causal, int dtype,
-                             const int32_t *tile_table, int query_tile, en_stream_t stream) {
-  using namespace en;
+namespace en {
+
+static int attn_fused(const void *q, const void *k, const void *v, void *ctx, const int32_t *k_lens, const
+                      int32_t *q_lens, int batch, int head_num, int q_seq_len, int k_seq_len, int size_per_head, const int64_t
+                      *q_strides, const int64_t *k_strides, const int64_t *v_strides, const int64_t *c_strides, const int32_t
+                      *q_row_offsets, const int32_t *k_row_offsets, float scale, int causal, int dtype, const int32_t
+                      *tile_table, int query_tile, const NormArgs *norm, en_stream_t stream) {
   if (!q || !k || !v || !ctx || !k_lens || !q_strides || !k_strides || !v_strides || !c_strides) return EN_ERR_NULL;
   if (batch < 1 || head_num < 1 || q_seq_len < 1 || k_seq_len < 1 || size_per_head < 1) return EN_ERR_SHAPE;
   if (dtype != EN_F16 && dtype != EN_BF16 && dtype != EN_F32) return EN_ERR_DTYPE;
@@ -460,10 +488,103 @@ extern "C" int en_attn_fused(const void *q, const void *k, const void *v, void *
   a.tile_table = tile_table;
   fa.scale = scale;
   hipStream_t s = (hipStream_t)stream;
-  if (f32) return launch_fused_f32(fa, s);
+  if (norm && (!fa.c_vec16 || query_tile == kWideQTile)) return EN_ERR_UNSUPPORTED;
+  if (f32) return launch_fused_f32(fa, norm, s);
   if (query_tile == kWideQTile) {
     a.ntq = (int)ceil_div(q_seq_len, kWideQTile);
     return launch_fused_wide(dtype, fa, s);
   }
-  return dtype == EN_F16 ? launch_fused<EN_F16>(fa, s) : launch_fused<EN_BF16>(fa, s);
+  return dtype == EN_F16 ? launch_fused<EN_F16>(fa, norm, s) : launch_fused<EN_BF16>(fa, norm, s);
 }
+
+// Workgroups that are resident at once: what LDS and registers leave room for on 256 CUs.
+static int64_t resident_workgroups(int size_per_head, int dtype) { return dtype == EN_F32 ? 512 : size_per_head <= 64 ? 1024 : 768; }
+
+// Where one launch is the faster form, us per layer, one launch / two (8 layers, hot operands).  Meeting costs about 7 us
+// (context written through, counted, seen, read back) plus a trip to memory for every two rows of a wave; a LayerNorm launch
+// costs 5 us and what its bytes take.
+//   16-bit: context of 7 MB and more and at most three rows per wave: 24 sequences of up to 384, 16 heads x 64 22.4 / 24.2,
+//     8 of up to 600, 16 x 96 27.1 / 28.7, 2 of 1024, 16 x 128 33.0 / 33.7; smaller ones lose (16 of up to 128, 12 x 64
+//     13.6 / 11.8, one of 509 17.9 / 15.7), as do few heads (64 of up to 128, 4 x 64 17.3 / 13.1).  Where the launches
+//     themselves are what bounds a layer, short prompts: one of 60 rows, 12 x 64 10.4 / 11.3, 64 of up to 30, 4 x 64 10.7 / 13.1
+//     (16 x 64, a full chip: 13.8 / 13.1).
+//   fp32 (64-row tiles): 4 of up to 128, 12 x 64 15.0 / 15.5, 16 of up to 128 21.3 / 21.9; 64 of up to 128, 4 x 64 22.2 / 21.8.
+static bool one_launch_pays(int heads, int seq_len, int64_t tiles, int64_t bytes, int dtype) {
+  const int64_t per_wave = ceil_div(std::min(seq_len, dtype == EN_F32 ? kF32QTile : kQTile), heads * (kBlock / kWave));
+  if (dtype == EN_F32) return per_wave <= 2;
+  return (bytes >= 7 << 20 && per_wave <= 3) || (seq_len <= 64 && per_wave <= 2 && tiles * heads <= 512);
+}
+
+constexpr int kNormPolls = 64;      // looks at a meeting word before a workgroup leaves its rows to the last one: tens of us
+
+static bool overlap(const void *a, int64_t a_bytes, const void *b, int64_t b_bytes) {
+  const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+  return x < y + (uintptr_t)b_bytes && y < x + (uintptr_t)a_bytes;
+}
+
+}  // namespace en
+
+extern "C" {
+
+int64_t en_attn_fused_norm_arrivals(int batch, int q_seq_len) {
+  return batch < 1 || q_seq_len < 1 ? 0 : batch * en::ceil_div(q_seq_len, en::kF32QTile) * en::kNormWordStride;      // the lower of the tile heights
+}
+
+int en_attn_fused_norm(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
+                       int max_seq_len, int size_per_head, int64_t total_tokens, float scale, int causal, int dtype,
+                       const int32_t *tile_table, const void *hidden_padded, const int32_t *residual_row_offsets, const void *gamma,
+                       const void *beta, void *y, float eps, uint64_t *arrivals, int polls, en_stream_t stream) {
+  using namespace en;
+  if (!qkv || !ctx || !seq_lens || !cu_seqlens || !hidden_padded || !residual_row_offsets || !gamma || !beta || !y || !arrivals)
+    return EN_ERR_NULL;
+  const int es = dtype_size(dtype);
+  if (!es) return EN_ERR_DTYPE;
+  if (batch < 1 || head_num < 1 || max_seq_len < 1 || size_per_head < 1 || total_tokens < 1) return EN_ERR_SHAPE;
+  const int64_t width = (int64_t)head_num * size_per_head, T = total_tokens;
+  if (head_num > kNormMaxHeads || width * es % 16 || width * es / 16 > kNormMaxVectors) return EN_ERR_UNSUPPORTED;
+  if ((int64_t)max_seq_len * width * es >= (1ll << 31)) return EN_ERR_UNSUPPORTED;              // 32-bit offsets into a sequence's context
+  for (const void *p : {qkv, (const void *)ctx, hidden_padded, gamma, beta, (const void *)y})
+    if (!aligned_to(p, 16)) return EN_ERR_UNSUPPORTED;
+  // Workgroups that wait for one another hold their place, so all of them have to be resident at once (half a tile a
+  // sequence is the ragged one, on average).
+  const int64_t tile = dtype == EN_F32 ? kF32QTile : kQTile;
+  const int64_t tiles = max_seq_len <= tile ? batch : T / tile + (batch + 1) / 2;
+  if (tiles * head_num > resident_workgroups(size_per_head, dtype)) return EN_ERR_UNSUPPORTED;
+  if (polls < 0 && !one_launch_pays(head_num, max_seq_len, tiles, T * width * es, dtype)) return EN_ERR_UNSUPPORTED;
+  // Rows are normalised while other tiles still read: buffers that a caller has laid over each other need two launches.
+  const int64_t bytes = T * width * es, meta = ((int64_t)batch + 1) * 4;
+  for (const void *p : {(const void *)ctx, (const void *)y}) {
+    if (overlap(p, bytes, qkv, 3 * bytes) || overlap(p, bytes, seq_lens, meta - 4) || overlap(p, bytes, cu_seqlens, meta) ||
+        overlap(p, bytes, gamma, width * es) || overlap(p, bytes, beta, width * es) || overlap(p, bytes, residual_row_offsets, T * 4) ||
+        overlap(p, bytes, hidden_padded, (int64_t)batch * max_seq_len * width * es))
+      return EN_ERR_UNSUPPORTED;
+  }
+  if (overlap(ctx, bytes, y, bytes)) return EN_ERR_UNSUPPORTED;
+  // A captured launch may run again on any stream, beside launches that use the same meeting words.
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess) {      // e.g. the null stream beside a capture
+    (void)hipGetLastError();
+    return EN_ERR_UNSUPPORTED;
+  }
+  if (capture != hipStreamCaptureStatusNone) return EN_ERR_UNSUPPORTED;
+  const NormArgs norm{hidden_padded, residual_row_offsets, gamma, beta, ctx, y, reinterpret_cast<unsigned long long *>(arrivals),
+                      (int)width, polls < 0 ? kNormPolls : polls, eps};
+  const char *pk = static_cast<const char *>(qkv);
+  const int64_t D = size_per_head, in_strides[3] = {0, 3 * D, 3 * width}, out_strides[3] = {0, D, width};
+  return attn_fused(pk, pk + D * es, pk + 2 * D * es, ctx, seq_lens, nullptr, batch, head_num, max_seq_len, max_seq_len, size_per_head,
+                    in_strides, in_strides, in_strides, out_strides, cu_seqlens, cu_seqlens, scale, causal, dtype,
+                    dtype == EN_F32 ? nullptr : tile_table, 0, &norm, stream);
+}
+
+int en_attn_fused(const void *q, const void *k, const void *v, void *ctx, const int32_t *k_lens,
+                             const int32_t *q_lens, int batch, int head_num, int q_seq_len, int k_seq_len,
+                             int size_per_head, const int64_t *q_strides, const int64_t *k_strides,
+                             const int64_t *v_strides, const int64_t *c_strides, const int32_t *q_row_offsets,
+                             const int32_t *k_row_offsets, float scale, int causal, int dtype,
+                             const int32_t *tile_table, int query_tile, en_stream_t stream) {
+  return en::attn_fused(q, k, v, ctx, k_lens, q_lens, batch, head_num, q_seq_len, k_seq_len,
+                        size_per_head, q_strides, k_strides, v_strides, c_strides, q_row_offsets, k_row_offsets, scale, causal,
+                        dtype, tile_table, query_tile, nullptr, stream);
+}
+
+}  // extern "C"

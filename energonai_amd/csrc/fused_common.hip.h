@@ -3,6 +3,8 @@
 
 #include "attn_common.hip.h"
 
+#include <math.h>
+
 namespace en {
 
 // The lane's number in its wave, counted afresh (two VALU instructions) where a value derived from it is needed only
@@ -24,6 +26,158 @@ struct FusedArgs {
   int c_vec16;               // ctx rows may be written with 128-bit stores (16-byte aligned base and strides)
 };
 
+// ---- residual + LayerNorm behind the attention, in its launch -----------------------------------------------------------
+// Where the LayerNorm follows the attention directly (its width is heads * size_per_head), the H workgroups of a query tile,
+// one per head, wait for each other once their context rows are written, and each normalises an H-th of the tile's rows.
+// That is worth it while the workgroups of a launch are all resident at once: one launch less per layer, and the residual
+// rows, gamma and beta are on their way while the workgroups meet.
+//
+// The meeting point is one 64-bit word per (sequence, query tile), zero between launches: bits 0..5 count the workgroups
+// that have arrived, bits 6..11 those that have gone on, bit 12 + h says that head h has gone without doing its rows.  No
+// workgroup waits without end: after `polls` looks it sets its bit and leaves, unless the last one arrived in the meantime;
+// the last to arrive finds the bits set before its own arrival and does those rows too.  So every row has exactly one owner
+// in whatever order the workgroups run, and the word returns to zero when all H shares have gone on.
+struct NormArgs {
+  const void *residual;
+  const int32_t *res_off;       // residual row of output row t is t + res_off[t]
+  const void *gamma, *beta;
+  const void *ctx;              // packed [T, width], written by this launch
+  void *out;
+  unsigned long long *arrivals; // [batch][ntq], kNormWordStride apart
+  int width, polls;
+  float eps;
+};
+// A memory channel's 256 bytes per word: neighbours in one line make all workgroups of a batch queue for it.
+constexpr int kNormWordStride = 32;
+constexpr int kNormMaxHeads = 48;         // shares that a meeting word has room for
+constexpr int kNormMaxVectors = 4 * kWave; // a wave per row, up to four 16-byte vectors per lane
+constexpr int kAgentScope = 16;           // cache policy of an access that all XCDs see (sc1)
+
+template <int DT, int VPL>
+__device__ __forceinline__ void norm_tile_rows(const NormArgs &n, unsigned long long *word, int64_t row0, int nrows, int share,
+                                               int shares, unsigned long long *s_take) {
+  typedef Elem<DT> E;
+  typedef typename E::T T;
+  constexpr int EPV = 16 / E::kSize, NW = kBlock / kWave;
+  typedef Pack<T, EPV> P;
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const int nvec = n.width / EPV;
+  constexpr bool EARLY = VPL <= 3;              // gamma and beta in registers while the workgroups meet: four vectors do not fit
+  // Rows of a wave in flight at once: the context comes from memory (other XCDs wrote it), a trip of 2 us per row otherwise.
+  constexpr int R = VPL <= 2 ? 2 : 1;
+  const int step = shares * NW;
+  uint4 res[R][VPL];
+  P g[VPL], bt[VPL];
+  auto load_residual = [&](int first) {
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const int64_t t = row0 + min(first + k * step, nrows - 1);
+      const T *p = reinterpret_cast<const T *>(n.residual) + (t + n.res_off[t]) * n.width;
+#pragma unroll
+      for (int j = 0; j < VPL; ++j) res[k][j] = *reinterpret_cast<const uint4 *>(p + min(lane + kWave * j, nvec - 1) * EPV);
+    }
+  };
+  auto load_affine = [&](int j) {
+    const int v = min(lane + kWave * j, nvec - 1) * EPV;
+    g[j] = load_pack<T, EPV>(reinterpret_cast<const T *>(n.gamma) + v);
+    bt[j] = load_pack<T, EPV>(reinterpret_cast<const T *>(n.beta) + v);
+  };
+  if constexpr (EARLY)
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) load_affine(j);
+  int held = share * NW + wave;                 // first of the rows whose residuals are in registers
+  if (held < nrows) load_residual(held);
+  if (threadIdx.x == 0) {
+    const unsigned long long arrived = atomicAdd(word, 1ull);
+    unsigned long long take = 0;                // shares to do here
+    if ((int)(arrived & 63) == shares - 1) {
+      take = arrived >> 12 | 1ull << share;
+    } else {
+      bool all = false;
+      for (int i = 0; i < n.polls && !all; ++i) {
+        __builtin_amdgcn_s_sleep(4);
+        all = (int)(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 63) == shares;
+      }
+      if (!all) all = (int)(atomicOr(word, 1ull << (12 + share)) & 63) == shares;
+      if (all) take = 1ull << share;
+    }
+    *s_take = take;
+  }
+  lds_barrier();
+  for (unsigned long long take = *s_take; take; take &= take - 1) {
+    const int base = __builtin_amdgcn_readfirstlane((__ffsll(take) - 1) * NW + wave);
+    for (int i = base; i < nrows; i += R * step) {
+      uint4 raw[R][VPL];
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        const rsrc_t ctx = make_rsrc(reinterpret_cast<const T *>(n.ctx) + (row0 + i + k * step) * n.width,
+                                     i + k * step < nrows ? (uint32_t)(n.width * E::kSize) : 0u);
+#pragma unroll
+        for (int j = 0; j < VPL; ++j) raw[k][j] = buffer_load16<kAgentScope>(ctx, (uint32_t)(lane + kWave * j) * 16u);
+      }
+      if (i != held) load_residual(i);
+      held = i;
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        if (i + k * step >= nrows) break;
+        float x[VPL][EPV], s = 0.f, d2 = 0.f;
+#pragma unroll
+        for (int j = 0; j < VPL; ++j) {
+          const P a = __builtin_bit_cast(P, raw[k][j]), r = __builtin_bit_cast(P, res[k][j]);
+          const bool in = lane + kWave * j < nvec;
+#pragma unroll
+          for (int e = 0; e < EPV; ++e) {
+            x[j][e] = in ? E::to_float(a.v[e]) + E::to_float(r.v[e]) : 0.f;
+            s += x[j][e];
+          }
+        }
+        const float mu = wave_allreduce<OpSum>(s) / (float)n.width;
+#pragma unroll
+        for (int j = 0; j < VPL; ++j)
+          if (lane + kWave * j < nvec)
+#pragma unroll
+            for (int e = 0; e < EPV; ++e) d2 += (x[j][e] - mu) * (x[j][e] - mu);
+        const float inv = 1.0f / sqrtf(wave_allreduce<OpSum>(d2) / (float)n.width + n.eps);
+        T *out = reinterpret_cast<T *>(n.out) + (row0 + i + k * step) * n.width;
+#pragma unroll
+        for (int j = 0; j < VPL; ++j) {
+          const int v = lane + kWave * j;
+          if constexpr (!EARLY) load_affine(j);
+          if (v < nvec) {
+            P o;
+#pragma unroll
+            for (int e = 0; e < EPV; ++e) {
+              float f = (x[j][e] - mu) * inv * E::to_float(g[j].v[e]) + E::to_float(bt[j].v[e]);
+              asm("" : "+v"(f));      // rounded to fp32 and then to the storage type, as layernorm.hip's wide rows are, not in one instruction
+              o.v[e] = E::from_float(f);
+            }
+            store_pack<T, EPV>(out + v * EPV, o);
+          }
+        }
+      }
+    }
+  }
+  // off the way of the rows: the shares done here have gone on, and the last of them leaves the word at zero
+  if (threadIdx.x == 0 && *s_take) {
+    const int mine = __popcll(*s_take);
+    const int before = (int)(atomicAdd(word, (unsigned long long)mine << 6) >> 6 & 63);
+    if (before + mine == shares) __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// Called by the whole workgroup of (batch b's query tile `word`, head `share`) when it has sent its context rows away with
+// agent-scope stores.  nrows rows of the tile, the first one packed row row0.
+template <int DT>
+__device__ __forceinline__ void norm_tile(const NormArgs &n, unsigned long long *word, int64_t row0, int nrows, int share, int shares) {
+  __shared__ unsigned long long s_take;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the wave's context rows are where every XCD sees them ...
+  lds_barrier();                                        // ... and the other waves' too, before the workgroup says so
+  const int nvec = n.width / (16 / Elem<DT>::kSize);
+  if (nvec <= 2 * kWave) norm_tile_rows<DT, 2>(n, word, row0, nrows, share, shares, &s_take);
+  else if (nvec <= 3 * kWave) norm_tile_rows<DT, 3>(n, word, row0, nrows, share, shares, &s_take);
+  else norm_tile_rows<DT, 4>(n, word, row0, nrows, share, shares, &s_take);
+}
+
 // Both halves of the wave get (x of lanes 0..31, x of lanes 32..63): one VALU swap, no LDS round trip.
 __device__ __forceinline__ void halves_of(float x, float &lo, float &hi) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -35,6 +189,7 @@ __device__ __forceinline__ void halves_of(float x, float &lo, float &hi) {
 constexpr int kWideQTile = 256;
 int launch_fused_wide(int dtype, FusedArgs &fa, hipStream_t s);
 // fused_f32.hip: fp32 storage, heads of up to 64 channels, 64-row query tiles.
-int launch_fused_f32(FusedArgs &fa, hipStream_t s);
+int launch_fused_f32(FusedArgs &fa, const NormArgs *norm, hipStream_t s);
+constexpr int kF32QTile = 64;
 
 }  // namespace en

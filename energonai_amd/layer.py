@@ -135,20 +135,25 @@ _FORMS = {False: 0, True: 1, "packed": 2, "varlen": 3, "varlen_packed": 4}
 
 def _layer_one_call(hidden_padded, qkv_packed, info, S, H, D, T, gamma, beta, eps, scale, causal, left_padded,
                     dense_out, fused_attention, fold_depad=False, ctx_out=None):
-    """The same seven ops through ``en_padding_removal_layer``: one native call per step."""
+    """The same seven ops through ``en_padding_removal_layer`` (small enough: ``en_attn_fused_norm``): one native call per step."""
     form = _FORMS[fused_attention]
     left = bool(left_padded)
     fused_f32 = hidden_padded.dtype == torch.float32 and form in (1, 2)      # the fp32 kernel's tiles are not the table's
     kv_bytes = 2 * S * D * hidden_padded.element_size()
-    table = None
-    if fold_depad and not fused_f32 and not info.ephemeral:
+    table = arrivals = None
+    if fold_depad and not info.ephemeral:
         offs, table = info.layer_tables(S, left, H, kv_bytes)
+        # asked for only where en_attn_fused_norm may take the step: the lookup is 0.4 us of a host-bound layer's 11
+        if form == 2 and dense_out is None and (fused_f32 or S <= 64 or T * H * D >= 7 << 19):
+            arrivals = info.arrivals(S)
+        if fused_f32:
+            table = None
     else:
         offs = info.row_offsets(S, left) if fold_depad else None
         if not fused_f32 and not info.ephemeral:
             table = info.tile_table(H, S, kv_bytes)
     return _lib.front.layer(hidden_padded, qkv_packed, dense_out, gamma, beta, ctx_out, info.cu_seqlens, info.lens, offs, table,
-                            H, D, T, scale, eps, bool(causal), left, form)
+                            H, D, T, scale, eps, bool(causal), left, form, arrivals)
 
 
 def padding_removal_layer_noalloc(hidden_padded: torch.Tensor, qkv_packed: torch.Tensor, seq_lens: torch.Tensor,

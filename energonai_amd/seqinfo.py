@@ -17,13 +17,14 @@ import torch
 from . import _lib
 
 _CACHE_SIZE = 16
+PER_THREAD_STREAMS = (2,)                 # hipStreamPerThread
 TILES_FIRST_MAX_KV_BYTES = 256 << 10     # see SeqInfo.tile_table
 
 
 class SeqInfo:
     """Device-resident int32 lengths and exclusive prefix for one batch."""
 
-    __slots__ = ("lens", "cu_seqlens", "batch_size", "_total", "_source", "_row_offsets", "_tile_tables", "_ready",
+    __slots__ = ("lens", "cu_seqlens", "batch_size", "_total", "_source", "_row_offsets", "_tile_tables", "_arrivals", "_ready",
                  "_ordered", "ephemeral", "_lens_host")
 
     def __init__(self, lens: torch.Tensor, cu_seqlens: torch.Tensor, batch_size: int, total: Optional[int], source):
@@ -34,6 +35,7 @@ class SeqInfo:
         self._source = source           # keeps the caller's tensor alive while cached
         self._row_offsets = {}          # (max_seq_len, left_padded, version of lens) -> int32 [T]
         self._tile_tables = {}          # (head_num, q_seq_len, order, version of lens, tile height) -> int32 workgroup order
+        self._arrivals = {}             # (bucket, stream) -> int64 meeting words of en_attn_fused_norm
         self._ready = []                # events recorded behind the kernels that produced the arrays above
         self._ordered = set()           # raw streams already ordered behind every event of _ready
         self.ephemeral = False          # built for one call only (lengths that cannot be cached): see tile_table_ptr
@@ -113,7 +115,8 @@ class SeqInfo:
         return off
 
     def layer_tables(self, max_seq_len: int, left_padded: bool, head_num: int, unit_kv_bytes: int):
-        """``(row_offsets, tile_table)`` of a layer step (128-row tiles), built by one launch when the batch has neither."""
+        """``(row_offsets, tile_table)`` of a layer step (128-row tiles), built by one launch when the batch has neither; the
+        launch clears the words of ``arrivals`` as well."""
         version = self._lens_version()
         first = unit_kv_bytes <= TILES_FIRST_MAX_KV_BYTES
         if self.cu_seqlens is None or (version is None and self._mutable()):
@@ -125,14 +128,23 @@ class SeqInfo:
         if off is not None or tab is not None:
             return self.row_offsets(max_seq_len, left_padded), self.tile_table(head_num, max_seq_len, unit_kv_bytes)
         self.order_current_stream()
-        off, tab = _lib.front.layer_tables(self.lens, self.cu_seqlens, self.batch_size, max_seq_len, left_padded, self.total,
-                                           head_num, first)
+        off, tab, arrivals = _lib.front.layer_tables(self.lens, self.cu_seqlens, self.batch_size, max_seq_len, left_padded,
+                                                     self.total, head_num, first)
         self.produced_on_current_stream()
         self._row_offsets = {k: o for k, o in self._row_offsets.items() if k[2] == version}
         self._row_offsets[off_key] = off
         self._tile_tables = {k: t for k, t in self._tile_tables.items() if k[3] == version}
         self._tile_tables[tab_key] = tab
+        raw = _lib.stream_of(self.lens)
+        if raw not in PER_THREAD_STREAMS and not torch.cuda.is_current_stream_capturing():
+            self._arrivals[(max_seq_len, raw)] = arrivals
         return off, tab
+
+    def arrivals(self, max_seq_len: int):
+        """The meeting words of ``en_attn_fused_norm`` for launches on the current stream, or ``None``.  They belong to the
+        stream they were cleared on, whose order keeps launches apart that share them; a handle that names another stream
+        in every thread has none."""
+        return self._arrivals.get((max_seq_len, _lib.stream_of(self.lens)))
 
     def _mutable(self) -> bool:
         """True when the lengths belong to a caller that may edit them in place (no prefix was computed from

@@ -352,9 +352,25 @@ int64_t en_attn_tile_table_elems(int batch, int head_num, int q_seq_len, int que
 int en_attn_tile_table(const int32_t *seq_lens, int batch, int head_num, int q_seq_len, int tiles_first,
                        int query_tile, int32_t *table, en_stream_t stream);
 /* The tile table (128-row tiles) and the row offsets of en_padding_offsets in one launch, for a batch whose prefix
- * sums exist: row_offsets gets cu_seqlens[batch] entries. */
+ * sums exist: row_offsets gets cu_seqlens[batch] entries.  `arrivals` (null: none), en_attn_fused_norm_arrivals words, is
+ * cleared for en_attn_fused_norm. */
 int en_layer_tables(const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int max_seq_len, int left_padded,
-                    int head_num, int tiles_first, int32_t *tile_table, int32_t *row_offsets, en_stream_t stream);
+                    int head_num, int tiles_first, int32_t *tile_table, int32_t *row_offsets, uint64_t *arrivals,
+                    en_stream_t stream);
+
+/* en_attn_fused on packed projections [T, head_num, 3 size_per_head] and the residual + LayerNorm that follows it directly
+ * (width head_num * size_per_head, residual rows from hidden_padded through en_padding_offsets) as one launch.  The
+ * workgroups of a query tile meet at a word of `arrivals` (en_attn_fused_norm_arrivals words, zero before the first launch
+ * and again after each): launches that share the array must be ordered by one stream.  `polls` bounds how often a workgroup
+ * looks for the others before it leaves its rows to the last of them (any value gives the same result; < 0: the library's
+ * choice, and a launch only where it is faster than two).  EN_ERR_UNSUPPORTED, with nothing launched, where it does not apply: more workgroups than are resident at once,
+ * widths of more than 256 16-byte vectors, more than 48 heads, operands off 16 bytes or overlapping, a stream under capture. */
+int64_t en_attn_fused_norm_arrivals(int batch, int q_seq_len);
+int en_attn_fused_norm(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
+                       int max_seq_len, int size_per_head, int64_t total_tokens, float scale, int causal, int dtype,
+                       const int32_t *tile_table, const void *hidden_padded, const int32_t *residual_row_offsets,
+                       const void *gamma, const void *beta, void *y, float eps, uint64_t *arrivals, int polls,
+                       en_stream_t stream);
 
 /* ---- one decode step of a pre-LN transformer block -------------------------------------------------------------------
  *

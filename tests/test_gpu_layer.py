@@ -483,3 +483,67 @@ def test_layer_tables_in_one_launch(lens, S, H, left):
         assert torch.equal(off[:sum(lens)], one.row_offsets(S, left)[:sum(lens)])
         assert torch.equal(tab, one.tile_table(H, S, kv_bytes))
         assert both.row_offsets(S, left) is off and both.tile_table(H, S, kv_bytes) is tab
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("lens,S,H,D,causal,left", [
+    ([1], 17, 1, 64, True, False),                          # one workgroup meets nobody
+    ([41], 64, 12, 64, True, True),                         # fewer rows than waves
+    ([127, 128, 129, 0, 65], 130, 4, 64, False, True),      # edges of the 128- and 64-row tiles, a sequence of no rows
+    ([300, 7, 256], 300, 20, 80, True, False),              # four vectors per lane (16-bit), ragged first tiles
+    ([200, 64, 63], 200, 16, 96, True, True),
+    ([140, 1], 257, 48, 16, True, False),                   # the most shares a word has room for
+    ([140, 30], 257, 49, 16, True, False),                  # one more: two launches
+    ([130, 3], 140, 16, 128, False, False),
+    ([100] * 200, 128, 16, 64, True, False),                # more than one round of workgroups: two launches
+])
+def test_attention_and_layernorm_in_one_launch(dtype, lens, S, H, D, causal, left):
+    """The step in one launch against the same step in two, with workgroups that wait for each other and (``polls`` = 0)
+    with none that does: the context is bit-identical; y differs by at most one rounding of the stored value (rows of more
+    than 192 vectors are added up in another order, and where the compiler fuses the last multiply-add with the conversion
+    one of two roundings is left out).  The meeting words return to zero."""
+    from energonai_amd import _lib, layer
+    from energonai_amd.seqinfo import build_seq_info
+    announce("one launch", dtype, lens[:5], S, H, D, causal, left)
+    if dtype == torch.float32 and D > 64:
+        pytest.skip("the fp32 kernel takes heads of up to 64 channels")
+    g = torch.Generator().manual_seed(S + H)
+    B, T, hid, scale = len(lens), sum(lens), H * D, D ** -0.5
+    hidden, qkv = torch.randn(B, S, hid, generator=g).to(dtype).cuda(), torch.randn(1, T, H, 3 * D, generator=g).to(dtype).cuda()
+    gamma, beta = (1 + 0.1 * torch.randn(hid, generator=g)).to(dtype).cuda(), torch.randn(hid, generator=g).to(dtype).cuda()
+    info = build_seq_info(torch.tensor(lens, dtype=torch.int32).cuda(), B, total=T)
+    offs, table = info.layer_tables(S, left, H, 2 * S * D * hidden.element_size())
+    words, f32 = info.arrivals(S), dtype == torch.float32
+    assert words is not None and int(words.abs().max()) == 0
+    want_ctx = torch.empty(1, T, H, D, dtype=dtype, device="cuda")
+    want = _lib.front.layer(hidden, qkv, None, gamma, beta, want_ctx, info.cu_seqlens, info.lens, offs, None if f32 else table, H, D,
+                            T, scale, 1e-5, causal, left, 2, None).float()
+    ulp = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7, torch.float32: 2.0 ** -18}[dtype]
+
+    def close(y):
+        return bool(((y.float() - want).abs() <= ulp * want.abs().clamp_min(2.0 ** -6)).all())
+
+    one_launch = H <= 48 and hid * hidden.element_size() <= 4096 and B < 200
+    for polls in (64, 0, 0, 64):
+        ctx, y = torch.full_like(want_ctx, 7.0), torch.full((1, T, hid), 7.0, dtype=dtype, device="cuda")
+        rc = _lib.fn.en_attn_fused_norm(qkv.data_ptr(), ctx.data_ptr(), info.lens.data_ptr(), info.cu_seqlens.data_ptr(), B, H, S, D, T,
+                                        scale, int(causal), _lib.dtype_tag(qkv, "test"), None if f32 else table.data_ptr(),
+                                        hidden.data_ptr(), offs.data_ptr(), gamma.data_ptr(), beta.data_ptr(), y.data_ptr(), 1e-5,
+                                        words.data_ptr(), polls, _lib.stream_of(qkv))
+        if not one_launch:
+            assert rc == -5, rc     # EN_ERR_UNSUPPORTED
+            assert bool((y == 7.0).all())
+            return
+        assert rc == 0, rc
+        torch.cuda.synchronize()
+        assert torch.equal(ctx, want_ctx)
+        assert close(y)
+        assert int(words.abs().max()) == 0
+    got = layer.padding_removal_layer(hidden, qkv, info, H, D, gamma, beta, 1e-5, scale, causal, left)
+    assert close(got)
+    with torch.cuda.stream(torch.cuda.Stream()):            # the words are the first stream's: two launches here
+        assert info.arrivals(S) is None
+        torch.cuda.current_stream().wait_stream(torch.cuda.default_stream())
+        again = layer.padding_removal_layer(hidden, qkv, info, H, D, gamma, beta, 1e-5, scale, causal, left)
+        torch.cuda.current_stream().synchronize()
+    assert torch.equal(again.float(), want)
