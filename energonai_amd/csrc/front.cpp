@@ -287,6 +287,9 @@ PyObject *decode_layer(PyObject *const *a) {
 // -> out[:, :position + 1] with the block's output for the newest position of `hidden` at `position`, or None, with nothing
 // done, where en_block_decode has no kernel for these tensors.
 PyObject *block_decode(PyObject *const *a) {
+  // a tensor subclass computes in its own way (quantised weights behind a plain Linear): the general path asks it
+  for (int i : {0, 1, 2, 4, 5, 6, 7, 8, 9, 11, 12, 13, 14})
+    if (a[i] != Py_None && !THPVariable_CheckExact(a[i])) Py_RETURN_NONE;
   const Tensor &x = gpu(a[0], "hidden_states", false);
   const Tensor &out = gpu(a[23], "out", false);
   const Tensor &k = gpu(a[18], "k_cache", false), &v = gpu(a[19], "v_cache", false), &lens = gpu(a[20], "lens");

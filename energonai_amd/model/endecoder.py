@@ -56,23 +56,25 @@ class Block1D(nn.Module):
     def _native_decode(self, hidden_states) -> Optional[torch.Tensor]:
         """One decode step of a pre-LN block of plain modules as ``en_block_decode``: five launches, the output written
         straight into the history.  ``None``, with nothing done, where it does not apply (post-LN, separate q, k, v
-        projections, gradients, autocast or tuned GEMMs asked for, modules replaced or hooked, shapes without a kernel)."""
+        projections, gradients, autocast or tuned GEMMs asked for, modules replaced, hooked or given a ``forward`` of their own, weights of
+        a tensor subclass, shapes without a kernel)."""
         m = self._modules
         attn, mlp, norm1, norm2 = m["attn"], m["mlp"], m["norm1"], m["norm2"]
         if self.apply_post_layernorm or type(self)._rows is not Block1D._rows or type(attn) is not MultiHeadAttention1D \
                 or type(mlp) is not MLP1D or type(norm1) is not LayerNorm or type(norm2) is not LayerNorm or not attn.fused_qkv \
                 or attn.kv_cache is None or hidden_states.dim() != 3 or torch.is_grad_enabled() or torch.is_autocast_enabled() \
-                or gemm_tuning():
+                or gemm_tuning() or nn.modules.module._has_any_global_hook():
             return None
         am, mm = attn._modules, mlp._modules
         qkv, dense, fc1, fc2 = am["query_key_value"], am["dense"], mm["dense_1"], mm["dense_2"]
         for sub in (qkv, dense, fc1, fc2):
             if type(sub) is not nn.Linear:
                 return None
-        for sub in (attn, mlp, norm1, norm2, qkv, dense, fc1, fc2):
-            if sub._forward_hooks or sub._forward_pre_hooks:
+        act_fn = mlp.activation
+        for sub in (attn, mlp, norm1, norm2, qkv, dense, fc1, fc2, act_fn if isinstance(act_fn, nn.Module) else qkv):
+            if sub._forward_hooks or sub._forward_pre_hooks or "forward" in sub.__dict__:
                 return None
-        act = activation_code(mlp.activation)
+        act = activation_code(act_fn)
         if act is None:
             return None
         cache, history = attn.kv_cache, self._history

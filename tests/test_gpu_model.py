@@ -370,3 +370,40 @@ def test_block_decode_in_one_native_call(dtype, B, heads, D, ratio, act, bias, p
             assert max_abs(got[:, -1].float().cpu(), want[:, -1]) <= tol, step
             assert blk.attn.kv_cache.lens.tolist() == [n + step + 1 for n in lens]
             assert blk.attn.kv_cache.lens._version > before
+
+
+@pytest.mark.parametrize("how", ["global_hook", "own_forward", "activation_hook", "weight_subclass"])
+def test_block_decode_sees_what_a_caller_put_in(how):
+    """Decode steps of a block whose modules a caller has instrumented run what the caller put there."""
+    _, M = _mods()
+    blk = M.Block1D(128, 2, 2.0, activation=torch.nn.ReLU(), dtype=torch.float16, max_seq_len=32).cuda()
+    _init(blk, 51)
+    calls = []
+
+    class Counted(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            calls.append(func)
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    lin, handle = blk.mlp.dense_2, None
+    announce("block decode instrumented", how)
+    x = torch.randn(2, 8, 128, dtype=torch.float16, device="cuda")
+    with torch.no_grad():
+        blk(x, first_cache=True, seq_lens=torch.tensor([8, 5], dtype=torch.int32, device="cuda"))
+        if how == "global_hook":
+            handle = torch.nn.modules.module.register_module_forward_hook(lambda m, a, y: calls.append(m))
+        elif how == "own_forward":
+            lin.forward = lambda h: (calls.append(h), torch.nn.functional.linear(h, lin.weight, lin.bias))[1]
+            blk.norm1.forward = (lambda f: lambda h: (calls.append(h), f(h))[1])(blk.norm1.forward)
+        elif how == "activation_hook":
+            blk.mlp.activation.register_forward_pre_hook(lambda m, a: calls.append(m))
+        else:
+            lin._parameters["weight"] = lin.weight.detach().as_subclass(Counted)
+        try:
+            del calls[:]
+            out = blk._native_decode(x[:, :1])
+        finally:
+            if handle is not None:
+                handle.remove()
+    assert out is None and blk._history.cur == 8 and blk.attn.kv_cache.lens.tolist() == [8, 5]
