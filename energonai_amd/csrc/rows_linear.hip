@@ -62,7 +62,7 @@ __device__ __forceinline__ floatx4 mfma16(const uint4 &a, const uint4 &b, floatx
 
 __device__ __forceinline__ float activate(float v, int act) {
   switch (act) {
-    case EN_ACT_RELU: return fmaxf(v, 0.f);
+    case EN_ACT_RELU: return v < 0.f ? 0.f : v;      // NaN stays NaN
     case EN_ACT_GELU_TANH: return 0.5f * v * (1.f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
     case EN_ACT_GELU: return 0.5f * v * (1.f + erff(v * 0.7071067811865476f));
     default: return v;

@@ -407,3 +407,18 @@ def test_block_decode_sees_what_a_caller_put_in(how):
             if handle is not None:
                 handle.remove()
     assert out is None and blk._history.cur == 8 and blk.attn.kv_cache.lens.tolist() == [8, 5]
+
+
+@pytest.mark.parametrize("act", [F.relu, F.gelu, torch.nn.GELU(approximate="tanh")])
+def test_block_decode_keeps_nan(act):
+    """A NaN that appears inside the MLP is in the decode step's output, whatever the activation."""
+    _, M = _mods()
+    blk = M.Block1D(128, 2, 2.0, activation=act, dtype=torch.float16, max_seq_len=32).cuda()
+    _init(blk, 52)
+    announce("block decode NaN", act)
+    x = torch.randn(2, 8, 128, dtype=torch.float16, device="cuda")
+    with torch.no_grad():
+        blk.mlp.dense_1.bias[5] = float("nan")
+        blk(x, first_cache=True, seq_lens=torch.tensor([8, 5], dtype=torch.int32, device="cuda"))
+        out = blk._native_decode(x[:, :1])
+    assert out[:, -1].isnan().all()
