@@ -74,7 +74,7 @@ class Block1D(nn.Module):
         for sub in (attn, mlp, norm1, norm2, qkv, dense, fc1, fc2, act_fn if isinstance(act_fn, nn.Module) else qkv):
             if sub._forward_hooks or sub._forward_pre_hooks or "forward" in sub.__dict__:
                 return None
-        act = activation_code(act_fn)
+        act = activation_code(act_fn, mlp._epilogue)
         if act is None:
             return None
         cache, history = attn.kv_cache, self._history

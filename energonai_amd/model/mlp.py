@@ -12,9 +12,10 @@ from .gemm import gemm_algo
 
 def _epilogue_of(activation) -> Optional[str]:
     """Name of the GEMM epilogue that computes ``activation`` exactly, if there is one."""
-    if activation in (nn.functional.relu, torch.relu) or isinstance(activation, nn.ReLU):
+    # the module classes themselves: a class derived from one computes what its own forward says
+    if activation in (nn.functional.relu, torch.relu) or type(activation) is nn.ReLU:
         return "relu"
-    if isinstance(activation, nn.GELU) and activation.approximate == "tanh":
+    if type(activation) is nn.GELU and activation.approximate == "tanh":
         return "gelu_tanh"
     if getattr(activation, "func", None) is nn.functional.gelu and \
             getattr(activation, "keywords", {}).get("approximate") == "tanh":
@@ -22,11 +23,14 @@ def _epilogue_of(activation) -> Optional[str]:
     return None
 
 
-def activation_code(activation) -> Optional[int]:
-    """The ``en_activation`` that computes ``activation`` exactly, if there is one."""
-    if activation is nn.functional.gelu or (isinstance(activation, nn.GELU) and activation.approximate == "none"):
-        return 3
-    return {"relu": 1, "gelu_tanh": 2}.get(_epilogue_of(activation))
+def activation_code(activation, epilogue: Optional[str] = None) -> Optional[int]:
+    """The ``en_activation`` that computes ``activation`` exactly, if there is one.  ``epilogue``: the one the MLP applies
+    in place of ``activation``, if any (``MLP1D.forward_rows``)."""
+    if epilogue is None:
+        if activation is nn.functional.gelu or (type(activation) is nn.GELU and activation.approximate == "none"):
+            return 3
+        epilogue = _epilogue_of(activation)
+    return {"relu": 1, "gelu_tanh": 2}.get(epilogue)
 
 
 class MLP1D(nn.Module):

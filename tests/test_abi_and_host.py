@@ -313,3 +313,24 @@ def test_paged_cache_bookkeeping_on_the_host():
         c._assign([(0, 5)])
     with pytest.raises(ValueError):
         PagedKVCache(1, 1, 64, 16, torch.float16, "cpu", page_size=24)
+
+
+@pytest.mark.parametrize("base", [torch.nn.ReLU, torch.nn.GELU, lambda: torch.nn.GELU(approximate="tanh")])
+def test_activation_subclasses_are_not_taken_for_their_base(base):
+    """A module that derives from ReLU or GELU computes what its own forward says: no GEMM epilogue and no kernel's
+    activation stands in for it; the plain modules and functions keep theirs."""
+    from energonai_amd.model.mlp import _epilogue_of, activation_code
+    plain = base()
+    own = type("Own", (type(plain),), {"forward": lambda self, x: 2 * x})()
+    own.__dict__.update({k: v for k, v in plain.__dict__.items() if k == "approximate"})
+    assert activation_code(plain) in (1, 2, 3)
+    assert activation_code(own) is None and _epilogue_of(own) is None
+
+
+def test_activation_code_follows_the_epilogue_the_mlp_was_built_with():
+    """The MLP's projection applies the epilogue chosen when it was built, whatever stands in ``activation`` later: the
+    decode step's kernel is told the same."""
+    from energonai_amd.model.mlp import activation_code
+    F = torch.nn.functional
+    assert [activation_code(a) for a in (F.relu, torch.relu, F.gelu, F.silu)] == [1, 1, 3, None]
+    assert activation_code(F.gelu, "relu") == 1 and activation_code(F.silu, "gelu_tanh") == 2

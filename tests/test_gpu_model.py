@@ -422,3 +422,29 @@ def test_block_decode_keeps_nan(act):
         blk(x, first_cache=True, seq_lens=torch.tensor([8, 5], dtype=torch.int32, device="cuda"))
         out = blk._native_decode(x[:, :1])
     assert out[:, -1].isnan().all()
+
+
+@pytest.mark.parametrize("how", ["gelu_subclass", "relu_subclass", "replaced_after_construction"])
+def test_block_decode_applies_the_activation_that_prefill_applies(how):
+    """Prompt and decode steps of a block go through one function: a module derived from GELU or ReLU runs its own forward,
+    and an activation put in later leaves the epilogue that the MLP was built with."""
+    _, M = _mods()
+    announce("block decode activation", how)
+    if how == "replaced_after_construction":
+        act = F.relu
+    else:
+        base = torch.nn.GELU if how == "gelu_subclass" else torch.nn.ReLU
+        act = type("Own", (base,), {"forward": lambda self, h: 1.5 * torch.sigmoid(h)})()
+    blk = M.Block1D(128, 2, 2.0, activation=act, dtype=torch.float16, max_seq_len=32).cuda()
+    _init(blk, 53)
+    if how == "replaced_after_construction":
+        blk.mlp.activation = F.gelu
+    p, lens = _fp32_params(blk), [8, 5]
+    x, valid = _padded_batch(2, 8, 128, lens, True, torch.float16, 54)
+    new = torch.randn(2, 1, 128, generator=torch.Generator().manual_seed(55)).half()
+    with torch.no_grad():
+        blk(x.cuda(), attention_mask=models.additive_mask(valid).half().cuda(), first_cache=True)
+        got = blk(new.cuda(), first_cache=False)
+    x, valid = torch.cat((x, new), 1), torch.cat((valid, torch.ones(2, 1)), 1)
+    want = models.block_forward(x, p, 2, 1e-5, False, True, models.additive_mask(valid), activation=act)
+    assert max_abs(got[:, -1].float().cpu(), want[:, -1]) <= 1.5e-2      # the bound of the block's decode steps above
