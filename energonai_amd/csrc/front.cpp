@@ -295,7 +295,7 @@ PyObject *block_decode(PyObject *const *a) {
   const Tensor &k = gpu(a[18], "k_cache", false), &v = gpu(a[19], "v_cache", false), &lens = gpu(a[20], "lens");
   const auto dt = x.scalar_type();
   const int64_t heads = integer(a[16]);
-  if ((dt != at::kHalf && dt != at::kBFloat16) || x.dim() != 3 || x.stride(2) != 1 || out.scalar_type() != dt || out.stride(2) != 1 ||
+  if ((dt != at::kHalf && dt != at::kBFloat16) || x.dim() != 3 || x.numel() == 0 || x.stride(2) != 1 || out.scalar_type() != dt || out.stride(2) != 1 ||
       k.scalar_type() != dt || k.dim() != 4 || k.stride(3) != 1 || v.sizes() != k.sizes() || v.strides() != k.strides())
     Py_RETURN_NONE;
   const int64_t B = x.size(0), hid = x.size(2), D = k.size(3), position = integer(a[24]);

@@ -448,3 +448,19 @@ def test_block_decode_applies_the_activation_that_prefill_applies(how):
     x, valid = torch.cat((x, new), 1), torch.cat((valid, torch.ones(2, 1)), 1)
     want = models.block_forward(x, p, 2, 1e-5, False, True, models.additive_mask(valid), activation=act)
     assert max_abs(got[:, -1].float().cpu(), want[:, -1]) <= 1.5e-2      # the bound of the block's decode steps above
+
+
+@pytest.mark.parametrize("shape", [(2, 0, 128), (0, 1, 128)])
+def test_block_decode_refuses_a_batch_without_a_newest_position(shape):
+    """No newest position: nothing is launched on a pointer in front of the tensor, and the general step refuses the call."""
+    _, M = _mods()
+    announce("block decode, empty", shape)
+    blk = M.Block1D(128, 2, 2.0, activation=F.relu, dtype=torch.float16, max_seq_len=32).cuda()
+    with torch.no_grad():
+        blk(torch.randn(2, 8, 128, device="cuda").half(), first_cache=True,
+            seq_lens=torch.tensor([8, 5], dtype=torch.int32, device="cuda"))
+        empty = torch.empty(shape, dtype=torch.float16, device="cuda")
+        assert blk._native_decode(empty) is None
+        with pytest.raises(RuntimeError):
+            blk(empty, first_cache=False)
+    assert blk._history.cur == 8 and blk.attn.kv_cache.lens.tolist() == [8, 5]
