@@ -254,21 +254,27 @@ PyObject *decode_layer(PyObject *const *a) {
   const auto dt = q_in.scalar_type();
   if (v.sizes() != k.sizes() || v.scalar_type() != k.scalar_type()) fail("decode_attn: k_cache and v_cache must share shape and dtype");
   if (q_in.numel() != B * H * D || dt != k.scalar_type()) fail("decode_attn: q must be [B,H,1,D] of the caches' dtype");
+  // the kernels read one length per sequence of the caches
+  if (q_in.dim() < 1 || q_in.size(0) != B || !lens.is_cuda() || lens.scalar_type() != at::kInt || lens.numel() < B || !lens.is_contiguous() ||
+      lens.device() != k.device())
+    fail("decode_attn: kv_lens must hold one int32 length for each of the caches' " + std::to_string(B) + " sequences");
   const int tag = dtype_tag(q_in, "decode_attn"), out_tag = dtype_tag(gamma_in, "layer_norm");
   if (gamma_in.scalar_type() != beta_in.scalar_type()) fail("gamma and beta must share one dtype");
-  if (beta_in.numel() != hid) fail("gamma and beta must have normalized_shape");
+  if (gamma_in.dim() != 1 || beta_in.sizes() != gamma_in.sizes()) fail("gamma and beta must have normalized_shape");
   Tensor dense;
   if (a[7] != Py_None) dense = gpu(a[7], "dense_out", false).contiguous();
   const auto in_dt = dense.defined() ? dense.scalar_type() : dt;
   if (in_dt != dt || (tag != out_tag && tag != EN_F32))
     fail("layer_norm: unsupported (input, output) dtypes (" + std::string(c10::toString(in_dt)) + ", " + c10::toString(gamma_in.scalar_type()) + ")");
-  if (dense.defined() ? (dense.size(-1) != hid || dense.numel() != B * hid) : H * D != hid)
+  if (dense.defined() ? (dense.dim() < 1 || dense.size(-1) != hid || dense.numel() != B * hid) : H * D != hid)
     fail("Given normalized_shape=[" + std::to_string(hid) + "], the LayerNorm input must have that last dimension and batch rows");
-  if (residual.scalar_type() != dt || residual.numel() != B * hid || residual.size(-1) != hid) fail("residual must match input in shape and dtype");
+  const int64_t rows[3] = {1, B, hid};
+  if (residual.scalar_type() != dt || residual.sizes() != (dense.defined() ? dense.sizes() : c10::IntArrayRef(rows)))
+    fail("residual must match input in shape and dtype");
   const c10::DeviceGuard guard(k.device());
   const Tensor q = q_in.contiguous(), res = residual.contiguous(), gamma = gamma_in.contiguous(), beta = beta_in.contiguous();
   const Tensor ctx = at::empty({B, H, 1, D}, q.options());
-  const Tensor y = at::empty(dense.defined() ? dense.sizes() : c10::IntArrayRef({1, B, hid}), gamma.options());
+  const Tensor y = at::empty(dense.defined() ? dense.sizes() : c10::IntArrayRef(rows), gamma.options());
   const int64_t need = en_decode_attn_workspace_bytes((int)B, (int)H, (int)S, (int)D);
   Tensor ws;
   if (need > 0) ws = at::empty({need}, q.options().dtype(at::kByte));

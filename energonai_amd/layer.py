@@ -224,7 +224,9 @@ def decode_layer(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
     scale = float(D) ** -0.5 if scale is None else scale
     if single_pass is None:
         single_pass = not keep and scale > 0
-    if single_pass and not keep:
+    # no residual, a projection's output of another type than the caches or of other rows than the new tokens: the calls below
+    if single_pass and not keep and residual is not None and \
+            (dense_out is None or (dense_out.dtype == q.dtype and dense_out.numel() == B * hid)):
         return _lib.front.decode_layer(q, k_cache, v_cache, info.lens, residual, gamma, beta, dense_out, eps, scale)
     probs = None
     if single_pass:

@@ -334,3 +334,34 @@ def test_activation_code_follows_the_epilogue_the_mlp_was_built_with():
     F = torch.nn.functional
     assert [activation_code(a) for a in (F.relu, torch.relu, F.gelu, F.silu)] == [1, 1, 3, None]
     assert activation_code(F.gelu, "relu") == 1 and activation_code(F.silu, "gelu_tanh") == 2
+
+
+def _decode_operands(**changes):
+    """Operands of a decode step of 2 sequences, 4 heads x 64, as fake tensors that say they are on the GPU."""
+    shapes = dict(q=(2, 4, 1, 64), k=(2, 4, 32, 64), v=(2, 4, 32, 64), lens=(2,), residual=(1, 2, 256), gamma=(256,), beta=(256,))
+    shapes.update({n: s for n, s in changes.items() if not isinstance(s, torch.dtype)})
+    types = {n: t for n, t in changes.items() if isinstance(t, torch.dtype)}
+    return [torch.empty(s, dtype=types.get(n, torch.int32 if n == "lens" else torch.float16), device="cuda") for n, s in shapes.items()]
+
+
+@pytest.mark.parametrize("changes,message", [
+    (dict(k=(8, 1, 32, 64), v=(8, 1, 32, 64)), "kv_lens must hold"),          # as many elements, other sequences than q's
+    (dict(q=(8, 1, 1, 64), k=(8, 1, 32, 64), v=(8, 1, 32, 64)), "kv_lens must hold"),
+    (dict(lens=(1,)), "kv_lens must hold"),
+    (dict(lens=torch.int64), "kv_lens must hold"),
+    (dict(q=(2, 4, 2, 64)), "q must be"),
+    (dict(gamma=(2, 128)), "normalized_shape"),
+    (dict(beta=(1, 256)), "normalized_shape"),
+    (dict(gamma=(128,), beta=(128,)), "normalized_shape"),
+    (dict(residual=(2, 1, 256)), "residual must match"),
+    (dict(residual=(512,)), "residual must match"),
+])
+def test_native_decode_layer_refuses_operands_that_do_not_fit(changes, message):
+    """The one-call decode step checks lengths, LayerNorm operands and residual as the calls it stands for do, before anything
+    is allocated or launched."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from energonai_amd import _lib
+    with FakeTensorMode():
+        q, k, v, lens, residual, gamma, beta = _decode_operands(**changes)
+        with pytest.raises(RuntimeError, match=message):
+            _lib.front.decode_layer(q, k, v, lens, residual, gamma, beta, None, 1e-5, 0.125)

@@ -547,3 +547,23 @@ def test_attention_and_layernorm_in_one_launch(dtype, lens, S, H, D, causal, lef
         again = layer.padding_removal_layer(hidden, qkv, info, H, D, gamma, beta, 1e-5, scale, causal, left)
         torch.cuda.current_stream().synchronize()
     assert torch.equal(again.float(), want)
+
+
+def test_decode_layer_operands_outside_the_native_call():
+    """A projection's output in fp32 behind fp16 caches, with more rows than new tokens, or no residual: the step takes them
+    as the separate calls do."""
+    from energonai_amd import kernel as K, layer
+    announce("decode layer, other operands")
+    g = torch.Generator().manual_seed(7)
+    B, H, S, D = 2, 4, 40, 64
+    q, kc, vc = (torch.randn(B, H, n, D, generator=g).half().cuda() for n in (1, S, S))
+    lens = torch.tensor([S, 9], dtype=torch.int32).cuda()
+    gamma, beta = torch.randn(H * D, generator=g).half().cuda(), torch.randn(H * D, generator=g).half().cuda()
+    ctx = K.decode_attn(q, kc, vc, lens).view(1, B, H * D)
+    assert torch.equal(layer.decode_layer(q, kc, vc, lens, None, gamma, beta), K.layer_norm_forward(ctx, gamma, beta, (H * D,)))
+    for dense in (torch.randn(1, B, H * D, generator=g).cuda(), torch.randn(3, B, H * D, generator=g).half().cuda()):
+        res = torch.randn(dense.shape, generator=g).to(dense.dtype).cuda()
+        got = layer.decode_layer(q, kc, vc, lens, res, gamma, beta, dense_out=dense)
+        assert torch.equal(got, K.layer_norm_forward(dense, gamma, beta, (H * D,), residual=res))
+    with pytest.raises(RuntimeError, match="kv_lens must hold"):
+        layer.decode_layer(q, kc.view(B * H, 1, S, D), vc.view(B * H, 1, S, D), lens, torch.zeros(1, B, H * D).half().cuda(), gamma, beta)
