@@ -76,12 +76,14 @@ hipStream_t stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.
 
 const int32_t *i32(const Tensor &t) { return t.data_ptr<int32_t>(); }
 
-// Launches run without the interpreter lock: a launch may wait for room in the stream's queue.
+// Launches run without the interpreter lock: a launch may wait for room in the stream's queue.  `f` is the C ABI call alone, on
+// pointers and a stream taken before; whatever it throws all the same leaves with the lock held again.
 template <typename F> int without_gil(F &&f) {
-  PyThreadState *saved = PyEval_SaveThread();
-  const int rc = f();
-  PyEval_RestoreThread(saved);
-  return rc;
+  struct Released {
+    PyThreadState *saved = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(saved); }
+  } released;
+  return f();
 }
 
 // ---- events (SeqInfo orders other streams behind the kernels that produced its arrays) -------------------------------
@@ -140,9 +142,10 @@ PyObject *prefix_sum(PyObject *const *a) {
   const c10::DeviceGuard guard(lens.device());
   const auto opt = lens.options().dtype(at::kInt);
   const Tensor cu = at::empty({batch + 1}, opt), lens32 = at::empty({batch}, opt);
-  check(without_gil([&] {
-          return en_prefix_sum(lens.data_ptr(), i64, (int)batch, cu.data_ptr<int32_t>(), lens32.data_ptr<int32_t>(), stream_of(lens));
-        }), "prefix_sum");
+  const void *src = lens.data_ptr();
+  int32_t *cu_out = cu.data_ptr<int32_t>(), *lens_out = lens32.data_ptr<int32_t>();
+  const hipStream_t stream = stream_of(lens);
+  check(without_gil([&] { return en_prefix_sum(src, i64, (int)batch, cu_out, lens_out, stream); }), "prefix_sum");
   return tuple({cu, lens32});
 }
 
@@ -156,10 +159,13 @@ PyObject *layer_tables(PyObject *const *a) {
   const int64_t n = en_attn_tile_table_elems((int)batch, (int)heads, (int)S, 0);
   const Tensor offs = at::empty({total > 0 ? total : 1}, lens.options()), table = at::empty({n > 0 ? n : 1}, lens.options()),
                arrivals = at::empty({en_attn_fused_norm_arrivals((int)batch, (int)S)}, lens.options().dtype(at::kLong));
+  const int32_t *lens_in = i32(lens), *cu_in = i32(cu);
+  int32_t *table_out = table.data_ptr<int32_t>(), *offs_out = offs.data_ptr<int32_t>();
+  uint64_t *words = reinterpret_cast<uint64_t *>(arrivals.data_ptr<int64_t>());
+  const hipStream_t stream = stream_of(lens);
   check(without_gil([&] {
-          return en_layer_tables(i32(lens), i32(cu), (int)batch, (int)S, (int)left, (int)heads, (int)tiles_first,
-                                 table.data_ptr<int32_t>(), offs.data_ptr<int32_t>(),
-                                 reinterpret_cast<uint64_t *>(arrivals.data_ptr<int64_t>()), stream_of(lens));
+          return en_layer_tables(lens_in, cu_in, (int)batch, (int)S, (int)left, (int)heads, (int)tiles_first, table_out, offs_out,
+                                 words, stream);
         }), "layer_tables");
   return tuple({offs, table, arrivals});
 }
@@ -218,12 +224,15 @@ PyObject *layer(PyObject *const *a) {
     scores = at::empty({n}, opt);
   }
   auto ptr = [](const Tensor &t) -> void * { return t.defined() ? t.data_ptr() : nullptr; };
+  const void *hidden_p = hidden.data_ptr(), *qkv_p = qkv.data_ptr(), *gamma_p = gamma.data_ptr(), *beta_p = beta.data_ptr();
+  void *x_p = ptr(x), *padded_p = ptr(padded), *scores_p = ptr(scores), *ctx_p = ptr(ctx), *packed_p = ctx_packed.data_ptr(), *y_p = y.data_ptr();
+  const int32_t *lens_p = i32(lens), *cu_p = i32(cu);
+  const hipStream_t stream = stream_of(hidden);
   if (form == 2 && !has_dense && offs && a[18] != Py_None && T > 0) {      // small enough: one launch
-    const Tensor &arrivals = tensor(a[18], "arrivals");
+    uint64_t *words = reinterpret_cast<uint64_t *>(tensor(a[18], "arrivals").data_ptr<int64_t>());
     const int rc = without_gil([&] {
-      return en_attn_fused_norm(qkv.data_ptr(), ctx_packed.data_ptr(), i32(lens), i32(cu), (int)B, (int)H, (int)S, (int)D, T, scale, causal,
-                                tag, table, hidden.data_ptr(), offs, gamma.data_ptr(), beta.data_ptr(), y.data_ptr(), eps,
-                                reinterpret_cast<uint64_t *>(arrivals.data_ptr<int64_t>()), -1, stream_of(hidden));
+      return en_attn_fused_norm(qkv_p, packed_p, lens_p, cu_p, (int)B, (int)H, (int)S, (int)D, T, scale, causal, tag, table, hidden_p, offs,
+                                gamma_p, beta_p, y_p, eps, words, -1, stream);
     });
     if (rc != EN_ERR_UNSUPPORTED) {
       check(rc, "padding_removal_layer");
@@ -231,10 +240,8 @@ PyObject *layer(PyObject *const *a) {
     }
   }
   check(without_gil([&] {
-          return en_padding_removal_layer(hidden.data_ptr(), qkv.data_ptr(), dense, gamma.data_ptr(), beta.data_ptr(), ptr(x),
-                                          ptr(padded), ptr(scores), ptr(ctx), ctx_packed.data_ptr(), y.data_ptr(), i32(cu), i32(lens),
-                                          (int)B, (int)S, (int)H, (int)D, hid, T, scale, eps, causal, left, form, offs, tag, table,
-                                          stream_of(hidden));
+          return en_padding_removal_layer(hidden_p, qkv_p, dense, gamma_p, beta_p, x_p, padded_p, scores_p, ctx_p, packed_p, y_p, cu_p, lens_p,
+                                          (int)B, (int)S, (int)H, (int)D, hid, T, scale, eps, causal, left, form, offs, tag, table, stream);
         }), "padding_removal_layer");
   return THPVariable_Wrap(y);
 }
@@ -279,11 +286,14 @@ PyObject *decode_layer(PyObject *const *a) {
   Tensor ws;
   if (need > 0) ws = at::empty({need}, q.options().dtype(at::kByte));
   const int64_t ks[3] = {k.stride(0), k.stride(1), k.stride(2)}, vs[3] = {v.stride(0), v.stride(1), v.stride(2)};
+  const void *q_p = q.data_ptr(), *k_p = k.data_ptr(), *v_p = v.data_ptr(), *dense_p = dense.defined() ? dense.data_ptr() : nullptr,
+             *res_p = res.data_ptr(), *gamma_p = gamma.data_ptr(), *beta_p = beta.data_ptr();
+  void *ctx_p = ctx.data_ptr(), *y_p = y.data_ptr(), *ws_p = need > 0 ? ws.data_ptr() : nullptr;
+  const int32_t *lens_p = i32(lens);
+  const hipStream_t stream = stream_of(k);
   check(without_gil([&] {
-          return en_decode_layer(q.data_ptr(), k.data_ptr(), v.data_ptr(), ctx.data_ptr(), i32(lens), (int)B, (int)H, (int)S, (int)D,
-                                 ks, vs, scale, dense.defined() ? dense.data_ptr() : nullptr, res.data_ptr(), gamma.data_ptr(),
-                                 beta.data_ptr(), y.data_ptr(), hid, eps, tag, out_tag, need > 0 ? ws.data_ptr() : nullptr, need,
-                                 stream_of(k));
+          return en_decode_layer(q_p, k_p, v_p, ctx_p, lens_p, (int)B, (int)H, (int)S, (int)D, ks, vs, scale, dense_p, res_p, gamma_p, beta_p,
+                                 y_p, hid, eps, tag, out_tag, ws_p, need, stream);
         }), "decode_layer");
   return THPVariable_Wrap(y);
 }
@@ -350,7 +360,8 @@ PyObject *block_decode(PyObject *const *a) {
   p.workspace_bytes = en_block_decode_workspace_bytes(p.batch, p.head_num, p.size_per_head, p.mlp_width, p.cache_len);
   const Tensor ws = at::empty({p.workspace_bytes}, x.options().dtype(at::kByte));
   p.workspace = ws.data_ptr();
-  const int rc = without_gil([&] { return en_block_decode(&p, stream_of(x)); });
+  const hipStream_t stream = stream_of(x);
+  const int rc = without_gil([&] { return en_block_decode(&p, stream); });
   if (rc == EN_ERR_UNSUPPORTED || rc == EN_ERR_ALIGN) Py_RETURN_NONE;      // found before anything was launched
   check(rc, "block_decode");
   if (!lens.is_inference()) lens.unsafeGetTensorImpl()->bump_version();      // the lengths have moved on

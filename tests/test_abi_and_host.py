@@ -365,3 +365,20 @@ def test_native_decode_layer_refuses_operands_that_do_not_fit(changes, message):
         q, k, v, lens, residual, gamma, beta = _decode_operands(**changes)
         with pytest.raises(RuntimeError, match=message):
             _lib.front.decode_layer(q, k, v, lens, residual, gamma, beta, None, 1e-5, 0.125)
+
+
+@pytest.mark.parametrize("entry", ["layer", "layer_tables"])
+def test_native_calls_raise_on_lengths_of_another_type(entry):
+    """A type that the C ABI does not take is found while the interpreter lock is held: an error, not the end of the process."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from energonai_amd import _lib
+    with FakeTensorMode():
+        lens, cu = torch.empty(2, dtype=torch.int64, device="cuda"), torch.empty(3, dtype=torch.int32, device="cuda")
+        x = torch.empty(2, 8, 128, dtype=torch.float16, device="cuda")
+        gamma = torch.empty(128, dtype=torch.float16, device="cuda")
+        qkv = torch.empty(1, 9, 2, 192, dtype=torch.float16, device="cuda")
+        with pytest.raises(RuntimeError, match="expected scalar type Int"):
+            if entry == "layer":
+                _lib.front.layer(x, qkv, None, gamma, gamma, None, cu, lens, None, None, 2, 64, 9, 0.125, 1e-5, True, False, 2, None)
+            else:
+                _lib.front.layer_tables(lens, cu, 2, 8, False, 9, 2, True)
