@@ -6,6 +6,7 @@
 //
 // A plain CPython module (METH_FASTCALL, no pybind11): a call has up to twenty arguments, and converting them costs more
 // than what the call does if each goes through a type caster.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -377,10 +378,9 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
     return nullptr;
   }
   try {
-    PyObject *r = F(args);
-    return r;
-  } catch (const std::exception &e) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+    return F(args);
+  } catch (...) {      // as torch's own calls raise it: an allocation that does not fit is torch.OutOfMemoryError
+    if (!PyErr_Occurred()) torch::translate_exception_to_python(std::current_exception());
     return nullptr;
   }
 }

@@ -567,3 +567,16 @@ def test_decode_layer_operands_outside_the_native_call():
         assert torch.equal(got, K.layer_norm_forward(dense, gamma, beta, (H * D,), residual=res))
     with pytest.raises(RuntimeError, match="kv_lens must hold"):
         layer.decode_layer(q, kc.view(B * H, 1, S, D), vc.view(B * H, 1, S, D), lens, torch.zeros(1, B, H * D).half().cuda(), gamma, beta)
+
+
+def test_layer_that_does_not_fit_raises_out_of_memory():
+    """A step whose intermediates do not fit raises what torch's allocator raises, the error that callers shrink a batch on."""
+    from energonai_amd import layer
+    from energonai_amd.seqinfo import build_seq_info
+    announce("layer out of memory")
+    S, D = 1 << 20, 8                                       # scores of one head: 2 TiB
+    hidden, gamma = torch.zeros(1, S, D, dtype=torch.float16, device="cuda"), torch.ones(D, dtype=torch.float16, device="cuda")
+    info = build_seq_info(torch.tensor([1], dtype=torch.int32).cuda(), 1, total=1)
+    with pytest.raises(torch.OutOfMemoryError):
+        layer.padding_removal_layer(hidden, torch.zeros(1, 1, 1, 3 * D, dtype=torch.float16, device="cuda"), info, 1, D, gamma, gamma,
+                                    fused_attention=False)
