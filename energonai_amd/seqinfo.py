@@ -55,12 +55,12 @@ class SeqInfo:
         on another stream (the arrays are cached and reused by later calls, whichever stream those run on)."""
         if not self._ready:
             return
-        raw = _lib.stream_of(self.lens)
-        if raw in self._ordered:
+        raw, ordered = _lib.stream_of(self.lens), self._ordered
+        if raw in ordered:
             return
         for ev in self._ready:
             _lib.front.wait_event(ev, self.lens)
-        self._ordered.add(raw)
+        ordered.add(raw)                # of no consequence where another thread's launch has begun a new set meanwhile
 
     @property
     def device(self) -> torch.device:
@@ -123,11 +123,11 @@ class SeqInfo:
             return self.row_offsets(max_seq_len, left_padded), self.tile_table(head_num, max_seq_len, unit_kv_bytes)
         off_key, tab_key = (max_seq_len, left_padded, version), (head_num, max_seq_len, first, version, 128)
         off, tab = self._row_offsets.get(off_key), self._tile_tables.get(tab_key)
+        self.order_current_stream()     # behind the lookup: what it found may be another thread's, on another stream
         if off is not None and tab is not None:
             return off, tab
         if off is not None or tab is not None:
             return self.row_offsets(max_seq_len, left_padded), self.tile_table(head_num, max_seq_len, unit_kv_bytes)
-        self.order_current_stream()
         off, tab, arrivals = _lib.front.layer_tables(self.lens, self.cu_seqlens, self.batch_size, max_seq_len, left_padded,
                                                      self.total, head_num, first)
         self.produced_on_current_stream()

@@ -382,3 +382,48 @@ def test_native_calls_raise_on_lengths_of_another_type(entry):
                 _lib.front.layer(x, qkv, None, gamma, gamma, None, cu, lens, None, None, 2, 64, 9, 0.125, 1e-5, True, False, 2, None)
             else:
                 _lib.front.layer_tables(lens, cu, 2, 8, False, 9, 2, True)
+
+
+def test_cached_layer_tables_are_ordered_behind_the_launch_that_fills_them(monkeypatch):
+    """A step that finds tables another thread has just built on its own stream orders the current stream behind them after
+    the lookup; a wait that overlaps such a launch does not count for it."""
+    from energonai_amd import _lib
+    from energonai_amd.seqinfo import SeqInfo
+    lens, cu = torch.tensor([8, 1], dtype=torch.int32), torch.tensor([0, 8, 9], dtype=torch.int32)
+    info = SeqInfo(lens, cu, 2, 9, None)
+    version, waited, stream = info._lens_version(), [], [1]
+
+    class Front:
+        on_wait = None
+
+        def wait_event(self, event, t):
+            waited.append((stream[0], event))
+            if self.on_wait:
+                self.on_wait()
+
+    front = Front()
+    monkeypatch.setattr(_lib, "front", front)
+    monkeypatch.setattr(_lib, "stream_of", lambda t: stream[0])
+
+    def publish(event):            # what another thread's launch on stream 1 leaves behind
+        info._ready.append(event)
+        info._ordered = {1}
+        info._row_offsets[(8, False, version)] = info._tile_tables[(2, 8, True, version, 128)] = lens
+
+    info._ready.append("lens")
+    info._ordered = {1, 2}
+    stream[0] = 2
+    info.order_current_stream()
+    assert waited == []
+    publish("tables")
+    assert info.layer_tables(8, False, 2, 1) == (lens, lens)
+    assert (2, "tables") in waited
+    # a third stream waits while the launch happens
+    del waited[:]
+    stream[0] = 3
+    front.on_wait = lambda: (setattr(front, "on_wait", None), info._ready.clear(), publish("later"))
+    info._ready.append("lens")
+    info.order_current_stream()
+    assert 3 not in info._ordered
+    info.layer_tables(8, False, 2, 1)
+    assert (3, "later") in waited and 3 in info._ordered
