@@ -55,35 +55,46 @@ class Block1D(nn.Module):
 
     def _native_decode(self, hidden_states) -> Optional[torch.Tensor]:
         """One decode step of a pre-LN block of plain modules as ``en_block_decode``: five launches, the output written
-        straight into the history.  ``None``, with nothing done, where it does not apply (post-LN, separate q, k, v
-        projections, gradients, autocast or tuned GEMMs asked for, modules replaced, hooked or given a ``forward`` of their own, weights of
-        a tensor subclass, shapes without a kernel)."""
+        straight into the history.  ``None``, with nothing written, where it does not apply (post-LN, separate q, k, v
+        projections, gradients, autocast or tuned GEMMs asked for, modules replaced, hooked or given a ``forward`` of
+        their own, weights that are not plain parameters, shapes without a kernel)."""
         m = self._modules
-        attn, mlp, norm1, norm2 = m["attn"], m["mlp"], m["norm1"], m["norm2"]
+        attn, mlp, norm1, norm2 = m.get("attn"), m.get("mlp"), m.get("norm1"), m.get("norm2")
         if self.apply_post_layernorm or type(self)._rows is not Block1D._rows or type(attn) is not MultiHeadAttention1D \
                 or type(mlp) is not MLP1D or type(norm1) is not LayerNorm or type(norm2) is not LayerNorm or not attn.fused_qkv \
-                or attn.kv_cache is None or hidden_states.dim() != 3 or torch.is_grad_enabled() or torch.is_autocast_enabled() \
+                or hidden_states.dim() != 3 or torch.is_grad_enabled() or torch.is_autocast_enabled() \
                 or gemm_tuning() or nn.modules.module._has_any_global_hook():
             return None
+        cache, history = attn.kv_cache, self._history
+        if cache is None:
+            return None
         am, mm = attn._modules, mlp._modules
-        qkv, dense, fc1, fc2 = am["query_key_value"], am["dense"], mm["dense_1"], mm["dense_2"]
-        for sub in (qkv, dense, fc1, fc2):
+        act_fn = mlp.activation
+        linears = (am.get("query_key_value"), am.get("dense"), mm.get("dense_1"), mm.get("dense_2"))
+        for sub in linears:
             if type(sub) is not nn.Linear:
                 return None
-        act_fn = mlp.activation
-        for sub in (attn, mlp, norm1, norm2, qkv, dense, fc1, fc2, act_fn if isinstance(act_fn, nn.Module) else qkv):
-            if sub._forward_hooks or sub._forward_pre_hooks or "forward" in sub.__dict__:
+        for sub in (attn, mlp, act_fn) if isinstance(act_fn, nn.Module) else (attn, mlp):
+            d = sub.__dict__
+            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
                 return None
+        args = []
+        for sub in (norm1, linears[0], linears[1], norm2, linears[2], linears[3]):
+            d = sub.__dict__
+            p = d["_parameters"]
+            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d \
+                    or "weight" not in p or "bias" not in p or "weight" in d or "bias" in d:
+                return None
+            args.append(p["weight"])
+            args.append(p["bias"])
+            if sub is norm1 or sub is norm2:
+                args.append(sub.eps)
         act = activation_code(act_fn, mlp._epilogue)
         if act is None:
             return None
-        cache, history = attn.kv_cache, self._history
         cache.prepare_append()
         buf = history.reserve()
-        p1, p2, pq, pd, pf, pg = (sub._parameters for sub in (norm1, norm2, qkv, dense, fc1, fc2))
-        out = _lib.front.block_decode(hidden_states, p1["weight"], p1["bias"], norm1.eps, pq["weight"], pq["bias"], pd["weight"],
-                                      pd["bias"], p2["weight"], p2["bias"], norm2.eps, pf["weight"], pf["bias"], pg["weight"],
-                                      pg["bias"], act, attn.num_heads, attn.scaling, cache.k, cache.v, cache.lens,
+        out = _lib.front.block_decode(hidden_states, *args, act, attn.num_heads, attn.scaling, cache.k, cache.v, cache.lens,
                                       cache.page_table, cache.max_seq_len, buf, history.cur)
         if out is not None:
             cache.appended()

@@ -1,0 +1,69 @@
+"""CPU-only checks of which decode steps of a block go to the native call: a block of plain modules does, and whatever a
+caller has put in the way of the general step keeps that step.  The native module is replaced by a recorder."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from energonai_amd import _lib
+from energonai_amd.model import Block1D
+from energonai_amd.model.kv_cache import KVCache
+
+
+class Recorder:
+    def __init__(self):
+        self.calls = []
+
+    def block_decode(self, *args):
+        self.calls.append(args)
+        return args[0]
+
+
+@pytest.fixture
+def step(monkeypatch):
+    """A block behind its prompt of 8 positions, and a function that runs one decode step's choice of route."""
+    front = Recorder()
+    monkeypatch.setattr(_lib, "front", front)
+    blk = Block1D(128, 2, 2.0, activation=torch.nn.GELU(), dtype=torch.float16, max_seq_len=32)
+    blk.attn.kv_cache = KVCache(2, 2, 32, 64, torch.float16, "cpu")
+    blk._history.start(torch.zeros(2, 8, 128, dtype=torch.float16), 32)
+
+    def run():
+        del front.calls[:]
+        with torch.no_grad():
+            blk._native_decode(torch.zeros(2, 1, 128, dtype=torch.float16))
+        return bool(front.calls)
+
+    return blk, run
+
+
+def test_a_block_of_plain_modules_takes_the_native_call(step, monkeypatch):
+    blk, run = step
+    assert run() and blk._history.cur == 9 and blk.attn.kv_cache._longest == 1
+    with torch.device("cpu"):           # a default device alone changes nothing
+        assert run()
+
+
+def _plain_attribute(name):
+    def change(module):
+        value = getattr(module, name).detach().clone()
+        delattr(module, name)
+        setattr(module, name, value)
+    return change
+
+
+CHANGES = {
+    "weight_as_plain_attribute": lambda blk: _plain_attribute("weight")(blk.attn.dense),
+    "bias_as_plain_attribute": lambda blk: _plain_attribute("bias")(blk.mlp.dense_1),
+    "norm_weight_as_plain_attribute": lambda blk: _plain_attribute("weight")(blk.norm2),
+    "weight_as_buffer": lambda blk: (blk.mlp.dense_2.__delattr__("weight"),
+                                     blk.mlp.dense_2.register_buffer("weight", torch.zeros(128, 256, dtype=torch.float16))),
+    "module_as_plain_attribute": lambda blk: (lambda mlp: (blk.__delattr__("mlp"), blk.__dict__.__setitem__("mlp", mlp)))(blk.mlp),
+}
+
+
+@pytest.mark.parametrize("name", list(CHANGES))
+def test_what_a_caller_put_in_keeps_the_general_step(step, name):
+    blk, run = step
+    CHANGES[name](blk)
+    assert not run()
+    assert blk._history.cur == 8 and blk.attn.kv_cache._longest == 0
