@@ -15,7 +15,7 @@ from ..kernel import LayerNorm, depad, layer_norm_forward, repad
 from ..seqinfo import SeqInfo, seq_info
 from .attention import MultiHeadAttention1D, lens_from_mask
 from .gemm import gemm_tuning
-from .kv_cache import OutputHistory
+from .kv_cache import KVCache, OutputHistory, PagedKVCache
 from .mlp import MLP1D, activation_code
 
 
@@ -56,17 +56,21 @@ class Block1D(nn.Module):
     def _native_decode(self, hidden_states) -> Optional[torch.Tensor]:
         """One decode step of a pre-LN block of plain modules as ``en_block_decode``: five launches, the output written
         straight into the history.  ``None``, with nothing written, where it does not apply (post-LN, separate q, k, v
-        projections, gradients, autocast or tuned GEMMs asked for, modules replaced, hooked or given a ``forward`` of
-        their own, weights that are not plain parameters, shapes without a kernel)."""
-        m = self._modules
+        projections, gradients, autocast or tuned GEMMs asked for, anything that the general step calls replaced, derived or
+        hooked, weights that are not plain parameters, shapes without a kernel)."""
+        m, own = self._modules, self.__dict__
         attn, mlp, norm1, norm2 = m.get("attn"), m.get("mlp"), m.get("norm1"), m.get("norm2")
-        if self.apply_post_layernorm or type(self)._rows is not Block1D._rows or type(attn) is not MultiHeadAttention1D \
-                or type(mlp) is not MLP1D or type(norm1) is not LayerNorm or type(norm2) is not LayerNorm or not attn.fused_qkv \
-                or hidden_states.dim() != 3 or torch.is_grad_enabled() or torch.is_autocast_enabled() \
-                or gemm_tuning() or nn.modules.module._has_any_global_hook():
+        if self.apply_post_layernorm or type(self)._rows is not Block1D._rows or "_rows" in own \
+                or type(attn) is not MultiHeadAttention1D or type(mlp) is not MLP1D or type(norm1) is not LayerNorm \
+                or type(norm2) is not LayerNorm or not attn.fused_qkv or hidden_states.dim() != 3 \
+                or torch.is_grad_enabled() or torch.is_autocast_enabled() or gemm_tuning() \
+                or nn.modules.module._has_any_global_hook():
             return None
         cache, history = attn.kv_cache, self._history
-        if cache is None:
+        cache_type = type(cache)
+        if cache_type not in _CACHE_STEP or type(history) is not OutputHistory or "push" in history.__dict__ \
+                or "append" in cache.__dict__ or "attend" in cache.__dict__ \
+                or (cache_type.append, cache_type.attend) != _CACHE_STEP[cache_type] or _step_methods() != _STEP_METHODS:
             return None
         am, mm = attn._modules, mlp._modules
         act_fn = mlp.activation
@@ -76,13 +80,14 @@ class Block1D(nn.Module):
                 return None
         for sub in (attn, mlp, act_fn) if isinstance(act_fn, nn.Module) else (attn, mlp):
             d = sub.__dict__
-            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
+            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d or "forward_last" in d \
+                    or "_project" in d or "forward_rows" in d or sub._compiled_call_impl is not None:
                 return None
         args = []
         for sub in (norm1, linears[0], linears[1], norm2, linears[2], linears[3]):
             d = sub.__dict__
             p = d["_parameters"]
-            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d \
+            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d or sub._compiled_call_impl is not None \
                     or "weight" not in p or "bias" not in p or "weight" in d or "bias" in d:
                 return None
             args.append(p["weight"])
@@ -125,3 +130,14 @@ class Block1D(nn.Module):
         if not self.disable_past_cache:
             return self._history.start(out, self.max_seq_len)
         return out
+
+
+def _step_methods():
+    """What the general decode step runs, as it stands now."""
+    return (Block1D._rows, MultiHeadAttention1D.forward_last, MultiHeadAttention1D._project, MLP1D.forward_rows, LayerNorm.forward,
+            nn.Linear.forward, OutputHistory.push)
+
+
+# ... and as it was written: where a caller has put something else in, the native step would pass it by
+_STEP_METHODS = _step_methods()
+_CACHE_STEP = {c: (c.append, c.attend) for c in (KVCache, PagedKVCache)}

@@ -338,7 +338,7 @@ def test_block_random_shapes(seed):
     (2, 17, 128, 1.0, "relu", True, None),        # too wide: the general path
     (33, 2, 64, 1.0, "relu", True, None),         # too many rows: the general path
 ])
-def test_block_decode_in_one_native_call(dtype, B, heads, D, ratio, act, bias, page):
+def test_block_decode_in_one_native_call(dtype, B, heads, D, ratio, act, bias, page, monkeypatch):
     """Decode steps of a pre-LN block through ``en_block_decode`` (where it applies) against the block recomputed over the
     whole extended batch in fp32, at the tolerance of the block's general path; lengths, caches and history move on alike."""
     _, M = _mods()
@@ -355,8 +355,9 @@ def test_block_decode_in_one_native_call(dtype, B, heads, D, ratio, act, bias, p
     with torch.no_grad():
         blk(x.cuda(), attention_mask=models.additive_mask(valid).to(dtype).cuda(), first_cache=True)
         native = B <= 32 and hid <= 2048
-        if native:      # the call itself must be what runs: with it in place the general path is never entered
-            blk.attn.forward_last = None
+        from energonai_amd import _lib
+        taken, call = [], _lib.front.block_decode      # the call itself must be what runs where it applies
+        monkeypatch.setattr(_lib.front, "block_decode", lambda *a: (lambda y: (taken.append(y is not None), y)[1])(call(*a)))
         for step in range(3):
             new = torch.randn(B, 1, hid, generator=g).to(dtype)
             x, valid = torch.cat((x, new), 1), torch.cat((valid, torch.ones(B, 1)), 1)
@@ -365,6 +366,7 @@ def test_block_decode_in_one_native_call(dtype, B, heads, D, ratio, act, bias, p
             wide = torch.zeros(B, 3, hid + 8, dtype=dtype)
             wide[:, 2:, :hid] = new
             got = blk(wide.cuda()[:, :, :hid], first_cache=False)
+            assert taken.pop() is native
             want = models.block_forward(x, p, heads, 1e-5, False, True, models.additive_mask(valid), activation=fn)
             assert got.shape == want.shape
             assert max_abs(got[:, -1].float().cpu(), want[:, -1]) <= tol, step
@@ -372,11 +374,12 @@ def test_block_decode_in_one_native_call(dtype, B, heads, D, ratio, act, bias, p
             assert blk.attn.kv_cache.lens._version > before
 
 
-@pytest.mark.parametrize("how", ["global_hook", "own_forward", "activation_hook", "weight_subclass"])
+@pytest.mark.parametrize("how", ["global_hook", "dense_2", "norm1", "forward_rows", "forward_last", "cache", "activation_hook",
+                                 "weight_subclass"])
 def test_block_decode_sees_what_a_caller_put_in(how):
     """Decode steps of a block whose modules a caller has instrumented run what the caller put there."""
     _, M = _mods()
-    blk = M.Block1D(128, 2, 2.0, activation=torch.nn.ReLU(), dtype=torch.float16, max_seq_len=32).cuda()
+    blk = M.Block1D(128, 2, 2.0, activation=torch.nn.GELU(), dtype=torch.float16, max_seq_len=32).cuda()
     _init(blk, 51)
     calls = []
 
@@ -393,20 +396,24 @@ def test_block_decode_sees_what_a_caller_put_in(how):
         blk(x, first_cache=True, seq_lens=torch.tensor([8, 5], dtype=torch.int32, device="cuda"))
         if how == "global_hook":
             handle = torch.nn.modules.module.register_module_forward_hook(lambda m, a, y: calls.append(m))
-        elif how == "own_forward":
-            lin.forward = lambda h: (calls.append(h), torch.nn.functional.linear(h, lin.weight, lin.bias))[1]
-            blk.norm1.forward = (lambda f: lambda h: (calls.append(h), f(h))[1])(blk.norm1.forward)
+        elif how in ("dense_2", "norm1", "forward_rows", "forward_last", "cache"):
+            owner, name = {"dense_2": (lin, "forward"), "norm1": (blk.norm1, "forward"), "forward_rows": (blk.mlp, "forward_rows"),
+                           "forward_last": (blk.attn, "forward_last"), "cache": (blk.attn.kv_cache, "attend")}[how]
+            method = getattr(owner, name)
+            setattr(owner, name, lambda *a, **k: (calls.append(name), method(*a, **k))[1])
         elif how == "activation_hook":
             blk.mlp.activation.register_forward_pre_hook(lambda m, a: calls.append(m))
         else:
             lin._parameters["weight"] = lin.weight.detach().as_subclass(Counted)
         try:
-            del calls[:]
             out = blk._native_decode(x[:, :1])
+            assert out is None and blk._history.cur == 8 and blk.attn.kv_cache.lens.tolist() == [8, 5]
+            del calls[:]
+            blk(x[:, :1], first_cache=False)
         finally:
             if handle is not None:
                 handle.remove()
-    assert out is None and blk._history.cur == 8 and blk.attn.kv_cache.lens.tolist() == [8, 5]
+    assert calls and blk._history.cur == 9 and blk.attn.kv_cache.lens.tolist() == [9, 6]
 
 
 @pytest.mark.parametrize("act", [F.relu, F.gelu, torch.nn.GELU(approximate="tanh")])
