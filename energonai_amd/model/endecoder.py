@@ -9,6 +9,8 @@ from typing import Callable, Optional
 
 import torch
 from torch import nn
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from .. import _lib
 from ..kernel import LayerNorm, depad, layer_norm_forward, repad
@@ -57,14 +59,14 @@ class Block1D(nn.Module):
         """One decode step of a pre-LN block of plain modules as ``en_block_decode``: five launches, the output written
         straight into the history.  ``None``, with nothing written, where it does not apply (post-LN, separate q, k, v
         projections, gradients, autocast or tuned GEMMs asked for, anything that the general step calls replaced, derived or
-        hooked, weights that are not plain parameters, shapes without a kernel)."""
+        hooked, weights that are not plain parameters, modes that want to see the projections, shapes without a kernel)."""
         m, own = self._modules, self.__dict__
         attn, mlp, norm1, norm2 = m.get("attn"), m.get("mlp"), m.get("norm1"), m.get("norm2")
         if self.apply_post_layernorm or type(self)._rows is not Block1D._rows or "_rows" in own \
                 or type(attn) is not MultiHeadAttention1D or type(mlp) is not MLP1D or type(norm1) is not LayerNorm \
                 or type(norm2) is not LayerNorm or not attn.fused_qkv or hidden_states.dim() != 3 \
                 or torch.is_grad_enabled() or torch.is_autocast_enabled() or gemm_tuning() \
-                or nn.modules.module._has_any_global_hook():
+                or nn.modules.module._has_any_global_hook() or _modes_active():
             return None
         cache, history = attn.kv_cache, self._history
         cache_type = type(cache)
@@ -141,3 +143,11 @@ def _step_methods():
 # ... and as it was written: where a caller has put something else in, the native step would pass it by
 _STEP_METHODS = _step_methods()
 _CACHE_STEP = {c: (c.append, c.attend) for c in (KVCache, PagedKVCache)}
+
+
+def _modes_active() -> bool:
+    """True under a torch function or dispatch mode (a FLOP counter, a quantising mode) other than a default device."""
+    if torch._C._len_torch_dispatch_stack() > 0:
+        return True
+    return torch._C._len_torch_function_stack() > 0 and \
+        any(type(mode) is not DeviceContext for mode in _get_current_function_mode_stack())

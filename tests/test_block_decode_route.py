@@ -2,6 +2,8 @@
 caller has put in the way of the general step keeps that step.  The native module is replaced by a recorder."""
 import pytest
 import torch
+from torch.overrides import TorchFunctionMode
+from torch.utils.flop_counter import FlopCounterMode
 
 from energonai_amd import _lib
 from energonai_amd.kernel import LayerNorm
@@ -132,3 +134,16 @@ def test_methods_replaced_on_the_class_keep_the_general_step(step, monkeypatch, 
     monkeypatch.setattr(owner, name, lambda *args, **kwargs: method(*args, **kwargs))
     assert not run()
     assert blk._history.cur == 8 and blk.attn.kv_cache._longest == 0
+
+
+class Passing(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("mode", [Passing, lambda: FlopCounterMode(display=False)])
+def test_modes_that_watch_the_projections_keep_the_general_step(step, mode):
+    blk, run = step
+    with mode():
+        assert not run()
+    assert run()
