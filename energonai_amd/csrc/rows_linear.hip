@@ -409,7 +409,9 @@ int en_block_decode(const en_block_decode_args *p, en_stream_t stream) {
   if (p->dtype != EN_F16 && p->dtype != EN_BF16) return EN_ERR_DTYPE;
   if (p->batch < 1 || p->head_num < 1 || p->size_per_head < 1 || p->mlp_width < 1 || p->cache_len < 1) return EN_ERR_SHAPE;
   const int64_t hid = (int64_t)p->head_num * p->size_per_head;
-  if (p->batch > kMaxRows || hid > kMaxWidth || p->size_per_head % 8 || p->size_per_head > 512 || p->mlp_width % 8 || p->mlp_width > INT32_MAX)
+  // the kernel's offsets into kMaxRows rows of the MLP's width and into sixteen columns of its weights are 32-bit bytes, the sign bit marking "absent"
+  if (p->batch > kMaxRows || hid > kMaxWidth || p->size_per_head % 8 || p->size_per_head > 512 || p->mlp_width % 8 ||
+      p->mlp_width * kMaxRows * 2 >= (1ll << 31))
     return EN_ERR_UNSUPPORTED;
   if ((int64_t)p->batch * p->x_stride * 2 >= (1ll << 31) || p->activation < EN_ACT_NONE || p->activation > EN_ACT_GELU) return EN_ERR_UNSUPPORTED;
   if (p->page_table && (log2_page(p->page_size) < 4 || p->max_pages_per_seq < 1 || p->num_pages < 1)) return EN_ERR_UNSUPPORTED;

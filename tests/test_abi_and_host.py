@@ -427,3 +427,41 @@ def test_cached_layer_tables_are_ordered_behind_the_launch_that_fills_them(monke
     assert 3 not in info._ordered
     info.layer_tables(8, False, 2, 1)
     assert (3, "later") in waited and 3 in info._ordered
+
+
+class _BlockDecodeArgs(ctypes.Structure):
+    """en_block_decode_args of include/energon_hip.h."""
+    _fields_ = [(name, {"p": ctypes.c_void_p, "i": ctypes.c_int, "l": ctypes.c_int64, "f": ctypes.c_float, "s": ctypes.c_int64 * 3}[kind])
+                for kind, names in (("p", "x"), ("l", "x_stride"),
+                                    ("p", "norm1_weight norm1_bias qkv_weight qkv_bias dense_weight dense_bias norm2_weight norm2_bias "
+                                          "mlp1_weight mlp1_bias mlp2_weight mlp2_bias"),
+                                    ("f", "norm1_eps norm2_eps scale"), ("i", "activation dtype batch head_num size_per_head"),
+                                    ("l", "mlp_width"), ("p", "k_cache v_cache"), ("s", "cache_strides"), ("i", "cache_len"),
+                                    ("p", "kv_lens page_table"), ("i", "max_pages_per_seq page_size num_pages"), ("p", "y"),
+                                    ("l", "y_stride"), ("p", "workspace"), ("l", "workspace_bytes")) for name in names.split()]
+
+
+@pytest.mark.parametrize("changes", [
+    dict(mlp_width=1 << 25),                       # 32 rows of it are 2 GiB: the kernel's offsets would wrap
+    dict(mlp_width=(1 << 31) - 8),
+])
+def test_block_decode_refuses_before_the_first_launch(changes):
+    """What en_block_decode has no kernels for is found before any of them runs (the addresses here are nobody's)."""
+    from energonai_amd import _lib
+    args = _BlockDecodeArgs()
+    for name, kind in args._fields_:
+        if kind is ctypes.c_void_p:
+            setattr(args, name, 1 << 20)
+    args.page_table = None
+    args.norm1_eps = args.norm2_eps = 1e-5
+    args.scale, args.activation, args.dtype, args.batch, args.head_num, args.size_per_head = 0.125, 1, 1, 2, 2, 64
+    args.x_stride = args.y_stride = 128
+    args.mlp_width, args.cache_len = 512, 32
+    args.cache_strides[:] = [2 * 32 * 64, 32 * 64, 64]
+    args.workspace_bytes = 1 << 62
+    for name, value in changes.items():
+        if name == "cache_strides":
+            args.cache_strides[:] = value
+        else:
+            setattr(args, name, value)
+    assert _lib.fn.en_block_decode(ctypes.byref(args), None) == -5      # EN_ERR_UNSUPPORTED
