@@ -238,10 +238,11 @@ int depad_and_transpose_pad(const void *hidden_padded, void *x_packed, const voi
                             int size_per_head, int elem_size, int left_padded, int zero_padding, hipStream_t stream);
 
 // decode.hip: en_decode_attn (page_table null) / en_decode_attn_paged over caches of one set of strides whose position
-// kv_lens[b] already holds the newest token: every sequence is taken one longer than its length says.
+// kv_lens[b] already holds the newest token: every sequence is taken one longer than its length says.  Without `launch`
+// the arguments are looked at and nothing runs.
 int decode_attn_ahead(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens,
                       const int32_t *page_table, int batch, int head_num, int cache_len, int max_pages_per_seq, int page_size,
                       int num_pages, int size_per_head, const int64_t *strides, float scale, int dtype, void *workspace,
-                      int64_t workspace_bytes, hipStream_t stream);
+                      int64_t workspace_bytes, bool launch, hipStream_t stream);
 
 }  // namespace en

@@ -837,14 +837,14 @@ static int dispatch_paged_dtype(const DecodeAttnArgs &a, int dtype, hipStream_t 
 int decode_attn_ahead(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens,
                       const int32_t *page_table, int batch, int head_num, int cache_len, int max_pages_per_seq, int page_size,
                       int num_pages, int size_per_head, const int64_t *strides, float scale, int dtype, void *workspace,
-                      int64_t workspace_bytes, hipStream_t stream) {
+                      int64_t workspace_bytes, bool launch, hipStream_t stream) {
   DecodeAttnArgs a;
   const int rc = page_table ? paged_attn_args(a, q, k_cache, v_cache, ctx, kv_lens, page_table, batch, head_num, max_pages_per_seq,
                                               page_size, num_pages, size_per_head, strides, strides, scale, dtype, workspace,
                                               workspace_bytes)
                             : attn_args(a, q, k_cache, v_cache, ctx, kv_lens, batch, head_num, cache_len, size_per_head, strides,
                                         strides, scale, dtype, workspace, workspace_bytes);
-  if (rc) return rc;
+  if (rc || !launch) return rc;
   a.len_add = 1;
   return page_table ? dispatch_paged_dtype(a, dtype, stream) : dispatch_attn_dtype(a, dtype, stream, true);
 }

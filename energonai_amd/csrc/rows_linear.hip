@@ -354,6 +354,12 @@ static int block_decode(const en_block_decode_args &p, hipStream_t s) {
   void *q = take(R * hid * 2), *ctx = take(R * hid * 2), *sum = take(R * hid * 4), *h = take(R * p.mlp_width * 2);
   const int64_t attn_bytes = en_decode_attn_workspace_bytes(R, p.head_num, p.cache_len, p.size_per_head);
   void *attn_ws = take(attn_bytes);
+  auto attend = [&](bool launch) {
+    return decode_attn_ahead(q, p.k_cache, p.v_cache, ctx, p.kv_lens, p.page_table, R, p.head_num, p.cache_len, p.max_pages_per_seq,
+                             p.page_size, p.num_pages, p.size_per_head, p.cache_strides, p.scale, p.dtype, attn_ws, attn_bytes, launch, s);
+  };
+  int rc = attend(false);      // whatever the attention refuses, before the caches are written
+  if (rc) return rc;
 
   // k, v, q of the new tokens; K and V straight into the caches
   RowsArgs a{};
@@ -364,11 +370,10 @@ static int block_decode(const en_block_decode_args &p, hipStream_t s) {
   a.c_sb = p.cache_strides[0]; a.c_sh = p.cache_strides[1]; a.c_ss = p.cache_strides[2];
   a.page_table = p.page_table; a.max_pages = p.max_pages_per_seq; a.num_pages = p.num_pages;
   a.lg_page = p.page_table ? log2_page(p.page_size) : 0;
-  int rc = rows_linear<DT, kNorm16, kScatterKVQ>(a, s);
+  rc = rows_linear<DT, kNorm16, kScatterKVQ>(a, s);
   if (rc) return rc;
   // attention over the caches, the new position included
-  rc = decode_attn_ahead(q, p.k_cache, p.v_cache, ctx, p.kv_lens, p.page_table, R, p.head_num, p.cache_len, p.max_pages_per_seq,
-                         p.page_size, p.num_pages, p.size_per_head, p.cache_strides, p.scale, p.dtype, attn_ws, attn_bytes, s);
+  rc = attend(true);
   if (rc) return rc;
   // output projection + residual; the lengths move on behind the last kernel that reads the old ones
   RowsArgs d{};

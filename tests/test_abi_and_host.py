@@ -444,6 +444,9 @@ class _BlockDecodeArgs(ctypes.Structure):
 @pytest.mark.parametrize("changes", [
     dict(mlp_width=1 << 25),                       # 32 rows of it are 2 GiB: the kernel's offsets would wrap
     dict(mlp_width=(1 << 31) - 8),
+    dict(scale=0.0), dict(scale=-1.0), dict(scale=float("nan")),
+    dict(cache_len=1 << 24, cache_strides=[2 << 30, 1 << 30, 64]),                            # a unit of 2 GiB
+    dict(page_table=1 << 20, max_pages_per_seq=2, page_size=16, num_pages=4, cache_strides=[1 << 32, 1 << 31, 1 << 26]),
 ])
 def test_block_decode_refuses_before_the_first_launch(changes):
     """What en_block_decode has no kernels for is found before any of them runs (the addresses here are nobody's)."""
