@@ -319,6 +319,8 @@ PyObject *block_decode(PyObject *const *a) {
   if (heads * D != hid || k.size(1) != heads || out.size(0) != B || out.size(2) != hid || position < 0 || position >= out.size(1) ||
       lens.numel() != B || lens.scalar_type() != at::kInt)
     Py_RETURN_NONE;
+  for (const Tensor *t : {&out, &k, &v, &lens})
+    if (t->device() != x.device()) Py_RETURN_NONE;
   bool usable = true;
   auto weight = [&](int i, int64_t rows, int64_t cols) -> const void * {
     if (a[i] == Py_None) return nullptr;
@@ -349,7 +351,7 @@ PyObject *block_decode(PyObject *const *a) {
   p.kv_lens = lens.data_ptr<int32_t>();
   if (a[21] != Py_None) {
     const Tensor &table = gpu(a[21], "page_table");
-    if (table.scalar_type() != at::kInt || table.dim() != 2 || table.size(0) != B) Py_RETURN_NONE;
+    if (table.scalar_type() != at::kInt || table.dim() != 2 || table.size(0) != B || table.device() != x.device()) Py_RETURN_NONE;
     p.page_table = i32(table);
     p.max_pages_per_seq = (int)table.size(1); p.page_size = (int)k.size(2); p.num_pages = (int)k.size(0);
   } else if (k.size(0) != B || k.size(2) != p.cache_len) {
