@@ -322,10 +322,14 @@ PyObject *block_decode(PyObject *const *a) {
   for (const Tensor *t : {&out, &k, &v, &lens})
     if (t->device() != x.device()) Py_RETURN_NONE;
   bool usable = true;
+  // [rows, cols] or, with rows = 1, [cols]: a weight laid out another way is the general path's to refuse
   auto weight = [&](int i, int64_t rows, int64_t cols) -> const void * {
     if (a[i] == Py_None) return nullptr;
     const Tensor &t = tensor(a[i], "weight");
-    if (!t.is_cuda() || t.device() != x.device() || t.scalar_type() != dt || !t.is_contiguous() || t.numel() != rows * cols) usable = false;
+    const int64_t shape[2] = {rows, cols};
+    if (!t.is_cuda() || t.device() != x.device() || t.scalar_type() != dt || !t.is_contiguous() ||
+        t.sizes() != (rows == 1 ? c10::IntArrayRef(&cols, 1) : c10::IntArrayRef(shape, 2)))
+      usable = false;
     return t.data_ptr();
   };
   const Tensor &w1 = tensor(a[11], "weight");

@@ -471,3 +471,19 @@ def test_block_decode_refuses_a_batch_without_a_newest_position(shape):
         with pytest.raises(RuntimeError):
             blk(empty, first_cache=False)
     assert blk._history.cur == 8 and blk.attn.kv_cache.lens.tolist() == [8, 5]
+
+
+@pytest.mark.parametrize("name", ["attn.query_key_value", "mlp.dense_1", "mlp.dense_2"])
+def test_block_decode_refuses_weights_laid_out_the_other_way(name):
+    """A weight of [in, out] has as many elements as one of [out, in] and is refused, as the library's projection refuses it."""
+    _, M = _mods()
+    announce("block decode, transposed weight", name)
+    blk = M.Block1D(128, 2, 2.0, activation=F.gelu, dtype=torch.float16, max_seq_len=32).cuda()
+    with torch.no_grad():
+        x = torch.randn(2, 8, 128, device="cuda").half()
+        blk(x, first_cache=True, seq_lens=torch.tensor([8, 5], dtype=torch.int32, device="cuda"))
+        lin = blk.get_submodule(name)
+        lin.weight = torch.nn.Parameter(lin.weight.t().contiguous())
+        assert blk._native_decode(x[:, -1:]) is None
+        with pytest.raises(RuntimeError):
+            blk(x[:, -1:], first_cache=False)
