@@ -222,8 +222,16 @@ __device__ __forceinline__ int split_share(int kl, int nsplit) {
 
 constexpr int kRankBatch = 256;
 
-__device__ __forceinline__ float2 *partial_ml(const DecodeAttnArgs &a, int64_t share_index) {
-  return reinterpret_cast<float2 *>(a.partial + (int64_t)a.B * a.H * a.nsplit * a.D) + share_index;
+// N floats of a workspace, which is 4-byte aligned and no more; the hardware takes wide accesses at such addresses.
+template <int N> struct Partial {
+  typedef float type __attribute__((ext_vector_type(N), aligned(4)));
+};
+template <> struct Partial<1> {
+  typedef float type;
+};
+
+__device__ __forceinline__ Partial<2>::type *partial_ml(const DecodeAttnArgs &a, int64_t share_index) {
+  return reinterpret_cast<Partial<2>::type *>(a.partial + (int64_t)a.B * a.H * a.nsplit * a.D) + share_index;
 }
 
 // From this size on (K and V together) the single pass reads the caches with non-temporal loads: a step walks the caches
@@ -425,7 +433,7 @@ __global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeA
     }
     if (a.nsplit > 1) {
       a.partial[share_index * a.D + d] = o;
-      if (d == 0) *partial_ml(a, share_index) = make_float2(m_all, l);
+      if (d == 0) *partial_ml(a, share_index) = Partial<2>::type{m_all, l};
     } else {
       ctx[d] = E::from_float(l > 0.f ? o / l : 0.f);
     }
@@ -438,13 +446,13 @@ __global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeA
 template <int N>
 __device__ __forceinline__ void combine_shares(const DecodeAttnArgs &a, int b, int64_t unit, int d, float (&out)[N]) {
   constexpr int kAhead = 4;
-  typedef Pack<float, N> P;
+  typedef typename Partial<N>::type P;
   float m_run = -INFINITY, l_run = 0.f;
 #pragma unroll
   for (int e = 0; e < N; ++e) out[e] = 0.f;
   int nvalid = a.nsplit;
   for (int z0 = 0; z0 < nvalid; z0 += kAhead) {
-    float2 ml[kAhead];
+    Partial<2>::type ml[kAhead];
     P o[kAhead];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
@@ -474,7 +482,10 @@ __device__ __forceinline__ void combine_shares(const DecodeAttnArgs &a, int b, i
       const float f = __builtin_amdgcn_exp2f(ml[i].x - m_new);
       l_run += ml[i].y * f;
 #pragma unroll
-      for (int e = 0; e < N; ++e) out[e] += o[i].v[e] * f;
+      for (int e = 0; e < N; ++e) {
+        if constexpr (N == 1) out[e] += o[i] * f;
+        else out[e] += o[i][e] * f;
+      }
     }
     m_run = m_new;
   }
@@ -777,7 +788,7 @@ static int attn_args(DecodeAttnArgs &a, const void *q, const void *k_cache, cons
     if (k_strides[i] < 0 || v_strides[i] < 0) return EN_ERR_UNSUPPORTED;
   // a unit's keys are shared between workgroups only when the caller brought the room for their partial results
   const int64_t need = en_decode_attn_workspace_bytes(batch, head_num, k_seq_len, size_per_head);
-  const bool split = need > 0 && workspace && workspace_bytes >= need && aligned_to(workspace, 16);
+  const bool split = need > 0 && workspace && workspace_bytes >= need && aligned_to(workspace, 4);
   a = DecodeAttnArgs{q, k_cache, v_cache, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
                      k_strides[2], v_strides[0], v_strides[1], v_strides[2], scale * 1.4426950408889634f,
                      split ? decode_split(batch, head_num, k_seq_len) : 1, static_cast<float *>(workspace)};
@@ -817,7 +828,7 @@ static int paged_attn_args(DecodeAttnArgs &a, const void *q, const void *k_pool,
   for (int i = 0; i < 3; ++i)
     if (k_strides[i] < 0 || v_strides[i] < 0) return EN_ERR_UNSUPPORTED;
   const int64_t need = en_decode_attn_workspace_bytes(batch, head_num, k_seq_len, size_per_head);
-  const bool split = need > 0 && workspace && workspace_bytes >= need && aligned_to(workspace, 16);
+  const bool split = need > 0 && workspace && workspace_bytes >= need && aligned_to(workspace, 4);
   a = DecodeAttnArgs{q, k_pool, v_pool, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides[0], k_strides[1],
                      k_strides[2], v_strides[0], v_strides[1], v_strides[2], scale * 1.4426950408889634f,
                      split ? decode_split(batch, head_num, k_seq_len) : 1, static_cast<float *>(workspace),

@@ -266,6 +266,7 @@ int en_decode_attn(const void *q, const void *k_cache, const void *v_cache, void
  * ([batch, hidden] rows), its input being dense_out or, with dense_out NULL (hidden == head_num * size_per_head), the
  * context.  Where the keys of a unit are shared between workgroups and no projection follows, the combination of the
  * shares is the LayerNorm's own first step: one launch less, and ctx (which is then not written) stays unrounded.
+ * workspace as in en_decode_attn.
  * out_dtype: type of gamma, beta and y, as in en_layernorm_fwd. */
 int en_decode_layer(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens, int batch,
                     int head_num, int k_seq_len, int size_per_head, const int64_t *k_strides, const int64_t *v_strides,

@@ -245,6 +245,26 @@ def test_decode_attn_single_pass(dtype, B, H, S, D, kv):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("skip", [4, 8, 12])
+def test_decode_attn_workspace_off_16_bytes_still_shares_units(dtype, skip):
+    """A workspace aligned to 4 bytes, as the header asks, has the keys of a unit shared as any other: same bits, and the
+    partial results in it."""
+    k = _kernel()
+    announce("decode attn workspace", dtype, skip)
+    B, H, S, D = 2, 2, 2048, 64
+    g = torch.Generator().manual_seed(skip)
+    q, kc, vc = (torch.randn(B, H, n, D, generator=g).to(dtype).cuda() for n in (1, S, S))
+    kv = torch.tensor([S, 700], dtype=torch.int32).cuda()
+    need = k.decode_attn_workspace_bytes(B, H, S, D)
+    assert need > 0
+    room = torch.full((need + 64,), 0xFF, dtype=torch.uint8, device="cuda")
+    want = k.decode_attn(q, kc, vc, kv)
+    got = k.decode_attn(q, kc, vc, kv, workspace=room[skip:skip + need])
+    assert torch.equal(got, want)
+    assert bool((room[skip:skip + 16] != 0xFF).any()) and bool((room[:skip] == 0xFF).all()) and bool((room[skip + need:] == 0xFF).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("B,H,S,D", [
     (12, 3, 256, 64),       # 256 lanes x 2 keys: short caches
     (12, 3, 257, 128),      # 256 lanes x 4 keys: few units, caches too short to share
