@@ -61,7 +61,16 @@ __global__ __launch_bounds__(rows_block(TPR)) void layernorm_rows_kernel(LnArgs 
   // they are loaded where they are used (14213 rows of 12288 fp16 166 us against 180; 9304 of 7168 67 against 70).
   // The row's own loads go out first: where the residual row is found through res_off, its address hangs on a load of
   // its own.
-  constexpr bool EARLY = VPL <= 4 && !STREAM;
+  // That takes registers, and past 64 of them a CU holds one workgroup of 1024 lanes instead of two, or three of 512 instead
+  // of four; rows of up to three vectors on up to 512 lanes are worth it.  1000 rows, without / with residual, all sent for
+  // early against a vector's operands where it is used: 16384 fp32 (1024 x 4) 26.2 / 34.1 against 21.3 / 31.2 us, 32768 fp16
+  // 27.3 / 36.6 against 21.3 / 32.0, 7168 fp32 (512 x 4) 11.4 / 14.5 against 10.0 / 14.6.
+  constexpr int HELD = VPL * (EPV + 4 + EPV * EO::kSize / 2);       // the row in fp32, residual, gamma and beta
+  constexpr bool AHEAD = HELD <= 48 || (VPL <= 3 && TPR <= 512);
+  constexpr bool EARLY = AHEAD && !STREAM;
+  // The residual alone is sent for ahead on 512 lanes (2000 rows of 7168 fp32 28.2 -> 25.9 us), and where one workgroup of
+  // 1024 is all that fits and has the room (1000 rows of 49152 fp16 63.4 -> 60 us; 65536 would spill).
+  constexpr bool RES_AHEAD = AHEAD || TPR <= 512 || (VPL * EPV > 32 && VPL * (EPV + 8) <= 96);
   uint4 raw[VPL], rraw[VPL];
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
@@ -71,17 +80,16 @@ __global__ __launch_bounds__(rows_block(TPR)) void layernorm_rows_kernel(LnArgs 
   const TO *gamma = reinterpret_cast<const TO *>(a.gamma);
   const TO *beta = reinterpret_cast<const TO *>(a.beta);
   Pack<TO, EPV> g[VPL], bt[VPL];
-  auto load_affine = [&]() {
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-      const int v = min(t + TPR * j, nvec - 1);
-      g[j] = load_pack<TO, EPV>(gamma + v * EPV);
-      bt[j] = load_pack<TO, EPV>(beta + v * EPV);
-    }
+  auto load_affine = [&](int j) {
+    const int v = min(t + TPR * j, nvec - 1);
+    g[j] = load_pack<TO, EPV>(gamma + v * EPV);
+    bt[j] = load_pack<TO, EPV>(beta + v * EPV);
   };
   const TI *res = a.residual ? reinterpret_cast<const TI *>(a.residual) + (row + (a.res_off ? a.res_off[row] : 0)) * a.n2 : nullptr;
-  if constexpr (EARLY) load_affine();
-  if (res) {
+  if constexpr (EARLY)
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) load_affine(j);
+  if (RES_AHEAD && res) {
 #pragma unroll
     for (int j = 0; j < VPL; ++j) {
       const int v = t + TPR * j;
@@ -99,7 +107,7 @@ __global__ __launch_bounds__(rows_block(TPR)) void layernorm_rows_kernel(LnArgs 
 #pragma unroll
       for (int e = 0; e < EPV; ++e) x[j][e] = EI::to_float(pk.v[e]);
       if (res) {
-        const Pack<TI, EPV> rk = __builtin_bit_cast(Pack<TI, EPV>, rraw[j]);
+        const Pack<TI, EPV> rk = __builtin_bit_cast(Pack<TI, EPV>, RES_AHEAD ? rraw[j] : load16<STREAM>(res + v * EPV));
 #pragma unroll
         for (int e = 0; e < EPV; ++e) x[j][e] += EI::to_float(rk.v[e]);
       }
@@ -134,12 +142,15 @@ __global__ __launch_bounds__(rows_block(TPR)) void layernorm_rows_kernel(LnArgs 
   const float var = d2 / (float)a.n2;
   const float inv = 1.0f / sqrtf(var + a.eps);
 
-  if constexpr (!EARLY) load_affine();
+  if constexpr (AHEAD && !EARLY)
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) load_affine(j);
   TO *out = reinterpret_cast<TO *>(a.out) + row * a.n2;
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
     const int v = t + TPR * j;
     if (v < nvec) {
+      if constexpr (!AHEAD) load_affine(j);
       Pack<TO, EPV> o;
 #pragma unroll
       for (int e = 0; e < EPV; ++e)
