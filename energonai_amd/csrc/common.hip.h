@@ -69,7 +69,8 @@ __device__ __forceinline__ Pack<T, N> load_pack(const T *p) { return *reinterpre
 template <typename T, int N>
 __device__ __forceinline__ void store_pack(T *p, const Pack<T, N> &x) { *reinterpret_cast<Pack<T, N> *>(p) = x; }
 
-// Outputs at least this large cannot stay in the 256 MB memory-side cache for the
+constexpr int64_t kMemorySideCache = 256ll << 20;
+// Outputs at least this large cannot stay in the memory-side cache for the
 // consumer kernel anyway, so they are written with non-temporal stores (measured:
 // +10..25 % on such tensors, -5 % when applied to small, cache-resident ones).
 constexpr int64_t kStreamStoreBytes = 96ll << 20;

@@ -31,8 +31,8 @@ struct LnArgs {
 // One wave per row: four rows share a workgroup and no barrier; else a workgroup is a row.
 constexpr int rows_block(int tpr) { return tpr == kWave ? kBlock : tpr; }
 
-// STREAM: the tensors are too large for the memory-side cache and pass by it with non-temporal accesses.
-template <int DTI, int DTO, int VPL, int TPR, bool STREAM>
+// STREAM, STREAM_LD: the output, and the inputs, pass by the memory-side cache with non-temporal accesses (see launch_rows).
+template <int DTI, int DTO, int VPL, int TPR, bool STREAM, bool STREAM_LD>
 __global__ __launch_bounds__(rows_block(TPR)) void layernorm_rows_kernel(LnArgs a) {
   typedef Elem<DTI> EI;
   typedef Elem<DTO> EO;
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(rows_block(TPR)) void layernorm_rows_kernel(LnArgs 
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
     const int v = t + TPR * j;
-    raw[j] = (v < nvec) ? load16<STREAM>(in + v * EPV) : make_uint4(0u, 0u, 0u, 0u);
+    raw[j] = (v < nvec) ? load16<STREAM_LD>(in + v * EPV) : make_uint4(0u, 0u, 0u, 0u);
   }
   const TO *gamma = reinterpret_cast<const TO *>(a.gamma);
   const TO *beta = reinterpret_cast<const TO *>(a.beta);
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(rows_block(TPR)) void layernorm_rows_kernel(LnArgs 
 #pragma unroll
     for (int j = 0; j < VPL; ++j) {
       const int v = t + TPR * j;
-      rraw[j] = (v < nvec) ? load16<STREAM>(res + v * EPV) : make_uint4(0u, 0u, 0u, 0u);
+      rraw[j] = (v < nvec) ? load16<STREAM_LD>(res + v * EPV) : make_uint4(0u, 0u, 0u, 0u);
     }
   }
 
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(rows_block(TPR)) void layernorm_rows_kernel(LnArgs 
 #pragma unroll
       for (int e = 0; e < EPV; ++e) x[j][e] = EI::to_float(pk.v[e]);
       if (res) {
-        const Pack<TI, EPV> rk = __builtin_bit_cast(Pack<TI, EPV>, RES_AHEAD ? rraw[j] : load16<STREAM>(res + v * EPV));
+        const Pack<TI, EPV> rk = __builtin_bit_cast(Pack<TI, EPV>, RES_AHEAD ? rraw[j] : load16<STREAM_LD>(res + v * EPV));
 #pragma unroll
         for (int e = 0; e < EPV; ++e) x[j][e] += EI::to_float(rk.v[e]);
       }
@@ -214,12 +214,16 @@ static void launch_rows(const LnArgs &a, hipStream_t s) {
   constexpr int BLOCK = rows_block(TPR);
   constexpr int ROWS_PER_BLOCK = BLOCK / TPR;
   const unsigned grid = (unsigned)ceil_div(a.n1, ROWS_PER_BLOCK);
-  // From this size on neither the inputs are still in the memory-side cache in full nor does the output stay there, and all
-  // of them go by it (in a layer: 14213 rows of 12288 fp16 with cached loads 180 us, non-temporal 166; 9304 rows of 7168,
-  // whose input the attention has just written, 68.2 against 67.2).
-  const int64_t bytes = a.n1 * a.n2 * Elem<DTO>::kSize;
-  if (bytes >= kStreamStoreBytes) layernorm_rows_kernel<DTI, DTO, VPL, TPR, true><<<grid, BLOCK, 0, s>>>(a);
-  else layernorm_rows_kernel<DTI, DTO, VPL, TPR, false><<<grid, BLOCK, 0, s>>>(a);
+  // From kStreamStoreBytes on the output does not stay in the memory-side cache.  Where input, residual and output together
+  // exceed that cache the inputs are not in it in full either, and all of them go by it (in a layer: 14213 rows of 12288 fp16
+  // with cached loads 180 us, non-temporal 166; 9304 rows of 7168, whose input the attention has just written, 68.2 against
+  // 67.2).  An input that fits it beside the output is read out of it (6000 rows of 9216 fp16 without residual, 211 MB:
+  // 33.3 us against 39.0).
+  const int64_t elems = a.n1 * a.n2, bytes = elems * Elem<DTO>::kSize;
+  const bool fits = bytes + elems * Elem<DTI>::kSize * (a.residual ? 2 : 1) <= kMemorySideCache;
+  if (bytes >= kStreamStoreBytes && !fits) layernorm_rows_kernel<DTI, DTO, VPL, TPR, true, true><<<grid, BLOCK, 0, s>>>(a);
+  else if (bytes >= kStreamStoreBytes) layernorm_rows_kernel<DTI, DTO, VPL, TPR, true, false><<<grid, BLOCK, 0, s>>>(a);
+  else layernorm_rows_kernel<DTI, DTO, VPL, TPR, false, false><<<grid, BLOCK, 0, s>>>(a);
 }
 
 // Launches the instance with the fewest of VPLS vectors per lane that cover the row.

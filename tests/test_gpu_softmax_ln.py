@@ -7,7 +7,7 @@ held to its own rounding step (2^-8 relative).
 import pytest
 import torch
 
-from gpu_util import announce, assert_stored_close, max_abs, ragged_lens
+from gpu_util import BASE, announce, assert_stored_close, max_abs, ragged_lens
 from oracle import eager
 
 pytestmark = pytest.mark.gpu
@@ -255,3 +255,26 @@ def test_layernorm_at_the_edges_of_its_lane_configurations(dtype, vectors):
     assert torch.equal(total.cpu(), (x.float() + res[torch.arange(rows) + off].float()).to(dtype))
     assert max_abs(mean.cpu(), s.mean(-1)) <= 1e-5
     assert max_abs(inv.cpu() * s.var(-1, unbiased=False).add(1e-5).sqrt(), torch.ones(rows)) <= 1e-5
+
+
+@pytest.mark.parametrize("with_residual", [False, True])
+@pytest.mark.parametrize("dtype,rows,width", [
+    (torch.float16, 6000, 9216),        # 105 MB: written past the memory-side cache; read out of it without a residual
+    (torch.float16, 1001, 65536),       # the same with eight vectors on each of 1024 lanes
+    (torch.float32, 4000, 8192),        # four vectors on 512 lanes
+    (torch.float32, 1000, 36864),       # 147 MB: input and output together pass the cache's 256 MB
+])
+def test_layernorm_of_tensors_around_the_size_of_the_memory_side_cache(dtype, rows, width, with_residual):
+    """Outputs of 96 MB and more, with inputs that fit the cache beside them and inputs that do not, in every lane of a row;
+    reference and bound as above (the reference in float32: its own error is a few 1e-7 of values up to 6)."""
+    from energonai_amd import kernel as K
+    announce("layernorm large", dtype, rows, width, with_residual)
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x, res = (torch.randn(rows, width, generator=g, device="cuda").to(dtype) for _ in range(2))
+    gamma, beta = ((c + 0.02 * torch.randn(width, generator=g, device="cuda")).to(dtype) for c in (1.0, 0.0))
+    got = K.layer_norm_forward(x, gamma, beta, (width,), 1e-5, residual=res if with_residual else None)
+    s = x.float() + res.float() if with_residual else x.float()
+    want = torch.nn.functional.layer_norm(s, (width,), gamma.float(), beta.float(), 1e-5)
+    for part in (slice(0, 64), slice(rows // 2, rows // 2 + 64), slice(rows - 64, rows)):
+        assert_stored_close(got[part].cpu(), want[part].cpu(), dtype)
+    assert float((got.float() - want).abs().max()) <= BASE[dtype] + 2.0 ** -9 * float(want.abs().max())
