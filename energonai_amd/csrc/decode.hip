@@ -257,7 +257,7 @@ __device__ __forceinline__ float across_groups(float v) {
 }
 
 template <int DT, int LPK, int NT, int U, bool STREAM, bool PAGED = false>
-__global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeAttnArgs a) {
+__global__ __launch_bounds__(NT, 4) void decode_attn_kernel(DecodeAttnArgs a) {
   typedef Elem<DT> E;
   typedef typename E::T T;
   constexpr int EPV = 16 / E::kSize;

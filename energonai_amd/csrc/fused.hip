@@ -82,17 +82,12 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
   const int b = unit / a.H, h = unit % a.H;
   int kl, ql;
   seq_extents(a, b, kl, ql);
-#ifdef EN_FUSED_START_ANCHORED
-  const int q0 = qi * kQTile;
-  if (q0 >= ql) return;
-#else
   // The query tiles of a sequence are laid from its END: tile i of n covers rows ql - (n - i) * 128 .. and the ragged
   // tile is the first one (rows below 0 do not exist), whose walk over the keys is the shortest under a causal mask.
   // Laid from the start, the ragged tile would be the last one: a few rows holding a slot for the longest walk.
   const int ntl = (ql + kQTile - 1) / kQTile;
   if (qi >= ntl) return;
   const int q0 = ql - (ntl - qi) * kQTile;
-#endif
   const int nk = tile_key_extent(a, min(q0 + kQTile, ql) - 1, kl, ql);
   const int nkt = (nk + BK - 1) / BK;
 

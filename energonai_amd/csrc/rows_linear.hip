@@ -85,7 +85,6 @@ __global__ __launch_bounds__(NW * kWave) void rows_linear_kernel(RowsArgs a) {
   constexpr int BK = HALF ? 128 : 64;           // channels per wave and step: two MFMAs per tile
   constexpr int XV = IN == kNormF32 ? 4 : 2;    // 16-byte loads of 16 channels of a row
   constexpr bool NORM = IN != kPlain;
-  constexpr bool AFFINE_EARLY = NORM && RTILES == 1 && CT == 1;   // gamma and beta travel with the weights where registers allow
   __shared__ __attribute__((aligned(16))) float s_acc[NW][RTILES * CT][kWave][4];
   __shared__ float s_sum[NORM ? 2 : 1][NW][RTILES * 16];
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
@@ -105,10 +104,10 @@ __global__ __launch_bounds__(NW * kWave) void rows_linear_kernel(RowsArgs a) {
 #pragma unroll
   for (int t = 0; t < RTILES; ++t) xrow[t] = t * 16 + jr < a.R ? (uint32_t)((int64_t)(t * 16 + jr) * a.x_stride * XS) : kOutOfRange;
 
-  uint4 w[U][CT][2], x[U][RTILES][XV], ga[AFFINE_EARLY ? U : 1][2], be[AFFINE_EARLY ? U : 1][2];
-  auto load_affine = [&](int slot, int half, int k) {
-    ga[slot][half] = buffer_load16(g_rsrc, (uint32_t)(k + 8 * half) * 2u);
-    be[slot][half] = buffer_load16(b_rsrc, (uint32_t)(k + 8 * half) * 2u);
+  uint4 w[U][CT][2], x[U][RTILES][XV], ga[2], be[2];
+  auto load_affine = [&](int half, int k) {
+    ga[half] = buffer_load16(g_rsrc, (uint32_t)(k + 8 * half) * 2u);
+    be[half] = buffer_load16(b_rsrc, (uint32_t)(k + 8 * half) * 2u);
   };
   auto fetch = [&](int u, int step) {
     const int k = step * BK + kl;
@@ -123,7 +122,6 @@ __global__ __launch_bounds__(NW * kWave) void rows_linear_kernel(RowsArgs a) {
 #pragma unroll
         for (int v = 0; v < XV / 2; ++v)
           x[u][t][half * (XV / 2) + v] = buffer_load16(x_rsrc, xrow[t] + (uint32_t)(k + 8 * half) * XS + v * 16 | xrow[t] & kOutOfRange | in);
-      if constexpr (AFFINE_EARLY) load_affine(u, half, k);
     }
   };
 #pragma unroll
@@ -198,13 +196,12 @@ __global__ __launch_bounds__(NW * kWave) void rows_linear_kernel(RowsArgs a) {
     for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
-        if constexpr (NORM && !AFFINE_EARLY) load_affine(0, half, (s0 + u * NW) * BK + kl);
+        if constexpr (NORM) load_affine(half, (s0 + u * NW) * BK + kl);
 #pragma unroll
         for (int t = 0; t < RTILES; ++t) {
           uint4 b;
           if constexpr (NORM) {
-            constexpr int slot = AFFINE_EARLY ? 1 : 0;
-            const P8 gp = __builtin_bit_cast(P8, ga[slot * u][half]), bp = __builtin_bit_cast(P8, be[slot * u][half]);
+            const P8 gp = __builtin_bit_cast(P8, ga[half]), bp = __builtin_bit_cast(P8, be[half]);
             P8 o;
 #pragma unroll
             for (int e = 0; e < 8; ++e)

@@ -20,7 +20,6 @@ from .kernel import (attn_fused, attn_fused_packed, attn_pv, attn_pv_varlen, att
                      depad, layer_norm_forward, scale_mask_softmax, scale_mask_softmax_packed, transpose_depad,
                      transpose_pad)
 from . import _lib
-from .kernel.attention import packed_scores_elems
 from .seqinfo import SeqInfo, seq_info
 
 
