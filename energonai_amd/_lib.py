@@ -50,6 +50,7 @@ SIGNATURES = {
     "en_attn_tile_table": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
     "en_layer_tables": (c_int, [c_void_p] * 2 + [c_int] * 5 + [c_void_p] * 4),
     "en_attn_fused_norm_arrivals": (c_int64, [c_int] * 2),
+    "en_attn_fused_norm_pays": (c_int, [c_int] * 4 + [c_int64, c_int]),
     "en_attn_fused_norm": (c_int, [c_void_p] * 4 + [c_int] * 4 + [c_int64, c_float, c_int, c_int] + [c_void_p] * 6 +
                            [c_float, c_void_p, c_int, c_void_p]),
     "en_attn_fused_query_tile": (c_int, [c_int] * 5),

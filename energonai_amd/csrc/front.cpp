@@ -171,8 +171,22 @@ PyObject *layer_tables(PyObject *const *a) {
   return tuple({offs, table, arrivals});
 }
 
+// The meeting words of en_attn_fused_norm for launches of this bucket on this stream, or an undefined tensor (SeqInfo.arrivals).
+Tensor meeting_words(PyObject *arrivals, int64_t max_seq_len, hipStream_t stream) {
+  if (!PyDict_Check(arrivals)) fail("arrivals must be a dict");
+  PyObject *key = Py_BuildValue("(LK)", (long long)max_seq_len, (unsigned long long)reinterpret_cast<uintptr_t>(stream));
+  if (!key) fail("arrivals: no key");
+  PyObject *words = PyDict_GetItemWithError(arrivals, key);
+  Py_DECREF(key);
+  if (!words) {
+    if (PyErr_Occurred()) fail("arrivals: no lookup");
+    return Tensor();
+  }
+  return tensor(words, "arrivals");
+}
+
 // layer(hidden_padded, qkv_packed, dense_out, gamma, beta, ctx_out, cu_seqlens, lens, row offsets or None, tile table or None,
-//       heads, size_per_head, total, scale, eps, causal, left_padded, form, meeting words or None) -> y
+//       heads, size_per_head, total, scale, eps, causal, left_padded, form, {(bucket, stream): meeting words} or None) -> y
 PyObject *layer(PyObject *const *a) {
   static const std::string who = "padding_removal_layer: ";
   const Tensor &hidden = gpu(a[0], "hidden_padded"), &qkv = gpu(a[1], "qkv_packed");
@@ -229,8 +243,11 @@ PyObject *layer(PyObject *const *a) {
   void *x_p = ptr(x), *padded_p = ptr(padded), *scores_p = ptr(scores), *ctx_p = ptr(ctx), *packed_p = ctx_packed.data_ptr(), *y_p = y.data_ptr();
   const int32_t *lens_p = i32(lens), *cu_p = i32(cu);
   const hipStream_t stream = stream_of(hidden);
-  if (form == 2 && !has_dense && offs && a[18] != Py_None && T > 0) {      // small enough: one launch
-    uint64_t *words = reinterpret_cast<uint64_t *>(tensor(a[18], "arrivals").data_ptr<int64_t>());
+  Tensor arrivals;      // small enough: one launch
+  if (form == 2 && !has_dense && offs && a[18] != Py_None && en_attn_fused_norm_pays((int)B, (int)H, (int)S, (int)D, T, tag))
+    arrivals = meeting_words(a[18], S, stream);
+  if (arrivals.defined()) {
+    uint64_t *words = reinterpret_cast<uint64_t *>(arrivals.data_ptr<int64_t>());
     const int rc = without_gil([&] {
       return en_attn_fused_norm(qkv_p, packed_p, lens_p, cu_p, (int)B, (int)H, (int)S, (int)D, T, scale, causal, tag, table, hidden_p, offs,
                                 gamma_p, beta_p, y_p, eps, words, -1, stream);

@@ -510,6 +510,12 @@ static bool one_launch_pays(int heads, int seq_len, int64_t tiles, int64_t bytes
   return (bytes >= 7 << 20 && per_wave <= 3) || (seq_len <= 64 && per_wave <= 2 && tiles * heads <= 512);
 }
 
+// Query tiles of a batch: half a tile a sequence is the ragged one, on average.
+static int64_t query_tiles(int batch, int max_seq_len, int64_t total_tokens, int dtype) {
+  const int64_t tile = dtype == EN_F32 ? kF32QTile : kQTile;
+  return max_seq_len <= tile ? batch : total_tokens / tile + (batch + 1) / 2;
+}
+
 constexpr int kNormPolls = 64;      // looks at a meeting word before a workgroup leaves its rows to the last one: tens of us
 
 static bool overlap(const void *a, int64_t a_bytes, const void *b, int64_t b_bytes) {
@@ -523,6 +529,13 @@ extern "C" {
 
 int64_t en_attn_fused_norm_arrivals(int batch, int q_seq_len) {
   return batch < 1 || q_seq_len < 1 ? 0 : batch * en::ceil_div(q_seq_len, en::kF32QTile) * en::kNormWordStride;      // the lower of the tile heights
+}
+
+int en_attn_fused_norm_pays(int batch, int head_num, int max_seq_len, int size_per_head, int64_t total_tokens, int dtype) {
+  const int es = en::dtype_size(dtype);
+  if (!es || batch < 1 || head_num < 1 || max_seq_len < 1 || size_per_head < 1 || total_tokens < 1) return 0;
+  return en::one_launch_pays(head_num, max_seq_len, en::query_tiles(batch, max_seq_len, total_tokens, dtype),
+                             total_tokens * head_num * size_per_head * es, dtype);
 }
 
 int en_attn_fused_norm(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
@@ -540,12 +553,9 @@ int en_attn_fused_norm(const void *qkv, void *ctx, const int32_t *seq_lens, cons
   if ((int64_t)max_seq_len * width * es >= (1ll << 31)) return EN_ERR_UNSUPPORTED;              // 32-bit offsets into a sequence's context
   for (const void *p : {qkv, (const void *)ctx, hidden_padded, gamma, beta, (const void *)y})
     if (!aligned_to(p, 16)) return EN_ERR_UNSUPPORTED;
-  // Workgroups that wait for one another hold their place, so all of them have to be resident at once (half a tile a
-  // sequence is the ragged one, on average).
-  const int64_t tile = dtype == EN_F32 ? kF32QTile : kQTile;
-  const int64_t tiles = max_seq_len <= tile ? batch : T / tile + (batch + 1) / 2;
-  if (tiles * head_num > resident_workgroups(size_per_head, dtype)) return EN_ERR_UNSUPPORTED;
-  if (polls < 0 && !one_launch_pays(head_num, max_seq_len, tiles, T * width * es, dtype)) return EN_ERR_UNSUPPORTED;
+  // Workgroups that wait for one another hold their place, so all of them have to be resident at once.
+  if (query_tiles(batch, max_seq_len, T, dtype) * head_num > resident_workgroups(size_per_head, dtype)) return EN_ERR_UNSUPPORTED;
+  if (polls < 0 && !en_attn_fused_norm_pays(batch, head_num, max_seq_len, size_per_head, T, dtype)) return EN_ERR_UNSUPPORTED;
   // Rows are normalised while other tiles still read: buffers that a caller has laid over each other need two launches.
   const int64_t bytes = T * width * es, meta = ((int64_t)batch + 1) * 4;
   for (const void *p : {(const void *)ctx, (const void *)y}) {

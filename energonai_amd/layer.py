@@ -142,9 +142,7 @@ def _layer_one_call(hidden_padded, qkv_packed, info, S, H, D, T, gamma, beta, ep
     table = arrivals = None
     if fold_depad and not info.ephemeral:
         offs, table = info.layer_tables(S, left, H, kv_bytes)
-        # asked for only where en_attn_fused_norm may take the step: the lookup is 0.4 us of a host-bound layer's 11
-        if form == 2 and dense_out is None and (fused_f32 or S <= 64 or T * H * D >= 7 << 19):
-            arrivals = info.arrivals(S)
+        arrivals = info._arrivals
         if fused_f32:
             table = None
     else:

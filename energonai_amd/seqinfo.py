@@ -143,7 +143,7 @@ class SeqInfo:
     def arrivals(self, max_seq_len: int):
         """The meeting words of ``en_attn_fused_norm`` for launches on the current stream, or ``None``.  They belong to the
         stream they were cleared on, whose order keeps launches apart that share them; a handle that names another stream
-        in every thread has none."""
+        in every thread has none.  (A layer step does this lookup natively, where one launch is for it.)"""
         return self._arrivals.get((max_seq_len, _lib.stream_of(self.lens)))
 
     def _mutable(self) -> bool:

@@ -364,9 +364,10 @@ int en_layer_tables(const int32_t *seq_lens, const int32_t *cu_seqlens, int batc
  * workgroups of a query tile meet at a word of `arrivals` (en_attn_fused_norm_arrivals words, zero before the first launch
  * and again after each): launches that share the array must be ordered by one stream.  `polls` bounds how often a workgroup
  * looks for the others before it leaves its rows to the last of them (any value gives the same result; < 0: the library's
- * choice, and a launch only where it is faster than two).  EN_ERR_UNSUPPORTED, with nothing launched, where it does not apply: more workgroups than are resident at once,
+ * choice, and a launch only where it is faster than two, which en_attn_fused_norm_pays says).  EN_ERR_UNSUPPORTED, with nothing launched, where it does not apply: more workgroups than are resident at once,
  * widths of more than 256 16-byte vectors, more than 48 heads, operands off 16 bytes or overlapping, a stream under capture. */
 int64_t en_attn_fused_norm_arrivals(int batch, int q_seq_len);
+int en_attn_fused_norm_pays(int batch, int head_num, int max_seq_len, int size_per_head, int64_t total_tokens, int dtype);
 int en_attn_fused_norm(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
                        int max_seq_len, int size_per_head, int64_t total_tokens, float scale, int causal, int dtype,
                        const int32_t *tile_table, const void *hidden_padded, const int32_t *residual_row_offsets,

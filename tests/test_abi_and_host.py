@@ -468,3 +468,18 @@ def test_block_decode_refuses_before_the_first_launch(changes):
         else:
             setattr(args, name, value)
     assert _lib.fn.en_block_decode(ctypes.byref(args), None) == -5      # EN_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("batch,heads,seq,D,total,dtype,pays", [
+    (24, 16, 384, 64, 3584, 2, 1),         # 16-bit context of exactly 7 MiB, three rows a wave
+    (24, 16, 384, 64, 3583, 2, 0),
+    (1, 12, 64, 64, 60, 1, 1), (1, 12, 65, 64, 60, 1, 0),       # short prompts: up to 64 rows
+    (64, 4, 64, 64, 999, 1, 0),            # four rows a wave
+    (32, 16, 64, 64, 999, 1, 1), (33, 16, 64, 64, 999, 1, 0),   # 512 workgroups
+    (8, 12, 128, 64, 600, 0, 1), (64, 4, 128, 64, 4000, 0, 0),  # fp32: two rows a wave
+    (0, 12, 64, 64, 60, 1, 0), (1, 12, 64, 64, 0, 1, 0), (1, 12, 64, 64, 60, 7, 0),
+])
+def test_one_launch_rule(batch, heads, seq, D, total, dtype, pays):
+    """Where attention and LayerNorm are one launch: the one rule that the entry point and the step in front of it follow."""
+    from energonai_amd import _lib
+    assert _lib.fn.en_attn_fused_norm_pays(batch, heads, seq, D, total, dtype) == pays
