@@ -24,8 +24,8 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kMaxWidth = 2048;
-constexpr int kMaxRows = 32;
+constexpr int kMaxWidth = EN_BLOCK_DECODE_MAX_HIDDEN;
+constexpr int kMaxRows = EN_BLOCK_DECODE_MAX_BATCH;
 
 enum RowsIn { kPlain, kNorm16, kNormF32 };                 // 16-bit rows; LayerNorm of 16-bit rows; LayerNorm of fp32 rows
 enum RowsOut { kStore, kResidualF32, kAddF32, kScatterKVQ };   // see RowsArgs

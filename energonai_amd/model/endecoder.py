@@ -21,6 +21,11 @@ from .kv_cache import KVCache, OutputHistory, PagedKVCache
 from .mlp import MLP1D, activation_code
 
 
+# what en_block_decode has kernels for (EN_BLOCK_DECODE_MAX_BATCH, EN_BLOCK_DECODE_MAX_HIDDEN)
+_NATIVE_TYPES = (torch.float16, torch.bfloat16)
+NATIVE_MAX_BATCH, NATIVE_MAX_HIDDEN = 32, 2048
+
+
 class Block1D(nn.Module):
     def __init__(self, hidden_size: int, num_heads: int, mlp_ratio: float, activation: Callable = nn.functional.gelu,
                  layernorm_epsilon: float = 1e-5, dtype: torch.dtype = torch.float16, bias: bool = True,
@@ -60,11 +65,20 @@ class Block1D(nn.Module):
         straight into the history.  ``None``, with nothing written, where it does not apply (post-LN, separate q, k, v
         projections, gradients, autocast or tuned GEMMs asked for, anything that the general step calls replaced, derived or
         hooked, weights that are not plain parameters, modes that want to see the projections, shapes without a kernel)."""
+        # first what costs least to see: blocks that stay with the general step pay for this look in every step (16 steps of
+        # fp32 or wide blocks and of other activations: 6 to 7 % of a host-bound step when the modules were gone through first)
+        if self.apply_post_layernorm or hidden_states.dim() != 3 or hidden_states.dtype not in _NATIVE_TYPES:
+            return None
+        B, _, hid = hidden_states.shape
         m, own = self._modules, self.__dict__
         attn, mlp, norm1, norm2 = m.get("attn"), m.get("mlp"), m.get("norm1"), m.get("norm2")
-        if self.apply_post_layernorm or type(self)._rows is not Block1D._rows or "_rows" in own \
-                or type(attn) is not MultiHeadAttention1D or type(mlp) is not MLP1D or type(norm1) is not LayerNorm \
-                or type(norm2) is not LayerNorm or not attn.fused_qkv or hidden_states.dim() != 3 \
+        if B > NATIVE_MAX_BATCH or hid > NATIVE_MAX_HIDDEN or type(mlp) is not MLP1D:
+            return None
+        act_fn = mlp.activation
+        act = activation_code(act_fn, mlp._epilogue)
+        if act is None or type(self)._rows is not Block1D._rows or "_rows" in own \
+                or type(attn) is not MultiHeadAttention1D or type(norm1) is not LayerNorm \
+                or type(norm2) is not LayerNorm or not attn.fused_qkv \
                 or torch.is_grad_enabled() or torch.is_autocast_enabled() or gemm_tuning() \
                 or nn.modules.module._has_any_global_hook() or _modes_active():
             return None
@@ -75,7 +89,6 @@ class Block1D(nn.Module):
                 or (cache_type.append, cache_type.attend) != _CACHE_STEP[cache_type] or _step_methods() != _STEP_METHODS:
             return None
         am, mm = attn._modules, mlp._modules
-        act_fn = mlp.activation
         linears = (am.get("query_key_value"), am.get("dense"), mm.get("dense_1"), mm.get("dense_2"))
         for sub in linears:
             if type(sub) is not nn.Linear:
@@ -96,9 +109,6 @@ class Block1D(nn.Module):
             args.append(p["bias"])
             if sub is norm1 or sub is norm2:
                 args.append(sub.eps)
-        act = activation_code(act_fn, mlp._epilogue)
-        if act is None:
-            return None
         cache.prepare_append()
         buf = history.reserve()
         out = _lib.front.block_decode(hidden_states, *args, act, attn.num_heads, attn.scaling, cache.k, cache.v, cache.lens,

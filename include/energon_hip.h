@@ -378,11 +378,14 @@ int en_attn_fused_norm(const void *qkv, void *ctx, const int32_t *seq_lens, cons
  *
  *   s = x + Wd attention(LN1(x)) + bd,   y = s + W2 act(W1 LN2(s) + b1) + b2          (energonai/model/endecoder.py:48-70)
  *
- * for the newest token of up to 32 sequences, fp16 or bf16, hidden = head_num * size_per_head of up to 2048 channels: five
+ * for the newest token of up to EN_BLOCK_DECODE_MAX_BATCH sequences, fp16 or bf16, hidden = head_num * size_per_head of up
+ * to EN_BLOCK_DECODE_MAX_HIDDEN channels: five
  * launches (seven where attention shares a unit's keys between workgroups).  The new K and V rows go to position kv_lens[b]
  * of the caches, attention sees them, and kv_lens is advanced by one; a sequence without room keeps its rows and loses the
  * new one (en_kv_append).  Weights are [out, in] as torch.nn.Linear holds them, the fused projection's outputs ordered
  * k, v, q (attention.py:74); biases may be NULL.  s stays fp32 between its two uses. */
+#define EN_BLOCK_DECODE_MAX_BATCH 32
+#define EN_BLOCK_DECODE_MAX_HIDDEN 2048
 enum en_activation { EN_ACT_NONE = 0, EN_ACT_RELU = 1, EN_ACT_GELU_TANH = 2, EN_ACT_GELU = 3 };
 typedef struct en_block_decode_args {
   const void *x;              /* [batch] rows of hidden, x_stride elements apart */

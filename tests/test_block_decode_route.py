@@ -45,6 +45,34 @@ def test_a_block_of_plain_modules_takes_the_native_call(step, monkeypatch):
         assert run()
 
 
+def test_the_limits_are_the_entry_points(step):
+    """The look that spares a call is at the limits of the header, so that neither side can move alone."""
+    import os
+    import re
+    from energonai_amd import build
+    from energonai_amd.model import endecoder
+    with open(os.path.join(build.INCLUDE, "energon_hip.h")) as f:
+        defines = dict(re.findall(r"#define EN_BLOCK_DECODE_MAX_(\w+) (\d+)", f.read()))
+    assert defines == {"BATCH": str(endecoder.NATIVE_MAX_BATCH), "HIDDEN": str(endecoder.NATIVE_MAX_HIDDEN)}
+
+
+@pytest.mark.parametrize("what", ["float32", "batch", "hidden", "activation", "post_layernorm"])
+def test_blocks_without_a_kernel_are_seen_before_their_modules_are_gone_through(step, monkeypatch, what):
+    """They stay with the general step, and what its look costs them is that of a few attributes."""
+    from energonai_amd.model import endecoder
+    blk, _ = step
+    looked = []
+    monkeypatch.setattr(endecoder, "_step_methods", lambda: looked.append(1))
+    x = torch.zeros((33 if what == "batch" else 2, 1, 2304 if what == "hidden" else 128),
+                    dtype=torch.float32 if what == "float32" else torch.float16)
+    if what == "activation":
+        blk.mlp.activation = torch.nn.SiLU()
+    blk.apply_post_layernorm = what == "post_layernorm"
+    with torch.no_grad():
+        assert blk._native_decode(x) is None
+    assert not looked and not _lib.front.calls and blk._history.cur == 8
+
+
 def _plain_attribute(name):
     def change(module):
         value = getattr(module, name).detach().clone()
