@@ -6,6 +6,7 @@
     python3 bench_profiles.py counters --workload c3     # one --pmc run of SQ counters: MFMA and VALU busy, LDS, waits
     python3 bench_profiles.py issue --workload c3        # one --pmc run: matrix / vector co-execution, address unit queues
     python3 bench_profiles.py memsys --workload c3       # three --pmc runs: L2 hit rate, requests to memory, stalled channels
+    python3 bench_profiles.py cases                      # rocprofv3 --kernel-trace --stats of every case of perf/cases.py
     python3 bench_profiles.py yardstick                  # no profiler: `bench.py --copy-yardstick` as a table
 
 Each sub-command starts rocprofv3 as a child process with `python3 bench.py ...` after `--`, reads the CSV files it
@@ -46,6 +47,7 @@ KERNEL_KEYS = [
     ("decode_qk", "decode_qk"),
     ("decode_pv", "decode_pv"),
     ("attn_fused_wide", "attn_fused_packed_wide"),
+    ("attn_fused_norm", "attn_fused_norm"),
     ("attn_fused", "attn_fused_packed"),
     ("copy_kernel", "copy"),
 ]
@@ -57,8 +59,8 @@ def key_of(kernel: str, decode: bool):
     return None
 
 
-def run_profiler(tag: str, prof_args, bench_args, timeout_s: int):
-    """rocprofv3 <prof_args> -d <raw dir>/<tag> -- python3 bench.py <bench_args>; returns (dir, bench line, command)."""
+def run_profiler(tag: str, prof_args, bench_args, timeout_s: int, script: str = "bench.py"):
+    """rocprofv3 <prof_args> -d <raw dir>/<tag> -- python3 <script> <bench_args>; returns (dir, bench line, command)."""
     global OUT
     if OUT is None:
         OUT = tempfile.mkdtemp(prefix="energon_prof_")
@@ -66,7 +68,7 @@ def run_profiler(tag: str, prof_args, bench_args, timeout_s: int):
     subprocess.run(["rm", "-rf", d], check=True)
     os.makedirs(d, exist_ok=True)
     cmd = ["rocprofv3"] + prof_args + ["--output-format", "csv", "-d", d, "-o", "run", "--",
-                                      "python3", os.path.join(ROOT, "bench.py")] + bench_args
+                                      "python3", os.path.join(ROOT, script)] + bench_args
     env = dict(os.environ, TMPDIR="/tmp")
     print("[bench_profiles] " + " ".join(cmd), file=sys.stderr, flush=True)
     proc = subprocess.run(cmd, cwd=ROOT, env=env, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True,
@@ -141,6 +143,43 @@ def cmd_trace(ns) -> int:
               f"{'' if ev is None else format(ev, '.1f')} |")
     other = sum(sum(v) for n, v in agg.items() if key_of(n, decode) is None)
     print(f"\nOther kernels in the trace (torch fills and copies while the inputs are made): {other / 1e3:.1f} ms in total.")
+    return 0
+
+
+def cmd_run_case(ns) -> int:
+    """The program that `cases` profiles: passes of one case of perf/cases.py."""
+    sys.path.insert(0, ROOT)
+    import torch
+
+    from perf import cases
+    state = cases.prepare(next(c for c in cases.listed() if c["name"] == ns.case), 1)
+    for _ in range(ns.steps):
+        cases.run(state)
+    torch.cuda.synchronize()
+    print(json.dumps({"case": ns.case, "passes": ns.steps}), flush=True)
+    return 0
+
+
+def cmd_cases(ns) -> int:
+    sys.path.insert(0, ROOT)
+    from perf import cases
+    names = [c["name"] for c in cases.listed()]
+    print("# rocprofv3 kernel-trace summary: the cases of `perf/cases.py`\n")
+    print("Command (MI355X box, repo root; the summary below is this command's stdout):\n")
+    print(f"```\npython3 bench_profiles.py cases --steps {ns.steps}\n```\n")
+    for i, name in enumerate(names):
+        d, _, _ = run_profiler(f"case_{name}", ["--kernel-trace", "--stats"],
+                                  ["run-case", "--case", name, "--steps", str(ns.steps)], ns.timeout, "bench_profiles.py")
+        if i == 0:
+            print_sources(None)
+            print(f"Kernels of the library and of hipBLASLt in {ns.steps} passes over one set of inputs, the first pass included; "
+                  "what torch launches (inputs, copies, fills) is left out.\n")
+            print("| case | kernel | calls a pass | avg us | min us | max us |\n|---|---|---|---|---|---|")
+        agg = trace_rows(find_csv(d, "kernel_trace.csv"))
+        for kernel, v in sorted(agg.items(), key=lambda kv: -sum(kv[1])):
+            if "en::" in kernel or kernel.startswith(("Cijk", "Custom_Cijk")):
+                print(f"| `{name}` | `{kernel[:110]}` | {len(v) / ns.steps:g} | {sum(v) / len(v):.1f} | {min(v):.1f} | {max(v):.1f} |")
+        print(f"[bench_profiles] {name} done", file=sys.stderr, flush=True)
     return 0
 
 
@@ -412,7 +451,7 @@ def cmd_decode(ns) -> int:
     print(f"```\npython3 bench_profiles.py decode\n  -> python3 bench.py --decode-sizes --steps {ns.steps}\n```\n")
     print_sources(line)
     print(f"{line['heads']} heads of {line['size_per_head']} channels, {line['dtype']}, every cache full; a (batch, head) "
-          "unit is one workgroup of 1024 lanes unless its keys are shared.  `as called`: what `en_decode_attn` does when "
+          "unit is one workgroup unless its keys are shared.  `as called`: what `en_decode_attn` does when "
           "the caller brings the workspace (fewer than 512 units and at least 1024 cached positions: the keys of a unit "
           "go to several workgroups and a second small kernel combines them; its time is included).  `pages`: "
           f"`en_decode_attn_paged` on the same contents in pages of {line['page']} positions with shuffled ids.  "
@@ -439,6 +478,15 @@ def main(argv=None) -> int:
     p.add_argument("--timeout", type=int, default=300)
     p.add_argument("--raw-dir", default=None)
     p.set_defaults(fn=cmd_yardstick)
+    p = sub.add_parser("cases")
+    p.add_argument("--steps", type=int, default=10)
+    p.add_argument("--timeout", type=int, default=120, help="seconds allowed for each rocprofv3 run")
+    p.add_argument("--raw-dir", default=None, help="directory for rocprofv3's raw output (default: a temporary one)")
+    p.set_defaults(fn=cmd_cases)
+    p = sub.add_parser("run-case")
+    p.add_argument("--case", required=True)
+    p.add_argument("--steps", type=int, default=10)
+    p.set_defaults(fn=cmd_run_case, raw_dir=None)
     for name, fn in (("trace", cmd_trace), ("traffic", cmd_traffic), ("counters", cmd_counters), ("issue", cmd_issue),
                      ("memsys", cmd_memsys)):
         p = sub.add_parser(name)
