@@ -214,13 +214,14 @@ static void launch_rows(const LnArgs &a, hipStream_t s) {
   constexpr int BLOCK = rows_block(TPR);
   constexpr int ROWS_PER_BLOCK = BLOCK / TPR;
   const unsigned grid = (unsigned)ceil_div(a.n1, ROWS_PER_BLOCK);
-  // From kStreamStoreBytes on the output does not stay in the memory-side cache.  Where input, residual and output together
-  // exceed that cache the inputs are not in it in full either, and all of them go by it (in a layer: 14213 rows of 12288 fp16
-  // with cached loads 180 us, non-temporal 166; 9304 rows of 7168, whose input the attention has just written, 68.2 against
-  // 67.2).  An input that fits it beside the output is read out of it (6000 rows of 9216 fp16 without residual, 211 MB:
-  // 33.3 us against 39.0).
-  const int64_t elems = a.n1 * a.n2, bytes = elems * Elem<DTO>::kSize;
-  const bool fits = bytes + elems * Elem<DTI>::kSize * (a.residual ? 2 : 1) <= kMemorySideCache;
+  // From kStreamStoreBytes on the output does not stay in the memory-side cache, and is stored past it.  The inputs are read out
+  // of that cache where they fit it, beside what the kernel that produced them read: both together, and one of them three
+  // quarters of it.  Cached / non-temporal loads, us, the input just written by a copy (and, in brackets, read again and
+  // again): 6000 rows of 9216 fp16 with residual, 222 MB, 53.6 / 54.9 (49.4 / 56.1), without 35.8 / 36.1 (34.5 / 41.5); 9304 of
+  // 7168 with residual, 267 MB, 63.4 / 63.8 (58.6 / 66.9); 8000 of 9216 with residual, 295 MB, 76.6 / 69.9 (73.5 / 73.5);
+  // 2000 of 49152 without, 197 MB, 77.1 / 74.3 (69.9 / 79.5), 9000 of 12288, 221 MB, 78.1 / 70.2 (64.6 / 75.5).
+  const int64_t elems = a.n1 * a.n2, bytes = elems * Elem<DTO>::kSize, in = elems * Elem<DTI>::kSize;
+  const bool fits = in * (a.residual ? 2 : 1) <= kMemorySideCache && in <= kMemorySideCache / 4 * 3;
   if (bytes >= kStreamStoreBytes && !fits) layernorm_rows_kernel<DTI, DTO, VPL, TPR, true, true><<<grid, BLOCK, 0, s>>>(a);
   else if (bytes >= kStreamStoreBytes) layernorm_rows_kernel<DTI, DTO, VPL, TPR, true, false><<<grid, BLOCK, 0, s>>>(a);
   else layernorm_rows_kernel<DTI, DTO, VPL, TPR, false, false><<<grid, BLOCK, 0, s>>>(a);
