@@ -147,7 +147,7 @@ class Block1D(nn.Module):
 def _step_methods():
     """What the general decode step runs, as it stands now."""
     return (Block1D._rows, MultiHeadAttention1D.forward_last, MultiHeadAttention1D._project, MLP1D.forward_rows, LayerNorm.forward,
-            nn.Linear.forward, OutputHistory.push)
+            nn.Linear.forward, nn.functional.linear, nn.GELU.forward, nn.functional.gelu, OutputHistory.push)
 
 
 # ... and as it was written: where a caller has put something else in, the native step would pass it by

@@ -154,7 +154,8 @@ def test_what_a_caller_put_in_keeps_the_general_step(step, name):
 
 
 @pytest.mark.parametrize("owner,name", [(Block1D, "_rows"), (MultiHeadAttention1D, "forward_last"), (MultiHeadAttention1D, "_project"),
-                                        (MLP1D, "forward_rows"), (LayerNorm, "forward"), (torch.nn.Linear, "forward"),
+                                        (MLP1D, "forward_rows"), (LayerNorm, "forward"), (torch.nn.Linear, "forward"), (torch.nn.functional, "linear"),
+                                        (torch.nn.GELU, "forward"), (torch.nn.functional, "gelu"),
                                         (OutputHistory, "push"), (KVCache, "append"), (KVCache, "attend")])
 def test_methods_replaced_on_the_class_keep_the_general_step(step, monkeypatch, owner, name):
     blk, run = step
