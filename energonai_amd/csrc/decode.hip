@@ -236,7 +236,8 @@ __device__ __forceinline__ Partial<2>::type *partial_ml(const DecodeAttnArgs &a,
 
 // From this size on (K and V together) the single pass reads the caches with non-temporal loads: a step walks the caches
 // of every layer before it comes back to these, and four layers of 64 MB are the whole memory-side cache (61 MB read
-// cold: 14.1 -> 13.2 us; 18 MB still in that cache: 6.3 -> 6.7 us).
+// cold: 14.1 -> 13.2 us; 18 MB still in that cache: 6.3 -> 6.7 us; 192 MB of 768 units x 64, walked full 29.4 -> 26.2 us, with
+// 1..40 keys in each sequence, which stay in the cache whatever its capacity, 6.1 -> 6.5 us).
 constexpr int64_t kAttnStreamBytes = 64ll << 20;
 
 // Sum or maximum over the lane groups of a wave (lanes that hold the same channels): every lane ends with the result.
@@ -257,7 +258,7 @@ __device__ __forceinline__ float across_groups(float v) {
 }
 
 template <int DT, int LPK, int NT, int U, bool STREAM, bool PAGED = false>
-__global__ __launch_bounds__(NT, 4) void decode_attn_kernel(DecodeAttnArgs a) {
+__global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeAttnArgs a) {
   typedef Elem<DT> E;
   typedef typename E::T T;
   constexpr int EPV = 16 / E::kSize;
@@ -403,7 +404,8 @@ __global__ __launch_bounds__(NT, 4) void decode_attn_kernel(DecodeAttnArgs a) {
 #pragma unroll
     for (int st = 0; st < NS; ++st) {
       load_stage(kr[(st + NS - 1) % NS], vr[(st + NS - 1) % NS], k0 + (st + NS - 1) * STEP);
-      compute_stage(kr[st], vr[st], k0 + st * STEP);
+      // one key per lane group and stage: a wave whose keys of this stage are all past the end has nothing to do
+      if (U > 1 || k0 + st * STEP + wkey < kend) compute_stage(kr[st], vr[st], k0 + st * STEP);
     }
   }
   // the lane groups of a wave share one maximum, add up in registers, and the waves combine through LDS
@@ -595,22 +597,36 @@ static int launch_combine_norm(const DecodeNormArgs &n, hipStream_t s) {
   return EN_OK;
 }
 
-// Which form of the kernel a call runs (lanes per workgroup x keys per lane group and stage; all hold two stages):
-//   kSmall  256 x 2   the keys of a unit are shared between workgroups, or the caches are short: start-up and the
+// Which form of the kernel a call runs (lanes per workgroup x keys per lane group and stage; all hold two stages).  The host
+// knows the capacity of the caches and not the lengths, so a form has to carry its range from caches that are nearly empty to
+// full ones.  Kernel times per call, caches of several layers walked in turn; "1..40" are lengths of 1..40 keys.
+//   kTiny   256 x 1   units that fill the chip on caches of few steps (a step: the keys 256 lanes take at once): what counts is
+//                     that all workgroups are resident (64 registers, eight waves a SIMD) and that a wave without keys left
+//                     does nothing.  1920 units x 64 fp16, capacity 128: 1..40 7.7 us, 32..128 12.9 (256 x 2: 10.0, 13.9;
+//                     512 x 4: 22.1, 26.3); capacity 512: 7.7, 128..512 30.3 (10.5, 29.1; 23.3, 36.3).  Where
+//                     few workgroups walk far, one key ahead is too few: 512 units x 64, 1..1024 keys 17.2 (256 x 2: 15.6), 768
+//                     units x 128, 1..2048 keys 76.3 (512 x 4: 70.2).
+//   kSmall  256 x 2   the keys of few units are shared between workgroups, or the caches are short: start-up and the
 //                     final combination count.  72 units of 1655 keys (61 MB), four shares each, without the combine
 //                     kernel: 13.2 us against 17.2 for 1024 x 1, 15.0 for 512 x 2; 96 units of ~70 keys 4.4 us.
-//   kDeep   512 x 4   enough units for the chip but not many rounds of them: more bytes in flight per workgroup.
-//                     640 units of 200..1000 keys 36.9 us (1024 x 1: 39.3, 256 x 4: 38.9), 768 units of 1..4000
-//                     keys 113.9 us (512 x 2: 116.1, 256 x 4: 116.0).
-//   kMany   256 x 4   many units, and few units on caches too short to share: 4608 units of 1..2048 keys (2.6 GB)
-//                     388 us, 6.8 TB/s (512 x 4: 396, 1024 x 1: 402); 72 units of 512 keys 7.9 us (256 x 2: 10.4).
-enum class AttnForm { kSmall, kDeep, kMany };
+//   kPair   512 x 2   the keys of 256..511 units are shared and a share is long: three and more workgroups a CU.  384 units x 128,
+//                     1..2048 keys, fp32 74.3 us, fp16 41.3 (256 x 2: 82.7, 45.2; 1024 x 1: 74.3, 40.5); 1..4096 147, 82 (162, 88).
+//   kDeep   512 x 4   enough units for the chip but not many rounds of them, long caches: more bytes in flight per workgroup.
+//                     768 units of 1..4000 keys 113.9 us (512 x 2: 116.1, 256 x 4: 116.0).  Nearly empty caches pay for it:
+//                     768 units x 128, capacity 2048, 1..40 fp16 13.5 us (256 x 4: 8.8, 1024 x 1: 12.2).
+//   kMany   256 x 4   between those two, many units, and few units on caches too short to share: 768 units x 64, 1..2048
+//                     keys 39.3 us (512 x 4: 40.6, 256 x 1: 41.1); 4608 units of 1..2048 keys (2.6 GB) 388 us, 6.8 TB/s
+//                     (512 x 4: 396, 1024 x 1: 402); 72 units of 512 keys 7.9 us (256 x 2: 10.4).
+enum class AttnForm { kTiny, kSmall, kPair, kDeep, kMany };
 
-static AttnForm attn_form(const DecodeAttnArgs &a) {
+static AttnForm attn_form(const DecodeAttnArgs &a, int lpk) {
   const int64_t units = (int64_t)a.B * a.H;
-  if (a.nsplit > 1) return AttnForm::kSmall;
-  if (units >= 512 && units < 2048) return AttnForm::kDeep;
-  return units < 512 && a.Sk <= 256 ? AttnForm::kSmall : AttnForm::kMany;
+  const int64_t steps = ceil_div(ceil_div(a.Sk, a.nsplit) * lpk, kBlock);      // of a workgroup, caches full
+  if (a.nsplit > 1) return units >= 256 && steps > 32 ? AttnForm::kPair : AttnForm::kSmall;
+  if (units < 256) return a.Sk <= 256 ? AttnForm::kSmall : AttnForm::kMany;
+  if (units < 512) return steps <= 8 ? AttnForm::kTiny : a.Sk <= 256 || steps <= 16 ? AttnForm::kSmall : AttnForm::kMany;
+  if (steps <= 32) return steps <= 16 || units >= 768 ? AttnForm::kTiny : AttnForm::kSmall;
+  return units < 2048 && steps > 64 ? AttnForm::kDeep : AttnForm::kMany;
 }
 
 template <int DT, int LPK, bool PAGED, int NT, int U>
@@ -621,8 +637,10 @@ static void launch_attn(const DecodeAttnArgs &a, dim3 grid, bool stream_cache, h
 
 template <int DT, int LPK, bool PAGED>
 static void launch_attn_form(const DecodeAttnArgs &a, dim3 grid, bool stream_cache, hipStream_t s) {
-  switch (attn_form(a)) {
+  switch (attn_form(a, LPK)) {
+    case AttnForm::kTiny: launch_attn<DT, LPK, PAGED, 256, 1>(a, grid, stream_cache, s); break;
     case AttnForm::kSmall: launch_attn<DT, LPK, PAGED, 256, 2>(a, grid, stream_cache, s); break;
+    case AttnForm::kPair: launch_attn<DT, LPK, PAGED, 512, 2>(a, grid, stream_cache, s); break;
     case AttnForm::kDeep: launch_attn<DT, LPK, PAGED, 512, 4>(a, grid, stream_cache, s); break;
     default: launch_attn<DT, LPK, PAGED, 256, 4>(a, grid, stream_cache, s); break;
   }

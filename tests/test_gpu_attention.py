@@ -268,9 +268,18 @@ def test_decode_attn_workspace_off_16_bytes_still_shares_units(dtype, skip):
 @pytest.mark.parametrize("B,H,S,D", [
     (12, 3, 256, 64),       # 256 lanes x 2 keys: short caches
     (12, 3, 257, 128),      # 256 lanes x 4 keys: few units, caches too short to share
-    (12, 43, 260, 96),      # 512 lanes x 4 keys: 516 units
-    (24, 86, 130, 32),      # 256 lanes x 4 keys: 2064 units
+    (12, 43, 260, 96),      # 516 units of 17 steps: 256 lanes x 1 key
+    (24, 86, 130, 32),      # 2064 units: 256 lanes x 1 key
     (12, 2, 1100, 80),      # shared keys: two shares per unit
+    (12, 22, 130, 64),      # 256 lanes x 1 key: 264 units on few steps
+    (12, 43, 131, 64),      # ... 516 units; capacities off the lane groups' multiples
+    (12, 64, 512, 128),     # ... 768 units up to 32 steps
+    (12, 43, 271, 128),     # 256 lanes x 2 keys: 516 units of 17 steps
+    (12, 43, 515, 128),     # 256 lanes x 4 keys from 33 steps on
+    (12, 43, 1028, 128),    # 512 lanes x 4 keys from 65 steps on
+    (12, 22, 259, 64),      # 256 lanes x 2 keys: 264 units from 9 steps on
+    (12, 22, 520, 80),      # ... 256 lanes x 4 keys from 17 steps on
+    (12, 22, 1029, 128),    # 512 lanes x 2 keys: shared keys of 264 units, 33 steps a share
 ])
 def test_decode_attn_forms_at_the_edges_of_their_stages(dtype, B, H, S, D):
     """Each form of the single-pass kernel with lengths around its lane groups, stages and shares."""
