@@ -9,6 +9,8 @@ from typing import Callable, Optional
 
 import torch
 from torch import nn
+from torch._C import _len_torch_dispatch_stack as _dispatch_modes, _len_torch_function_stack as _function_modes
+from torch.nn.modules.module import _has_any_global_hook
 from torch.overrides import _get_current_function_mode_stack
 from torch.utils._device import DeviceContext
 
@@ -80,7 +82,7 @@ class Block1D(nn.Module):
                 or type(attn) is not MultiHeadAttention1D or type(norm1) is not LayerNorm \
                 or type(norm2) is not LayerNorm or not attn.fused_qkv \
                 or torch.is_grad_enabled() or torch.is_autocast_enabled() or gemm_tuning() \
-                or nn.modules.module._has_any_global_hook() or _modes_active():
+                or _has_any_global_hook() or _dispatch_modes() or (_function_modes() and _modes_active()):
             return None
         cache, history = attn.kv_cache, self._history
         cache_type = type(cache)
@@ -89,17 +91,16 @@ class Block1D(nn.Module):
                 or (cache_type.append, cache_type.attend) != _CACHE_STEP[cache_type] or _step_methods() != _STEP_METHODS:
             return None
         am, mm = attn._modules, mlp._modules
-        linears = (am.get("query_key_value"), am.get("dense"), mm.get("dense_1"), mm.get("dense_2"))
-        for sub in linears:
-            if type(sub) is not nn.Linear:
-                return None
+        qkv, dense, fc1, fc2 = am.get("query_key_value"), am.get("dense"), mm.get("dense_1"), mm.get("dense_2")
+        if not (type(qkv) is type(dense) is type(fc1) is type(fc2) is nn.Linear):
+            return None
         for sub in (attn, mlp, act_fn) if isinstance(act_fn, nn.Module) else (attn, mlp):
             d = sub.__dict__
             if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d or "forward_last" in d \
                     or "_project" in d or "forward_rows" in d or sub._compiled_call_impl is not None:
                 return None
         args = []
-        for sub in (norm1, linears[0], linears[1], norm2, linears[2], linears[3]):
+        for sub in (norm1, qkv, dense, norm2, fc1, fc2):
             d = sub.__dict__
             p = d["_parameters"]
             if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d or sub._compiled_call_impl is not None \
@@ -125,11 +126,13 @@ class Block1D(nn.Module):
         return self._rows(x, lambda h: self.attn.forward_packed(h, info, batch_size, max_seq_len, fill_cache))
 
     def forward(self, hidden_states, attention_mask=None, first_cache=False, seq_lens=None):
-        B, S, hid = hidden_states.shape
-        if not self.disable_past_cache and not first_cache:
+        step = not self.disable_past_cache and not first_cache
+        if step:
             out = self._native_decode(hidden_states)
             if out is not None:
                 return out
+        B, S, hid = hidden_states.shape
+        if step:
             return self._history.push(self._rows(hidden_states[:, -1:, :].contiguous(), self.attn.forward_last))
         if seq_lens is None:
             seq_lens = lens_from_mask(attention_mask) if attention_mask is not None else \
@@ -156,8 +159,5 @@ _CACHE_STEP = {c: (c.append, c.attend) for c in (KVCache, PagedKVCache)}
 
 
 def _modes_active() -> bool:
-    """True under a torch function or dispatch mode (a FLOP counter, a quantising mode) other than a default device."""
-    if torch._C._len_torch_dispatch_stack() > 0:
-        return True
-    return torch._C._len_torch_function_stack() > 0 and \
-        any(type(mode) is not DeviceContext for mode in _get_current_function_mode_stack())
+    """True under a torch function mode (a quantising mode, a counter) other than a default device."""
+    return any(type(mode) is not DeviceContext for mode in _get_current_function_mode_stack())
