@@ -316,6 +316,76 @@ PyObject *decode_layer(PyObject *const *a) {
   return THPVariable_Wrap(y);
 }
 
+// ---- the look at a block's modules in front of block_decode ------------------------------------------------------------
+
+PyObject *name(const char *s) { return PyUnicode_InternFromString(s); }
+
+// A module without hooks, without a compiled call and without any of the methods `own` set on the instance.  `dict`: its
+// __dict__, borrowed.  -1 with a Python error set, 0 no, 1 yes.
+int plain_module(PyObject *module, std::initializer_list<PyObject *> own, PyObject *&dict) {
+  static PyObject *const hooks = name("_forward_hooks"), *const pre_hooks = name("_forward_pre_hooks"), *const compiled = name("_compiled_call_impl");
+  PyObject **at = _PyObject_GetDictPtr(module);
+  if (!at || !*at) return 0;
+  dict = *at;
+  for (PyObject *key : {hooks, pre_hooks}) {
+    PyObject *d = PyDict_GetItemWithError(dict, key);
+    if (!d) return PyErr_Occurred() ? -1 : 0;
+    const int used = PyObject_IsTrue(d);
+    if (used) return used < 0 ? -1 : 0;
+  }
+  for (PyObject *key : own) {
+    const int there = PyDict_Contains(dict, key);
+    if (there) return there < 0 ? -1 : 0;
+  }
+  PyObject *c = PyObject_GetAttr(module, compiled);
+  if (!c) return -1;
+  const bool none = c == Py_None;
+  Py_DECREF(c);
+  return none;
+}
+
+// plain_step(attention, MLP, activation or None, norm1, qkv, dense, norm2, mlp1, mlp2)
+// -> [norm1 w, b, eps, qkv w, b, dense w, b, norm2 w, b, eps, mlp1 w, b, mlp2 w, b], or None where a module is hooked or
+// compiled, has a method of its own, or holds weight or bias otherwise than as a parameter
+PyObject *plain_step(PyObject *const *a) {
+  static PyObject *const forward = name("forward"), *const last = name("forward_last"), *const project = name("_project"),
+                         *const rows = name("forward_rows"), *const parameters = name("_parameters"), *const weight = name("weight"),
+                         *const bias = name("bias"), *const eps = name("eps");
+  PyObject *dict = nullptr;
+  for (int i = 0; i < 3; ++i) {
+    if (a[i] == Py_None) continue;
+    const int ok = plain_module(a[i], {forward, last, project, rows}, dict);
+    if (ok < 0) return nullptr;
+    if (!ok) Py_RETURN_NONE;
+  }
+  PyObject *out = PyList_New(0);
+  auto done = [&](bool error) -> PyObject * {
+    Py_XDECREF(out);
+    if (error) return nullptr;
+    Py_RETURN_NONE;
+  };
+  if (!out) return nullptr;
+  for (int i = 3; i < 9; ++i) {
+    const int ok = plain_module(a[i], {forward, weight, bias}, dict);
+    if (ok != 1) return done(ok < 0);
+    PyObject *p = PyDict_GetItemWithError(dict, parameters);
+    if (!p || !PyDict_Check(p)) return done(PyErr_Occurred());
+    for (PyObject *key : {weight, bias}) {
+      PyObject *t = PyDict_GetItemWithError(p, key);
+      if (!t) return done(PyErr_Occurred());
+      if (PyList_Append(out, t)) return done(true);
+    }
+    if (i == 3 || i == 6) {
+      PyObject *e = PyObject_GetAttr(a[i], eps);
+      if (!e) return done(true);
+      const int failed = PyList_Append(out, e);
+      Py_DECREF(e);
+      if (failed) return done(true);
+    }
+  }
+  return out;
+}
+
 // block_decode(hidden, norm1 w, b, eps, qkv w, b, dense w, b, norm2 w, b, eps, mlp1 w, b, mlp2 w, b, activation, heads, scale,
 //              k_cache, v_cache, lens, page_table or None, cache_len, out [B, positions, hidden], position)
 // -> out[:, :position + 1] with the block's output for the newest position of `hidden` at `position`, or None, with nothing
@@ -421,6 +491,7 @@ PyMethodDef kMethods[] = {
     EN_FAST(layer_tables, 8, "(row offsets, tile table, meeting words) of a batch"),
     EN_FAST(layer, 19, "en_padding_removal_layer on new outputs"),
     EN_FAST(decode_layer, 10, "en_decode_layer on new outputs"),
+    EN_FAST(plain_step, 9, "what block_decode takes of a block's modules, or None where the general step has to see them"),
     EN_FAST(block_decode, 25, "en_block_decode into a position of an output history"),
     {nullptr, nullptr, 0, nullptr}};
 

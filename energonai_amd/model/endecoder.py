@@ -94,22 +94,9 @@ class Block1D(nn.Module):
         qkv, dense, fc1, fc2 = am.get("query_key_value"), am.get("dense"), mm.get("dense_1"), mm.get("dense_2")
         if not (type(qkv) is type(dense) is type(fc1) is type(fc2) is nn.Linear):
             return None
-        for sub in (attn, mlp, act_fn) if isinstance(act_fn, nn.Module) else (attn, mlp):
-            d = sub.__dict__
-            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d or "forward_last" in d \
-                    or "_project" in d or "forward_rows" in d or sub._compiled_call_impl is not None:
-                return None
-        args = []
-        for sub in (norm1, qkv, dense, norm2, fc1, fc2):
-            d = sub.__dict__
-            p = d["_parameters"]
-            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d or sub._compiled_call_impl is not None \
-                    or "weight" not in p or "bias" not in p or "weight" in d or "bias" in d:
-                return None
-            args.append(p["weight"])
-            args.append(p["bias"])
-            if sub is norm1 or sub is norm2:
-                args.append(sub.eps)
+        args = _lib.load_front().plain_step(attn, mlp, act_fn if isinstance(act_fn, nn.Module) else None, norm1, qkv, dense, norm2, fc1, fc2)
+        if args is None:
+            return None
         cache.prepare_append()
         buf = history.reserve()
         out = _lib.front.block_decode(hidden_states, *args, act, attn.num_heads, attn.scaling, cache.k, cache.v, cache.lens,
