@@ -609,8 +609,10 @@ static int launch_combine_norm(const DecodeNormArgs &n, hipStream_t s) {
 //   kSmall  256 x 2   the keys of few units are shared between workgroups, or the caches are short: start-up and the
 //                     final combination count.  72 units of 1655 keys (61 MB), four shares each, without the combine
 //                     kernel: 13.2 us against 17.2 for 1024 x 1, 15.0 for 512 x 2; 96 units of ~70 keys 4.4 us.
-//   kPair   512 x 2   the keys of 256..511 units are shared and a share is long: three and more workgroups a CU.  384 units x 128,
-//                     1..2048 keys, fp32 74.3 us, fp16 41.3 (256 x 2: 82.7, 45.2; 1024 x 1: 74.3, 40.5); 1..4096 147, 82 (162, 88).
+//   kPair   512 x 2   keys are shared and there are fewer workgroups than CUs: 48 units x 128, two shares of 700 keys each, fp16
+//                     13.7 us, fp32 19.4 with the combine kernel (256 x 2: 18.2, 27.8), 12 units x 64, 1024 keys, fp16 6.9 (7.1);
+//                     nearly empty caches 0.4 us more.  Or the keys of 256..511 units in long shares, three and more workgroups
+//                     a CU: 384 units x 128, 1..2048 keys, fp32 74.3 us, fp16 41.3 (82.7, 45.2), 1..4096 147, 82 (162, 88).
 //   kDeep   512 x 4   enough units for the chip but not many rounds of them, long caches: more bytes in flight per workgroup.
 //                     768 units of 1..4000 keys 113.9 us (512 x 2: 116.1, 256 x 4: 116.0).  Nearly empty caches pay for it:
 //                     768 units x 128, capacity 2048, 1..40 fp16 13.5 us (256 x 4: 8.8, 1024 x 1: 12.2).
@@ -622,7 +624,7 @@ enum class AttnForm { kTiny, kSmall, kPair, kDeep, kMany };
 static AttnForm attn_form(const DecodeAttnArgs &a, int lpk) {
   const int64_t units = (int64_t)a.B * a.H;
   const int64_t steps = ceil_div(ceil_div(a.Sk, a.nsplit) * lpk, kBlock);      // of a workgroup, caches full
-  if (a.nsplit > 1) return units >= 256 && steps > 32 ? AttnForm::kPair : AttnForm::kSmall;
+  if (a.nsplit > 1) return units * a.nsplit < 256 || (units >= 256 && steps > 32) ? AttnForm::kPair : AttnForm::kSmall;
   if (units < 256) return a.Sk <= 256 ? AttnForm::kSmall : AttnForm::kMany;
   if (units < 512) return steps <= 8 ? AttnForm::kTiny : a.Sk <= 256 || steps <= 16 ? AttnForm::kSmall : AttnForm::kMany;
   if (steps <= 32) return steps <= 16 || units >= 768 ? AttnForm::kTiny : AttnForm::kSmall;

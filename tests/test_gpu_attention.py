@@ -270,7 +270,8 @@ def test_decode_attn_workspace_off_16_bytes_still_shares_units(dtype, skip):
     (12, 3, 257, 128),      # 256 lanes x 4 keys: few units, caches too short to share
     (12, 43, 260, 96),      # 516 units of 17 steps: 256 lanes x 1 key
     (24, 86, 130, 32),      # 2064 units: 256 lanes x 1 key
-    (12, 2, 1100, 80),      # shared keys: two shares per unit
+    (12, 2, 1100, 80),      # 512 lanes x 2 keys: keys shared by 48 workgroups
+    (12, 11, 1100, 64),     # 256 lanes x 2 keys: keys shared by 264 workgroups
     (12, 22, 130, 64),      # 256 lanes x 1 key: 264 units on few steps
     (12, 43, 131, 64),      # ... 516 units; capacities off the lane groups' multiples
     (12, 64, 512, 128),     # ... 768 units up to 32 steps
