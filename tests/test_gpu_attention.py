@@ -268,7 +268,7 @@ def test_decode_attn_workspace_off_16_bytes_still_shares_units(dtype, skip):
 @pytest.mark.parametrize("B,H,S,D", [
     (12, 3, 256, 64),       # 256 lanes x 2 keys: short caches
     (12, 3, 257, 128),      # 256 lanes x 4 keys: few units, caches too short to share
-    (12, 43, 260, 96),      # 516 units of 17 steps: 256 lanes x 1 key
+    (12, 43, 260, 96),      # 256 lanes x 2 keys: 516 units of 17 steps
     (24, 86, 130, 32),      # 2064 units: 256 lanes x 1 key
     (12, 2, 1100, 80),      # 512 lanes x 2 keys: keys shared by 48 workgroups
     (12, 11, 1100, 64),     # 256 lanes x 2 keys: keys shared by 264 workgroups
