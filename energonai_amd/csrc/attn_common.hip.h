@@ -96,8 +96,7 @@ __device__ __forceinline__ int64_t score_row_offset(const AttnArgs &a, int q) {
 // en_attn_tile_table) the workgroups of the sequences' real query tiles come first, longest sequence first, and the
 // rest of the grid finds -1 and leaves; without one every (unit, tile) pair of the padded shape has a workgroup and
 // those past a sequence's end leave after reading its length.
-__device__ __forceinline__ bool map_block(const AttnArgs &a, int &unit, int &qi) {
-  const int bid = blockIdx.x;
+__device__ __forceinline__ bool map_block(const AttnArgs &a, int &unit, int &qi, int bid = blockIdx.x) {
   if (a.tile_table) {
     const int code = a.tile_table[bid];
     if (code < 0) return false;

@@ -238,6 +238,15 @@ int depad_and_transpose_pad(const void *hidden_padded, void *x_packed, const voi
                             const int32_t *cu_seqlens, int batch, int max_seq_len, int64_t hidden, int head_num,
                             int size_per_head, int elem_size, int left_padded, int zero_padding, hipStream_t stream);
 
+// fused.hip: en_attn_fused on packed projections and, in workgroups of the same launch, y = LayerNorm(in + residual rows) of
+// `total_tokens` rows of `hidden` channels, which does not read the context.  residual holds residual_rows rows.
+// EN_ERR_UNSUPPORTED, with nothing launched, where two launches have to do it.
+int attn_fused_beside_norm(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
+                           int max_seq_len, int size_per_head, int64_t total_tokens, float scale, int causal, int dtype,
+                           const int32_t *tile_table, const void *in, const void *residual, int64_t residual_rows,
+                           const int32_t *residual_row_offsets, const void *gamma, const void *beta, void *y, int64_t hidden,
+                           float eps, en_stream_t stream);
+
 // decode.hip: en_decode_attn (page_table null) / en_decode_attn_paged over caches of one set of strides whose position
 // kv_lens[b] already holds the newest token: every sequence is taken one longer than its length says.  Without `launch`
 // the arguments are looked at and nothing runs.

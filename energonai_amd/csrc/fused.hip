@@ -45,6 +45,7 @@
 // makes every instruction touch 32 rows, and the queue of the address unit then
 // stands full and holds back the tile loads of every wave on the CU.
 #include "fused_common.hip.h"
+#include "norm_rows.hip.h"
 
 #include <algorithm>
 
@@ -53,7 +54,7 @@ namespace en {
 // DP: channels of a row in LDS (the head size rounded up to 64, 96 or 128); NVS: MFMA steps of 16 channels that hold any.
 // NORM: the residual + LayerNorm of fused_common.hip.h follows (16-byte context rows, no separate query lengths).
 template <int DT, int DP, int NVS, bool NORM>
-__device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *norm) {
+__device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *norm, int bid = blockIdx.x) {
   static_assert(DT != EN_F32, "the fused kernel is built for 16-bit storage");
   typedef Elem<DT> E;
   typedef typename E::T T;
@@ -78,7 +79,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
   auto vswz = [](int row) { return DP == 128 ? 4 * (row & 3) : DP == 96 ? 0 : 4 * ((row >> 1) & 1); };
 
   int unit, qi;
-  if (!map_block(a, unit, qi)) return;
+  if (!map_block(a, unit, qi, bid)) return;
   const int b = unit / a.H, h = unit % a.H;
   int kl, ql;
   seq_extents(a, b, kl, ql);
@@ -407,20 +408,39 @@ __global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_norm_kern
   fused_tile<DT, DP, NVS, true>(fa, &norm);
 }
 
+// The attention and, in workgroups of their own, a residual + LayerNorm that does not read its output (a row-parallel
+// projection lies between them).  The attention is bound by instruction issue and by the chain of its longest workgroup, the
+// rows by memory: side by side they take less than one after the other, and a launch less.  us a layer, two launches / one:
+// 14213 tokens, 12 heads x 128, rows of 12288 252 / 240; 3485, 32 x 128, 8192 114 / 107; 3569, 16 x 64, 8192 49 / 43.5;
+// 3866, 10 x 80, 3200 42 / 32; 1033, 8 x 64, 2048 19.3 / 15.7; 300, 5 x 64, 640 18.3 / 15.3.  (Rows of 14336, which a
+// workgroup could hold with one load in flight less: 170 / 182, so 12288 is where it ends.)
+template <int DT, int DP, int NVS, bool STREAM>
+__global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_beside_norm_kernel(FusedArgs fa, NormRows rows) {
+  const int j = blockIdx.x / kXcds, x = blockIdx.x % kXcds;
+  const int before = min((int)(((uint64_t)j * rows.step) >> 16), rows.groups);
+  const int behind = min((int)(((uint64_t)(j + 1) * rows.step) >> 16), rows.groups);
+  if (behind > before) norm_rows<DT, STREAM>(rows, before * kXcds + x);
+  else fused_tile<DT, DP, NVS, false>(fa, nullptr, (j - before) * kXcds + x);
+}
+
 template <int DT, int DP, int NVS>
-static void launch_form(const FusedArgs &fa, const NormArgs *norm, unsigned grid, hipStream_t s) {
-  if (norm) attn_fused_norm_kernel<DT, DP, NVS><<<grid, kBlock, 0, s>>>(fa, *norm);
+static void launch_form(const FusedArgs &fa, const NormArgs *norm, const NormRows *rows, unsigned grid, hipStream_t s) {
+  if (rows) {
+    grid += (unsigned)rows->groups * kXcds;
+    if (rows->rows * rows->width * 2 >= kStreamStoreBytes) attn_fused_beside_norm_kernel<DT, DP, NVS, true><<<grid, kBlock, 0, s>>>(fa, *rows);
+    else attn_fused_beside_norm_kernel<DT, DP, NVS, false><<<grid, kBlock, 0, s>>>(fa, *rows);
+  } else if (norm) attn_fused_norm_kernel<DT, DP, NVS><<<grid, kBlock, 0, s>>>(fa, *norm);
   else attn_fused_kernel<DT, DP, NVS><<<grid, kBlock, 0, s>>>(fa);
 }
 
 template <int DT>
-static int launch_fused(FusedArgs &fa, const NormArgs *norm, hipStream_t s) {
+static int launch_fused(FusedArgs &fa, const NormArgs *norm, const NormRows *rows, hipStream_t s) {
   const AttnArgs &a = fa.base;
   const unsigned grid = (unsigned)(ceil_div(a.units, kXcds) * kXcds * a.ntq);
-  if (a.D <= 64) launch_form<DT, 64, 4>(fa, norm, grid, s);
-  else if (a.D <= 80) launch_form<DT, 96, 5>(fa, norm, grid, s);
-  else if (a.D <= 96) launch_form<DT, 96, 6>(fa, norm, grid, s);
-  else launch_form<DT, 128, 8>(fa, norm, grid, s);
+  if (a.D <= 64) launch_form<DT, 64, 4>(fa, norm, rows, grid, s);
+  else if (a.D <= 80) launch_form<DT, 96, 5>(fa, norm, rows, grid, s);
+  else if (a.D <= 96) launch_form<DT, 96, 6>(fa, norm, rows, grid, s);
+  else launch_form<DT, 128, 8>(fa, norm, rows, grid, s);
   EN_RETURN_IF_LAUNCH_FAILED();
   return EN_OK;
 }
@@ -442,7 +462,7 @@ static int attn_fused(const void *q, const void *k, const void *v, void *ctx, co
                       int32_t *q_lens, int batch, int head_num, int q_seq_len, int k_seq_len, int size_per_head, const int64_t
                       *q_strides, const int64_t *k_strides, const int64_t *v_strides, const int64_t *c_strides, const int32_t
                       *q_row_offsets, const int32_t *k_row_offsets, float scale, int causal, int dtype, const int32_t
-                      *tile_table, int query_tile, const NormArgs *norm, en_stream_t stream) {
+                      *tile_table, int query_tile, const NormArgs *norm, const NormRows *rows, en_stream_t stream) {
   if (!q || !k || !v || !ctx || !k_lens || !q_strides || !k_strides || !v_strides || !c_strides) return EN_ERR_NULL;
   if (batch < 1 || head_num < 1 || q_seq_len < 1 || k_seq_len < 1 || size_per_head < 1) return EN_ERR_SHAPE;
   if (dtype != EN_F16 && dtype != EN_BF16 && dtype != EN_F32) return EN_ERR_DTYPE;
@@ -484,12 +504,13 @@ static int attn_fused(const void *q, const void *k, const void *v, void *ctx, co
   fa.scale = scale;
   hipStream_t s = (hipStream_t)stream;
   if (norm && (!fa.c_vec16 || query_tile == kWideQTile)) return EN_ERR_UNSUPPORTED;
+  if (rows && (f32 || query_tile == kWideQTile)) return EN_ERR_UNSUPPORTED;
   if (f32) return launch_fused_f32(fa, norm, s);
   if (query_tile == kWideQTile) {
     a.ntq = (int)ceil_div(q_seq_len, kWideQTile);
     return launch_fused_wide(dtype, fa, s);
   }
-  return dtype == EN_F16 ? launch_fused<EN_F16>(fa, norm, s) : launch_fused<EN_BF16>(fa, norm, s);
+  return dtype == EN_F16 ? launch_fused<EN_F16>(fa, norm, rows, s) : launch_fused<EN_BF16>(fa, norm, rows, s);
 }
 
 // Workgroups that are resident at once: what LDS and registers leave room for on 256 CUs.
@@ -521,6 +542,40 @@ constexpr int kNormPolls = 64;      // looks at a meeting word before a workgrou
 static bool overlap(const void *a, int64_t a_bytes, const void *b, int64_t b_bytes) {
   const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
   return x < y + (uintptr_t)b_bytes && y < x + (uintptr_t)a_bytes;
+}
+
+int attn_fused_beside_norm(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
+                           int max_seq_len, int size_per_head, int64_t total_tokens, float scale, int causal, int dtype,
+                           const int32_t *tile_table, const void *in, const void *residual, int64_t residual_rows,
+                           const int32_t *residual_row_offsets, const void *gamma, const void *beta, void *y, int64_t hidden,
+                           float eps, en_stream_t stream) {
+  if (dtype != EN_F16 && dtype != EN_BF16) return EN_ERR_UNSUPPORTED;
+  if (batch < 1 || head_num < 1 || max_seq_len < 1 || size_per_head < 1 || total_tokens < 1) return EN_ERR_SHAPE;
+  const int64_t T = total_tokens, D = size_per_head, width = head_num * D, out_bytes = T * hidden * 2, ctx_bytes = T * width * 2;
+  if (hidden % 8 || hidden / 8 > kNormRowsMaxVectors || T > INT32_MAX) return EN_ERR_UNSUPPORTED;
+  for (const void *p : {in, residual, gamma, beta, (const void *)y})
+    if (!aligned_to(p, 16)) return EN_ERR_UNSUPPORTED;
+  // Each role reads while the other writes: buffers that a caller has laid over each other need two launches.
+  const int64_t meta = ((int64_t)batch + 1) * 4;
+  if (overlap(ctx, ctx_bytes, in, out_bytes) || overlap(ctx, ctx_bytes, residual, residual_rows * hidden * 2) ||
+      overlap(ctx, ctx_bytes, gamma, hidden * 2) || overlap(ctx, ctx_bytes, beta, hidden * 2) ||
+      (residual_row_offsets && overlap(ctx, ctx_bytes, residual_row_offsets, T * 4)) || overlap(y, out_bytes, ctx, ctx_bytes) ||
+      overlap(y, out_bytes, qkv, 3 * ctx_bytes) || overlap(y, out_bytes, seq_lens, meta - 4) || overlap(y, out_bytes, cu_seqlens, meta) ||
+      (tile_table && overlap(y, out_bytes, tile_table, en_attn_tile_table_elems(batch, head_num, max_seq_len, 0) * 4)))
+    return EN_ERR_UNSUPPORTED;
+  NormRows rows{in, residual, residual_row_offsets, gamma, beta, y, T, (int)hidden, eps, 0, 0};
+  rows.groups = (int)ceil_div(ceil_div(T, norm_rows_per_workgroup((int)hidden)), kXcds);
+  // Rows are dealt out between the attention's workgroups, as if those were twice their likely number: the long ones, which
+  // come first, start the earlier for it (10 heads x 80, 3866 tokens: 34 us by the likely number itself, 32 by twice that); but over no more groups than the launch has for the attention:
+  // all groups of rows then come before its last one, and no workgroup looks behind the end of the tile table.
+  const int64_t attention = std::min(2 * ceil_div(query_tiles(batch, max_seq_len, T, dtype) * head_num, kXcds),
+                                     ceil_div((int64_t)batch * head_num, kXcds) * ceil_div(max_seq_len, kQTile));
+  rows.step = (uint32_t)ceil_div((int64_t)rows.groups << 16, attention + rows.groups);
+  const char *pk = static_cast<const char *>(qkv);
+  const int64_t in_strides[3] = {0, 3 * D, 3 * width}, out_strides[3] = {0, D, width};
+  return attn_fused(pk, pk + D * 2, pk + 2 * D * 2, ctx, seq_lens, nullptr, batch, head_num, max_seq_len, max_seq_len, size_per_head,
+                    in_strides, in_strides, in_strides, out_strides, cu_seqlens, cu_seqlens, scale, causal, dtype, tile_table, 0,
+                    nullptr, &rows, stream);
 }
 
 }  // namespace en
@@ -578,7 +633,7 @@ int en_attn_fused_norm(const void *qkv, void *ctx, const int32_t *seq_lens, cons
   const int64_t D = size_per_head, in_strides[3] = {0, 3 * D, 3 * width}, out_strides[3] = {0, D, width};
   return attn_fused(pk, pk + D * es, pk + 2 * D * es, ctx, seq_lens, nullptr, batch, head_num, max_seq_len, max_seq_len, size_per_head,
                     in_strides, in_strides, in_strides, out_strides, cu_seqlens, cu_seqlens, scale, causal, dtype,
-                    dtype == EN_F32 ? nullptr : tile_table, 0, &norm, stream);
+                    dtype == EN_F32 ? nullptr : tile_table, 0, &norm, nullptr, stream);
 }
 
 int en_attn_fused(const void *q, const void *k, const void *v, void *ctx, const int32_t *k_lens,
@@ -589,7 +644,7 @@ int en_attn_fused(const void *q, const void *k, const void *v, void *ctx, const 
                              const int32_t *tile_table, int query_tile, en_stream_t stream) {
   return en::attn_fused(q, k, v, ctx, k_lens, q_lens, batch, head_num, q_seq_len, k_seq_len,
                         size_per_head, q_strides, k_strides, v_strides, c_strides, q_row_offsets, k_row_offsets, scale, causal,
-                        dtype, tile_table, query_tile, nullptr, stream);
+                        dtype, tile_table, query_tile, nullptr, nullptr, stream);
 }
 
 }  // extern "C"

@@ -100,6 +100,13 @@ extern "C" int en_padding_removal_layer(const void *hidden_padded, const void *q
   const unsigned char *qkv_bytes = static_cast<const unsigned char *>(qkv_padded);
   if (attention_form == 2) {
     // fused attention on the packed projections: no padded tensor at all
+    if (dense_out) {
+      // the LayerNorm does not wait for the context: both in one launch
+      rc = attn_fused_beside_norm(qkv_packed, ctx_packed, seq_lens, cu_seqlens, B, H, S, D, total_tokens, scale, causal, dtype, tile_table,
+                                  dense_out, fold_depad_offsets ? hidden_padded : x_packed,
+                                  fold_depad_offsets ? (int64_t)B * S : total_tokens, fold_depad_offsets, gamma, beta, y, hidden, eps, stream);
+      if (rc != EN_ERR_UNSUPPORTED) return rc;
+    }
     const unsigned char *pk = static_cast<const unsigned char *>(qkv_packed);
     const int64_t in_strides[3] = {0, 3 * D, (int64_t)3 * H * D};
     const int64_t out_strides[3] = {0, D, (int64_t)H * D};

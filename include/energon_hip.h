@@ -420,7 +420,7 @@ int en_block_decode(const en_block_decode_args *args, en_stream_t stream);
  * buffer: x_packed [T,hid] (residual stream), qkv_padded [B,H,S,3D], scores [B,H,S,S],
  * ctx [B,H,S,D], ctx_packed [T,H*D], y [T,hid].  dense_out [T,hid], if not NULL, is what
  * the LayerNorm adds to x_packed instead of ctx_packed (the output projection lies between
- * the two in a real layer).  attention_form: 0 = the three separate ops, 1 = en_attn_fused
+ * the two in a real layer); form 2 in 16-bit storage then runs the LayerNorm beside the attention, in its launch.  attention_form: 0 = the three separate ops, 1 = en_attn_fused
  * on the padded buffer (scores unused), 2 = en_attn_fused on the packed projections
  * (qkv_padded, scores and ctx unused), 3 = the three separate ops on the packed projections
  * (row offsets into qkv_packed and ctx_packed: transpose_pad and transpose_depad do not run;

@@ -549,6 +549,51 @@ def test_attention_and_layernorm_in_one_launch(dtype, lens, S, H, D, causal, lef
     assert torch.equal(again.float(), want)
 
 
+@pytest.mark.parametrize("dtype,lens,S,H,D,hid", [
+    (torch.float16, [256, 256, 256], 256, 3, 64, 8),               # every tile of the launch a real one; a vector a row
+    (torch.bfloat16, [1], 17, 1, 64, 512),                         # fewer rows than a workgroup has waves
+    (torch.float16, [130, 0, 7], 130, 5, 64, 520),                 # a wave per row, more than one vector a lane
+    (torch.bfloat16, [127, 128, 129], 140, 4, 80, 1536),
+    (torch.float16, [33, 65], 70, 9, 96, 1544),                    # a workgroup per row
+    (torch.bfloat16, [512], 512, 2, 128, 4104),
+    (torch.float16, [40, 3], 64, 8, 128, 8200),
+    (torch.bfloat16, [21], 32, 2, 128, 12288),
+    (torch.float16, [21], 32, 2, 128, 12296),                      # wider than a workgroup holds: two launches
+    (torch.float16, [100] * 60, 1000, 4, 64, 768),                 # a bucket that is mostly empty
+])
+def test_layernorm_of_a_projection_beside_the_attention(dtype, lens, S, H, D, hid):
+    """With ``dense_out`` the LayerNorm shares the attention's launch: the context is that of the attention alone bit for bit,
+    y differs from the LayerNorm's own call by at most one rounding of the stored value (the order of a row's sums).  A context
+    written over the projection is read by the LayerNorm as two launches do."""
+    from energonai_amd import layer
+    from energonai_amd.kernel import attn_fused_packed, depad, layer_norm_forward
+    from energonai_amd.seqinfo import build_seq_info
+    announce("beside", dtype, lens[:5], S, H, D, hid)
+    g = torch.Generator().manual_seed(S + hid)
+    B, T = len(lens), sum(lens)
+    hidden, qkv = torch.randn(B, S, hid, generator=g).to(dtype).cuda(), torch.randn(1, T, H, 3 * D, generator=g).to(dtype).cuda()
+    dense = torch.randn(1, T, hid, generator=g).to(dtype).cuda()
+    gamma, beta = (1 + 0.1 * torch.randn(hid, generator=g)).to(dtype).cuda(), torch.randn(hid, generator=g).to(dtype).cuda()
+    info = build_seq_info(torch.tensor(lens, dtype=torch.int32).cuda(), B, total=T)
+    want_ctx = attn_fused_packed(qkv, B, S, info, H, D, scale=D ** -0.5)
+    ulp = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+    for left in (False, True):
+        x = depad(hidden, B, info, left_padded=left, sum_seq=T)
+        want = layer_norm_forward(dense, gamma, beta, (hid,), 1e-5, residual=x).float()
+        for fold in (True, False):
+            ctx = torch.full_like(want_ctx, 7.0)
+            y = layer.padding_removal_layer(hidden, qkv, info, H, D, gamma, beta, 1e-5, left_padded=left, dense_out=dense, ctx_out=ctx,
+                                            fold_depad=fold)
+            assert torch.equal(ctx, want_ctx)
+            assert bool(((y.float() - want).abs() <= ulp * want.abs().clamp_min(2.0 ** -6)).all())
+    if hid <= H * D:
+        both = torch.zeros_like(want_ctx)
+        y = layer.padding_removal_layer(hidden, qkv, info, H, D, gamma, beta, 1e-5, left_padded=True, ctx_out=both,
+                                        dense_out=both.view(-1)[:T * hid].view(1, T, hid))
+        want = layer_norm_forward(want_ctx.view(-1)[:T * hid].view(1, T, hid), gamma, beta, (hid,), 1e-5, residual=x)
+        assert torch.equal(y, want)
+
+
 def test_decode_layer_operands_outside_the_native_call():
     """A projection's output in fp32 behind fp16 caches, with more rows than new tokens, or no residual: the step takes them
     as the separate calls do."""
