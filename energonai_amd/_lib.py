@@ -29,8 +29,10 @@ SIGNATURES = {
     "en_prefix_sum": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "en_depad": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int, c_int, c_void_p]),
     "en_repad": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int, c_int, c_void_p]),
+    "en_repad_rows": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int64, c_int, c_int, c_void_p]),
     "en_transpose_pad": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "en_transpose_pad_heads": (c_int, [c_void_p, c_void_p, c_void_p] + [c_int] * 8 + [c_void_p]),
+    "en_kv_fill_pair": (c_int, [c_void_p] * 4 + [c_int] * 8 + [c_void_p]),
     "en_kv_append": (c_int, [c_void_p] * 5 + [c_int] * 4 + [c_int64] * 5 + [c_int, c_void_p, c_void_p]),
     "en_transpose_depad": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "en_ft_build_offsets": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p]),

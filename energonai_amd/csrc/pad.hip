@@ -79,17 +79,18 @@ struct DepadRowsMap {
   }
 };
 
-// repad: inverse of depad; every row of the padded output is written (copy or zeros).
+// repad: inverse of depad; the S rows of every sequence are written (copy or zeros), sequences `pitch` rows apart.
 struct RepadRowsMap {
   const int32_t *cu;
   int S, R, left;
+  int64_t pitch;
   __device__ bool active(int, int) const { return true; }
   __device__ void operator()(int tx, int b, int r, int64_t &src, int64_t &dst) const {
     const int s = tx * R + r;
     const int start = cu[b];
     const int len = cu[b + 1] - start;
     const int i = s - (left ? S - len : 0);     // position inside the sequence
-    dst = (s < S) ? (int64_t)b * S + s : kSkipRow;
+    dst = (s < S) ? (int64_t)b * pitch + s : kSkipRow;
     src = (i >= 0 && i < len) ? (int64_t)start + i : kZeroRow;
   }
 };
@@ -416,15 +417,20 @@ int en_depad(const void *src, void *dst, const int32_t *cu_seqlens, int batch, i
 
 int en_repad(const void *src, void *dst, const int32_t *cu_seqlens, int batch, int max_seq_len, int64_t hidden,
              int elem_size, int left_padded, en_stream_t stream) {
+  return en_repad_rows(src, dst, cu_seqlens, batch, max_seq_len, max_seq_len, hidden, elem_size, left_padded, stream);
+}
+
+int en_repad_rows(const void *src, void *dst, const int32_t *cu_seqlens, int batch, int max_seq_len, int64_t dst_rows,
+                  int64_t hidden, int elem_size, int left_padded, en_stream_t stream) {
   if (!src || !dst || !cu_seqlens) return EN_ERR_NULL;
   if (check_elem(elem_size)) return EN_ERR_DTYPE;
-  if (batch < 1 || max_seq_len < 1 || hidden < 1) return EN_ERR_SHAPE;
+  if (batch < 1 || max_seq_len < 1 || hidden < 1 || dst_rows < max_seq_len) return EN_ERR_SHAPE;
   if (!aligned_to(src, elem_size) || !aligned_to(dst, elem_size)) return EN_ERR_ALIGN;
   Ptrs3 p = {{src, nullptr, nullptr}, {dst, nullptr, nullptr}};
   return launch_row_gather<RepadRowsMap, 1>(hidden * elem_size, max_seq_len,
                                             (int64_t)batch * max_seq_len * hidden * elem_size, p, [&](int R, dim3 &grid) {
     grid = dim3((unsigned)ceil_div(max_seq_len, R), (unsigned)batch, 1);
-    return RepadRowsMap{cu_seqlens, max_seq_len, R, left_padded ? 1 : 0};
+    return RepadRowsMap{cu_seqlens, max_seq_len, R, left_padded ? 1 : 0, dst_rows};
   }, (hipStream_t)stream);
 }
 
@@ -442,6 +448,35 @@ int en_transpose_pad_heads(const void *src, void *dst, const int32_t *cu_seqlens
     grid = dim3((unsigned)(ceil_div(max_seq_len, R) * head_num), (unsigned)batch, 1);
     return PadMap{cu_seqlens, head_num, max_seq_len, R, src_head_rows, src_head_first, zero_padding ? 1 : 0};
   }, (hipStream_t)stream);
+}
+
+int en_kv_fill_pair(const void *src, void *k_cache, void *v_cache, const int32_t *cu_seqlens, int batch, int cache_len, int head_num,
+                    int size_per_head, int src_head_rows, int k_head_first, int v_head_first, int elem_size, en_stream_t stream) {
+  if (!src || !k_cache || !v_cache || !cu_seqlens) return EN_ERR_NULL;
+  if (check_elem(elem_size)) return EN_ERR_DTYPE;
+  if (batch < 1 || cache_len < 1 || head_num < 1 || size_per_head < 1) return EN_ERR_SHAPE;
+  for (int first : {k_head_first, v_head_first})
+    if (first < 0 || src_head_rows < first + head_num) return EN_ERR_SHAPE;
+  for (const void *p : {src, (const void *)k_cache, (const void *)v_cache})
+    if (!aligned_to(p, elem_size)) return EN_ERR_ALIGN;
+  const Ptrs3 pk = {{src, nullptr, nullptr}, {k_cache, nullptr, nullptr}}, pv = {{src, nullptr, nullptr}, {v_cache, nullptr, nullptr}};
+  const int64_t row = (int64_t)size_per_head * elem_size, vpr = row / 16;
+  const int R = vpr > 0 && vpr <= INT32_MAX / kMaxTileRows ? tile_rows(vpr, cache_len) : 1;
+  const int64_t grid_x = ceil_div(cache_len, R) * head_num, blocks = grid_x * batch;
+  // caches so large that they are written past the memory-side cache gain nothing from a shared launch
+  if (pick_vec_bytes(row, pk, 1) != 16 || pick_vec_bytes(row, pv, 1) != 16 || vpr > INT32_MAX / kMaxTileRows || 2 * blocks > INT32_MAX ||
+      (int64_t)batch * cache_len * head_num * row >= kStreamStoreBytes) {
+    const int rc = en_transpose_pad_heads(src, k_cache, cu_seqlens, batch, cache_len, head_num, size_per_head, src_head_rows, k_head_first, 1,
+                                          elem_size, stream);
+    if (rc) return rc;
+    return en_transpose_pad_heads(src, v_cache, cu_seqlens, batch, cache_len, head_num, size_per_head, src_head_rows, v_head_first, 1, elem_size,
+                                  stream);
+  }
+  const GatherPart gk{pk, (int)vpr, R, (unsigned)grid_x}, gv{pv, (int)vpr, R, (unsigned)grid_x};
+  const PadMap mk{cu_seqlens, head_num, cache_len, R, src_head_rows, k_head_first, 1}, mv{cu_seqlens, head_num, cache_len, R, src_head_rows, v_head_first, 1};
+  row_gather_pair_kernel<PadMap, PadMap><<<(unsigned)(2 * blocks), kBlock, 0, (hipStream_t)stream>>>(mk, gk, mv, gv, (unsigned)blocks);
+  EN_RETURN_IF_LAUNCH_FAILED();
+  return EN_OK;
 }
 
 int en_transpose_pad(const void *src, void *dst, const int32_t *cu_seqlens, int batch, int max_seq_len, int head_num,

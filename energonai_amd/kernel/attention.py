@@ -317,6 +317,22 @@ def kv_cache_fill(src, cache, batch_size: int, seq_len_list, head_first: int = 0
     return cache
 
 
+def kv_cache_start(src, k_cache, v_cache, batch_size: int, seq_len_list, k_head_first: int, v_head_first: int) -> None:
+    """``kv_cache_fill`` of both caches from heads ``k_head_first`` .. and ``v_head_first`` .. of one packed projection, zeros
+    behind each sequence, in one launch."""
+    for t, n in ((src, "src"), (k_cache, "k_cache"), (v_cache, "v_cache")):
+        _lib.require_gpu(t, n)
+    if src.dim() != 3 or k_cache.dim() != 4 or v_cache.shape != k_cache.shape or k_cache.shape[0] != batch_size \
+            or k_cache.shape[3] != src.shape[2] or k_cache.dtype != src.dtype or v_cache.dtype != src.dtype:
+        raise RuntimeError("kv_cache_start: src must be [T,Hs,D] and the caches [B,H,Smax,D] of one dtype")
+    B, H, Smax, D = k_cache.shape
+    info = seq_info(seq_len_list, batch_size, src.device)
+    with _lib.device_guard(src):
+        _lib.check(_lib.fn.en_kv_fill_pair(src.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), info.cu_seqlens.data_ptr(), B, Smax, H, D,
+                                           src.shape[1], int(k_head_first), int(v_head_first), src.element_size(),
+                                           _lib.stream_of(src)), "kv_cache_start")
+
+
 def kv_cache_append(k_new, v_new, k_cache, v_cache, kv_len_list, overflow: Optional[torch.Tensor] = None):
     """Writes the new token's rows ``k_new`` / ``v_new`` (``[B,H,D]`` views) into the ``[B,H,Smax,D]`` caches at
     position ``kv_len[b]``.  The caller advances the lengths afterwards.  A sequence whose cache is full keeps

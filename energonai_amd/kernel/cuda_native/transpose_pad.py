@@ -112,8 +112,9 @@ def depad(src, batch_size, seq_lens, left_padded=False, sum_seq=None):
     return dst
 
 
-def repad(src, batch_size, max_seq_len, seq_lens, left_padded=False):
-    """[1,T,hid] -> [B,S,hid] with zero padding rows: the inverse of :func:`depad`.
+def repad(src, batch_size, max_seq_len, seq_lens, left_padded=False, out=None):
+    """[1,T,hid] -> [B,S,hid] with zero padding rows: the inverse of :func:`depad`.  ``out``: a contiguous ``[B,rows,hid]``
+    tensor of at least S rows a sequence, whose first S rows are written.
 
     An addition for the exit of the packed path; the reference callers rebuild
     right-padded batches with ``ft_rebuild_padding`` (examples/gpt/gpt.py:321-323)
@@ -126,11 +127,17 @@ def repad(src, batch_size, max_seq_len, seq_lens, left_padded=False):
     if src.numel() % hid != 0 or src.dim() < 2:
         raise RuntimeError("repad: src must be [1, total, hidden]")
     S = _as_int(max_seq_len)
-    dst = torch.empty((batch_size, S, hid), dtype=src.dtype, device=src.device)
+    if out is None:
+        out = torch.empty((batch_size, S, hid), dtype=src.dtype, device=src.device)
+    else:
+        _lib.require_gpu(out, "out")
+        if out.dim() != 3 or out.shape[0] != batch_size or out.shape[1] < S or out.shape[2] != hid or out.dtype != src.dtype \
+                or out.device != src.device:
+            raise RuntimeError("repad: out must be [batch, rows, hidden] of src's dtype with room for max_seq_len rows")
     with _lib.device_guard(src):
-        _lib.check(_lib.fn.en_repad(src.data_ptr(), dst.data_ptr(), info.cu_seqlens.data_ptr(), batch_size, S, hid,
-                                    _elem_size(src, "repad"), int(bool(left_padded)), _lib.stream_of(src)), "repad")
-    return dst
+        _lib.check(_lib.fn.en_repad_rows(src.data_ptr(), out.data_ptr(), info.cu_seqlens.data_ptr(), batch_size, S, out.shape[1], hid,
+                                         _elem_size(src, "repad"), int(bool(left_padded)), _lib.stream_of(src)), "repad")
+    return out
 
 
 # From FasterTransformer

@@ -102,7 +102,7 @@ class MultiHeadAttention1D(nn.Module):
                 self.kv_cache = PagedKVCache(batch_size, H, self.max_seq_len, D, x.dtype, x.device,
                                              page_size=self.kv_page_size, pool_pages=self.kv_pool_pages)
             else:
-                self.kv_cache = KVCache(batch_size, H, self.max_seq_len, D, x.dtype, x.device)
+                self.kv_cache = KVCache(batch_size, H, self.max_seq_len, D, x.dtype, x.device, zeroed=False)
             if kvq is not None:
                 self.kv_cache.fill(kvq, kvq, info, 0, H, longest=max_seq_len)
             else:
@@ -132,10 +132,9 @@ class MultiHeadAttention1D(nn.Module):
         info = seq_info(seq_lens, B, hidden_states.device)
         x = depad(hidden_states, B, info, left_padded=self.left_padded)
         y = self.forward_packed(x, info, B, S, fill_cache=not self.disable_past_cache)
-        out = repad(y, B, S, info, left_padded=self.left_padded)
         if not self.disable_past_cache:
-            return self._history.start(out, self.max_seq_len)
-        return out
+            return self._history.start_packed(y, B, S, info, self.left_padded, self.max_seq_len)
+        return repad(y, B, S, info, left_padded=self.left_padded)
 
 
 _ONES = {}

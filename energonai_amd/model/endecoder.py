@@ -128,10 +128,9 @@ class Block1D(nn.Module):
         left = self.attn.left_padded
         x = depad(hidden_states, B, info, left_padded=left)
         y = self.forward_packed(x, info, B, S, fill_cache=not self.disable_past_cache)
-        out = repad(y, B, S, info, left_padded=left)
         if not self.disable_past_cache:
-            return self._history.start(out, self.max_seq_len)
-        return out
+            return self._history.start_packed(y, B, S, info, left, self.max_seq_len)
+        return repad(y, B, S, info, left_padded=left)
 
 
 def _step_methods():

@@ -14,15 +14,19 @@ from typing import Optional
 
 import torch
 
-from ..kernel import decode_attn, decode_attn_paged, kv_cache_append, kv_cache_fill, kv_pages_append, kv_pages_fill
+from ..kernel import decode_attn, decode_attn_paged, kv_cache_append, kv_cache_fill, kv_pages_append, kv_pages_fill, repad
+from ..kernel.attention import kv_cache_start
 from ..seqinfo import SeqInfo
 
 
 class KVCache:
-    def __init__(self, batch_size: int, head_num: int, max_seq_len: int, size_per_head: int, dtype, device):
-        self.k = torch.zeros((batch_size, head_num, max_seq_len, size_per_head), dtype=dtype, device=device)
-        self.v = torch.zeros_like(self.k)
-        self.lens = torch.zeros(batch_size, dtype=torch.int32, device=device)
+    def __init__(self, batch_size: int, head_num: int, max_seq_len: int, size_per_head: int, dtype, device, zeroed: bool = True):
+        """``zeroed=False``: for a caller that fills the cache next; ``fill`` writes the zeros with the rows."""
+        new = torch.zeros if zeroed else torch.empty
+        self.k = new((batch_size, head_num, max_seq_len, size_per_head), dtype=dtype, device=device)
+        self.v = new(self.k.shape, dtype=dtype, device=device)
+        self.lens = new(batch_size, dtype=torch.int32, device=device)
+        self._zeroed = zeroed
         self.batch_size = batch_size
         self.max_seq_len = max_seq_len
         self._longest = 0       # host-side bound of the longest cached sequence (no device read per step)
@@ -34,9 +38,14 @@ class KVCache:
              v_head_first: int = 0, longest: Optional[int] = None) -> None:
         """Prefill from packed projections seen as ``[T,Hs,D]`` (see ``kv_cache_fill``).  ``longest`` is the
         longest sequence length if the caller knows it on the host (the bucket length is an upper bound)."""
-        # the buffers were zeroed when they were allocated and no reader goes past the lengths
-        kv_cache_fill(k_src, self.k, self.batch_size, info, k_head_first, zero_padding=False)
-        kv_cache_fill(v_src, self.v, self.batch_size, info, v_head_first, zero_padding=False)
+        if not self._zeroed and k_src is v_src:
+            # both caches and the zeros behind each sequence in one launch: two fills and two movers were four
+            kv_cache_start(k_src, self.k, self.v, self.batch_size, info, k_head_first, v_head_first)
+        else:
+            # buffers that were zeroed when they were allocated keep their zeros: no reader goes past the lengths
+            kv_cache_fill(k_src, self.k, self.batch_size, info, k_head_first, zero_padding=not self._zeroed)
+            kv_cache_fill(v_src, self.v, self.batch_size, info, v_head_first, zero_padding=not self._zeroed)
+        self._zeroed = True
         self.lens.copy_(info.lens)
         # the fill kernel is given at most max_seq_len rows per sequence; the bound is tightened when the
         # caller has the true maximum on the host
@@ -192,6 +201,15 @@ class OutputHistory:
         self.buf[:, :S].copy_(out)
         self.cur = S
         return self.buf[:, :S]
+
+    def start_packed(self, y: torch.Tensor, batch_size: int, max_seq_len: int, info: SeqInfo, left_padded: bool, planned: int) -> torch.Tensor:
+        """``start(repad(y))`` without the copy: the padding is restored in the buffer itself."""
+        if type(self).start is not OutputHistory.start or "start" in self.__dict__:
+            return self.start(repad(y, batch_size, max_seq_len, info, left_padded=left_padded), planned)
+        self.buf = repad(y, batch_size, max_seq_len, info, left_padded=left_padded,
+                         out=torch.empty((batch_size, max(int(planned), max_seq_len), y.shape[-1]), dtype=y.dtype, device=y.device))
+        self.cur = max_seq_len
+        return self.buf[:, :max_seq_len]
 
     def reserve(self) -> torch.Tensor:
         """The buffer, with room at position ``cur``."""

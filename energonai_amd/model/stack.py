@@ -42,7 +42,7 @@ class PackedStack(nn.Module):
         for blk in self.blocks:
             x = blk.forward_packed(x, info, B, S, fill_cache=caching)
             if caching:   # each block keeps its own padded output for the later steps, as the reference blocks do
-                blk._history.start(repad(x, B, S, info, left_padded=left), blk.max_seq_len)
+                blk._history.start_packed(x, B, S, info, left, blk.max_seq_len)
         if self.norm is not None:
             x = self.norm(x)
         return repad(x, B, S, info, left_padded=left)

@@ -71,6 +71,9 @@ int en_depad(const void *src, void *dst, const int32_t *cu_seqlens, int batch, i
  * of dst is written. */
 int en_repad(const void *src, void *dst, const int32_t *cu_seqlens, int batch, int max_seq_len, int64_t hidden,
              int elem_size, int left_padded, en_stream_t stream);
+/* The same into sequences that lie dst_rows >= max_seq_len rows apart (a history that later positions are written into). */
+int en_repad_rows(const void *src, void *dst, const int32_t *cu_seqlens, int batch, int max_seq_len, int64_t dst_rows,
+                  int64_t hidden, int elem_size, int left_padded, en_stream_t stream);
 
 /* transpose_pad_wrapper (csrc/transpose_pad_fusion_wrapper.cpp:33-57, kernel
  * csrc/transpose_pad_fusion_kernel.cu:58-96): [T,H,Dk] -> [B,H,S,Dk]; every
@@ -273,6 +276,12 @@ int en_decode_layer(const void *q, const void *k_cache, const void *v_cache, voi
                     float scale, const void *dense_out, const void *residual, const void *gamma, const void *beta, void *y,
                     int64_t hidden, float eps, int dtype, int out_dtype, void *workspace, int64_t workspace_bytes,
                     en_stream_t stream);
+
+/* New K/V caches [batch, head_num, cache_len, size_per_head] from a projection's packed rows [T, src_head_rows, size_per_head],
+ * K from its heads k_head_first .., V from v_head_first .., zeros behind each sequence: en_transpose_pad_heads for both in one
+ * launch (8 sequences, 12 heads x 64, 512 positions: 4 launches of 3.9 us, two fills and two movers, become one of 6.3). */
+int en_kv_fill_pair(const void *src, void *k_cache, void *v_cache, const int32_t *cu_seqlens, int batch, int cache_len, int head_num,
+                    int size_per_head, int src_head_rows, int k_head_first, int v_head_first, int elem_size, en_stream_t stream);
 
 /* Appends the new token's K and V rows to [B,H,Smax,D] caches at position
  * kv_lens[b] (the caller then adds one to kv_lens); replaces the reference's

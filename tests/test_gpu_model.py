@@ -117,6 +117,45 @@ def test_kv_cache_fill_and_append_bit_exact(dtype):
     assert overflow.item() == 2
 
 
+@pytest.mark.parametrize("dtype,H,D,Smax,lens", [
+    (torch.float16, 4, 64, 50, [7, 30, 1]), (torch.bfloat16, 3, 80, 129, [129, 0, 64, 65]), (torch.float32, 2, 64, 700, [700, 3]),
+    (torch.float16, 3, 10, 20, [20, 5]),                 # rows of 20 bytes: no 16-byte pieces, two launches
+    (torch.float16, 24, 128, 4096, [4096, 17, 0, 1]),    # 96 MB a cache: two launches
+])
+def test_kv_caches_filled_from_scratch_in_one_launch(dtype, H, D, Smax, lens):
+    """A cache allocated without zeros is filled with the rows and the zeros behind them: the same buffers as zeros and two movers."""
+    K, M = _mods()
+    from energonai_amd.seqinfo import seq_info
+    announce("kv start", dtype, H, D, Smax, lens)
+    B, T = len(lens), sum(lens)
+    g = torch.Generator().manual_seed(33)
+    kvq = torch.randn(T, 3 * H, D, generator=g).to(dtype).cuda()
+    info = seq_info(torch.tensor(lens, dtype=torch.int32).cuda(), B, torch.device("cuda"))
+    want = M.KVCache(B, H, Smax, D, dtype, "cuda")
+    want.fill(kvq, kvq, info, 0, H, longest=max(lens))
+    for k_src, v_src, v_first in ((kvq, kvq, H), (kvq, kvq[:, H:2 * H].contiguous(), 0)):
+        got = M.KVCache(B, H, Smax, D, dtype, "cuda", zeroed=False)
+        got.k.fill_(7.0), got.v.fill_(7.0), got.lens.fill_(7)
+        got.fill(k_src, v_src, info, 0, v_first, longest=max(lens))
+        assert torch.equal(got.k, want.k) and torch.equal(got.v, want.v) and torch.equal(got.lens, want.lens)
+        assert got._longest == want._longest
+
+
+@pytest.mark.parametrize("left", [False, True])
+def test_repad_into_a_longer_buffer(left):
+    K, _ = _mods()
+    lens, S, hid = [5, 0, 9], 9, 40
+    g = torch.Generator().manual_seed(34)
+    x = torch.randn(1, sum(lens), hid, generator=g).half().cuda()
+    lens_t = torch.tensor(lens, dtype=torch.int32).cuda()
+    buf = torch.full((3, 13, hid), 7.0, dtype=torch.float16, device="cuda")
+    assert K.repad(x, 3, S, lens_t, left_padded=left, out=buf) is buf
+    assert torch.equal(buf[:, :S], K.repad(x, 3, S, lens_t, left_padded=left)) and bool((buf[:, S:] == 7.0).all())
+    for bad in (buf[:, :8].contiguous(), buf[:2], buf.float(), buf[:, :, :32].contiguous()):
+        with pytest.raises(RuntimeError, match="out must be"):
+            K.repad(x, 3, S, lens_t, left_padded=left, out=bad)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_kv_cache_fill_without_zero_fill_leaves_padding_untouched(dtype):
     """zero_padding=False: rows below each length are written, every other row keeps the bits it had
