@@ -462,6 +462,88 @@ PyObject *block_decode(PyObject *const *a) {
   return THPVariable_Wrap(out.narrow(1, 0, position + 1));
 }
 
+// block_prefill(x [1,T,hidden], norm1 w, b, eps, qkv w, b, dense w, b, norm2 w, b, eps, mlp1 w, b, mlp2 w, b, activation, heads, scale,
+//               causal, lens, cu_seqlens, tile table or None, batch, max_seq_len, address of en_linear or 0, its workspace or None)
+// -> (block's output [1,T,hidden], packed projections [1,T,3 hidden]), or None, with nothing done, where a tensor is not what the
+// kernels take.  The ops are those of the general step one by one: LayerNorm, projection, fused attention on packed rows,
+// projection, residual + LayerNorm that keeps the sum, MLP (both GEMMs by en_linear with the activation in its epilogue, or by
+// torch around exact GELU), sum.
+typedef int (*en_linear_fn)(const void *, const void *, const void *, void *, int64_t, int64_t, int64_t, int, int, int, void *, int64_t,
+                            hipStream_t);
+PyObject *block_prefill(PyObject *const *a) {
+  for (int i : {0, 1, 2, 4, 5, 6, 7, 8, 9, 11, 12, 13, 14})
+    if (a[i] != Py_None && !THPVariable_CheckExact(a[i])) Py_RETURN_NONE;
+  const Tensor &x = gpu(a[0], "x", false);
+  const auto dt = x.scalar_type();
+  const int64_t heads = integer(a[16]), batch = integer(a[22]), S = integer(a[23]);
+  if ((dt != at::kHalf && dt != at::kBFloat16) || x.dim() != 3 || x.size(0) != 1 || x.numel() == 0 || !x.is_contiguous()) Py_RETURN_NONE;
+  const int64_t T = x.size(1), hid = x.size(2), D = heads > 0 ? hid / heads : 0;
+  if (D * heads != hid || D % 8 || D > 128) Py_RETURN_NONE;
+  bool usable = true;
+  auto weight = [&](int i, int64_t rows, int64_t cols) -> Tensor {
+    if (a[i] == Py_None) return Tensor();
+    const Tensor &t = tensor(a[i], "weight");
+    const int64_t shape[2] = {rows, cols};
+    if (!t.is_cuda() || t.device() != x.device() || t.scalar_type() != dt || !t.is_contiguous() ||
+        t.sizes() != (rows == 1 ? c10::IntArrayRef(&cols, 1) : c10::IntArrayRef(shape, 2)))
+      usable = false;
+    return t;
+  };
+  const Tensor &w1 = tensor(a[11], "weight");
+  if (w1.dim() != 2) Py_RETURN_NONE;
+  const int64_t mlp = w1.size(0);
+  const Tensor n1w = weight(1, 1, hid), n1b = weight(2, 1, hid), qkv_w = weight(4, 3 * hid, hid), qkv_b = weight(5, 1, 3 * hid),
+               dense_w = weight(6, hid, hid), dense_b = weight(7, 1, hid), n2w = weight(8, 1, hid), n2b = weight(9, 1, hid),
+               m1w = weight(11, mlp, hid), m1b = weight(12, 1, mlp), m2w = weight(13, hid, mlp), m2b = weight(14, 1, hid);
+  const float eps1 = real(a[3]), eps2 = real(a[10]), scale = real(a[17]);
+  const int act = (int)integer(a[15]), causal = (int)integer(a[18]);
+  const Tensor &lens = gpu(a[19], "lens"), &cu = gpu(a[20], "cu_seqlens");
+  const int32_t *table = a[21] == Py_None ? nullptr : i32(gpu(a[21], "tile_table"));
+  const auto linear = reinterpret_cast<en_linear_fn>((uintptr_t)PyLong_AsUnsignedLongLong(a[24]));
+  Tensor ws;
+  if (a[25] != Py_None) ws = gpu(a[25], "workspace");
+  if (!usable || !n1w.defined() || !n1b.defined() || !n2w.defined() || !n2b.defined() || !qkv_w.defined() || !dense_w.defined() ||
+      !m1w.defined() || !m2w.defined() || lens.device() != x.device() || cu.device() != x.device() || lens.numel() < batch ||
+      cu.numel() < batch + 1 || !(scale > 0.f) || (linear && !ws.defined()) || (!linear && act != EN_ACT_GELU))
+    Py_RETURN_NONE;
+  const c10::DeviceGuard guard(x.device());
+  const int tag = dtype_tag(x, "block_prefill");
+  const hipStream_t stream = stream_of(x);
+  const int32_t *lens_p = i32(lens), *cu_p = i32(cu);
+  Tensor y, kvq;
+  auto run = [&]() -> int {
+    const Tensor h = at::empty_like(x);
+    check(en_layernorm_fwd(h.data_ptr(), nullptr, nullptr, nullptr, x.data_ptr(), nullptr, nullptr, n1w.data_ptr(), n1b.data_ptr(), T, hid,
+                           eps1, tag, tag, stream), "layer_norm");
+    kvq = at::linear(h, qkv_w, qkv_b);
+    // packed rows of 3 heads x D, ordered k, v, q (attention.py:74)
+    const Tensor ctx = at::empty({1, T, hid}, x.options());
+    const int64_t in[3] = {0, D, 3 * hid}, out[3] = {0, D, hid};
+    const char *rows = static_cast<const char *>(kvq.data_ptr());
+    check(en_attn_fused(rows + 2 * hid * 2, rows, rows + hid * 2, ctx.data_ptr(), lens_p, nullptr, (int)batch, (int)heads, (int)S, (int)S, (int)D,
+                        in, in, in, out, cu_p, cu_p, scale, causal, tag, table, 0, stream), "attn_fused_varlen");
+    const Tensor att = at::linear(ctx, dense_w, dense_b);
+    const Tensor h2 = at::empty_like(x), sum = at::empty_like(x);
+    check(en_layernorm_fwd(h2.data_ptr(), nullptr, nullptr, sum.data_ptr(), att.data_ptr(), x.data_ptr(), nullptr, n2w.data_ptr(), n2b.data_ptr(),
+                           T, hid, eps2, tag, tag, stream), "layer_norm");
+    Tensor m;
+    if (linear) {
+      const Tensor f = at::empty({1, T, mlp}, x.options());
+      m = at::empty_like(x);
+      auto ptr = [](const Tensor &t) -> const void * { return t.defined() ? t.data_ptr() : nullptr; };
+      if (linear(h2.data_ptr(), m1w.data_ptr(), ptr(m1b), f.data_ptr(), T, hid, mlp, act, tag, -1, ws.data_ptr(), ws.numel(), stream) < 0 ||
+          linear(f.data_ptr(), m2w.data_ptr(), ptr(m2b), m.data_ptr(), T, mlp, hid, 0, tag, -1, ws.data_ptr(), ws.numel(), stream) < 0)
+        fail("linear: the GEMM could not be launched");
+    } else {
+      m = at::linear(at::gelu(at::linear(h2, m1w, m1b)), m2w, m2b);
+    }
+    y = at::add(sum, m);
+    return EN_OK;
+  };
+  (void)without_gil(run);
+  return tuple({y, kvq});
+}
+
 // ---- module --------------------------------------------------------------------------------------------------------
 
 template <PyObject *(*F)(PyObject *const *), int N>
@@ -492,6 +574,7 @@ PyMethodDef kMethods[] = {
     EN_FAST(layer, 19, "en_padding_removal_layer on new outputs"),
     EN_FAST(decode_layer, 10, "en_decode_layer on new outputs"),
     EN_FAST(plain_step, 9, "what block_decode takes of a block's modules, or None where the general step has to see them"),
+    EN_FAST(block_prefill, 26, "a pre-LN block over packed rows, its attention on the packed projections"),
     EN_FAST(block_decode, 25, "en_block_decode into a position of an output history"),
     {nullptr, nullptr, 0, nullptr}};
 

@@ -10,6 +10,7 @@ additions: hipBLASLt applies them in the GEMM epilogue, where the reference's ca
 """
 from __future__ import annotations
 
+import ctypes
 import time
 from typing import Dict, Optional
 
@@ -30,6 +31,17 @@ def _workspace(device: torch.device) -> torch.Tensor:
         ws = torch.empty(_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
         _workspaces[device.index] = ws
     return ws
+
+
+def linear_entry(device: torch.device):
+    """Address of ``en_linear`` and the workspace it is handed, for native callers."""
+    global _entry
+    if _entry is None:
+        _entry = ctypes.cast(_lib.load_linear().en_linear, ctypes.c_void_p).value
+    return _entry, _workspace(device)
+
+
+_entry = None
 
 
 def _check(status: int, op: str) -> None:

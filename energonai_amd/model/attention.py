@@ -95,19 +95,25 @@ class MultiHeadAttention1D(nn.Module):
             ctx = transpose_depad(attn_pv(probs, pads[2], info, causal=self.is_decoder), batch_size, T, max_seq_len,
                                   info, H, D)
         if fill_cache:
-            if max_seq_len > self.max_seq_len:
-                raise RuntimeError(f"the batch is padded to {max_seq_len} positions but the K/V cache was planned for "
-                                   f"max_seq_len = {self.max_seq_len}")
-            if self.kv_page_size:
-                self.kv_cache = PagedKVCache(batch_size, H, self.max_seq_len, D, x.dtype, x.device,
-                                             page_size=self.kv_page_size, pool_pages=self.kv_pool_pages)
-            else:
-                self.kv_cache = KVCache(batch_size, H, self.max_seq_len, D, x.dtype, x.device, zeroed=False)
-            if kvq is not None:
-                self.kv_cache.fill(kvq, kvq, info, 0, H, longest=max_seq_len)
-            else:
-                self.kv_cache.fill(k.contiguous(), v.contiguous(), info, longest=max_seq_len)
+            self._start_cache(k, v, kvq, info, batch_size, max_seq_len)
         return project(self.dense, ctx.view(1, T, self.hidden_size))
+
+    def _start_cache(self, k, v, kvq, info: SeqInfo, batch_size: int, max_seq_len: int) -> None:
+        """A new cache filled with the prompt's K and V: ``[rows, H, D]`` views, or all three as ``kvq`` ``[rows, 3 H, D]``."""
+        H, D = self.num_heads, self.attention_head_size
+        if max_seq_len > self.max_seq_len:
+            raise RuntimeError(f"the batch is padded to {max_seq_len} positions but the K/V cache was planned for "
+                               f"max_seq_len = {self.max_seq_len}")
+        src = k if kvq is None else kvq
+        if self.kv_page_size:
+            self.kv_cache = PagedKVCache(batch_size, H, self.max_seq_len, D, src.dtype, src.device,
+                                         page_size=self.kv_page_size, pool_pages=self.kv_pool_pages)
+        else:
+            self.kv_cache = KVCache(batch_size, H, self.max_seq_len, D, src.dtype, src.device, zeroed=False)
+        if kvq is not None:
+            self.kv_cache.fill(kvq, kvq, info, 0, H, longest=max_seq_len)
+        else:
+            self.kv_cache.fill(k.contiguous(), v.contiguous(), info, longest=max_seq_len)
 
     # ---- one decode step: newest position only ----------------------------------------------
     def forward_last(self, last: torch.Tensor) -> torch.Tensor:

@@ -16,6 +16,7 @@ from torch.utils._device import DeviceContext
 
 from .. import _lib
 from ..kernel import LayerNorm, depad, layer_norm_forward, repad
+from ..kernel.cuda_native.linear_func import linear_entry
 from ..seqinfo import SeqInfo, seq_info
 from .attention import MultiHeadAttention1D, lens_from_mask
 from .gemm import gemm_tuning
@@ -62,6 +63,53 @@ class Block1D(nn.Module):
                                     self.norm2.normalized_shape, self.norm2.eps, residual=x, return_sum=True)
         return s1 + self.mlp.forward_rows(h2)
 
+    def _plain(self, attn, mlp) -> bool:
+        """True where nothing that the general form of a pre-LN block asks is out of the ordinary: the package's own modules, no
+        gradients, autocast or tuned GEMMs asked for, no global hooks, no modes that want to see the projections."""
+        m = self._modules
+        return not (type(self)._rows is not Block1D._rows or "_rows" in self.__dict__ or type(attn) is not MultiHeadAttention1D
+                    or type(m.get("norm1")) is not LayerNorm or type(m.get("norm2")) is not LayerNorm or not attn.fused_qkv
+                    or torch.is_grad_enabled() or torch.is_autocast_enabled() or gemm_tuning()
+                    or _has_any_global_hook() or _dispatch_modes() or (_function_modes() and _modes_active()))
+
+    def _plain_parameters(self, attn, mlp) -> Optional[list]:
+        """Weights, biases and epsilons of the block in the order they are used, or ``None`` where a module is hooked, compiled,
+        derived, has a method of its own or holds its weights otherwise than as parameters."""
+        m, am, mm, act_fn = self._modules, attn._modules, mlp._modules, mlp.activation
+        qkv, dense, fc1, fc2 = am.get("query_key_value"), am.get("dense"), mm.get("dense_1"), mm.get("dense_2")
+        if not (type(qkv) is type(dense) is type(fc1) is type(fc2) is nn.Linear):
+            return None
+        return _lib.load_front().plain_step(attn, mlp, act_fn if isinstance(act_fn, nn.Module) else None, m.get("norm1"), qkv, dense,
+                                            m.get("norm2"), fc1, fc2)
+
+    def _native_prefill(self, x, info: SeqInfo, batch_size: int, max_seq_len: int, fill_cache: bool) -> Optional[torch.Tensor]:
+        """The general form's ops on packed rows issued by one native call (``block_prefill``), the cache started behind them:
+        in Python two blocks of a short prompt are 400 us of host time for 100 on the GPU.  ``None``, with nothing done, where
+        the block is not one of plain modules."""
+        if self.apply_post_layernorm or x.dtype not in _NATIVE_TYPES or not x.is_cuda:
+            return None
+        m = self._modules
+        attn, mlp = m.get("attn"), m.get("mlp")
+        if type(mlp) is not MLP1D:
+            return None
+        act = activation_code(mlp.activation, mlp._epilogue)
+        if act is None or not self._plain(attn, mlp) or "forward_packed" in attn.__dict__ or "_start_cache" in attn.__dict__ \
+                or _prefill_methods() != _PREFILL_METHODS or (fill_cache and max_seq_len > attn.max_seq_len):
+            return None
+        args = self._plain_parameters(attn, mlp)
+        if args is None:
+            return None
+        H, D = attn.num_heads, attn.attention_head_size
+        table = None if info.ephemeral else info.tile_table(H, max_seq_len, 2 * max_seq_len * D * x.element_size())
+        linear, workspace = (0, None) if mlp._epilogue is None else linear_entry(x.device)
+        out = _lib.front.block_prefill(x, *args, act, H, attn.scaling, attn.is_decoder, info.lens, info.cu_seqlens, table, batch_size,
+                                       max_seq_len, linear, workspace)
+        if out is None:
+            return None
+        if fill_cache:
+            attn._start_cache(None, None, out[1].view(-1, 3 * H, D), info, batch_size, max_seq_len)
+        return out[0]
+
     def _native_decode(self, hidden_states) -> Optional[torch.Tensor]:
         """One decode step of a pre-LN block of plain modules as ``en_block_decode``: five launches, the output written
         straight into the history.  ``None``, with nothing written, where it does not apply (post-LN, separate q, k, v
@@ -72,17 +120,12 @@ class Block1D(nn.Module):
         if self.apply_post_layernorm or hidden_states.dim() != 3 or hidden_states.dtype not in _NATIVE_TYPES:
             return None
         B, _, hid = hidden_states.shape
-        m, own = self._modules, self.__dict__
-        attn, mlp, norm1, norm2 = m.get("attn"), m.get("mlp"), m.get("norm1"), m.get("norm2")
+        m = self._modules
+        attn, mlp = m.get("attn"), m.get("mlp")
         if B > NATIVE_MAX_BATCH or hid > NATIVE_MAX_HIDDEN or type(mlp) is not MLP1D:
             return None
-        act_fn = mlp.activation
-        act = activation_code(act_fn, mlp._epilogue)
-        if act is None or type(self)._rows is not Block1D._rows or "_rows" in own \
-                or type(attn) is not MultiHeadAttention1D or type(norm1) is not LayerNorm \
-                or type(norm2) is not LayerNorm or not attn.fused_qkv \
-                or torch.is_grad_enabled() or torch.is_autocast_enabled() or gemm_tuning() \
-                or _has_any_global_hook() or _dispatch_modes() or (_function_modes() and _modes_active()):
+        act = activation_code(mlp.activation, mlp._epilogue)
+        if act is None or not self._plain(attn, mlp):
             return None
         cache, history = attn.kv_cache, self._history
         cache_type = type(cache)
@@ -90,11 +133,7 @@ class Block1D(nn.Module):
                 or "append" in cache.__dict__ or "attend" in cache.__dict__ \
                 or (cache_type.append, cache_type.attend) != _CACHE_STEP[cache_type] or _step_methods() != _STEP_METHODS:
             return None
-        am, mm = attn._modules, mlp._modules
-        qkv, dense, fc1, fc2 = am.get("query_key_value"), am.get("dense"), mm.get("dense_1"), mm.get("dense_2")
-        if not (type(qkv) is type(dense) is type(fc1) is type(fc2) is nn.Linear):
-            return None
-        args = _lib.load_front().plain_step(attn, mlp, act_fn if isinstance(act_fn, nn.Module) else None, norm1, qkv, dense, norm2, fc1, fc2)
+        args = self._plain_parameters(attn, mlp)
         if args is None:
             return None
         cache.prepare_append()
@@ -110,6 +149,9 @@ class Block1D(nn.Module):
                        fill_cache: bool = False) -> torch.Tensor:
         """``[1,T,hid]`` valid tokens in, ``[1,T,hid]`` out: lets a model drop the padding once
         in front of its first block instead of once per block."""
+        y = self._native_prefill(x, info, batch_size, max_seq_len, fill_cache)
+        if y is not None:
+            return y
         return self._rows(x, lambda h: self.attn.forward_packed(h, info, batch_size, max_seq_len, fill_cache))
 
     def forward(self, hidden_states, attention_mask=None, first_cache=False, seq_lens=None):
@@ -139,8 +181,15 @@ def _step_methods():
             nn.Linear.forward, nn.functional.linear, nn.GELU.forward, nn.functional.gelu, OutputHistory.push)
 
 
+def _prefill_methods():
+    """What the general form runs over packed rows, as it stands now."""
+    return (Block1D._rows, MultiHeadAttention1D.forward_packed, MultiHeadAttention1D._project, MLP1D.forward_rows, LayerNorm.forward,
+            nn.Linear.forward, nn.functional.linear, nn.GELU.forward, nn.functional.gelu)
+
+
 # ... and as it was written: where a caller has put something else in, the native step would pass it by
 _STEP_METHODS = _step_methods()
+_PREFILL_METHODS = _prefill_methods()
 _CACHE_STEP = {c: (c.append, c.attend) for c in (KVCache, PagedKVCache)}
 
 

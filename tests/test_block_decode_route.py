@@ -176,3 +176,77 @@ def test_modes_that_watch_the_projections_keep_the_general_step(step, mode):
     with mode():
         assert not run()
     assert run()
+
+
+@pytest.fixture
+def prefill(monkeypatch):
+    """A block and a function that runs one prefill's choice of route on packed rows that claim to be on the GPU."""
+    from energonai_amd.model import endecoder
+    from energonai_amd.seqinfo import SeqInfo
+
+    class Rows(torch.Tensor):
+        is_cuda = True
+
+    calls = []
+
+    class Front:
+        def block_prefill(self, *args):
+            calls.append(args)
+            return None
+
+    monkeypatch.setattr(_lib, "front", Front())
+    monkeypatch.setattr(endecoder, "linear_entry", lambda device: (1, None))
+    blk = Block1D(128, 2, 2.0, activation=torch.nn.GELU(approximate="tanh"), dtype=torch.float16, max_seq_len=32)
+    lens = torch.tensor([3, 5], dtype=torch.int32)
+    info = SeqInfo(lens, lens, 2, 8, None)
+    info.ephemeral = True
+
+    def run(fill=True, S=8):
+        del calls[:]
+        with torch.no_grad():
+            assert blk._native_prefill(torch.zeros(1, 8, 128, dtype=torch.float16).as_subclass(Rows), info, 2, S, fill) is None
+        return bool(calls)
+
+    return blk, run
+
+
+def test_a_prefill_of_plain_modules_takes_the_native_call(prefill):
+    blk, run = prefill
+    assert run() and run(fill=False)
+    assert not run(S=33) and run(fill=False, S=33)        # longer than the cache: the general form says so
+
+
+PREFILL_CHANGES = {name: CHANGES[name] for name in CHANGES
+                   if "cache" not in name and "history" not in name and "activation" not in name and "forward_last" not in name}
+PREFILL_CHANGES.update({
+    "forward_packed_on_instance": _on_instance("attn", "forward_packed"),
+    "start_cache_on_instance": _on_instance("attn", "_start_cache"),
+    "post_layernorm": lambda blk: setattr(blk, "apply_post_layernorm", True),
+    "other_activation": lambda blk: setattr(blk.mlp, "activation", torch.nn.SiLU()) or setattr(blk.mlp, "_epilogue", None),
+    "separate_projections": lambda blk: setattr(blk.attn, "fused_qkv", False),
+})
+
+
+@pytest.mark.parametrize("name", list(PREFILL_CHANGES))
+def test_what_a_caller_put_in_keeps_the_general_prefill(prefill, name):
+    blk, run = prefill
+    PREFILL_CHANGES[name](blk)
+    assert not run()
+
+
+@pytest.mark.parametrize("owner,name", [(Block1D, "_rows"), (MultiHeadAttention1D, "forward_packed"), (MultiHeadAttention1D, "_project"),
+                                        (MLP1D, "forward_rows"), (LayerNorm, "forward"), (torch.nn.Linear, "forward"),
+                                        (torch.nn.functional, "linear"), (torch.nn.functional, "gelu")])
+def test_methods_replaced_on_the_class_keep_the_general_prefill(prefill, monkeypatch, owner, name):
+    blk, run = prefill
+    method = getattr(owner, name)
+    monkeypatch.setattr(owner, name, lambda *args, **kwargs: method(*args, **kwargs))
+    assert not run()
+
+
+@pytest.mark.parametrize("mode", [Passing, lambda: FlopCounterMode(display=False)])
+def test_modes_that_watch_the_projections_keep_the_general_prefill(prefill, mode):
+    blk, run = prefill
+    with mode():
+        assert not run()
+    assert run()

@@ -117,6 +117,52 @@ def test_kv_cache_fill_and_append_bit_exact(dtype):
     assert overflow.item() == 2
 
 
+@pytest.mark.parametrize("dtype,activation,heads,D,bias,page,lens", [
+    (torch.float16, torch.nn.functional.relu, 4, 64, True, None, [7, 30, 1]),
+    (torch.bfloat16, torch.nn.GELU(), 3, 80, True, 16, [1]),
+    (torch.float16, torch.nn.GELU(approximate="tanh"), 2, 128, False, None, [33, 0, 16]),
+    (torch.float16, torch.nn.functional.gelu, 5, 24, False, None, [4, 4]),
+    (torch.float16, torch.nn.SiLU(), 2, 64, True, None, [5]),             # no code for it: the general form
+    (torch.float16, torch.nn.functional.relu, 2, 136, True, None, None),  # heads the fused kernel does not take
+])
+def test_native_prefill_gives_the_general_forms_bits(monkeypatch, dtype, activation, heads, D, bias, page, lens):
+    """A prefill through the native call against the same block op by op: output, caches, lengths and the steps behind them."""
+    _, M = _mods()
+    from energonai_amd import _lib
+    from energonai_amd.model import endecoder
+    announce("native prefill", dtype, activation, heads, D, bias, page, lens)
+    hid, S = heads * D, 40
+    torch.manual_seed(heads + D)
+    blocks = [M.Block1D(hid, heads, 2.0, activation=activation, dtype=dtype, bias=bias, max_seq_len=64, kv_page_size=page) for _ in range(2)]
+    stack = M.PackedStack(blocks).cuda()
+    calls = []
+    real = _lib.load_front().block_prefill
+    monkeypatch.setattr(_lib.front, "block_prefill", lambda *args: calls.append(real(*args)) or calls[-1], raising=False)
+    if lens is None:
+        with torch.no_grad(), pytest.raises(RuntimeError):
+            stack(torch.randn(1, S, hid, device="cuda").to(dtype), first_cache=True, seq_lens=torch.tensor([5], dtype=torch.int32).cuda())
+        assert calls == [None]
+        return
+    x = torch.randn(len(lens), S, hid, device="cuda").to(dtype)
+    tokens = [torch.randn(len(lens), 1, hid, device="cuda").to(dtype) for _ in range(2)]
+    lens_t = torch.tensor(lens, dtype=torch.int32).cuda()
+
+    def run():
+        with torch.no_grad():
+            out = [stack(x, first_cache=True, seq_lens=lens_t)]
+            state = [t.clone() for b in blocks for t in (b.attn.kv_cache.k, b.attn.kv_cache.v, b.attn.kv_cache.lens)]
+            out += [stack(t).clone() for t in tokens]
+            out.append(blocks[0](x, first_cache=True, seq_lens=lens_t).clone())       # a block by itself
+        return out + state
+
+    got = run()
+    native = endecoder.activation_code(activation, blocks[0].mlp._epilogue)
+    assert len(calls) == (3 if native is not None else 0) and all(c is not None for c in calls)
+    monkeypatch.setattr(M.Block1D, "_native_prefill", lambda *args: None)
+    want = run()
+    assert len(got) == len(want) and all(torch.equal(g, w) for g, w in zip(got, want))
+
+
 @pytest.mark.parametrize("dtype,H,D,Smax,lens", [
     (torch.float16, 4, 64, 50, [7, 30, 1]), (torch.bfloat16, 3, 80, 129, [129, 0, 64, 65]), (torch.float32, 2, 64, 700, [700, 3]),
     (torch.float16, 3, 10, 20, [20, 5]),                 # rows of 20 bytes: no 16-byte pieces, two launches
