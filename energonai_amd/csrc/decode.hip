@@ -210,6 +210,7 @@ struct DecodeAttnArgs {
   const int32_t *page_table;
   int max_pages, lg_page, num_pages;
   int len_add;        // 1: the newest token sits at position kv_lens[b] already, the length does not count it yet
+  int ranked;         // sequences are taken longest first
 };
 
 __device__ __forceinline__ int cached_len(const DecodeAttnArgs &a, int b) { return max(min(a.kv_lens[b] + a.len_add, a.Sk), 0); }
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeA
   const int tid = threadIdx.x;
   const int h = blockIdx.x;
   int b = blockIdx.y;
-  if (a.nsplit == 1 && a.B <= kRankBatch && a.B > 1) {
+  if (a.ranked) {
     // batch index whose length ranks blockIdx.y-th (longest first, ties by index)
     for (int i = tid; i < a.B; i += NT) s_len[i] = cached_len(a, i);
     __syncthreads();
@@ -619,6 +620,10 @@ static int launch_combine_norm(const DecodeNormArgs &n, hipStream_t s) {
 //   kMany   256 x 4   between those two, many units, and few units on caches too short to share: 768 units x 64, 1..2048
 //                     keys 39.3 us (512 x 4: 40.6, 256 x 1: 41.1); 4608 units of 1..2048 keys (2.6 GB) 388 us, 6.8 TB/s
 //                     (512 x 4: 396, 1024 x 1: 402); 72 units of 512 keys 7.9 us (256 x 2: 10.4).
+// Up to one unit a CU none waits for another, whatever their order: the lengths of the whole batch, two barriers and the ranks
+// are saved (8 sequences x 12 heads x 64 of 100 keys 5.0 -> 4.4 us).
+constexpr int64_t kUnrankedUnits = 256;
+
 enum class AttnForm { kTiny, kSmall, kPair, kDeep, kMany };
 
 static AttnForm attn_form(const DecodeAttnArgs &a, int lpk) {
@@ -633,8 +638,10 @@ static AttnForm attn_form(const DecodeAttnArgs &a, int lpk) {
 
 template <int DT, int LPK, bool PAGED, int NT, int U>
 static void launch_attn(const DecodeAttnArgs &a, dim3 grid, bool stream_cache, hipStream_t s) {
-  if (stream_cache) decode_attn_kernel<DT, LPK, NT, U, true, PAGED><<<grid, NT, 0, s>>>(a);
-  else decode_attn_kernel<DT, LPK, NT, U, false, PAGED><<<grid, NT, 0, s>>>(a);
+  DecodeAttnArgs args = a;
+  args.ranked = a.nsplit == 1 && a.B > 1 && a.B <= kRankBatch && (int64_t)a.B * a.H > kUnrankedUnits;
+  if (stream_cache) decode_attn_kernel<DT, LPK, NT, U, true, PAGED><<<grid, NT, 0, s>>>(args);
+  else decode_attn_kernel<DT, LPK, NT, U, false, PAGED><<<grid, NT, 0, s>>>(args);
 }
 
 template <int DT, int LPK, bool PAGED>
