@@ -50,11 +50,12 @@ __global__ __launch_bounds__(kBlock) void attn_qk_kernel(AttnArgs a) {
   static_assert(BN * KVEC_ROW % kBlock == 0 && kQTile * CVEC_ROW % kBlock == 0, "tile must divide over the block");
   __shared__ __attribute__((aligned(16))) T lds[LDS_ELEMS];
 
+  const SeqAhead ahead = seq_ahead(a, a.q_row0, a.k_row0);
   int unit, qi;
   if (!map_block(a, unit, qi)) return;
   const int b = unit / a.H, h = unit % a.H;
-  int kl, ql;
-  seq_extents(a, b, kl, ql);
+  const Seq seq = seq_of(a, ahead, b, a.q_row0, a.k_row0);
+  const int kl = seq.kl, ql = seq.ql;
   const int q0 = qi * kQTile;
   if (q0 >= ql) return;
   const int nk = tile_key_extent(a, min(q0 + kQTile, ql) - 1, kl, ql);
@@ -66,8 +67,8 @@ __global__ __launch_bounds__(kBlock) void attn_qk_kernel(AttnArgs a) {
   const int r = lane & 31, g = lane >> 5;
   const int wq = wave & 1, wk = wave >> 1;
 
-  const T *qbase = reinterpret_cast<const T *>(a.a_ptr) + q_unit_offset(a, b, h);
-  const T *kbase = reinterpret_cast<const T *>(a.b_ptr) + k_unit_offset(a, b, h);
+  const T *qbase = reinterpret_cast<const T *>(a.a_ptr) + q_unit_offset(a, seq, b, h);
+  const T *kbase = reinterpret_cast<const T *>(a.b_ptr) + k_unit_offset(a, seq, b, h);
   T *sbase = reinterpret_cast<T *>(a.out) + ((int64_t)unit * a.Sq) * a.Sk;
 
   // Q fragments stay in registers for the whole key loop.
@@ -215,11 +216,12 @@ __global__ __launch_bounds__(kBlock, 3) void attn_qk_strip_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) T lds_k[2][BK * KP];
   __shared__ __attribute__((aligned(16))) T lds_c[kBlock / kWave][32 * CPITCH];
 
+  const SeqAhead ahead = seq_ahead(a, a.q_row0, a.k_row0);
   int unit, qi;
   if (!map_block(a, unit, qi)) return;
   const int b = unit / a.H, h = unit % a.H;
-  int kl, ql;
-  seq_extents(a, b, kl, ql);
+  const Seq seq = seq_of(a, ahead, b, a.q_row0, a.k_row0);
+  const int kl = seq.kl, ql = seq.ql;
   const int q0 = qi * kQTile;
   if (q0 >= ql) return;
   const int nk = tile_key_extent(a, min(q0 + kQTile, ql) - 1, kl, ql);
@@ -232,8 +234,8 @@ __global__ __launch_bounds__(kBlock, 3) void attn_qk_strip_kernel(AttnArgs a) {
   const int qw = q0 + wave * 32;                 // first query of this wave
   const int q = qw + r;                          // query whose scores this lane accumulates
 
-  const T *qbase = reinterpret_cast<const T *>(a.a_ptr) + q_unit_offset(a, b, h);
-  const T *kbase = reinterpret_cast<const T *>(a.b_ptr) + k_unit_offset(a, b, h);
+  const T *qbase = reinterpret_cast<const T *>(a.a_ptr) + q_unit_offset(a, seq, b, h);
+  const T *kbase = reinterpret_cast<const T *>(a.b_ptr) + k_unit_offset(a, seq, b, h);
   T *sbase = reinterpret_cast<T *>(a.out) + score_unit_offset<EPV>(a, unit);
 
   // Q fragments (B operand): this lane's query row, 8 channels per step; rows >= ql read as zero.  With direct loads
@@ -411,14 +413,15 @@ __global__ __launch_bounds__(kBlock) void attn_pv_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) T lds_p[kQTile * PITCH];
   __shared__ __attribute__((aligned(16))) T lds_v[DP * PITCH];
 
+  const SeqAhead ahead = seq_ahead(a, a.q_row0, a.k_row0);
   int unit, qi;
   if (!map_block(a, unit, qi)) return;
   const int b = unit / a.H, h = unit % a.H;
-  int kl, ql;
-  seq_extents(a, b, kl, ql);
+  const Seq seq = seq_of(a, ahead, b, a.q_row0, a.k_row0);
+  const int kl = seq.kl, ql = seq.ql;
   const int q0 = qi * kQTile;
   const int tid = threadIdx.x;
-  T *cbase = reinterpret_cast<T *>(a.out) + q_unit_offset(a, b, h);
+  T *cbase = reinterpret_cast<T *>(a.out) + q_unit_offset(a, seq, b, h);
 
   if (q0 >= ql) {
     if (a.zero_padding) {  // whole tile is padding
@@ -438,7 +441,7 @@ __global__ __launch_bounds__(kBlock) void attn_pv_kernel(AttnArgs a) {
   const int wq = wave & 1, wd = wave >> 1;
 
   const T *pbase = reinterpret_cast<const T *>(a.a_ptr) + ((int64_t)unit * a.Sq) * a.Sk;
-  const T *vbase = reinterpret_cast<const T *>(a.b_ptr) + k_unit_offset(a, b, h);
+  const T *vbase = reinterpret_cast<const T *>(a.b_ptr) + k_unit_offset(a, seq, b, h);
 
   floatx16 acc[MT][NT];
 #pragma unroll
@@ -605,14 +608,15 @@ __global__ __launch_bounds__(kBlock, 3) void attn_pv_strip_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) T lds_v[2][BK * DP];
   __shared__ __attribute__((aligned(16))) T lds_p[kBlock / kWave][32 * BK];
 
+  const SeqAhead ahead = seq_ahead(a, a.q_row0, a.k_row0);
   int unit, qi;
   if (!map_block(a, unit, qi)) return;
   const int b = unit / a.H, h = unit % a.H;
-  int kl, ql;
-  seq_extents(a, b, kl, ql);
+  const Seq seq = seq_of(a, ahead, b, a.q_row0, a.k_row0);
+  const int kl = seq.kl, ql = seq.ql;
   const int q0 = qi * kQTile;
   const int tid = threadIdx.x;
-  T *cbase = reinterpret_cast<T *>(a.out) + q_unit_offset(a, b, h);
+  T *cbase = reinterpret_cast<T *>(a.out) + q_unit_offset(a, seq, b, h);
 
   if (q0 >= ql) {
     if (a.zero_padding) {  // whole tile is padding
@@ -633,7 +637,7 @@ __global__ __launch_bounds__(kBlock, 3) void attn_pv_strip_kernel(AttnArgs a) {
   const int q = qw + r;                          // query whose context this lane accumulates
 
   const T *pbase = reinterpret_cast<const T *>(a.a_ptr) + score_unit_offset<EPV>(a, unit);
-  const T *vbase = reinterpret_cast<const T *>(a.b_ptr) + k_unit_offset(a, b, h);
+  const T *vbase = reinterpret_cast<const T *>(a.b_ptr) + k_unit_offset(a, seq, b, h);
   // rows of padded queries lie past the end of the descriptor and arrive as zeros; so do V rows >= kl
   const desc_t p_desc = make_desc(pbase, (uint32_t)(score_row_offset<EPV>(a, ql) * E::kSize));
   const desc_t v_desc = make_desc(vbase, kl > 0 ? (uint32_t)(((int64_t)(kl - 1) * a.k_ss + a.D) * E::kSize) : 0u);

@@ -78,11 +78,12 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
   auto kswz = [](int row) { return DP == 128 ? (row & 15) : DP == 96 ? ((row >> 2) & 3) : ((row >> 1) & 7); };
   auto vswz = [](int row) { return DP == 128 ? 4 * (row & 3) : DP == 96 ? 0 : 4 * ((row >> 1) & 1); };
 
+  const SeqAhead ahead = seq_ahead(a, fa.q_row0, fa.k_row0);
   int unit, qi;
   if (!map_block(a, unit, qi, bid)) return;
   const int b = unit / a.H, h = unit % a.H;
-  int kl, ql;
-  seq_extents(a, b, kl, ql);
+  const Seq seq = seq_of(a, ahead, b, fa.q_row0, fa.k_row0);
+  const int kl = seq.kl, ql = seq.ql;
   // The query tiles of a sequence are laid from its END: tile i of n covers rows ql - (n - i) * 128 .. and the ragged
   // tile is the first one (rows below 0 do not exist), whose walk over the keys is the shortest under a causal mask.
   // Laid from the start, the ragged tile would be the last one: a few rows holding a slot for the longest walk.
@@ -102,7 +103,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
   const int vis_max = (q_first < ql && q_first + 31 >= 0) ? (a.causal ? min(kl, min(q_first + 31, ql - 1) + (kl - ql) + 1) : kl) : 0;
 
   // batch base: b * batch stride (padded layout) or first-row * row stride (packed layout)
-  const int64_t qr = fa.q_row0 ? fa.q_row0[b] : 0, kr = fa.k_row0 ? fa.k_row0[b] : 0;
+  const int64_t qr = seq.q_row, kr = seq.k_row;
   const T *qbase = reinterpret_cast<const T *>(a.a_ptr) + (int64_t)b * a.q_sb + qr * a.q_ss + (int64_t)h * a.q_sh;
   const T *kbase = reinterpret_cast<const T *>(a.b_ptr) + (int64_t)b * a.k_sb + kr * a.k_ss + (int64_t)h * a.k_sh;
   const T *vbase = reinterpret_cast<const T *>(fa.v) + (int64_t)b * fa.v_sb + kr * fa.v_ss + (int64_t)h * fa.v_sh;

@@ -39,8 +39,9 @@ __device__ __forceinline__ void fused_f32_tile(const FusedArgs &fa, const NormAr
 
   const int unit = blockIdx.y, qi = blockIdx.x;
   const int b = unit / a.H, h = unit % a.H;
-  int kl, ql;
-  seq_extents(a, b, kl, ql);
+  const SeqAhead ahead = seq_ahead(a, fa.q_row0, fa.k_row0);
+  const Seq seq = seq_of(a, ahead, b, fa.q_row0, fa.k_row0);
+  const int kl = seq.kl, ql = seq.ql;
   const int q0 = qi * kF32QTile;
   if (q0 >= ql) return;
   const int nk = tile_key_extent(a, min(q0 + kF32QTile, ql) - 1, kl, ql);
@@ -57,7 +58,7 @@ __device__ __forceinline__ void fused_f32_tile(const FusedArgs &fa, const NormAr
   const int vis_min = (q_first + 31 < ql) ? (a.causal ? min(kl, q_first + (kl - ql) + 1) : kl) : 0;
   const int vis_max = (q_first < ql) ? (a.causal ? min(kl, min(q_first + 31, ql - 1) + (kl - ql) + 1) : kl) : 0;
 
-  const int64_t qr = fa.q_row0 ? fa.q_row0[b] : 0, kr = fa.k_row0 ? fa.k_row0[b] : 0;
+  const int64_t qr = seq.q_row, kr = seq.k_row;
   const T *qbase = reinterpret_cast<const T *>(a.a_ptr) + (int64_t)b * a.q_sb + qr * a.q_ss + (int64_t)h * a.q_sh;
   const T *kbase = reinterpret_cast<const T *>(a.b_ptr) + (int64_t)b * a.k_sb + kr * a.k_ss + (int64_t)h * a.k_sh;
   const T *vbase = reinterpret_cast<const T *>(fa.v) + (int64_t)b * fa.v_sb + kr * fa.v_ss + (int64_t)h * fa.v_sh;

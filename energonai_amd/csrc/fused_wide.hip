@@ -51,11 +51,12 @@ __global__ __launch_bounds__(kBlock, EN_WIDE_WPE) void attn_fused_wide_kernel(Fu
   __shared__ __attribute__((aligned(16))) T lds_k[2][BK * ROW];
   __shared__ __attribute__((aligned(16))) T lds_v[2][BK * ROW];
 
+  const SeqAhead ahead = seq_ahead(a, fa.q_row0, fa.k_row0);
   int unit, qi;
   if (!map_block(a, unit, qi)) return;
   const int b = unit / a.H, h = unit % a.H;
-  int kl, ql;
-  seq_extents(a, b, kl, ql);
+  const Seq seq = seq_of(a, ahead, b, fa.q_row0, fa.k_row0);
+  const int kl = seq.kl, ql = seq.ql;
   const int q0 = qi * kWideQTile;
   if (q0 >= ql) return;
   const int nk = tile_key_extent(a, min(q0 + kWideQTile, ql) - 1, kl, ql);
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(kBlock, EN_WIDE_WPE) void attn_fused_wide_kernel(Fu
   const int vis_min = (q_first + 63 < ql) ? (a.causal ? min(kl, q_first + (kl - ql) + 1) : kl) : 0;
   const int vis_max = (q_first < ql) ? (a.causal ? min(kl, min(q_first + 63, ql - 1) + (kl - ql) + 1) : kl) : 0;
 
-  const int64_t qr = fa.q_row0 ? fa.q_row0[b] : 0, kr = fa.k_row0 ? fa.k_row0[b] : 0;
+  const int64_t qr = seq.q_row, kr = seq.k_row;
   const T *qbase = reinterpret_cast<const T *>(a.a_ptr) + (int64_t)b * a.q_sb + qr * a.q_ss + (int64_t)h * a.q_sh;
   const T *kbase = reinterpret_cast<const T *>(a.b_ptr) + (int64_t)b * a.k_sb + kr * a.k_ss + (int64_t)h * a.k_sh;
   const T *vbase = reinterpret_cast<const T *>(fa.v) + (int64_t)b * fa.v_sb + kr * fa.v_ss + (int64_t)h * fa.v_sh;
