@@ -42,9 +42,13 @@ def _unit_kv_bytes(k_seq_len: int, size_per_head: int, t: torch.Tensor) -> int:
     return 2 * int(k_seq_len) * int(size_per_head) * t.element_size()
 
 
-def _tile_table_ptr(k_info, q_ptr, head_num: int, q_seq_len: int, unit_kv_bytes: int, query_tile: int = 128):
+def _tile_table_ptr(k_info, q_ptr, head_num: int, q_seq_len: int, unit_kv_bytes: int, query_tile: int = 128,
+                    causal: Optional[bool] = None):
     """Workgroup order for the batch (cached in its SeqInfo) when the query lengths are the key lengths."""
-    return None if q_ptr else k_info.tile_table_ptr(head_num, q_seq_len, unit_kv_bytes, query_tile)
+    if q_ptr:
+        return None
+    mask = {} if causal is None else {"causal": bool(causal)}
+    return k_info.tile_table_ptr(head_num, q_seq_len, unit_kv_bytes, query_tile, **mask)
 
 
 def _fused_dtype_ok(t: torch.Tensor, size_per_head: int, who: str) -> None:
@@ -93,7 +97,7 @@ def attn_qk(q, k, seq_len_list, *, alpha: float = 1.0, causal: bool = True, q_le
         _lib.check(_lib.fn.en_attn_qk(q.data_ptr(), k.data_ptr(), out.data_ptr(), k_info.lens.data_ptr(), q_ptr,
                                           B, H, Sq, Sk, D, *qs, *ks, float(alpha), int(bool(causal)),
                                           _lib.dtype_tag(q, "attn_qk"), None, None, 0,
-                                          _tile_table_ptr(k_info, q_ptr, H, Sq, _unit_kv_bytes(Sk, D, q)), _lib.stream_of(q)), "attn_qk")
+                                          _tile_table_ptr(k_info, q_ptr, H, Sq, _unit_kv_bytes(Sk, D, q), causal=causal), _lib.stream_of(q)), "attn_qk")
     return out
 
 
@@ -123,7 +127,7 @@ def attn_pv(p, v, seq_len_list, *, causal: bool = True, q_len_list=None, zero_pa
         _lib.check(_lib.fn.en_attn_pv(p.data_ptr(), v.data_ptr(), out.data_ptr(), k_info.lens.data_ptr(), q_ptr,
                                           B, H, Sq, Sk, D, *vs, *cs, int(bool(causal)), int(bool(zero_padding)),
                                           _lib.dtype_tag(p, "attn_pv"), None, None, 0,
-                                          _tile_table_ptr(k_info, q_ptr, H, Sq, _unit_kv_bytes(Sk, D, p)), _lib.stream_of(p)), "attn_pv")
+                                          _tile_table_ptr(k_info, q_ptr, H, Sq, _unit_kv_bytes(Sk, D, p), causal=causal), _lib.stream_of(p)), "attn_pv")
     return out
 
 
@@ -160,7 +164,7 @@ def attn_fused(q, k, v, seq_len_list, *, scale: Optional[float] = None, causal: 
                                          k_info.lens.data_ptr(), q_ptr, B, H, Sq, Sk, D, arr(*qs), arr(*ks), arr(*vs),
                                          arr(*cs), None, None, scale, int(bool(causal)),
                                          _lib.dtype_tag(q, "attn_fused"),
-                                         None if qt == 64 else _tile_table_ptr(k_info, q_ptr, H, Sq, _unit_kv_bytes(Sk, D, q), qt),
+                                         None if qt == 64 else _tile_table_ptr(k_info, q_ptr, H, Sq, _unit_kv_bytes(Sk, D, q), qt, causal),
                                          qt, _lib.stream_of(q)), "attn_fused")
     return out
 
@@ -198,7 +202,7 @@ def attn_fused_varlen(q, k, v, batch_size: int, max_seq_len: int, seq_len_list, 
                                          int(max_seq_len), D, arr(*qs), arr(*ks), arr(*vs), arr(0, D, H * D), cu, cu,
                                          scale, int(bool(causal)), _lib.dtype_tag(q, "attn_fused_varlen"),
                                          None if qt == 64 else
-                                         info.tile_table_ptr(H, int(max_seq_len), _unit_kv_bytes(max_seq_len, D, q), qt),
+                                         info.tile_table_ptr(H, int(max_seq_len), _unit_kv_bytes(max_seq_len, D, q), qt, bool(causal)),
                                          qt, _lib.stream_of(q)), "attn_fused_varlen")
     return out
 
@@ -236,7 +240,7 @@ def attn_qk_varlen(q, k, batch_size: int, max_seq_len: int, seq_len_list, *, alp
     with _lib.device_guard(q):
         _lib.check(_lib.fn.en_attn_qk(q.data_ptr(), k.data_ptr(), out.data_ptr(), info.lens.data_ptr(), None, B, H, S, S, D,
                                       *qs, *ks, float(alpha), int(bool(causal)), _lib.dtype_tag(q, "attn_qk_varlen"), cu, cu,
-                                      int(bool(packed_scores)), info.tile_table_ptr(H, S, _unit_kv_bytes(S, D, q)),
+                                      int(bool(packed_scores)), info.tile_table_ptr(H, S, _unit_kv_bytes(S, D, q), causal=bool(causal)),
                                       _lib.stream_of(q)), "attn_qk_varlen")
     return out
 
@@ -275,7 +279,7 @@ def attn_pv_varlen(p, v, batch_size: int, max_seq_len: int, seq_len_list, *, cau
     with _lib.device_guard(v):
         _lib.check(_lib.fn.en_attn_pv(p.data_ptr(), v.data_ptr(), out.data_ptr(), info.lens.data_ptr(), None, B, H, S, S, D,
                                       *vs, 0, D, H * D, int(bool(causal)), 0, _lib.dtype_tag(v, "attn_pv_varlen"), cu, cu,
-                                      int(bool(packed_scores)), info.tile_table_ptr(H, S, _unit_kv_bytes(S, D, v)),
+                                      int(bool(packed_scores)), info.tile_table_ptr(H, S, _unit_kv_bytes(S, D, v), causal=bool(causal)),
                                       _lib.stream_of(v)), "attn_pv_varlen")
     return out
 

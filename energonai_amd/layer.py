@@ -141,14 +141,14 @@ def _layer_one_call(hidden_padded, qkv_packed, info, S, H, D, T, gamma, beta, ep
     kv_bytes = 2 * S * D * hidden_padded.element_size()
     table = arrivals = None
     if fold_depad and not info.ephemeral:
-        offs, table = info.layer_tables(S, left, H, kv_bytes)
+        offs, table = info.layer_tables(S, left, H, kv_bytes, bool(causal))
         arrivals = info._arrivals
         if fused_f32:
             table = None
     else:
         offs = info.row_offsets(S, left) if fold_depad else None
         if not fused_f32 and not info.ephemeral:
-            table = info.tile_table(H, S, kv_bytes)
+            table = info.tile_table(H, S, kv_bytes, causal=bool(causal))
     return _lib.front.layer(hidden_padded, qkv_packed, dense_out, gamma, beta, ctx_out, info.cu_seqlens, info.lens, offs, table,
                             H, D, T, scale, eps, bool(causal), left, form, arrivals)
 

@@ -100,7 +100,7 @@ class Block1D(nn.Module):
         if args is None:
             return None
         H, D = attn.num_heads, attn.attention_head_size
-        table = None if info.ephemeral else info.tile_table(H, max_seq_len, 2 * max_seq_len * D * x.element_size())
+        table = None if info.ephemeral else info.tile_table(H, max_seq_len, 2 * max_seq_len * D * x.element_size(), causal=bool(attn.is_decoder))
         linear, workspace = (0, None) if mlp._epilogue is None else linear_entry(x.device)
         out = _lib.front.block_prefill(x, *args, act, H, attn.scaling, attn.is_decoder, info.lens, info.cu_seqlens, table, batch_size,
                                        max_seq_len, linear, workspace)

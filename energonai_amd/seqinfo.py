@@ -18,7 +18,31 @@ from . import _lib
 
 _CACHE_SIZE = 16
 PER_THREAD_STREAMS = (2,)                 # hipStreamPerThread
-TILES_FIRST_MAX_KV_BYTES = 256 << 10     # see SeqInfo.tile_table
+TILES_FIRST_MAX_KV_BYTES = 256 << 10     # see tiles_first
+TILES_FIRST_MAX_TOTAL_BYTES = 96 << 20
+TILES_FIRST_FEW_UNITS = 256
+TILES_FIRST_FEW_UNITS_TOTAL_BYTES = 160 << 20
+
+
+def tiles_first(units: int, unit_kv_bytes: int, causal: Optional[bool] = None) -> bool:
+    """Whether the last query tiles of all (batch, head) units run before any unit's others, or a unit's tiles stay together
+    (``en_attn_tile_table``).  ``unit_kv_bytes``: K and V of a unit at full length; ``causal`` ``None``: by these alone.
+
+    Under a causal mask a unit's tiles differ in length, last tile longest, and a launch of few units ends on the long tiles of the
+    units that came last; the last tiles first, nothing long is left for the end.  The tiles of a unit then no longer share its
+    K and V in the XCD's L2, which costs nothing while the memory-side cache holds them all beside what else it holds, or with
+    units so few that the tiles running at any time (about 96 an XCD) are several of each.  us a layer, units together / last
+    tiles first: 7 sequences of up to 1531, 20 heads x 80, bf16 82 / 78; 1 of 2048, 64 x 128 123 / 102; 3 of up to 1100, 24 x 96
+    47 / 39; 8 of up to 2048, 16 x 64 100 / 90; 16 of up to 1024, 16 x 128 (256 units, 128 MB) 93 / 91; 64 of up to 1100, 5 x 64 (320, 85
+    MB) 60 / 58; 32 of up to 512, 16 x 64 (512, 64 MB) 38.5 / 37.4.  Beyond: 24 of up to 900, 24 x 64 (576, 126 MB) 69 / 75; 24 of
+    768, 16 x 128 (384, 144 MB) 134 / 146; 64 of up to 256, 20 x 128 (1280, 160 MB) 71 / 74; 4 of up to 2048, 72 x 128 (288, 288 MB)
+    298 / 322; 16 of up to 2048, 12 x 128 (192, 192 MB) 244 / 247.  Without the mask all tiles of a unit are as long, and its K and V
+    are what counts: 32 of up to 512, 16 x 64 44.1 / 46.5, 5 of up to 1300, 20 x 128 66.5 / 71.4."""
+    if causal is None:
+        return unit_kv_bytes <= TILES_FIRST_MAX_KV_BYTES
+    total = units * unit_kv_bytes
+    return causal and (total <= TILES_FIRST_MAX_TOTAL_BYTES or
+                       (units <= TILES_FIRST_FEW_UNITS and total <= TILES_FIRST_FEW_UNITS_TOTAL_BYTES))
 
 
 class SeqInfo:
@@ -114,20 +138,20 @@ class SeqInfo:
                 self._row_offsets[key] = off
         return off
 
-    def layer_tables(self, max_seq_len: int, left_padded: bool, head_num: int, unit_kv_bytes: int):
+    def layer_tables(self, max_seq_len: int, left_padded: bool, head_num: int, unit_kv_bytes: int, causal: Optional[bool] = None):
         """``(row_offsets, tile_table)`` of a layer step (128-row tiles), built by one launch when the batch has neither; the
         launch clears the words of ``arrivals`` as well."""
         version = self._lens_version()
-        first = unit_kv_bytes <= TILES_FIRST_MAX_KV_BYTES
+        first = tiles_first(self.batch_size * head_num, unit_kv_bytes, causal)
         if self.cu_seqlens is None or (version is None and self._mutable()):
-            return self.row_offsets(max_seq_len, left_padded), self.tile_table(head_num, max_seq_len, unit_kv_bytes)
+            return self.row_offsets(max_seq_len, left_padded), self.tile_table(head_num, max_seq_len, unit_kv_bytes, causal=causal)
         off_key, tab_key = (max_seq_len, left_padded, version), (head_num, max_seq_len, first, version, 128)
         off, tab = self._row_offsets.get(off_key), self._tile_tables.get(tab_key)
         self.order_current_stream()     # behind the lookup: what it found may be another thread's, on another stream
         if off is not None and tab is not None:
             return off, tab
         if off is not None or tab is not None:
-            return self.row_offsets(max_seq_len, left_padded), self.tile_table(head_num, max_seq_len, unit_kv_bytes)
+            return self.row_offsets(max_seq_len, left_padded), self.tile_table(head_num, max_seq_len, unit_kv_bytes, causal=causal)
         off, tab, arrivals = _lib.front.layer_tables(self.lens, self.cu_seqlens, self.batch_size, max_seq_len, left_padded,
                                                      self.total, head_num, first)
         self.produced_on_current_stream()
@@ -152,15 +176,17 @@ class SeqInfo:
         return self.cu_seqlens is None or self._source is self.lens
 
 
-    def tile_table(self, head_num: int, q_seq_len: int, unit_kv_bytes: int = 1 << 30, query_tile: int = 128) -> torch.Tensor:
+    def tile_table(self, head_num: int, q_seq_len: int, unit_kv_bytes: int = 1 << 30, query_tile: int = 128,
+                   causal: Optional[bool] = None) -> torch.Tensor:
         """Workgroup order of the attention kernels for this batch (``en_attn_tile_table``): the query tiles the
         sequences really have, longest sequence first.  ``unit_kv_bytes`` is what one (batch, head) unit's K and V
-        hold at full length: up to 256 KB the last tiles of all units run first, above that a unit's tiles stay
-        together.  ``query_tile`` is the tile height of the kernel that will read the table (128; 256 for the fused
+        hold at full length and ``causal`` the mask of the call it is for (``None``: by ``unit_kv_bytes`` alone); they decide
+        whether the last tiles of all units run first or a unit's tiles stay together (``tiles_first``).  ``query_tile`` is the tile height of the kernel that will read the table (128; 256 for the fused
         kernel's 64-queries-per-wave form).  Computed once per batch, head count, bucket, order and tile height by one
         small kernel and reused by every layer."""
         version = self._lens_version()
-        key = (int(head_num), int(q_seq_len), int(unit_kv_bytes) <= TILES_FIRST_MAX_KV_BYTES, version, int(query_tile))
+        first = tiles_first(self.batch_size * int(head_num), int(unit_kv_bytes), causal)
+        key = (int(head_num), int(q_seq_len), first, version, int(query_tile))
         tab = None if version is None and self._mutable() else self._tile_tables.get(key)
         self.order_current_stream()
         if tab is None:
@@ -177,14 +203,15 @@ class SeqInfo:
         return tab
 
 
-    def tile_table_ptr(self, head_num: int, q_seq_len: int, unit_kv_bytes: int = 1 << 30, query_tile: int = 128):
+    def tile_table_ptr(self, head_num: int, q_seq_len: int, unit_kv_bytes: int = 1 << 30, query_tile: int = 128,
+                       causal: Optional[bool] = None):
         """Raw pointer of the workgroup order for an attention call, or ``None`` (the kernels then compute their
         own order) when this object lives for one call only: building the table is a launch of its own, which pays
         off when every layer reuses it, not when every call would rebuild it (lengths given as Python lists or as
         tensors made under ``torch.inference_mode()`` are never cached -- pass a ``SeqInfo`` to keep one)."""
         if self.ephemeral:
             return None
-        return self.tile_table(head_num, q_seq_len, unit_kv_bytes, query_tile).data_ptr()
+        return self.tile_table(head_num, q_seq_len, unit_kv_bytes, query_tile, causal).data_ptr()
 
 
 _cache: "OrderedDict[tuple, SeqInfo]" = OrderedDict()

@@ -356,7 +356,7 @@ int en_attn_fused(const void *q, const void *k, const void *v, void *ctx, const 
  * longest sequence first, so that the launch wastes no workgroup slots on tiles past a sequence's end and its long
  * workgroups start first.  tiles_first == 0 keeps the query tiles of a (batch, head) unit together (they share its
  * K and V in L2); tiles_first != 0 runs the last tiles of all units first, then the second-to-last ... (the better
- * order when a unit's K and V are small: about 256 KB or less).  Built once per batch and reused by every layer;
+ * order under a causal mask while K and V of all units are small, up to about 96 MB, 160 with 256 units and fewer).  Built once per batch and reused by every layer;
  * one small kernel on `stream`. */
 int64_t en_attn_tile_table_elems(int batch, int head_num, int q_seq_len, int query_tile);
 int en_attn_tile_table(const int32_t *seq_lens, int batch, int head_num, int q_seq_len, int tiles_first,

@@ -483,3 +483,13 @@ def test_one_launch_rule(batch, heads, seq, D, total, dtype, pays):
     """Where attention and LayerNorm are one launch: the one rule that the entry point and the step in front of it follow."""
     from energonai_amd import _lib
     assert _lib.fn.en_attn_fused_norm_pays(batch, heads, seq, D, total, dtype) == pays
+
+
+@pytest.mark.parametrize("units,unit_kv_bytes,causal,first", [
+    (1, 1, True, True), (1, 1, False, False), (384, 256 << 10, True, True), (385, 256 << 10, True, False),   # 96 MB of K and V
+    (256, 640 << 10, True, True), (257, 640 << 10, True, False), (256, (640 << 10) + 1, True, False),         # 160 MB in few units
+    (1 << 20, 256 << 10, None, True), (1, (256 << 10) + 1, None, False),                                     # no mask named
+])
+def test_order_of_the_attention_workgroups(units, unit_kv_bytes, causal, first):
+    from energonai_amd.seqinfo import tiles_first
+    assert tiles_first(units, unit_kv_bytes, causal) is first
