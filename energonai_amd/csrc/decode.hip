@@ -258,8 +258,107 @@ __device__ __forceinline__ float across_groups(float v) {
   return v;
 }
 
-template <int DT, int LPK, int NT, int U, bool STREAM, bool PAGED = false>
-__global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeAttnArgs a) {
+// The residual + LayerNorm of a decode step behind the attention, in its launch, where few units leave the launch short and a
+// second one, its start and the trip through the caches are much of what the step consists of.  Nobody waits: the workgroups of a
+// sequence count themselves at a word once their results are where every XCD sees them, and the last one normalises the
+// sequence's row, combining the shares of each unit first where keys are shared.  It leaves the word at zero.
+struct DecodeTail {
+  const void *residual, *gamma, *beta;
+  void *y;
+  uint32_t *words;      // one a sequence, kTailWordStride apart
+  int hidden;
+  float eps;
+};
+constexpr int kTailWordStride = 16;       // a 64-byte line each
+constexpr int kTailVectors = 2;           // 16-byte vectors of a row a lane takes
+constexpr int kAgentScope = 16;           // cache policy of an access that all XCDs see (sc1)
+
+template <typename T>
+__device__ __forceinline__ void store_agent(T *p, T v) {
+  if constexpr (sizeof(T) == 2)
+    __hip_atomic_store(reinterpret_cast<uint16_t *>(p), __builtin_bit_cast(uint16_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    __hip_atomic_store(reinterpret_cast<uint32_t *>(p), __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float load_agent(const float *p) {
+  return __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// Called by the whole workgroup behind its agent-scope stores: true in the last of `all` workgroups.
+__device__ __forceinline__ bool last_to_arrive(uint32_t *word, int all, int *s_last) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the wave's results are where every XCD sees them ...
+  lds_barrier();                                        // ... and the other waves' too, before the workgroup counts itself
+  if (threadIdx.x == 0) {
+    const bool last = (int)atomicAdd(word, 1u) == all - 1;
+    if (last) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *s_last = last;
+  }
+  lds_barrier();
+  return *s_last != 0;
+}
+
+template <int N, bool AGENT = false>
+__device__ __forceinline__ void combine_shares(const DecodeAttnArgs &a, int b, int64_t unit, int d, float (&out)[N]);
+
+// y = LayerNorm(x + residual) of sequence b's row; x is the context, or (SHARED) what its units' shares combine to, four channels a
+// lane.
+template <int DT, int NT, bool SHARED>
+__device__ __forceinline__ void tail_row(const DecodeAttnArgs &a, const DecodeTail &n, int b, float *s_a, float *s_b) {
+  typedef Elem<DT> E;
+  typedef typename E::T T;
+  constexpr int N = SHARED ? 4 : 16 / E::kSize, VPL = SHARED ? 1 : kTailVectors;
+  typedef Pack<T, N> P;
+  const int tid = threadIdx.x, nvec = n.hidden / N;
+  const int64_t row = (int64_t)b * n.hidden;
+  const rsrc_t ctx = make_rsrc(reinterpret_cast<const T *>(a.ctx) + row, (uint32_t)(n.hidden * E::kSize));
+  uint4 raw[VPL];
+  P r[VPL];
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int v = min(tid + NT * j, nvec - 1) * N;
+    if constexpr (!SHARED) raw[j] = buffer_load16<kAgentScope>(ctx, (uint32_t)(v * E::kSize));
+    r[j] = load_pack<T, N>(reinterpret_cast<const T *>(n.residual) + row + v);
+  }
+  float x[VPL][N], s = 0.f, d2 = 0.f;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const bool in = tid + NT * j < nvec;
+    if constexpr (SHARED) {
+      const int v = min(tid, nvec - 1) * N, h = v / a.D;
+      combine_shares<N, true>(a, b, (int64_t)b * a.H + h, v - h * a.D, x[j]);
+    } else {
+      const P c = __builtin_bit_cast(P, raw[j]);
+#pragma unroll
+      for (int e = 0; e < N; ++e) x[j][e] = E::to_float(c.v[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      x[j][e] = in ? x[j][e] + E::to_float(r[j].v[e]) : 0.f;
+      s += x[j][e];
+    }
+  }
+  const float mu = block_allreduce<OpSum, NT / kWave>(s, s_a) / (float)n.hidden;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j)
+    if (tid + NT * j < nvec)
+#pragma unroll
+      for (int e = 0; e < N; ++e) d2 += (x[j][e] - mu) * (x[j][e] - mu);
+  const float inv = 1.0f / sqrtf(block_allreduce<OpSum, NT / kWave>(d2, s_b) / (float)n.hidden + n.eps);
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int v = (tid + NT * j) * N;
+    if (tid + NT * j < nvec) {
+      const P g = load_pack<T, N>(reinterpret_cast<const T *>(n.gamma) + v), bt = load_pack<T, N>(reinterpret_cast<const T *>(n.beta) + v);
+      P o;
+#pragma unroll
+      for (int e = 0; e < N; ++e) o.v[e] = E::from_float((x[j][e] - mu) * inv * E::to_float(g.v[e]) + E::to_float(bt.v[e]));
+      store_pack<T, N>(reinterpret_cast<T *>(n.y) + row + v, o);
+    }
+  }
+}
+
+template <int DT, int LPK, int NT, int U, bool STREAM, bool PAGED, bool TAIL>
+__device__ __forceinline__ void decode_attn_unit(const DecodeAttnArgs &a, const DecodeTail *tail) {
   typedef Elem<DT> E;
   typedef typename E::T T;
   constexpr int EPV = 16 / E::kSize;
@@ -295,7 +394,7 @@ __global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeA
   // workgroup's worth of work and leaves no partial (the combine kernel derives the same shares from the length)
   const int share = split_share(kl, a.nsplit);
   const int kbeg = (int)blockIdx.z * share, kend = min(kl, kbeg + share);
-  if (a.nsplit > 1 && kbeg >= kl) return;
+  if (a.nsplit > 1 && kbeg >= kl && !(TAIL && blockIdx.z == 0)) return;      // an empty sequence has a row to normalise as well
   const T *q = reinterpret_cast<const T *>(a.q) + ((int64_t)b * a.H + h) * a.D;
   const T *kbase = reinterpret_cast<const T *>(a.k) + (PAGED ? 0 : (int64_t)b * a.k_sb) + (int64_t)h * a.k_sh;
   const T *vbase = reinterpret_cast<const T *>(a.v) + (PAGED ? 0 : (int64_t)b * a.v_sb) + (int64_t)h * a.v_sh;
@@ -435,18 +534,48 @@ __global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeA
       o += s_acc[w][d] * f;
     }
     if (a.nsplit > 1) {
-      a.partial[share_index * a.D + d] = o;
-      if (d == 0) *partial_ml(a, share_index) = Partial<2>::type{m_all, l};
+      if constexpr (TAIL) {
+        store_agent(a.partial + share_index * a.D + d, o);
+        if (d == 0) {
+          float *ml = reinterpret_cast<float *>(partial_ml(a, share_index));
+          store_agent(ml, m_all);
+          store_agent(ml + 1, l);
+        }
+      } else {
+        a.partial[share_index * a.D + d] = o;
+        if (d == 0) *partial_ml(a, share_index) = Partial<2>::type{m_all, l};
+      }
     } else {
-      ctx[d] = E::from_float(l > 0.f ? o / l : 0.f);
+      const T c_d = E::from_float(l > 0.f ? o / l : 0.f);
+      if constexpr (TAIL) store_agent(ctx + d, c_d);
+      else ctx[d] = c_d;
     }
   }
+  if constexpr (TAIL) {
+    __shared__ int s_last;
+    // workgroups of a sequence: a unit's shares that had keys, one for an empty sequence
+    const int shares = a.nsplit > 1 && share > 0 ? (kl + share - 1) / share : 1;
+    if (!last_to_arrive(tail->words + b * kTailWordStride, a.H * shares, &s_last)) return;
+    if (a.nsplit > 1) tail_row<DT, NT, true>(a, *tail, b, s_m, s_l);
+    else tail_row<DT, NT, false>(a, *tail, b, s_m, s_l);
+  }
+}
+
+template <int DT, int LPK, int NT, int U, bool STREAM, bool PAGED = false>
+__global__ __launch_bounds__(NT, U == 1 ? 8 : 4) void decode_attn_kernel(DecodeAttnArgs a) {
+  decode_attn_unit<DT, LPK, NT, U, STREAM, PAGED, false>(a, nullptr);
+}
+// At most two units a CU: registers for four waves a SIMD are enough, and the row at the end needs them.
+template <int DT, int LPK, int NT, int U, bool STREAM>
+__global__ __launch_bounds__(NT, 4) void decode_attn_norm_kernel(DecodeAttnArgs a, DecodeTail tail) {
+  decode_attn_unit<DT, LPK, NT, U, STREAM, false, true>(a, &tail);
 }
 
 // Combines N channels, from channel d on, of the partial results of a unit's shares.  The partials of kAhead shares are
 // sent for together with the length that says how many of them were written (the workspace holds nsplit of them whatever
 // the length), so that one trip to memory is waited for instead of three.
-template <int N>
+// AGENT: other workgroups of the same launch wrote them.
+template <int N, bool AGENT>
 __device__ __forceinline__ void combine_shares(const DecodeAttnArgs &a, int b, int64_t unit, int d, float (&out)[N]) {
   constexpr int kAhead = 4;
   typedef typename Partial<N>::type P;
@@ -460,8 +589,15 @@ __device__ __forceinline__ void combine_shares(const DecodeAttnArgs &a, int b, i
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
       const int64_t share_index = unit * a.nsplit + min(z0 + i, a.nsplit - 1);
-      o[i] = *reinterpret_cast<const P *>(a.partial + share_index * a.D + d);
-      ml[i] = *partial_ml(a, share_index);
+      if constexpr (AGENT) {
+        static_assert(N == 4, "one 16-byte load");
+        const float *p_ml = reinterpret_cast<const float *>(partial_ml(a, share_index));
+        o[i] = __builtin_bit_cast(P, buffer_load16<kAgentScope>(make_rsrc(a.partial, 0x7fffffffu), (uint32_t)((share_index * a.D + d) * 4)));
+        ml[i] = Partial<2>::type{load_agent(p_ml), load_agent(p_ml + 1)};
+      } else {
+        o[i] = *reinterpret_cast<const P *>(a.partial + share_index * a.D + d);
+        ml[i] = *partial_ml(a, share_index);
+      }
     }
     if (z0 == 0) {
       const int kl = cached_len(a, b);
@@ -675,6 +811,49 @@ static int dispatch_attn(const DecodeAttnArgs &a, bool stream_cache, hipStream_t
     EN_RETURN_IF_LAUNCH_FAILED();
   }
   return EN_OK;
+}
+
+template <int DT, int LPK, int NT, int U>
+static void launch_attn_norm(const DecodeAttnArgs &a, const DecodeTail &tail, dim3 grid, bool stream_cache, hipStream_t s) {
+  DecodeAttnArgs args = a;
+  args.ranked = a.nsplit == 1 && a.B > 1 && a.B <= kRankBatch && (int64_t)a.B * a.H > kUnrankedUnits;
+  if (stream_cache) decode_attn_norm_kernel<DT, LPK, NT, U, true><<<grid, NT, 0, s>>>(args, tail);
+  else decode_attn_norm_kernel<DT, LPK, NT, U, false><<<grid, NT, 0, s>>>(args, tail);
+}
+
+// The forms of attn_form below 512 units, for heads of 33..128 channels (fp32: 17..128).  From 512 units on the attention is several
+// times what the second launch costs.
+template <int DT, int LPK>
+static int launch_attn_norm_form(const DecodeAttnArgs &a, const DecodeTail &tail, dim3 grid, bool stream_cache, hipStream_t s) {
+  const AttnForm form = attn_form(a, LPK);
+  const int lanes = form == AttnForm::kPair ? 512 : 256;
+  // One workgroup has the whole row to read.  us a layer, two launches / one: 1 x 12 heads x 64, up to 300 keys 8.5 / 6.3, 8 x 12 x 64
+  // 8.4 / 6.9, 2 x 8 x 64 fp32, up to 800 9.2 / 8.0, 16 x 24 x 64, up to 900 15.0 / 14.7, 16 x 32 x 128, up to 128 10.1 / 10.1; of five
+  // vectors a lane, 2 x 60 x 128, up to 500 10.3 / 10.7, 5 x 72 x 128 35.8 / 36.8.  Rows of shares are four channels a lane, sixteen
+  // bytes from each share: 1 x 5 x 64, 4000 keys 9.3 / 8.6, 10 x 16 x 64, up to 2000 15.2 / 14.2; combined unit by unit in front of
+  // the row, which takes wider ones, 6 x 64 x 128 41.9 / 43.9.
+  if (a.nsplit > 1 ? tail.hidden > 4 * lanes : tail.hidden * Elem<DT>::kSize > kTailVectors * 16 * lanes) return EN_ERR_UNSUPPORTED;
+  switch (form) {
+    case AttnForm::kTiny: launch_attn_norm<DT, LPK, 256, 1>(a, tail, grid, stream_cache, s); break;
+    case AttnForm::kSmall: launch_attn_norm<DT, LPK, 256, 2>(a, tail, grid, stream_cache, s); break;
+    case AttnForm::kPair: launch_attn_norm<DT, LPK, 512, 2>(a, tail, grid, stream_cache, s); break;
+    case AttnForm::kMany: launch_attn_norm<DT, LPK, 256, 4>(a, tail, grid, stream_cache, s); break;
+    default: return EN_ERR_UNSUPPORTED;
+  }
+  EN_RETURN_IF_LAUNCH_FAILED();
+  return EN_OK;
+}
+
+template <int DT>
+static int dispatch_attn_norm(const DecodeAttnArgs &a, const DecodeTail &tail, bool stream_cache, hipStream_t s) {
+  constexpr int EPV = 16 / Elem<DT>::kSize;
+  const dim3 grid((unsigned)a.H, (unsigned)a.B, (unsigned)a.nsplit);
+  if (a.D > 128) return EN_ERR_UNSUPPORTED;
+  if constexpr (DT == EN_F32)
+    if (a.D > 16 * EPV) return launch_attn_norm_form<DT, 32>(a, tail, grid, stream_cache, s);
+  if (a.D > 8 * EPV) return launch_attn_norm_form<DT, 16>(a, tail, grid, stream_cache, s);
+  if (a.D > 4 * EPV) return launch_attn_norm_form<DT, 8>(a, tail, grid, stream_cache, s);
+  return EN_ERR_UNSUPPORTED;
 }
 
 // How many workgroups share one unit's keys: none while the units alone fill the chip (512 units and more); else
@@ -970,6 +1149,53 @@ int en_decode_layer(const void *q, const void *k_cache, const void *v_cache, voi
     case EN_F32: return launch_combine_norm<EN_F32>(n, s);
     case EN_F16: return launch_combine_norm<EN_F16>(n, s);
     default: return launch_combine_norm<EN_BF16>(n, s);
+  }
+}
+
+int64_t en_decode_layer_norm_words(void) { return (int64_t)en::kRankBatch * en::kTailWordStride; }
+
+int en_decode_layer_norm(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens, int batch,
+                         int head_num, int k_seq_len, int size_per_head, const int64_t *k_strides, const int64_t *v_strides,
+                         float scale, const void *residual, const void *gamma, const void *beta, void *y, float eps, int dtype,
+                         void *workspace, int64_t workspace_bytes, uint32_t *words, en_stream_t stream) {
+  using namespace en;
+  if (!residual || !gamma || !beta || !y || !words) return EN_ERR_NULL;
+  DecodeAttnArgs a;
+  const int rc = attn_args(a, q, k_cache, v_cache, ctx, kv_lens, batch, head_num, k_seq_len, size_per_head, k_strides, v_strides,
+                           scale, dtype, workspace, workspace_bytes);
+  if (rc) return rc;
+  const int64_t es = dtype_size(dtype), hidden = (int64_t)head_num * size_per_head, rows = batch * hidden * es, S = k_seq_len;
+  if (batch > kRankBatch || (int64_t)batch * head_num >= 512 || size_per_head % (16 / es)) return EN_ERR_UNSUPPORTED;
+  for (const void *p : {(const void *)ctx, residual, gamma, beta, (const void *)y})
+    if (!aligned_to(p, 16)) return EN_ERR_UNSUPPORTED;
+  if (!aligned_to(words, 4) || (a.nsplit > 1 && !aligned_to(workspace, 16))) return EN_ERR_UNSUPPORTED;
+  // A row is normalised while others are still attended to: buffers that a caller has laid over each other need two launches.
+  auto cache = [&](const int64_t *st) { return ((batch - 1) * st[0] + (head_num - 1) * st[1] + (S - 1) * st[2] + size_per_head) * es; };
+  struct Range { const void *p; int64_t bytes; };
+  const Range read[] = {{q, rows}, {k_cache, cache(k_strides)}, {v_cache, cache(v_strides)}, {kv_lens, (int64_t)batch * 4},
+                        {residual, rows}, {gamma, hidden * es}, {beta, hidden * es}};
+  const Range written[] = {{y, rows}, {ctx, rows}, {workspace, a.nsplit > 1 ? workspace_bytes : 0}};
+  auto meet = [](const Range &x, const Range &w) {
+    const uintptr_t u = (uintptr_t)x.p, v = (uintptr_t)w.p;
+    return u < v + (uintptr_t)w.bytes && v < u + (uintptr_t)x.bytes;
+  };
+  for (const Range &w : written)
+    for (const Range &x : read)
+      if (meet(x, w)) return EN_ERR_UNSUPPORTED;
+  if (meet(written[0], written[1]) || meet(written[0], written[2]) || meet(written[1], written[2])) return EN_ERR_UNSUPPORTED;
+  // A captured launch may run again on any stream, beside launches that use the same words.
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess) {      // e.g. the null stream beside a capture
+    (void)hipGetLastError();
+    return EN_ERR_UNSUPPORTED;
+  }
+  if (capture != hipStreamCaptureStatusNone) return EN_ERR_UNSUPPORTED;
+  const DecodeTail tail{residual, gamma, beta, y, words, (int)hidden, eps};
+  const bool stream_cache = 2 * cache_bytes(a.B, a.H, a.Sk, a.D, dtype) >= kAttnStreamBytes;
+  switch (dtype) {
+    case EN_F32: return dispatch_attn_norm<EN_F32>(a, tail, stream_cache, (hipStream_t)stream);
+    case EN_F16: return dispatch_attn_norm<EN_F16>(a, tail, stream_cache, (hipStream_t)stream);
+    default: return dispatch_attn_norm<EN_BF16>(a, tail, stream_cache, (hipStream_t)stream);
   }
 }
 

@@ -13,8 +13,10 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <map>
 #include <stdexcept>
 #include <string>
+#include <utility>
 
 #include "energon_hip.h"
 
@@ -264,6 +266,28 @@ PyObject *layer(PyObject *const *a) {
   return THPVariable_Wrap(y);
 }
 
+// The words of en_decode_layer_norm for launches on torch's current stream of a device, 16 KB a stream, or null.  They belong to
+// the stream: its order keeps launches apart that share them, and torch's own streams (a fixed pool a device, which bounds this) live
+// as long as the process.  An external stream's handle may come back as another stream's while the first one's work still runs,
+// so it gets none; nor does a capture, whose launches may run again beside others.
+uint32_t *decode_words(const Tensor &t) {
+  static std::map<std::pair<int, hipStream_t>, Tensor> &pool = *new std::map<std::pair<int, hipStream_t>, Tensor>;     // under the interpreter lock
+  const auto stream = c10::hip::getCurrentHIPStream(t.device().index());
+  if (stream.id() != 0 && stream.id() == (c10::StreamId) reinterpret_cast<intptr_t>(stream.stream())) return nullptr;   // external
+  const auto key = std::make_pair((int)t.device().index(), stream.stream());
+  auto at = pool.find(key);
+  if (at == pool.end()) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream.stream(), &capture) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    if (capture != hipStreamCaptureStatusNone) return nullptr;
+    at = pool.emplace(key, at::zeros({en_decode_layer_norm_words()}, t.options().dtype(at::kInt))).first;
+  }
+  return reinterpret_cast<uint32_t *>(at->second.data_ptr<int32_t>());
+}
+
 // decode_layer(q, k_cache, v_cache, lens, residual, gamma, beta, dense_out, eps, scale) -> y
 PyObject *decode_layer(PyObject *const *a) {
   const Tensor &q_in = gpu(a[0], "q", false), &k = gpu(a[1], "k_cache", false), &v = gpu(a[2], "v_cache", false);
@@ -309,6 +333,18 @@ PyObject *decode_layer(PyObject *const *a) {
   void *ctx_p = ctx.data_ptr(), *y_p = y.data_ptr(), *ws_p = need > 0 ? ws.data_ptr() : nullptr;
   const int32_t *lens_p = i32(lens);
   const hipStream_t stream = stream_of(k);
+  // small enough: one launch
+  uint32_t *words = !dense_p && tag == out_tag && B * H < 512 ? decode_words(k) : nullptr;
+  if (words) {
+    const int rc = without_gil([&] {
+      return en_decode_layer_norm(q_p, k_p, v_p, ctx_p, lens_p, (int)B, (int)H, (int)S, (int)D, ks, vs, scale, res_p, gamma_p, beta_p, y_p,
+                                  eps, tag, ws_p, need, words, stream);
+    });
+    if (rc != EN_ERR_UNSUPPORTED) {
+      check(rc, "decode_layer");
+      return THPVariable_Wrap(y);
+    }
+  }
   check(without_gil([&] {
           return en_decode_layer(q_p, k_p, v_p, ctx_p, lens_p, (int)B, (int)H, (int)S, (int)D, ks, vs, scale, dense_p, res_p, gamma_p, beta_p,
                                  y_p, hid, eps, tag, out_tag, ws_p, need, stream);

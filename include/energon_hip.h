@@ -277,6 +277,17 @@ int en_decode_layer(const void *q, const void *k_cache, const void *v_cache, voi
                     int64_t hidden, float eps, int dtype, int out_dtype, void *workspace, int64_t workspace_bytes,
                     en_stream_t stream);
 
+/* en_decode_layer without a projection in between, out_dtype == dtype, in one launch for batches of few units (fewer than 512
+ * (sequence, head) pairs): the last workgroup of a sequence normalises its row.  words: en_decode_layer_norm_words() uint32,
+ * zero before the first launch that uses them and after every one; launches that may overlap must not share them.  workspace
+ * as in en_decode_layer; ctx is written only where no keys are shared.  Captured streams, overlapping buffers, wider rows and other head
+ * sizes return EN_ERR_UNSUPPORTED with nothing launched: en_decode_layer takes those. */
+int64_t en_decode_layer_norm_words(void);
+int en_decode_layer_norm(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens, int batch,
+                         int head_num, int k_seq_len, int size_per_head, const int64_t *k_strides, const int64_t *v_strides,
+                         float scale, const void *residual, const void *gamma, const void *beta, void *y, float eps, int dtype,
+                         void *workspace, int64_t workspace_bytes, uint32_t *words, en_stream_t stream);
+
 /* New K/V caches [batch, head_num, cache_len, size_per_head] from a projection's packed rows [T, src_head_rows, size_per_head],
  * K from its heads k_head_first .., V from v_head_first .., zeros behind each sequence: en_transpose_pad_heads for both in one
  * launch (8 sequences, 12 heads x 64, 512 positions: 4 launches of 3.9 us, two fills and two movers, become one of 6.3). */

@@ -8,6 +8,8 @@ size-independent properties (bit-exact pack round trips, rows of probabilities
 summing to one, LayerNorm row statistics) plus an oracle comparison on a
 subset of sequences, so the CPU side stays within seconds.
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -468,6 +470,89 @@ def test_decode_layer_one_native_call(dtype, B, H, S, D):
                              beta.cuda(), 1e-5, dense_out=dense.cuda())
     want = torch.nn.functional.layer_norm(dense.double() + res.double(), (H * D,), gamma.double(), beta.double(), 1e-5)
     assert_stored_close(got.cpu(), want, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,S,D", [
+    (1, 1, 40, 64),         # one workgroup is the last one
+    (3, 5, 300, 80),        # lanes past the head size
+    (16, 20, 100, 64),      # one key a lane group and step; sequences ranked
+    (15, 32, 250, 128),     # 4096 channels, as many as 256 lanes take (fp32: more than that)
+    (2, 33, 250, 128),      # one head more
+    (5, 8, 700, 96),        # four keys a lane group
+    (2, 16, 1100, 128),     # two shares, fewer workgroups than CUs: 512 lanes, 2048 channels, as many as they take
+    (2, 17, 1100, 128),     # one head more
+    (30, 16, 1500, 64),     # two shares of 480 units: 256 lanes, 1024 channels
+    (3, 10, 5000, 64),      # nine shares, more than are sent for at once
+])
+def test_decode_layer_in_one_launch(dtype, B, H, S, D):
+    """``en_decode_layer_norm`` against the float64 oracle, empty sequences among them; the same bits again and again, and the words
+    back at zero.  The bound is that of ``test_decode_layer_one_native_call``."""
+    from energonai_amd import _lib
+    announce("decode layer, one launch", dtype, B, H, S, D)
+    g = torch.Generator().manual_seed(S + H)
+    kv = ([S, 0, 1, 513, 700, 64, 65] * 5)[:B] if B > 1 else [S - 3]
+    kv = [min(n, S) for n in kv]
+    q = torch.randn(B, H, 1, D, generator=g).to(dtype)
+    kc, vc = (torch.randn(B, H, S, D, generator=g).to(dtype) for _ in range(2))
+    res = torch.randn(1, B, H * D, generator=g).to(dtype)
+    gamma, beta = (1 + 0.02 * torch.randn(H * D, generator=g)).to(dtype), (0.02 * torch.randn(H * D, generator=g)).to(dtype)
+    args = [t.cuda() for t in (q, kc, vc, res, gamma, beta)]
+    lens = torch.tensor(kv, dtype=torch.int32).cuda()
+    words = torch.zeros(_lib.fn.en_decode_layer_norm_words(), dtype=torch.int32, device="cuda")
+    need = _lib.fn.en_decode_attn_workspace_bytes(B, H, S, D)
+    ws = torch.full((max(need, 16),), 0xff, dtype=torch.uint8, device="cuda")       # NaN wherever nothing is written
+    strides = (ctypes.c_int64 * 3)(H * S * D, S * D, D)
+    out = []
+    for _ in range(3):
+        ctx, y = torch.empty(B, H, 1, D, dtype=dtype, device="cuda"), torch.empty(1, B, H * D, dtype=dtype, device="cuda")
+        rc = _lib.fn.en_decode_layer_norm(args[0].data_ptr(), args[1].data_ptr(), args[2].data_ptr(), ctx.data_ptr(), lens.data_ptr(), B, H,
+                                          S, D, strides, strides, D ** -0.5, args[3].data_ptr(), args[4].data_ptr(), args[5].data_ptr(),
+                                          y.data_ptr(), 1e-5, _lib.dtype_tag(q, "test"), ws.data_ptr(), need, words.data_ptr(),
+                                          _lib.stream_of(args[0]))
+        if H in (17, 33) or (dtype == torch.float32 and H == 32):
+            assert rc == -5
+            return
+        assert rc == 0
+        out.append(y)
+    assert not words.any() and torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    _, _, ctx = eager.decode_attention(q, kc, vc, kv, D ** -0.5, acc_dtype=torch.float64)
+    want = torch.nn.functional.layer_norm(ctx.view(1, B, H * D) + res.double(), (H * D,), gamma.double(), beta.double(), 1e-5)
+    assert_stored_close(out[0].cpu(), want, dtype)
+    # rows that the call's own output overlaps, and a capture, are for the two launches
+    assert _lib.fn.en_decode_layer_norm(args[0].data_ptr(), args[1].data_ptr(), args[2].data_ptr(), out[0].data_ptr(), lens.data_ptr(), B, H, S,
+                                        D, strides, strides, D ** -0.5, args[3].data_ptr(), args[4].data_ptr(), args[5].data_ptr(),
+                                        out[0].data_ptr(), 1e-5, _lib.dtype_tag(q, "test"), ws.data_ptr(), need, words.data_ptr(),
+                                        _lib.stream_of(args[0])) == -5
+
+
+def test_decode_layer_words_belong_to_their_stream():
+    """Steps on several streams at once, and one in a graph beside them, each give what a step alone gives."""
+    from energonai_amd import layer
+    from energonai_amd.seqinfo import SeqInfo
+    B, H, S, D = 2, 12, 1500, 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+    def rand(*shape):
+        return torch.randn(shape, generator=g, device="cuda", dtype=torch.float16)
+    lens = torch.tensor([1500, 700], dtype=torch.int32, device="cuda")
+    info = SeqInfo(lens, None, B, None, lens)
+    a = (rand(B, H, 1, D), rand(B, H, S, D), rand(B, H, S, D), info, rand(1, B, H * D), rand(H * D), rand(H * D))
+    want = layer.decode_layer(*a)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        recorded = layer.decode_layer(*a)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    got = []
+    for _ in range(8):
+        graph.replay()
+        for s in streams:
+            with torch.cuda.stream(s):
+                got.append(layer.decode_layer(*a))
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, want) for y in got)
+    # the graph holds the two launches: combined and normalised in another order of summation
+    assert (recorded.float() - want.float()).abs().max() <= 2 ** -9 * want.float().abs().max()
 
 
 @pytest.mark.parametrize("lens,S,H,left", [([1], 17, 1, False), ([64, 0, 300, 7, 128, 129], 300, 5, True),
