@@ -92,6 +92,9 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
   const int q0 = ql - (ntl - qi) * kQTile;
   const int nk = tile_key_extent(a, min(q0 + kQTile, ql) - 1, kl, ql);
   const int nkt = (nk + BK - 1) / BK;
+  NormTile rows;
+  if constexpr (NORM)
+    rows = norm_tile_of(*norm, (int64_t)b * a.ntq + qi, seq.q_row + max(q0, 0), min(q0 + kQTile, ql) - max(q0, 0), h, a.H);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -378,8 +381,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
       if ((unsigned)qrow < (unsigned)ql && c * EPV < a.D) *reinterpret_cast<uint4 *>(cbase + (int64_t)qrow * fa.c_ss + c * EPV) = v;
     }
     if constexpr (NORM) {
-      const int first = max(q0, 0);
-      norm_tile<DT>(*norm, norm->arrivals + ((int64_t)b * a.ntq + qi) * kNormWordStride, qr + first, min(q0 + kQTile, ql) - first, h, a.H);
+      norm_tile<DT>(*norm, rows);
     }
     return;
   }

@@ -53,42 +53,72 @@ constexpr int kNormMaxHeads = 48;         // shares that a meeting word has room
 constexpr int kNormMaxVectors = 4 * kWave; // a wave per row, up to four 16-byte vectors per lane
 constexpr int kAgentScope = 16;           // cache policy of an access that all XCDs see (sc1)
 
+// Rows of a wave in flight at once: the context comes from memory (other XCDs wrote it), a trip of 2 us each time otherwise.
+constexpr int norm_rows_ahead(int dt, int vpl) { return dt == EN_F32 ? (vpl <= 3 ? 2 : 1) : vpl <= 2 ? 3 : 1; }
+constexpr int kNormRowsAhead = 3;
+
+// A workgroup's share of its tile's rows, and where the residuals of the first ones lie: scalars that are looked up before the
+// keys are walked, a trip to memory less behind them.
+struct NormTile {
+  unsigned long long *word;
+  int64_t row0;                 // packed row of the tile's first
+  int nrows, share, shares;
+  int res_off[kNormRowsAhead];  // of the wave's first rows
+};
+
+__device__ __forceinline__ NormTile norm_tile_of(const NormArgs &n, int64_t word, int64_t row0, int nrows, int share, int shares) {
+  NormTile t{n.arrivals + word * kNormWordStride, row0, nrows, share, shares, {}};
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), step = shares * (kBlock / kWave);
+#pragma unroll
+  for (int k = 0; k < kNormRowsAhead; ++k)
+    t.res_off[k] = n.res_off[row0 + min(share * (kBlock / kWave) + wave + k * step, nrows - 1)];
+  return t;
+}
+
 template <int DT, int VPL>
-__device__ __forceinline__ void norm_tile_rows(const NormArgs &n, unsigned long long *word, int64_t row0, int nrows, int share,
-                                               int shares, unsigned long long *s_take) {
+__device__ __forceinline__ void norm_tile_rows(const NormArgs &n, const NormTile &t, unsigned long long *s_take) {
+  unsigned long long *const word = t.word;
+  const int64_t row0 = t.row0;
+  const int nrows = t.nrows, share = t.share, shares = t.shares;
   typedef Elem<DT> E;
   typedef typename E::T T;
   constexpr int EPV = 16 / E::kSize, NW = kBlock / kWave;
   typedef Pack<T, EPV> P;
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
   const int nvec = n.width / EPV;
+  const uint32_t bytes = (uint32_t)(n.width * E::kSize);      // the loads of vectors past the row give zeros
   constexpr bool EARLY = VPL <= 3;              // gamma and beta in registers while the workgroups meet: four vectors do not fit
-  // Rows of a wave in flight at once: the context comes from memory (other XCDs wrote it), a trip of 2 us per row otherwise.
-  constexpr int R = VPL <= 2 ? 2 : 1;
+  constexpr int R = norm_rows_ahead(DT, VPL);
+  static_assert(R <= kNormRowsAhead, "offsets looked up ahead");
   const int step = shares * NW;
   uint4 res[R][VPL];
   P g[VPL], bt[VPL];
-  auto load_residual = [&](int first) {
+  auto load_residual = [&](int first, auto off_of) {
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      const int64_t t = row0 + min(first + k * step, nrows - 1);
-      const T *p = reinterpret_cast<const T *>(n.residual) + (t + n.res_off[t]) * n.width;
+      const int64_t row = row0 + min(first + k * step, nrows - 1);
+      const rsrc_t p = make_rsrc(reinterpret_cast<const T *>(n.residual) + (row + off_of(k, row)) * n.width,
+                                 first + k * step < nrows ? bytes : 0u);
 #pragma unroll
-      for (int j = 0; j < VPL; ++j) res[k][j] = *reinterpret_cast<const uint4 *>(p + min(lane + kWave * j, nvec - 1) * EPV);
+      for (int j = 0; j < VPL; ++j) res[k][j] = buffer_load16(p, (uint32_t)(lane + kWave * j) * 16u);
     }
   };
   auto load_affine = [&](int j) {
-    const int v = min(lane + kWave * j, nvec - 1) * EPV;
-    g[j] = load_pack<T, EPV>(reinterpret_cast<const T *>(n.gamma) + v);
-    bt[j] = load_pack<T, EPV>(reinterpret_cast<const T *>(n.beta) + v);
+    g[j] = __builtin_bit_cast(P, buffer_load16(make_rsrc(n.gamma, bytes), (uint32_t)(lane + kWave * j) * 16u));
+    bt[j] = __builtin_bit_cast(P, buffer_load16(make_rsrc(n.beta, bytes), (uint32_t)(lane + kWave * j) * 16u));
   };
+  unsigned long long arrived = 0;               // what it answers comes back ahead of the loads behind it
+  if (threadIdx.x == 0) {
+    int at = 0;
+    asm("" : "+v"(at));                         // a lane's own address: behind a uniform one the answer is waited for here and passed round
+    arrived = atomicAdd(word + at, 1ull);
+  }
   if constexpr (EARLY)
 #pragma unroll
     for (int j = 0; j < VPL; ++j) load_affine(j);
   int held = share * NW + wave;                 // first of the rows whose residuals are in registers
-  if (held < nrows) load_residual(held);
+  load_residual(held, [&](int k, int64_t) { return t.res_off[k]; });
   if (threadIdx.x == 0) {
-    const unsigned long long arrived = atomicAdd(word, 1ull);
     unsigned long long take = 0;                // shares to do here
     if ((int)(arrived & 63) == shares - 1) {
       take = arrived >> 12 | 1ull << share;
@@ -111,14 +141,15 @@ __device__ __forceinline__ void norm_tile_rows(const NormArgs &n, unsigned long 
 #pragma unroll
       for (int k = 0; k < R; ++k) {
         const rsrc_t ctx = make_rsrc(reinterpret_cast<const T *>(n.ctx) + (row0 + i + k * step) * n.width,
-                                     i + k * step < nrows ? (uint32_t)(n.width * E::kSize) : 0u);
+                                     i + k * step < nrows ? bytes : 0u);
 #pragma unroll
         for (int j = 0; j < VPL; ++j) raw[k][j] = buffer_load16<kAgentScope>(ctx, (uint32_t)(lane + kWave * j) * 16u);
       }
-      if (i != held) load_residual(i);
+      if (i != held) load_residual(i, [&](int, int64_t row) { return __builtin_amdgcn_readfirstlane(n.res_off[row]); });
       held = i;
 #pragma unroll
       for (int k = 0; k < R; ++k) {
+        __builtin_amdgcn_sched_barrier(0);      // row by row: their sums side by side take more registers than there are
         if (i + k * step >= nrows) break;
         float x[VPL][EPV], s = 0.f, d2 = 0.f;
 #pragma unroll
@@ -165,17 +196,16 @@ __device__ __forceinline__ void norm_tile_rows(const NormArgs &n, unsigned long 
   }
 }
 
-// Called by the whole workgroup of (batch b's query tile `word`, head `share`) when it has sent its context rows away with
-// agent-scope stores.  nrows rows of the tile, the first one packed row row0.
+// Called by the whole workgroup when it has sent its context rows away with agent-scope stores.
 template <int DT>
-__device__ __forceinline__ void norm_tile(const NormArgs &n, unsigned long long *word, int64_t row0, int nrows, int share, int shares) {
+__device__ __forceinline__ void norm_tile(const NormArgs &n, const NormTile &t) {
   __shared__ unsigned long long s_take;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the wave's context rows are where every XCD sees them ...
   lds_barrier();                                        // ... and the other waves' too, before the workgroup says so
   const int nvec = n.width / (16 / Elem<DT>::kSize);
-  if (nvec <= 2 * kWave) norm_tile_rows<DT, 2>(n, word, row0, nrows, share, shares, &s_take);
-  else if (nvec <= 3 * kWave) norm_tile_rows<DT, 3>(n, word, row0, nrows, share, shares, &s_take);
-  else norm_tile_rows<DT, 4>(n, word, row0, nrows, share, shares, &s_take);
+  if (nvec <= 2 * kWave) norm_tile_rows<DT, 2>(n, t, &s_take);
+  else if (nvec <= 3 * kWave) norm_tile_rows<DT, 3>(n, t, &s_take);
+  else norm_tile_rows<DT, 4>(n, t, &s_take);
 }
 
 // Both halves of the wave get (x of lanes 0..31, x of lanes 32..63): one VALU swap, no LDS round trip.

@@ -46,6 +46,8 @@ __device__ __forceinline__ void fused_f32_tile(const FusedArgs &fa, const NormAr
   if (q0 >= ql) return;
   const int nk = tile_key_extent(a, min(q0 + kF32QTile, ql) - 1, kl, ql);
   const int nkt = (nk + BK - 1) / BK;
+  NormTile rows;
+  if constexpr (NORM) rows = norm_tile_of(*norm, (int64_t)b * gridDim.x + qi, seq.q_row + q0, min(kF32QTile, ql - q0), h, a.H);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -236,7 +238,7 @@ __device__ __forceinline__ void fused_f32_tile(const FusedArgs &fa, const NormAr
       buffer_store16<kAgentScope>(c_rsrc, q0 + row < ql && d < a.D ? (uint32_t)((int64_t)(q0 + row) * fa.c_ss + d) * 4u : kOutOfRange,
                                   *reinterpret_cast<const uint4 *>(&lds_k[row * KP + d]));
     }
-    norm_tile<EN_F32>(*norm, norm->arrivals + ((int64_t)b * gridDim.x + qi) * kNormWordStride, qr + q0, min(kF32QTile, ql - q0), h, a.H);
+    norm_tile<EN_F32>(*norm, rows);
   }
 }
 
