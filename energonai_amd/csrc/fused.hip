@@ -381,7 +381,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
       if ((unsigned)qrow < (unsigned)ql && c * EPV < a.D) *reinterpret_cast<uint4 *>(cbase + (int64_t)qrow * fa.c_ss + c * EPV) = v;
     }
     if constexpr (NORM) {
-      norm_tile<DT>(*norm, rows);
+      norm_tile<DT, DP>(*norm, rows);
     }
     return;
   }
@@ -519,15 +519,17 @@ static int attn_fused(const void *q, const void *k, const void *v, void *ctx, co
 // Workgroups that are resident at once: what LDS and registers leave room for on 256 CUs.
 static int64_t resident_workgroups(int size_per_head, int dtype) { return dtype == EN_F32 ? 512 : size_per_head <= 64 ? 1024 : 768; }
 
-// Where one launch is the faster form, us per layer, one launch / two (8 layers, hot operands).  Meeting costs about 7 us
-// (context written through, counted, seen, read back) plus a trip to memory for every two rows of a wave; a LayerNorm launch
-// costs 5 us and what its bytes take.
-//   16-bit: context of 7 MB and more and at most three rows per wave: 24 sequences of up to 384, 16 heads x 64 22.4 / 24.2,
-//     8 of up to 600, 16 x 96 27.1 / 28.7, 2 of 1024, 16 x 128 33.0 / 33.7; smaller ones lose (16 of up to 128, 12 x 64
-//     13.6 / 11.8, one of 509 17.9 / 15.7), as do few heads (64 of up to 128, 4 x 64 17.3 / 13.1).  Where the launches
-//     themselves are what bounds a layer, short prompts: one of 60 rows, 12 x 64 10.4 / 11.3, 64 of up to 30, 4 x 64 10.7 / 13.1
-//     (16 x 64, a full chip: 13.8 / 13.1).
-//   fp32 (64-row tiles): 4 of up to 128, 12 x 64 15.0 / 15.5, 16 of up to 128 21.3 / 21.9; 64 of up to 128, 4 x 64 22.2 / 21.8.
+// Where one launch is the faster form, us per layer, one launch / two (6 layers, hot operands).  Meeting costs about 6 us
+// (context written through, counted, seen, read back), a trip to memory for every round of a wave's rows (norm_rows_ahead); a
+// LayerNorm launch costs 5 us and what its bytes take.
+//   16-bit: context of 7 MB and more and at most three rows per wave: 24 sequences of up to 384, 16 heads x 64 22.4 / 24.2, 4 of up
+//     to 700, 16 x 128 22.4 / 23.6 (not every one: 8 of up to 665, 14 x 96 25.2 / 24.7).  From 3.5 to 7 MB the two are close, one launch
+//     ahead since three rows of a wave go out at once (32 of up to 128, 16 x 64 11.6 / 11.9, 1 of 1024, 16 x 128 28.6 / 28.9, 14 of up to
+//     356, 11 x 80 16.1 / 17.0, 8 of up to 256, 32 x 64 14.6 / 15.5), at 3 MB they meet (8 of up to 300, 12 x 80 14.8 / 14.5), and
+//     smaller ones lose (16 of up to 128, 12 x 64 10.7 / 9.5, one of 509 15.1 / 13.4), as do few heads (64 of up to 128, 4 x 64
+//     15.1 / 10.5).  Where the launches themselves are what bounds a layer, short prompts: one of 60 rows, 12 x 64 10.4 / 11.3 with the
+//     host's part, 64 of up to 30, 4 x 64 10.7 / 13.1 (16 x 64, a full chip: 13.8 / 13.1).
+//   fp32 (64-row tiles): 4 of up to 128, 12 x 64 15.0 / 15.5, 21 of up to 73, 6 x 64 12.3 / 12.5; 58 of up to 239, 3 x 64 39.0 / 34.8.
 static bool one_launch_pays(int heads, int seq_len, int64_t tiles, int64_t bytes, int dtype) {
   const int64_t per_wave = ceil_div(std::min(seq_len, dtype == EN_F32 ? kF32QTile : kQTile), heads * (kBlock / kWave));
   if (dtype == EN_F32) return per_wave <= 2;

@@ -53,8 +53,12 @@ constexpr int kNormMaxHeads = 48;         // shares that a meeting word has room
 constexpr int kNormMaxVectors = 4 * kWave; // a wave per row, up to four 16-byte vectors per lane
 constexpr int kAgentScope = 16;           // cache policy of an access that all XCDs see (sc1)
 
-// Rows of a wave in flight at once: the context comes from memory (other XCDs wrote it), a trip of 2 us each time otherwise.
-constexpr int norm_rows_ahead(int dt, int vpl) { return dt == EN_F32 ? (vpl <= 3 ? 2 : 1) : vpl <= 2 ? 3 : 1; }
+// Rows of a wave in flight at once: the context comes from memory (other XCDs wrote it), a trip of 2 us each time otherwise.  As
+// many as a wave has in most tiles and as the registers of the attention hold (head_pitch: channels of a head in LDS; at 64
+// four waves share a SIMD's registers, above that three).
+constexpr int norm_rows_ahead(int dt, int head_pitch, int vpl) {
+  return dt == EN_F32 ? (vpl <= 3 ? 2 : 1) : vpl <= 2 ? 3 : head_pitch > 64 ? 2 : 1;
+}
 constexpr int kNormRowsAhead = 3;
 
 // A workgroup's share of its tile's rows, and where the residuals of the first ones lie: scalars that are looked up before the
@@ -75,7 +79,7 @@ __device__ __forceinline__ NormTile norm_tile_of(const NormArgs &n, int64_t word
   return t;
 }
 
-template <int DT, int VPL>
+template <int DT, int DP, int VPL>
 __device__ __forceinline__ void norm_tile_rows(const NormArgs &n, const NormTile &t, unsigned long long *s_take) {
   unsigned long long *const word = t.word;
   const int64_t row0 = t.row0;
@@ -88,7 +92,7 @@ __device__ __forceinline__ void norm_tile_rows(const NormArgs &n, const NormTile
   const int nvec = n.width / EPV;
   const uint32_t bytes = (uint32_t)(n.width * E::kSize);      // the loads of vectors past the row give zeros
   constexpr bool EARLY = VPL <= 3;              // gamma and beta in registers while the workgroups meet: four vectors do not fit
-  constexpr int R = norm_rows_ahead(DT, VPL);
+  constexpr int R = norm_rows_ahead(DT, DP, VPL);
   static_assert(R <= kNormRowsAhead, "offsets looked up ahead");
   const int step = shares * NW;
   uint4 res[R][VPL];
@@ -197,15 +201,15 @@ __device__ __forceinline__ void norm_tile_rows(const NormArgs &n, const NormTile
 }
 
 // Called by the whole workgroup when it has sent its context rows away with agent-scope stores.
-template <int DT>
+template <int DT, int DP>
 __device__ __forceinline__ void norm_tile(const NormArgs &n, const NormTile &t) {
   __shared__ unsigned long long s_take;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the wave's context rows are where every XCD sees them ...
   lds_barrier();                                        // ... and the other waves' too, before the workgroup says so
   const int nvec = n.width / (16 / Elem<DT>::kSize);
-  if (nvec <= 2 * kWave) norm_tile_rows<DT, 2>(n, t, &s_take);
-  else if (nvec <= 3 * kWave) norm_tile_rows<DT, 3>(n, t, &s_take);
-  else norm_tile_rows<DT, 4>(n, t, &s_take);
+  if (nvec <= 2 * kWave) norm_tile_rows<DT, DP, 2>(n, t, &s_take);
+  else if (nvec <= 3 * kWave) norm_tile_rows<DT, DP, 3>(n, t, &s_take);
+  else norm_tile_rows<DT, DP, 4>(n, t, &s_take);
 }
 
 // Both halves of the wave get (x of lanes 0..31, x of lanes 32..63): one VALU swap, no LDS round trip.

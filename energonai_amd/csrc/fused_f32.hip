@@ -238,7 +238,7 @@ __device__ __forceinline__ void fused_f32_tile(const FusedArgs &fa, const NormAr
       buffer_store16<kAgentScope>(c_rsrc, q0 + row < ql && d < a.D ? (uint32_t)((int64_t)(q0 + row) * fa.c_ss + d) * 4u : kOutOfRange,
                                   *reinterpret_cast<const uint4 *>(&lds_k[row * KP + d]));
     }
-    norm_tile<EN_F32>(*norm, rows);
+    norm_tile<EN_F32, DP>(*norm, rows);
   }
 }
 
