@@ -580,6 +580,8 @@ def test_layer_tables_in_one_launch(lens, S, H, left):
     ([140, 1], 257, 48, 16, True, False),                   # the most shares a word has room for
     ([140, 30], 257, 49, 16, True, False),                  # one more: two launches
     ([130, 3], 140, 16, 128, False, False),
+    ([128, 77], 128, 3, 64, False, True),                   # eleven rows a wave: rounds of three, the last one of two
+    ([129, 300], 300, 9, 128, True, True),                  # three vectors a lane, four rows a wave: rounds of two
     ([100] * 200, 128, 16, 64, True, False),                # more than one round of workgroups: two launches
 ])
 def test_attention_and_layernorm_in_one_launch(dtype, lens, S, H, D, causal, left):
