@@ -296,11 +296,6 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
         pf[2 * kb] = __builtin_bit_cast(uint4, pk[0]);
         pf[2 * kb + 1] = __builtin_bit_cast(uint4, pk[1]);
       }
-      {
-        float lo, hi;
-        halves_of(l_tile, lo, hi);
-        l_tile = lo + hi;
-      }
       l_run += l_tile;
 
     }
@@ -347,7 +342,10 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
   }
 
   // ---- normalise and store: register 4j+i of tile mt holds channel 32mt + 8j + 4g + i of this lane's query
-  const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+  // each half of the wave has added up its own keys: both were scaled alike, so they are put together once
+  float l_lo, l_hi;
+  halves_of(l_run, l_lo, l_hi);
+  const float l_all = l_lo + l_hi, inv = l_all > 0.f ? 1.0f / l_all : 0.f;
   const int lane_e = lane_now(), r_e = lane_e & 31, g_e = lane_e >> 5;
   if (NORM || fa.c_vec16) {
     // A lane holds 8-byte pieces of its own row, 32 rows per store instruction; through LDS (the K buffers are free
