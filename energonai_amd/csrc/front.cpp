@@ -539,8 +539,8 @@ PyObject *block_prefill(PyObject *const *a) {
   Tensor ws;
   if (a[25] != Py_None) ws = gpu(a[25], "workspace");
   if (!usable || !n1w.defined() || !n1b.defined() || !n2w.defined() || !n2b.defined() || !qkv_w.defined() || !dense_w.defined() ||
-      !m1w.defined() || !m2w.defined() || lens.device() != x.device() || cu.device() != x.device() || lens.numel() < batch ||
-      cu.numel() < batch + 1 || !(scale > 0.f) || (linear && !ws.defined()) || (!linear && act != EN_ACT_GELU))
+      !m1w.defined() || !m2w.defined() || lens.device() != x.device() || cu.device() != x.device() || lens.numel() != batch ||
+      cu.numel() != batch + 1 || !(scale > 0.f) || (linear && !ws.defined()) || (!linear && act != EN_ACT_GELU))
     Py_RETURN_NONE;
   const c10::DeviceGuard guard(x.device());
   const int tag = dtype_tag(x, "block_prefill");

@@ -190,6 +190,9 @@ def prefill(monkeypatch):
     calls = []
 
     class Front:
+        def prefix_sum(self, lens, batch):
+            return torch.cat((lens.new_zeros(1), lens.cumsum(0).int())), lens
+
         def block_prefill(self, *args):
             calls.append(args)
             return None
@@ -198,13 +201,13 @@ def prefill(monkeypatch):
     monkeypatch.setattr(endecoder, "linear_entry", lambda device: (1, None))
     blk = Block1D(128, 2, 2.0, activation=torch.nn.GELU(approximate="tanh"), dtype=torch.float16, max_seq_len=32)
     lens = torch.tensor([3, 5], dtype=torch.int32)
-    info = SeqInfo(lens, lens, 2, 8, None)
-    info.ephemeral = True
+    batch = SeqInfo(lens, lens, 2, 8, None)
+    batch.ephemeral = True
 
-    def run(fill=True, S=8):
+    def run(fill=True, S=8, info=batch, batch_size=2):
         del calls[:]
         with torch.no_grad():
-            assert blk._native_prefill(torch.zeros(1, 8, 128, dtype=torch.float16).as_subclass(Rows), info, 2, S, fill) is None
+            assert blk._native_prefill(torch.zeros(1, 8, 128, dtype=torch.float16).as_subclass(Rows), info, batch_size, S, fill) is None
         return bool(calls)
 
     return blk, run
@@ -214,6 +217,31 @@ def test_a_prefill_of_plain_modules_takes_the_native_call(prefill):
     blk, run = prefill
     assert run() and run(fill=False)
     assert not run(S=33) and run(fill=False, S=33)        # longer than the cache: the general form says so
+
+
+def test_a_native_prefill_waits_for_the_lengths(prefill, monkeypatch):
+    """The prefix sum may have been launched on another stream; a SeqInfo without a tile table is waited for as well."""
+    from energonai_amd.seqinfo import SeqInfo
+    blk, run = prefill
+    events = []
+    monkeypatch.setattr(SeqInfo, "order_current_stream", lambda self: events.append("ordered"))
+    native = _lib.front.block_prefill
+    monkeypatch.setattr(_lib.front, "block_prefill", lambda *args: events.append("launched") or native(*args), raising=False)
+    assert run() and events[0] == "ordered" and events.count("launched") == 1 and events[-1] == "launched"
+
+
+@pytest.mark.parametrize("batch_size", [1, 3])
+def test_a_native_prefill_refuses_lengths_of_another_batch(prefill, batch_size):
+    blk, run = prefill
+    with pytest.raises(RuntimeError, match="SeqInfo was built for batch 2"):
+        run(batch_size=batch_size)
+    assert blk.attn.kv_cache is None
+
+
+def test_a_native_prefill_takes_plain_lengths(prefill):
+    """Lengths that are not a SeqInfo become one, as in the general form's attention."""
+    blk, run = prefill
+    assert run(info=[3, 5], fill=False)
 
 
 PREFILL_CHANGES = {name: CHANGES[name] for name in CHANGES

@@ -163,6 +163,32 @@ def test_native_prefill_gives_the_general_forms_bits(monkeypatch, dtype, activat
     assert len(got) == len(want) and all(torch.equal(g, w) for g, w in zip(got, want))
 
 
+def test_native_prefill_takes_the_lengths_that_the_general_form_takes(monkeypatch):
+    """Packed rows with a lengths tensor or a list in place of the SeqInfo; lengths of another batch never reach a launch."""
+    _, M = _mods()
+    from energonai_amd import _lib
+    from energonai_amd.seqinfo import seq_info
+    announce("native prefill, lengths")
+    torch.manual_seed(6)
+    blk = M.Block1D(128, 2, 2.0, dtype=torch.float16, max_seq_len=64).cuda()
+    x, lens = torch.randn(1, 37, 128, device="cuda").half(), [7, 30]
+    lens_t, calls = torch.tensor(lens, dtype=torch.int32).cuda(), []
+    native = _lib.load_front().block_prefill
+    monkeypatch.setattr(_lib.front, "block_prefill", lambda *args: calls.append(args) or native(*args), raising=False)
+    with torch.no_grad():
+        want = blk.forward_packed(x, seq_info(lens_t, 2, x.device), 2, 32)
+        for given in (lens_t, lens):
+            assert torch.equal(blk.forward_packed(x, given, 2, 32), want)
+        assert len(calls) == 3
+        for batch in (1, 3):
+            with pytest.raises(RuntimeError, match="SeqInfo was built for batch 2"):
+                blk.forward_packed(x, seq_info(lens_t, 2, x.device), batch, 32)
+            args = list(calls[0])
+            args[22] = batch
+            assert native(*args) is None
+    assert len(calls) == 3
+
+
 @pytest.mark.parametrize("dtype,H,D,Smax,lens", [
     (torch.float16, 4, 64, 50, [7, 30, 1]), (torch.bfloat16, 3, 80, 129, [129, 0, 64, 65]), (torch.float32, 2, 64, 700, [700, 3]),
     (torch.float16, 3, 10, 20, [20, 5]),                 # rows of 20 bytes: no 16-byte pieces, two launches
