@@ -99,8 +99,10 @@ class Block1D(nn.Module):
         args = self._plain_parameters(attn, mlp)
         if args is None:
             return None
-        info = seq_info(info, batch_size, x.device)     # as the general form's attention asks for it: this batch, this stream
         H, D = attn.num_heads, attn.attention_head_size
+        if H * D != x.shape[-1]:                        # heads set to what the projections are not: the general form refuses them
+            return None
+        info = seq_info(info, batch_size, x.device)     # as the general form's attention asks for it: this batch, this stream
         table = None if info.ephemeral else info.tile_table(H, max_seq_len, 2 * max_seq_len * D * x.element_size(), causal=bool(attn.is_decoder))
         linear, workspace = (0, None) if mlp._epilogue is None else linear_entry(x.device)
         out = _lib.front.block_prefill(x, *args, act, H, attn.scaling, attn.is_decoder, info.lens, info.cu_seqlens, table, batch_size,

@@ -251,6 +251,7 @@ PREFILL_CHANGES.update({
     "start_cache_on_instance": _on_instance("attn", "_start_cache"),
     "post_layernorm": lambda blk: setattr(blk, "apply_post_layernorm", True),
     "other_activation": lambda blk: setattr(blk.mlp, "activation", torch.nn.SiLU()) or setattr(blk.mlp, "_epilogue", None),
+    "heads_that_the_projections_do_not_have": lambda blk: setattr(blk.attn, "num_heads", 4),
     "separate_projections": lambda blk: setattr(blk.attn, "fused_qkv", False),
 })
 
