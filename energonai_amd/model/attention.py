@@ -106,14 +106,15 @@ class MultiHeadAttention1D(nn.Module):
                                f"max_seq_len = {self.max_seq_len}")
         src = k if kvq is None else kvq
         if self.kv_page_size:
-            self.kv_cache = PagedKVCache(batch_size, H, self.max_seq_len, D, src.dtype, src.device,
-                                         page_size=self.kv_page_size, pool_pages=self.kv_pool_pages)
+            cache = PagedKVCache(batch_size, H, self.max_seq_len, D, src.dtype, src.device,
+                                 page_size=self.kv_page_size, pool_pages=self.kv_pool_pages)
         else:
-            self.kv_cache = KVCache(batch_size, H, self.max_seq_len, D, src.dtype, src.device, zeroed=False)
+            cache = KVCache(batch_size, H, self.max_seq_len, D, src.dtype, src.device, zeroed=False)
         if kvq is not None:
-            self.kv_cache.fill(kvq, kvq, info, 0, H, longest=max_seq_len)
+            cache.fill(kvq, kvq, info, 0, H, longest=max_seq_len)
         else:
-            self.kv_cache.fill(k.contiguous(), v.contiguous(), info, longest=max_seq_len)
+            cache.fill(k.contiguous(), v.contiguous(), info, longest=max_seq_len)
+        self.kv_cache = cache       # only now: rows and lengths of a cache that was not filled are whatever the memory held
 
     # ---- one decode step: newest position only ----------------------------------------------
     def forward_last(self, last: torch.Tensor) -> torch.Tensor:

@@ -244,6 +244,25 @@ def test_a_native_prefill_takes_plain_lengths(prefill):
     assert run(info=[3, 5], fill=False)
 
 
+@pytest.mark.parametrize("page", [None, 16])
+def test_a_cache_that_could_not_be_filled_is_not_kept(monkeypatch, page):
+    """Its rows and lengths are uninitialised memory: the module keeps the cache it had."""
+    from energonai_amd.model.kv_cache import PagedKVCache
+
+    def fail(self, *args, **kwargs):
+        raise RuntimeError("not filled")
+
+    for cache in (KVCache, PagedKVCache):
+        monkeypatch.setattr(cache, "fill", fail)
+    attn = MultiHeadAttention1D(128, 2, max_seq_len=32, kv_page_size=page)
+    kvq = torch.zeros(8, 6, 64, dtype=torch.float16)
+    for before in (None, KVCache(2, 2, 32, 64, torch.float16, "cpu")):
+        attn.kv_cache = before
+        with pytest.raises(RuntimeError, match="not filled"):
+            attn._start_cache(None, None, kvq, None, 2, 8)
+        assert attn.kv_cache is before
+
+
 PREFILL_CHANGES = {name: CHANGES[name] for name in CHANGES
                    if "cache" not in name and "history" not in name and "activation" not in name and "forward_last" not in name}
 PREFILL_CHANGES.update({
