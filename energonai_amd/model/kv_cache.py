@@ -20,6 +20,8 @@ from ..seqinfo import SeqInfo
 
 
 class KVCache:
+    _zeroed = True          # what is not there in a cache saved before there was a choice
+
     def __init__(self, batch_size: int, head_num: int, max_seq_len: int, size_per_head: int, dtype, device, zeroed: bool = True):
         """``zeroed=False``: for a caller that fills the cache next; ``fill`` writes the zeros with the rows."""
         new = torch.zeros if zeroed else torch.empty

@@ -263,6 +263,20 @@ def test_a_cache_that_could_not_be_filled_is_not_kept(monkeypatch, page):
         assert attn.kv_cache is before
 
 
+def test_a_cache_saved_before_it_could_be_unzeroed_is_filled(monkeypatch):
+    """A pickled cache of that time has zeros in its buffers and says nothing about them."""
+    from energonai_amd.model import kv_cache
+    from energonai_amd.seqinfo import SeqInfo
+    filled = []
+    monkeypatch.setattr(kv_cache, "kv_cache_fill", lambda *args, zero_padding: filled.append(zero_padding))
+    monkeypatch.setattr(kv_cache, "kv_cache_start", lambda *args: filled.append("start"))
+    cache = KVCache(2, 2, 32, 64, torch.float16, "cpu")
+    del cache.__dict__["_zeroed"]
+    lens, rows = torch.tensor([3, 5], dtype=torch.int32), torch.zeros(8, 6, 64, dtype=torch.float16)
+    cache.fill(rows, rows, SeqInfo(lens, lens, 2, 8, None), 0, 2)
+    assert filled == [False, False] and cache.lens.tolist() == [3, 5]
+
+
 PREFILL_CHANGES = {name: CHANGES[name] for name in CHANGES
                    if "cache" not in name and "history" not in name and "activation" not in name and "forward_last" not in name}
 PREFILL_CHANGES.update({
