@@ -499,11 +499,13 @@ PyObject *block_decode(PyObject *const *a) {
 }
 
 // block_prefill(x [1,T,hidden], norm1 w, b, eps, qkv w, b, dense w, b, norm2 w, b, eps, mlp1 w, b, mlp2 w, b, activation, heads, scale,
-//               causal, lens, cu_seqlens, tile table or None, batch, max_seq_len, address of en_linear or 0, its workspace or None)
-// -> (block's output [1,T,hidden], packed projections [1,T,3 hidden]), or None, with nothing done, where a tensor is not what the
-// kernels take.  The ops are those of the general step one by one: LayerNorm, projection, fused attention on packed rows,
-// projection, residual + LayerNorm that keeps the sum, MLP (both GEMMs by en_linear with the activation in its epilogue, or by
-// torch around exact GELU), sum.
+//               causal, lens, cu_seqlens, tile table or None, batch, max_seq_len, address of en_linear or 0, its workspace or None,
+//               what to call with the packed projections [1,T,3 hidden] or None)
+// -> block's output [1,T,hidden], or None, with nothing done, where a tensor is not what the kernels take.  The ops are those of the
+// general step one by one: LayerNorm, projection, fused attention on packed rows, the call with the projections (it fills a cache),
+// projection, residual + LayerNorm that keeps the sum, MLP (both GEMMs by en_linear with the activation in its epilogue, or by torch
+// around exact GELU), sum.  A tensor is given up where it is last read: at its peak, the MLP, the call holds x, sum, h2 and the MLP's
+// own, a row of hidden less than the general form, which keeps the first LayerNorm's output.
 typedef int (*en_linear_fn)(const void *, const void *, const void *, void *, int64_t, int64_t, int64_t, int, int, int, void *, int64_t,
                             hipStream_t);
 PyObject *block_prefill(PyObject *const *a) {
@@ -546,22 +548,37 @@ PyObject *block_prefill(PyObject *const *a) {
   const int tag = dtype_tag(x, "block_prefill");
   const hipStream_t stream = stream_of(x);
   const int32_t *lens_p = i32(lens), *cu_p = i32(cu);
-  Tensor y, kvq;
-  auto run = [&]() -> int {
+  Tensor kvq, ctx, y;
+  auto attend = [&]() -> int {
     const Tensor h = at::empty_like(x);
     check(en_layernorm_fwd(h.data_ptr(), nullptr, nullptr, nullptr, x.data_ptr(), nullptr, nullptr, n1w.data_ptr(), n1b.data_ptr(), T, hid,
                            eps1, tag, tag, stream), "layer_norm");
     kvq = at::linear(h, qkv_w, qkv_b);
     // packed rows of 3 heads x D, ordered k, v, q (attention.py:74)
-    const Tensor ctx = at::empty({1, T, hid}, x.options());
+    ctx = at::empty({1, T, hid}, x.options());
     const int64_t in[3] = {0, D, 3 * hid}, out[3] = {0, D, hid};
     const char *rows = static_cast<const char *>(kvq.data_ptr());
     check(en_attn_fused(rows + 2 * hid * 2, rows, rows + hid * 2, ctx.data_ptr(), lens_p, nullptr, (int)batch, (int)heads, (int)S, (int)S, (int)D,
                         in, in, in, out, cu_p, cu_p, scale, causal, tag, table, 0, stream), "attn_fused_varlen");
-    const Tensor att = at::linear(ctx, dense_w, dense_b);
-    const Tensor h2 = at::empty_like(x), sum = at::empty_like(x);
+    return EN_OK;
+  };
+  (void)without_gil(attend);
+  if (a[26] != Py_None) {
+    PyObject *rows = THPVariable_Wrap(kvq);
+    PyObject *done = rows ? PyObject_CallOneArg(a[26], rows) : nullptr;
+    Py_XDECREF(rows);
+    if (!done) return nullptr;
+    Py_DECREF(done);
+  }
+  kvq.reset();      // under the lock: a Python object may belong to it
+  auto rest = [&]() -> int {
+    Tensor att = at::linear(ctx, dense_w, dense_b);
+    ctx.reset();
+    Tensor h2 = at::empty_like(x);
+    const Tensor sum = at::empty_like(x);
     check(en_layernorm_fwd(h2.data_ptr(), nullptr, nullptr, sum.data_ptr(), att.data_ptr(), x.data_ptr(), nullptr, n2w.data_ptr(), n2b.data_ptr(),
                            T, hid, eps2, tag, tag, stream), "layer_norm");
+    att.reset();
     Tensor m;
     if (linear) {
       const Tensor f = at::empty({1, T, mlp}, x.options());
@@ -571,13 +588,16 @@ PyObject *block_prefill(PyObject *const *a) {
           linear(f.data_ptr(), m2w.data_ptr(), ptr(m2b), m.data_ptr(), T, mlp, hid, 0, tag, -1, ws.data_ptr(), ws.numel(), stream) < 0)
         fail("linear: the GEMM could not be launched");
     } else {
-      m = at::linear(at::gelu(at::linear(h2, m1w, m1b)), m2w, m2b);
+      Tensor f = at::linear(h2, m1w, m1b);
+      f = at::gelu(f);
+      m = at::linear(f, m2w, m2b);
     }
+    h2.reset();
     y = at::add(sum, m);
     return EN_OK;
   };
-  (void)without_gil(run);
-  return tuple({y, kvq});
+  (void)without_gil(rest);
+  return THPVariable_Wrap(y);
 }
 
 // ---- module --------------------------------------------------------------------------------------------------------
@@ -610,7 +630,7 @@ PyMethodDef kMethods[] = {
     EN_FAST(layer, 19, "en_padding_removal_layer on new outputs"),
     EN_FAST(decode_layer, 10, "en_decode_layer on new outputs"),
     EN_FAST(plain_step, 9, "what block_decode takes of a block's modules, or None where the general step has to see them"),
-    EN_FAST(block_prefill, 26, "a pre-LN block over packed rows, its attention on the packed projections"),
+    EN_FAST(block_prefill, 27, "a pre-LN block over packed rows, its attention on the packed projections"),
     EN_FAST(block_decode, 25, "en_block_decode into a position of an output history"),
     {nullptr, nullptr, 0, nullptr}};
 

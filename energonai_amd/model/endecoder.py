@@ -83,7 +83,7 @@ class Block1D(nn.Module):
                                             m.get("norm2"), fc1, fc2)
 
     def _native_prefill(self, x, info: SeqInfo, batch_size: int, max_seq_len: int, fill_cache: bool) -> Optional[torch.Tensor]:
-        """The general form's ops on packed rows issued by one native call (``block_prefill``), the cache started behind them:
+        """The general form's ops on packed rows issued by one native call (``block_prefill``), the cache started among them:
         in Python two blocks of a short prompt are 400 us of host time for 100 on the GPU.  ``None``, with nothing done, where
         the block is not one of plain modules."""
         if self.apply_post_layernorm or x.dtype not in _NATIVE_TYPES or not x.is_cuda:
@@ -105,13 +105,12 @@ class Block1D(nn.Module):
         info = seq_info(info, batch_size, x.device)     # as the general form's attention asks for it: this batch, this stream
         table = None if info.ephemeral else info.tile_table(H, max_seq_len, 2 * max_seq_len * D * x.element_size(), causal=bool(attn.is_decoder))
         linear, workspace = (0, None) if mlp._epilogue is None else linear_entry(x.device)
-        out = _lib.front.block_prefill(x, *args, act, H, attn.scaling, attn.is_decoder, info.lens, info.cu_seqlens, table, batch_size,
-                                       max_seq_len, linear, workspace)
-        if out is None:
-            return None
+        start_cache = None
         if fill_cache:
-            attn._start_cache(None, None, out[1].view(-1, 3 * H, D), info, batch_size, max_seq_len)
-        return out[0]
+            def start_cache(kvq):
+                attn._start_cache(None, None, kvq.view(-1, 3 * H, D), info, batch_size, max_seq_len)
+        return _lib.front.block_prefill(x, *args, act, H, attn.scaling, attn.is_decoder, info.lens, info.cu_seqlens, table, batch_size,
+                                        max_seq_len, linear, workspace, start_cache)
 
     def _native_decode(self, hidden_states) -> Optional[torch.Tensor]:
         """One decode step of a pre-LN block of plain modules as ``en_block_decode``: five launches, the output written

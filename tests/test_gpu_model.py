@@ -189,6 +189,39 @@ def test_native_prefill_takes_the_lengths_that_the_general_form_takes(monkeypatc
     assert len(calls) == 3
 
 
+@pytest.mark.parametrize("activation", [torch.nn.functional.relu, torch.nn.GELU()])
+@pytest.mark.parametrize("fill", [True, False])
+def test_native_prefill_holds_no_more_memory_than_the_general_form(monkeypatch, activation, fill):
+    """Peaks of torch's allocator over one block, in bytes: a batch that fits the general form fits the native call."""
+    _, M = _mods()
+    from energonai_amd.seqinfo import seq_info
+    announce("native prefill, peak memory", activation, fill)
+    torch.manual_seed(7)
+    blk = M.Block1D(512, 8, 4.0, activation=activation, dtype=torch.float16, max_seq_len=512).cuda()
+    x = torch.randn(1, 2048, 512, device="cuda").half()
+    info = seq_info(torch.tensor([512] * 4, dtype=torch.int32).cuda(), 4, x.device)
+
+    def peak():
+        with torch.no_grad():
+            for _ in range(2):                      # the first pass makes what is kept: tables, the GEMMs' scratch
+                blk.attn.kv_cache = None
+                torch.cuda.synchronize()
+                torch.cuda.reset_peak_memory_stats()
+                before = torch.cuda.memory_allocated()
+                y = blk.forward_packed(x, info, 4, 512, fill)
+                torch.cuda.synchronize()
+                bytes_ = torch.cuda.max_memory_allocated() - before
+                assert y.shape == x.shape
+                del y
+        return bytes_
+
+    native = peak()
+    monkeypatch.setattr(M.Block1D, "_native_prefill", lambda *args: None)
+    general = peak()
+    announce("peak, rows of hidden", native / (2048 * 512 * 2), general / (2048 * 512 * 2))
+    assert native <= general
+
+
 @pytest.mark.parametrize("dtype,H,D,Smax,lens", [
     (torch.float16, 4, 64, 50, [7, 30, 1]), (torch.bfloat16, 3, 80, 129, [129, 0, 64, 65]), (torch.float32, 2, 64, 700, [700, 3]),
     (torch.float16, 3, 10, 20, [20, 5]),                 # rows of 20 bytes: no 16-byte pieces, two launches
