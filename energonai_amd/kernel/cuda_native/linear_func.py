@@ -25,7 +25,12 @@ _tuned: Dict[tuple, int] = {}
 
 
 def _workspace(device: torch.device) -> torch.Tensor:
-    """hipBLASLt scratch, one buffer per device from torch's allocator (the library never allocates)."""
+    """hipBLASLt scratch from torch's allocator (the library never allocates), for a GEMM on the current stream.  A solution
+    may keep partial sums in it, so GEMMs that can overlap must not share it: the default stream, whose order keeps its GEMMs
+    apart, has one buffer per device, and any other (a captured one among them) takes one for the call, which the allocator
+    hands out again to that stream alone."""
+    if torch._C._cuda_getCurrentRawStream(device.index) != 0:
+        return torch.empty(_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
     ws = _workspaces.get(device.index)
     if ws is None:
         ws = torch.empty(_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
@@ -34,7 +39,7 @@ def _workspace(device: torch.device) -> torch.Tensor:
 
 
 def linear_entry(device: torch.device):
-    """Address of ``en_linear`` and the workspace it is handed, for native callers."""
+    """Address of ``en_linear`` and the workspace it is handed, for native callers on the current stream."""
     global _entry
     if _entry is None:
         _entry = ctypes.cast(_lib.load_linear().en_linear, ctypes.c_void_p).value

@@ -485,6 +485,26 @@ def test_one_launch_rule(batch, heads, seq, D, total, dtype, pays):
     assert _lib.fn.en_attn_fused_norm_pays(batch, heads, seq, D, total, dtype) == pays
 
 
+def test_gemm_scratch_is_not_shared_between_streams(monkeypatch):
+    """What a GEMM keeps in its scratch is safe from GEMMs of other streams: the default stream has a buffer of its own, every other
+    call one that lives no longer than the call."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from energonai_amd.kernel.cuda_native import linear_func
+    stream, device = [0], torch.device("cuda", 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: stream[0], raising=False)
+    monkeypatch.setattr(linear_func, "_workspaces", {})
+    with FakeTensorMode():
+        stream[0] = 7                       # also the first call of all
+        first = linear_func._workspace(device)
+        stream[0] = 0
+        default = linear_func._workspace(device)
+        assert linear_func._workspace(device) is default and default is not first
+        stream[0] = 7
+        again, (_, native) = linear_func._workspace(device), linear_func.linear_entry(device)
+        assert len({id(t) for t in (first, default, again, native)}) == 4
+        assert {t.numel() for t in (first, default, native)} == {64 << 20} and list(linear_func._workspaces.values()) == [default]
+
+
 @pytest.mark.parametrize("units,unit_kv_bytes,causal,first", [
     (1, 1, True, True), (1, 1, False, False), (384, 256 << 10, True, True), (385, 256 << 10, True, False),   # 96 MB of K and V
     (256, 640 << 10, True, True), (257, 640 << 10, True, False), (256, (640 << 10) + 1, True, False),         # 160 MB in few units

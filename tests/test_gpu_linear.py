@@ -86,3 +86,25 @@ def test_auto_algo_is_searched_once_per_problem_and_gives_the_same_product():
     assert len(lf._tuned) == 2
     with pytest.raises(RuntimeError):
         lf.linear(x, w, "fastest")
+
+
+def test_gemms_on_several_streams_at_once():
+    """Short, deep products (the kind that is split over k and summed in the scratch) on four streams beside each other."""
+    lf = _lf()
+    announce("linear, several streams")
+    g = torch.Generator().manual_seed(45)
+    streams = [torch.cuda.default_stream()] + [torch.cuda.Stream() for _ in range(3)]
+    ops = [[(torch.randn(n, generator=g) / 64).half().cuda().view(shape) for n, shape in ((16 * 4096, (1, 16, 4096)), (256 * 4096, (256, 4096)))]
+           for _ in streams]
+    want = [lf.linear(x, w) for x, w in ops]
+    torch.cuda.synchronize()
+    scratch, got = set(), [[] for _ in streams]
+    for _ in range(20):
+        for s, (x, w), out in zip(streams, ops, got):
+            with torch.cuda.stream(s):
+                out.append(lf.linear(x, w))
+                scratch.add((s.cuda_stream, lf._workspace(x.device).data_ptr()))
+    torch.cuda.synchronize()
+    for w, out in zip(want, got):
+        assert all(torch.equal(y, w) for y in out)
+    assert len({p for _, p in scratch}) == len(scratch) >= len(streams)      # no buffer on two streams
