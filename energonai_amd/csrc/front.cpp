@@ -266,26 +266,46 @@ PyObject *layer(PyObject *const *a) {
   return THPVariable_Wrap(y);
 }
 
-// The words of en_decode_layer_norm for launches on torch's current stream of a device, 16 KB a stream, or null.  They belong to
-// the stream: its order keeps launches apart that share them, and torch's own streams (a fixed pool a device, which bounds this) live
-// as long as the process.  An external stream's handle may come back as another stream's while the first one's work still runs,
-// so it gets none; nor does a capture, whose launches may run again beside others.
-uint32_t *decode_words(const Tensor &t) {
-  static std::map<std::pair<int, hipStream_t>, Tensor> &pool = *new std::map<std::pair<int, hipStream_t>, Tensor>;     // under the interpreter lock
+// The words of en_decode_layer_norm for a launch on torch's current stream of a device, or null.  They belong to the stream: its
+// order keeps launches apart that share them, and torch's own streams (a fixed pool a device, which bounds this) live as long as the
+// process.  An external stream's handle may come back as another stream's while the first one's work still runs, so it gets none;
+// nor does a capture, whose launches may run again beside others.  A launch whose lengths are changed under it may leave its words
+// off zero, and they are to spoil no later step: launches take turns on 64 sets, 1 MB a stream, all cleared before the first is taken
+// again (2 us every 64 launches).  Counting every workgroup, so that lengths do not matter, costs 10 ns for each share without keys: 1
+// sequence x 16 heads x 64, up to 100 keys in caches of 16000, 5.6 -> 10.7 us a layer.
+constexpr int kWordSets = 64;
+struct WordSets {
+  Tensor sets;
+  int next = kWordSets;
+};
+uint32_t *next_decode_words(const Tensor &t) {
+  static std::map<std::pair<int, hipStream_t>, WordSets> &pool = *new std::map<std::pair<int, hipStream_t>, WordSets>;   // under the interpreter lock
   const auto stream = c10::hip::getCurrentHIPStream(t.device().index());
   if (stream.id() != 0 && stream.id() == (c10::StreamId) reinterpret_cast<intptr_t>(stream.stream())) return nullptr;   // external
-  const auto key = std::make_pair((int)t.device().index(), stream.stream());
-  auto at = pool.find(key);
-  if (at == pool.end()) {
+  WordSets &w = pool[std::make_pair((int)t.device().index(), stream.stream())];
+  const int64_t words = en_decode_layer_norm_words();
+  if (w.next == kWordSets) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream.stream(), &capture) != hipSuccess) {
       (void)hipGetLastError();
       return nullptr;
     }
     if (capture != hipStreamCaptureStatusNone) return nullptr;
-    at = pool.emplace(key, at::zeros({en_decode_layer_norm_words()}, t.options().dtype(at::kInt))).first;
+    if (!w.sets.defined()) w.sets = at::empty({kWordSets, words}, t.options().dtype(at::kInt));
+    if (hipMemsetAsync(w.sets.data_ptr(), 0, (size_t)w.sets.nbytes(), stream.stream()) != hipSuccess) fail("decode_layer: hipMemsetAsync failed");
+    w.next = 0;
   }
-  return reinterpret_cast<uint32_t *>(at->second.data_ptr<int32_t>());
+  return reinterpret_cast<uint32_t *>(w.sets.data_ptr<int32_t>()) + words * w.next++;
+}
+
+// decode_words(tensor) -> address of the words that the next decode layer on the tensor's device and current stream would take, a
+// turn of theirs, or None
+PyObject *decode_words(PyObject *const *a) {
+  const Tensor &t = gpu(a[0], "tensor", false);
+  const c10::DeviceGuard guard(t.device());
+  uint32_t *words = next_decode_words(t);
+  if (!words) Py_RETURN_NONE;
+  return PyLong_FromVoidPtr(words);
 }
 
 // decode_layer(q, k_cache, v_cache, lens, residual, gamma, beta, dense_out, eps, scale) -> y
@@ -334,7 +354,7 @@ PyObject *decode_layer(PyObject *const *a) {
   const int32_t *lens_p = i32(lens);
   const hipStream_t stream = stream_of(k);
   // small enough: one launch
-  uint32_t *words = !dense_p && tag == out_tag && B * H < 512 ? decode_words(k) : nullptr;
+  uint32_t *words = !dense_p && tag == out_tag && B * H < 512 ? next_decode_words(k) : nullptr;
   if (words) {
     const int rc = without_gil([&] {
       return en_decode_layer_norm(q_p, k_p, v_p, ctx_p, lens_p, (int)B, (int)H, (int)S, (int)D, ks, vs, scale, res_p, gamma_p, beta_p, y_p,
@@ -628,6 +648,7 @@ PyMethodDef kMethods[] = {
     EN_FAST(prefix_sum, 2, "(cu_seqlens, lens) of a batch"),
     EN_FAST(layer_tables, 8, "(row offsets, tile table, meeting words) of a batch"),
     EN_FAST(layer, 19, "en_padding_removal_layer on new outputs"),
+    EN_FAST(decode_words, 1, "address of the meeting words of a decode layer on the current stream, or None"),
     EN_FAST(decode_layer, 10, "en_decode_layer on new outputs"),
     EN_FAST(plain_step, 9, "what block_decode takes of a block's modules, or None where the general step has to see them"),
     EN_FAST(block_prefill, 27, "a pre-LN block over packed rows, its attention on the packed projections"),

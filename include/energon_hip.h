@@ -279,9 +279,10 @@ int en_decode_layer(const void *q, const void *k_cache, const void *v_cache, voi
 
 /* en_decode_layer without a projection in between, out_dtype == dtype, in one launch for batches of few units (fewer than 512
  * (sequence, head) pairs): the last workgroup of a sequence normalises its row.  words: en_decode_layer_norm_words() uint32,
- * zero before the first launch that uses them and after every one; launches that may overlap must not share them.  workspace
- * as in en_decode_layer; ctx is written only where no keys are shared.  Captured streams, overlapping buffers, wider rows and other head
- * sizes return EN_ERR_UNSUPPORTED with nothing launched: en_decode_layer takes those. */
+ * zero before the first launch that uses them and after every one (but clear them behind a launch whose kv_lens were changed
+ * under it); launches that may overlap must not share them.  workspace as in en_decode_layer; ctx is written only where no keys
+ * are shared.  Captured streams, overlapping buffers, wider rows and other head sizes return EN_ERR_UNSUPPORTED with nothing
+ * launched: en_decode_layer takes those. */
 int64_t en_decode_layer_norm_words(void);
 int en_decode_layer_norm(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens, int batch,
                          int head_num, int k_seq_len, int size_per_head, const int64_t *k_strides, const int64_t *v_strides,

@@ -526,6 +526,31 @@ def test_decode_layer_in_one_launch(dtype, B, H, S, D):
                                         _lib.stream_of(args[0])) == -5
 
 
+def test_decode_layer_is_spoilt_by_one_launch_only():
+    """Lengths that change under a launch may leave its words off zero (here they are set so): no later step meets them."""
+    from energonai_amd import _lib, layer
+    from energonai_amd.seqinfo import SeqInfo
+    announce("decode layer, words off zero")
+    B, H, S, D = 3, 4, 300, 64
+    g = torch.Generator(device="cuda").manual_seed(8)
+    q, kc, vc = (torch.randn(B, H, n, D, generator=g, device="cuda").half() for n in (1, S, S))
+    res, gamma, beta = (torch.randn(n, H * D, generator=g, device="cuda").half() for n in (B, 1, 1))
+    lens = torch.tensor([300, 0, 17], dtype=torch.int32, device="cuda")
+    a = (q, kc, vc, SeqInfo(lens, None, B, None, lens), res.view(1, B, H * D), gamma[0], beta[0])
+    want = layer.decode_layer(*a)
+    bad = torch.full((_lib.fn.en_decode_layer_norm_words(),), 1000, dtype=torch.int32, device="cuda")     # nobody would be the last
+
+    def step():
+        # outputs and scratch of the call are allocated where these were: what nobody writes is NaN
+        del [torch.full((B * H * D,), float("nan"), dtype=torch.float16, device="cuda") for _ in range(8)][:]
+        return layer.decode_layer(*a)
+
+    for _ in range(3):
+        words = _lib.front.decode_words(kc)
+        assert _lib.fn.en_copy_bytes(bad.data_ptr(), words, bad.numel() * 4, _lib.stream_of(kc)) == 0
+        assert all(torch.equal(step(), want) for _ in range(70))
+
+
 def test_decode_layer_words_belong_to_their_stream():
     """Steps on several streams at once, and one in a graph beside them, each give what a step alone gives."""
     from energonai_amd import layer
