@@ -64,6 +64,7 @@ SIGNATURES = {
     "en_decode_layer": (c_int, [c_void_p] * 5 + [c_int] * 4 + [c_void_p, c_void_p, c_float] + [c_void_p] * 5 +
                         [c_int64, c_float, c_int, c_int, c_void_p, c_int64, c_void_p]),
     "en_decode_layer_norm_words": (c_int64, []),
+    "en_decode_layer_norm_pays": (c_int, [c_int] * 5),
     "en_decode_layer_norm": (c_int, [c_void_p] * 5 + [c_int] * 4 + [c_void_p, c_void_p, c_float] + [c_void_p] * 4 +
                              [c_float, c_int, c_void_p, c_int64, c_void_p, c_void_p]),
     "en_decode_attn_workspace_bytes": (c_int64, [c_int] * 4),

@@ -821,19 +821,25 @@ static void launch_attn_norm(const DecodeAttnArgs &a, const DecodeTail &tail, di
   else decode_attn_norm_kernel<DT, LPK, NT, U, false><<<grid, NT, 0, s>>>(args, tail);
 }
 
-// The forms of attn_form below 512 units, for heads of 33..128 channels (fp32: 17..128).  From 512 units on the attention is several
-// times what the second launch costs.
-template <int DT, int LPK>
-static int launch_attn_norm_form(const DecodeAttnArgs &a, const DecodeTail &tail, dim3 grid, bool stream_cache, hipStream_t s) {
-  const AttnForm form = attn_form(a, LPK);
-  const int lanes = form == AttnForm::kPair ? 512 : 256;
+// Whether a decode layer is one launch: the forms of attn_form below 512 units, for heads of 33..128 channels (fp32: 17..128).  From
+// 512 units on the attention is several times what the second launch costs.
+static bool one_launch_takes(const DecodeAttnArgs &a, int elem_size) {
+  const int epv = 16 / elem_size;
+  if (a.B > kRankBatch || (int64_t)a.B * a.H >= 512 || a.D % epv || a.D <= 4 * epv || a.D > 128) return false;
+  int lpk = 8;
+  while (lpk * epv < a.D) lpk *= 2;
+  const int64_t hidden = (int64_t)a.H * a.D, lanes = attn_form(a, lpk) == AttnForm::kPair ? 512 : 256;
   // One workgroup has the whole row to read.  us a layer, two launches / one: 1 x 12 heads x 64, up to 300 keys 8.5 / 6.3, 8 x 12 x 64
   // 8.4 / 6.9, 2 x 8 x 64 fp32, up to 800 9.2 / 8.0, 16 x 24 x 64, up to 900 15.0 / 14.7, 16 x 32 x 128, up to 128 10.1 / 10.1; of five
   // vectors a lane, 2 x 60 x 128, up to 500 10.3 / 10.7, 5 x 72 x 128 35.8 / 36.8.  Rows of shares are four channels a lane, sixteen
   // bytes from each share: 1 x 5 x 64, 4000 keys 9.3 / 8.6, 10 x 16 x 64, up to 2000 15.2 / 14.2; combined unit by unit in front of
   // the row, which takes wider ones, 6 x 64 x 128 41.9 / 43.9.
-  if (a.nsplit > 1 ? tail.hidden > 4 * lanes : tail.hidden * Elem<DT>::kSize > kTailVectors * 16 * lanes) return EN_ERR_UNSUPPORTED;
-  switch (form) {
+  return a.nsplit > 1 ? hidden <= 4 * lanes : hidden * elem_size <= kTailVectors * 16 * lanes;
+}
+
+template <int DT, int LPK>
+static int launch_attn_norm_form(const DecodeAttnArgs &a, const DecodeTail &tail, dim3 grid, bool stream_cache, hipStream_t s) {
+  switch (attn_form(a, LPK)) {
     case AttnForm::kTiny: launch_attn_norm<DT, LPK, 256, 1>(a, tail, grid, stream_cache, s); break;
     case AttnForm::kSmall: launch_attn_norm<DT, LPK, 256, 2>(a, tail, grid, stream_cache, s); break;
     case AttnForm::kPair: launch_attn_norm<DT, LPK, 512, 2>(a, tail, grid, stream_cache, s); break;
@@ -848,12 +854,10 @@ template <int DT>
 static int dispatch_attn_norm(const DecodeAttnArgs &a, const DecodeTail &tail, bool stream_cache, hipStream_t s) {
   constexpr int EPV = 16 / Elem<DT>::kSize;
   const dim3 grid((unsigned)a.H, (unsigned)a.B, (unsigned)a.nsplit);
-  if (a.D > 128) return EN_ERR_UNSUPPORTED;
   if constexpr (DT == EN_F32)
     if (a.D > 16 * EPV) return launch_attn_norm_form<DT, 32>(a, tail, grid, stream_cache, s);
   if (a.D > 8 * EPV) return launch_attn_norm_form<DT, 16>(a, tail, grid, stream_cache, s);
-  if (a.D > 4 * EPV) return launch_attn_norm_form<DT, 8>(a, tail, grid, stream_cache, s);
-  return EN_ERR_UNSUPPORTED;
+  return launch_attn_norm_form<DT, 8>(a, tail, grid, stream_cache, s);
 }
 
 // How many workgroups share one unit's keys: none while the units alone fill the chip (512 units and more); else
@@ -1152,6 +1156,15 @@ int en_decode_layer(const void *q, const void *k_cache, const void *v_cache, voi
   }
 }
 
+int en_decode_layer_norm_pays(int batch, int head_num, int k_seq_len, int size_per_head, int dtype) {
+  using namespace en;
+  const int es = dtype_size(dtype);
+  if (!es || batch < 1 || head_num < 1 || k_seq_len < 1 || size_per_head < 1) return 0;
+  DecodeAttnArgs a{};
+  a.B = batch, a.H = head_num, a.Sk = k_seq_len, a.D = size_per_head, a.nsplit = decode_split(batch, head_num, k_seq_len);
+  return one_launch_takes(a, es);
+}
+
 int64_t en_decode_layer_norm_words(void) { return (int64_t)en::kRankBatch * en::kTailWordStride; }
 
 int en_decode_layer_norm(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens, int batch,
@@ -1165,7 +1178,7 @@ int en_decode_layer_norm(const void *q, const void *k_cache, const void *v_cache
                            scale, dtype, workspace, workspace_bytes);
   if (rc) return rc;
   const int64_t es = dtype_size(dtype), hidden = (int64_t)head_num * size_per_head, rows = batch * hidden * es, S = k_seq_len;
-  if (batch > kRankBatch || (int64_t)batch * head_num >= 512 || size_per_head % (16 / es)) return EN_ERR_UNSUPPORTED;
+  if (!one_launch_takes(a, (int)es)) return EN_ERR_UNSUPPORTED;
   for (const void *p : {(const void *)ctx, residual, gamma, beta, (const void *)y})
     if (!aligned_to(p, 16)) return EN_ERR_UNSUPPORTED;
   if (!aligned_to(words, 4) || (a.nsplit > 1 && !aligned_to(workspace, 16))) return EN_ERR_UNSUPPORTED;

@@ -354,7 +354,7 @@ PyObject *decode_layer(PyObject *const *a) {
   const int32_t *lens_p = i32(lens);
   const hipStream_t stream = stream_of(k);
   // small enough: one launch
-  uint32_t *words = !dense_p && tag == out_tag && B * H < 512 ? next_decode_words(k) : nullptr;
+  uint32_t *words = !dense_p && tag == out_tag && en_decode_layer_norm_pays((int)B, (int)H, (int)S, (int)D, tag) ? next_decode_words(k) : nullptr;
   if (words) {
     const int rc = without_gil([&] {
       return en_decode_layer_norm(q_p, k_p, v_p, ctx_p, lens_p, (int)B, (int)H, (int)S, (int)D, ks, vs, scale, res_p, gamma_p, beta_p, y_p,

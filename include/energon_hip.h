@@ -284,6 +284,9 @@ int en_decode_layer(const void *q, const void *k_cache, const void *v_cache, voi
  * are shared.  Captured streams, overlapping buffers, wider rows and other head sizes return EN_ERR_UNSUPPORTED with nothing
  * launched: en_decode_layer takes those. */
 int64_t en_decode_layer_norm_words(void);
+/* Whether en_decode_layer_norm takes a layer of these sizes (in a workspace of en_decode_attn_workspace_bytes): a caller asks
+ * before it looks words up. */
+int en_decode_layer_norm_pays(int batch, int head_num, int k_seq_len, int size_per_head, int dtype);
 int en_decode_layer_norm(const void *q, const void *k_cache, const void *v_cache, void *ctx, const int32_t *kv_lens, int batch,
                          int head_num, int k_seq_len, int size_per_head, const int64_t *k_strides, const int64_t *v_strides,
                          float scale, const void *residual, const void *gamma, const void *beta, void *y, float eps, int dtype,

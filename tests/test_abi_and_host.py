@@ -485,6 +485,22 @@ def test_one_launch_rule(batch, heads, seq, D, total, dtype, pays):
     assert _lib.fn.en_attn_fused_norm_pays(batch, heads, seq, D, total, dtype) == pays
 
 
+@pytest.mark.parametrize("batch,heads,seq,D,dtype,pays", [
+    (1, 12, 300, 64, 1, 1), (1, 72, 2048, 128, 1, 0),             # a shared row of 9216 channels is no single workgroup's
+    (2, 16, 1100, 128, 2, 1), (2, 17, 1100, 128, 2, 0),           # shared, 512 lanes: 2048 channels
+    (30, 16, 1500, 64, 1, 1), (30, 17, 1500, 64, 1, 0),           # shared, 256 lanes: 1024 channels
+    (15, 32, 250, 128, 1, 1), (2, 33, 250, 128, 1, 0), (15, 32, 250, 128, 0, 0), (31, 16, 250, 128, 0, 1),    # 8 KB of a row
+    (127, 4, 64, 64, 1, 1), (128, 4, 64, 64, 1, 0), (257, 1, 64, 64, 1, 0),      # 512 units, 256 sequences
+    (1, 4, 64, 32, 1, 0), (1, 4, 64, 40, 1, 1), (1, 4, 64, 32, 0, 1), (1, 4, 64, 136, 1, 0), (1, 4, 64, 60, 1, 0),
+    (0, 4, 64, 64, 1, 0), (1, 4, 0, 64, 1, 0), (1, 4, 64, 64, 7, 0),
+])
+def test_decode_one_launch_rule(batch, heads, seq, D, dtype, pays):
+    """Where a decode layer is one launch: the one rule that the entry point and the step in front of it follow, so that a layer which
+    is none pays for no words and no refused call."""
+    from energonai_amd import _lib
+    assert _lib.fn.en_decode_layer_norm_pays(batch, heads, seq, D, dtype) == pays
+
+
 def test_gemm_scratch_is_not_shared_between_streams(monkeypatch):
     """What a GEMM keeps in its scratch is safe from GEMMs of other streams: the default stream has a buffer of its own, every other
     call one that lives no longer than the call."""

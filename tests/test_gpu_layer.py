@@ -551,6 +551,19 @@ def test_decode_layer_is_spoilt_by_one_launch_only():
         assert all(torch.equal(step(), want) for _ in range(70))
 
 
+@pytest.mark.parametrize("H,S,D,turns", [(72, 2048, 128, 1), (4, 300, 64, 2)])
+def test_only_a_decode_layer_of_one_launch_takes_words(H, S, D, turns):
+    """A row too wide for one launch is known by its sizes, before words are looked up and a call is refused."""
+    from energonai_amd import _lib, layer
+    announce("decode layer, words", H, S, D)
+    q, kc, vc = (torch.zeros(1, H, n, D, dtype=torch.float16, device="cuda") for n in (1, S, S))
+    row, lens = torch.zeros(1, 1, H * D, dtype=torch.float16, device="cuda"), torch.tensor([S], dtype=torch.int32, device="cuda")
+    first = _lib.front.decode_words(kc)
+    layer.decode_layer(q, kc, vc, lens, row, row[0, 0], row[0, 0])
+    size = 4 * _lib.fn.en_decode_layer_norm_words()
+    assert (_lib.front.decode_words(kc) - first) % (64 * size) == turns * size
+
+
 def test_decode_layer_words_belong_to_their_stream():
     """Steps on several streams at once, and one in a graph beside them, each give what a step alone gives."""
     from energonai_amd import layer
