@@ -17,9 +17,10 @@ the OPT-30B-shaped layer: the largest of the five that fits one GPU -- 1.9 GB of
 scores, 45 GFLOP per contraction -- and the one whose kernels are bound by HBM
 bandwidth rather than by launch cost); the other workloads, the per-kernel
 bandwidths, the PyTorch-ROCm eager pipeline and the CPU oracle are reported beside
-it in the same JSON line.
+it: as one JSON line on stderr, behind "details ", and in the file named by --details.
 
-The line also carries
+Standard output is one JSON line of under 2000 characters (a reader that keeps the end of a
+log keeps all of it) with the headline and
   roofline      achieved vs peak for the kernel that takes the largest share of the step,
                 from algorithmic bytes (or FLOPs) per launch and the kernel's launch-to-launch
                 time measured with events on the launch stream;
@@ -951,6 +952,15 @@ def roofline_of(res, workload_name, form="default"):
     return roofline
 
 
+HEADLINE = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling", "vs_baseline",
+            "dtype", "data", "library_source_hash", "config", "step_form", "roofline", "cpu_baseline")
+
+
+def headline(out: dict) -> str:
+    """The line on standard output: the headline, its roofline and the CPU baseline of everything measured."""
+    return json.dumps({k: out[k] for k in HEADLINE})
+
+
 def main(argv=None) -> int:
     ap = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
     ap.add_argument("--gpus", type=int, default=1)
@@ -961,6 +971,7 @@ def main(argv=None) -> int:
                     help="the step that is timed: the product's default form, or QK^T / softmax / PV as three kernels")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--no-extra", action="store_true", help="only the headline workload, no eager / other workloads")
+    ap.add_argument("--details", metavar="FILE", help="write everything measured to FILE as JSON as well")
     ap.add_argument("--step-only", action="store_true",
                     help="with --no-extra: launch nothing but the step and its own kernels (for profiles)")
     ap.add_argument("--copy-yardstick", action="store_true",
@@ -1072,7 +1083,11 @@ def main(argv=None) -> int:
                         out["cpu_baselines"][ow.name] = {"error": str(exc)[:300]}
     else:
         out["cpu_baseline"] = None
-    print(json.dumps(out))
+    if ns.details:
+        with open(ns.details, "w") as f:
+            json.dump(out, f)
+    print("details " + json.dumps(out), file=sys.stderr, flush=True)
+    print(headline(out), flush=True)
     return 0
 
 

@@ -69,6 +69,10 @@ def run_profiler(tag: str, prof_args, bench_args, timeout_s: int, script: str = 
     os.makedirs(d, exist_ok=True)
     cmd = ["rocprofv3"] + prof_args + ["--output-format", "csv", "-d", d, "-o", "run", "--",
                                       "python3", os.path.join(ROOT, script)] + bench_args
+    details = os.path.join(d, "details.json")
+    shown = " ".join(cmd[:1] + prof_args + ["--", "python3", "bench.py"] + bench_args)
+    if script == "bench.py":
+        cmd += ["--details", details]
     env = dict(os.environ, TMPDIR="/tmp")
     print("[bench_profiles] " + " ".join(cmd), file=sys.stderr, flush=True)
     proc = subprocess.run(cmd, cwd=ROOT, env=env, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True,
@@ -80,7 +84,10 @@ def run_profiler(tag: str, prof_args, bench_args, timeout_s: int, script: str = 
     for ln in proc.stdout.splitlines():
         if ln.startswith("{"):
             line = json.loads(ln)
-    return d, line, " ".join(cmd[:1] + prof_args + ["--", "python3", "bench.py"] + bench_args)
+    if os.path.exists(details):
+        with open(details) as f:
+            line = json.load(f)
+    return d, line, shown
 
 
 def print_sources(line) -> None:

@@ -230,6 +230,31 @@ def test_public_attention_calls_pass_the_tile_table_when_there_are_no_query_leng
     assert attention._tile_table_ptr(info, 0x7f0000001000, 12, 512, 1 << 17) is None and len(info.asked) == 2
 
 
+def test_bench_prints_one_short_line_whatever_it_measured():
+    """Standard output carries the keys that a reader of the benchmark needs in a line of under 2000 characters; tables of kernels and
+    other workloads go elsewhere."""
+    import json
+
+    import bench
+    from energonai_amd import workloads
+    w = workloads.BY_NAME["c3"]
+    number = 12345678.901234567
+    row = dict.fromkeys(("us", "alg_MB", "GBps", "hbm_frac", "TFLOPs", "mfma_frac"), number)
+    roofline = bench.roofline_of({"step_kernels": {"attn_fused_packed": row}, "dtype": "f16"}, w.name)
+    cpu = {"value": number, "unit": "tokens/s", "cores": 16, "kind": "port", "host_cpu_count": 256, "cpu_model": "AMD EPYC 9575F 64-Core",
+           "sample": "s" * 320}
+    out = {"metric": "per_layer_tokens_per_s", "value": number, "unit": "tokens/s", "n_gpus": 1, "steps": 50, "warmup": 10,
+           "ms_per_step": number, "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f16", "data": "synthetic",
+           "library_source_hash": "0" * 32, "config": {"workload": w.title + "x" * 120}, "step_form": "packed", "roofline": roofline,
+           "cpu_baseline": cpu, "kernels": {f"kernel {i}": row for i in range(200)}, "workloads": {"c4": {"kernels": [row] * 50}}}
+    line = bench.headline(out)
+    assert "\n" not in line and len(line) < 2000
+    parsed = json.loads(line)
+    assert {"metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling", "vs_baseline", "dtype",
+            "data", "config", "roofline", "cpu_baseline"} <= set(parsed)
+    assert all(parsed[k] == out[k] for k in parsed)
+
+
 def test_missing_library_fails_loudly(tmp_path, monkeypatch):
     """No CPU fallback: without the shared object the product refuses to load."""
     from energonai_amd import _lib
