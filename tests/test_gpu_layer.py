@@ -519,7 +519,7 @@ def test_decode_layer_in_one_launch(dtype, B, H, S, D):
     _, _, ctx = eager.decode_attention(q, kc, vc, kv, D ** -0.5, acc_dtype=torch.float64)
     want = torch.nn.functional.layer_norm(ctx.view(1, B, H * D) + res.double(), (H * D,), gamma.double(), beta.double(), 1e-5)
     assert_stored_close(out[0].cpu(), want, dtype)
-    # rows that the call's own output overlaps, and a capture, are for the two launches
+    # rows that the call's own output overlaps are for the two launches
     assert _lib.fn.en_decode_layer_norm(args[0].data_ptr(), args[1].data_ptr(), args[2].data_ptr(), out[0].data_ptr(), lens.data_ptr(), B, H, S,
                                         D, strides, strides, D ** -0.5, args[3].data_ptr(), args[4].data_ptr(), args[5].data_ptr(),
                                         out[0].data_ptr(), 1e-5, _lib.dtype_tag(q, "test"), ws.data_ptr(), need, words.data_ptr(),
@@ -565,32 +565,68 @@ def test_only_a_decode_layer_of_one_launch_takes_words(H, S, D, turns):
 
 
 def test_decode_layer_words_belong_to_their_stream():
-    """Steps on several streams at once, and one in a graph beside them, each give what a step alone gives."""
-    from energonai_amd import layer
+    """Steps of different operands that overlap on several streams, and one in a graph beside them, each give what a step alone gives.
+    No two streams have words in common; a stream of somebody else's and a capture have none and take two launches."""
+    from energonai_amd import _lib, layer
     from energonai_amd.seqinfo import SeqInfo
+    announce("decode layer, words of a stream")
     B, H, S, D = 2, 12, 1500, 64
     g = torch.Generator(device="cuda").manual_seed(5)
-    def rand(*shape):
-        return torch.randn(shape, generator=g, device="cuda", dtype=torch.float16)
-    lens = torch.tensor([1500, 700], dtype=torch.int32, device="cuda")
-    info = SeqInfo(lens, None, B, None, lens)
-    a = (rand(B, H, 1, D), rand(B, H, S, D), rand(B, H, S, D), info, rand(1, B, H * D), rand(H * D), rand(H * D))
-    want = layer.decode_layer(*a)
+
+    def operands(*kv):
+        def rand(*shape):
+            return torch.randn(shape, generator=g, device="cuda", dtype=torch.float16)
+        lens = torch.tensor(kv, dtype=torch.int32, device="cuda")
+        return (rand(B, H, 1, D), rand(B, H, S, D), rand(B, H, S, D), SeqInfo(lens, None, B, None, lens), rand(1, B, H * D), rand(H * D),
+                rand(H * D))
+
+    need = _lib.fn.en_decode_attn_workspace_bytes(B, H, S, D)
+    zeros, ws = torch.zeros(_lib.fn.en_decode_layer_norm_words(), dtype=torch.int32, device="cuda"), torch.zeros(need, dtype=torch.uint8, device="cuda")
+    strides = (ctypes.c_int64 * 3)(H * S * D, S * D, D)
+
+    def one_launch(a, ctx, y):
+        return _lib.fn.en_decode_layer_norm(a[0].data_ptr(), a[1].data_ptr(), a[2].data_ptr(), ctx.data_ptr(), a[3].lens.data_ptr(), B, H, S, D,
+                                            strides, strides, D ** -0.5, a[4].data_ptr(), a[5].data_ptr(), a[6].data_ptr(), y.data_ptr(), 1e-5,
+                                            _lib.dtype_tag(a[0], "test"), ws.data_ptr(), need, zeros.data_ptr(), _lib.stream_of(a[0]))
+
+    steps = [operands(*kv) for kv in ((1500, 700), (3, 1500), (1024, 1), (600, 0))]
+    ctx, y = torch.empty(B, H, 1, D, dtype=torch.float16, device="cuda"), torch.empty(1, B, H * D, dtype=torch.float16, device="cuda")
+    want = []
+    for a in steps:
+        want.append(layer.decode_layer(*a))
+        assert one_launch(a, ctx, y) == 0 and torch.equal(y, want[-1])
+    streams = [torch.cuda.default_stream()] + [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.ExternalStream(streams[1].cuda_stream)):
+        assert _lib.front.decode_words(steps[0][1]) is None
+        two_launches = layer.decode_layer(*steps[0])
+    words = []
+    for s in streams:
+        with torch.cuda.stream(s):
+            words.append({_lib.front.decode_words(steps[0][1]) for _ in range(128)})      # every set, whichever was next
+    assert [len(w) for w in words] == [64] * 4 and len(set().union(*words)) == 256
     graph = torch.cuda.CUDAGraph()
     torch.cuda.synchronize()
     with torch.cuda.graph(graph):
-        recorded = layer.decode_layer(*a)
-    streams = [torch.cuda.Stream() for _ in range(3)]
-    got = []
+        refused = one_launch(steps[0], ctx, y)
+        recorded = layer.decode_layer(*steps[0])
+    assert refused == -5
+    got = [[] for _ in streams]
     for _ in range(8):
-        graph.replay()
-        for s in streams:
+        recorded.fill_(float("nan"))
+        for s, a, out in zip(streams, steps, got):
             with torch.cuda.stream(s):
-                got.append(layer.decode_layer(*a))
-    torch.cuda.synchronize()
-    assert all(torch.equal(y, want) for y in got)
-    # the graph holds the two launches: combined and normalised in another order of summation
-    assert (recorded.float() - want.float()).abs().max() <= 2 ** -9 * want.float().abs().max()
+                torch.cuda._sleep(200_000)                       # all four are queued before the first runs
+                for n in (need, B * H * D * 2, B * H * D * 2):   # scratch and outputs are allocated where these were
+                    torch.full((n // 2,), float("nan"), dtype=torch.float16, device="cuda")
+                for _ in range(3):
+                    out.append(layer.decode_layer(*a))
+        graph.replay()
+        torch.cuda.synchronize()
+        # bit for bit the two launches, which add up in another order
+        assert torch.equal(recorded, two_launches)
+    for w, out in zip(want, got):
+        assert all(torch.equal(y, w) for y in out)
 
 
 @pytest.mark.parametrize("lens,S,H,left", [([1], 17, 1, False), ([64, 0, 300, 7, 128, 129], 300, 5, True),
