@@ -19,7 +19,7 @@ from ..kernel import (attn_fused_varlen, attn_pv, attn_qk, decode_attn, decode_p
 from ..kernel.attention import kv_cache_fill
 from ..seqinfo import SeqInfo, seq_info
 from .gemm import project
-from .kv_cache import KVCache, OutputHistory, PagedKVCache
+from .kv_cache import KVCache, OutputHistory, PagedKVCache, start_history
 
 
 def lens_from_mask(attention_mask: torch.Tensor) -> torch.Tensor:
@@ -140,7 +140,7 @@ class MultiHeadAttention1D(nn.Module):
         x = depad(hidden_states, B, info, left_padded=self.left_padded)
         y = self.forward_packed(x, info, B, S, fill_cache=not self.disable_past_cache)
         if not self.disable_past_cache:
-            return self._history.start_packed(y, B, S, info, self.left_padded, self.max_seq_len)
+            return start_history(self._history, y, B, S, info, self.left_padded, self.max_seq_len)
         return repad(y, B, S, info, left_padded=self.left_padded)
 
 

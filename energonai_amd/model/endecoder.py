@@ -20,7 +20,7 @@ from ..kernel.cuda_native.linear_func import linear_entry
 from ..seqinfo import SeqInfo, seq_info
 from .attention import MultiHeadAttention1D, lens_from_mask
 from .gemm import gemm_tuning
-from .kv_cache import KVCache, OutputHistory, PagedKVCache
+from .kv_cache import KVCache, OutputHistory, PagedKVCache, start_history
 from .mlp import MLP1D, activation_code
 
 
@@ -173,7 +173,7 @@ class Block1D(nn.Module):
         x = depad(hidden_states, B, info, left_padded=left)
         y = self.forward_packed(x, info, B, S, fill_cache=not self.disable_past_cache)
         if not self.disable_past_cache:
-            return self._history.start_packed(y, B, S, info, left, self.max_seq_len)
+            return start_history(self._history, y, B, S, info, left, self.max_seq_len)
         return repad(y, B, S, info, left_padded=left)
 
 

@@ -206,8 +206,6 @@ class OutputHistory:
 
     def start_packed(self, y: torch.Tensor, batch_size: int, max_seq_len: int, info: SeqInfo, left_padded: bool, planned: int) -> torch.Tensor:
         """``start(repad(y))`` without the copy: the padding is restored in the buffer itself."""
-        if type(self).start is not OutputHistory.start or "start" in self.__dict__:
-            return self.start(repad(y, batch_size, max_seq_len, info, left_padded=left_padded), planned)
         self.buf = repad(y, batch_size, max_seq_len, info, left_padded=left_padded,
                          out=torch.empty((batch_size, max(int(planned), max_seq_len), y.shape[-1]), dtype=y.dtype, device=y.device))
         self.cur = max_seq_len
@@ -229,3 +227,10 @@ class OutputHistory:
         self.buf[:, self.cur:self.cur + 1].copy_(new)
         self.cur += 1
         return self.buf[:, :self.cur]
+
+
+def start_history(history, y: torch.Tensor, batch_size: int, max_seq_len: int, info: SeqInfo, left_padded: bool, planned: int) -> torch.Tensor:
+    """``history.start`` with the padded form of packed rows ``y``; any object with ``start`` and ``push`` will do."""
+    if type(history) is not OutputHistory or "start" in history.__dict__:
+        return history.start(repad(y, batch_size, max_seq_len, info, left_padded=left_padded), planned)
+    return history.start_packed(y, batch_size, max_seq_len, info, left_padded, planned)

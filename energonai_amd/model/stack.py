@@ -13,6 +13,7 @@ from ..kernel import depad, repad
 from ..seqinfo import seq_info
 from .attention import lens_from_mask
 from .endecoder import Block1D
+from .kv_cache import start_history
 
 
 class PackedStack(nn.Module):
@@ -42,7 +43,7 @@ class PackedStack(nn.Module):
         for blk in self.blocks:
             x = blk.forward_packed(x, info, B, S, fill_cache=caching)
             if caching:   # each block keeps its own padded output for the later steps, as the reference blocks do
-                blk._history.start_packed(x, B, S, info, left, blk.max_seq_len)
+                start_history(blk._history, x, B, S, info, left, blk.max_seq_len)
         if self.norm is not None:
             x = self.norm(x)
         return repad(x, B, S, info, left_padded=left)

@@ -263,6 +263,38 @@ def test_a_cache_that_could_not_be_filled_is_not_kept(monkeypatch, page):
         assert attn.kv_cache is before
 
 
+class DuckHistory:
+    """Only what a module asks of a history."""
+    __slots__ = ("got",)
+
+    def start(self, out, max_seq_len):
+        self.got = (out, max_seq_len)
+        return out
+
+    def push(self, new):
+        return new
+
+
+class StartsByItself(OutputHistory):
+    def start(self, out, max_seq_len):
+        self.got = (out, max_seq_len)
+        return out
+
+
+def test_a_history_of_the_callers_own_is_started_with_padded_rows(monkeypatch):
+    """Whatever has ``start`` and ``push``; the package's own takes the packed rows."""
+    from energonai_amd.model import attention, endecoder, kv_cache, stack
+    assert attention.start_history is endecoder.start_history is stack.start_history is kv_cache.start_history
+    packed, padded = torch.ones(1, 8, 128), torch.zeros(2, 8, 128)
+    monkeypatch.setattr(kv_cache, "repad", lambda y, *args, out=None, **kwargs: padded if out is None else out)
+    on_instance = OutputHistory()
+    on_instance.start = lambda out, max_seq_len: setattr(on_instance, "got", (out, max_seq_len)) or out
+    for history in (DuckHistory(), StartsByItself(), on_instance):
+        assert kv_cache.start_history(history, packed, 2, 8, None, False, 32) is padded and history.got == (padded, 32)
+    own = OutputHistory()
+    assert kv_cache.start_history(own, packed, 2, 8, None, False, 32).shape == (2, 8, 128) and own.buf.shape == (2, 32, 128) and own.cur == 8
+
+
 def test_a_cache_saved_before_it_could_be_unzeroed_is_filled(monkeypatch):
     """A pickled cache of that time has zeros in its buffers and says nothing about them."""
     from energonai_amd.model import kv_cache
