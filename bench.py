@@ -807,7 +807,48 @@ def decode_sizes(torch, iters):
                 row[name] = {"us": us, "GBps": nbytes / us / 1e3}
             rows.append(row)
             del kc, vc, k_pool, v_pool
-    return {"heads": H, "size_per_head": D, "page": P, "dtype": "f16", "rows": rows}
+    return {"heads": H, "size_per_head": D, "page": P, "dtype": "f16", "rows": rows, "layers": decode_layers(torch, iters)}
+
+
+def decode_layers(torch, iters):
+    """Decode layers (attention, residual, LayerNorm) of few units: as called, one launch where the rows allow it, and as two launches
+    (a stream that is not torch's own has no meeting words).  Eight layers' operands in turn, with the calls queued ahead of the GPU
+    and with the host in step, as a decode loop has it."""
+    from energonai_amd import _lib, layer
+    from energonai_amd.seqinfo import SeqInfo
+    two_launches = torch.cuda.ExternalStream(torch.cuda.Stream().cuda_stream)
+    rows = []
+    for B, H, D, S, top in ((1, 12, 64, 300, 300), (8, 12, 64, 300, 300), (16, 24, 64, 900, 900), (1, 5, 64, 4000, 4000), (10, 16, 64, 2000, 2000),
+                            (10, 16, 64, 4000, 100), (1, 72, 128, 2048, 2048)):
+        g = torch.Generator(device="cuda").manual_seed(S)
+        lens = torch.randint(1, top + 1, (B,), generator=g, device="cuda", dtype=torch.int32)
+        info = SeqInfo(lens, None, B, None, lens)
+        shapes = ((B, H, 1, D), (B, H, S, D), (B, H, S, D), (1, B, H * D), (H * D,), (H * D,))
+        sets = [[torch.randn(s, generator=g, device="cuda").half() for s in shapes] for _ in range(8)]
+        torch.cuda.synchronize()
+
+        def us(stream, ahead):
+            times = []
+            with torch.cuda.stream(stream):
+                for _ in range(max(5, iters) + 3):
+                    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                    if ahead:
+                        torch.cuda._sleep(5_000_000)
+                    start.record()
+                    for _ in range(4):
+                        for q, k, v, res, gamma, beta in sets:
+                            layer.decode_layer(q, k, v, info, res, gamma, beta)
+                    stop.record()
+                    stop.synchronize()
+                    times.append(start.elapsed_time(stop) * 1e3 / (4 * len(sets)))
+            times = sorted(times[3:])
+            return times[len(times) // 2]
+
+        rows.append({"batch": B, "heads": H, "size_per_head": D, "positions": S, "longest": top,
+                     "one_launch": bool(_lib.fn.en_decode_layer_norm_pays(B, H, S, D, 1)),
+                     "as_called_us": [us(torch.cuda.current_stream(), ahead) for ahead in (True, False)],
+                     "two_launches_us": [us(two_launches, ahead) for ahead in (True, False)]})
+    return rows
 
 
 STREAM_MODES = {"copy": 0, "read": 1, "write": 2, "inplace": 0}

@@ -469,6 +469,16 @@ def cmd_decode(ns) -> int:
     for r in line["rows"]:
         print(f"| {r['batch']} | {r['cached_positions']} | {r['units']} | {r['cache_MB']:.0f} | {r['shares_per_unit']} | "
               f"{cell(r['one_workgroup_per_unit'])} | {cell(r['as_called'])} | {cell(r['paged'])} |")
+    print("\n## Decode layers of few units: attention, residual and LayerNorm in one launch\n")
+    print("`layer.decode_layer`, fp16, lengths 1..longest, the operands of eight layers in turn; GPU: calls queued ahead of it, with host: "
+          "the host in step, as a decode loop has it.  As called: one launch of `decode_attn_norm_kernel` where a row is narrow enough for the workgroup that normalises it; two "
+          "launches: the same call on a stream without meeting words.\n")
+    print("| sequences | heads x channels | positions | longest | form as called | GPU: as called, us | two launches, us | "
+          "with host: as called, us | two launches, us |\n|---|---|---|---|---|---|---|---|---|")
+    for r in line["layers"]:
+        one, two = r["as_called_us"], r["two_launches_us"]
+        print(f"| {r['batch']} | {r['heads']} x {r['size_per_head']} | {r['positions']} | {r['longest']} | "
+              f"{'one launch' if r['one_launch'] else 'two launches'} | {one[0]:.1f} | {two[0]:.1f} | {one[1]:.1f} | {two[1]:.1f} |")
     return 0
 
 

@@ -893,7 +893,8 @@ __global__ __launch_bounds__(1024) void attn_tile_table_kernel(const int32_t *__
 }
 
 // Both arrays a layer step looks rows up in, once per batch: workgroup 0 fills the tile table, workgroup 1 + b the row
-// offsets of sequence b (row of token t in the padded [B*S] numbering minus t) and clears its `words` meeting words.  Two launches took 2.8 + 4.7 us and the gap
+// offsets of sequence b (row of token t in the padded [B*S] numbering minus t) and clears its `words` meeting words.  Two
+// launches took 2.8 + 4.7 us and the gap
 // between them for 32 sequences; together they take the longer one.
 __global__ __launch_bounds__(1024) void layer_tables_kernel(const int32_t *__restrict__ lens, const int32_t *__restrict__ cu,
                                                             int batch, int heads, int seq_len, int ntq,

@@ -829,11 +829,12 @@ static bool one_launch_takes(const DecodeAttnArgs &a, int elem_size) {
   int lpk = 8;
   while (lpk * epv < a.D) lpk *= 2;
   const int64_t hidden = (int64_t)a.H * a.D, lanes = attn_form(a, lpk) == AttnForm::kPair ? 512 : 256;
-  // One workgroup has the whole row to read.  us a layer, two launches / one: 1 x 12 heads x 64, up to 300 keys 8.5 / 6.3, 8 x 12 x 64
-  // 8.4 / 6.9, 2 x 8 x 64 fp32, up to 800 9.2 / 8.0, 16 x 24 x 64, up to 900 15.0 / 14.7, 16 x 32 x 128, up to 128 10.1 / 10.1; of five
-  // vectors a lane, 2 x 60 x 128, up to 500 10.3 / 10.7, 5 x 72 x 128 35.8 / 36.8.  Rows of shares are four channels a lane, sixteen
-  // bytes from each share: 1 x 5 x 64, 4000 keys 9.3 / 8.6, 10 x 16 x 64, up to 2000 15.2 / 14.2; combined unit by unit in front of
-  // the row, which takes wider ones, 6 x 64 x 128 41.9 / 43.9.
+  // One workgroup has the whole row to read.  us a layer of a decode loop, two launches / one, where the host's second launch is most
+  // of what is saved (in brackets the GPU alone): 1 x 12 heads x 64, up to 300 keys 8.5 / 6.1 (6.2 / 6.1), 8 x 12 x 64 8.5 / 6.4
+  // (6.9 / 6.4), 2 x 8 x 64 fp32, up to 800 9.2 / 8.0, 16 x 24 x 64, up to 900 15.8 / 15.0 (15.8 / 15.0), 16 x 32 x 128, up to 128
+  // 10.1 / 10.1; of five vectors a lane, 2 x 60 x 128, up to 500 10.3 / 10.7, 5 x 72 x 128 35.8 / 36.8.  Rows of shares are four
+  // channels a lane, sixteen bytes from each share: 1 x 5 x 64, 4000 keys 9.3 / 7.5 (7.9 / 7.5), 10 x 16 x 64, up to 2000 15.5 / 14.3
+  // (15.4 / 14.3); combined unit by unit in front of the row, which takes wider ones, 6 x 64 x 128 41.9 / 43.9.
   return a.nsplit > 1 ? hidden <= 4 * lanes : hidden * elem_size <= kTailVectors * 16 * lanes;
 }
 

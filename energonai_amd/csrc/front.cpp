@@ -79,8 +79,11 @@ hipStream_t stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.
 
 const int32_t *i32(const Tensor &t) { return t.data_ptr<int32_t>(); }
 
-// Launches run without the interpreter lock: a launch may wait for room in the stream's queue.  `f` is the C ABI call alone, on
-// pointers and a stream taken before; whatever it throws all the same leaves with the lock held again.
+// Launches run without the interpreter lock: a launch may wait for room in the stream's queue.  `f` touches no Python object, and what
+// it throws is a C++ exception, which leaves with the lock held again.  Most are the C ABI call alone, on pointers and a stream taken
+// before.  One that calls ATen as well (block_prefill) may because nothing in it comes back to Python: its tensors are exact ones and
+// its caller has seen that gradients and autocast are off and no dispatch or function mode is on; ATen takes the lock by itself where
+// it needs it.
 template <typename F> int without_gil(F &&f) {
   struct Released {
     PyThreadState *saved = PyEval_SaveThread();
@@ -279,7 +282,8 @@ struct WordSets {
   int next = kWordSets;
 };
 uint32_t *next_decode_words(const Tensor &t) {
-  static std::map<std::pair<int, hipStream_t>, WordSets> &pool = *new std::map<std::pair<int, hipStream_t>, WordSets>;   // under the interpreter lock
+  typedef std::map<std::pair<int, hipStream_t>, WordSets> Pool;
+  static Pool &pool = *new Pool;     // under the interpreter lock
   const auto stream = c10::hip::getCurrentHIPStream(t.device().index());
   if (stream.id() != 0 && stream.id() == (c10::StreamId) reinterpret_cast<intptr_t>(stream.stream())) return nullptr;   // external
   WordSets &w = pool[std::make_pair((int)t.device().index(), stream.stream())];

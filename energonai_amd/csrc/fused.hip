@@ -517,16 +517,18 @@ static int attn_fused(const void *q, const void *k, const void *v, void *ctx, co
 // Workgroups that are resident at once: what LDS and registers leave room for on 256 CUs.
 static int64_t resident_workgroups(int size_per_head, int dtype) { return dtype == EN_F32 ? 512 : size_per_head <= 64 ? 1024 : 768; }
 
-// Where one launch is the faster form, us per layer, one launch / two (6 layers, hot operands).  Meeting costs about 6 us
+// Where one launch is the faster form, us per layer, one launch / two (6 layers, hot operands, launches queued ahead of the GPU).  Meeting costs about 6 us
 // (context written through, counted, seen, read back), a trip to memory for every round of a wave's rows (norm_rows_ahead); a
 // LayerNorm launch costs 5 us and what its bytes take.
-//   16-bit: context of 7 MB and more and at most three rows per wave: 24 sequences of up to 384, 16 heads x 64 22.4 / 24.2, 4 of up
-//     to 700, 16 x 128 22.4 / 23.6 (not every one: 8 of up to 665, 14 x 96 25.2 / 24.7).  From 3.5 to 7 MB the two are close, one launch
-//     ahead since three rows of a wave go out at once (32 of up to 128, 16 x 64 11.6 / 11.9, 1 of 1024, 16 x 128 28.6 / 28.9, 14 of up to
-//     356, 11 x 80 16.1 / 17.0, 8 of up to 256, 32 x 64 14.6 / 15.5), at 3 MB they meet (8 of up to 300, 12 x 80 14.8 / 14.5), and
-//     smaller ones lose (16 of up to 128, 12 x 64 10.7 / 9.5, one of 509 15.1 / 13.4), as do few heads (64 of up to 128, 4 x 64
-//     15.1 / 10.5).  Where the launches themselves are what bounds a layer, short prompts: one of 60 rows, 12 x 64 10.4 / 11.3 with the
-//     host's part, 64 of up to 30, 4 x 64 10.7 / 13.1 (16 x 64, a full chip: 13.8 / 13.1).
+//   16-bit: context of 7 MB and more and at most three rows per wave: 24 sequences of up to 384, 16 heads x 64 19.1 / 21.1, 32 of up
+//     to 512, 12 x 64 20.9 / 23.1, 8 of up to 665, 14 x 96 22.0 / 22.8.  That is where the two met while two rows of a wave were in
+//     flight; now that three go out at once they meet near 3 MB (8 of up to 300, 12 x 80 13.8 / 13.1; 32 of up to 128, 16 x 64, 4.0 MB
+//     12.25 / 12.2), and the line leaves up to 1 us a layer from there to 7 MB (8 of up to 256, 32 x 64 13.3 / 13.6, 24 of up to 300,
+//     12 x 64 14.5 / 15.0, 14 of up to 356, 11 x 80 17.0 / 18.0, 4 of up to 700, 16 x 128 22.8 / 23.7, 1 of 1024 29.4 / 29.6).  Smaller
+//     ones lose (16 of up to 128, 12 x 64 10.7 / 9.5, one of 509 15.1 / 13.4), as do few heads (64 of up to 128, 4 x 64 15.1 / 10.5).
+//     Short prompts: where the host is what bounds a layer, one launch less is what counts (one of 60 rows, 12 x 64 10.4 / 11.3, 64 of
+//     up to 30, 4 x 64 10.7 / 13.1).  The GPU alone takes longer for it: 8.2 / 7.35 and 8.4 / 7.3, 64 of up to 64, 8 x 64 9.35 / 8.8,
+//     32 of up to 64, 16 x 64 9.3 / 9.15.
 //   fp32 (64-row tiles): 4 of up to 128, 12 x 64 15.0 / 15.5, 21 of up to 73, 6 x 64 12.3 / 12.5; 58 of up to 239, 3 x 64 39.0 / 34.8.
 static bool one_launch_pays(int heads, int seq_len, int64_t tiles, int64_t bytes, int dtype) {
   const int64_t per_wave = ceil_div(std::min(seq_len, dtype == EN_F32 ? kF32QTile : kQTile), heads * (kBlock / kWave));
@@ -569,8 +571,9 @@ int attn_fused_beside_norm(const void *qkv, void *ctx, const int32_t *seq_lens, 
   NormRows rows{in, residual, residual_row_offsets, gamma, beta, y, T, (int)hidden, eps, 0, 0};
   rows.groups = (int)ceil_div(ceil_div(T, norm_rows_per_workgroup((int)hidden)), kXcds);
   // Rows are dealt out between the attention's workgroups, as if those were twice their likely number: the long ones, which
-  // come first, start the earlier for it (10 heads x 80, 3866 tokens: 34 us by the likely number itself, 32 by twice that); but over no more groups than the launch has for the attention:
-  // all groups of rows then come before its last one, and no workgroup looks behind the end of the tile table.
+  // come first, start the earlier for it (10 heads x 80, 3866 tokens: 34 us by the likely number itself, 32 by twice that); but
+  // over no more groups than the launch has for the attention: all groups of rows then come before its last one, and no
+  // workgroup looks behind the end of the tile table.
   const int64_t attention = std::min(2 * ceil_div(query_tiles(batch, max_seq_len, T, dtype) * head_num, kXcds),
                                      ceil_div((int64_t)batch * head_num, kXcds) * ceil_div(max_seq_len, kQTile));
   rows.step = (uint32_t)ceil_div((int64_t)rows.groups << 16, attention + rows.groups);

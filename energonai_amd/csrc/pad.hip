@@ -473,7 +473,8 @@ int en_kv_fill_pair(const void *src, void *k_cache, void *v_cache, const int32_t
                                   stream);
   }
   const GatherPart gk{pk, (int)vpr, R, (unsigned)grid_x}, gv{pv, (int)vpr, R, (unsigned)grid_x};
-  const PadMap mk{cu_seqlens, head_num, cache_len, R, src_head_rows, k_head_first, 1}, mv{cu_seqlens, head_num, cache_len, R, src_head_rows, v_head_first, 1};
+  const PadMap mk{cu_seqlens, head_num, cache_len, R, src_head_rows, k_head_first, 1};
+  const PadMap mv{cu_seqlens, head_num, cache_len, R, src_head_rows, v_head_first, 1};
   row_gather_pair_kernel<PadMap, PadMap><<<(unsigned)(2 * blocks), kBlock, 0, (hipStream_t)stream>>>(mk, gk, mv, gv, (unsigned)blocks);
   EN_RETURN_IF_LAUNCH_FAILED();
   return EN_OK;

@@ -97,7 +97,8 @@ def attn_qk(q, k, seq_len_list, *, alpha: float = 1.0, causal: bool = True, q_le
         _lib.check(_lib.fn.en_attn_qk(q.data_ptr(), k.data_ptr(), out.data_ptr(), k_info.lens.data_ptr(), q_ptr,
                                           B, H, Sq, Sk, D, *qs, *ks, float(alpha), int(bool(causal)),
                                           _lib.dtype_tag(q, "attn_qk"), None, None, 0,
-                                          _tile_table_ptr(k_info, q_ptr, H, Sq, _unit_kv_bytes(Sk, D, q), causal=causal), _lib.stream_of(q)), "attn_qk")
+                                          _tile_table_ptr(k_info, q_ptr, H, Sq, _unit_kv_bytes(Sk, D, q), causal=causal),
+                                          _lib.stream_of(q)), "attn_qk")
     return out
 
 
@@ -127,7 +128,8 @@ def attn_pv(p, v, seq_len_list, *, causal: bool = True, q_len_list=None, zero_pa
         _lib.check(_lib.fn.en_attn_pv(p.data_ptr(), v.data_ptr(), out.data_ptr(), k_info.lens.data_ptr(), q_ptr,
                                           B, H, Sq, Sk, D, *vs, *cs, int(bool(causal)), int(bool(zero_padding)),
                                           _lib.dtype_tag(p, "attn_pv"), None, None, 0,
-                                          _tile_table_ptr(k_info, q_ptr, H, Sq, _unit_kv_bytes(Sk, D, p), causal=causal), _lib.stream_of(p)), "attn_pv")
+                                          _tile_table_ptr(k_info, q_ptr, H, Sq, _unit_kv_bytes(Sk, D, p), causal=causal),
+                                          _lib.stream_of(p)), "attn_pv")
     return out
 
 

@@ -188,9 +188,9 @@ class SeqInfo:
         """Workgroup order of the attention kernels for this batch (``en_attn_tile_table``): the query tiles the
         sequences really have, longest sequence first.  ``unit_kv_bytes`` is what one (batch, head) unit's K and V
         hold at full length and ``causal`` the mask of the call it is for (``None``: by ``unit_kv_bytes`` alone); they decide
-        whether the last tiles of all units run first or a unit's tiles stay together (``tiles_first``).  ``query_tile`` is the tile height of the kernel that will read the table (128; 256 for the fused
-        kernel's 64-queries-per-wave form).  Computed once per batch, head count, bucket, order and tile height by one
-        small kernel and reused by every layer."""
+        whether the last tiles of all units run first or a unit's tiles stay together (``tiles_first``).  ``query_tile`` is the
+        tile height of the kernel that will read the table (128; 256 for the fused kernel's 64-queries-per-wave form).  Computed
+        once per batch, head count, bucket, order and tile height by one small kernel and reused by every layer."""
         version = self._lens_version()
         first = tiles_first(self.batch_size * int(head_num), int(unit_kv_bytes), causal)
         key = (int(head_num), int(q_seq_len), first, version, int(query_tile))

@@ -352,7 +352,8 @@ int en_decode_attn_paged(const void *q, const void *k_pool, const void *v_pool, 
  * lengths; batch b then starts at row offsets[b] (give stride[0] = 0), so neither
  * transpose_pad before nor transpose_depad after is needed; q_seq_len / k_seq_len
  * are then upper bounds of the lengths.  Null offsets select the padded layout.
- * scale must be positive.  Rows i >= q_lens[b] of ctx are left untouched.  fp16 / bf16, fp32 accumulation and statistics; D a multiple of 8, D <= 128.
+ * scale must be positive.  Rows i >= q_lens[b] of ctx are left untouched.  fp16 / bf16, fp32 accumulation and statistics; D a
+ * multiple of 8, D <= 128.
  * query_tile: query rows per workgroup.  128 = four waves of 32 queries; 256 = four waves of 64 queries (heads of
  * 65..128 channels only): half the LDS reads, tile loads and barriers per FLOP at two waves per SIMD instead of
  * three; 0 = what en_attn_fused_query_tile names for these arguments.  tile_table as in en_attn_qk, built for the
@@ -371,8 +372,8 @@ int en_attn_fused(const void *q, const void *k, const void *v, void *ctx, const 
  * longest sequence first, so that the launch wastes no workgroup slots on tiles past a sequence's end and its long
  * workgroups start first.  tiles_first == 0 keeps the query tiles of a (batch, head) unit together (they share its
  * K and V in L2); tiles_first != 0 runs the last tiles of all units first, then the second-to-last ... (the better
- * order under a causal mask while K and V of all units are small, up to about 96 MB, 160 with 256 units and fewer).  Built once per batch and reused by every layer;
- * one small kernel on `stream`. */
+ * order under a causal mask while K and V of all units are small, up to about 96 MB, 160 with 256 units and fewer).  Built
+ * once per batch and reused by every layer; one small kernel on `stream`. */
 int64_t en_attn_tile_table_elems(int batch, int head_num, int q_seq_len, int query_tile);
 int en_attn_tile_table(const int32_t *seq_lens, int batch, int head_num, int q_seq_len, int tiles_first,
                        int query_tile, int32_t *table, en_stream_t stream);
@@ -388,8 +389,9 @@ int en_layer_tables(const int32_t *seq_lens, const int32_t *cu_seqlens, int batc
  * workgroups of a query tile meet at a word of `arrivals` (en_attn_fused_norm_arrivals words, zero before the first launch
  * and again after each): launches that share the array must be ordered by one stream.  `polls` bounds how often a workgroup
  * looks for the others before it leaves its rows to the last of them (any value gives the same result; < 0: the library's
- * choice, and a launch only where it is faster than two, which en_attn_fused_norm_pays says).  EN_ERR_UNSUPPORTED, with nothing launched, where it does not apply: more workgroups than are resident at once,
- * widths of more than 256 16-byte vectors, more than 48 heads, operands off 16 bytes or overlapping, a stream under capture. */
+ * choice, and a launch only where en_attn_fused_norm_pays says so).  EN_ERR_UNSUPPORTED, with nothing launched, where it does
+ * not apply: more workgroups than are resident at once, widths of more than 256 16-byte vectors, more than 48 heads, operands off
+ * 16 bytes or overlapping, a stream under capture. */
 int64_t en_attn_fused_norm_arrivals(int batch, int q_seq_len);
 int en_attn_fused_norm_pays(int batch, int head_num, int max_seq_len, int size_per_head, int64_t total_tokens, int dtype);
 int en_attn_fused_norm(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
@@ -444,8 +446,8 @@ int en_block_decode(const en_block_decode_args *args, en_stream_t stream);
  * buffer: x_packed [T,hid] (residual stream), qkv_padded [B,H,S,3D], scores [B,H,S,S],
  * ctx [B,H,S,D], ctx_packed [T,H*D], y [T,hid].  dense_out [T,hid], if not NULL, is what
  * the LayerNorm adds to x_packed instead of ctx_packed (the output projection lies between
- * the two in a real layer); form 2 in 16-bit storage then runs the LayerNorm beside the attention, in its launch.  attention_form: 0 = the three separate ops, 1 = en_attn_fused
- * on the padded buffer (scores unused), 2 = en_attn_fused on the packed projections
+ * the two in a real layer); form 2 in 16-bit storage then runs the LayerNorm beside the attention, in its launch.
+ * attention_form: 0 = the three separate ops, 1 = en_attn_fused on the padded buffer (scores unused), 2 = en_attn_fused on the packed projections
  * (qkv_padded, scores and ctx unused), 3 = the three separate ops on the packed projections
  * (row offsets into qkv_packed and ctx_packed: transpose_pad and transpose_depad do not run;
  * qkv_padded and ctx unused), 4 = form 3 with the scores in the packed causal layout

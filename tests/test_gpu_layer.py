@@ -581,7 +581,8 @@ def test_decode_layer_words_belong_to_their_stream():
                 rand(H * D))
 
     need = _lib.fn.en_decode_attn_workspace_bytes(B, H, S, D)
-    zeros, ws = torch.zeros(_lib.fn.en_decode_layer_norm_words(), dtype=torch.int32, device="cuda"), torch.zeros(need, dtype=torch.uint8, device="cuda")
+    zeros = torch.zeros(_lib.fn.en_decode_layer_norm_words(), dtype=torch.int32, device="cuda")
+    ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
     strides = (ctypes.c_int64 * 3)(H * S * D, S * D, D)
 
     def one_launch(a, ctx, y):
