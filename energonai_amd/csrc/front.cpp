@@ -1,4 +1,4 @@
-// The host side of a layer step, a decode step and a batch's bookkeeping as one native call each: argument checks, output
+// The host side of a layer step, a decode step, the single operations and a batch's bookkeeping as one native call each: argument checks, output
 // allocation (torch's caching allocator), stream lookup and the C ABI call.  The same work in Python and ctypes costs 16 us
 // per layer step and 23 us per decode step against 6 us of kernel launches, which is more than the GPU needs for a short
 // prompt (9 us) or a decode step of one sequence.  Nothing is computed here; every launch is an entry point of
@@ -10,9 +10,12 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
+#include <cmath>
 #include <map>
 #include <stdexcept>
 #include <string>
@@ -376,6 +379,341 @@ PyObject *decode_layer(PyObject *const *a) {
   return THPVariable_Wrap(y);
 }
 
+// ---- single operations -------------------------------------------------------------------------------------------------
+// What the Python calls of kernel/ do with plain operands: tensors of torch's own class on one GPU, contiguous where the entry point
+// takes no strides, shapes and types as the call wants them, no function or dispatch mode on.  Anything else returns None with nothing
+// launched, and the Python call goes on: it names what is wrong, copies, or has a mode see what it does.  A call takes 9..11 us of host time
+// in Python and ctypes, more than most of these kernels do on a small batch.  us a layer where the host bounds it, before / now: paged
+// decode (append, attention, LayerNorm: three calls) 32 / 14, the reference's sequence of operations (six calls) 72 / 48.
+
+struct Lens {
+  const Tensor *lens = nullptr, *cu = nullptr;
+  int64_t batch = 0;
+};
+
+bool modes_on() { return at::impl::PythonTorchFunctionTLS::stack_len() > 0 || c10::impl::TorchDispatchModeTLS::any_modes_set(); }
+
+const Tensor *plain(PyObject *o) {
+  if (!THPVariable_CheckExact(o)) return nullptr;
+  const Tensor &t = THPVariable_Unpack(o);
+  return t.is_cuda() && t.layout() == at::kStrided && t.numel() > 0 ? &t : nullptr;
+}
+const Tensor *plain_contiguous(PyObject *o) {
+  const Tensor *t = plain(o);
+  return t && t->is_contiguous() ? t : nullptr;
+}
+const Tensor *plain_rows(PyObject *o, int64_t dim) {      // the last dimension is contiguous
+  const Tensor *t = plain(o);
+  return t && t->dim() == dim && t->stride(dim - 1) == 1 ? t : nullptr;
+}
+
+int known_tag(const Tensor &t) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return EN_F32;
+    case at::kHalf: return EN_F16;
+    case at::kBFloat16: return EN_BF16;
+    default: return -1;
+  }
+}
+
+// An attribute of a SeqInfo, which holds it on.
+PyObject *held(PyObject *info, PyObject *key) {
+  PyObject *v = PyObject_GetAttr(info, key);
+  if (!v) fail("SeqInfo: attribute missing");
+  Py_DECREF(v);
+  return v;
+}
+
+// Lengths and prefix of a SeqInfo on t's device for `batch` sequences.
+bool lens_of(PyObject *info, const Tensor &t, int64_t batch, bool with_cu, Lens &out) {
+  static PyObject *const lens = PyUnicode_InternFromString("lens"), *const cu = PyUnicode_InternFromString("cu_seqlens"),
+                         *const size = PyUnicode_InternFromString("batch_size");
+  out.batch = integer(held(info, size));
+  PyObject *l = held(info, lens), *c = held(info, cu);
+  if (out.batch != batch || !THPVariable_CheckExact(l) || (with_cu && !THPVariable_CheckExact(c))) return false;
+  out.lens = &THPVariable_Unpack(l);
+  out.cu = with_cu ? &THPVariable_Unpack(c) : nullptr;
+  for (const Tensor *x : {out.lens, out.cu})
+    if (x && (x->device() != t.device() || x->scalar_type() != at::kInt || !x->is_contiguous())) return false;
+  return out.lens->numel() >= batch && (!with_cu || out.cu->numel() > batch);
+}
+
+// SeqInfo.order_current_stream, looked at natively: most calls find their stream among the ordered ones.
+void order_stream(PyObject *info, const Tensor &t) {
+  static PyObject *const ready = PyUnicode_InternFromString("_ready"), *const ordered = PyUnicode_InternFromString("_ordered"),
+                         *const order = PyUnicode_InternFromString("order_current_stream");
+  const int pending = PyObject_IsTrue(held(info, ready));
+  if (pending == 0) return;
+  PyObject *raw = PyLong_FromVoidPtr(stream_of(t));
+  const int there = pending < 0 || !raw ? -1 : PySet_Contains(held(info, ordered), raw);
+  Py_XDECREF(raw);
+  if (there < 0) fail("SeqInfo: streams");
+  if (there) return;
+  PyObject *done = PyObject_CallMethodNoArgs(info, order);
+  if (!done) fail("SeqInfo: order_current_stream");
+  Py_DECREF(done);
+}
+
+bool number(PyObject *o) { return PyFloat_Check(o) || PyLong_Check(o); }
+
+bool is_width(PyObject *shape, int64_t n) {      // n, or (n,)
+  if (PyTuple_Check(shape) && PyTuple_GET_SIZE(shape) == 1) shape = PyTuple_GET_ITEM(shape, 0);
+  return PyLong_CheckExact(shape) && integer(shape) == n;
+}
+
+// layer_norm(input, weight, bias, normalized_shape, eps, residual or None) -> y or None
+PyObject *layer_norm(PyObject *const *a) {
+  const Tensor *x = plain_contiguous(a[0]), *w = plain_contiguous(a[1]), *b = plain_contiguous(a[2]), *r = nullptr;
+  if (!x || !w || !b || modes_on() || w->dim() != 1 || b->sizes() != w->sizes() || b->scalar_type() != w->scalar_type()) Py_RETURN_NONE;
+  const int64_t n2 = w->numel();
+  const int in = known_tag(*x), out = known_tag(*w);
+  if (in < 0 || out < 0 || (in != out && in != EN_F32) || x->dim() < 1 || x->size(-1) != n2 || !is_width(a[3], n2) || !number(a[4])) Py_RETURN_NONE;
+  if (a[5] != Py_None) {
+    r = plain_contiguous(a[5]);
+    if (!r || r->scalar_type() != x->scalar_type() || r->sizes() != x->sizes() || r->device() != x->device()) Py_RETURN_NONE;
+  }
+  if (w->device() != x->device() || b->device() != x->device()) Py_RETURN_NONE;
+  const float eps = real(a[4]);
+  const c10::DeviceGuard guard(x->device());
+  const Tensor y = at::empty(x->sizes(), w->options());
+  void *y_p = y.data_ptr();
+  const void *x_p = x->data_ptr(), *r_p = r ? r->data_ptr() : nullptr, *w_p = w->data_ptr(), *b_p = b->data_ptr();
+  const int64_t n1 = x->numel() / n2;
+  const hipStream_t stream = stream_of(*x);
+  check(without_gil([&] { return en_layernorm_fwd(y_p, nullptr, nullptr, nullptr, x_p, r_p, nullptr, w_p, b_p, n1, n2, eps, in, out, stream); }),
+        "layer_norm");
+  return THPVariable_Wrap(y);
+}
+
+const Tensor *page_table(PyObject *o, const Tensor &pool, int64_t batch) {
+  const Tensor *t = plain_contiguous(o);
+  return t && t->dim() == 2 && t->size(0) == batch && t->scalar_type() == at::kInt && t->device() == pool.device() ? t : nullptr;
+}
+
+// kv_pages_append(k_new, v_new, k_pool, v_pool, SeqInfo, page_table, overflow or None) -> True or None
+PyObject *kv_pages_append(PyObject *const *a) {
+  const Tensor *kn = plain_rows(a[0], 3), *vn = plain_rows(a[1], 3), *kp = plain_rows(a[2], 4), *vp = plain_rows(a[3], 4), *over = nullptr;
+  if (!kn || !vn || !kp || !vp || modes_on()) Py_RETURN_NONE;
+  const int64_t N = kp->size(0), H = kp->size(1), P = kp->size(2), D = kp->size(3), B = kn->size(0), rows[3] = {B, H, D};
+  Lens info;
+  if (vp->sizes() != kp->sizes() || vp->strides() != kp->strides() || kn->sizes() != c10::IntArrayRef(rows) || vn->sizes() != kn->sizes() ||
+      vn->strides() != kn->strides() || !lens_of(a[4], *kp, B, false, info))
+    Py_RETURN_NONE;
+  for (const Tensor *t : {kn, vn, vp})
+    if (t->scalar_type() != kp->scalar_type() || t->device() != kp->device()) Py_RETURN_NONE;
+  const Tensor *table = page_table(a[5], *kp, B);
+  if (a[6] != Py_None) {
+    over = plain_contiguous(a[6]);
+    if (!over || over->scalar_type() != at::kInt || over->device() != kp->device()) Py_RETURN_NONE;
+  }
+  if (!table) Py_RETURN_NONE;
+  const c10::DeviceGuard guard(kp->device());
+  order_stream(a[4], *kp);
+  const int64_t strides[3] = {kp->stride(0), kp->stride(1), kp->stride(2)}, n_sb = kn->stride(0), n_sh = kn->stride(1), pages = table->size(1);
+  const void *kn_p = kn->data_ptr(), *vn_p = vn->data_ptr();
+  void *kp_p = kp->data_ptr(), *vp_p = vp->data_ptr();
+  const int32_t *lens_p = i32(*info.lens), *table_p = i32(*table);
+  int32_t *over_p = over ? over->data_ptr<int32_t>() : nullptr;
+  const int es = (int)kp->element_size();
+  const hipStream_t stream = stream_of(*kp);
+  check(without_gil([&] {
+          return en_kv_append_paged(kn_p, vn_p, kp_p, vp_p, lens_p, table_p, (int)B, (int)H, (int)pages, (int)P, (int)N, (int)D, n_sb, n_sh,
+                                    strides, es, over_p, stream);
+        }), "kv_pages_append");
+  Py_RETURN_TRUE;
+}
+
+// decode_attn_paged(q, k_pool, v_pool, SeqInfo, page_table, scale or None) -> ctx or None
+PyObject *decode_attn_paged(PyObject *const *a) {
+  const Tensor *q = plain_contiguous(a[0]), *kp = plain_rows(a[1], 4), *vp = plain_rows(a[2], 4);
+  if (!q || !kp || !vp || modes_on()) Py_RETURN_NONE;
+  const int64_t N = kp->size(0), H = kp->size(1), P = kp->size(2), D = kp->size(3), B = q->numel() / (H * D);
+  const int tag = known_tag(*q);
+  Lens info;
+  if (tag < 0 || q->dim() < 2 || q->numel() != B * H * D || vp->sizes() != kp->sizes() || !lens_of(a[3], *q, B, false, info)) Py_RETURN_NONE;
+  for (const Tensor *t : {kp, vp})
+    if (t->scalar_type() != q->scalar_type() || t->device() != q->device()) Py_RETURN_NONE;
+  const Tensor *table = page_table(a[4], *q, B);
+  if (!table || (a[5] != Py_None && !number(a[5]))) Py_RETURN_NONE;
+  const float scale = a[5] == Py_None ? (float)std::pow((double)D, -0.5) : real(a[5]);
+  const c10::DeviceGuard guard(q->device());
+  order_stream(a[3], *q);
+  const int64_t pages = table->size(1), need = en_decode_attn_workspace_bytes((int)B, (int)H, (int)(pages * P), (int)D);
+  const Tensor out = at::empty({B, H, 1, D}, q->options());
+  Tensor ws;
+  if (need > 0) ws = at::empty({need}, q->options().dtype(at::kByte));
+  const int64_t ks[3] = {kp->stride(0), kp->stride(1), kp->stride(2)}, vs[3] = {vp->stride(0), vp->stride(1), vp->stride(2)};
+  const void *q_p = q->data_ptr(), *k_p = kp->data_ptr(), *v_p = vp->data_ptr();
+  void *out_p = out.data_ptr(), *ws_p = need > 0 ? ws.data_ptr() : nullptr;
+  const int32_t *lens_p = i32(*info.lens), *table_p = i32(*table);
+  const hipStream_t stream = stream_of(*q);
+  check(without_gil([&] {
+          return en_decode_attn_paged(q_p, k_p, v_p, out_p, lens_p, table_p, (int)B, (int)H, (int)pages, (int)P, (int)N, (int)D, ks, vs, scale,
+                                      tag, ws_p, need, stream);
+        }), "decode_attn_paged");
+  return THPVariable_Wrap(out);
+}
+
+bool fits_int(std::initializer_list<int64_t> values) {
+  for (const int64_t v : values)
+    if (v < 1 || v > INT32_MAX) return false;
+  return true;
+}
+
+// depad(src, SeqInfo, batch, left_padded, total) -> packed rows or None
+PyObject *depad(PyObject *const *a) {
+  const Tensor *src = plain_contiguous(a[0]);
+  if (!src || modes_on() || src->dim() != 3) Py_RETURN_NONE;
+  const int64_t batch = integer(a[2]), left = PyObject_IsTrue(a[3]), total = integer(a[4]), S = src->size(1), hid = src->size(2);
+  const int es = (int)src->element_size();
+  Lens info;
+  if ((es != 2 && es != 4) || left < 0 || !fits_int({batch, S, total}) || !lens_of(a[1], *src, batch, true, info)) Py_RETURN_NONE;
+  const c10::DeviceGuard guard(src->device());
+  order_stream(a[1], *src);
+  const Tensor dst = at::empty({1, total, hid}, src->options());
+  const void *src_p = src->data_ptr();
+  void *dst_p = dst.data_ptr();
+  const int32_t *cu_p = i32(*info.cu);
+  const hipStream_t stream = stream_of(*src);
+  check(without_gil([&] { return en_depad(src_p, dst_p, cu_p, (int)batch, (int)S, hid, es, (int)left, stream); }), "depad");
+  return THPVariable_Wrap(dst);
+}
+
+// transpose_pad(src, SeqInfo, batch, max_seq_len, heads, size_per_head) -> padded tensor or None
+PyObject *transpose_pad(PyObject *const *a) {
+  const Tensor *src = plain_contiguous(a[0]);
+  if (!src || modes_on()) Py_RETURN_NONE;
+  const int64_t batch = integer(a[2]), S = integer(a[3]), H = integer(a[4]), D = integer(a[5]);
+  const int es = (int)src->element_size();
+  Lens info;
+  if ((es != 2 && es != 4) || !fits_int({batch, S, H, D}) || src->numel() % (H * D) || !lens_of(a[1], *src, batch, true, info)) Py_RETURN_NONE;
+  const c10::DeviceGuard guard(src->device());
+  order_stream(a[1], *src);
+  const Tensor dst = at::empty({batch, H, S, D}, src->options());
+  const void *src_p = src->data_ptr();
+  void *dst_p = dst.data_ptr();
+  const int32_t *cu_p = i32(*info.cu);
+  const hipStream_t stream = stream_of(*src);
+  check(without_gil([&] { return en_transpose_pad(src_p, dst_p, cu_p, (int)batch, (int)S, (int)H, (int)D, es, stream); }), "transpose_pad");
+  return THPVariable_Wrap(dst);
+}
+
+// transpose_depad(src, SeqInfo, batch, total, max_seq_len, heads, size_per_head) -> packed tensor or None
+PyObject *transpose_depad(PyObject *const *a) {
+  const Tensor *src = plain_contiguous(a[0]);
+  if (!src || modes_on()) Py_RETURN_NONE;
+  const int64_t batch = integer(a[2]), total = integer(a[3]), S = integer(a[4]), H = integer(a[5]), D = integer(a[6]);
+  const int es = (int)src->element_size();
+  Lens info;
+  if ((es != 2 && es != 4) || !fits_int({batch, total, S, H, D}) || src->numel() / batch / H / S != D || src->numel() != batch * H * S * D ||
+      !lens_of(a[1], *src, batch, true, info))
+    Py_RETURN_NONE;
+  const c10::DeviceGuard guard(src->device());
+  order_stream(a[1], *src);
+  const Tensor dst = at::empty({1, total, H, D}, src->options());
+  const void *src_p = src->data_ptr();
+  void *dst_p = dst.data_ptr();
+  const int32_t *cu_p = i32(*info.cu);
+  const hipStream_t stream = stream_of(*src);
+  check(without_gil([&] { return en_transpose_depad(src_p, dst_p, cu_p, (int)batch, (int)S, (int)H, (int)D, es, stream); }), "transpose_depad");
+  return THPVariable_Wrap(dst);
+}
+
+// scale_mask_softmax(src, SeqInfo, batch, max_seq_len, heads, scale, causal, tail_rows) -> True (in place) or None
+PyObject *scale_mask_softmax(PyObject *const *a) {
+  const Tensor *src = plain_contiguous(a[0]);
+  if (!src || modes_on()) Py_RETURN_NONE;
+  const int64_t batch = integer(a[2]), S = integer(a[3]), H = integer(a[4]), causal = PyObject_IsTrue(a[6]), tail = integer(a[7]);
+  const int tag = known_tag(*src);
+  Lens info;
+  if (tag < 0 || causal < 0 || !number(a[5]) || !fits_int({batch, S, H}) || tail < 0 || tail > INT32_MAX || src->numel() / batch / H / S != S ||
+      src->numel() != batch * H * S * S || !lens_of(a[1], *src, batch, false, info))
+    Py_RETURN_NONE;
+  const float scale = real(a[5]);
+  const c10::DeviceGuard guard(src->device());
+  order_stream(a[1], *src);
+  void *src_p = src->data_ptr();
+  const int32_t *lens_p = i32(*info.lens);
+  const hipStream_t stream = stream_of(*src);
+  check(without_gil([&] {
+          return en_scale_mask_softmax(src_p, lens_p, nullptr, (int)batch, (int)H, (int)S, (int)S, scale, (int)causal, (int)tail, tag, stream);
+        }), "scale_mask_softmax");
+  Py_RETURN_TRUE;
+}
+
+// The workgroup order of an attention call (SeqInfo.tile_table), None for a SeqInfo of one call.  It lives on in the SeqInfo, or in
+// `keep` until the launch.
+const int32_t *tile_table(PyObject *info, int64_t heads, int64_t q_len, int64_t k_len, int64_t channels, int64_t elem, bool causal, Tensor &keep) {
+  static PyObject *const ephemeral = PyUnicode_InternFromString("ephemeral"), *const get = PyUnicode_InternFromString("tile_table");
+  const int once = PyObject_IsTrue(held(info, ephemeral));
+  if (once) {
+    if (once < 0) fail("SeqInfo: ephemeral");
+    return nullptr;
+  }
+  PyObject *args[6] = {info, PyLong_FromLongLong(heads), PyLong_FromLongLong(q_len), PyLong_FromLongLong(2 * k_len * channels * elem),
+                       PyLong_FromLong(128), causal ? Py_True : Py_False};
+  PyObject *t = args[1] && args[2] && args[3] && args[4] ? PyObject_VectorcallMethod(get, args, 6, nullptr) : nullptr;
+  for (int i = 1; i < 5; ++i) Py_XDECREF(args[i]);
+  if (!t) fail("SeqInfo: tile_table");
+  if (THPVariable_Check(t)) keep = THPVariable_Unpack(t);
+  Py_DECREF(t);
+  if (!keep.defined()) fail("SeqInfo: tile_table gives no tensor");
+  return i32(keep);
+}
+
+// attn_qk(q, k, SeqInfo, alpha, causal) -> scores or None
+PyObject *attn_qk(PyObject *const *a) {
+  const Tensor *q = plain_rows(a[0], 4), *k = plain_rows(a[1], 4);
+  if (!q || !k || modes_on()) Py_RETURN_NONE;
+  const int64_t B = q->size(0), H = q->size(1), Sq = q->size(2), D = q->size(3), Sk = k->size(2);
+  const int tag = known_tag(*q), causal = PyObject_IsTrue(a[4]);
+  Lens info;
+  if (tag < 0 || causal < 0 || !number(a[3]) || k->size(0) != B || k->size(1) != H || k->size(3) != D || k->scalar_type() != q->scalar_type() ||
+      k->device() != q->device() || !fits_int({B, H, Sq, Sk, D}) || !lens_of(a[2], *q, B, false, info))
+    Py_RETURN_NONE;
+  const float alpha = real(a[3]);
+  const c10::DeviceGuard guard(q->device());
+  order_stream(a[2], *q);
+  Tensor keep;
+  const int32_t *table = tile_table(a[2], H, Sq, Sk, D, q->element_size(), causal, keep), *lens_p = i32(*info.lens);
+  const Tensor out = at::empty({B, H, Sq, Sk}, q->options());
+  const void *q_p = q->data_ptr(), *k_p = k->data_ptr();
+  void *out_p = out.data_ptr();
+  const int64_t q0 = q->stride(0), q1 = q->stride(1), q2 = q->stride(2), k0 = k->stride(0), k1 = k->stride(1), k2 = k->stride(2);
+  const hipStream_t stream = stream_of(*q);
+  check(without_gil([&] {
+          return en_attn_qk(q_p, k_p, out_p, lens_p, nullptr, (int)B, (int)H, (int)Sq, (int)Sk, (int)D, q0, q1, q2, k0, k1, k2, alpha, causal, tag,
+                            nullptr, nullptr, 0, table, stream);
+        }), "attn_qk");
+  return THPVariable_Wrap(out);
+}
+
+// attn_pv(p, v, SeqInfo, causal) -> context or None
+PyObject *attn_pv(PyObject *const *a) {
+  const Tensor *p = plain_contiguous(a[0]), *v = plain_rows(a[1], 4);
+  if (!p || !v || modes_on() || p->dim() != 4) Py_RETURN_NONE;
+  const int64_t B = p->size(0), H = p->size(1), Sq = p->size(2), Sk = p->size(3), D = v->size(3);
+  const int tag = known_tag(*p), causal = PyObject_IsTrue(a[3]);
+  Lens info;
+  if (tag < 0 || causal < 0 || v->size(0) != B || v->size(1) != H || v->size(2) != Sk || v->scalar_type() != p->scalar_type() ||
+      v->device() != p->device() || !fits_int({B, H, Sq, Sk, D}) || !lens_of(a[2], *p, B, false, info))
+    Py_RETURN_NONE;
+  const c10::DeviceGuard guard(p->device());
+  order_stream(a[2], *p);
+  Tensor keep;
+  const int32_t *table = tile_table(a[2], H, Sq, Sk, D, p->element_size(), causal, keep), *lens_p = i32(*info.lens);
+  const Tensor out = at::empty({B, H, Sq, D}, p->options());
+  const void *p_p = p->data_ptr(), *v_p = v->data_ptr();
+  void *out_p = out.data_ptr();
+  const int64_t v0 = v->stride(0), v1 = v->stride(1), v2 = v->stride(2), c0 = H * Sq * D, c1 = Sq * D, c2 = D;
+  const hipStream_t stream = stream_of(*p);
+  check(without_gil([&] {
+          return en_attn_pv(p_p, v_p, out_p, lens_p, nullptr, (int)B, (int)H, (int)Sq, (int)Sk, (int)D, v0, v1, v2, c0, c1, c2, causal, 0, tag,
+                            nullptr, nullptr, 0, table, stream);
+        }), "attn_pv");
+  return THPVariable_Wrap(out);
+}
+
 // ---- the look at a block's modules in front of block_decode ------------------------------------------------------------
 
 PyObject *name(const char *s) { return PyUnicode_InternFromString(s); }
@@ -654,6 +992,15 @@ PyMethodDef kMethods[] = {
     EN_FAST(layer, 19, "en_padding_removal_layer on new outputs"),
     EN_FAST(decode_words, 1, "address of the meeting words of a decode layer on the current stream, or None"),
     EN_FAST(decode_layer, 10, "en_decode_layer on new outputs"),
+    EN_FAST(layer_norm, 6, "layer_norm_forward of plain operands, or None"),
+    EN_FAST(kv_pages_append, 7, "kv_pages_append of plain operands, or None"),
+    EN_FAST(decode_attn_paged, 6, "decode_attn_paged of plain operands, or None"),
+    EN_FAST(depad, 5, "depad of plain operands, or None"),
+    EN_FAST(transpose_pad, 6, "transpose_pad of plain operands, or None"),
+    EN_FAST(transpose_depad, 7, "transpose_depad of plain operands, or None"),
+    EN_FAST(scale_mask_softmax, 8, "scale_mask_softmax of plain operands, or None"),
+    EN_FAST(attn_qk, 5, "attn_qk of plain operands, or None"),
+    EN_FAST(attn_pv, 4, "attn_pv of plain operands, or None"),
     EN_FAST(plain_step, 9, "what block_decode takes of a block's modules, or None where the general step has to see them"),
     EN_FAST(block_prefill, 27, "a pre-LN block over packed rows, its attention on the packed projections"),
     EN_FAST(block_decode, 25, "en_block_decode into a position of an output history"),

@@ -16,7 +16,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
-from ..seqinfo import seq_info
+from ..seqinfo import SeqInfo, seq_info
 
 
 def _bhsd(t: torch.Tensor, name: str):
@@ -80,6 +80,10 @@ def attn_qk(q, k, seq_len_list, *, alpha: float = 1.0, causal: bool = True, q_le
     they can see are written; the rest of ``scores`` is uninitialised, exactly
     the region ``scale_mask_softmax`` never reads.
     """
+    if type(seq_len_list) is SeqInfo and q_len_list is None and out is None:
+        scores = _lib.front.attn_qk(q, k, seq_len_list, alpha, causal)
+        if scores is not None:
+            return scores
     qs = _bhsd(q, "q")
     ks = _bhsd(k, "k")
     B, H, Sq, D = q.shape
@@ -108,6 +112,10 @@ def attn_pv(p, v, seq_len_list, *, causal: bool = True, q_len_list=None, zero_pa
 
     Rows of padded queries are left uninitialised unless ``zero_padding``.
     """
+    if type(seq_len_list) is SeqInfo and q_len_list is None and out is None and not zero_padding:
+        ctx = _lib.front.attn_pv(p, v, seq_len_list, causal)
+        if ctx is not None:
+            return ctx
     _lib.require_gpu(p, "p")
     vs = _bhsd(v, "v")
     if p.dim() != 4:
@@ -414,6 +422,8 @@ def kv_pages_append(k_new, v_new, k_pool, v_pool, kv_len_list, page_table, overf
     """``kv_cache_append`` for paged caches: the new ``[B,H,D]`` rows go to row ``kv_len[b] % P`` of page
     ``page_table[b, kv_len[b] // P]``.  A sequence whose next position has no page in the pool keeps its rows, loses
     the new one and is counted in ``overflow``."""
+    if type(kv_len_list) is SeqInfo and _lib.front.kv_pages_append(k_new, v_new, k_pool, v_pool, kv_len_list, page_table, overflow):
+        return
     for t, n in ((k_new, "k_new"), (v_new, "v_new")):
         _lib.require_gpu(t, n, contiguous=False)
         if t.dim() != 3 or t.stride(2) != 1:
@@ -441,6 +451,10 @@ def decode_attn_paged(q, k_pool, v_pool, kv_len_list, page_table, *, scale: Opti
     """``decode_attn`` over paged caches: position ``j`` of sequence ``b`` is row ``j % P`` of page
     ``page_table[b, j // P]`` of the ``[pages, H, P, D]`` pools (``P`` a power of two, at least 16).  ``[B,H,1,D]``.
     A page id outside the pool reads as zeros."""
+    if type(kv_len_list) is SeqInfo and out is None and workspace is None and split:
+        ctx = _lib.front.decode_attn_paged(q, k_pool, v_pool, kv_len_list, page_table, scale)
+        if ctx is not None:
+            return ctx
     _lib.require_gpu(q, "q", contiguous=False)
     ks = _pool(k_pool, "k_pool")
     vs = _pool(v_pool, "v_pool")

@@ -55,6 +55,10 @@ def layer_norm_forward(input, weight, bias, normalized_shape, eps=1e-5, residual
     ``t`` is row ``t + offsets[t]`` of ``residual``, i.e. it is read straight from the padded ``[B,S,hid]``
     activations and no depad copy is needed.
     """
+    if not return_stats and not return_sum and residual_row_offsets is None:
+        output = _lib.front.layer_norm(input, weight, bias, normalized_shape, eps, residual)
+        if output is not None:
+            return output
     if isinstance(normalized_shape, numbers.Integral):
         normalized_shape = (normalized_shape,)
     _lib.require_gpu(input, "input", contiguous=False)

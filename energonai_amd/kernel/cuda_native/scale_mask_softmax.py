@@ -26,7 +26,7 @@ from __future__ import annotations
 import torch
 
 from ... import _lib
-from ...seqinfo import seq_info
+from ...seqinfo import SeqInfo, seq_info
 
 try:
     _lib.load()
@@ -36,6 +36,10 @@ except RuntimeError as _exc:
 
 def scale_mask_softmax(batch_size, batch_seq_len, head_num, src, seq_len_list, *, scale=1.0, causal=True,
                        k_seq_len=None, q_len_list=None, tail_rows=0):
+    if type(seq_len_list) is SeqInfo and k_seq_len is None and q_len_list is None and \
+            type(batch_size) is type(batch_seq_len) is type(head_num) is type(tail_rows) is int and \
+            _lib.front.scale_mask_softmax(src, seq_len_list, batch_size, batch_seq_len, head_num, scale, causal, tail_rows):
+        return src
     _lib.require_gpu(src, "correlation", contiguous=False)
     if src.dtype not in (torch.float32, torch.float16, torch.bfloat16):
         raise RuntimeError("Datatype not implemented")

@@ -54,6 +54,10 @@ def transpose_pad(src, batch_size, max_seq_len, seq_len_list, head_num, size_per
     new tensor uninitialised: for callers whose consumers are bounded by the sequence lengths, as the attention
     kernels of this package are.
     """
+    if type(seq_len_list) is SeqInfo and zero_padding and type(batch_size) is type(max_seq_len) is type(head_num) is type(size_per_head) is int:
+        dst = _lib.front.transpose_pad(src, seq_len_list, batch_size, max_seq_len, head_num, size_per_head)
+        if dst is not None:
+            return dst
     src = src.contiguous()
     _lib.require_gpu(src, "src")
     info = seq_info(seq_len_list, batch_size, src.device)
@@ -75,6 +79,11 @@ def transpose_pad(src, batch_size, max_seq_len, seq_len_list, head_num, size_per
 
 def transpose_depad(src, batch_size, sum_seq, max_seq_len, seq_len_list, head_num, size_per_head):
     """[B,H,S,D] -> [1,T,H,D]  (transpose_pad.py:21-27)."""
+    if type(seq_len_list) is SeqInfo and \
+            type(batch_size) is type(sum_seq) is type(max_seq_len) is type(head_num) is type(size_per_head) is int:
+        dst = _lib.front.transpose_depad(src, seq_len_list, batch_size, sum_seq, max_seq_len, head_num, size_per_head)
+        if dst is not None:
+            return dst
     src = src.contiguous()
     _lib.require_gpu(src, "src")
     info = seq_info(seq_len_list, batch_size, src.device)
@@ -97,6 +106,10 @@ def depad(src, batch_size, seq_lens, left_padded=False, sum_seq=None):
     read from the device once per distinct ``seq_lens`` (the reference's slicing
     with tensor lengths synchronises on every sequence).
     """
+    if type(seq_lens) is SeqInfo and type(batch_size) is int and type(sum_seq) is int:
+        dst = _lib.front.depad(src, seq_lens, batch_size, left_padded, sum_seq)
+        if dst is not None:
+            return dst
     _lib.require_gpu(src, "src", contiguous=False)
     src = src.contiguous()
     if src.dim() != 3:

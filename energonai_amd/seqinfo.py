@@ -49,7 +49,7 @@ class SeqInfo:
     """Device-resident int32 lengths and exclusive prefix for one batch."""
 
     __slots__ = ("lens", "cu_seqlens", "batch_size", "_total", "_source", "_row_offsets", "_tile_tables", "_arrivals", "_ready",
-                 "_last_tables", "_ordered", "ephemeral", "_lens_host")
+                 "_last_tables", "_last_table", "_ordered", "ephemeral", "_lens_host")
 
     def __init__(self, lens: torch.Tensor, cu_seqlens: torch.Tensor, batch_size: int, total: Optional[int], source):
         self.lens = lens                # int32 [B] on the device
@@ -60,6 +60,7 @@ class SeqInfo:
         self._row_offsets = {}          # (max_seq_len, left_padded, version of lens) -> int32 [T]
         self._tile_tables = {}          # (head_num, q_seq_len, order, version of lens, tile height) -> int32 workgroup order
         self._last_tables = None        # (what layer_tables was asked for, row offsets, tile table): the last it found
+        self._last_table = None         # (what tile_table was asked for, tile table): the last it found
         self._arrivals = {}             # (bucket, stream) -> int64 meeting words of en_attn_fused_norm
         self._ready = []                # events recorded behind the kernels that produced the arrays above
         self._ordered = set()           # raw streams already ordered behind every event of _ready
@@ -192,6 +193,11 @@ class SeqInfo:
         tile height of the kernel that will read the table (128; 256 for the fused kernel's 64-queries-per-wave form).  Computed
         once per batch, head count, bucket, order and tile height by one small kernel and reused by every layer."""
         version = self._lens_version()
+        call = (head_num, q_seq_len, unit_kv_bytes, query_tile, causal, version)
+        found = self._last_table        # QK^T and PV of every layer ask for the same one
+        if found is not None and found[0] == call:
+            self.order_current_stream()
+            return found[1]
         first = tiles_first(self.batch_size * int(head_num), int(unit_kv_bytes), causal)
         key = (int(head_num), int(q_seq_len), first, version, int(query_tile))
         tab = None if version is None and self._mutable() else self._tile_tables.get(key)
@@ -207,6 +213,8 @@ class SeqInfo:
                 # tables of older versions of the lengths can never be found again: drop them
                 self._tile_tables = {k: t for k, t in self._tile_tables.items() if k[3] == version}
                 self._tile_tables[key] = tab
+        if version is not None or not self._mutable():
+            self._last_table = (call, tab)
         return tab
 
 

@@ -267,3 +267,105 @@ def test_yardstick_kernels_touch_exactly_their_pattern():
                 assert bool((buf.cpu()[touched] == 0).all()) and torch.equal(buf.cpu()[~touched], src.cpu()[~touched])
             if mode == 3:
                 assert torch.equal(out.cpu()[touched], src.cpu()[touched]) and bool((out.cpu()[~touched] == 5.0).all())
+
+
+NATIVE_OPS = ("layer_norm", "kv_pages_append", "decode_attn_paged", "depad", "transpose_pad", "transpose_depad", "scale_mask_softmax",
+              "attn_qk", "attn_pv")
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("form", ["plain", "strided", "subclass", "side stream", "function mode"])
+def test_single_operations_give_the_same_natively_and_in_python(dtype, form, monkeypatch):
+    """Each call that has a native form against the same call with that form turned off, bit for bit, over what either accepts; what
+    one refuses the other refuses in the same words."""
+    from energonai_amd import _lib, kernel as K
+    from energonai_amd.seqinfo import build_seq_info
+    announce("native single ops", dtype, form)
+    g = torch.Generator().manual_seed(11)
+    B, S, H, D, P, lens = 3, 23, 5, 64, 16, [23, 1, 17]
+    T, hid = sum(lens), 5 * 64
+
+    def rnd(*shape):
+        t = torch.randn(*shape, generator=g).to(dtype).cuda()
+        if form == "strided" and len(shape) > 1:      # rows further apart than they are long
+            return torch.cat([t, t], -1)[..., :shape[-1]]
+        return t.as_subclass(_Sub) if form == "subclass" else t
+
+    x, qkv, w, b = rnd(B, S, hid), rnd(1, T, H, 3 * D), rnd(hid), rnd(hid)
+    q1, kn, vn = rnd(B, H, 1, D), rnd(B, H, D), rnd(B, H, D)
+    pools = [torch.randn(7, H, P, D, generator=g).to(dtype).cuda() for _ in range(2)]
+    table = torch.tensor([[3, 5], [0, -1], [6, 1]], dtype=torch.int32).cuda()
+    lens_gpu = torch.tensor(lens, dtype=torch.int32).cuda()
+    over = torch.zeros(1, dtype=torch.int32).cuda()
+
+    def run():
+        info = build_seq_info(lens_gpu, B, total=T)
+        if form == "side stream":      # the lengths are ready on another stream than the one the calls run on
+            side = torch.cuda.Stream()
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                out = ops(info)
+            torch.cuda.current_stream().wait_stream(side)
+            torch.cuda.synchronize()
+            return out
+        if form == "function mode":
+            class Seen(torch.overrides.TorchFunctionMode):
+                def __torch_function__(self, func, types, args=(), kwargs=None):
+                    return func(*args, **(kwargs or {}))
+            with Seen():
+                return ops(info)
+        return ops(info)
+
+    def ops(info):
+        rows = K.depad(x, B, info, left_padded=True, sum_seq=T)
+        q, k, v = torch.chunk(K.transpose_pad(qkv, B, S, info, H, 3 * D), 3, dim=-1)
+        probs = K.scale_mask_softmax(B, S, H, K.attn_qk(q, k, info, alpha=0.5).nan_to_num(0, 0, 0), info, scale=0.125)
+        ctx = K.transpose_depad(K.attn_pv(probs, v, info), B, T, S, info, H, D)
+        mine = [p.clone() for p in pools]
+        K.kv_pages_append(kn, vn, *mine, info, table, over)
+        paged = K.decode_attn_paged(q1, *mine, info, table)
+        y = K.layer_norm_forward(ctx.view(1, T, hid), w, b, (hid,), 1e-5, residual=rows)
+        plain_y = K.layer_norm_forward(rows, w, b, hid)
+        wide = K.layer_norm_forward(rows.float(), w, b, torch.Size([hid]), 1e-3)
+        refused = []
+        for call in (lambda: K.layer_norm_forward(rows, w, b, (hid + 8,)), lambda: K.layer_norm_forward(rows, w.double(), b.double(), (hid,)),
+                     lambda: K.layer_norm_forward(rows, w, b, (hid,), residual=rows[:, :-1]), lambda: K.attn_qk(q, k[:, :-1], info),
+                     lambda: K.attn_pv(probs, v.double(), info), lambda: K.transpose_pad(qkv.cpu(), B, S, info, H, 3 * D),
+                     lambda: K.transpose_depad(ctx, B, T, S, info, H, D), lambda: K.depad(rows[0], B, info, sum_seq=T),
+                     lambda: K.decode_attn_paged(q1, mine[0], mine[1][:-1], info, table), lambda: K.kv_pages_append(kn[:2], vn, *mine, info, table),
+                     lambda: K.decode_attn_paged(q1, *mine, info, table.long()), lambda: K.scale_mask_softmax(B, S, H + 1, probs, info)):
+            with pytest.raises(RuntimeError) as e:
+                call()
+            refused.append(str(e.value))
+        return [rows, ctx, *mine, paged, y, plain_y, wide], refused
+
+    native, native_refused = run()
+
+    class General:
+        def __getattr__(self, name):
+            return (lambda *args: None) if name in NATIVE_OPS else getattr(front, name)
+
+    front = _lib.front
+    monkeypatch.setattr(_lib, "front", General())
+    general, general_refused = run()
+    torch.cuda.synchronize()
+    assert native_refused == general_refused
+    for got, want in zip(native, general):
+        assert got.shape == want.shape and got.dtype == want.dtype and torch.equal(torch.Tensor(got), torch.Tensor(want))
+
+
+def test_which_operands_a_native_operation_takes():
+    """The native forms take plain operands and leave everything else, with nothing launched, to the Python calls."""
+    from energonai_amd import _lib
+    announce("native operands")
+    x, w = torch.randn(4, 64).half().cuda(), torch.randn(64).half().cuda()
+    take = lambda *a: _lib.front.layer_norm(*a) is not None
+    assert take(x, w, w, (64,), 1e-5, None) and take(x, w, w, 64, 1e-5, x) and take(x.float(), w, w, (64,), 1, None)
+    for args in ((x.t().contiguous().t(), w, w, (64,), 1e-5, None), (x.as_subclass(_Sub), w, w, (64,), 1e-5, None), (x.cpu(), w, w, (64,), 1e-5, None),
+                 (x, w.float(), w.float(), (64,), 1e-5, None), (x, w, w.float(), (64,), 1e-5, None), (x, w, w, (4, 64), 1e-5, None),
+                 (x, w, w, (32,), 1e-5, None), (x, w, w, (64,), "1e-5", None), (x, w, w, (64,), 1e-5, x.float()), (x[:0], w, w, (64,), 1e-5, None)):
+        assert not take(*args)
