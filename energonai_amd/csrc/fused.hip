@@ -69,6 +69,12 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
   constexpr int KLOADS = BK * KVEC_ROW / kBlock; // direct-load instructions per wave and tile, for each of K and V
   constexpr float kLog2e = 1.4426950408889634f;
   constexpr int NVB = DP <= 96 ? 2 : 1;          // V buffers
+  // Q is read once, and non-temporal it leaves the caches to what is read again, K and V by the unit's other tiles and the context
+  // by the LayerNorm.  Layers in us, cached / non-temporal: 4 of 16 sequences of up to 1024, 56 heads x 128 986 / 980, 6 of 32 of up to
+  // 256, 16 x 128 231 / 225, 4 of 8 of up to 512, 32 x 128 206 / 201, 4 of 7 of up to 1531, 20 x 80 316 / 315.  With the LayerNorm in
+  // the launch, where K and V of all tiles come in at once, it loses (4 of 4 of up to 700, 16 x 128 114 / 116), and at 64 channels (12
+  // of 39 of up to 557, 5 x 64 304 / 316).
+  constexpr int QAUX = DP > 64 && !NORM ? 2 : 0;
   static_assert(DP == 64 || DP == 96 || DP == 128, "swizzles are written for 8, 12 or 16 slots per row");
   static_assert(NVS * 16 <= DP, "a step reads channels the tile has");
   static_assert(BK * KVEC_ROW % kBlock == 0 && 32 * KVEC_ROW % kWave == 0, "tiles must divide over the block");
@@ -127,7 +133,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
       const int c = slot ^ kswz(rr);
       const int qq = q0 + wave * 32 + rr;
       const uint32_t off = (uint32_t)(((int64_t)qq * a.q_ss + c * EPV) * E::kSize);
-      buffer_load16_to_lds(q_desc, lds_address(q_stage) + n * kWave * 16, ((unsigned)qq < (unsigned)ql && c * EPV < a.D) ? off : kOutOfRange);
+      buffer_load16_to_lds<QAUX>(q_desc, lds_address(q_stage) + n * kWave * 16, ((unsigned)qq < (unsigned)ql && c * EPV < a.D) ? off : kOutOfRange);
     }
   }
 
