@@ -55,6 +55,8 @@ SIGNATURES = {
     "en_attn_fused_norm_pays": (c_int, [c_int] * 4 + [c_int64, c_int]),
     "en_attn_fused_norm": (c_int, [c_void_p] * 4 + [c_int] * 4 + [c_int64, c_float, c_int, c_int] + [c_void_p] * 6 +
                            [c_float, c_void_p, c_int, c_void_p]),
+    "en_attn_fused_f32_wide_pays": (c_int, [c_int] * 4),
+    "en_attn_fused_f32_wide": (c_int, [c_void_p] * 4 + [c_int] * 4 + [c_float, c_int, c_void_p]),
     "en_attn_fused_query_tile": (c_int, [c_int] * 5),
     "en_packed_scores_elems": (c_int64, [c_int] * 4),
     "en_scale_mask_softmax_packed": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_void_p]),

@@ -247,6 +247,225 @@ __global__ __launch_bounds__(kBlock) void attn_fused_f32_kernel(FusedArgs fa) { 
 template <int DP>
 __global__ __launch_bounds__(kBlock) void attn_fused_norm_f32_kernel(FusedArgs fa, NormArgs norm) { fused_f32_tile<DP, true>(fa, &norm); }
 
+// Heads of 65..128 channels.  Bound by the matrix cores: a wave's share of a 64-key tile is 2 x 64 MFMAs of 64 cycles, and the loads,
+// the softmax and the LDS reads of one workgroup run beside the MFMAs of the other on its CU.  The same split as above (64 query
+// rows, wave (wq, wk) takes 32 of them and 32 keys of every tile, the pair is combined at the end), but the tiles travel from
+// memory straight into LDS, one buffer each for K and V: V of a tile is sent for at the top of its step and needed behind S^T, K of
+// the next one behind the barrier in mid-step, when every wave has left this one's, and needed at the end.  64 KB (48 at 96
+// channels) and no registers for tiles in flight: two workgroups (three) on a CU.  2 sequences of 375..1500, 16 heads x 128, causal,
+// with the LayerNorm: 229 us in four launches, 136 in two; 22 of 110, 45 x 128: 260 -> 137.
+//
+// Rows are DP channels without padding; chunk c (16 bytes) of a K row r sits in slot c ^ kswz(r), so that the fragment reads of
+// sixteen consecutive rows at one chunk cover all banks; V is read a channel a lane, rows four keys apart in the wave's halves: with
+// rows of 512 bytes every key's chunks 8..15 and 0..7 trade places for keys with bit 2 set, rows of 384 bytes lie 32 banks apart,
+// and there such keys trade places with their neighbour.
+template <int DP>
+__global__ __launch_bounds__(kBlock, DP == 96 ? 3 : 2) void attn_fused_f32_wide_kernel(FusedArgs fa) {
+  typedef float T;
+  typedef Mma<EN_F32> M;
+  const AttnArgs &a = fa.base;
+  constexpr int EPV = 4, BK = 64, NVS = DP / M::KPV, DMT = DP / 32, CPR = DP / EPV, LOADS = BK * CPR / kBlock;
+  constexpr float kLog2e = 1.4426950408889634f;
+  static_assert(DP == 96 || DP == 128, "swizzles are written for 24 or 32 slots per row");
+  __shared__ __attribute__((aligned(16))) float lds[2 * BK * DP];
+  float *const lds_k = lds, *const lds_v = lds + BK * DP;
+  static_assert(2 * (2 + DMT * 16) * kWave <= 2 * BK * DP, "the pairs are combined in the tiles' room");
+  auto kswz = [](int row) { return DP == 128 ? (row & 15) : ((row >> 1) & 7); };
+  auto vflip = [](int key) { return (key >> 2) & 1; };
+
+  const SeqAhead ahead = seq_ahead(a, fa.q_row0, fa.k_row0);
+  int unit, qi;
+  if (!map_block(a, unit, qi)) return;
+  const int b = unit / a.H, h = unit % a.H;
+  const Seq seq = seq_of(a, ahead, b, fa.q_row0, fa.k_row0);
+  const int kl = seq.kl, ql = seq.ql;
+  const int q0 = qi * kF32QTile;
+  if (q0 >= ql) return;
+  const int nk = tile_key_extent(a, min(q0 + kF32QTile, ql) - 1, kl, ql);
+  const int nkt = (nk + BK - 1) / BK;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, g = lane >> 5;
+  const int wq = wave & 1, wk = wave >> 1;
+  const int q_first = q0 + wq * 32, q_lane = q_first + r;
+  // keys this lane's query may see, and the wave's smallest and largest such extent
+  const int vis_l = (q_lane < ql) ? (a.causal ? min(kl, q_lane + (kl - ql) + 1) : kl) : 0;
+  const int vis_min = (q_first + 31 < ql) ? (a.causal ? min(kl, q_first + (kl - ql) + 1) : kl) : 0;
+  const int vis_max = (q_first < ql) ? (a.causal ? min(kl, min(q_first + 31, ql - 1) + (kl - ql) + 1) : kl) : 0;
+
+  const int64_t qr = seq.q_row, kr = seq.k_row;
+  const T *qbase = reinterpret_cast<const T *>(a.a_ptr) + (int64_t)b * a.q_sb + qr * a.q_ss + (int64_t)h * a.q_sh;
+  const T *kbase = reinterpret_cast<const T *>(a.b_ptr) + (int64_t)b * a.k_sb + kr * a.k_ss + (int64_t)h * a.k_sh;
+  const T *vbase = reinterpret_cast<const T *>(fa.v) + (int64_t)b * fa.v_sb + kr * fa.v_ss + (int64_t)h * fa.v_sh;
+  T *cbase = reinterpret_cast<T *>(a.out) + (int64_t)b * fa.c_sb + qr * fa.c_ss + (int64_t)h * fa.c_sh;
+
+  // K / V tiles: the descriptors end with the last valid key, so rows past it arrive as zeros
+  const desc_t k_desc = make_desc(kbase, kl > 0 ? (uint32_t)(((int64_t)(kl - 1) * a.k_ss + a.D) * 4) : 0u);
+  const desc_t v_desc = make_desc(vbase, kl > 0 ? (uint32_t)(((int64_t)(kl - 1) * fa.v_ss + a.D) * 4) : 0u);
+  const uint32_t k_row_bytes = (uint32_t)(a.k_ss * 4), v_row_bytes = (uint32_t)(fa.v_ss * 4);
+  uint32_t k_off[LOADS], v_off[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = (i * kBlock + tid) / CPR, slot = (i * kBlock + tid) % CPR;
+    const int k_c = slot ^ kswz(row), v_c = DP == 128 ? slot ^ (8 * vflip(row)) : slot, v_key = DP == 128 ? row : row ^ vflip(row);
+    k_off[i] = k_c * EPV < a.D ? row * k_row_bytes + k_c * 16 : kOutOfRange;
+    v_off[i] = v_c * EPV < a.D ? v_key * v_row_bytes + v_c * 16 : kOutOfRange;
+  }
+  auto fetch = [&](const desc_t &desc, const float *dst, uint32_t (&off)[LOADS], uint32_t row_bytes) {
+    const uint32_t at = lds_address(dst) + wave * kWave * 16;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      buffer_load16_to_lds(desc, at + i * kBlock * 16, off[i]);
+      off[i] += BK * row_bytes;
+    }
+  };
+  fetch(k_desc, lds_k, k_off, k_row_bytes);
+
+  // Q fragments: this lane's query row, four channels per step (rows past the last valid one are never stored)
+  uint4 qf[NVS];
+  {
+    const T *qrow = qbase + (int64_t)min(q_lane, ql - 1) * a.q_ss;
+#pragma unroll
+    for (int vs = 0; vs < NVS; ++vs) {
+      const int d = M::k_of(vs, g, NVS);
+      qf[vs] = (d < a.D) ? *reinterpret_cast<const uint4 *>(qrow + d) : zero4();
+    }
+  }
+
+  floatx16 o[DMT];
+#pragma unroll
+  for (int mt = 0; mt < DMT; ++mt)
+#pragma unroll
+    for (int x = 0; x < 16; ++x) o[mt][x] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  const float c_exp = fa.scale * kLog2e;
+  const float lazy_gap = 8.0f / c_exp;
+  const int ksw = kswz(r);
+  const float *const krow = lds_k + (wk * 32 + r) * DP;          // wk * 32 leaves the swizzle of a row alone
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  lds_barrier();
+
+  for (int kt = 0; kt < nkt; ++kt) {
+    fetch(v_desc, lds_v, v_off, v_row_bytes);     // V tile kt: its room was in use until the barrier that ended the step before
+    const int k0 = kt * BK + wk * 32;             // first key of this wave's block
+    const bool live = k0 < vis_max;               // wave-uniform
+    floatx16 s;
+    if (live) {
+      // ---- S^T = K Q^T, the fragments read a step ahead
+#pragma unroll
+      for (int x = 0; x < 16; ++x) s[x] = 0.f;
+      uint4 kf[2];
+      auto load_step = [&](int vs) { return *reinterpret_cast<const uint4 *>(krow + ((M::k_of(vs, g, NVS) / EPV) ^ ksw) * EPV); };
+      kf[0] = load_step(0);
+#pragma unroll
+      for (int vs = 0; vs < NVS; ++vs) {
+        if (vs + 1 < NVS) kf[(vs + 1) & 1] = load_step(vs + 1);
+        M::step(kf[vs & 1], qf[vs], s);
+      }
+
+      // ---- mask + online softmax; register 4j+i holds key k0 + 8j + 4g + i of this lane's query
+      float m_tile = -INFINITY;
+      if (k0 + 32 <= vis_min) {
+#pragma unroll
+        for (int x = 0; x < 16; ++x) m_tile = fmaxf(m_tile, s[x]);
+      } else {
+        const int lim = vis_l - k0 - 4 * g;
+#pragma unroll
+        for (int x = 0; x < 16; ++x) {
+          const float v = (8 * (x >> 2) + (x & 3) < lim) ? s[x] : -INFINITY;
+          s[x] = v;
+          m_tile = fmaxf(m_tile, v);
+        }
+      }
+      float lo, hi;
+      halves_of(m_tile, lo, hi);
+      m_tile = fmaxf(lo, hi);
+      if (__builtin_amdgcn_ballot_w64(m_tile - lazy_gap > m_run) != 0) {
+        const float m_new = fmaxf(m_run, m_tile);
+        const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m_new) * c_exp);
+        l_run *= alpha;
+#pragma unroll
+        for (int mt = 0; mt < DMT; ++mt)
+#pragma unroll
+          for (int x = 0; x < 16; ++x) o[mt][x] *= alpha;
+        m_run = m_new;
+      }
+      const float moff = (m_run == -INFINITY) ? 0.f : -m_run * c_exp;
+      float l_tile = 0.f;
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        s[x] = __builtin_amdgcn_exp2f(fmaf(s[x], c_exp, moff));       // exp2(-inf) = 0: masked keys
+        l_tile += s[x];
+      }
+      l_run += l_tile;                            // each half of the wave adds up its own keys
+    }
+
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();                                // V tile kt is there, K tile kt has been read
+    fetch(k_desc, lds_k, k_off, k_row_bytes);     // K tile kt + 1 (past the end: zeros, no traffic)
+    if (live) {
+      // ---- O^T += V^T P^T: step (j, i) contracts over keys 8j + i (lanes 0..31) and 8j + 4 + i (lanes 32..63)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint4 pb = make_uint4(__float_as_uint(s[4 * j]), __float_as_uint(s[4 * j + 1]), __float_as_uint(s[4 * j + 2]),
+                                    __float_as_uint(s[4 * j + 3]));
+        // keys 8 j + 4 g + i: bit 2 is g
+        auto v_at = [&](int i, int mt) {
+          const int key = wk * 32 + 8 * j + 4 * g + i;
+          return __float_as_uint(DP == 128 ? lds_v[key * DP + ((mt * 32) ^ (32 * g)) + r] : lds_v[(key ^ g) * DP + mt * 32 + r]);
+        };
+#pragma unroll
+        for (int mt = 0; mt < DMT; ++mt) M::step(make_uint4(v_at(0, mt), v_at(1, mt), v_at(2, mt), v_at(3, mt)), pb, o[mt]);
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();                                // K tile kt + 1 is there, V tile kt has been read
+  }
+
+  // ---- combine the two waves of a query half (they saw disjoint keys), then normalise and store.
+  float l_lo, l_hi;
+  halves_of(l_run, l_lo, l_hi);
+  l_run = l_lo + l_hi;
+  float *comb = lds + wq * (2 + DMT * 16) * kWave;
+  if (wk == 1) {
+    comb[lane] = m_run;
+    comb[kWave + lane] = l_run;
+#pragma unroll
+    for (int mt = 0; mt < DMT; ++mt)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) comb[(2 + mt * 16 + x) * kWave + lane] = o[mt][x];
+  }
+  lds_barrier();
+  if (wk == 1 || q_lane >= ql) return;
+  const float m1 = comb[lane], l1 = comb[kWave + lane];
+  const float m = fmaxf(m_run, m1);
+  const float w0 = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m) * c_exp);
+  const float w1 = (m1 == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m1 - m) * c_exp);
+  const float l = l_run * w0 + l1 * w1;
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  T *crow = cbase + (int64_t)q_lane * fa.c_ss;
+#pragma unroll
+  for (int mt = 0; mt < DMT; ++mt)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int d = mt * 32 + 8 * j + 4 * g;
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (o[mt][4 * j + i] * w0 + comb[(2 + mt * 16 + 4 * j + i) * kWave + lane] * w1) * inv;
+      if (d < a.D) *reinterpret_cast<float4 *>(crow + d) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+}
+
+static int launch_fused_f32_wide(const FusedArgs &fa, hipStream_t s) {
+  const AttnArgs &a = fa.base;
+  const unsigned grid = (unsigned)(ceil_div(a.units, kXcds) * kXcds * a.ntq);
+  if (a.D <= 96) attn_fused_f32_wide_kernel<96><<<grid, kBlock, 0, s>>>(fa);
+  else attn_fused_f32_wide_kernel<128><<<grid, kBlock, 0, s>>>(fa);
+  EN_RETURN_IF_LAUNCH_FAILED();
+  return EN_OK;
+}
+
 int launch_fused_f32(FusedArgs &fa, const NormArgs *norm, hipStream_t s) {
   const AttnArgs &a = fa.base;
   if (a.units > 65535) return EN_ERR_SHAPE;
@@ -258,3 +477,45 @@ int launch_fused_f32(FusedArgs &fa, const NormArgs *norm, hipStream_t s) {
 }
 
 }  // namespace en
+
+extern "C" {
+
+int en_attn_fused_f32_wide_pays(int batch, int head_num, int max_seq_len, int size_per_head) {
+  if (batch < 1 || head_num < 1 || max_seq_len < 1 || size_per_head <= 64 || size_per_head > 128 || size_per_head % 4) return 0;
+  // us a layer, QK^T + softmax + PV / this, with the LayerNorm behind either: 1 prompt of 64, 12 heads x 128 28 / 18, 4 of up to 128, 8 x
+  // 80 39 / 21, 8 of up to 128, 16 x 96 43 / 23, 1 of 1000, 4 x 128 155 / 76, 4 of up to 512, 12 x 96 103 / 49, 22 of 110, 45 x 128 260 / 137,
+  // 16 of up to 384, 20 x 80, no mask 199 / 128.  It is the faster form at every size; the line is where the scores of the three
+  // kernels pass 2 MiB, below which the step keeps giving the bits of the separate calls, as a caller who compares the two expects.
+  return 4.0 * batch * head_num * max_seq_len * max_seq_len > 2.0 * (1 << 20);
+}
+
+int en_attn_fused_f32_wide(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
+                           int max_seq_len, int size_per_head, float scale, int causal, en_stream_t stream) {
+  using namespace en;
+  if (!qkv || !ctx || !seq_lens || !cu_seqlens) return EN_ERR_NULL;
+  if (batch < 1 || head_num < 1 || max_seq_len < 1 || size_per_head < 1) return EN_ERR_SHAPE;
+  if (size_per_head <= 64 || size_per_head > 128 || size_per_head % 4 || !(scale > 0.f)) return EN_ERR_UNSUPPORTED;
+  if (!aligned_to(qkv, 16) || !aligned_to(ctx, 16)) return EN_ERR_ALIGN;
+  const int64_t D = size_per_head, row = (int64_t)3 * head_num * D;
+  if ((int64_t)batch * head_num > INT32_MAX / 64) return EN_ERR_SHAPE;
+  // 32-bit byte offsets, advanced a tile at a time up to two tiles past the end, and a grid of 32 bits
+  if (((int64_t)max_seq_len + 256) * row * 4 >= (1ll << 31)) return EN_ERR_UNSUPPORTED;
+  FusedArgs fa{};
+  AttnArgs &a = fa.base;
+  const float *pk = static_cast<const float *>(qkv);
+  a.a_ptr = pk; a.b_ptr = pk + D; a.out = ctx; a.k_lens = seq_lens;
+  a.B = batch; a.H = head_num; a.Sq = max_seq_len; a.Sk = max_seq_len; a.D = size_per_head;
+  a.q_sh = a.k_sh = fa.v_sh = 3 * D;
+  a.q_ss = a.k_ss = fa.v_ss = row;
+  a.alpha = 1.f; a.causal = causal ? 1 : 0;
+  a.ntq = (int)ceil_div(max_seq_len, kF32QTile);
+  a.units = batch * head_num;
+  fa.v = pk + 2 * D;
+  fa.c_sh = D; fa.c_ss = head_num * D;
+  fa.q_row0 = fa.k_row0 = cu_seqlens;
+  fa.scale = scale;
+  if (ceil_div(a.units, kXcds) * kXcds * a.ntq > INT32_MAX) return EN_ERR_SHAPE;
+  return launch_fused_f32_wide(fa, (hipStream_t)stream);
+}
+
+}  // extern "C"

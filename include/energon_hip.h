@@ -365,6 +365,14 @@ int en_attn_fused(const void *q, const void *k, const void *v, void *ctx, const 
                   const int64_t *c_strides, const int32_t *q_row_offsets, const int32_t *k_row_offsets, float scale,
                   int causal, int dtype, const int32_t *tile_table, int query_tile, en_stream_t stream);
 
+/* Attention of a self-attention batch of fp32 heads of 65..128 channels (a multiple of 4) in one kernel: qkv [T, head_num,
+ * 3 size_per_head] and ctx [T, head_num, size_per_head] are packed, both on 16 bytes, scale is positive.  Not en_attn_qk,
+ * en_scale_mask_softmax and en_attn_pv to the bit: no score is stored and the sums run in another order.  _pays: 1 where the step
+ * takes it by itself, 0 where it takes those three. */
+int en_attn_fused_f32_wide_pays(int batch, int head_num, int max_seq_len, int size_per_head);
+int en_attn_fused_f32_wide(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
+                           int max_seq_len, int size_per_head, float scale, int causal, en_stream_t stream);
+
 /* Workgroup order for en_attn_qk, en_attn_pv and en_attn_fused on one batch of sequences (no counterpart in the
  * reference, whose callers run torch.matmul): table gets en_attn_tile_table_elems(batch, head_num, q_seq_len,
  * query_tile) int32 entries that list the query tiles of query_tile rows (128, or 256 for en_attn_fused with that

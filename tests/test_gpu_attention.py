@@ -7,7 +7,7 @@ fp32: 1e-5 relative to the score scale.
 import pytest
 import torch
 
-from gpu_util import BASE, announce, assert_ctx_close, assert_stored_close, max_abs, pad_bhsd, packed_randn
+from gpu_util import BASE, announce, assert_ctx_close, assert_stored_close, excess, max_abs, pad_bhsd, packed_randn
 from oracle import eager
 
 pytestmark = pytest.mark.gpu
@@ -902,3 +902,71 @@ def test_tile_table_of_256_row_tiles():
     got = [c for c in tab if c >= 0]
     assert len(got) == len(set(got)) and set(got) == want
     assert len(tab) == -(-B * H // 8) * 8 * ntq
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("lens,S,H,D", [
+    ([1], 1, 1, 68),                                        # one row, 17 chunks of 24
+    ([64, 65, 63, 0, 128], 130, 3, 80),                     # edges of the tiles, a sequence of no rows
+    ([33, 200], 201, 2, 96),                                # all 24 chunks
+    ([31, 97, 96], 97, 5, 100),                             # 25 of 32
+    ([129, 5, 64, 300], 300, 9, 128),                       # more units than XCDs
+    ([40] * 70, 41, 2, 72),                                 # more sequences than a wave's lanes
+])
+def test_attn_fused_f32_wide(lens, S, H, D, causal):
+    """The fp32 kernel for heads of 65..128 channels on packed projections against the float64 reference, with what lies behind
+    the batch's last row not to be read."""
+    from energonai_amd import _lib
+    from energonai_amd.seqinfo import build_seq_info
+    announce("fused f32 wide", lens[:6], S, H, D, causal)
+    T, B = sum(lens), len(lens)
+    qkv = torch.full((T + 64, H, 3 * D), float("nan"))
+    qkv[:T] = packed_randn(T, H * 3 * D, torch.float32, 17 + S).reshape(T, H, 3 * D)
+    scale = D ** -0.5
+    want, t = torch.zeros(T, H, D, dtype=torch.float64), 0
+    for n in lens:
+        q, k, v = (x.permute(1, 0, 2).double() for x in torch.chunk(qkv[t:t + n], 3, dim=-1))
+        s = scale * q @ k.transpose(1, 2)
+        if causal:
+            s = s.masked_fill(torch.ones(n, n, dtype=torch.bool).triu(1), float("-inf"))
+        want[t:t + n] = (torch.softmax(s, -1) @ v).permute(1, 0, 2)
+        t += n
+    info = build_seq_info(torch.tensor(lens, dtype=torch.int32).cuda(), B, total=T)
+    gpu, ctx = qkv.cuda(), torch.full((T + 1, H, D), 7.0).cuda()
+    _lib.check(_lib.fn.en_attn_fused_f32_wide(gpu.data_ptr(), ctx.data_ptr(), info.lens.data_ptr(), info.cu_seqlens.data_ptr(), B, H, S, D, scale,
+                                              int(causal), _lib.stream_of(gpu)), "attn_fused_f32_wide")
+    assert bool((ctx[T] == 7.0).all())
+    # half a unit in the last place of the result and the sums of n products in fp32
+    assert excess(ctx[:T].cpu(), want, torch.float32) <= BASE[torch.float32]
+
+
+@pytest.mark.parametrize("dense,left,fold", [(False, True, None), (True, False, None), (False, False, False)])
+def test_layer_of_wide_fp32_heads_takes_one_kernel(dense, left, fold):
+    """The default step of a batch whose fp32 scores would pass 2 MiB: the fused kernel, against the three kernels at the
+    accuracy of either, at the sizes on both sides of the line."""
+    from energonai_amd import _lib, layer
+    announce("layer f32 wide", dense, left, fold)
+    assert _lib.fn.en_attn_fused_f32_wide_pays(4, 2, 257, 128) == 1 and _lib.fn.en_attn_fused_f32_wide_pays(4, 2, 256, 128) == 0
+    assert [_lib.fn.en_attn_fused_f32_wide_pays(64, 16, 512, d) for d in (64, 68, 70, 128, 132)] == [0, 1, 0, 1, 0]
+    B, H, S, D = 4, 16, 256, 72
+    lens = [256, 3, 130, 64]
+    T, hid = sum(lens), H * D if not dense else 200
+    g = torch.Generator().manual_seed(5)
+    x, qkv = torch.randn(B, S, hid, generator=g).cuda(), torch.randn(1, T, H, 3 * D, generator=g).cuda()
+    gamma, beta = torch.randn(hid, generator=g).cuda(), torch.randn(hid, generator=g).cuda()
+    out = torch.randn(1, T, hid, generator=g).cuda() if dense else None
+    lens_gpu = torch.tensor(lens, dtype=torch.int32).cuda()
+    ctx = [torch.zeros(1, T, H, D, device="cuda") for _ in range(2)]
+    y = [layer.padding_removal_layer(x, qkv, lens_gpu, H, D, gamma, beta, left_padded=left, dense_out=out, fused_attention=form, fold_depad=fold,
+                                     ctx_out=c) for form, c in zip((None, "varlen"), ctx)]
+    assert not torch.equal(*ctx)                            # two ways of adding up
+    assert max_abs(*ctx) <= 2 * BASE[torch.float32] and max_abs(*y) <= 2 * BASE[torch.float32] * float(y[1].abs().max())
+    assert _lib.fn.en_attn_fused_f32_wide_pays(1, H, 128, D) == 0
+    x, qkv, lens_gpu = x[:1, :128].contiguous(), qkv[:, :100].contiguous(), lens_gpu.new_tensor([100])
+    small = layer.padding_removal_layer(x, qkv, lens_gpu, H, D, gamma, beta, left_padded=left, fold_depad=fold,
+                                        dense_out=None if out is None else out[:, :100].contiguous())
+    three = layer.padding_removal_layer(x, qkv, lens_gpu, H, D, gamma, beta, left_padded=left, fold_depad=fold,
+                                        fused_attention="varlen", dense_out=None if out is None else out[:, :100].contiguous())
+    assert torch.equal(small, three)
+    with pytest.raises(KeyError):
+        layer.padding_removal_layer(x, qkv, lens_gpu, H, D, gamma, beta, dense_out=out, fused_attention="wide")
