@@ -100,6 +100,29 @@ __device__ __forceinline__ void store16(void *p, const uint4 &v) {
   }
 }
 
+// The same for an address that is aligned to its elements only: global memory takes 128-bit accesses at any element's
+// address (a wave's neighbouring lanes then share the cache lines that they straddle).
+typedef u32x4 u32x4_by2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_by4 __attribute__((aligned(4)));
+template <bool NT, int ALIGN>
+__device__ __forceinline__ uint4 load16_at(const void *p) {
+  u32x4 v;
+  if constexpr (ALIGN == 2) v = NT ? __builtin_nontemporal_load((const u32x4_by2 *)p) : *(const u32x4_by2 *)p;
+  else v = NT ? __builtin_nontemporal_load((const u32x4_by4 *)p) : *(const u32x4_by4 *)p;
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <bool NT, int ALIGN>
+__device__ __forceinline__ void store16_at(void *p, const uint4 &v) {
+  const u32x4 x = {v.x, v.y, v.z, v.w};
+  if constexpr (ALIGN == 2) {
+    if (NT) __builtin_nontemporal_store(x, (u32x4_by2 *)p);
+    else *(u32x4_by2 *)p = x;
+  } else {
+    if (NT) __builtin_nontemporal_store(x, (u32x4_by4 *)p);
+    else *(u32x4_by4 *)p = x;
+  }
+}
+
 // Buffer accesses with hardware bounds checking: a load whose offset lies outside
 // [0, bytes) returns zero and a store there is dropped, so ragged edges need no
 // branches and the compiler can count outstanding operations statically.

@@ -5,8 +5,10 @@
 // row with DPP row operations, and the whole row (probabilities, then the zero
 // tail) is written back once.  LPR lanes share a row (8..64, so short rows do
 // not idle most of a wave) and each lane holds VPL vectors of it.  Rows of
-// padded queries exit without touching memory.  Rows too long for registers,
-// or not 16-byte aligned, take the three-pass workgroup-per-row kernel.
+// padded queries exit without touching memory.  Rows that do not start on
+// 16-byte boundaries are moved by the same lanes with element-aligned 128-bit
+// accesses.  Rows too long for registers, and scales that are not positive, take
+// the three-pass workgroup-per-row kernel.
 #include "common.hip.h"
 
 #include <math.h>
@@ -75,12 +77,36 @@ constexpr int64_t kStreamSoftmaxBytes = 512ll << 20;
 // flight and the R independent reduction chains interleave.  rowp[i] is row i's first element, ri[i] its
 // geometry, l the lane's index inside its group.  Rows whose write extent lies past the LPR*VPL vectors the
 // registers hold get the rest of their zero tail from a store loop (TAIL_LOOP).
-template <int DT, int VPL, int LPR, int R, bool STREAM, bool TAIL_LOOP>
+//
+// VEC: rows start on 16-byte boundaries and are whole vectors long.  Without it the vectors of a row lie at any
+// element's address and its last one may be cut short by the row's end: that one moves by elements.
+template <int DT, int VPL, int LPR, int R, bool STREAM, bool TAIL_LOOP, bool VEC>
 __device__ __forceinline__ void softmax_lane_group(const SoftmaxArgs &a, typename Elem<DT>::T *const (&rowp)[R],
                                                    const RowInfo (&ri)[R], int l) {
   typedef Elem<DT> E;
   typedef typename E::T T;
   constexpr int EPV = 16 / E::kSize;          // elements per 128-bit vector
+  auto load_vec = [&](const T *row, int e0) -> uint4 {
+    if constexpr (VEC) return load16<STREAM>(row + e0);
+    if (e0 + EPV <= a.Sk) return load16_at<STREAM, E::kSize>(row + e0);
+    Pack<T, EPV> pk = __builtin_bit_cast(Pack<T, EPV>, make_uint4(0u, 0u, 0u, 0u));   // past the row: masked like the rest
+#pragma unroll
+    for (int e = 0; e < EPV - 1; ++e)
+      if (e0 + e < a.Sk) pk.v[e] = row[e0 + e];
+    return __builtin_bit_cast(uint4, pk);
+  };
+  auto store_vec = [&](T *row, int e0, const uint4 &v) {
+    if constexpr (VEC) {
+      store16<STREAM>(row + e0, v);
+    } else if (e0 + EPV <= a.Sk) {
+      store16_at<STREAM, E::kSize>(row + e0, v);
+    } else {
+      const Pack<T, EPV> pk = __builtin_bit_cast(Pack<T, EPV>, v);
+#pragma unroll
+      for (int e = 0; e < EPV - 1; ++e)
+        if (e0 + e < a.Sk) row[e0 + e] = pk.v[e];
+    }
+  };
   uint4 raw[R][VPL];
 #pragma unroll
   for (int i = 0; i < R; ++i) {
@@ -88,7 +114,7 @@ __device__ __forceinline__ void softmax_lane_group(const SoftmaxArgs &a, typenam
     for (int j = 0; j < VPL; ++j) {
       const int e0 = (l + LPR * j) * EPV;
       raw[i][j] = make_uint4(E::kNegInfWord, E::kNegInfWord, E::kNegInfWord, E::kNegInfWord);   // not visible: -inf
-      if (ri[i].active && e0 < ri[i].n) raw[i][j] = load16<STREAM>(rowp[i] + e0);
+      if (ri[i].active && e0 < ri[i].n) raw[i][j] = load_vec(rowp[i], e0);
     }
   }
 
@@ -110,7 +136,7 @@ __device__ __forceinline__ void softmax_lane_group(const SoftmaxArgs &a, typenam
       if (any[j]) {
         const Pack<T, EPV> pk = __builtin_bit_cast(Pack<T, EPV>, raw[i][j]);
 #pragma unroll
-        for (int e = 0; e < EPV; ++e) x[j][e] = E::to_float(pk.v[e]);
+        for (int e = 0; e < EPV; ++e) x[j][e] = VEC ? E::to_float(pk.v[e]) : E::to_float(pk.v[e]) * a.scale;
         const int nv = n - e0;                      // visible elements of this vector
         if (nv > 0 && nv < EPV) {
 #pragma unroll
@@ -123,15 +149,18 @@ __device__ __forceinline__ void softmax_lane_group(const SoftmaxArgs &a, typenam
     }
     m = group_allreduce<OpMax, LPR>(m);
     // exp(scale * (x - m)) = exp2(x * c - m * c), c = scale * log2(e) > 0 (other scales take the generic kernel)
+    // Rows off the 16-byte boundaries are scaled first and subtract before they multiply, as the generic kernel that
+    // took them before: scores near the type's lowest value then end as they did there.
     const float c = a.scale * kLog2e;
-    const float moff = (m == -INFINITY) ? 0.f : -m * c;  // nothing visible: all zeros, no NaN
+    const float msafe = (m == -INFINITY) ? 0.f : m;      // nothing visible: all zeros, no NaN
+    const float moff = -msafe * c;
     float s = 0.f;
 #pragma unroll
     for (int j = 0; j < VPL; ++j) {
       if (any[j]) {
 #pragma unroll
         for (int e = 0; e < EPV; ++e) {
-          const float ex = __builtin_amdgcn_exp2f(fmaf(x[j][e], c, moff));
+          const float ex = VEC ? __builtin_amdgcn_exp2f(fmaf(x[j][e], c, moff)) : __expf(x[j][e] - msafe);
           x[j][e] = ex;
           s += ex;
         }
@@ -149,17 +178,17 @@ __device__ __forceinline__ void softmax_lane_group(const SoftmaxArgs &a, typenam
         for (int e = 0; e < EPV; ++e) pk.v[e] = E::from_float(x[j][e] * inv);
         out = __builtin_bit_cast(uint4, pk);
       }
-      if (ri[i].active && e0 < ri[i].lim) store16<STREAM>(rowp[i] + e0, out);
+      if (ri[i].active && e0 < ri[i].lim) store_vec(rowp[i], e0, out);
     }
     if (TAIL_LOOP && ri[i].active) {
       for (int e0 = (l + LPR * VPL) * EPV; e0 < ri[i].lim; e0 += LPR * EPV)
-        store16<STREAM>(rowp[i] + e0, make_uint4(0u, 0u, 0u, 0u));
+        store_vec(rowp[i], e0, make_uint4(0u, 0u, 0u, 0u));
     }
   }
 }
 
 // Rows of up to 64 * 16 vectors, one lane-group shape for the whole launch (chosen from the row length Sk).
-template <int DT, int VPL, int LPR, int R>
+template <int DT, int VPL, int LPR, int R, bool VEC>
 __global__ __launch_bounds__(kRowsBlock) void softmax_rows_kernel(SoftmaxArgs a) {
   typedef typename Elem<DT>::T T;
   constexpr int GROUPS_PER_WAVE = kWave / LPR;
@@ -182,7 +211,7 @@ __global__ __launch_bounds__(kRowsBlock) void softmax_rows_kernel(SoftmaxArgs a)
     any |= ri[i].active;
   }
   if (__ballot(any) == 0ull) return;  // whole wave has nothing to do
-  softmax_lane_group<DT, VPL, LPR, R, false, false>(a, rowp, ri, l);
+  softmax_lane_group<DT, VPL, LPR, R, false, false, VEC>(a, rowp, ri, l);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -233,7 +262,7 @@ __device__ __forceinline__ BandLayout band_layout(const SoftmaxArgs &a, int kl, 
   return L;
 }
 
-template <int DT, int K, int R, bool STREAM>
+template <int DT, int K, int R, bool STREAM, bool VEC>
 __device__ __forceinline__ void softmax_band_wave(const SoftmaxArgs &a, typename Elem<DT>::T *unit, int q0, int q_end,
                                                   int kl, int ql, int lane) {
   typedef typename Elem<DT>::T T;
@@ -259,10 +288,10 @@ __device__ __forceinline__ void softmax_band_wave(const SoftmaxArgs &a, typename
     }
     rowp[i] = unit + (a.packed ? packed_row_start<EPV * kPackedRowVectors>(q) : (int64_t)q * a.Sk);
   }
-  softmax_lane_group<DT, kBandVpl, LPR, R, STREAM, true>(a, rowp, ri, l);
+  softmax_lane_group<DT, kBandVpl, LPR, R, STREAM, true, VEC>(a, rowp, ri, l);
 }
 
-template <int DT, int R, bool STREAM>
+template <int DT, int R, bool STREAM, bool VEC>
 __global__ __launch_bounds__(kWave) void softmax_bands_kernel(SoftmaxArgs a) {
   typedef typename Elem<DT>::T T;
   constexpr int EPV = 16 / Elem<DT>::kSize;
@@ -270,25 +299,42 @@ __global__ __launch_bounds__(kWave) void softmax_bands_kernel(SoftmaxArgs a) {
   // the heads, a few hundred at a time, instead of forming one long run of empty workgroups per batch, during
   // which the machine would drain
   const int b = blockIdx.z, h = blockIdx.y;
-  int i = blockIdx.x;
-  const int kl = min(a.k_lens[b], a.Sk);           // a key length past the row length means the whole row
+  // a key length past the row length means the whole row; rows off the 16-byte boundaries take it as it stands, as in
+  // the generic kernel: a causal row then sees as many keys more, and the row count below may pass the grid's
+  const int kl = VEC ? min(a.k_lens[b], a.Sk) : a.k_lens[b];
   const int ql = min(a.q_lens ? a.q_lens[b] : min(kl, a.Sq), a.Sq);
   if (ql <= 0) return;
   const BandLayout L = band_layout<EPV, R>(a, kl, ql);
-  if (i >= L.total) return;
   T *unit = reinterpret_cast<T *>(a.src) +
             ((int64_t)b * a.H + h) * (a.packed ? packed_row_start<EPV * kPackedRowVectors>(a.Sq) : (int64_t)a.Sq * a.Sk);
   const int lane = threadIdx.x;
-  // longest rows first
-  if (i < L.blocks[4]) return softmax_band_wave<DT, 4, R, STREAM>(a, unit, L.first[4] + i * 1 * R, L.first[5], kl, ql, lane);
-  i -= L.blocks[4];
-  if (i < L.blocks[3]) return softmax_band_wave<DT, 3, R, STREAM>(a, unit, L.first[3] + i * 2 * R, L.first[4], kl, ql, lane);
-  i -= L.blocks[3];
-  if (i < L.blocks[2]) return softmax_band_wave<DT, 2, R, STREAM>(a, unit, L.first[2] + i * 4 * R, L.first[3], kl, ql, lane);
-  i -= L.blocks[2];
-  if (i < L.blocks[1]) return softmax_band_wave<DT, 1, R, STREAM>(a, unit, L.first[1] + i * 8 * R, L.first[2], kl, ql, lane);
-  i -= L.blocks[1];
-  softmax_band_wave<DT, 0, R, STREAM>(a, unit, L.first[0] + i * 16 * R, L.first[1], kl, ql, lane);
+  int block = blockIdx.x;
+  while (block < L.total) {
+    int i = block;
+    block = VEC ? L.total : block + (int)gridDim.x;
+    // longest rows first
+    if (i < L.blocks[4]) {
+      softmax_band_wave<DT, 4, R, STREAM, VEC>(a, unit, L.first[4] + i * 1 * R, L.first[5], kl, ql, lane);
+      continue;
+    }
+    i -= L.blocks[4];
+    if (i < L.blocks[3]) {
+      softmax_band_wave<DT, 3, R, STREAM, VEC>(a, unit, L.first[3] + i * 2 * R, L.first[4], kl, ql, lane);
+      continue;
+    }
+    i -= L.blocks[3];
+    if (i < L.blocks[2]) {
+      softmax_band_wave<DT, 2, R, STREAM, VEC>(a, unit, L.first[2] + i * 4 * R, L.first[3], kl, ql, lane);
+      continue;
+    }
+    i -= L.blocks[2];
+    if (i < L.blocks[1]) {
+      softmax_band_wave<DT, 1, R, STREAM, VEC>(a, unit, L.first[1] + i * 8 * R, L.first[2], kl, ql, lane);
+      continue;
+    }
+    i -= L.blocks[1];
+    softmax_band_wave<DT, 0, R, STREAM, VEC>(a, unit, L.first[0] + i * 16 * R, L.first[1], kl, ql, lane);
+  }
 }
 
 // Upper bound, over all lengths a batch may have, of the workgroups one head needs (host side of band_layout).
@@ -359,14 +405,14 @@ __global__ __launch_bounds__(kBlock) void softmax_generic_kernel(SoftmaxArgs a) 
   }
 }
 
-template <int DT, int VPL, int LPR, int R>
+template <int DT, bool VEC, int VPL, int LPR, int R>
 static void launch_rows(const SoftmaxArgs &a, hipStream_t s) {
   constexpr int ROWS_PER_BLOCK = (kWave / LPR) * R;
   const dim3 grid((unsigned)ceil_div(a.rows_per_batch, ROWS_PER_BLOCK), (unsigned)a.B, 1);
-  softmax_rows_kernel<DT, VPL, LPR, R><<<grid, kRowsBlock, 0, s>>>(a);
+  softmax_rows_kernel<DT, VPL, LPR, R, VEC><<<grid, kRowsBlock, 0, s>>>(a);
 }
 
-template <int DT>
+template <int DT, bool VEC>
 static int launch_bands(const SoftmaxArgs &a, hipStream_t s) {
   constexpr int EPV = 16 / Elem<DT>::kSize;
   constexpr int R = 1;   // rows per lane group; two at once were slower on every workload measured
@@ -377,8 +423,29 @@ static int launch_bands(const SoftmaxArgs &a, hipStream_t s) {
   if (blocks > INT32_MAX) return EN_ERR_SHAPE;
   // a tensor too large to stay in the memory-side cache is read and written with the non-temporal policy
   const bool stream = (int64_t)a.B * a.rows_per_batch * a.Sk * Elem<DT>::kSize / (a.packed ? 2 : 1) >= kStreamSoftmaxBytes;
-  if (stream) softmax_bands_kernel<DT, R, true><<<grid, kWave, 0, s>>>(a);
-  else softmax_bands_kernel<DT, R, false><<<grid, kWave, 0, s>>>(a);
+  if (stream) softmax_bands_kernel<DT, R, true, VEC><<<grid, kWave, 0, s>>>(a);
+  else softmax_bands_kernel<DT, R, false, VEC><<<grid, kWave, 0, s>>>(a);
+  EN_RETURN_IF_LAUNCH_FAILED();
+  return EN_OK;
+}
+
+template <int DT>
+static void launch_generic(const SoftmaxArgs &a, hipStream_t s) {
+  softmax_generic_kernel<DT><<<dim3((unsigned)a.rows_per_batch, (unsigned)a.B, 1), kBlock, 0, s>>>(a);
+}
+
+template <int DT, bool VEC>
+static int dispatch_rows(const SoftmaxArgs &a, hipStream_t s) {
+  const int64_t nvec = ceil_div(a.Sk, 16 / Elem<DT>::kSize);
+  // Rows of up to 128 vectors (1024 16-bit keys): lane groups sized by what each row sees.  Measured against one
+  // shape per launch: 512-key rows 18.7 -> 16.3 us, 1024-key rows 160 -> 142 us; with 2048-key rows the banded form
+  // is slower (144 -> 183 us: two 512-byte pieces per instruction, a row pitch apart, instead of one 1024-byte piece),
+  // so those keep 64 lanes per row.
+  if (nvec <= 128) return launch_bands<DT, VEC>(a, s);
+  if (nvec <= 256) launch_rows<DT, VEC, 4, 64, 1>(a, s);
+  else if (nvec <= 512) launch_rows<DT, VEC, 8, 64, 1>(a, s);
+  else if (nvec <= 64 * 16) launch_rows<DT, VEC, 16, 64, 1>(a, s);
+  else launch_generic<DT>(a, s);
   EN_RETURN_IF_LAUNCH_FAILED();
   return EN_OK;
 }
@@ -386,21 +453,18 @@ static int launch_bands(const SoftmaxArgs &a, hipStream_t s) {
 template <int DT>
 static int dispatch(const SoftmaxArgs &a, hipStream_t s) {
   constexpr int EPV = 16 / Elem<DT>::kSize;
-  const bool vec_ok = (a.Sk % EPV) == 0 && aligned_to(a.src, 16);
-  const int64_t nvec = vec_ok ? a.Sk / EPV : 0;
-  if (!vec_ok || nvec > 64 * 16 || !(a.scale > 0.f)) {
-    softmax_generic_kernel<DT><<<dim3((unsigned)a.rows_per_batch, (unsigned)a.B, 1), kBlock, 0, s>>>(a);
+  const bool vec = (a.Sk % EPV) == 0 && aligned_to(a.src, 16);
+  // Rows off the 16-byte boundaries move with element-aligned vectors: a workgroup of 256 lanes a row, element by
+  // element in three passes, took far longer.  us for two layers of the seven operations, generic / this one:
+  // 32 sequences of up to 509, 12 heads x 64, fp16 465 / 319; 8 of 1001, 16 x 128, bf16 436 / 364;
+  // 16 of 301, 12 x 96, fp32 313 / 273.  More heads than a grid dimension holds: refused on aligned rows, the generic
+  // kernel's on others.
+  if (!(a.scale > 0.f) || (!vec && a.H > 65535)) {
+    launch_generic<DT>(a, s);
+    EN_RETURN_IF_LAUNCH_FAILED();
+    return EN_OK;
   }
-  // Rows of up to 128 vectors (1024 16-bit keys): lane groups sized by what each row sees.  Measured against one
-  // shape per launch: 512-key rows 18.7 -> 16.3 us, 1024-key rows 160 -> 142 us; with 2048-key rows the banded form
-  // is slower (144 -> 183 us: two 512-byte pieces per instruction, a row pitch apart, instead of one 1024-byte piece),
-  // so those keep 64 lanes per row.
-  else if (nvec <= 128) return launch_bands<DT>(a, s);
-  else if (nvec <= 256) launch_rows<DT, 4, 64, 1>(a, s);
-  else if (nvec <= 512) launch_rows<DT, 8, 64, 1>(a, s);
-  else launch_rows<DT, 16, 64, 1>(a, s);
-  EN_RETURN_IF_LAUNCH_FAILED();
-  return EN_OK;
+  return vec ? dispatch_rows<DT, true>(a, s) : dispatch_rows<DT, false>(a, s);
 }
 
 }  // namespace en
@@ -451,8 +515,8 @@ extern "C" int en_scale_mask_softmax_packed(void *scores, const int32_t *seq_len
                 head_num * seq_len, 1.0f / (float)seq_len, 1};
   hipStream_t s = (hipStream_t)stream;
   switch (dtype) {
-    case EN_F32: return launch_bands<EN_F32>(a, s);
-    case EN_F16: return launch_bands<EN_F16>(a, s);
-    default: return launch_bands<EN_BF16>(a, s);
+    case EN_F32: return launch_bands<EN_F32, true>(a, s);
+    case EN_F16: return launch_bands<EN_F16, true>(a, s);
+    default: return launch_bands<EN_BF16, true>(a, s);
   }
 }

@@ -69,7 +69,7 @@ def test_softmax_random_shapes(seed):
     ri = _draw(7100 + seed)
     B, H = ri(1, 5), ri(1, 4)
     rect = bool(ri(0, 1))
-    Sk = ri(1, 130) * [1, 1, 8][ri(0, 2)]        # odd widths take the scalar kernel, multiples of 8 the row kernel
+    Sk = ri(1, 130) * [1, 1, 8][ri(0, 2)]        # rows off the 16-byte boundaries, and on them
     Sq = ri(1, 40) if rect else Sk
     dtype = [torch.float16, torch.float32, torch.bfloat16][ri(0, 2)]
     causal = bool(ri(0, 1))

@@ -36,7 +36,7 @@ SOFTMAX_CASES = [
     (2, 1, 1024, [1024, 513]),
     (1, 2, 2048, [1500]),          # above the reference's 1024 limit
     (1, 1, 4096, [4096]),
-    (2, 2, 37, [37, 5]),           # row length not a multiple of the vector: generic kernel
+    (2, 2, 37, [37, 5]),           # row length not a multiple of the vector
     (1, 1, 8200, [8200]),          # too long for registers (fp32): generic kernel
 ]
 
@@ -105,6 +105,67 @@ def test_softmax_rectangular_decode(dtype):
     got2 = k.scale_mask_softmax(B, 1, H, src.clone().cuda(), torch.tensor(kv, dtype=torch.int32).cuda(), scale=0.5,
                                 k_seq_len=Sk).cpu()
     assert torch.equal(got, got2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shift", [0, 1])                       # elements between a 16-byte boundary and the first row
+@pytest.mark.parametrize("Sq,Sk,lens", [
+    (1, 1, [1]), (7, 7, [7, 3]), (301, 301, [301, 40, 0]),      # shorter than a vector; all bands of 16-bit rows
+    (5, 8, [8, 5]), (6, 509, [509, 6]), (6, 511, [511, 128]),
+    (4, 513, [513]), (4, 1023, [1023, 4]), (4, 1025, [1025]), (4, 2047, [2047]), (4, 2049, [2049, 1024]),
+    (3, 4097, [4096]), (3, 8191, [8191, 17]), (2, 8193, [8193]),    # up to and past what the registers hold
+    (9, 9, [30, 9]), (130, 130, [5000, 77]),                        # key lengths past the row
+])
+def test_softmax_rows_off_the_16_byte_boundaries(dtype, shift, Sq, Sk, lens):
+    """Rows at any element's address against float64, the tail zeroed to the row's end and nothing else touched.
+
+    Bound: half an ulp of a probability of at most one (2^-12, 2^-9) for 16 bits; in fp32 the argument of the exponential
+    is rounded at its size (|x| <= 16: 2^-20) and the sum once per addition."""
+    k = _kernel()
+    H = 2
+    B = len(lens)
+    announce("softmax unaligned", dtype, shift, Sq, Sk, lens)
+    g = torch.Generator().manual_seed(Sq * Sk + shift)
+    n = B * H * Sq * Sk
+    flat = (3.0 * torch.randn(n + 32, generator=g)).clamp(-16, 16).to(dtype)
+    buf = flat.clone().cuda()
+    src = flat[shift:shift + n].view(B, H, Sq, Sk)
+    lens_t = torch.tensor(lens, dtype=torch.int32).cuda()
+    ql = [min(x, Sq) for x in lens]
+    k.scale_mask_softmax(B, Sq, H, buf[shift:shift + n].view(B, H, Sq, Sk), lens_t, scale=0.37, k_seq_len=Sk,
+                         q_len_list=torch.tensor(ql, dtype=torch.int32).cuda())
+    after = buf.cpu()
+    assert torch.equal(after[:shift], flat[:shift]) and torch.equal(after[shift + n:], flat[shift + n:])
+    got = after[shift:shift + n].view(B, H, Sq, Sk)
+    tol = {torch.float32: 2e-6, torch.float16: 2.0 ** -12 + 2e-6, torch.bfloat16: 2.0 ** -9 + 2e-6}[dtype]
+    for b in range(B):
+        assert torch.equal(got[b, :, ql[b]:], src[b, :, ql[b]:])
+        for q in range(ql[b]):
+            vis = min(q + lens[b] - ql[b] + 1, Sk)
+            want = torch.softmax(src[b, :, q, :vis].double() * 0.37, -1)
+            assert max_abs(got[b, :, q, :vis].double(), want) <= tol, (b, q)
+            assert not got[b, :, q, vis:].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("S", [9, 515])
+def test_softmax_odd_rows_of_extreme_scores(dtype, S):
+    """Rows of the type's lowest value, of -inf, and with one of either: as the definition has it."""
+    k = _kernel()
+    announce("softmax extremes", dtype, S)
+    low = torch.finfo(dtype).min
+    src = torch.zeros(1, 1, S, S, dtype=dtype)
+    src[..., 4, :] = low
+    src[..., 5, :] = -float("inf")
+    src[..., 6, 1:] = low
+    src[..., 7, 2:] = -float("inf")
+    got = k.scale_mask_softmax(1, S, 1, src.clone().cuda(), torch.tensor([S], dtype=torch.int32).cuda(), scale=0.5,
+                               causal=False).cpu()[0, 0]
+    want = torch.full((S, S), 1.0 / S, dtype=torch.float64)
+    want[5] = 0                                     # nothing to see: zeros, no NaN
+    want[6], want[7] = 0, 0
+    want[6, 0], want[7, :2] = 1, 0.5
+    assert max_abs(got.double(), want) <= {torch.float32: 1e-6, torch.float16: 2e-4, torch.bfloat16: 2e-3}[dtype]
 
 
 def test_softmax_rectangular_chunked_prefill():
