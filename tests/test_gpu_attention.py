@@ -98,6 +98,47 @@ def test_attn_qk_pv_fused_layout(dtype, causal, B, H, S, D, lens):
         assert torch.equal(ctx0[rows_ok], ctx[rows_ok])
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shift", [0, 1])                       # elements between a 16-byte boundary and the first row
+@pytest.mark.parametrize("Sq,Sk,D,lens", [
+    (1, 1, 64, [1]), (5, 5, 80, [5, 2]), (63, 63, 64, [63, 9]), (65, 65, 128, [65, 0, 64]),
+    (129, 129, 64, [129, 127]), (131, 131, 96, [131]), (259, 259, 128, [259, 130]), (7, 301, 64, [301, 7]),
+])
+def test_attn_rows_off_the_16_byte_boundaries(dtype, shift, Sq, Sk, D, lens):
+    """Score rows at any element's address: every visible score, nothing past a row's end or before the first row; and
+    probabilities whose rows hold NaN past what the query sees, which must not be read into the sum."""
+    k = _kernel()
+    H, B = 2, len(lens)
+    ql = [min(n, Sq) for n in lens]
+    announce("attn unaligned", dtype, shift, Sq, Sk, D, lens)
+    g = torch.Generator().manual_seed(Sq + Sk + D)
+    q = torch.randn(B, H, Sq, D, generator=g).to(dtype)
+    kk, v = (torch.randn(B, H, Sk, D, generator=g).to(dtype) for _ in range(2))
+    lens_t, ql_t = (torch.tensor(x, dtype=torch.int32).cuda() for x in (lens, ql))
+    n = B * H * Sq * Sk
+    sentinel = 777.0
+    buf = torch.full((n + 32,), sentinel, dtype=dtype, device="cuda")
+    k.attn_qk(q.cuda(), kk.cuda(), lens_t, causal=True, q_len_list=ql_t, out=buf[shift:shift + n].view(B, H, Sq, Sk))
+    after = buf.cpu()
+    assert bool((after[:shift] == sentinel).all()) and bool((after[shift + n:] == sentinel).all())
+    scores = after[shift:shift + n].view(B, H, Sq, Sk)
+    want = eager.attn_qk(q, kk, torch.float64)
+    vis = _visible_mask(B, H, Sq, Sk, lens, ql, True)
+    step = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -16}[dtype]
+    assert ((scores.double() - want).abs() / (want.abs() + 1.0))[vis].max().item() <= 1.5 * step
+    for b, m in enumerate(ql):
+        assert bool((scores[b, :, m:] == sentinel).all())
+    probs = torch.softmax(want.masked_fill(~vis, -float("inf")) * D ** -0.5, -1).to(dtype)
+    probs[~vis] = float("nan")
+    flat = torch.full((n + 32,), float("nan"), dtype=dtype)
+    flat[shift:shift + n] = probs.flatten()
+    ctx = k.attn_pv(flat.cuda()[shift:shift + n].view(B, H, Sq, Sk), v.cuda(), lens_t, causal=True, q_len_list=ql_t).cpu()
+    want_ctx = eager.attn_pv(torch.nan_to_num(probs, nan=0.0), v, torch.float64)
+    for b, m in enumerate(ql):
+        if m:
+            assert_ctx_close(ctx[b, :, :m], want_ctx[b, :, :m], dtype, "attn_pv")
+
+
 def test_attn_nan_in_padding_of_v_is_ignored():
     """Cache rows past the valid length may hold anything (torch.empty caches)."""
     k = _kernel()
