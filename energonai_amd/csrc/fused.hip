@@ -52,8 +52,9 @@
 namespace en {
 
 // DP: channels of a row in LDS (the head size rounded up to 64, 96 or 128); NVS: MFMA steps of 16 channels that hold any.
-// NORM: the residual + LayerNorm of fused_common.hip.h follows (16-byte context rows, no separate query lengths).
-template <int DT, int DP, int NVS, bool NORM>
+// NORM: the residual + LayerNorm of fused_common.hip.h follows (16-byte context rows, no separate query lengths).  Q_ONCE: Q is read
+// non-temporal (a parameter: chosen by a branch in the kernel, it cost the key loop registers and layers of 128 channels 10 %).
+template <int DT, int DP, int NVS, bool NORM, bool Q_ONCE>
 __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *norm, int bid = blockIdx.x) {
   static_assert(DT != EN_F32, "the fused kernel is built for 16-bit storage");
   typedef Elem<DT> E;
@@ -69,12 +70,6 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
   constexpr int KLOADS = BK * KVEC_ROW / kBlock; // direct-load instructions per wave and tile, for each of K and V
   constexpr float kLog2e = 1.4426950408889634f;
   constexpr int NVB = DP <= 96 ? 2 : 1;          // V buffers
-  // Q is read once, and non-temporal it leaves the caches to what is read again, K and V by the unit's other tiles and the context
-  // by the LayerNorm.  Layers in us, cached / non-temporal: 4 of 16 sequences of up to 1024, 56 heads x 128 986 / 980, 6 of 32 of up to
-  // 256, 16 x 128 231 / 225, 4 of 8 of up to 512, 32 x 128 206 / 201, 4 of 7 of up to 1531, 20 x 80 316 / 315.  With the LayerNorm in
-  // the launch, where K and V of all tiles come in at once, it loses (4 of 4 of up to 700, 16 x 128 114 / 116), and at 64 channels (12
-  // of 39 of up to 557, 5 x 64 304 / 316).
-  constexpr int QAUX = DP > 64 && !NORM ? 2 : 0;
   static_assert(DP == 64 || DP == 96 || DP == 128, "swizzles are written for 8, 12 or 16 slots per row");
   static_assert(NVS * 16 <= DP, "a step reads channels the tile has");
   static_assert(BK * KVEC_ROW % kBlock == 0 && 32 * KVEC_ROW % kWave == 0, "tiles must divide over the block");
@@ -133,7 +128,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
       const int c = slot ^ kswz(rr);
       const int qq = q0 + wave * 32 + rr;
       const uint32_t off = (uint32_t)(((int64_t)qq * a.q_ss + c * EPV) * E::kSize);
-      buffer_load16_to_lds<QAUX>(q_desc, lds_address(q_stage) + n * kWave * 16, ((unsigned)qq < (unsigned)ql && c * EPV < a.D) ? off : kOutOfRange);
+      buffer_load16_to_lds<Q_ONCE ? 2 : 0>(q_desc, lds_address(q_stage) + n * kWave * 16, ((unsigned)qq < (unsigned)ql && c * EPV < a.D) ? off : kOutOfRange);
     }
   }
 
@@ -406,13 +401,13 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &fa, const NormArgs *
     }
 }
 
-template <int DT, int DP, int NVS>
+template <int DT, int DP, int NVS, bool Q_ONCE>
 __global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_kernel(FusedArgs fa) {
-  fused_tile<DT, DP, NVS, false>(fa, nullptr);
+  fused_tile<DT, DP, NVS, false, Q_ONCE>(fa, nullptr);
 }
 template <int DT, int DP, int NVS>
 __global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_norm_kernel(FusedArgs fa, NormArgs norm) {
-  fused_tile<DT, DP, NVS, true>(fa, &norm);
+  fused_tile<DT, DP, NVS, true, false>(fa, &norm);
 }
 
 // The attention and, in workgroups of their own, a residual + LayerNorm that does not read its output (a row-parallel
@@ -421,33 +416,47 @@ __global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_norm_kern
 // 14213 tokens, 12 heads x 128, rows of 12288 252 / 240; 3485, 32 x 128, 8192 114 / 107; 3569, 16 x 64, 8192 49 / 43.5;
 // 3866, 10 x 80, 3200 42 / 32; 1033, 8 x 64, 2048 19.3 / 15.7; 300, 5 x 64, 640 18.3 / 15.3.  (Rows of 14336, which a
 // workgroup could hold with one load in flight less: 170 / 182, so 12288 is where it ends.)
-template <int DT, int DP, int NVS, bool STREAM>
+template <int DT, int DP, int NVS, bool Q_ONCE, bool STREAM>
 __global__ __launch_bounds__(kBlock, DP == 64 ? 4 : 3) void attn_fused_beside_norm_kernel(FusedArgs fa, NormRows rows) {
   const int j = blockIdx.x / kXcds, x = blockIdx.x % kXcds;
   const int before = min((int)(((uint64_t)j * rows.step) >> 16), rows.groups);
   const int behind = min((int)(((uint64_t)(j + 1) * rows.step) >> 16), rows.groups);
   if (behind > before) norm_rows<DT, STREAM>(rows, before * kXcds + x);
-  else fused_tile<DT, DP, NVS, false>(fa, nullptr, (j - before) * kXcds + x);
+  else fused_tile<DT, DP, NVS, false, Q_ONCE>(fa, nullptr, (j - before) * kXcds + x);
 }
 
-template <int DT, int DP, int NVS>
+template <int DT, int DP, int NVS, bool Q_ONCE = false>
 static void launch_form(const FusedArgs &fa, const NormArgs *norm, const NormRows *rows, unsigned grid, hipStream_t s) {
   if (rows) {
     grid += (unsigned)rows->groups * kXcds;
-    if (rows->rows * rows->width * 2 >= kStreamStoreBytes) attn_fused_beside_norm_kernel<DT, DP, NVS, true><<<grid, kBlock, 0, s>>>(fa, *rows);
-    else attn_fused_beside_norm_kernel<DT, DP, NVS, false><<<grid, kBlock, 0, s>>>(fa, *rows);
+    constexpr bool ONCE = Q_ONCE && DP == 128;
+    if (rows->rows * rows->width * 2 >= kStreamStoreBytes) attn_fused_beside_norm_kernel<DT, DP, NVS, ONCE, true><<<grid, kBlock, 0, s>>>(fa, *rows);
+    else attn_fused_beside_norm_kernel<DT, DP, NVS, ONCE, false><<<grid, kBlock, 0, s>>>(fa, *rows);
   } else if (norm) attn_fused_norm_kernel<DT, DP, NVS><<<grid, kBlock, 0, s>>>(fa, *norm);
-  else attn_fused_kernel<DT, DP, NVS><<<grid, kBlock, 0, s>>>(fa);
+  else attn_fused_kernel<DT, DP, NVS, Q_ONCE><<<grid, kBlock, 0, s>>>(fa);
 }
 
+// Q is read once, and non-temporal it leaves the caches to what is read again, K and V by the unit's other tiles and the context by the
+// LayerNorm.  That pays with heads of 128 channels, whose Q rows are whole 128-byte lines, and hardly with 96 (a line and a half); the
+// others lose, their lines being shared with the rows beside them.  us, cached / non-temporal:
+//   128: 4 layers of 8 sequences of up to 512, 32 heads 154.4 / 150.5, 6 of 16 of up to 256, 32 241 / 236, 6 of 64 of up to 40, 20 143.4 /
+//     141.7, 4 of 3 of up to 700, 72, no mask 245.6 / 242.5, 4 of 16 of up to 1024, 56 864 / 858; with the LayerNorm's rows beside it 6 of 40
+//     of up to 128, 24 365 / 357, 8 of 1 of up to 100, 12 97.5 / 97.5, 4 of 16 of up to 512, 32 327 / 326;
+//   96: 6 of 8 of up to 200, 32 121 / 119, 4 of 4 of up to 1000, 24 213 / 211, 6 of 24 of up to 256, 20 173.8 / 174.4; rows beside it 6 of 24 of
+//     up to 256, 20 243.5 / 250.3, 6 of 8 of up to 600, 16 235.6 / 241.4;
+//   others: 80 channels 4 of 7 of up to 1531, 20 231 / 235, 6 of 16 of up to 400, 20, rows beside it 297 / 306; 112 6 of 16 of up to 512, 24
+//     290 / 297; 120 6 of 40 of up to 100, 40 277 / 283; 64 12 of 39 of up to 557, 5 304 / 316.
+// With the LayerNorm in the launch K and V of all tiles come in at once, and it loses at 128 too: 4 of 4 of up to 700, 16 114 / 116.
 template <int DT>
 static int launch_fused(FusedArgs &fa, const NormArgs *norm, const NormRows *rows, hipStream_t s) {
   const AttnArgs &a = fa.base;
   const unsigned grid = (unsigned)(ceil_div(a.units, kXcds) * kXcds * a.ntq);
   if (a.D <= 64) launch_form<DT, 64, 4>(fa, norm, rows, grid, s);
   else if (a.D <= 80) launch_form<DT, 96, 5>(fa, norm, rows, grid, s);
-  else if (a.D <= 96) launch_form<DT, 96, 6>(fa, norm, rows, grid, s);
-  else launch_form<DT, 128, 8>(fa, norm, rows, grid, s);
+  else if (a.D < 96) launch_form<DT, 96, 6>(fa, norm, rows, grid, s);
+  else if (a.D == 96) launch_form<DT, 96, 6, true>(fa, norm, rows, grid, s);
+  else if (a.D < 128) launch_form<DT, 128, 8>(fa, norm, rows, grid, s);
+  else launch_form<DT, 128, 8, true>(fa, norm, rows, grid, s);
   EN_RETURN_IF_LAUNCH_FAILED();
   return EN_OK;
 }
