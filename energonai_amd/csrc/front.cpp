@@ -222,7 +222,7 @@ PyObject *layer(PyObject *const *a) {
   const int tag = dtype_tag(hidden, "padding_removal_layer");
   if (form == 4 && dt == at::kFloat) fail(who + "the packed scores are for float16 and bfloat16");
   if ((form == 1 || form == 2) && dt == at::kFloat && D > 64) fail(who + "the fused kernel takes float32 heads of up to 64 channels");
-  if (form == 5 && dt != at::kFloat) fail(who + "the wide form is for float32");
+  if (form == 5 && (dt != at::kFloat || D <= 64 || D > 128)) fail(who + "packed_f32_wide is for float32 heads of 65..128 channels");
   if (form == 4 && !causal) fail(who + "the packed score layout is that of a causal mask");
   const c10::DeviceGuard guard(hidden.device());
   const auto opt = hidden.options();
@@ -265,18 +265,6 @@ PyObject *layer(PyObject *const *a) {
       check(rc, "padding_removal_layer");
       return THPVariable_Wrap(y);
     }
-  }
-  if (form == 5) {
-    if (T == 0) return THPVariable_Wrap(y);
-    check(without_gil([&] {
-            int rc = offs ? EN_OK : en_depad(hidden_p, x_p, cu_p, (int)B, (int)S, hid, 4, left, stream);
-            if (rc == EN_OK) rc = en_attn_fused_f32_wide(qkv_p, packed_p, lens_p, cu_p, (int)B, (int)H, (int)S, (int)D, scale, causal, stream);
-            if (rc == EN_OK)
-              rc = en_layernorm_fwd(y_p, nullptr, nullptr, nullptr, dense ? dense : packed_p, offs ? hidden_p : x_p, offs, gamma_p, beta_p, T, hid,
-                                    eps, tag, tag, stream);
-            return rc;
-          }), "padding_removal_layer");
-    return THPVariable_Wrap(y);
   }
   check(without_gil([&] {
           return en_padding_removal_layer(hidden_p, qkv_p, dense, gamma_p, beta_p, x_p, padded_p, scores_p, ctx_p, packed_p, y_p, cu_p, lens_p,

@@ -1,5 +1,5 @@
-// Fused attention for fp32 storage and heads of up to 64 channels (the BERT-base shape of the reference's CPU
-// path, examples/bert/bert.py:108-119 in fp32): ctx = softmax(scale * Q K^T, mask) V in one kernel, no score
+// Fused attention for fp32 storage (heads of up to 64 channels, the BERT-base shape of the reference's CPU
+// path, examples/bert/bert.py:108-119 in fp32; wider ones have the second kernel below): ctx = softmax(scale * Q K^T, mask) V in one kernel, no score
 // tensor.  The 16-bit kernels of fused.hip are built around 16-bit operand vectors (probabilities as 16-bit B
 // operands, the transposing LDS read); here everything is fp32 on the 32x32x2 MFMA.
 //
@@ -16,6 +16,8 @@
 //                    for register (j, i) contracts over the two keys 8j + i and 8j + 4 + i that the lane's two
 //                    halves hold; A = V at those keys, one channel per lane, read from the row-major V tile.
 #include "fused_common.hip.h"
+
+#include <type_traits>
 
 namespace en {
 
@@ -269,7 +271,8 @@ __global__ __launch_bounds__(kBlock, DP == 96 ? 3 : 2) void attn_fused_f32_wide_
   static_assert(DP == 96 || DP == 128, "swizzles are written for 24 or 32 slots per row");
   __shared__ __attribute__((aligned(16))) float lds[2 * BK * DP];
   float *const lds_k = lds, *const lds_v = lds + BK * DP;
-  static_assert(2 * (2 + DMT * 16) * kWave <= 2 * BK * DP, "the pairs are combined in the tiles' room");
+  constexpr int HANDED = (2 + DMT * 8) * kWave;    // what a wave hands to the other of its pair: maximum, sum and half of its channels
+  static_assert(4 * HANDED <= 2 * BK * DP, "the pairs are combined in the tiles' room");
   auto kswz = [](int row) { return DP == 128 ? (row & 15) : ((row >> 1) & 7); };
   auto vflip = [](int key) { return (key >> 2) & 1; };
 
@@ -423,38 +426,53 @@ __global__ __launch_bounds__(kBlock, DP == 96 ? 3 : 2) void attn_fused_f32_wide_
     lds_barrier();                                // K tile kt + 1 is there, V tile kt has been read
   }
 
-  // ---- combine the two waves of a query half (they saw disjoint keys), then normalise and store.
+  // ---- combine the two waves of a query half (they saw disjoint keys), then normalise and store: each hands over half of its channels and
+  // finishes the others.  The quotient is refined: its rounding comes once, not in 1 / l and again in the product, which rows of a few
+  // keys showed (context of 17 keys, 68 channels against float64 1.35e-7 -> 1.32e-7, of 40, 100 1.93e-7 -> 1.915e-7; QK^T, softmax and PV
+  // 1.31e-7 and 1.91e-7; from 64 keys on theirs is the larger).
   float l_lo, l_hi;
   halves_of(l_run, l_lo, l_hi);
   l_run = l_lo + l_hi;
-  float *comb = lds + wq * (2 + DMT * 16) * kWave;
-  if (wk == 1) {
-    comb[lane] = m_run;
-    comb[kWave + lane] = l_run;
+  float *const mine = lds + (2 * wq + wk) * HANDED, *const other = lds + (2 * wq + (wk ^ 1)) * HANDED;
+  auto hand = [&](auto half) {
+    mine[lane] = m_run;
+    mine[kWave + lane] = l_run;
 #pragma unroll
     for (int mt = 0; mt < DMT; ++mt)
 #pragma unroll
-      for (int x = 0; x < 16; ++x) comb[(2 + mt * 16 + x) * kWave + lane] = o[mt][x];
-  }
+      for (int x = 0; x < 8; ++x) mine[(2 + mt * 8 + x) * kWave + lane] = o[mt][8 * decltype(half)::value + x];
+  };
+  auto finish = [&](auto half) {
+    const float m1 = other[lane], l1 = other[kWave + lane];
+    const float m = fmaxf(m_run, m1);
+    const float w0 = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m) * c_exp);
+    const float w1 = (m1 == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m1 - m) * c_exp);
+    const float l = l_run * w0 + l1 * w1;
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    T *crow = cbase + (int64_t)q_lane * fa.c_ss;
+#pragma unroll
+    for (int mt = 0; mt < DMT; ++mt)
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj) {
+        const int j = 2 * decltype(half)::value + jj, d = mt * 32 + 8 * j + 4 * g;
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float sum = o[mt][4 * j + i] * w0 + other[(2 + mt * 8 + 4 * jj + i) * kWave + lane] * w1, quot = sum * inv;
+          const float rest = fmaf(-quot, l, sum);
+          v[i] = rest == rest ? fmaf(rest, inv, quot) : quot;      // a sum that is not finite stays what it is
+        }
+        if (d < a.D) *reinterpret_cast<float4 *>(crow + d) = make_float4(v[0], v[1], v[2], v[3]);
+      }
+  };
+  typedef std::integral_constant<int, 0> Low;
+  typedef std::integral_constant<int, 1> High;
+  if (wk == 0) hand(High());
+  else hand(Low());
   lds_barrier();
-  if (wk == 1 || q_lane >= ql) return;
-  const float m1 = comb[lane], l1 = comb[kWave + lane];
-  const float m = fmaxf(m_run, m1);
-  const float w0 = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m) * c_exp);
-  const float w1 = (m1 == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m1 - m) * c_exp);
-  const float l = l_run * w0 + l1 * w1;
-  const float inv = l > 0.f ? 1.0f / l : 0.f;
-  T *crow = cbase + (int64_t)q_lane * fa.c_ss;
-#pragma unroll
-  for (int mt = 0; mt < DMT; ++mt)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = mt * 32 + 8 * j + 4 * g;
-      float v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (o[mt][4 * j + i] * w0 + comb[(2 + mt * 16 + 4 * j + i) * kWave + lane] * w1) * inv;
-      if (d < a.D) *reinterpret_cast<float4 *>(crow + d) = make_float4(v[0], v[1], v[2], v[3]);
-    }
+  if (q_lane >= ql) return;
+  if (wk == 0) finish(Low());
+  else finish(High());
 }
 
 static int launch_fused_f32_wide(const FusedArgs &fa, hipStream_t s) {
@@ -480,13 +498,14 @@ int launch_fused_f32(FusedArgs &fa, const NormArgs *norm, hipStream_t s) {
 
 extern "C" {
 
+// us a layer, QK^T + softmax + PV / this, with the LayerNorm behind either: 1 prompt of 64, 12 heads x 128 28 / 18, 4 of up to 128, 8 x
+// 80 39 / 21, 8 of up to 128, 16 x 96 43 / 23, 1 of 1000, 4 x 128 155 / 76, 4 of up to 512, 12 x 96 103 / 49, 22 of 110, 45 x 128 260 / 137,
+// 16 of up to 384, 20 x 80, no mask 199 / 128, 4 of up to 35, 12 x 96 26 / 15, 64 of up to 20, 4 x 128 22 / 16, 1 of 17, 4 x 68 (the host's
+// time) 23 / 15.  The faster form at every size: wherever it takes the heads, it is theirs.  Its context against float64, three kernels /
+// this, 60 draws: 17 keys, 68 channels 1.306e-7 / 1.324e-7, 20, 128 1.504e-7 / 1.499e-7, 40, 100, no mask 2.985e-7 / 2.950e-7, 64, 128, no
+// mask 3.585e-7 / 3.462e-7, 1200, 128, no mask 7.45e-7 / 6.04e-7.
 int en_attn_fused_f32_wide_pays(int batch, int head_num, int max_seq_len, int size_per_head) {
-  if (batch < 1 || head_num < 1 || max_seq_len < 1 || size_per_head <= 64 || size_per_head > 128 || size_per_head % 4) return 0;
-  // us a layer, QK^T + softmax + PV / this, with the LayerNorm behind either: 1 prompt of 64, 12 heads x 128 28 / 18, 4 of up to 128, 8 x
-  // 80 39 / 21, 8 of up to 128, 16 x 96 43 / 23, 1 of 1000, 4 x 128 155 / 76, 4 of up to 512, 12 x 96 103 / 49, 22 of 110, 45 x 128 260 / 137,
-  // 16 of up to 384, 20 x 80, no mask 199 / 128.  It is the faster form at every size; the line is where the scores of the three
-  // kernels pass 2 MiB, below which the step keeps giving the bits of the separate calls, as a caller who compares the two expects.
-  return 4.0 * batch * head_num * max_seq_len * max_seq_len > 2.0 * (1 << 20);
+  return batch > 0 && head_num > 0 && max_seq_len > 0 && size_per_head > 64 && size_per_head <= 128 && size_per_head % 4 == 0;
 }
 
 int en_attn_fused_f32_wide(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
@@ -494,7 +513,7 @@ int en_attn_fused_f32_wide(const void *qkv, void *ctx, const int32_t *seq_lens, 
   using namespace en;
   if (!qkv || !ctx || !seq_lens || !cu_seqlens) return EN_ERR_NULL;
   if (batch < 1 || head_num < 1 || max_seq_len < 1 || size_per_head < 1) return EN_ERR_SHAPE;
-  if (size_per_head <= 64 || size_per_head > 128 || size_per_head % 4 || !(scale > 0.f)) return EN_ERR_UNSUPPORTED;
+  if (!en_attn_fused_f32_wide_pays(batch, head_num, max_seq_len, size_per_head) || !(scale > 0.f)) return EN_ERR_UNSUPPORTED;
   if (!aligned_to(qkv, 16) || !aligned_to(ctx, 16)) return EN_ERR_ALIGN;
   const int64_t D = size_per_head, row = (int64_t)3 * head_num * D;
   if ((int64_t)batch * head_num > INT32_MAX / 64) return EN_ERR_SHAPE;

@@ -81,9 +81,9 @@ extern "C" int en_padding_removal_layer(const void *hidden_padded, const void *q
   if (!hidden_padded || !qkv_packed || !gamma || !beta || !ctx_packed || !y || !cu_seqlens || !seq_lens)
     return EN_ERR_NULL;
   if (!x_packed && !fold_depad_offsets) return EN_ERR_NULL;
-  if (attention_form < 0 || attention_form > 4) return EN_ERR_UNSUPPORTED;
+  if (attention_form < 0 || attention_form > 5 || (attention_form == 5 && dtype != EN_F32)) return EN_ERR_UNSUPPORTED;
   if (attention_form < 2 && (!qkv_padded || !ctx)) return EN_ERR_NULL;
-  if ((attention_form == 0 || attention_form >= 3) && !scores) return EN_ERR_NULL;
+  if ((attention_form == 0 || attention_form == 3 || attention_form == 4) && !scores) return EN_ERR_NULL;
   const int es = dtype_size(dtype);
   if (!es) return EN_ERR_DTYPE;
   if (total_tokens < 0 || hidden < 1) return EN_ERR_SHAPE;
@@ -113,6 +113,9 @@ extern "C" int en_padding_removal_layer(const void *hidden_padded, const void *q
     rc = en_attn_fused(pk, pk + (int64_t)D * es, pk + (int64_t)2 * D * es, ctx_packed, seq_lens, nullptr, B, H, S, S, D,
                        in_strides, in_strides, in_strides, out_strides, cu_seqlens, cu_seqlens, scale, causal, dtype,
                        dtype == EN_F32 ? nullptr : tile_table, 0, stream);      // the fp32 kernel's tiles are not the table's
+    if (rc) return rc;
+  } else if (attention_form == 5) {
+    rc = en_attn_fused_f32_wide(qkv_packed, ctx_packed, seq_lens, cu_seqlens, B, H, S, D, scale, causal, stream);
     if (rc) return rc;
   } else if (attention_form >= 3) {
     // The three kernels on the packed projections: q, k, v are read where the projection left them (batch b at
@@ -178,7 +181,7 @@ extern "C" int en_padding_removal_layer_noalloc(const void *hidden_padded, const
                                                 int fold_depad, int dtype, en_stream_t stream) {
   using namespace en;
   if (!hidden_padded || !qkv_packed || !gamma || !beta || !y || !seq_lens) return EN_ERR_NULL;
-  if (attention_form < 0 || attention_form > 4) return EN_ERR_UNSUPPORTED;
+  if (attention_form < 0 || attention_form > 5 || (attention_form == 5 && dtype != EN_F32)) return EN_ERR_UNSUPPORTED;
   const int64_t es = dtype_size(dtype);
   if (!es) return EN_ERR_DTYPE;
   if (batch < 1 || batch > 65536 || max_seq_len < 1 || head_num < 1 || size_per_head < 1 || hidden < 1 ||
@@ -197,7 +200,7 @@ extern "C" int en_padding_removal_layer_noalloc(const void *hidden_padded, const
       ? (scores_fit ? en_packed_scores_elems(batch, head_num, max_seq_len, dtype) * es : kLayerScratchBytes + 1)
       : piece_bytes({B, H, S, S, es});
   const int64_t o_qkv = l.take(padded, piece_bytes({B, H, S, 3 * D, es}));
-  const int64_t o_scores = l.take(attention_form == 0 || attention_form >= 3, score_bytes);
+  const int64_t o_scores = l.take(attention_form == 0 || attention_form == 3 || attention_form == 4, score_bytes);
   const int64_t o_ctx = l.take(padded, piece_bytes({B, H, S, D, es})), o_ctxp = l.take(true, piece_bytes({T, H, D, es}));
   if (l.used > kLayerScratchBytes) return EN_ERR_SCRATCH;
   unsigned char *base = nullptr;   // the array's address on the current device; never the array's name

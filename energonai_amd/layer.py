@@ -27,6 +27,9 @@ from .seqinfo import SeqInfo, seq_info
 SOFTMAX_TAIL_ROWS = 1
 
 
+LEAST_F32_SCALE = 2.0 ** -150      # what is no larger is zero in fp32, and a zero scale is the three kernels'
+
+
 def three_kernel_form(causal: bool, dtype: torch.dtype, max_seq_len: int) -> str:
     """QK^T, softmax and PV as three kernels on packed operands: with the scores in the packed causal layout where
     that layout exists and is smaller than ``[B,H,S,S]``."""
@@ -37,15 +40,16 @@ def three_kernel_form(causal: bool, dtype: torch.dtype, max_seq_len: int) -> str
 
 def default_attention_form(causal: bool, dtype: torch.dtype, max_seq_len: int, size_per_head: int,
                            scale: float = 1.0) -> str:
-    """The form ``padding_removal_layer`` runs when the caller names none: the fused kernel on the packed
-    projections wherever it applies (16-bit storage with heads of at most 128 channels in multiples of 8, fp32
-    with heads of at most 64 in multiples of 4, a positive scale) -- the score tensor then never exists and the
-    step is two launches -- else the three kernels.  (fp32 heads of 65..128 channels are the three kernels' here; where their scores
-    would pass 2 MiB the step runs a fused kernel of its own in their place, ``en_attn_fused_f32_wide``.)"""
+    """The form ``padding_removal_layer`` runs when the caller names none: a fused kernel on the packed
+    projections wherever one applies (16-bit storage with heads of at most 128 channels in multiples of 8, fp32
+    with heads of at most 128 in multiples of 4, a positive scale) -- the score tensor then never exists and the
+    step is two launches -- else the three kernels."""
     if dtype in (torch.float16, torch.bfloat16) and size_per_head <= 128 and size_per_head % 8 == 0 and scale > 0:
         return "packed"
     if dtype == torch.float32 and size_per_head <= 64 and size_per_head % 4 == 0 and scale > 0:
         return "packed"      # the fp32 fused kernel (heads of up to 64 channels: the BERT-base shape)
+    if dtype == torch.float32 and size_per_head <= 128 and size_per_head % 4 == 0 and scale > LEAST_F32_SCALE:
+        return "packed_f32_wide"
     return three_kernel_form(causal, dtype, max_seq_len)
 
 
@@ -68,10 +72,10 @@ def padding_removal_layer(hidden_padded: torch.Tensor, qkv_packed: torch.Tensor,
     ``True``             QK^T / softmax / PV in the single fused kernel on the padded buffer (16-bit dtypes
                          only); the score tensor is then never written;
     ``"packed"``         the fused kernel on the packed projections;
-    ``None`` (default)   ``"packed"`` wherever the fused kernel applies (16-bit dtypes, heads of at most 128
+    ``"packed_f32_wide"``  the same for fp32 heads of 65..128 channels, a kernel of their own;
+    ``None`` (default)   ``"packed"`` or ``"packed_f32_wide"`` wherever the kernel applies (heads of at most 128
                          channels), else the three kernels: ``"varlen_packed"`` under a causal mask with rows of
-                         at least 256 keys, ``"varlen"`` otherwise (fp32 heads of 65..128 channels: one kernel, another order
-                         of summation, where the scores of those would pass 2 MiB); with ``keep`` the reference's sequence, whose
+                         at least 256 keys, ``"varlen"`` otherwise; with ``keep`` the reference's sequence, whose
                          intermediates are the ones a caller can name.  (The packed score layout halves the score
                          tensor and keeps every row on whole 128-byte groups: the three kernels together take
                          415 -> 349 us on 2048-key rows, 461 -> 457 us on 1024-key rows; short rows would only grow.)
@@ -90,8 +94,6 @@ def padding_removal_layer(hidden_padded: torch.Tensor, qkv_packed: torch.Tensor,
     scale = float(D) ** -0.5 if scale is None else scale
     if fused_attention is None:
         fused_attention = False if keep else default_attention_form(causal, hidden_padded.dtype, S, D, scale)
-        if not keep and hidden_padded.dtype == torch.float32 and D > 64 and scale > 0 and _lib.fn.en_attn_fused_f32_wide_pays(B, H, S, D):
-            fused_attention = _WIDE
     if fold_depad is None:
         fold_depad = not keep
     if not keep:
@@ -101,6 +103,11 @@ def padding_removal_layer(hidden_padded: torch.Tensor, qkv_packed: torch.Tensor,
         raise RuntimeError("padding_removal_layer: fold_depad has no intermediates to keep")
 
     x = depad(hidden_padded, B, info, left_padded=left_padded, sum_seq=T)
+    if fused_attention == "packed_f32_wide":
+        ctx_packed = torch.empty((1, T, H, D), dtype=qkv_packed.dtype, device=qkv_packed.device)
+        y = _layer_one_call(hidden_padded, qkv_packed, info, S, H, D, T, gamma, beta, eps, scale, causal, left_padded, dense_out,
+                            fused_attention, ctx_out=ctx_packed)
+        return dict(x=x, qkv=None, probs=None, ctx=None, ctx_packed=ctx_packed, y=y)
     if fused_attention in ("packed", "varlen", "varlen_packed"):
         probs = None
         if fused_attention == "packed":
@@ -133,16 +140,15 @@ def padding_removal_layer(hidden_padded: torch.Tensor, qkv_packed: torch.Tensor,
     return dict(x=x, qkv=qkv, probs=probs, ctx=ctx, ctx_packed=ctx_packed, y=y)
 
 
-_FORMS = {False: 0, True: 1, "packed": 2, "varlen": 3, "varlen_packed": 4}
-_WIDE, _WIDE_FORM = object(), 5      # the default's alone: fp32 heads above 64 channels in one kernel
+_FORMS = {False: 0, True: 1, "packed": 2, "varlen": 3, "varlen_packed": 4, "packed_f32_wide": 5}
 
 
 def _layer_one_call(hidden_padded, qkv_packed, info, S, H, D, T, gamma, beta, eps, scale, causal, left_padded,
                     dense_out, fused_attention, fold_depad=False, ctx_out=None):
     """The same seven ops through ``en_padding_removal_layer`` (small enough: ``en_attn_fused_norm``): one native call per step."""
-    form = _WIDE_FORM if fused_attention is _WIDE else _FORMS[fused_attention]
+    form = _FORMS[fused_attention]
     left = bool(left_padded)
-    fused_f32 = hidden_padded.dtype == torch.float32 and form in (1, 2, _WIDE_FORM)      # the fp32 kernel's tiles are not the table's
+    fused_f32 = hidden_padded.dtype == torch.float32 and form in (1, 2, 5)      # the fp32 kernels' tiles are not the table's
     kv_bytes = 2 * S * D * hidden_padded.element_size()
     table = arrivals = None
     if fold_depad and not info.ephemeral:

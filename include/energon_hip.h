@@ -367,8 +367,8 @@ int en_attn_fused(const void *q, const void *k, const void *v, void *ctx, const 
 
 /* Attention of a self-attention batch of fp32 heads of 65..128 channels (a multiple of 4) in one kernel: qkv [T, head_num,
  * 3 size_per_head] and ctx [T, head_num, size_per_head] are packed, both on 16 bytes, scale is positive.  Not en_attn_qk,
- * en_scale_mask_softmax and en_attn_pv to the bit: no score is stored and the sums run in another order.  _pays: 1 where the step
- * takes it by itself, 0 where it takes those three. */
+ * en_scale_mask_softmax and en_attn_pv to the bit: no score is stored and the sums run in another order.  _pays: 1 for sizes it
+ * takes, all of which it is the faster form for. */
 int en_attn_fused_f32_wide_pays(int batch, int head_num, int max_seq_len, int size_per_head);
 int en_attn_fused_f32_wide(const void *qkv, void *ctx, const int32_t *seq_lens, const int32_t *cu_seqlens, int batch, int head_num,
                            int max_seq_len, int size_per_head, float scale, int causal, en_stream_t stream);
@@ -459,7 +459,8 @@ int en_block_decode(const en_block_decode_args *args, en_stream_t stream);
  * (qkv_padded, scores and ctx unused), 3 = the three separate ops on the packed projections
  * (row offsets into qkv_packed and ctx_packed: transpose_pad and transpose_depad do not run;
  * qkv_padded and ctx unused), 4 = form 3 with the scores in the packed causal layout
- * (causal, 16-bit dtypes; scores needs en_packed_scores_elems elements).  fold_depad_offsets (en_padding_offsets of this
+ * (causal, 16-bit dtypes; scores needs en_packed_scores_elems elements), 5 = en_attn_fused_f32_wide on the packed
+ * projections (fp32; qkv_padded, scores and ctx unused).  fold_depad_offsets (en_padding_offsets of this
  * batch, or NULL): if given, depad is not run and x_packed may be NULL; the LayerNorm takes
  * its residual rows straight from hidden_padded.  gamma/beta in the activation dtype.  tile_table
  * (en_attn_tile_table for seq_lens, batch, head_num, max_seq_len, or NULL) is handed to the attention kernels of

@@ -134,7 +134,9 @@ def test_entry_points_validate_before_launch():
     assert lib.en_attn_fused(16, 32, 48, 64, 80, None, 1, 1, 8, 8, 200, i64x3, i64x3, i64x3, i64x3, None, None, 1.0, 1, 1,
                              None, 0, None) == -5                        # head size above 128
     assert lib.en_padding_removal_layer(16, 32, None, 48, 64, 80, 96, 112, 128, 144, 160, 176, 192, 1, 8, 2, 8, 16, 4,
-                                        1.0, 1e-5, 1, 0, 5, None, 1, None, None) == -5   # unknown attention form
+                                        1.0, 1e-5, 1, 0, 5, None, 1, None, None) == -5   # the fp32 form in fp16
+    assert lib.en_padding_removal_layer(16, 32, None, 48, 64, 80, 96, 112, 128, 144, 160, 176, 192, 1, 8, 2, 8, 16, 4,
+                                        1.0, 1e-5, 1, 0, 6, None, 0, None, None) == -5   # unknown attention form
     assert lib.en_padding_removal_layer(16, 32, None, 48, 64, 80, 96, 112, 128, 144, 160, 176, 192, 1, 8, 2, 8, 32, 4,
                                         1.0, 1e-5, 1, 0, 0, None, 1, None, None) == -2   # LayerNorm width 32 != 2 heads x 8, no dense_out
     assert lib.en_padding_removal_layer(16, 32, None, 48, 64, 80, None, 112, 128, 144, 160, 176, 192, 1, 8, 2, 8, 16, 4,

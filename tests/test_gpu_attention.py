@@ -983,11 +983,11 @@ def test_attn_fused_f32_wide(lens, S, H, D, causal):
 
 @pytest.mark.parametrize("dense,left,fold", [(False, True, None), (True, False, None), (False, False, False)])
 def test_layer_of_wide_fp32_heads_takes_one_kernel(dense, left, fold):
-    """The default step of a batch whose fp32 scores would pass 2 MiB: the fused kernel, against the three kernels at the
-    accuracy of either, at the sizes on both sides of the line."""
+    """The default step of fp32 heads of 65..128 channels, large and small: the fused kernel, against the three kernels at the
+    accuracy of either."""
     from energonai_amd import _lib, layer
     announce("layer f32 wide", dense, left, fold)
-    assert _lib.fn.en_attn_fused_f32_wide_pays(4, 2, 257, 128) == 1 and _lib.fn.en_attn_fused_f32_wide_pays(4, 2, 256, 128) == 0
+    assert _lib.fn.en_attn_fused_f32_wide_pays(4, 2, 257, 128) == 1 and _lib.fn.en_attn_fused_f32_wide_pays(1, 1, 1, 128) == 1
     assert [_lib.fn.en_attn_fused_f32_wide_pays(64, 16, 512, d) for d in (64, 68, 70, 128, 132)] == [0, 1, 0, 1, 0]
     B, H, S, D = 4, 16, 256, 72
     lens = [256, 3, 130, 64]
@@ -1002,12 +1002,24 @@ def test_layer_of_wide_fp32_heads_takes_one_kernel(dense, left, fold):
                                      ctx_out=c) for form, c in zip((None, "varlen"), ctx)]
     assert not torch.equal(*ctx)                            # two ways of adding up
     assert max_abs(*ctx) <= 2 * BASE[torch.float32] and max_abs(*y) <= 2 * BASE[torch.float32] * float(y[1].abs().max())
-    assert _lib.fn.en_attn_fused_f32_wide_pays(1, H, 128, D) == 0
     x, qkv, lens_gpu = x[:1, :128].contiguous(), qkv[:, :100].contiguous(), lens_gpu.new_tensor([100])
-    small = layer.padding_removal_layer(x, qkv, lens_gpu, H, D, gamma, beta, left_padded=left, fold_depad=fold,
-                                        dense_out=None if out is None else out[:, :100].contiguous())
-    three = layer.padding_removal_layer(x, qkv, lens_gpu, H, D, gamma, beta, left_padded=left, fold_depad=fold,
-                                        fused_attention="varlen", dense_out=None if out is None else out[:, :100].contiguous())
-    assert torch.equal(small, three)
+    out = None if out is None else out[:, :100].contiguous()
+
+    def step(form, **more):
+        return layer.padding_removal_layer(x, qkv, lens_gpu, H, D, gamma, beta, left_padded=left, dense_out=out, fused_attention=form, **more)
+
+    small, named, three = (step(form, fold_depad=fold) for form in (None, "packed_f32_wide", "varlen"))
+    assert torch.equal(small, named)
+    assert max_abs(small, three) <= 2 * BASE[torch.float32] * float(three.abs().max())
+    kept = step("packed_f32_wide", keep=True)
+    assert torch.equal(kept["y"], small) and max_abs(kept["ctx_packed"], step("varlen", keep=True)["ctx_packed"]) <= 2 * BASE[torch.float32]
+    y = layer.padding_removal_layer_noalloc(x, qkv, lens_gpu, H, D, gamma, beta, torch.empty_like(small), 100, left_padded=left, dense_out=out,
+                                            fused_attention="packed_f32_wide", fold_depad=fold is not False)
+    assert torch.equal(y, small)
+    # a scale that is zero in fp32 is the three kernels', which take it
+    assert torch.equal(step(None, fold_depad=fold, scale=2.0 ** -150), step("varlen", fold_depad=fold, scale=2.0 ** -150))
+    with pytest.raises(RuntimeError):
+        layer.padding_removal_layer(x.half(), qkv.half(), lens_gpu, H, D, gamma.half(), beta.half(), left_padded=left,
+                                    dense_out=None if out is None else out.half(), fused_attention="packed_f32_wide")
     with pytest.raises(KeyError):
         layer.padding_removal_layer(x, qkv, lens_gpu, H, D, gamma, beta, dense_out=out, fused_attention="wide")

@@ -330,7 +330,7 @@ def test_layer_single_call_equals_the_op_by_op_sequence(name, form):
 @pytest.mark.parametrize("name,want_form", [("c1", "packed"), ("c2", "packed")])
 def test_layer_default_form(name, want_form):
     """With no form named the step runs the fused kernel on the packed projections where it applies (16-bit
-    storage; fp32 with heads of up to 64 channels), else the three kernels on packed operands; depad is folded
+    storage; fp32), else the three kernels on packed operands; depad is folded
     into the LayerNorm either way."""
     layer, wl = _mods()
     w = wl.BY_NAME[name]
@@ -344,8 +344,9 @@ def test_layer_default_form(name, want_form):
     default = layer.padding_removal_layer(*args, dense_out=dense)
     named = layer.padding_removal_layer(*args, dense_out=dense, fused_attention=want_form, fold_depad=True)
     assert torch.equal(default, named)
-    # fp32 heads above 64 channels have no fused kernel: the three kernels on packed operands
-    assert layer.default_attention_form(False, torch.float32, 128, 128, 0.1) == "varlen"
+    # fp32 heads of 65..128 channels have a kernel of their own; what neither takes goes to the three kernels on packed operands
+    assert layer.default_attention_form(False, torch.float32, 128, 128, 0.1) == "packed_f32_wide"
+    assert layer.default_attention_form(False, torch.float32, 128, 70, 0.1) == "varlen"
     assert layer.default_attention_form(True, torch.float32, 128, 64, 0.1) == "packed"
     # and the default form meets the bound against the oracle that rounds nothing in between
     want = eager.layer_unpadded(inp["hidden_padded"], inp["qkv_packed"], inp["lens_list"], w.heads, w.head_dim,
@@ -668,7 +669,7 @@ def test_attention_and_layernorm_in_one_launch(dtype, lens, S, H, D, causal, lef
     from energonai_amd.seqinfo import build_seq_info
     announce("one launch", dtype, lens[:5], S, H, D, causal, left)
     if dtype == torch.float32 and D > 64:
-        pytest.skip("the fp32 kernel takes heads of up to 64 channels")
+        pytest.skip("the fp32 kernel with the LayerNorm in its launch takes heads of up to 64 channels")
     g = torch.Generator().manual_seed(S + H)
     B, T, hid, scale = len(lens), sum(lens), H * D, D ** -0.5
     hidden, qkv = torch.randn(B, S, hid, generator=g).to(dtype).cuda(), torch.randn(1, T, H, 3 * D, generator=g).to(dtype).cuda()

@@ -200,11 +200,22 @@ def test_ft_family_random_shapes(seed):
 def test_layer_random_shapes(seed):
     """The whole step on drawn shapes (LayerNorm width equal to or different from heads x head size, either
     padding side, causal or not, every attention form, depad folded or not) against the oracle's layer."""
-    from energonai_amd import layer
     ri = _draw(7500 + seed)
     B, S, H = ri(1, 6), 8 * ri(1, 40), ri(1, 4)
     D = [32, 64, 80, 128][ri(0, 3)]
-    dtype = [torch.float16, torch.bfloat16, torch.float32][ri(0, 2)]
+    _check_layer(seed, ri, B, S, H, D, [torch.float16, torch.bfloat16, torch.float32][ri(0, 2)])
+
+
+@pytest.mark.parametrize("seed", list(range(8)))
+def test_layer_random_fp32_heads_above_64_channels(seed):
+    """The same on fp32 heads of 68..128 channels in buckets of any length, from a few rows to scores of several MiB."""
+    ri = _draw(7800 + seed)
+    B, S, H = ri(1, 6), [ri(1, 60), ri(61, 420)][ri(0, 1)], ri(1, 9)
+    _check_layer(seed, ri, B, S, H, 4 * ri(17, 32), torch.float32)
+
+
+def _check_layer(seed, ri, B, S, H, D, dtype):
+    from energonai_amd import layer
     wide = bool(ri(0, 1))                       # a dense projection between attention and LayerNorm
     hid = 8 * ri(4, 160) if wide else H * D
     causal, left = bool(ri(0, 1)), bool(ri(0, 1))
@@ -242,11 +253,13 @@ def test_layer_random_shapes(seed):
         forms += [(True, False), ("packed", False), ("packed", True)]
         if causal:
             forms += [("varlen_packed", False), ("varlen_packed", True)]
+    elif D > 64:
+        forms += [("packed_f32_wide", False), ("packed_f32_wide", True)]
     for form, fold in forms:
         y = layer.padding_removal_layer(*args, dense_out=dense_g, fused_attention=form, fold_depad=fold)
         assert y.shape == (1, T, hid)
         if form is None:        # the default: the fused kernel wherever it applies, else the three kernels
-            three_kernels = layer.default_attention_form(causal, dtype, S, D, scale) != "packed"
+            three_kernels = layer.default_attention_form(causal, dtype, S, D, scale) not in ("packed", "packed_f32_wide")
         else:
             three_kernels = form in (False, "varlen", "varlen_packed")
         assert_stored_close(y.cpu(), (want_r if three_kernels else want)["y"], dtype, base=base_y, what=f"y {form} {fold}")
