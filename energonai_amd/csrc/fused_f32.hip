@@ -21,6 +21,60 @@
 
 namespace en {
 
+// A wave's 32 keys of the online softmax: the scores of this lane's query (register 4j + i: key 8j + i of the lane's half) become
+// probabilities over the running maximum; returns the sum of the lane's own.  `seen`: keys from the half's first on that the query
+// sees; `all`: the wave's queries see every key.  The maximum moves only where a tile's lies above it by more than 8 in the exponent of two,
+// and from -inf with the first tile: the gap stays finite where the scale is so small that 8 over it is not.
+template <int DMT>
+__device__ __forceinline__ float softmax_f32_keys(floatx16 &s, floatx16 (&o)[DMT], float &m_run, float &l_run, int seen, bool all, float c_exp) {
+  const float lazy_gap = fminf(8.0f / c_exp, 1e30f);
+  float m_tile = -INFINITY;
+  if (all) {
+#pragma unroll
+    for (int x = 0; x < 16; ++x) m_tile = fmaxf(m_tile, s[x]);
+  } else {
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      const float v = (8 * (x >> 2) + (x & 3) < seen) ? s[x] : -INFINITY;
+      s[x] = v;
+      m_tile = fmaxf(m_tile, v);
+    }
+  }
+  float lo, hi;
+  halves_of(m_tile, lo, hi);
+  m_tile = fmaxf(lo, hi);
+  if (__builtin_amdgcn_ballot_w64(m_tile - lazy_gap > m_run) != 0) {
+    const float m_new = fmaxf(m_run, m_tile);
+    const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m_new) * c_exp);
+    l_run *= alpha;
+#pragma unroll
+    for (int mt = 0; mt < DMT; ++mt)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) o[mt][x] *= alpha;
+    m_run = m_new;
+  }
+  const float moff = (m_run == -INFINITY) ? 0.f : -m_run * c_exp;
+  float l_tile = 0.f;
+#pragma unroll
+  for (int x = 0; x < 16; ++x) {
+    s[x] = __builtin_amdgcn_exp2f(fmaf(s[x], c_exp, moff));       // exp2(-inf) = 0: masked keys
+    l_tile += s[x];
+  }
+  return l_tile;
+}
+
+// What two waves that saw disjoint keys are weighed with: the factors of this wave's and the other's output, the sum of both and its inverse.
+struct PairWeights {
+  float mine, other, sum, inv;
+};
+__device__ __forceinline__ PairWeights pair_weights(float m0, float l0, float m1, float l1, float c_exp) {
+  const float m = fmaxf(m0, m1);
+  const float w0 = (m0 == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m0 - m) * c_exp);
+  const float w1 = (m1 == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m1 - m) * c_exp);
+  const float l = l0 * w0 + l1 * w1;
+  return {w0, w1, l, l > 0.f ? 1.0f / l : 0.f};
+}
+
 template <int DP, bool NORM>
 __device__ __forceinline__ void fused_f32_tile(const FusedArgs &fa, const NormArgs *norm) {
   typedef float T;
@@ -104,7 +158,6 @@ __device__ __forceinline__ void fused_f32_tile(const FusedArgs &fa, const NormAr
     for (int x = 0; x < 16; ++x) o[mt][x] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
   const float c_exp = fa.scale * kLog2e;
-  const float lazy_gap = 8.0f / c_exp;
 
   for (int kt = 0; kt < nkt; ++kt) {
     __syncthreads();                              // every wave has left the previous tile
@@ -131,47 +184,9 @@ __device__ __forceinline__ void fused_f32_tile(const FusedArgs &fa, const NormAr
       M::step(kf, qf[vs], s);
     }
 
-    // ---- mask + online softmax; register 4j+i holds key k0 + 8j + 4g + i of this lane's query
-    float m_tile = -INFINITY;
-    if (k0 + 32 <= vis_min) {
-#pragma unroll
-      for (int x = 0; x < 16; ++x) m_tile = fmaxf(m_tile, s[x]);
-    } else {
-      const int lim = vis_l - k0 - 4 * g;
-#pragma unroll
-      for (int x = 0; x < 16; ++x) {
-        const float v = (8 * (x >> 2) + (x & 3) < lim) ? s[x] : -INFINITY;
-        s[x] = v;
-        m_tile = fmaxf(m_tile, v);
-      }
-    }
-    {
-      float lo, hi;
-      halves_of(m_tile, lo, hi);
-      m_tile = fmaxf(lo, hi);
-    }
-    if (__builtin_amdgcn_ballot_w64(m_tile - lazy_gap > m_run) != 0) {
-      const float m_new = fmaxf(m_run, m_tile);
-      const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m_new) * c_exp);
-      l_run *= alpha;
-#pragma unroll
-      for (int mt = 0; mt < DMT; ++mt)
-#pragma unroll
-        for (int x = 0; x < 16; ++x) o[mt][x] *= alpha;
-      m_run = m_new;
-    }
-    const float moff = (m_run == -INFINITY) ? 0.f : -m_run * c_exp;
-    float l_tile = 0.f;
-#pragma unroll
-    for (int x = 0; x < 16; ++x) {
-      s[x] = __builtin_amdgcn_exp2f(fmaf(s[x], c_exp, moff));       // exp2(-inf) = 0: masked keys
-      l_tile += s[x];
-    }
-    {
-      float lo, hi;
-      halves_of(l_tile, lo, hi);
-      l_run += lo + hi;
-    }
+    float lo, hi;
+    halves_of(softmax_f32_keys(s, o, m_run, l_run, vis_l - k0 - 4 * g, k0 + 32 <= vis_min, c_exp), lo, hi);
+    l_run += lo + hi;
 
     // ---- O^T += V^T P^T: step (j, i) contracts over keys 8j + i (lanes 0..31) and 8j + 4 + i (lanes 32..63)
 #pragma unroll
@@ -203,12 +218,7 @@ __device__ __forceinline__ void fused_f32_tile(const FusedArgs &fa, const NormAr
   __syncthreads();
   if (!NORM && wk == 1) return;
   if (wk == 0) {
-    const float m1 = comb[lane], l1 = comb[kWave + lane];
-    const float m = fmaxf(m_run, m1);
-    const float w0 = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m) * c_exp);
-    const float w1 = (m1 == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m1 - m) * c_exp);
-    const float l = l_run * w0 + l1 * w1;
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const auto [w0, w1, l, inv] = pair_weights(m_run, l_run, comb[lane], comb[kWave + lane], c_exp);
     if (!NORM && q_lane >= ql) return;
     T *crow = cbase + (int64_t)q_lane * fa.c_ss;
 #pragma unroll
@@ -343,7 +353,6 @@ __global__ __launch_bounds__(kBlock, DP == 96 ? 3 : 2) void attn_fused_f32_wide_
     for (int x = 0; x < 16; ++x) o[mt][x] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
   const float c_exp = fa.scale * kLog2e;
-  const float lazy_gap = 8.0f / c_exp;
   const int ksw = kswz(r);
   const float *const krow = lds_k + (wk * 32 + r) * DP;          // wk * 32 leaves the swizzle of a row alone
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -367,41 +376,8 @@ __global__ __launch_bounds__(kBlock, DP == 96 ? 3 : 2) void attn_fused_f32_wide_
         M::step(kf[vs & 1], qf[vs], s);
       }
 
-      // ---- mask + online softmax; register 4j+i holds key k0 + 8j + 4g + i of this lane's query
-      float m_tile = -INFINITY;
-      if (k0 + 32 <= vis_min) {
-#pragma unroll
-        for (int x = 0; x < 16; ++x) m_tile = fmaxf(m_tile, s[x]);
-      } else {
-        const int lim = vis_l - k0 - 4 * g;
-#pragma unroll
-        for (int x = 0; x < 16; ++x) {
-          const float v = (8 * (x >> 2) + (x & 3) < lim) ? s[x] : -INFINITY;
-          s[x] = v;
-          m_tile = fmaxf(m_tile, v);
-        }
-      }
-      float lo, hi;
-      halves_of(m_tile, lo, hi);
-      m_tile = fmaxf(lo, hi);
-      if (__builtin_amdgcn_ballot_w64(m_tile - lazy_gap > m_run) != 0) {
-        const float m_new = fmaxf(m_run, m_tile);
-        const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m_new) * c_exp);
-        l_run *= alpha;
-#pragma unroll
-        for (int mt = 0; mt < DMT; ++mt)
-#pragma unroll
-          for (int x = 0; x < 16; ++x) o[mt][x] *= alpha;
-        m_run = m_new;
-      }
-      const float moff = (m_run == -INFINITY) ? 0.f : -m_run * c_exp;
-      float l_tile = 0.f;
-#pragma unroll
-      for (int x = 0; x < 16; ++x) {
-        s[x] = __builtin_amdgcn_exp2f(fmaf(s[x], c_exp, moff));       // exp2(-inf) = 0: masked keys
-        l_tile += s[x];
-      }
-      l_run += l_tile;                            // each half of the wave adds up its own keys
+      // each half of the wave adds up its own keys
+      l_run += softmax_f32_keys(s, o, m_run, l_run, vis_l - k0 - 4 * g, k0 + 32 <= vis_min, c_exp);
     }
 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -443,12 +419,7 @@ __global__ __launch_bounds__(kBlock, DP == 96 ? 3 : 2) void attn_fused_f32_wide_
       for (int x = 0; x < 8; ++x) mine[(2 + mt * 8 + x) * kWave + lane] = o[mt][8 * decltype(half)::value + x];
   };
   auto finish = [&](auto half) {
-    const float m1 = other[lane], l1 = other[kWave + lane];
-    const float m = fmaxf(m_run, m1);
-    const float w0 = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m) * c_exp);
-    const float w1 = (m1 == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m1 - m) * c_exp);
-    const float l = l_run * w0 + l1 * w1;
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const auto [w0, w1, l, inv] = pair_weights(m_run, l_run, other[lane], other[kWave + lane], c_exp);
     T *crow = cbase + (int64_t)q_lane * fa.c_ss;
 #pragma unroll
     for (int mt = 0; mt < DMT; ++mt)

@@ -981,6 +981,23 @@ def test_attn_fused_f32_wide(lens, S, H, D, causal):
     assert excess(ctx[:T].cpu(), want, torch.float32) <= BASE[torch.float32]
 
 
+@pytest.mark.parametrize("scale", [1e-38, 1e-40])
+@pytest.mark.parametrize("D", [64, 96, 128])
+def test_fused_f32_of_a_scale_near_zero(D, scale):
+    """A scale so small that 8 over it is no finite number: every key weighs the same, as the three kernels have it."""
+    from energonai_amd import layer
+    announce("fused f32 scale near zero", D, scale)
+    lens, S, H = [100, 5, 70], 100, 3
+    T, hid = sum(lens), H * D
+    g = torch.Generator().manual_seed(D)
+    qkv, x = torch.randn(1, T, H, 3 * D, generator=g), torch.randn(3, S, hid, generator=g)
+    ones, ctx = torch.ones(hid, device="cuda"), torch.zeros(1, T, H, D, device="cuda")
+    layer.padding_removal_layer(x.cuda(), qkv.cuda(), torch.tensor(lens, dtype=torch.int32).cuda(), H, D, ones, ones, scale=scale, ctx_out=ctx)
+    v = qkv[0, :, :, 2 * D:].double()
+    want = torch.cat([torch.cumsum(v[t:t + n], 0) / torch.arange(1, n + 1).view(n, 1, 1) for t, n in zip((0, 100, 105), lens)])
+    assert_stored_close(ctx[0].cpu(), want, torch.float32)
+
+
 @pytest.mark.parametrize("dense,left,fold", [(False, True, None), (True, False, None), (False, False, False)])
 def test_layer_of_wide_fp32_heads_takes_one_kernel(dense, left, fold):
     """The default step of fp32 heads of 65..128 channels, large and small: the fused kernel, against the three kernels at the
