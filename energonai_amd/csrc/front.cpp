@@ -1,5 +1,5 @@
-// The host side of a layer step, a decode step, the single operations and a batch's bookkeeping as one native call each: argument checks, output
-// allocation (torch's caching allocator), stream lookup and the C ABI call.  The same work in Python and ctypes costs 16 us
+// The host side of a layer step, a decode step, the single operations and a batch's bookkeeping as one native call each: argument
+// checks, output allocation (torch's caching allocator), stream lookup and the C ABI call.  The same work in Python and ctypes costs 16 us
 // per layer step and 23 us per decode step against 6 us of kernel launches, which is more than the GPU needs for a short
 // prompt (9 us) or a decode step of one sequence.  Nothing is computed here; every launch is an entry point of
 // libenergon_hip.so.
@@ -455,11 +455,33 @@ void order_stream(PyObject *info, const Tensor &t) {
   Py_DECREF(done);
 }
 
-bool number(PyObject *o) { return PyFloat_Check(o) || PyLong_Check(o); }
+// Numbers and flags of a plain call.  False, with no Python error left, for what is none or does not fit: the Python call names it.
+bool whole(PyObject *o, int64_t &v) {
+  if (!PyLong_Check(o)) return false;
+  int overflow = 0;
+  v = PyLong_AsLongLongAndOverflow(o, &overflow);
+  return overflow == 0;
+}
+bool number(PyObject *o, float &v) {
+  if (!PyFloat_Check(o) && !PyLong_Check(o)) return false;
+  const double d = PyFloat_AsDouble(o);
+  if (d == -1.0 && PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  v = (float)d;
+  return true;
+}
+bool flag(PyObject *o, int &v) {      // True, False or a plain int: asking others may run their code, fail, or wait for a GPU
+  if (!PyBool_Check(o) && !PyLong_CheckExact(o)) return false;
+  v = PyObject_IsTrue(o);
+  return true;
+}
 
 bool is_width(PyObject *shape, int64_t n) {      // n, or (n,)
   if (PyTuple_Check(shape) && PyTuple_GET_SIZE(shape) == 1) shape = PyTuple_GET_ITEM(shape, 0);
-  return PyLong_CheckExact(shape) && integer(shape) == n;
+  int64_t width;
+  return PyLong_CheckExact(shape) && whole(shape, width) && width == n;
 }
 
 // layer_norm(input, weight, bias, normalized_shape, eps, residual or None) -> y or None
@@ -468,13 +490,13 @@ PyObject *layer_norm(PyObject *const *a) {
   if (!x || !w || !b || modes_on() || w->dim() != 1 || b->sizes() != w->sizes() || b->scalar_type() != w->scalar_type()) Py_RETURN_NONE;
   const int64_t n2 = w->numel();
   const int in = known_tag(*x), out = known_tag(*w);
-  if (in < 0 || out < 0 || (in != out && in != EN_F32) || x->dim() < 1 || x->size(-1) != n2 || !is_width(a[3], n2) || !number(a[4])) Py_RETURN_NONE;
+  float eps;
+  if (in < 0 || out < 0 || (in != out && in != EN_F32) || x->dim() < 1 || x->size(-1) != n2 || !is_width(a[3], n2) || !number(a[4], eps)) Py_RETURN_NONE;
   if (a[5] != Py_None) {
     r = plain_contiguous(a[5]);
     if (!r || r->scalar_type() != x->scalar_type() || r->sizes() != x->sizes() || r->device() != x->device()) Py_RETURN_NONE;
   }
   if (w->device() != x->device() || b->device() != x->device()) Py_RETURN_NONE;
-  const float eps = real(a[4]);
   const c10::DeviceGuard guard(x->device());
   const Tensor y = at::empty(x->sizes(), w->options());
   void *y_p = y.data_ptr();
@@ -535,8 +557,8 @@ PyObject *decode_attn_paged(PyObject *const *a) {
   for (const Tensor *t : {kp, vp})
     if (t->scalar_type() != q->scalar_type() || t->device() != q->device()) Py_RETURN_NONE;
   const Tensor *table = page_table(a[4], *q, B);
-  if (!table || (a[5] != Py_None && !number(a[5]))) Py_RETURN_NONE;
-  const float scale = a[5] == Py_None ? (float)std::pow((double)D, -0.5) : real(a[5]);
+  float scale = (float)std::pow((double)D, -0.5);
+  if (!table || (a[5] != Py_None && !number(a[5], scale))) Py_RETURN_NONE;
   const c10::DeviceGuard guard(q->device());
   order_stream(a[3], *q);
   const int64_t pages = table->size(1), need = en_decode_attn_workspace_bytes((int)B, (int)H, (int)(pages * P), (int)D);
@@ -565,10 +587,12 @@ bool fits_int(std::initializer_list<int64_t> values) {
 PyObject *depad(PyObject *const *a) {
   const Tensor *src = plain_contiguous(a[0]);
   if (!src || modes_on() || src->dim() != 3) Py_RETURN_NONE;
-  const int64_t batch = integer(a[2]), left = PyObject_IsTrue(a[3]), total = integer(a[4]), S = src->size(1), hid = src->size(2);
+  const int64_t S = src->size(1), hid = src->size(2);
   const int es = (int)src->element_size();
+  int64_t batch, total;
+  int left;
   Lens info;
-  if ((es != 2 && es != 4) || left < 0 || !fits_int({batch, S, total}) || !lens_of(a[1], *src, batch, true, info)) Py_RETURN_NONE;
+  if ((es != 2 && es != 4) || !whole(a[2], batch) || !flag(a[3], left) || !whole(a[4], total) || !fits_int({batch, S, total}) || !lens_of(a[1], *src, batch, true, info)) Py_RETURN_NONE;
   const c10::DeviceGuard guard(src->device());
   order_stream(a[1], *src);
   const Tensor dst = at::empty({1, total, hid}, src->options());
@@ -576,7 +600,7 @@ PyObject *depad(PyObject *const *a) {
   void *dst_p = dst.data_ptr();
   const int32_t *cu_p = i32(*info.cu);
   const hipStream_t stream = stream_of(*src);
-  check(without_gil([&] { return en_depad(src_p, dst_p, cu_p, (int)batch, (int)S, hid, es, (int)left, stream); }), "depad");
+  check(without_gil([&] { return en_depad(src_p, dst_p, cu_p, (int)batch, (int)S, hid, es, left, stream); }), "depad");
   return THPVariable_Wrap(dst);
 }
 
@@ -584,10 +608,10 @@ PyObject *depad(PyObject *const *a) {
 PyObject *transpose_pad(PyObject *const *a) {
   const Tensor *src = plain_contiguous(a[0]);
   if (!src || modes_on()) Py_RETURN_NONE;
-  const int64_t batch = integer(a[2]), S = integer(a[3]), H = integer(a[4]), D = integer(a[5]);
   const int es = (int)src->element_size();
+  int64_t batch, S, H, D;
   Lens info;
-  if ((es != 2 && es != 4) || !fits_int({batch, S, H, D}) || src->numel() % (H * D) || !lens_of(a[1], *src, batch, true, info)) Py_RETURN_NONE;
+  if ((es != 2 && es != 4) || !whole(a[2], batch) || !whole(a[3], S) || !whole(a[4], H) || !whole(a[5], D) || !fits_int({batch, S, H, D}) || src->numel() % (H * D) || !lens_of(a[1], *src, batch, true, info)) Py_RETURN_NONE;
   const c10::DeviceGuard guard(src->device());
   order_stream(a[1], *src);
   const Tensor dst = at::empty({batch, H, S, D}, src->options());
@@ -603,10 +627,10 @@ PyObject *transpose_pad(PyObject *const *a) {
 PyObject *transpose_depad(PyObject *const *a) {
   const Tensor *src = plain_contiguous(a[0]);
   if (!src || modes_on()) Py_RETURN_NONE;
-  const int64_t batch = integer(a[2]), total = integer(a[3]), S = integer(a[4]), H = integer(a[5]), D = integer(a[6]);
   const int es = (int)src->element_size();
+  int64_t batch, total, S, H, D;
   Lens info;
-  if ((es != 2 && es != 4) || !fits_int({batch, total, S, H, D}) || src->numel() / batch / H / S != D || src->numel() != batch * H * S * D ||
+  if ((es != 2 && es != 4) || !whole(a[2], batch) || !whole(a[3], total) || !whole(a[4], S) || !whole(a[5], H) || !whole(a[6], D) || !fits_int({batch, total, S, H, D}) || src->numel() / batch / H / S != D || src->numel() != batch * H * S * D ||
       !lens_of(a[1], *src, batch, true, info))
     Py_RETURN_NONE;
   const c10::DeviceGuard guard(src->device());
@@ -624,20 +648,22 @@ PyObject *transpose_depad(PyObject *const *a) {
 PyObject *scale_mask_softmax(PyObject *const *a) {
   const Tensor *src = plain_contiguous(a[0]);
   if (!src || modes_on()) Py_RETURN_NONE;
-  const int64_t batch = integer(a[2]), S = integer(a[3]), H = integer(a[4]), causal = PyObject_IsTrue(a[6]), tail = integer(a[7]);
   const int tag = known_tag(*src);
+  int64_t batch, S, H, tail;
+  int causal;
+  float scale;
   Lens info;
-  if (tag < 0 || causal < 0 || !number(a[5]) || !fits_int({batch, S, H}) || tail < 0 || tail > INT32_MAX || src->numel() / batch / H / S != S ||
+  if (tag < 0 || !whole(a[2], batch) || !whole(a[3], S) || !whole(a[4], H) || !number(a[5], scale) || !flag(a[6], causal) || !whole(a[7], tail) ||
+      !fits_int({batch, S, H}) || tail < 0 || tail > INT32_MAX || src->numel() / batch / H / S != S ||
       src->numel() != batch * H * S * S || !lens_of(a[1], *src, batch, false, info))
     Py_RETURN_NONE;
-  const float scale = real(a[5]);
   const c10::DeviceGuard guard(src->device());
   order_stream(a[1], *src);
   void *src_p = src->data_ptr();
   const int32_t *lens_p = i32(*info.lens);
   const hipStream_t stream = stream_of(*src);
   check(without_gil([&] {
-          return en_scale_mask_softmax(src_p, lens_p, nullptr, (int)batch, (int)H, (int)S, (int)S, scale, (int)causal, (int)tail, tag, stream);
+          return en_scale_mask_softmax(src_p, lens_p, nullptr, (int)batch, (int)H, (int)S, (int)S, scale, causal, (int)tail, tag, stream);
         }), "scale_mask_softmax");
   Py_RETURN_TRUE;
 }
@@ -667,12 +693,13 @@ PyObject *attn_qk(PyObject *const *a) {
   const Tensor *q = plain_rows(a[0], 4), *k = plain_rows(a[1], 4);
   if (!q || !k || modes_on()) Py_RETURN_NONE;
   const int64_t B = q->size(0), H = q->size(1), Sq = q->size(2), D = q->size(3), Sk = k->size(2);
-  const int tag = known_tag(*q), causal = PyObject_IsTrue(a[4]);
+  const int tag = known_tag(*q);
+  int causal;
+  float alpha;
   Lens info;
-  if (tag < 0 || causal < 0 || !number(a[3]) || k->size(0) != B || k->size(1) != H || k->size(3) != D || k->scalar_type() != q->scalar_type() ||
+  if (tag < 0 || !number(a[3], alpha) || !flag(a[4], causal) || k->size(0) != B || k->size(1) != H || k->size(3) != D || k->scalar_type() != q->scalar_type() ||
       k->device() != q->device() || !fits_int({B, H, Sq, Sk, D}) || !lens_of(a[2], *q, B, false, info))
     Py_RETURN_NONE;
-  const float alpha = real(a[3]);
   const c10::DeviceGuard guard(q->device());
   order_stream(a[2], *q);
   Tensor keep;
@@ -694,9 +721,10 @@ PyObject *attn_pv(PyObject *const *a) {
   const Tensor *p = plain_contiguous(a[0]), *v = plain_rows(a[1], 4);
   if (!p || !v || modes_on() || p->dim() != 4) Py_RETURN_NONE;
   const int64_t B = p->size(0), H = p->size(1), Sq = p->size(2), Sk = p->size(3), D = v->size(3);
-  const int tag = known_tag(*p), causal = PyObject_IsTrue(a[3]);
+  const int tag = known_tag(*p);
+  int causal;
   Lens info;
-  if (tag < 0 || causal < 0 || v->size(0) != B || v->size(1) != H || v->size(2) != Sk || v->scalar_type() != p->scalar_type() ||
+  if (tag < 0 || !flag(a[3], causal) || v->size(0) != B || v->size(1) != H || v->size(2) != Sk || v->scalar_type() != p->scalar_type() ||
       v->device() != p->device() || !fits_int({B, H, Sq, Sk, D}) || !lens_of(a[2], *p, B, false, info))
     Py_RETURN_NONE;
   const c10::DeviceGuard guard(p->device());

@@ -358,6 +358,44 @@ def test_single_operations_give_the_same_natively_and_in_python(dtype, form, mon
         assert got.shape == want.shape and got.dtype == want.dtype and torch.equal(torch.Tensor(got), torch.Tensor(want))
 
 
+def test_single_operations_word_odd_flags_and_numbers_as_the_python_calls(monkeypatch):
+    """A flag that is an array of several values, a number past 64 bits or past a double: the error of the Python call."""
+    import numpy as np
+    from energonai_amd import _lib, kernel as K
+    from energonai_amd.seqinfo import build_seq_info
+    announce("native odd flags")
+    B, S, H, D = 2, 8, 2, 64
+    info = build_seq_info([8, 3], B)
+    q, rows = torch.randn(B, H, S, D).half().cuda(), torch.randn(B, S, H * D).half().cuda()
+    probs, w = torch.rand(B, H, S, S).half().cuda(), torch.ones(H * D).half().cuda()
+    two, many, huge = np.array([True, False]), 2 ** 70, 10 ** 400
+    calls = (lambda: K.attn_qk(q, q, info, causal=two), lambda: K.attn_pv(probs, q, info, causal=two),
+             lambda: K.scale_mask_softmax(B, S, H, probs, info, causal=two), lambda: K.depad(rows, B, info, left_padded=two, sum_seq=11),
+             lambda: K.attn_qk(q, q, info, alpha=huge), lambda: K.scale_mask_softmax(B, S, H, probs, info, scale=huge),
+             lambda: K.layer_norm_forward(rows, w, w, (H * D,), huge), lambda: K.layer_norm_forward(rows, w, w, (many,)),
+             lambda: K.depad(rows, many, info, sum_seq=11), lambda: K.transpose_pad(rows, many, S, info, H, D),
+             lambda: K.scale_mask_softmax(many, S, H, probs, info), lambda: K.transpose_depad(q, B, 11, many, info, H, D))
+
+    def refusals():
+        out = []
+        for call in calls:
+            with pytest.raises(Exception) as e:
+                call()
+            out.append((e.type, str(e.value)))
+        return out
+
+    native = refusals()
+
+    class General:
+        def __getattr__(self, name):
+            return (lambda *args: None) if name in NATIVE_OPS else getattr(front, name)
+
+    front = _lib.front
+    monkeypatch.setattr(_lib, "front", General())
+    assert native == refusals()
+    assert [t for t, _ in native[:4]] == [ValueError] * 4
+
+
 def test_which_operands_a_native_operation_takes():
     """The native forms take plain operands and leave everything else, with nothing launched, to the Python calls."""
     from energonai_amd import _lib
