@@ -592,7 +592,7 @@ PyObject *depad(PyObject *const *a) {
   int64_t batch, total;
   int left;
   Lens info;
-  if ((es != 2 && es != 4) || !whole(a[2], batch) || !flag(a[3], left) || !whole(a[4], total) || !fits_int({batch, S, total}) || !lens_of(a[1], *src, batch, true, info)) Py_RETURN_NONE;
+  if ((es != 2 && es != 4) || !whole(a[2], batch) || !flag(a[3], left) || !whole(a[4], total) || !fits_int({batch, S, total}) || src->size(0) < batch || !lens_of(a[1], *src, batch, true, info)) Py_RETURN_NONE;
   const c10::DeviceGuard guard(src->device());
   order_stream(a[1], *src);
   const Tensor dst = at::empty({1, total, hid}, src->options());

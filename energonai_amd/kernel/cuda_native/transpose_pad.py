@@ -114,6 +114,8 @@ def depad(src, batch_size, seq_lens, left_padded=False, sum_seq=None):
     src = src.contiguous()
     if src.dim() != 3:
         raise RuntimeError("depad: src must be [batch, seq, hidden]")
+    if src.shape[0] < batch_size:
+        raise RuntimeError(f"depad: src holds {src.shape[0]} sequences, batch_size is {batch_size}")
     info = seq_info(seq_lens, batch_size, src.device)
     total = info.total if sum_seq is None else _as_int(sum_seq)
     S, hid = src.shape[1], src.shape[2]

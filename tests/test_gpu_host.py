@@ -336,6 +336,7 @@ def test_single_operations_give_the_same_natively_and_in_python(dtype, form, mon
                      lambda: K.layer_norm_forward(rows, w, b, (hid,), residual=rows[:, :-1]), lambda: K.attn_qk(q, k[:, :-1], info),
                      lambda: K.attn_pv(probs, v.double(), info), lambda: K.transpose_pad(qkv.cpu(), B, S, info, H, 3 * D),
                      lambda: K.transpose_depad(ctx, B, T, S, info, H, D), lambda: K.depad(rows[0], B, info, sum_seq=T),
+                     lambda: K.depad(x[:B - 1], B, info, sum_seq=T),      # fewer sequences than the batch has
                      lambda: K.decode_attn_paged(q1, mine[0], mine[1][:-1], info, table), lambda: K.kv_pages_append(kn[:2], vn, *mine, info, table),
                      lambda: K.decode_attn_paged(q1, *mine, info, table.long()), lambda: K.scale_mask_softmax(B, S, H + 1, probs, info)):
             with pytest.raises(RuntimeError) as e:
