@@ -28,6 +28,8 @@ struct SoftmaxArgs {
   int packed;          // rows are the packed causal prefixes of common.hip.h instead of Sk elements apart
 };
 
+// Keys that row q of ql sees; kl: the keys that are there, at most a row's Sk (a key length past the row means the whole row, as it
+// does for the contractions on either side).
 __device__ __forceinline__ int visible_keys(int q, int ql, int kl, int Sk, int causal) {
   int n = causal ? min(kl, q + (kl - ql) + 1) : kl;
   n = max(n, 0);
@@ -196,7 +198,7 @@ __global__ __launch_bounds__(kRowsBlock) void softmax_rows_kernel(SoftmaxArgs a)
   const int sub = lane / LPR;
   const int l = lane % LPR;
   const int b = blockIdx.y;
-  const int kl = a.k_lens[b];
+  const int kl = min(a.k_lens[b], a.Sk);
   const int ql = min(a.q_lens ? a.q_lens[b] : min(kl, a.Sq), a.Sq);
   const int row0 = (blockIdx.x * GROUPS_PER_WAVE + sub) * R;  // inside the batch
 
@@ -299,42 +301,25 @@ __global__ __launch_bounds__(kWave) void softmax_bands_kernel(SoftmaxArgs a) {
   // the heads, a few hundred at a time, instead of forming one long run of empty workgroups per batch, during
   // which the machine would drain
   const int b = blockIdx.z, h = blockIdx.y;
-  // a key length past the row length means the whole row; rows off the 16-byte boundaries take it as it stands, as in
-  // the generic kernel: a causal row then sees as many keys more, and the row count below may pass the grid's
-  const int kl = VEC ? min(a.k_lens[b], a.Sk) : a.k_lens[b];
+  const int kl = min(a.k_lens[b], a.Sk);
   const int ql = min(a.q_lens ? a.q_lens[b] : min(kl, a.Sq), a.Sq);
   if (ql <= 0) return;
   const BandLayout L = band_layout<EPV, R>(a, kl, ql);
   T *unit = reinterpret_cast<T *>(a.src) +
             ((int64_t)b * a.H + h) * (a.packed ? packed_row_start<EPV * kPackedRowVectors>(a.Sq) : (int64_t)a.Sq * a.Sk);
   const int lane = threadIdx.x;
-  int block = blockIdx.x;
-  while (block < L.total) {
-    int i = block;
-    block = VEC ? L.total : block + (int)gridDim.x;
-    // longest rows first
-    if (i < L.blocks[4]) {
-      softmax_band_wave<DT, 4, R, STREAM, VEC>(a, unit, L.first[4] + i * 1 * R, L.first[5], kl, ql, lane);
-      continue;
-    }
-    i -= L.blocks[4];
-    if (i < L.blocks[3]) {
-      softmax_band_wave<DT, 3, R, STREAM, VEC>(a, unit, L.first[3] + i * 2 * R, L.first[4], kl, ql, lane);
-      continue;
-    }
-    i -= L.blocks[3];
-    if (i < L.blocks[2]) {
-      softmax_band_wave<DT, 2, R, STREAM, VEC>(a, unit, L.first[2] + i * 4 * R, L.first[3], kl, ql, lane);
-      continue;
-    }
-    i -= L.blocks[2];
-    if (i < L.blocks[1]) {
-      softmax_band_wave<DT, 1, R, STREAM, VEC>(a, unit, L.first[1] + i * 8 * R, L.first[2], kl, ql, lane);
-      continue;
-    }
-    i -= L.blocks[1];
-    softmax_band_wave<DT, 0, R, STREAM, VEC>(a, unit, L.first[0] + i * 16 * R, L.first[1], kl, ql, lane);
-  }
+  int i = blockIdx.x;
+  if (i >= L.total) return;
+  // longest rows first
+  if (i < L.blocks[4]) return softmax_band_wave<DT, 4, R, STREAM, VEC>(a, unit, L.first[4] + i * 1 * R, L.first[5], kl, ql, lane);
+  i -= L.blocks[4];
+  if (i < L.blocks[3]) return softmax_band_wave<DT, 3, R, STREAM, VEC>(a, unit, L.first[3] + i * 2 * R, L.first[4], kl, ql, lane);
+  i -= L.blocks[3];
+  if (i < L.blocks[2]) return softmax_band_wave<DT, 2, R, STREAM, VEC>(a, unit, L.first[2] + i * 4 * R, L.first[3], kl, ql, lane);
+  i -= L.blocks[2];
+  if (i < L.blocks[1]) return softmax_band_wave<DT, 1, R, STREAM, VEC>(a, unit, L.first[1] + i * 8 * R, L.first[2], kl, ql, lane);
+  i -= L.blocks[1];
+  softmax_band_wave<DT, 0, R, STREAM, VEC>(a, unit, L.first[0] + i * 16 * R, L.first[1], kl, ql, lane);
 }
 
 // Upper bound, over all lengths a batch may have, of the workgroups one head needs (host side of band_layout).
@@ -380,7 +365,7 @@ __global__ __launch_bounds__(kBlock) void softmax_generic_kernel(SoftmaxArgs a) 
   __shared__ float s_max[kBlock / kWave];
   __shared__ float s_sum[kBlock / kWave];
   const int b = blockIdx.y;
-  const int kl = a.k_lens[b];
+  const int kl = min(a.k_lens[b], a.Sk);
   const int ql = min(a.q_lens ? a.q_lens[b] : min(kl, a.Sq), a.Sq);
   const RowInfo ri = row_info(a, (int)blockIdx.x, kl, ql);
   if (!ri.active) return;

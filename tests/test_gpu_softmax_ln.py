@@ -141,10 +141,24 @@ def test_softmax_rows_off_the_16_byte_boundaries(dtype, shift, Sq, Sk, lens):
     for b in range(B):
         assert torch.equal(got[b, :, ql[b]:], src[b, :, ql[b]:])
         for q in range(ql[b]):
-            vis = min(q + lens[b] - ql[b] + 1, Sk)
+            vis = q + min(lens[b], Sk) - ql[b] + 1
             want = torch.softmax(src[b, :, q, :vis].double() * 0.37, -1)
             assert max_abs(got[b, :, q, :vis].double(), want) <= tol, (b, q)
             assert not got[b, :, q, vis:].any()
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("scale", [0.5, -0.5])                  # a scale that is not positive: the general kernel
+@pytest.mark.parametrize("Sq,Sk", [(9, 9), (16, 16), (40, 24), (3, 1031), (2, 2056), (2, 8200)])
+def test_softmax_of_key_lengths_past_the_row(Sq, Sk, scale, causal):
+    """A key length past the row means the whole row, in every kernel: the bits of the length cut to it."""
+    k = _kernel()
+    announce("softmax lengths past the row", Sq, Sk, scale, causal)
+    src = torch.randn(2, 2, Sq, Sk, generator=torch.Generator().manual_seed(Sk)).half().cuda()
+    for q_lens in (None, torch.tensor([Sq, 1], dtype=torch.int32).cuda()):
+        got, want = (k.scale_mask_softmax(2, Sq, 2, src.clone(), torch.tensor(lens, dtype=torch.int32).cuda(), scale=scale, causal=causal,
+                                          k_seq_len=Sk, q_len_list=q_lens) for lens in ([Sk + 21, 5000], [Sk, min(5000, Sk)]))
+        assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
