@@ -143,6 +143,7 @@ int en_ft_transpose_remove(const void *src, void *dst, int valid_word_num, int b
  * For each b and each query row q < q_lens[b]: the first n visible entries
  * become softmax(scale * src[..., :n]) and the remaining Sk-n entries zero;
  * n = k_lens[b] when causal == 0, else min(k_lens[b], q + k_lens[b] - q_lens[b] + 1).
+ * A k_lens[b] past k_seq_len counts as k_seq_len.
  * Rows q >= q_lens[b] are not touched (as in the reference, kernel.cu:14-17).
  * q_lens == NULL means q_lens[b] = min(k_lens[b], Sq).  tail_rows == 0 zeroes the
  * whole tail of every row as the reference does; tail_rows == t > 0 (a power of

@@ -237,7 +237,7 @@ def scale_mask_softmax(batch_size: int, batch_seq_len: int, head_num: int, src: 
     """
     Sq = batch_seq_len
     Sk = Sq if k_seq_len is None else k_seq_len
-    k_lens = _as_len_list(seq_lens)
+    k_lens = [min(n, Sk) for n in _as_len_list(seq_lens)]      # a length past the row: the whole row
     ql = [min(n, Sq) for n in k_lens] if q_lens is None else _as_len_list(q_lens)
     out_dtype = out_dtype or src.dtype
     x = src.reshape(batch_size, head_num, Sq, Sk)

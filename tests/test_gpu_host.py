@@ -277,11 +277,40 @@ class _Sub(torch.Tensor):
     pass
 
 
+class _General:
+    """The native module without the single operations: the Python calls do all of it."""
+
+    def __init__(self, front):
+        self._front = front
+
+    def __getattr__(self, name):
+        return (lambda *args: None) if name in NATIVE_OPS else getattr(self._front, name)
+
+
+class _Watched:
+    """The native module, noting the operands and results of the single operations."""
+
+    def __init__(self, front):
+        self._front, self.seen = front, {name: [] for name in NATIVE_OPS}
+
+    def __getattr__(self, name):
+        native = getattr(self._front, name)
+        if name not in NATIVE_OPS:
+            return native
+
+        def call(*args):
+            result = native(*args)
+            self.seen[name].append((args, result))
+            return result
+        return call
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("form", ["plain", "strided", "subclass", "side stream", "function mode"])
+@pytest.mark.parametrize("form", ["plain", "strided", "subclass", "side stream", "function mode", "dispatch mode"])
 def test_single_operations_give_the_same_natively_and_in_python(dtype, form, monkeypatch):
     """Each call that has a native form against the same call with that form turned off, bit for bit, over what either accepts; what
-    one refuses the other refuses in the same words."""
+    one refuses the other refuses in the same words.  The native forms do run where operands are plain, and leave a subclass's and a
+    mode's calls alone."""
     from energonai_amd import _lib, kernel as K
     from energonai_amd.seqinfo import build_seq_info
     announce("native single ops", dtype, form)
@@ -318,6 +347,14 @@ def test_single_operations_give_the_same_natively_and_in_python(dtype, form, mon
                     return func(*args, **(kwargs or {}))
             with Seen():
                 return ops(info)
+        if form == "dispatch mode":
+            from torch.utils._python_dispatch import TorchDispatchMode
+
+            class SeenBelow(TorchDispatchMode):
+                def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+                    return func(*args, **(kwargs or {}))
+            with SeenBelow():
+                return ops(info)
         return ops(info)
 
     def ops(info):
@@ -344,16 +381,20 @@ def test_single_operations_give_the_same_natively_and_in_python(dtype, form, mon
             refused.append(str(e.value))
         return [rows, ctx, *mine, paged, y, plain_y, wide], refused
 
-    native, native_refused = run()
-
-    class General:
-        def __getattr__(self, name):
-            return (lambda *args: None) if name in NATIVE_OPS else getattr(front, name)
-
     front = _lib.front
-    monkeypatch.setattr(_lib, "front", General())
+    watched = _Watched(front)
+    monkeypatch.setattr(_lib, "front", watched)
+    native, native_refused = run()
+    monkeypatch.setattr(_lib, "front", _General(front))
     general, general_refused = run()
     torch.cuda.synchronize()
+    for name, calls in watched.seen.items():
+        assert calls, name
+        if form in ("plain", "side stream"):
+            assert any(result is not None for _, result in calls), name
+        for args, result in calls:
+            if form in ("function mode", "dispatch mode") or any(type(a) is _Sub for a in args):
+                assert result is None, name
     assert native_refused == general_refused
     for got, want in zip(native, general):
         assert got.shape == want.shape and got.dtype == want.dtype and torch.equal(torch.Tensor(got), torch.Tensor(want))
@@ -386,13 +427,7 @@ def test_single_operations_word_odd_flags_and_numbers_as_the_python_calls(monkey
         return out
 
     native = refusals()
-
-    class General:
-        def __getattr__(self, name):
-            return (lambda *args: None) if name in NATIVE_OPS else getattr(front, name)
-
-    front = _lib.front
-    monkeypatch.setattr(_lib, "front", General())
+    monkeypatch.setattr(_lib, "front", _General(_lib.front))
     assert native == refusals()
     assert [t for t, _ in native[:4]] == [ValueError] * 4
 
@@ -408,3 +443,43 @@ def test_which_operands_a_native_operation_takes():
                  (x, w.float(), w.float(), (64,), 1e-5, None), (x, w, w.float(), (64,), 1e-5, None), (x, w, w, (4, 64), 1e-5, None),
                  (x, w, w, (32,), 1e-5, None), (x, w, w, (64,), "1e-5", None), (x, w, w, (64,), 1e-5, x.float()), (x[:0], w, w, (64,), 1e-5, None)):
         assert not take(*args)
+
+
+def test_which_operands_the_other_native_operations_take():
+    """Each with operands that it takes and, one at a time, with one that it leaves to the Python call."""
+    from energonai_amd import _lib
+    from energonai_amd.seqinfo import build_seq_info
+    announce("native operands of the other operations")
+    B, S, H, D, P, lens = 2, 24, 3, 64, 16, [24, 5]
+    T = sum(lens)
+    info, other = build_seq_info(lens, B), build_seq_info([3, 4, 5], 3)
+    half = lambda *shape: torch.randn(*shape).half().cuda()
+    strided = lambda *shape: torch.randn(*shape, 2).half().cuda()[..., 0]
+    x, qkv, q, ctx, probs = half(B, S, H * D), half(1, T, H, D), half(B, H, S, D), half(B, H, S, D), torch.rand(B, H, S, S).half().cuda()
+    kn, pool, q1 = half(B, H, D), half(4, H, P, D), half(B, H, 1, D)
+    table, over = torch.tensor([[0, 1], [2, 3]], dtype=torch.int32).cuda(), torch.zeros(1, dtype=torch.int32).cuda()
+    cases = {
+        "depad": ((x, info, B, True, T), {0: [strided(B, S, H * D), x.cpu(), x.double(), x[0], x[:1], x.as_subclass(_Sub)], 1: [other], 2: [3, 0], 3: [None, "left"],
+                                          4: [0, 2 ** 40]}),
+        "transpose_pad": ((qkv, info, B, S, H, D), {0: [strided(1, T, H, D), qkv.cpu(), qkv.double(), qkv.as_subclass(_Sub)], 1: [other], 2: [3], 3: [0], 4: [H + 1],
+                                                    5: [0, 2 ** 40]}),
+        "transpose_depad": ((ctx, info, B, T, S, H, D), {0: [strided(B, H, S, D), ctx.cpu(), ctx.double(), ctx[:1].clone()], 1: [other], 2: [3], 3: [0], 4: [S + 1],
+                                                         5: [H + 1], 6: [D + 1]}),
+        "scale_mask_softmax": ((probs.clone(), info, B, S, H, 0.5, True, 1), {0: [strided(B, H, S, S), probs.cpu(), probs.double(), probs[:1].clone()], 1: [other],
+                                                                               2: [3], 3: [S + 1], 4: [H + 1], 5: ["1"], 6: [None], 7: [-1]}),
+        "attn_qk": ((q, q, info, 1.0, True), {0: [strided(B, H, S, D), q.cpu(), q[0], q.double()], 1: [q[:, :2], q.float(), q[..., :32]], 2: [other], 3: ["1"], 4: [None]}),
+        "attn_pv": ((probs, q, info, False), {0: [strided(B, H, S, S), probs.cpu(), probs[0]], 1: [q[:, :2], q.float(), q[:, :, :8]], 2: [other], 3: [None]}),
+        "kv_pages_append": ((kn, kn, pool.clone(), pool.clone(), info, table, over), {
+            0: [strided(B, H, D), kn.cpu(), kn[:1], kn.float()], 1: [kn[:, :2], kn.float()], 2: [pool[:2], pool.cpu()], 3: [pool[:2], pool.float()], 4: [other],
+            5: [table.long(), table[:1], table.cpu()], 6: [over.long(), over.cpu()]}),
+        "decode_attn_paged": ((q1, pool, pool, info, table, None), {0: [strided(B, H, 1, D), q1.cpu(), q1.float(), q1[:1]], 1: [pool[:2], pool.float()],
+                                                                     2: [pool[:2], pool.float()], 3: [other], 4: [table.long(), table[:1]], 5: ["1"]}),
+    }
+    assert set(cases) == set(NATIVE_OPS) - {"layer_norm"}
+    for name, (args, others) in cases.items():
+        native = getattr(_lib.front, name)
+        assert native(*args) is not None, name
+        for i, values in others.items():
+            for value in values:
+                assert native(*args[:i], value, *args[i + 1:]) is None, (name, i, value if not isinstance(value, torch.Tensor) else value.shape)
+    torch.cuda.synchronize()
