@@ -7,6 +7,7 @@
     python3 bench_profiles.py issue --workload c3        # one --pmc run: matrix / vector co-execution, address unit queues
     python3 bench_profiles.py memsys --workload c3       # three --pmc runs: L2 hit rate, requests to memory, stalled channels
     python3 bench_profiles.py cases                      # rocprofv3 --kernel-trace --stats of every case of perf/cases.py
+    python3 bench_profiles.py f32-wide                   # kernel trace and SQ counters of layers of fp32 heads above 64 channels
     python3 bench_profiles.py yardstick                  # no profiler: `bench.py --copy-yardstick` as a table
 
 Each sub-command starts rocprofv3 as a child process with `python3 bench.py ...` after `--`, reads the CSV files it
@@ -293,6 +294,71 @@ def cmd_counters(ns) -> int:
     return 0
 
 
+# layers of fp32 heads above 64 channels: sequences, shortest, longest, heads, channels, causal
+F32_WIDE_SHAPES = [(8, 16, 128, 16, 96, False), (16, 100, 384, 20, 80, False), (22, 110, 110, 45, 128, True), (2, 375, 1500, 16, 128, True)]
+
+
+def f32_wide_name(shape) -> str:
+    batch, lo, hi, heads, channels, causal = shape
+    return f"{batch} of {hi if lo == hi else f'{lo}..{hi}'}, {heads} x {channels}{'' if causal else ', no mask'}"
+
+
+def cmd_run_f32_wide(ns) -> int:
+    """The program that `f32-wide` profiles: layers of one shape, the lengths spread evenly over their range."""
+    sys.path.insert(0, ROOT)
+    import torch
+
+    from energonai_amd import layer
+    from energonai_amd.seqinfo import build_seq_info
+    batch, lo, hi, heads, channels, causal = F32_WIDE_SHAPES[ns.shape]
+    lens = [hi - (hi - lo) * i // max(batch - 1, 1) for i in range(batch)]
+    total, hidden = sum(lens), heads * channels
+    g = torch.Generator().manual_seed(1)
+    x, qkv = (torch.randn(*s, generator=g).cuda() for s in ((batch, hi, hidden), (1, total, heads, 3 * channels)))
+    gamma, beta = torch.ones(hidden, device="cuda"), torch.zeros(hidden, device="cuda")
+    info = build_seq_info(torch.tensor(lens, dtype=torch.int32, device="cuda"), batch, total=total)
+    for _ in range(ns.steps):
+        layer.padding_removal_layer(x, qkv, info, heads, channels, gamma, beta, causal=causal, sum_seq=total)
+    torch.cuda.synchronize()
+    print(json.dumps({"shape": f32_wide_name(F32_WIDE_SHAPES[ns.shape]), "layers": ns.steps}), flush=True)
+    return 0
+
+
+def cmd_f32_wide(ns) -> int:
+    print("# Layers of fp32 heads above 64 channels: kernel trace and SQ counters of the attention\n")
+    print("Command (MI355X box, repo root; the summary below is this command's stdout):\n")
+    print(f"```\npython3 bench_profiles.py f32-wide --steps {ns.steps}\n```\n")
+    print_sources(None)
+    print(f"{ns.steps} layers of one batch in each run, times and counters in runs of their own.  Matrix floor: the products of the visible "
+          "scores at the 0.153 PFLOP/s that a large fp32 matrix product reaches on this card.  Columns as in the other counter summaries.\n")
+    print("| sequences, heads x channels | kernel | avg us | min us | max us | matrix floor, us | MFMA busy, share of SIMD cycles | VALU issue, share "
+          "of SIMD cycles | resident waves per SIMD | waves waiting at s_waitcnt, share of wave time | LDS bank conflict cycles / LDS active cycles "
+          "|\n|---|---|---|---|---|---|---|---|---|---|---|")
+    for i, shape in enumerate(F32_WIDE_SHAPES):
+        run = ["run-f32-wide", "--shape", str(i), "--steps", str(ns.steps)]
+        d, _, _ = run_profiler(f"f32_wide_trace{i}", ["--kernel-trace", "--stats"], run, ns.timeout, "bench_profiles.py")
+        times = trace_rows(find_csv(d, "kernel_trace.csv"))
+        d, _, _ = run_profiler(f"f32_wide_sq{i}", ["--pmc"] + SQ_COUNTERS, run, ns.timeout, "bench_profiles.py")
+        path = find_csv(d, "counter_collection.csv")
+        counters = {c: counter_rows(path, c) for c in SQ_COUNTERS}
+        batch, lo, hi, heads, channels, causal = shape
+        lens = [hi - (hi - lo) * k // max(batch - 1, 1) for k in range(batch)]
+        flops = 4.0 * heads * channels * sum(n * (n + 1) // 2 if causal else n * n for n in lens)
+        for kernel, us in sorted(times.items()):
+            if "attn_fused_f32_wide" not in kernel:
+                if "en::layernorm" in kernel:
+                    print(f"| {f32_wide_name(shape)} | `{kernel[:60]}` | {sum(us) / len(us):.1f} | {min(us):.1f} | {max(us):.1f} | | | | | | |")
+                continue
+            v = {c: sum(counters[c][kernel]) for c in SQ_COUNTERS}
+            simd = v["GRBM_GUI_ACTIVE"] / 8 * 1024
+            print(f"| {f32_wide_name(shape)} | `{kernel[:60]}` | {sum(us) / len(us):.1f} | {min(us):.1f} | {max(us):.1f} | {flops / 0.153e9:.1f} | "
+                  f"{v['SQ_VALU_MFMA_BUSY_CYCLES'] / simd:.3f} | {4 * v['SQ_ACTIVE_INST_VALU'] / simd:.3f} | "
+                  f"{4 * v['SQ_WAVE_CYCLES'] / simd:.2f} | {v['SQ_WAIT_INST_ANY'] / max(v['SQ_WAVE_CYCLES'], 1):.3f} | "
+                  f"{v['SQ_LDS_BANK_CONFLICT'] / max(v['SQ_LDS_IDX_ACTIVE'], 1):.3f} |")
+        print(f"[bench_profiles] {f32_wide_name(shape)} done", file=sys.stderr, flush=True)
+    return 0
+
+
 ISSUE_COUNTERS = ["SQ_VALU_MFMA_BUSY_CYCLES", "SQ_VALU_MFMA_COEXEC_CYCLES", "SQ_VMEM_TA_CMD_FIFO_FULL",
                   "SQ_VMEM_TA_ADDR_FIFO_FULL", "SQ_INSTS_VALU", "SQ_INSTS_MFMA", "SQ_INSTS_LDS", "GRBM_GUI_ACTIVE"]
 
@@ -500,6 +566,15 @@ def main(argv=None) -> int:
     p.add_argument("--timeout", type=int, default=120, help="seconds allowed for each rocprofv3 run")
     p.add_argument("--raw-dir", default=None, help="directory for rocprofv3's raw output (default: a temporary one)")
     p.set_defaults(fn=cmd_cases)
+    p = sub.add_parser("f32-wide")
+    p.add_argument("--steps", type=int, default=20)
+    p.add_argument("--timeout", type=int, default=60, help="seconds allowed for each rocprofv3 run")
+    p.add_argument("--raw-dir", default=None, help="directory for rocprofv3's raw output (default: a temporary one)")
+    p.set_defaults(fn=cmd_f32_wide)
+    p = sub.add_parser("run-f32-wide")
+    p.add_argument("--shape", type=int, required=True)
+    p.add_argument("--steps", type=int, default=20)
+    p.set_defaults(fn=cmd_run_f32_wide, raw_dir=None)
     p = sub.add_parser("run-case")
     p.add_argument("--case", required=True)
     p.add_argument("--steps", type=int, default=10)

@@ -259,13 +259,16 @@ __global__ __launch_bounds__(kBlock) void attn_fused_f32_kernel(FusedArgs fa) { 
 template <int DP>
 __global__ __launch_bounds__(kBlock) void attn_fused_norm_f32_kernel(FusedArgs fa, NormArgs norm) { fused_f32_tile<DP, true>(fa, &norm); }
 
-// Heads of 65..128 channels.  Bound by the matrix cores: a wave's share of a 64-key tile is 2 x 64 MFMAs of 64 cycles, and the loads,
-// the softmax and the LDS reads of one workgroup run beside the MFMAs of the other on its CU.  The same split as above (64 query
-// rows, wave (wq, wk) takes 32 of them and 32 keys of every tile, the pair is combined at the end), but the tiles travel from
-// memory straight into LDS, one buffer each for K and V: V of a tile is sent for at the top of its step and needed behind S^T, K of
-// the next one behind the barrier in mid-step, when every wave has left this one's, and needed at the end.  64 KB (48 at 96
-// channels) and no registers for tiles in flight: two workgroups (three) on a CU.  2 sequences of 375..1500, 16 heads x 128, causal,
-// with the LayerNorm: 229 us in four launches, 136 in two; 22 of 110, 45 x 128: 260 -> 137.
+// Heads of 65..128 channels.  A wave's share of a 64-key tile is 2 x 64 MFMAs of 64 cycles, and the loads, the softmax and the LDS reads of
+// one workgroup run beside the MFMAs of the others on its CU.  The matrix cores are busy 0.55 of the time where workgroups fill them evenly
+// (16 of 100..384, 20 x 80, no mask: 109 us for 45 us of products), 0.31 with rows of two tiles (22 of 110, 45 x 128: 109 us), 0.37 where
+// the longest tiles end alone (2 of 375..1500, 16 x 128: 176 us, 0.87 waves a SIMD); small batches are one workgroup's chain (8 of 16..128,
+// 16 x 96: 15 us, 0.11).  The same split as above (64 query rows, wave (wq, wk) takes 32 of them and 32 keys of every tile, the pair is
+// combined at the end), but the tiles travel from memory straight into LDS, one buffer each for K and V: V of a tile is sent for at the
+// top of its step and needed behind S^T, K of the next one behind the barrier in mid-step, when every wave has left this one's, and
+// needed at the end.  64 KB (48 at 96 channels) and no registers for tiles in flight: two workgroups (three) on a CU.  Layers with the
+// LayerNorm, QK^T + softmax + PV / this: 2 layers of 2 sequences of up to 1500, 16 heads x 128 281 / 188 us, 6 of 8 of up to 128, 16 x 96
+// 252 / 128.
 //
 // Rows are DP channels without padding; chunk c (16 bytes) of a K row r sits in slot c ^ kswz(r), so that the fragment reads of
 // sixteen consecutive rows at one chunk cover all banks; V is read a channel a lane, rows four keys apart in the wave's halves: with
